@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define NHA_ABI_VERSION 9
+#define NHA_ABI_VERSION 10
 
 enum { NHA_DTYPE_F32 = 0, NHA_DTYPE_BF16 = 1 };
 enum {
@@ -225,8 +225,14 @@ typedef struct NhaDecodeArgs {
   void* o;
   void* stream;
   int32_t* count_next; /* ring mode, optional: receives count[b] + 1 (must not alias count) */
+  void* scratch;       /* optional: nha_decode_scratch_bytes() bytes, ZERO before the first step that uses them; a step
+                          leaves its counters zero again, so steps of any shape may share it one after the other (on one
+                          stream).  Without it a call with few (sequence, kv-head) pairs runs on as few workgroups. */
+  size_t scratch_bytes;
 } NhaDecodeArgs;
 
+/* Bytes of NhaDecodeArgs.scratch, the same for every call. */
+size_t nha_decode_scratch_bytes(void);
 int nha_decode_step(const NhaDecodeArgs* a);
 /* count[b] += 1 for b < B (ring mode bookkeeping between steps). */
 int nha_decode_advance(int32_t* count, int32_t B, void* stream);

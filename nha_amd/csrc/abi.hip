@@ -186,6 +186,8 @@ int nha_prefill_bwd(const NhaPrefillBwdArgs* a) {
   return prefill_bwd_impl(a);
 }
 
+size_t nha_decode_scratch_bytes(void) { return decode_scratch_bytes(); }
+
 int nha_decode_step(const NhaDecodeArgs* a) { return decode_step_impl(a); }
 
 int nha_decode_advance(int32_t* count, int32_t B, void* stream) { return decode_advance_impl(count, B, stream); }

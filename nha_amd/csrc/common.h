@@ -143,6 +143,10 @@ int decode_step_impl(const NhaDecodeArgs* a);
 int decode_advance_impl(int32_t* count, int32_t B, void* stream);
 bool decode_mfma_supported(const NhaDecodeArgs* a);
 int decode_mfma_impl(const NhaDecodeArgs* a);
+// decode_split.hip: the calls of decode_mfma_impl with too few (sequence, kv-head) pairs to fill the chip
+size_t decode_scratch_bytes();
+bool decode_split_wanted(const NhaDecodeArgs* a);
+int decode_split_impl(const NhaDecodeArgs* a);
 size_t prefill_simple_scratch_bytes(const NhaPrefillArgs* a);
 // phase: 0 = whole op, 1 = state pass only, 2 = output pass only (scratch filled by an earlier state pass)
 int prefill_simple_impl(const NhaPrefillArgs* a, int phase);

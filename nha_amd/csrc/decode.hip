@@ -692,7 +692,7 @@ int decode_step_impl(const NhaDecodeArgs* a) {
 #else
   constexpr bool valu_only = false;
 #endif
-  if (!valu_only && decode_mfma_supported(a)) return decode_mfma_impl(a);
+  if (!valu_only && decode_mfma_supported(a)) return decode_split_wanted(a) ? decode_split_impl(a) : decode_mfma_impl(a);
   int G = 1;
   while (G < NG) G <<= 1;
   // two VALU kernels: the two-sweep kernel keeps all window logits in LDS (fewest VALU operations per

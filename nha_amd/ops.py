@@ -92,13 +92,30 @@ def _workspace(nbytes: int, dev, stream: int) -> torch.Tensor:
     return ws
 
 
+# scratch of the decode steps (arrival counters, partial results): one small buffer per (device, stream), zero when it is
+# made; a step leaves its counters zero again, so it serves every decode call of the stream
+_DECODE_SCRATCH: dict = {}
+
+
+def decode_scratch(dev, stream: int) -> torch.Tensor:
+    if torch.cuda.is_current_stream_capturing():       # a recording keeps its own, zeroed at every replay
+        return torch.zeros(_lib.load().nha_decode_scratch_bytes(), dtype=torch.uint8, device=dev)
+    ws = _DECODE_SCRATCH.get((dev, stream))
+    if ws is None:
+        while len(_DECODE_SCRATCH) >= _WORKSPACE_MAX_STREAMS:
+            _DECODE_SCRATCH.pop(next(iter(_DECODE_SCRATCH)))
+        ws = _DECODE_SCRATCH[(dev, stream)] = torch.zeros(_lib.load().nha_decode_scratch_bytes(), dtype=torch.uint8, device=dev)
+    return ws
+
+
 def release_workspaces() -> int:
-    """Drop the cached prefill workspaces (forward and backward) of every device and stream and return
+    """Drop the cached workspaces (prefill forward and backward, decode scratch) of every device and stream and return
     the bytes they held.  The buffers are grow-only: one large prefill otherwise keeps its scratch for the life of the
     process, out of reach of `torch.cuda.empty_cache()`.  Work already queued keeps its buffer alive through the
     caching allocator's stream ordering, so this is safe to call between steps."""
-    held = sum(ws.numel() for ws in _WORKSPACE.values())
+    held = sum(ws.numel() for pool in (_WORKSPACE, _DECODE_SCRATCH) for ws in pool.values())
     _WORKSPACE.clear()
+    _DECODE_SCRATCH.clear()
     return held
 
 
@@ -866,6 +883,8 @@ def fused_recurrent_nha_decode(
     a.cos, a.sin, a.cos_sb, a.cos_sw = _ptr(cos), _ptr(sin), c_sb, c_sw
     a.hk_in, a.hv_in, a.hk_out, a.hv_out = _ptr(hk0), _ptr(hv0), _ptr(hkt), _ptr(hvt)
     a.o, a.stream = _ptr(o), _stream(dev)
+    scratch = decode_scratch(dev, a.stream or 0)
+    a.scratch, a.scratch_bytes = _ptr(scratch), scratch.numel()
     _lib.check(_lib.load().nha_decode_step(C.byref(a)))
     return o, (hkt, hvt)
 

@@ -13,7 +13,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .ops import _dtype_code, _need_cuda, _ptr, _stream
+from .ops import _dtype_code, _need_cuda, _ptr, _stream, decode_scratch
 
 
 @dataclass
@@ -32,6 +32,9 @@ class NHARingState:
     # the slots never absorb anything (every cached log-gate is 0 and every write strength 0: the zero-sink layers of
     # the hybrid models): hk and hv stay zero, and the step neither reads nor writes them
     zero_state: bool = False
+    # the step's scratch, where it must not be the stream's shared one: a recorded step keeps its own (zeroed before the
+    # recording, so that a replay need not clear it)
+    scratch: Optional[torch.Tensor] = None
 
     @classmethod
     def empty(cls, B, H, K, V, M, W, dtype=torch.bfloat16, device="cuda") -> "NHARingState":
@@ -127,6 +130,8 @@ def ring_decode_step(state: NHARingState, q: torch.Tensor, sq: torch.Tensor, k_n
             state.count_alt = torch.empty_like(state.count)
         a.count_next = _ptr(state.count_alt)
     lib = _lib.load()
+    scratch = state.scratch if state.scratch is not None else decode_scratch(q.device, a.stream or 0)
+    a.scratch, a.scratch_bytes = _ptr(scratch), scratch.numel()
     _lib.check(lib.nha_decode_step(C.byref(a)))
     if advance:
         state.count, state.count_alt = state.count_alt, state.count

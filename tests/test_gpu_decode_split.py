@@ -1,0 +1,63 @@
+"""The decode step of few (sequence, kv-head) pairs (decode_split.hip) against the ring recurrence of the oracle: pairs
+around the edges of its dispatch (1, an uneven number, 64, 128, 256 and more), windows of one task, of fewer and of more
+32-key blocks than the workgroups have waves, empty, partly filled and wrapped rings, and three steps on one scratch (the
+arrival counters must be zero again after each)."""
+import pytest
+import torch
+
+from oracle import nha_ref as R
+from tests.util import assert_close, randn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,NG,H,K,W", [(1, 8, 1, 128, 33), (1, 4, 2, 128, 700), (3, 3, 3, 64, 64), (2, 1, 2, 256, 300),
+                                        (3, 2, 3, 256, 40), (16, 4, 4, 128, 130), (43, 5, 3, 64, 150), (64, 8, 2, 128, 96),
+                                        (70, 4, 4, 128, 65), (130, 2, 2, 128, 48)])
+def test_split_ring_steps(B, NG, H, K, W):
+    from nha_amd import NHARingState, ring_decode_step
+    dtype, HQ, M = torch.bfloat16, NG * H, 64
+    gen = torch.Generator().manual_seed(B * W + K)
+    ring = [randn(gen, B, W, H, d, dtype=dtype) for d in (K, K, K)]
+    ring.append((torch.nn.functional.logsigmoid(torch.randn(B, W, H, M, generator=gen)) / 8).to(dtype))
+    hk, hv = randn(gen, B, H, K, M, dtype=torch.float32, scale=0.3), randn(gen, B, H, M, K, dtype=torch.float32, scale=0.3)
+    count = torch.randint(0, 3 * W, (B,), generator=gen, dtype=torch.int32)
+    count[0] = 0 if B > 1 else 2 * W + 5
+    count[-1] = W
+    st = NHARingState(*[x.clone().cuda() for x in (hk, hv, *ring, count)])
+    for i in range(3):
+        new = [randn(gen, B, h, K, dtype=dtype) for h in (HQ, HQ, H, H, H)]
+        g = (torch.nn.functional.logsigmoid(torch.randn(B, H, M, generator=gen)) / 8).to(dtype)
+        o = ring_decode_step(st, *[x.cuda() for x in (*new, g)])
+        ro, hk, hv, ring = R.decode_ring_ref(*new, g, *ring, count, hk, hv)
+        count = count + 1
+        assert_close(f"step {i} o", o, ro, dtype)
+        assert_close(f"step {i} hk", st.hk, hk, dtype)
+        assert_close(f"step {i} hv", st.hv, hv, dtype)
+        assert torch.equal(st.count.cpu(), count)
+        for a, b in zip((st.ring_k, st.ring_kg, st.ring_v, st.ring_g), ring):
+            assert torch.equal(a.cpu().double(), b)
+    from nha_amd import ops
+    assert not any(ws[:512].any() for ws in ops._DECODE_SCRATCH.values())      # the counters the next step starts from
+
+
+def test_split_step_in_a_graph_without_scratch_of_its_own():
+    """The window form recorded into a graph on fresh scratch, replayed with eager steps in between: every replay equals
+    the eager result (the arrival counters of a recording are its own)."""
+    from nha_amd import fused_recurrent_nha_decode
+    B, HQ, H, K, W, M, dt = 2, 8, 2, 128, 200, 64, torch.bfloat16
+    gen = torch.Generator().manual_seed(3)
+    r = lambda *s: randn(gen, *s, dtype=dt).cuda()
+    a = dict(q=r(B, 1, HQ, K), sq=r(B, 1, HQ, K), k=r(B, 1, H, K), v=r(B, 1, H, K), g=-r(B, 1, H, M).abs() / 8, sw_k=r(B, W, H, K),
+             sw_v=r(B, W, H, K), initial_state=(r(B, H, K, M).float(), r(B, H, M, K).float()), output_final_state=True)
+    want, (whk, whv) = fused_recurrent_nha_decode(**a)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        o, (hk, hv) = fused_recurrent_nha_decode(**a)
+    for _ in range(4):
+        o.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, want) and torch.equal(hk, whk) and torch.equal(hv, whv)
+        assert torch.equal(fused_recurrent_nha_decode(**a)[0], want)
