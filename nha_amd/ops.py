@@ -37,7 +37,12 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _stream(dev) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(dev.index)      # a tensor's device: its index is never None
+
+
+def _as(x: Optional[torch.Tensor], dt) -> Optional[torch.Tensor]:
+    """x contiguous in dtype dt; x itself where it is that already (two attribute reads instead of two dispatched calls)."""
+    return x if x is None or (x.dtype == dt and x.is_contiguous()) else x.to(dt).contiguous()
 
 
 def _dtype_code(t: torch.Tensor) -> int:
@@ -791,7 +796,7 @@ def fused_chunk_nha_prefill(
 
 def _decode_state(initial_state, output_final_state, NG, B, H, K, V, M, dev):
     """State plumbing shared by the two T == 1 ops (fused_recurrent.py:169-179, :533-545)."""
-    if initial_state is not None and initial_state != (None, None) and initial_state[0] is not None:
+    if initial_state is not None and initial_state[0] is not None:
         hk0, hv0 = initial_state
         if hk0.dtype != torch.float32 or hv0.dtype != torch.float32:
             raise TypeError("the slot state must be float32")
@@ -860,8 +865,9 @@ def fused_recurrent_nha_decode(
         assert cos.shape[0] in (1, B) and cos.shape[1] >= W and cos.shape[2] == K, \
             f"rotary cos/sin must be [1|{B}, W2>={W}, K={K}], got {tuple(cos.shape)}"
         assert K % 2 == 0, "in-kernel rotate-half requires an even head dim"
-        cos = cos[:, -W:].to(dt).contiguous()
-        sin = sin[:, -W:].to(dt).contiguous()
+        if cos.shape[1] > W:
+            cos, sin = cos[:, -W:], sin[:, -W:]
+        cos, sin = _as(cos, dt), _as(sin, dt)
         c_sb = cos.stride(0) if cos.shape[0] == B else 0
         c_sw = cos.stride(1)
     else:
@@ -869,23 +875,19 @@ def fused_recurrent_nha_decode(
     if s is not None:
         assert s.shape == g.shape
     dev = q.device
-    cont = lambda x: None if x is None else x.to(dt).contiguous()
-    q_, sq_, k_, v_, g_, s_, swk_, swv_ = map(cont, (q, sq, k, v, g, s, sw_k, sw_v))
+    q_, sq_, k_, v_, g_, s_, swk_, swv_ = (_as(x, dt) for x in (q, sq, k, v, g, s, sw_k, sw_v))
     hk0, hv0, hkt, hvt = _decode_state(initial_state, output_final_state, NG, B, H, K, V, M, dev)
     o = torch.empty(B, 1, HQ, V, dtype=dt, device=dev)
-    a = _lib.NhaDecodeArgs()
-    a.mode, a.dtype = _lib.NHA_DECODE_WINDOW, _dtype_code(q_)
-    a.B, a.HQ, a.H, a.K, a.V, a.M, a.W = B, HQ, H, K, V, M, W
-    a.scale = float(scale)
-    a.q, a.sq = _ptr(q_), _ptr(sq_)
-    a.k_pop, a.v_pop, a.g_pop, a.s_pop = _ptr(k_), _ptr(v_), _ptr(g_), _ptr(s_)
-    a.win_k, a.win_v = _ptr(swk_), _ptr(swv_)
-    a.cos, a.sin, a.cos_sb, a.cos_sw = _ptr(cos), _ptr(sin), c_sb, c_sw
-    a.hk_in, a.hv_in, a.hk_out, a.hv_out = _ptr(hk0), _ptr(hv0), _ptr(hkt), _ptr(hvt)
-    a.o, a.stream = _ptr(o), _stream(dev)
-    scratch = decode_scratch(dev, a.stream or 0)
-    a.scratch, a.scratch_bytes = _ptr(scratch), scratch.numel()
-    _lib.check(_lib.load().nha_decode_step(C.byref(a)))
+    stream = _stream(dev)
+    scratch = decode_scratch(dev, stream)
+    p = lambda x: 0 if x is None else x.data_ptr()
+    args = _lib.pack_decode(
+        _lib.NHA_DECODE_WINDOW, _dtype_code(q_), B, HQ, H, K, V, M, W, float(scale), p(q_), p(sq_), p(k_), p(v_), p(g_), p(s_),
+        p(swk_), p(swv_), p(cos), p(sin), c_sb, c_sw, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, p(hk0), p(hv0), p(hkt), p(hvt), p(o),
+        stream, 0, p(scratch), scratch.numel())
+    rc = _lib.load().decode_step_packed(args)
+    if rc:
+        _lib.check(rc)
     return o, (hkt, hvt)
 
 

@@ -6,7 +6,6 @@ reference (nha_fla/models/nha_cache.py:105-131, :143-154; models/qwen3_moe_nha/q
 slot and attends over the valid entries, reading state and window once per kv-head."""
 from __future__ import annotations
 
-import ctypes as C
 from dataclasses import dataclass
 from typing import Optional
 
@@ -106,33 +105,30 @@ def ring_decode_step(state: NHARingState, q: torch.Tensor, sq: torch.Tensor, k_n
     _, W, H, _ = state.ring_k.shape
     V, M = state.ring_v.shape[-1], state.ring_g.shape[-1]
     dt = state.ring_k.dtype
-    for name, x, shp in (("q", q, (B, HQ, K)), ("sq", sq, (B, HQ, K)), ("k_new", k_new, (B, H, K)),
-                         ("kg_new", kg_new, (B, H, K)), ("v_new", v_new, (B, H, V)), ("g_new", g_new, (B, H, M))):
-        if tuple(x.shape) != shp or x.dtype != dt or not x.is_contiguous():
+    qshape, kshape = (B, HQ, K), (B, H, K)
+    for name, x, shp in (("q", q, qshape), ("sq", sq, qshape), ("k_new", k_new, kshape), ("kg_new", kg_new, kshape),
+                         ("v_new", v_new, (B, H, V)), ("g_new", g_new, (B, H, M))):
+        if x.shape != shp or x.dtype != dt or not x.is_contiguous():
             raise ValueError(f"{name} must be a contiguous {dt} tensor of shape {shp}, got {tuple(x.shape)} {x.dtype}")
     if scale is None:
         scale = K ** -0.5
-    o = out if out is not None else torch.empty(B, HQ, V, dtype=dt, device=q.device)
-    a = _lib.NhaDecodeArgs()
-    a.mode, a.dtype = _lib.NHA_DECODE_RING, _dtype_code(q)
-    a.B, a.HQ, a.H, a.K, a.V, a.M, a.W = B, HQ, H, K, V, M, W
-    a.scale = float(scale)
-    a.q, a.sq = _ptr(q), _ptr(sq)
-    a.ring_k, a.ring_kg, a.ring_v, a.ring_g = map(_ptr, (state.ring_k, state.ring_kg, state.ring_v, state.ring_g))
-    a.k_new, a.kg_new, a.v_new, a.g_new = _ptr(k_new), _ptr(kg_new), _ptr(v_new), _ptr(g_new)
-    a.count = _ptr(state.count)
-    if not state.zero_state:      # NULL states: the kernel takes zeros and writes nothing back
-        a.hk_in, a.hv_in, a.hk_out, a.hv_out = _ptr(state.hk), _ptr(state.hv), _ptr(state.hk), _ptr(state.hv)
-    a.o, a.stream = _ptr(o), _stream(q.device)
-    if advance:
-        # the kernel writes count + 1 into the second array; the two arrays then trade places
-        if state.count_alt is None:
-            state.count_alt = torch.empty_like(state.count)
-        a.count_next = _ptr(state.count_alt)
-    lib = _lib.load()
-    scratch = state.scratch if state.scratch is not None else decode_scratch(q.device, a.stream or 0)
-    a.scratch, a.scratch_bytes = _ptr(scratch), scratch.numel()
-    _lib.check(lib.nha_decode_step(C.byref(a)))
-    if advance:
+    dev = q.device
+    o = out if out is not None else torch.empty(B, HQ, V, dtype=dt, device=dev)
+    if advance and state.count_alt is None:
+        state.count_alt = torch.empty_like(state.count)
+    stream = _stream(dev)
+    scratch = state.scratch if state.scratch is not None else decode_scratch(dev, stream)
+    # NULL states (zero_state): the kernel takes zeros and writes nothing back
+    hk, hv = (0, 0) if state.zero_state else (state.hk.data_ptr(), state.hv.data_ptr())
+    args = _lib.pack_decode(
+        _lib.NHA_DECODE_RING, _dtype_code(q), B, HQ, H, K, V, M, W, float(scale), q.data_ptr(), sq.data_ptr(), 0, 0, 0, 0, 0, 0,
+        0, 0, 0, 0, 0, 0, state.ring_k.data_ptr(), state.ring_kg.data_ptr(), state.ring_v.data_ptr(), state.ring_g.data_ptr(),
+        k_new.data_ptr(), kg_new.data_ptr(), v_new.data_ptr(), g_new.data_ptr(), state.count.data_ptr(), hk, hv, hk, hv,
+        o.data_ptr(), stream, state.count_alt.data_ptr() if advance else 0,      # the kernel writes count + 1 there
+        scratch.data_ptr(), scratch.numel())
+    rc = _lib.load().decode_step_packed(args)
+    if rc:
+        _lib.check(rc)
+    if advance:      # the two counter arrays trade places
         state.count, state.count_alt = state.count_alt, state.count
     return o
