@@ -96,6 +96,13 @@ static bool use_mfma(const NhaPrefillArgs* a) {
   return prefill_mfma_supported(a);
 }
 
+// fp32 calls run on the fp32 matrix cores where the shape allows (NHA_IMPL_SIMPLE asks for the generic kernels)
+static int run_prefill(const NhaPrefillArgs* a, bool mfma, int phase) {
+  if (mfma) return prefill_mfma_impl(a, phase);
+  if (a->impl != NHA_IMPL_SIMPLE && prefill_f32_supported(a)) return prefill_f32_impl(a, phase);
+  return prefill_simple_impl(a, phase);
+}
+
 }  // namespace nha
 
 using namespace nha;
@@ -137,7 +144,7 @@ static int prefill_fwd_phase(const NhaPrefillArgs* a, int phase) {
     set_error("nha_prefill_fwd: scratch has %zu bytes, %zu needed", a->scratch_bytes, need);
     return NHA_ERR_SCRATCH;
   }
-  return mfma ? prefill_mfma_impl(a, phase) : prefill_simple_impl(a, phase);
+  return run_prefill(a, mfma, phase);
 }
 
 int nha_prefill_fwd_noalloc(const NhaPrefillArgs* a) {
@@ -163,7 +170,7 @@ int nha_prefill_fwd_noalloc(const NhaPrefillArgs* a) {
   NhaPrefillArgs b = *a;
   b.scratch = ptr;
   b.scratch_bytes = (size_t)NHA_NOALLOC_SCRATCH_BYTES;
-  return mfma ? prefill_mfma_impl(&b, 0) : prefill_simple_impl(&b, 0);
+  return run_prefill(&b, mfma, 0);
 }
 
 size_t nha_prefill_bwd_scratch_bytes(const NhaPrefillBwdArgs* a) {

@@ -150,6 +150,9 @@ int decode_split_impl(const NhaDecodeArgs* a);
 size_t prefill_simple_scratch_bytes(const NhaPrefillArgs* a);
 // phase: 0 = whole op, 1 = state pass only, 2 = output pass only (scratch filled by an earlier state pass)
 int prefill_simple_impl(const NhaPrefillArgs* a, int phase);
+// prefill_f32.hip: fp32 tensors at K == V in {64,128,256}, M == 64 (scratch: prefill_simple_scratch_bytes)
+bool prefill_f32_supported(const NhaPrefillArgs* a);
+int prefill_f32_impl(const NhaPrefillArgs* a, int phase);
 bool prefill_mfma_supported(const NhaPrefillArgs* a);
 size_t prefill_mfma_scratch_bytes(const NhaPrefillArgs* a);
 int prefill_mfma_impl(const NhaPrefillArgs* a, int phase);

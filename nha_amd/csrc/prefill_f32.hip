@@ -1,0 +1,427 @@
+// fp32 NHA prefill on the fp32 matrix cores of gfx950 (v_mfma_f32_16x16x4_f32): K == V == D in {64,128,256}, M == 64, any
+// grouping, window, shift, varlen.  Same op as prefill_simple.hip (which keeps every other shape) with no precision given
+// up: fp32 operands, products and sums, exact decays.
+//
+//   state_local : per (chunk, kv-head, state) the chunk's own contribution  U = K^T (S exp(gc_last - gc)), [m][d], and the
+//                 chunk-local gate cumsum gc
+//   state_scan  : h_c+1 = exp(gc_last) h_c + U_c element by element over the chunks of a sequence; U_c is replaced by h_c
+//   out         : one WAVE per (16 rows of a chunk, query head): window, slot logits, slot read, one softmax
+//
+// The generic kernels walk a sequence's chunks in one workgroup per 16 slots, every row's loads waited for one by one
+// (115 us per chunk), and their output pass redoes the slot algebra per token; here the chunks are independent but for
+// an element-wise scan, and everything else is matrix products.  Bound: launches and latencies at prompt sizes (B=1, T=512, 4
+// heads of 64: 1037 -> 31 us per call), the fp32 matrix rate beyond.
+//
+// Everything is computed transposed (a query per lane), with operands loaded from global memory in MFMA layout: A = a
+// row of keys / slots per lane (16 bytes of consecutive columns, four products per load; both operands number the
+// contraction the same way, so its order is free), and the accumulator of a score product is the B operand of the next
+// product as it stands.  No LDS, no barriers.
+#include "common.h"
+
+namespace nha {
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int BT = 64;
+constexpr int MS = 64;
+// A factored decay exp(gc_i - gr) exp(gr - gc_j) with its reference at the start of the 16 rows has one growing factor;
+// blocks in which it would pass e^60 take the pairwise form instead.
+constexpr float GROWTH_MAX = 60.f;
+
+struct FP {
+  const float *q_swa, *k_swa, *q_gsa, *k_gsa, *v, *s, *g;
+  float* o;
+  float *lse_swa, *lse_gsa;
+  const float *h0k, *h0v;
+  float *hkt, *hvt;
+  const int32_t *cu, *cidx, *coff;
+  float* gc;          // [T_tot][H][M]   chunk-local inclusive gate cumsum
+  float *hkc, *hvc;   // [NT][H][M][D]   chunk increments, then chunk-start states
+  int T_tot, N, NT, HQ, H, NG, wl, shift;
+  float scale;
+};
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+// over the four 16-lane rows of a wave
+__device__ __forceinline__ float rows_max(float x) { x = fmaxf(x, __shfl_xor(x, 16, 64)); return fmaxf(x, __shfl_xor(x, 32, 64)); }
+__device__ __forceinline__ float rows_sum(float x) { x += __shfl_xor(x, 16, 64); return x + __shfl_xor(x, 32, 64); }
+
+// grid (NT * H, 2): y = 0 the k-state and gc, 1 the v-state.  A wave owns 16 slots: lane (slot l%16, rows 16 (l/16) + i).
+template <int D>
+__global__ __launch_bounds__(256) void f32_state_local_kernel(const FP p) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, qd = lane >> 4;
+  const int m0 = 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = m0 + l16;
+  const int chunk = blockIdx.x / p.H, h = blockIdx.x % p.H;
+  const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
+  const int bos = p.cu[n] + 0, eos = p.cu[n + 1];
+  const int rows = min(BT, eos - bos - it * BT), base = it * BT - p.shift;   // row j absorbs token bos + base + j
+  const int jlo = base < 0 ? -base : 0;                                      // first row with a source token
+  float g[16], s[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int j = 16 * qd + i, jc = max(min(j, rows - 1), jlo);
+    // rows before jlo or from `rows` on absorb nothing; their loads go to a row that exists
+    const bool on = j >= jlo && j < rows;
+    const int64_t row = jlo < rows ? ((int64_t)(bos + base + jc) * p.H + h) * MS + m : ((int64_t)bos * p.H + h) * MS + m;
+    const float gv = p.g[row], sv = p.s[row];
+    g[i] = on ? gv : 0.f;
+    s[i] = on ? sv : 0.f;
+  }
+#pragma unroll
+  for (int i = 1; i < 16; ++i) g[i] += g[i - 1];
+  const float t0 = __shfl(g[15], l16, 64), t1 = __shfl(g[15], 16 + l16, 64), t2 = __shfl(g[15], 32 + l16, 64), t3 = __shfl(g[15], 48 + l16, 64);
+  const float before = qd == 0 ? 0.f : qd == 1 ? t0 : qd == 2 ? t0 + t1 : t0 + t1 + t2;
+  const float last = t0 + t1 + t2 + t3;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    g[i] += before;
+    const int j = 16 * qd + i;
+    if (blockIdx.y == 0 && j < rows) p.gc[((int64_t)(bos + it * BT + j) * p.H + h) * MS + m] = g[i];
+    s[i] *= expf(last - g[i]);
+  }
+  const float* x = blockIdx.y == 0 ? p.k_gsa : p.v;
+  float* u = (blockIdx.y == 0 ? p.hkc : p.hvc) + ((int64_t)chunk * p.H + h) * MS * D;
+  if (jlo >= rows) {
+    for (int c = 0; c < D / 16; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u[(m0 + 4 * qd + r) * D + 16 * c + l16] = 0.f;
+    return;
+  }
+#pragma unroll 2
+  for (int c = 0; c < D / 16; ++c) {
+    float b[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int j = max(min(16 * qd + i, rows - 1), jlo);
+      b[i] = x[((int64_t)(bos + base + j) * p.H + h) * D + 16 * c + l16];
+    }
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc = mfma4(s[i], b[i], acc);   // [slot 4 (l/16) + r][column l%16]
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[(m0 + 4 * qd + r) * D + 16 * c + l16] = acc[r];
+  }
+}
+
+// one thread per (sequence, kv-head, state, slot, four columns); loads of eight chunks are requested together
+template <int D>
+__global__ __launch_bounds__(256) void f32_state_scan_kernel(const FP p) {
+  constexpr int Q = D / 4;
+  int64_t x = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int c4 = 4 * (int)(x % Q); x /= Q;
+  const int m = (int)(x % MS); x /= MS;
+  const bool vs = x % 2; x /= 2;
+  const int h = (int)(x % p.H), n = (int)(x / p.H);
+  if (n >= p.N) return;
+  const int bos = p.cu[n], eos = p.cu[n + 1], c0 = p.coff[n], nc = p.coff[n + 1] - c0;
+  const int64_t sh = (int64_t)n * p.H + h;
+  f32x4 st = {0.f, 0.f, 0.f, 0.f};
+  const float* h0 = vs ? p.h0v : p.h0k;
+  if (h0) {
+    if (vs) st = ld4(h0 + (sh * MS + m) * D + c4);
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e) st[e] = h0[(sh * D + c4 + e) * MS + m];
+  }
+  float* u = (vs ? p.hvc : p.hkc) + (((int64_t)c0 * p.H + h) * MS + m) * D + c4;
+  const int64_t step = (int64_t)p.H * MS * D;
+  const float* gc = p.gc + (int64_t)h * MS + m;
+  for (int c = 0; c < nc; c += 8) {
+    f32x4 in[8];
+    float gl[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int cc = min(c + e, nc - 1), last = min(bos + (cc + 1) * BT, eos) - 1;
+      in[e] = ld4(u + cc * step);
+      gl[e] = gc[(int64_t)last * p.H * MS];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (c + e < nc) {
+        *reinterpret_cast<f32x4*>(u + (c + e) * step) = st;
+        st = st * expf(gl[e]) + in[e];
+      }
+  }
+  if (vs && p.hvt) *reinterpret_cast<f32x4*>(p.hvt + (sh * MS + m) * D + c4) = st;
+  if (!vs && p.hkt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p.hkt[(sh * D + c4 + e) * MS + m] = st[e];
+}
+
+template <int D, int WPB>
+__global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
+  constexpr int KK = D / 16;   // 16-column pieces of a row
+  const int lane = threadIdx.x & 63, l16 = lane & 15, qd = lane >> 4;
+  int unit = blockIdx.x * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int gq = unit % p.NG; unit /= p.NG;       // the heads of a group and the rows of a chunk share keys: neighbours
+  const int sub = unit & 3; unit >>= 2;
+  const int h = unit % p.H, chunk = unit / p.H;
+  if (chunk >= p.NT) return;
+  const int hq = h * p.NG + gq;
+  const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
+  const int bos = p.cu[n], eos = p.cu[n + 1];
+  const int cb = bos + it * BT, rows = min(BT, eos - cb);
+  if (16 * sub >= rows) return;
+  const int t0 = cb + 16 * sub, t = t0 + l16, tq = min(t, eos - 1);   // the lane's query; rows past the end are not stored
+  f32x4 O[KK];
+#pragma unroll
+  for (int c = 0; c < KK; ++c) O[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  f32x4 q[KK];
+  auto load_q = [&](const float* src) {
+#pragma unroll
+    for (int c = 0; c < KK; ++c) q[c] = ld4(src + ((int64_t)tq * p.HQ + hq) * D + 16 * c + 4 * qd) * p.scale;
+  };
+  // S^T[row][query] of 16 rows whose row l%16 starts at x
+  auto scores = [&](const float* x) {
+    f32x4 a[KK], acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < KK; ++c) a[c] = ld4(x + 16 * c + 4 * qd);
+#pragma unroll
+    for (int c = 0; c < KK; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        acc0 = mfma4(a[c][e], q[c][e], acc0);
+        acc1 = mfma4(a[c][e + 1], q[c][e + 1], acc1);
+      }
+    return acc0 + acc1;
+  };
+  // O^T += X^T W^T for 16 rows: W in accumulator layout, row(r) = where row 4 (l/16) + r starts
+  auto read = [&](auto row, const f32x4& w) {
+    float a[4][KK];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float* x = row(r) + l16;
+#pragma unroll
+      for (int c = 0; c < KK; ++c) a[r][c] = x[16 * c];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int c = 0; c < KK; ++c) O[c] = mfma4(a[r][c], w[r], O[c]);
+  };
+
+  // ---- window: keys max(bos, t - wl) .. t, newest 16 first (every query meets its own key in the first block) --------
+  load_q(p.q_swa);
+  const int lo = p.wl < 0 ? bos : max(bos, t0 - p.wl), mylo = p.wl < 0 ? bos : max(bos, t - p.wl);
+  float mw = -INFINITY, lw = 0.f;
+  for (int kb = t0; kb > lo - 16; kb -= 16) {
+    const int jr = max(bos, min(kb + l16, eos - 1));
+    f32x4 s = scores(p.k_swa + ((int64_t)jr * p.H + h) * D);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = kb + 4 * qd + r;
+      if (j > tq || j < mylo) s[r] = -INFINITY;
+    }
+    const float mx = rows_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
+    const float mn = fmaxf(mw, mx);
+    if (__any(mn != mw)) {   // no lane's maximum moved: nothing to rescale
+      const float alpha = expf(mw - mn);
+      lw *= alpha;
+#pragma unroll
+      for (int c = 0; c < KK; ++c) O[c] *= alpha;
+      mw = mn;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      s[r] = expf(s[r] - mw);
+      lw += s[r];
+    }
+    read([&](int r) { return p.v + ((int64_t)max(bos, min(kb + 4 * qd + r, eos - 1)) * p.H + h) * D; }, s);
+  }
+  lw = rows_sum(lw);
+
+  // ---- slot logits L[m][query], m = 16 b + 4 (l/16) + r -------------------------------------------------------------
+  load_q(p.q_gsa);
+  const int64_t ch = (int64_t)chunk * p.H + h;
+  const float* gcb = p.gc + ((int64_t)cb * p.H + h) * MS;    // gate row of chunk row j: gcb + j * H * MS
+  const int gs = p.H * MS;
+  const int base = it * BT - p.shift;                         // chunk row j absorbs token bos + base + j
+  auto src = [&](int j) { return bos + max(0, min(base + j, eos - bos - 1)); };
+  auto live = [&](int j) { return base + j >= 0 && j < rows; };
+  f32x4 gi[4], gr[4], L[4], L2[4];
+  float ga[4], growth = 0.f;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    gi[b] = ld4(gcb + (int64_t)(tq - cb) * gs + 16 * b + 4 * qd);
+    const int last = min(16 * sub + 15, rows - 1), ref = max(16 * sub - 1, 0);
+    gr[b] = sub ? ld4(gcb + (int64_t)ref * gs + 16 * b + 4 * qd) : (f32x4){0.f, 0.f, 0.f, 0.f};
+    ga[b] = sub ? gcb[(int64_t)ref * gs + 16 * b + l16] : 0.f;
+    growth = fmaxf(growth, ga[b] - gcb[(int64_t)last * gs + 16 * b + l16]);
+    L[b] = scores(p.hkc + (ch * MS + 16 * b + l16) * D);
+    L2[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) L[b][r] *= expf(gi[b][r]);
+  }
+  const bool pairwise = __any(growth > GROWTH_MAX);
+  f32x4 A;   // intra-chunk scores [row][query] of the 16 rows of `sub`
+  for (int J = 0; J <= sub; ++J) {
+    A = scores(p.k_gsa + ((int64_t)src(16 * J + l16) * p.H + h) * D);
+    if (J == sub) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * qd + r > l16) A[r] = 0.f;
+      if (pairwise) break;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = 16 * J + 4 * qd + r;
+      const float* srow = p.s + ((int64_t)src(j) * p.H + h) * MS + l16;
+      const float* grow = gcb + (int64_t)min(j, rows - 1) * gs + l16;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const float sd = live(j) ? srow[16 * b] * expf(ga[b] - grow[16 * b]) : 0.f;
+        L2[b] = mfma4(sd, A[r], L2[b]);
+      }
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) L[b][r] += L2[b][r] * expf(gi[b][r] - gr[b][r]);
+  if (pairwise)
+    for (int jj = 0; jj < 16; ++jj) {
+      const int j = 16 * sub + jj;
+      const float a = __shfl(jj & 2 ? (jj & 1 ? A[3] : A[2]) : (jj & 1 ? A[1] : A[0]), 16 * (jj >> 2) + l16, 64);
+      if (!live(j)) continue;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const f32x4 sv = ld4(p.s + ((int64_t)src(j) * p.H + h) * MS + 16 * b + 4 * qd), gj = ld4(gcb + (int64_t)j * gs + 16 * b + 4 * qd);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (jj <= l16) L[b][r] += a * sv[r] * expf(gi[b][r] - gj[r]);
+      }
+    }
+
+  // ---- one softmax over [slots | window] ----------------------------------------------------------------------------
+  float mg = -INFINITY, lg = 0.f;
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) mg = fmaxf(mg, L[b][r]);
+  mg = rows_max(mg);
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      L[b][r] = expf(L[b][r] - mg);
+      lg += L[b][r];
+    }
+  lg = rows_sum(lg);
+  if (qd == 0 && t < eos) {
+    if (p.lse_gsa) p.lse_gsa[(int64_t)t * p.HQ + hq] = mg + logf(lg);
+    if (p.lse_swa) p.lse_swa[(int64_t)t * p.HQ + hq] = mw + logf(lw);
+  }
+  const float mt = fmaxf(mg, mw), eg = expf(mg - mt), ew = expf(mw - mt);
+  const float inv = 1.f / (lg * eg + lw * ew);
+#pragma unroll
+  for (int c = 0; c < KK; ++c) O[c] *= ew * inv;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) L[b] *= eg * inv;
+
+  // ---- slot read ----------------------------------------------------------------------------------------------------
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    f32x4 w;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      w[r] = L[b][r] * expf(gi[b][r]);
+      L2[b][r] = L[b][r] * expf(gi[b][r] - gr[b][r]);
+    }
+    read([&](int r) { return p.hvc + (ch * MS + 16 * b + 4 * qd + r) * D; }, w);
+  }
+  for (int J = 0; J <= sub; ++J) {
+    f32x4 w = {0.f, 0.f, 0.f, 0.f};   // weights [row][query]
+    if (J < sub || !pairwise) {
+      const int j = 16 * J + l16;
+      const float* srow = p.s + ((int64_t)src(j) * p.H + h) * MS + 4 * qd;
+      const float* grow = gcb + (int64_t)min(j, rows - 1) * gs + 4 * qd;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const f32x4 sv = ld4(srow + 16 * b), gj = ld4(grow + 16 * b);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float sd = live(j) ? sv[r] * expf(gr[b][r] - gj[r]) : 0.f;
+          w = mfma4(sd, L2[b][r], w);
+        }
+      }
+    } else {
+      for (int jj = 0; jj < 16; ++jj) {
+        const int j = 16 * sub + jj;
+        if (!live(j)) continue;
+        float x = 0.f;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const f32x4 sv = ld4(p.s + ((int64_t)src(j) * p.H + h) * MS + 16 * b + 4 * qd), gj = ld4(gcb + (int64_t)j * gs + 16 * b + 4 * qd);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (jj <= l16) x += L[b][r] * sv[r] * expf(gi[b][r] - gj[r]);
+        }
+        x = rows_sum(x);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (jj == 4 * qd + r) w[r] = x;
+      }
+    }
+    if (J == sub)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * qd + r > l16) w[r] = 0.f;
+    read([&](int r) { return p.v + ((int64_t)src(16 * J + 4 * qd + r) * p.H + h) * D; }, w);
+  }
+  if (t < eos)
+#pragma unroll
+    for (int c = 0; c < KK; ++c) *reinterpret_cast<f32x4*>(p.o + ((int64_t)t * p.HQ + hq) * D + 16 * c + 4 * qd) = O[c];
+}
+
+template <int D>
+int run(const FP& p, int phase, hipStream_t st) {
+  if (phase != 2) {
+    hipLaunchKernelGGL((f32_state_local_kernel<D>), dim3(p.NT * p.H, 2), dim3(256), 0, st, p);
+    const int64_t threads = (int64_t)p.N * p.H * 2 * MS * (D / 4);
+    hipLaunchKernelGGL((f32_state_scan_kernel<D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, p);
+    NHA_CHECK_LAUNCH("nha_prefill_fwd(fp32 state pass)");
+  }
+  if (phase != 1) {
+    // Workgroups of four waves (neighbouring units share keys through L1) once there are four per CU, of one wave before.
+    const int64_t units = (int64_t)p.NT * p.H * 4 * p.NG;
+    if (units >= 1024) hipLaunchKernelGGL((f32_out_kernel<D, 4>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((f32_out_kernel<D, 1>), dim3((unsigned)units), dim3(64), 0, st, p);
+    NHA_CHECK_LAUNCH("nha_prefill_fwd(fp32 output pass)");
+  }
+  return NHA_OK;
+}
+
+size_t aligned(size_t x) { return (x + 255) & ~(size_t)255; }
+
+}  // namespace
+
+bool prefill_f32_supported(const NhaPrefillArgs* a) {
+  return a->dtype == NHA_DTYPE_F32 && a->K == a->V && (a->K == 64 || a->K == 128 || a->K == 256) && a->M == MS &&
+         (int64_t)a->NT * a->H * 4 * (a->HQ / a->H) < ((int64_t)1 << 31);
+}
+
+// the scratch is that of prefill_simple.hip: gc | k-states | v-states
+int prefill_f32_impl(const NhaPrefillArgs* a, int phase) {
+  FP p;
+  p.q_swa = (const float*)a->q_swa; p.k_swa = (const float*)a->k_swa; p.q_gsa = (const float*)a->q_gsa; p.k_gsa = (const float*)a->k_gsa;
+  p.v = (const float*)a->v; p.s = (const float*)a->s; p.g = (const float*)a->g; p.o = (float*)a->o;
+  p.lse_swa = a->lse_swa; p.lse_gsa = a->lse_gsa;
+  p.h0k = a->h0k; p.h0v = a->h0v; p.hkt = a->hkt; p.hvt = a->hvt;
+  p.cu = a->cu_seqlens; p.cidx = a->chunk_indices; p.coff = a->chunk_offsets;
+  char* sc = (char*)a->scratch;
+  p.gc = (float*)sc;
+  sc += aligned((size_t)a->T_tot * a->H * a->M * 4);
+  p.hkc = (float*)sc;
+  sc += aligned((size_t)a->NT * a->H * a->K * a->M * 4);
+  p.hvc = (float*)sc;
+  p.T_tot = a->T_tot; p.N = a->N; p.NT = a->NT; p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H;
+  p.wl = a->wl; p.shift = a->shift; p.scale = a->scale;
+  hipStream_t st = (hipStream_t)a->stream;
+  if (a->K == 64) return run<64>(p, phase, st);
+  if (a->K == 128) return run<128>(p, phase, st);
+  return run<256>(p, phase, st);
+}
+
+}  // namespace nha

@@ -1,0 +1,37 @@
+"""The fp32 matrix-core prefill (prefill_f32.hip) against the fp64 oracle: head sizes, groupings, lengths around the
+16-row and 64-row edges, sequences shorter than the shift, unbounded windows, initial states, and gates that forget by more
+than e^-60 within 16 rows (the pairwise decay form), everywhere or in single slots."""
+import numpy as np
+import pytest
+import torch
+
+from tests.test_gpu_prefill import run_case
+from tests.util import prefill_inputs
+
+pytestmark = pytest.mark.gpu
+F32 = torch.float32
+
+
+@pytest.mark.parametrize("D,HQ,H", [(64, 4, 4), (64, 10, 2), (128, 8, 2), (128, 3, 1), (256, 2, 1)])
+@pytest.mark.parametrize("T,wl,shift", [(15, 3, 0), (17, 16, 17), (64, 63, 64), (65, 0, 1), (200, 15, 16), (333, 100, 0), (150, -1, 3)])
+def test_f32_edges(D, HQ, H, T, wl, shift):
+    d = prefill_inputs(T * D + HQ, 2, T, HQ, H, D, D, 64, dtype=F32, qk_scale=0.5, with_state=T % 2 == 1)
+    run_case(f"D{D} {HQ}/{H} T{T} wl{wl} shift{shift}", d, wl=wl, shift=shift, dtype=F32, impl=None)
+
+
+@pytest.mark.parametrize("lens,wl,shift", [((1, 200, 3, 50, 4, 130, 2, 7), 31, 32), ((128, 64, 70, 10), 40, 0), ((300, 1, 129), 200, 70)])
+def test_f32_varlen(lens, wl, shift):
+    cu = [0] + np.cumsum(lens).tolist()
+    d = prefill_inputs(len(lens), 1, cu[-1], 4, 2, 64, 64, 64, dtype=F32, with_state=True, N=len(lens))
+    run_case(f"varlen {lens}", d, wl=wl, shift=shift, dtype=F32, impl=None, cu=cu)
+
+
+@pytest.mark.parametrize("mean", [-4.0, -8.0])
+def test_f32_strong_gates(mean):
+    """16 rows forget by up to e^-130 (mean -8): growing decay factors would pass the fp32 range.  Then single fast slots."""
+    d = prefill_inputs(7, 1, 150, 4, 2, 64, 64, 64, dtype=F32, gate_div=1.0, gate_mean=mean, with_state=True)
+    run_case(f"gates {mean}", d, wl=20, shift=0, dtype=F32, impl=None)
+    d = prefill_inputs(8, 1, 150, 4, 2, 128, 128, 64, dtype=F32)
+    d["g"][:, 40:75, :, 5] = mean
+    d["s"] = 1 - d["g"].exp()
+    run_case(f"one fast slot {mean}", d, wl=20, shift=5, dtype=F32, impl=None)
