@@ -10,7 +10,9 @@
 // The generic kernels walk a sequence's chunks in one workgroup per 16 slots, every row's loads waited for one by one
 // (115 us per chunk), and their output pass redoes the slot algebra per token; here the chunks are independent but for
 // an element-wise scan, and everything else is matrix products.  Bound: launches and latencies at prompt sizes (B=1, T=512, 4
-// heads of 64: 1037 -> 31 us per call), the fp32 matrix rate beyond.
+// heads of 64, W=64: 1028 -> 34 us of kernels), the fp32 matrix rate beyond (per call, generic kernels / these: B=1, T=2048,
+// 8/2 heads of 128, W=64 8.2 ms / 62 us; B=2, T=4096, 32/8 heads 30.7 / 0.57 ms = 46 TFLOP/s; B=1, T=4096, 16 heads of 64,
+// W=1024 16.9 / 0.29 ms = 67 TFLOP/s; a library matrix product reaches 150).
 //
 // Everything is computed transposed (a query per lane), with operands loaded from global memory in MFMA layout: A = a
 // row of keys / slots per lane (16 bytes of consecutive columns, four products per load; both operands number the
@@ -44,6 +46,15 @@ struct FP {
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+// e^x to about an ulp: 2^t of the rounded t = x log2(e), corrected to first order for what rounding t lost (an fma recovers
+// it exactly).  v_exp_f32 of the rounded product alone is off by |x| 2^-24, the library's expf takes twice the instructions
+// for ranges that do not occur here; below e^-200 everything is 0, -inf and -inf - -inf included.
+__device__ __forceinline__ float exp_f32(float x) {
+  constexpr float HI = 1.44269502f, LO = 1.92596299e-8f, LN2 = 0.693147181f;   // HI + LO = log2(e)
+  x = fmaxf(x, -200.f);
+  const float t = x * HI, lost = fmaf(x, HI, -t) + x * LO, e = __builtin_amdgcn_exp2f(t);
+  return fmaf(e, lost * LN2, e);
+}
 // over the four 16-lane rows of a wave
 __device__ __forceinline__ float rows_max(float x) { x = fmaxf(x, __shfl_xor(x, 16, 64)); return fmaxf(x, __shfl_xor(x, 32, 64)); }
 __device__ __forceinline__ float rows_sum(float x) { x += __shfl_xor(x, 16, 64); return x + __shfl_xor(x, 32, 64); }
@@ -79,7 +90,7 @@ __global__ __launch_bounds__(256) void f32_state_local_kernel(const FP p) {
     g[i] += before;
     const int j = 16 * qd + i;
     if (blockIdx.y == 0 && j < rows) p.gc[((int64_t)(bos + it * BT + j) * p.H + h) * MS + m] = g[i];
-    s[i] *= expf(last - g[i]);
+    s[i] *= exp_f32(last - g[i]);
   }
   const float* x = blockIdx.y == 0 ? p.k_gsa : p.v;
   float* u = (blockIdx.y == 0 ? p.hkc : p.hvc) + ((int64_t)chunk * p.H + h) * MS * D;
@@ -141,7 +152,7 @@ __global__ __launch_bounds__(256) void f32_state_scan_kernel(const FP p) {
     for (int e = 0; e < 8; ++e)
       if (c + e < nc) {
         *reinterpret_cast<f32x4*>(u + (c + e) * step) = st;
-        st = st * expf(gl[e]) + in[e];
+        st = st * exp_f32(gl[e]) + in[e];
       }
   }
   if (vs && p.hvt) *reinterpret_cast<f32x4*>(p.hvt + (sh * MS + m) * D + c4) = st;
@@ -173,11 +184,17 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
 #pragma unroll
     for (int c = 0; c < KK; ++c) q[c] = ld4(src + ((int64_t)tq * p.HQ + hq) * D + 16 * c + 4 * qd) * p.scale;
   };
-  // S^T[row][query] of 16 rows whose row l%16 starts at x
-  auto scores = [&](const float* x) {
-    f32x4 a[KK], acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+  // S^T[row][query] of 16 rows whose row l%16 starts at x: the loads, the products
+  struct Rows { f32x4 a[KK]; };
+  auto fetch = [&](const float* x) {
+    Rows k;
 #pragma unroll
-    for (int c = 0; c < KK; ++c) a[c] = ld4(x + 16 * c + 4 * qd);
+    for (int c = 0; c < KK; ++c) k.a[c] = ld4(x + 16 * c + 4 * qd);
+    return k;
+  };
+  auto scores = [&](const Rows& k) {
+    const f32x4* a = k.a;
+    f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < KK; ++c)
 #pragma unroll
@@ -188,27 +205,36 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
     return acc0 + acc1;
   };
   // O^T += X^T W^T for 16 rows: W in accumulator layout, row(r) = where row 4 (l/16) + r starts
-  auto read = [&](auto row, const f32x4& w) {
-    float a[4][KK];
+  struct Cols { float a[4][KK]; };
+  auto fetch_cols = [&](auto row) {
+    Cols v;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float* x = row(r) + l16;
 #pragma unroll
-      for (int c = 0; c < KK; ++c) a[r][c] = x[16 * c];
+      for (int c = 0; c < KK; ++c) v.a[r][c] = x[16 * c];
     }
+    return v;
+  };
+  auto read = [&](const Cols& v, const f32x4& w) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int c = 0; c < KK; ++c) O[c] = mfma4(a[r][c], w[r], O[c]);
+      for (int c = 0; c < KK; ++c) O[c] = mfma4(v.a[r][c], w[r], O[c]);
   };
 
   // ---- window: keys max(bos, t - wl) .. t, newest 16 first (every query meets its own key in the first block) --------
   load_q(p.q_swa);
   const int lo = p.wl < 0 ? bos : max(bos, t0 - p.wl), mylo = p.wl < 0 ? bos : max(bos, t - p.wl);
   float mw = -INFINITY, lw = 0.f;
+  auto keys = [&](int kb) { return fetch(p.k_swa + ((int64_t)max(bos, min(kb + l16, eos - 1)) * p.H + h) * D); };
+  Rows kr = keys(t0);
   for (int kb = t0; kb > lo - 16; kb -= 16) {
-    const int jr = max(bos, min(kb + l16, eos - 1));
-    f32x4 s = scores(p.k_swa + ((int64_t)jr * p.H + h) * D);
+    // the values of this block and the keys of the next are under way while its scores are formed
+    const Cols vc = fetch_cols([&](int r) { return p.v + ((int64_t)max(bos, min(kb + 4 * qd + r, eos - 1)) * p.H + h) * D; });
+    const Rows kn = keys(kb - 16);
+    f32x4 s = scores(kr);
+    kr = kn;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int j = kb + 4 * qd + r;
@@ -217,7 +243,7 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
     const float mx = rows_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
     const float mn = fmaxf(mw, mx);
     if (__any(mn != mw)) {   // no lane's maximum moved: nothing to rescale
-      const float alpha = expf(mw - mn);
+      const float alpha = exp_f32(mw - mn);
       lw *= alpha;
 #pragma unroll
       for (int c = 0; c < KK; ++c) O[c] *= alpha;
@@ -225,10 +251,10 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      s[r] = expf(s[r] - mw);
+      s[r] = exp_f32(s[r] - mw);
       lw += s[r];
     }
-    read([&](int r) { return p.v + ((int64_t)max(bos, min(kb + 4 * qd + r, eos - 1)) * p.H + h) * D; }, s);
+    read(vc, s);
   }
   lw = rows_sum(lw);
 
@@ -239,7 +265,9 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
   const int gs = p.H * MS;
   const int base = it * BT - p.shift;                         // chunk row j absorbs token bos + base + j
   auto src = [&](int j) { return bos + max(0, min(base + j, eos - bos - 1)); };
-  auto live = [&](int j) { return base + j >= 0 && j < rows; };
+  // 1 where row j absorbs a token, else 0: a factor and not a condition, so that the loads it guards need no branch (each
+  // branch's loads were waited for on their own)
+  auto live = [&](int j) { return base + j >= 0 && j < rows ? 1.f : 0.f; };
   f32x4 gi[4], gr[4], L[4], L2[4];
   float ga[4], growth = 0.f;
 #pragma unroll
@@ -249,15 +277,27 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
     gr[b] = sub ? ld4(gcb + (int64_t)ref * gs + 16 * b + 4 * qd) : (f32x4){0.f, 0.f, 0.f, 0.f};
     ga[b] = sub ? gcb[(int64_t)ref * gs + 16 * b + l16] : 0.f;
     growth = fmaxf(growth, ga[b] - gcb[(int64_t)last * gs + 16 * b + l16]);
-    L[b] = scores(p.hkc + (ch * MS + 16 * b + l16) * D);
+    L[b] = scores(fetch(p.hkc + (ch * MS + 16 * b + l16) * D));
     L2[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) L[b][r] *= expf(gi[b][r]);
+    for (int r = 0; r < 4; ++r) L[b][r] *= exp_f32(gi[b][r]);
   }
   const bool pairwise = __any(growth > GROWTH_MAX);
   f32x4 A;   // intra-chunk scores [row][query] of the 16 rows of `sub`
   for (int J = 0; J <= sub; ++J) {
-    A = scores(p.k_gsa + ((int64_t)src(16 * J + l16) * p.H + h) * D);
+    float sv[4][4], gv[4][4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = 16 * J + 4 * qd + r;
+      const float* srow = p.s + ((int64_t)src(j) * p.H + h) * MS + l16;
+      const float* grow = gcb + (int64_t)min(j, rows - 1) * gs + l16;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        sv[r][b] = srow[16 * b];
+        gv[r][b] = grow[16 * b];
+      }
+    }
+    A = scores(fetch(p.k_gsa + ((int64_t)src(16 * J + l16) * p.H + h) * D));
     if (J == sub) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -267,30 +307,25 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int j = 16 * J + 4 * qd + r;
-      const float* srow = p.s + ((int64_t)src(j) * p.H + h) * MS + l16;
-      const float* grow = gcb + (int64_t)min(j, rows - 1) * gs + l16;
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const float sd = live(j) ? srow[16 * b] * expf(ga[b] - grow[16 * b]) : 0.f;
-        L2[b] = mfma4(sd, A[r], L2[b]);
-      }
+      for (int b = 0; b < 4; ++b) L2[b] = mfma4(sv[r][b] * live(j) * exp_f32(ga[b] - gv[r][b]), A[r], L2[b]);
     }
   }
 #pragma unroll
   for (int b = 0; b < 4; ++b)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) L[b][r] += L2[b][r] * expf(gi[b][r] - gr[b][r]);
+    for (int r = 0; r < 4; ++r) L[b][r] += L2[b][r] * exp_f32(gi[b][r] - gr[b][r]);
   if (pairwise)
     for (int jj = 0; jj < 16; ++jj) {
       const int j = 16 * sub + jj;
       const float a = __shfl(jj & 2 ? (jj & 1 ? A[3] : A[2]) : (jj & 1 ? A[1] : A[0]), 16 * (jj >> 2) + l16, 64);
-      if (!live(j)) continue;
+      if (live(j) == 0.f) continue;
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
         const f32x4 sv = ld4(p.s + ((int64_t)src(j) * p.H + h) * MS + 16 * b + 4 * qd), gj = ld4(gcb + (int64_t)j * gs + 16 * b + 4 * qd);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (jj <= l16) L[b][r] += a * sv[r] * expf(gi[b][r] - gj[r]);
+          if (jj <= l16) L[b][r] += a * sv[r] * exp_f32(gi[b][r] - gj[r]);
       }
     }
 
@@ -305,7 +340,7 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
   for (int b = 0; b < 4; ++b)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      L[b][r] = expf(L[b][r] - mg);
+      L[b][r] = exp_f32(L[b][r] - mg);
       lg += L[b][r];
     }
   lg = rows_sum(lg);
@@ -313,7 +348,7 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
     if (p.lse_gsa) p.lse_gsa[(int64_t)t * p.HQ + hq] = mg + logf(lg);
     if (p.lse_swa) p.lse_swa[(int64_t)t * p.HQ + hq] = mw + logf(lw);
   }
-  const float mt = fmaxf(mg, mw), eg = expf(mg - mt), ew = expf(mw - mt);
+  const float mt = fmaxf(mg, mw), eg = exp_f32(mg - mt), ew = exp_f32(mw - mt);
   const float inv = 1.f / (lg * eg + lw * ew);
 #pragma unroll
   for (int c = 0; c < KK; ++c) O[c] *= ew * inv;
@@ -326,12 +361,13 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
     f32x4 w;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      w[r] = L[b][r] * expf(gi[b][r]);
-      L2[b][r] = L[b][r] * expf(gi[b][r] - gr[b][r]);
+      w[r] = L[b][r] * exp_f32(gi[b][r]);
+      L2[b][r] = L[b][r] * exp_f32(gi[b][r] - gr[b][r]);
     }
-    read([&](int r) { return p.hvc + (ch * MS + 16 * b + 4 * qd + r) * D; }, w);
+    read(fetch_cols([&](int r) { return p.hvc + (ch * MS + 16 * b + 4 * qd + r) * D; }), w);
   }
   for (int J = 0; J <= sub; ++J) {
+    const Cols vc = fetch_cols([&](int r) { return p.v + ((int64_t)src(16 * J + 4 * qd + r) * p.H + h) * D; });
     f32x4 w = {0.f, 0.f, 0.f, 0.f};   // weights [row][query]
     if (J < sub || !pairwise) {
       const int j = 16 * J + l16;
@@ -342,21 +378,20 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
         const f32x4 sv = ld4(srow + 16 * b), gj = ld4(grow + 16 * b);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float sd = live(j) ? sv[r] * expf(gr[b][r] - gj[r]) : 0.f;
-          w = mfma4(sd, L2[b][r], w);
+          w = mfma4(sv[r] * live(j) * exp_f32(gr[b][r] - gj[r]), L2[b][r], w);
         }
       }
     } else {
       for (int jj = 0; jj < 16; ++jj) {
         const int j = 16 * sub + jj;
-        if (!live(j)) continue;
+        if (live(j) == 0.f) continue;
         float x = 0.f;
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
           const f32x4 sv = ld4(p.s + ((int64_t)src(j) * p.H + h) * MS + 16 * b + 4 * qd), gj = ld4(gcb + (int64_t)j * gs + 16 * b + 4 * qd);
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            if (jj <= l16) x += L[b][r] * sv[r] * expf(gi[b][r] - gj[r]);
+            if (jj <= l16) x += L[b][r] * sv[r] * exp_f32(gi[b][r] - gj[r]);
         }
         x = rows_sum(x);
 #pragma unroll
@@ -368,7 +403,7 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (4 * qd + r > l16) w[r] = 0.f;
-    read([&](int r) { return p.v + ((int64_t)src(16 * J + 4 * qd + r) * p.H + h) * D; }, w);
+    read(vc, w);
   }
   if (t < eos)
 #pragma unroll
