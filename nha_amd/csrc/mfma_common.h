@@ -132,6 +132,11 @@ __device__ __forceinline__ int seb_base(int Q) { return Q == 0 ? 0 : Q == 1 ? 2 
 
 }  // namespace mf
 
+// prefill_mfma.hip: the state pass in segment form
+int prefill_mfma_segment_states(const NhaPrefillArgs* a, mf::MP* out);
+// prefill_bwd_slot.hip: the slot branch of the backward but for the carried state gradient, from a state pass in segment form
+int bwd_slot_branch(const NhaPrefillBwdArgs* a, const mf::MP& m, float* delta, float* xg, float* dsi, float* ek, float* ev, float* dks,
+                    float* dvs);
 // output pass with LDS-direct window loads (prefill_ring.hip); false when the shape is not served
 bool prefill_ring_supported(const mf::MP& p, int D);
 int prefill_ring_launch(const mf::MP& p, int D, hipStream_t st);

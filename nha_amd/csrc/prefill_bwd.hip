@@ -16,13 +16,14 @@
 //   dg_r  = dg_(r+1) + sum_a (du u + p dp)_r - s_r ds_r        (dg past the end = <dh_T, h_T>)
 // (the last line is the usual reverse cumulative sum of gated linear attention: <Dh_r, h_r> telescopes).
 //
-// Launches: forward state pass (chunk-start states, gate cumsums) -> bwd_q_kernel (per token: the
+// Launches (bf16 tensors with K == V in {64,128,256}, M == 64: prefill_bwd_slot.hip takes the place of everything up to the
+// recurrence over chunks): forward state pass (chunk-start states, gate cumsums) -> bwd_q_kernel (per token: the
 // vectors du, p) -> bwd_intra_kernel (per chunk: intra-chunk matrices and the intra part of ds)
 // -> bwd_dqg_kernel (per token: dq_gsa) -> bwd_state_{direct,scan,inter}_kernel (state gradients as a linear recurrence over
 // chunks: dk_gsa, slot-branch dv, inter-chunk part of ds, dh0) -> bwd_gate_*_kernel (reverse scan: ds, dg)
 // -> bwd_kv_window_kernel (per key: dk_swa, dv).  For bf16 tensors with K == V in {64,128,256} the
 // window parts (dq_swa, dk_swa, dv) run on the matrix cores instead (prefill_bwd_mfma.hip).
-#include "common.h"
+#include "mfma_common.h"
 
 namespace nha {
 namespace {
@@ -42,19 +43,17 @@ struct BP {
   float *hkct, *hvct; // [NT][H][M][K], [NT][H][V][M]   the same, transposed
   float *hkT, *hvT;   // [N][H][K][M], [N][H][M][V]     final states (for the end term of dg)
   // per-token vectors of the slot branch
-  float *dus, *pp, *xg;   // [T_tot][HQ][M]   scale*du, p, du*u + p*dp
+  float *dus, *pp, *xg;   // [T_tot][HQ][M]   scale*du, p, du*u + p*dp (xg: [T_tot][H * xNG][M])
   float *delta;           // [T_tot][HQ]
   float *ck, *cv;         // [NT][HQ][BT][BT]  sum_m dus_i s_r e^(gc_i-gc_r), same with p   (i >= r)
   float *dsi;             // [T_tot][H][M]     intra-chunk part of ds, indexed by row token
   float *dsp;             // [nbk+nbv][T_tot][H][M]  inter-chunk part of ds per column block
   float *dvs;             // [T_tot][H][V]     slot-branch dv, indexed by SOURCE token
-  const bf16_t *ap, *bp;  // [NT][HQ][BT][BT]  q_gsa_i . k'_j and do_i . v'_j from the matrix cores (bf16), or NULL
-  const float *ust, *dpst; // [T_tot][HQ][M]    q_gsa_t . hk0[:,m] and do_t . hv0[m,:] (chunk-start states), or NULL
-  const int* big;         // [NT][H] chunks the matrix-core slot kernels leave to the VALU kernels, or NULL (all)
+  const float* gcx;       // [NT][H][BT][M]    the gate cumsums by chunk (matrix-core slot branch), or NULL: gc
   float *gtot;            // [NT][H][M]        chunk sums of the dg summand, then sums of all later chunks
   float *dks;             // [T_tot][H][K]     intra-chunk part of dk_gsa, indexed by SOURCE token
   float *ek, *ev;         // [NT][H][K][M], [NT][H][V][M]  N_c, then E_c (see the state-gradient kernels)
-  int T_tot, N, NT, HQ, H, K, V, M, wl, shift, nbk, nbv;
+  int T_tot, N, NT, HQ, H, K, V, M, wl, shift, nbk, nbv, xNG;   // xNG: heads of a group that xg still keeps apart
   float scale;
 };
 
@@ -94,20 +93,9 @@ __global__ __launch_bounds__(256) void bwd_q_kernel(const BP p) {
   float* Aj = dov + V;        // [BT] q_gsa . k'_j
   float* Bj = Aj + BT;        // [BT] do . v'_j
   float* gct = Bj + BT;       // [M]
-  // Two launch shapes.  Alone (no flags): grid (NT * 16, HQ), one wave per (token, q-head).  Behind
-  // the matrix-core kernel: grid (NT, H), a workgroup leaves at once unless its (chunk, kv-head) is
-  // flagged and otherwise walks the chunk's 64 * NG (token, q-head) pairs, four at a time.
-  const bool looped = p.big != nullptr;
-  const int chunk = looped ? blockIdx.x : blockIdx.x / (BT / 4);
+  const int chunk = blockIdx.x / (BT / 4), r = (blockIdx.x % (BT / 4)) * 4 + wv, hq = blockIdx.y;
   const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
   const int bos = p.cu[n], eos = p.cu[n + 1];
-  if (looped && !p.big[(int64_t)chunk * H + blockIdx.y]) return;   // the matrix-core kernel has done this chunk
-  const int nit = looped ? BT * NG / 4 : 1;
-  for (int itx = 0; itx < nit; ++itx) {
-  if (itx) __syncthreads();   // the previous pair's vectors in LDS are no longer read
-  const int item = 4 * itx + wv;
-  const int r = looped ? item % BT : (blockIdx.x % (BT / 4)) * 4 + wv;
-  const int hq = looped ? blockIdx.y * NG + item / BT : blockIdx.y;
   const int h = hq / NG;
   const bool valid = bos + it * BT + r < eos;   // waves past the end compute on row 0 and write nothing
   const int rr = valid ? r : 0;
@@ -131,14 +119,8 @@ __global__ __launch_bounds__(256) void bwd_q_kernel(const BP p) {
     const int j = lane;
     const bool has = j <= rr && tl0 + j >= 0;
     const int64_t sj = (int64_t)bos + tl0 + j;
-    if (p.ap) {
-      const int64_t pi = (((int64_t)chunk * HQ + hq) * BT + rr) * BT + j;
-      Aj[j] = has ? bf16_to_f32(p.ap[pi]) * p.scale : 0.f;
-      Bj[j] = has ? bf16_to_f32(p.bp[pi]) : 0.f;
-    } else {
-      Aj[j] = has ? dot_row<T>(qg, kgs + (sj * H + h) * K, K) : 0.f;
-      Bj[j] = has ? dot_row<T>(dov, vv_ + (sj * H + h) * V, V) : 0.f;
-    }
+    Aj[j] = has ? dot_row<T>(qg, kgs + (sj * H + h) * K, K) : 0.f;
+    Bj[j] = has ? dot_row<T>(dov, vv_ + (sj * H + h) * V, V) : 0.f;
   }
   __syncthreads();
   const float* hk0 = p.hkc + ((int64_t)chunk * H + h) * K * M;
@@ -150,15 +132,10 @@ __global__ __launch_bounds__(256) void bwd_q_kernel(const BP p) {
   if (lane < M) {
     const int m = lane;
     float au = 0.f, ad = 0.f;
-    if (p.ust) {
-      au = p.ust[tq * M + m] * p.scale;
-      ad = p.dpst[tq * M + m];
-    } else {
 #pragma unroll 8
-      for (int kk = 0; kk < K; ++kk) au += qg[kk] * hk0[(int64_t)kk * M + m];
+    for (int kk = 0; kk < K; ++kk) au += qg[kk] * hk0[(int64_t)kk * M + m];
 #pragma unroll 8
-      for (int c = 0; c < V; ++c) ad += dov[c] * hv0t[(int64_t)c * M + m];
-    }
+    for (int c = 0; c < V; ++c) ad += dov[c] * hv0t[(int64_t)c * M + m];
     const float gm = gct[m];
     const float e = expf(gm);
     au *= e;
@@ -179,7 +156,6 @@ __global__ __launch_bounds__(256) void bwd_q_kernel(const BP p) {
     }
   }
   if (lane == 0 && valid) p.delta[tq] = delta;
-  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -310,7 +286,6 @@ __global__ __launch_bounds__(512) void bwd_intra_kernel(const BP p) {
   const int c0 = bos + it * BT;
   const int R = (eos - c0) < BT ? (eos - c0) : BT;
   const T* ss = (const T*)p.s;
-  if (p.big && !p.big[(int64_t)chunk * H + h]) return;   // the matrix-core kernel has done this chunk
   if (tid < BT) {
     const int tl = it * BT + tid - p.shift;
     src[tid] = (tid < R && tl >= 0) ? bos + tl : -1;
@@ -336,10 +311,7 @@ __global__ __launch_bounds__(512) void bwd_intra_kernel(const BP p) {
       if (i < r) continue;
       const int sj = src[r];
       float av = 0.f, bv = 0.f;
-      if (sj >= 0 && p.ap) {
-        av = bf16_to_f32(p.ap[(((int64_t)chunk * HQ + hq) * BT + i) * BT + r]);
-        bv = bf16_to_f32(p.bp[(((int64_t)chunk * HQ + hq) * BT + i) * BT + r]);
-      } else if (sj >= 0) {
+      if (sj >= 0) {
         const T* qrow = (const T*)p.q_gsa + ((int64_t)(c0 + i) * HQ + hq) * K;
         const T* krow = (const T*)p.k_gsa + ((int64_t)sj * H + h) * K;
         av = dot_rows<T>(qrow, krow, K);
@@ -550,6 +522,7 @@ __global__ __launch_bounds__(256) void bwd_state_scan_kernel(const BP p) {
   float* ebn = eb + (((int64_t)p.coff[n] * H + h) * X + x) * M + m;
   auto gl_of = [&](int it) {
     const int R = (L - it * BT) < BT ? (L - it * BT) : BT;
+    if (p.gcx) return p.gcx[(((int64_t)(p.coff[n] + it) * H + h) * BT + R - 1) * M + m];
     return p.gc[((int64_t)(bos + it * BT + R - 1) * H + h) * M + m];
   };
   int it = nchunks - 1;
@@ -717,8 +690,8 @@ __global__ __launch_bounds__(256) void bwd_gate_local_kernel(const BP p) {
           ds4.x += a.x; ds4.y += a.y; ds4.z += a.z; ds4.w += a.w;
         }
         float4 x4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int a = 0; a < NG; ++a) {
-          const float4 v = *reinterpret_cast<const float4*>(p.xg + ((int64_t)t * HQ + h * NG + a) * M + m);
+        for (int a = 0; a < p.xNG; ++a) {
+          const float4 v = *reinterpret_cast<const float4*>(p.xg + (((int64_t)t * H + h) * p.xNG + a) * M + m);
           x4.x += v.x; x4.y += v.y; x4.z += v.z; x4.w += v.w;
         }
         float sv[4];
@@ -771,7 +744,7 @@ __global__ __launch_bounds__(256) void bwd_gate_local_kernel(const BP p) {
       float dstot = p.dsi[rt];
       for (int b = 0; b < nslab; ++b) dstot += p.dsp[(int64_t)b * p.T_tot * H * M + rt];
       float x = 0.f;
-      for (int a = 0; a < NG; ++a) x += p.xg[((int64_t)t * HQ + h * NG + a) * M + m];
+      for (int a = 0; a < p.xNG; ++a) x += p.xg[(((int64_t)t * H + h) * p.xNG + a) * M + m];
       const float sval = Elem<T>::ld((const T*)p.s + ((int64_t)sj * H + h) * M + m);
       z[q] = x - sval * dstot;
       dst[q] = dstot;
@@ -984,53 +957,46 @@ __global__ __launch_bounds__(256) void bwd_kv_window_kernel(const BP p) {
 size_t aligned(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct BwdPlan {
-  size_t fwd, mfma, hkct, hvct, hkb, hvb, hkl, hvl, ap, bp, ust, dpst, big, hkT, hvT, dus, pp, xg, delta, ld, ck, cv, dsi, dsp, dvs, gtot, dks, ek, ev, total;
-  bool use_mfma;
+  size_t fwd, hkct, hvct, hkT, hvT, dus, pp, xg, delta, ld, ck, cv, dsi, dsp, dvs, gtot, dks, ek, ev, total;
+  bool use_mfma;   // the slot branch runs on the matrix cores
   int nbk, nbv;
 };
 BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f) {
-  BwdPlan s;
-  s.nbk = (a->K + CB - 1) / CB;
-  s.nbv = (a->V + CB - 1) / CB;
-  size_t off = 0;
-  s.fwd = off; off += aligned(prefill_simple_scratch_bytes(&f));
-  // bf16 shapes the matrix-core state pass covers: recompute the states with it and convert
+  BwdPlan s = {};
+  // bf16 shapes the matrix-core state pass covers
   s.use_mfma = prefill_mfma_supported(&f);
-  s.mfma = off;
-  if (s.use_mfma) off += aligned(prefill_mfma_scratch_bytes(&f));
-  s.hkct = off; off += aligned((size_t)a->NT * a->H * a->K * a->M * 4);
-  s.hvct = off; off += aligned((size_t)a->NT * a->H * a->V * a->M * 4);
-  s.hkb = s.hvb = s.hkl = s.hvl = s.ap = s.bp = s.ust = s.dpst = s.big = off;
-  if (s.use_mfma) {
-    s.hkb = off; off += aligned((size_t)a->NT * a->H * a->M * a->K * 2);
-    s.hvb = off; off += aligned((size_t)a->NT * a->H * a->M * a->V * 2);
-    s.hkl = off; off += aligned((size_t)a->NT * a->H * a->M * a->K * 2);
-    s.hvl = off; off += aligned((size_t)a->NT * a->H * a->M * a->V * 2);
-    s.ap = off; off += aligned((size_t)a->NT * a->HQ * BT * BT * 2);
-    s.bp = off; off += aligned((size_t)a->NT * a->HQ * BT * BT * 2);
-    s.ust = off; off += aligned((size_t)a->T_tot * a->HQ * a->M * 4);
-    s.dpst = off; off += aligned((size_t)a->T_tot * a->HQ * a->M * 4);
-    s.big = off; off += aligned((size_t)a->NT * a->H * 4);
+  s.nbk = s.use_mfma ? bwd_slot_inter_slabs(a) : (a->K + CB - 1) / CB;
+  s.nbv = s.use_mfma ? bwd_slot_inter_slabs(a) : (a->V + CB - 1) / CB;
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off += aligned(bytes);
+    return at;
+  };
+  const size_t states_k = (size_t)a->NT * a->H * a->K * a->M * 4, states_v = (size_t)a->NT * a->H * a->V * a->M * 4;
+  const size_t tqm = (size_t)a->T_tot * a->HQ * a->M * 4, thm = (size_t)a->T_tot * a->H * a->M * 4;
+  s.fwd = take(s.use_mfma ? prefill_mfma_scratch_bytes(&f) : prefill_simple_scratch_bytes(&f));
+  s.hkT = take((size_t)a->N * a->H * a->K * a->M * 4);
+  s.hvT = take((size_t)a->N * a->H * a->M * a->V * 4);
+  if (!s.use_mfma) {
+    s.hkct = take(states_k);
+    s.hvct = take(states_v);
+    s.dus = take(tqm);
+    s.pp = take(tqm);
+    const size_t cc = (size_t)a->NT * a->HQ * BT * BT * 4;
+    s.ck = take(cc);
+    s.cv = take(cc);
   }
-  s.hkT = off; off += aligned((size_t)a->N * a->H * a->K * a->M * 4);
-  s.hvT = off; off += aligned((size_t)a->N * a->H * a->M * a->V * 4);
-  const size_t tqm = aligned((size_t)a->T_tot * a->HQ * a->M * 4);
-  s.dus = off; off += tqm;
-  s.pp = off; off += tqm;
-  s.xg = off; off += tqm;
-  s.delta = off; off += aligned((size_t)a->T_tot * a->HQ * 4);
-  s.ld = off; off += aligned((size_t)a->T_tot * a->HQ * 8);   // (-lse / scale, -delta) pairs of the LDS-direct window kernels
-  const size_t cc = aligned((size_t)a->NT * a->HQ * BT * BT * 4);
-  s.ck = off; off += cc;
-  s.cv = off; off += cc;
-  const size_t thm = (size_t)a->T_tot * a->H * a->M * 4;
-  s.dsi = off; off += aligned(thm);
-  s.dsp = off; off += aligned(thm * (s.nbk + s.nbv));
-  s.dvs = off; off += aligned((size_t)a->T_tot * a->H * a->V * 4);
-  s.gtot = off; off += aligned((size_t)a->NT * a->H * a->M * 4);
-  s.dks = off; off += aligned((size_t)a->T_tot * a->H * a->K * 4);
-  s.ek = off; off += aligned((size_t)a->NT * a->H * a->K * a->M * 4);
-  s.ev = off; off += aligned((size_t)a->NT * a->H * a->V * a->M * 4);
+  s.xg = take(s.use_mfma ? thm : tqm);
+  s.delta = take((size_t)a->T_tot * a->HQ * 4);
+  s.ld = take((size_t)a->T_tot * a->HQ * 8);   // (-lse / scale, -delta) pairs of the LDS-direct window kernels
+  s.dsi = take(thm);
+  s.dsp = take(thm * (s.nbk + s.nbv));
+  s.dvs = take((size_t)a->T_tot * a->H * a->V * 4);
+  s.gtot = take((size_t)a->NT * a->H * a->M * 4);
+  s.dks = take((size_t)a->T_tot * a->H * a->K * 4);
+  s.ek = take(states_k);
+  s.ev = take(states_v);
   s.total = off;
   return s;
 }
@@ -1061,26 +1027,17 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
   float* hkc = (float*)fs;
   fs += aligned((size_t)a->NT * a->H * a->K * a->M * 4);
   float* hvc = (float*)fs;
-#ifdef NHA_AB_SWITCHES   // measurement builds only (-DNHA_AB_SWITCHES)
-  static const bool intra_mfma = getenv("NHA_BWD_INTRA_VALU") == nullptr;
-#else
-  constexpr bool intra_mfma = true;
-#endif
   int rc;
+  mf::MP states;
+  f.scratch = sc + sp.fwd;
   if (sp.use_mfma) {
     f.impl = NHA_IMPL_MFMA;
-    f.scratch = sc + sp.mfma;
     f.scratch_bytes = prefill_mfma_scratch_bytes(&f);
-    // state pass (segment form) and its export; every consumer of the states on this path reads
-    // the bf16 copies
-    rc = prefill_mfma_export_states(&f, gc, nullptr, nullptr, nullptr, sc + sp.hkb, sc + sp.hvb, sc + sp.hkl, sc + sp.hvl, (int*)(sc + sp.big));
-    // the decay-free products of the slot branch on the matrix cores
-    // (with the decay-coupled terms on the matrix cores too, the per-token stage rides along)
-    if (rc == NHA_OK) rc = bwd_slot_products(a, sc + sp.hkb, sc + sp.hvb, sc + sp.hkl, sc + sp.hvl, (bf16_t*)(sc + sp.ap), (bf16_t*)(sc + sp.bp), (float*)(sc + sp.ust), (float*)(sc + sp.dpst),
-                                             (float*)(sc + sp.delta), intra_mfma ? (const int*)(sc + sp.big) : nullptr, gc,
-                                             (float*)(sc + sp.dus), (float*)(sc + sp.pp), (float*)(sc + sp.xg));
+    rc = prefill_mfma_segment_states(&f, &states);
+    if (rc == NHA_OK)
+      rc = bwd_slot_branch(a, states, (float*)(sc + sp.delta), (float*)(sc + sp.xg), (float*)(sc + sp.dsi), (float*)(sc + sp.ek),
+                           (float*)(sc + sp.ev), (float*)(sc + sp.dks), (float*)(sc + sp.dvs));
   } else {
-    f.scratch = sc + sp.fwd;
     f.scratch_bytes = prefill_simple_scratch_bytes(&f);
     rc = prefill_simple_impl(&f, 1);   // the state pass only
   }
@@ -1096,14 +1053,8 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
   p.cu = a->cu_seqlens; p.cidx = a->chunk_indices; p.coff = a->chunk_offsets;
   p.gc = gc; p.hkc = hkc; p.hvc = hvc;
   p.hkct = (float*)(sc + sp.hkct); p.hvct = (float*)(sc + sp.hvct);
-  p.ap = p.bp = nullptr;
-  p.ust = p.dpst = nullptr;
-  p.big = nullptr;
-  if (sp.use_mfma) {
-    if (intra_mfma) p.big = (const int*)(sc + sp.big);
-    p.ap = (const bf16_t*)(sc + sp.ap); p.bp = (const bf16_t*)(sc + sp.bp);
-    p.ust = (float*)(sc + sp.ust); p.dpst = (float*)(sc + sp.dpst);
-  }
+  p.gcx = sp.use_mfma ? states.gc : nullptr;
+  p.xNG = sp.use_mfma ? 1 : a->HQ / a->H;
   p.hkT = (float*)(sc + sp.hkT); p.hvT = (float*)(sc + sp.hvT);
   p.dus = (float*)(sc + sp.dus); p.pp = (float*)(sc + sp.pp); p.xg = (float*)(sc + sp.xg);
   p.delta = (float*)(sc + sp.delta);
@@ -1133,13 +1084,11 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
     configured = true;
   }
   const bool wmfma = bwd_window_mfma_supported(a);
-  if (!sp.use_mfma) hipLaunchKernelGGL(bwd_transpose_states_kernel, dim3(a->NT * a->H), dim3(256), 0, st, p);
-  if (sp.use_mfma && intra_mfma && !bwd_slot_products_fuses_q(a)) {
-    rc = bwd_slot_products3(a, 0, p.big, p.ap, p.bp, p.ust, p.dpst, p.gc, p.delta, p.dus, p.pp, p.xg, p.ck, p.cv, p.dsi);
-    if (rc != NHA_OK) return rc;
+  if (!sp.use_mfma) {
+    hipLaunchKernelGGL(bwd_transpose_states_kernel, dim3(a->NT * a->H), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((bwd_q_kernel<T>), dim3(a->NT * (BT / 4), a->HQ), dim3(256), lds_q, st, p);
+    NHA_CHECK_LAUNCH("nha_prefill_bwd(query pass)");
   }
-  hipLaunchKernelGGL((bwd_q_kernel<T>), p.big ? dim3(a->NT, a->H) : dim3(a->NT * (BT / 4), a->HQ), dim3(256), lds_q, st, p);
-  NHA_CHECK_LAUNCH("nha_prefill_bwd(query pass)");
   if (wmfma) {
     rc = bwd_window_mfma_dq(a, p.delta, sc + sp.ld);
     if (rc != NHA_OK) return rc;
@@ -1147,31 +1096,17 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
     hipLaunchKernelGGL((bwd_q_window_kernel<T>), dim3(a->NT * BT, a->HQ), dim3(256), lds_qw, st, p);
     NHA_CHECK_LAUNCH("nha_prefill_bwd(window query pass)");
   }
-  if (sp.use_mfma && intra_mfma) {
-    rc = bwd_slot_products3(a, 1, p.big, p.ap, p.bp, p.ust, p.dpst, p.gc, p.delta, p.dus, p.pp, p.xg, p.ck, p.cv, p.dsi);
-    if (rc != NHA_OK) return rc;
-  }
-  hipLaunchKernelGGL((bwd_intra_kernel<T>), dim3(a->NT, a->H), dim3(512), lds_i, st, p);
-  NHA_CHECK_LAUNCH("nha_prefill_bwd(intra-chunk pass)");
-  if (sp.use_mfma) {
-    rc = bwd_slot_products2(a, 0, sc + sp.hkb, p.dus, p.pp, p.ck, p.cv, p.gc, p.ek, p.ev, p.dks, p.dvs, p.dsp);
-    if (rc != NHA_OK) return rc;
-  } else {
+  const int nbmax = sp.nbk > sp.nbv ? sp.nbk : sp.nbv;
+  if (!sp.use_mfma) {
+    hipLaunchKernelGGL((bwd_intra_kernel<T>), dim3(a->NT, a->H), dim3(512), lds_i, st, p);
+    NHA_CHECK_LAUNCH("nha_prefill_bwd(intra-chunk pass)");
     hipLaunchKernelGGL((bwd_dqg_kernel<T>), dim3(a->NT * (BT / 4), a->HQ), dim3(256), (size_t)4 * (M + BT) * 4, st, p);
     NHA_CHECK_LAUNCH("nha_prefill_bwd(dq_gsa pass)");
-  }
-  const int nbmax = sp.nbk > sp.nbv ? sp.nbk : sp.nbv;
-  if (sp.use_mfma) {
-    rc = bwd_slot_products2(a, 1, sc + sp.hkb, p.dus, p.pp, p.ck, p.cv, p.gc, p.ek, p.ev, p.dks, p.dvs, p.dsp);
-    if (rc != NHA_OK) return rc;
-  } else {
     hipLaunchKernelGGL((bwd_state_direct_kernel<T>), dim3(a->NT, a->H * nbmax, 2), dim3(256), lds_s1, st, p);
   }
   hipLaunchKernelGGL(bwd_state_scan_kernel, dim3(a->N * a->H, ((K + V) * M + 255) / 256), dim3(256), 0, st, p);
   if (sp.use_mfma) {
-    // one partial-ds slab per state and column range of a workgroup instead of one per 32-column block
-    p.nbk = p.nbv = bwd_slot_inter_slabs(a);
-    rc = bwd_slot_products2(a, 2, sc + sp.hkb, p.dus, p.pp, p.ck, p.cv, p.gc, p.ek, p.ev, p.dks, p.dvs, p.dsp);
+    rc = bwd_slot_inter(a, states.gc, p.ek, p.ev, p.dks, p.dvs, p.dsp);
     if (rc != NHA_OK) return rc;
   } else {
     hipLaunchKernelGGL((bwd_state_inter_kernel<T>), dim3(a->NT, a->H * nbmax, 2), dim3(256), lds_s3, st, p);

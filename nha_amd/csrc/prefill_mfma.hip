@@ -1258,79 +1258,6 @@ int launch_repair(const MP& p, hipStream_t st) {
   return NHA_OK;
 }
 
-// ==========================================================================================
-// fp32 copies of what the state pass left in the scratch for the backward pass: true chunk-start
-// states as hk [K][M] and transposed hk^T [M][K], hv^T [V][M], plus bf16 copies hk^T [M][K] and
-// hv [M][V] as matrix-core operands; gate cumsums per row token
-// ==========================================================================================
-template <int D>
-__global__ __launch_bounds__(256) void export_states_kernel(const MP p, float* gc, float* hkc, float* hkct, float* hvct, bf16_t* hkb, bf16_t* hvb, bf16_t* hkl,
-                                                          bf16_t* hvl, int* big) {
-  const int chunk = blockIdx.x, h = blockIdx.y, H = p.H;
-  const int tid = threadIdx.x;
-  const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
-  const int bos = p.cu[n], eos = p.cu[n + 1];
-  const int c0 = bos + it * BT;
-  const int R = (eos - c0) < BT ? (eos - c0) : BT;
-  const int64_t cg = (int64_t)chunk * H + h;
-  const int64_t sl = (int64_t)seg_slot(p.coff, n, it) * H + h;
-  // eight consecutive d of one slot per thread and trip: 16-byte reads of the bf16 local states, 32-byte
-  // reads of the fp32 segment states, 16-byte writes of the four bf16 copies
-  for (int e8 = tid; e8 < MS * D / 8; e8 += 256) {
-    const int m = e8 / (D / 8), d = (e8 % (D / 8)) * 8;
-    const float dc = p.dcum[cg * MS + m];
-    const int64_t li = (cg * MS + m) * D + d, si = (sl * MS + m) * D + d;
-    float lk[8], lv[8], sk[8], sv[8], hk[8], hv[8];
-    Elem<bf16_t>::ld8(p.hkT + li, lk);
-    Elem<bf16_t>::ld8(p.hvc + li, lv);
-    Elem<float>::ld8(p.hseg_k + si, sk);
-    Elem<float>::ld8(p.hseg_v + si, sv);
-    uint32_t kh[4], vh[4], kl[4], vl[4];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      hk[j] = lk[j] + sk[j] * dc;
-      hv[j] = lv[j] + sv[j] * dc;
-    }
-    // bf16 pairs hi + lo: the backward multiplies by hi and by lo
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bf16_t k0 = f32_to_bf16(hk[2 * j]), k1 = f32_to_bf16(hk[2 * j + 1]);
-      const bf16_t v0 = f32_to_bf16(hv[2 * j]), v1 = f32_to_bf16(hv[2 * j + 1]);
-      kh[j] = (uint32_t)k0 | ((uint32_t)k1 << 16);
-      vh[j] = (uint32_t)v0 | ((uint32_t)v1 << 16);
-      kl[j] = (uint32_t)f32_to_bf16(hk[2 * j] - bf16_to_f32(k0)) | ((uint32_t)f32_to_bf16(hk[2 * j + 1] - bf16_to_f32(k1)) << 16);
-      vl[j] = (uint32_t)f32_to_bf16(hv[2 * j] - bf16_to_f32(v0)) | ((uint32_t)f32_to_bf16(hv[2 * j + 1] - bf16_to_f32(v1)) << 16);
-    }
-    *reinterpret_cast<uint4*>(hkb + li) = make_uint4(kh[0], kh[1], kh[2], kh[3]);
-    *reinterpret_cast<uint4*>(hvb + li) = make_uint4(vh[0], vh[1], vh[2], vh[3]);
-    *reinterpret_cast<uint4*>(hkl + li) = make_uint4(kl[0], kl[1], kl[2], kl[3]);
-    *reinterpret_cast<uint4*>(hvl + li) = make_uint4(vl[0], vl[1], vl[2], vl[3]);
-    if (hkc) {   // fp32 copies: only the VALU kernels of the backward read them
-      Elem<float>::st8(hkct + li, hk);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        hkc[(cg * D + d + j) * MS + m] = hk[j];
-        hvct[(cg * D + d + j) * MS + m] = hv[j];
-      }
-    }
-  }
-  for (int e4 = tid; e4 < R * MS / 4; e4 += 256) {
-    const int r = e4 / (MS / 4), m4 = (e4 % (MS / 4)) * 4;
-    *reinterpret_cast<float4*>(gc + ((int64_t)(c0 + r) * H + h) * MS + m4) = *reinterpret_cast<const float4*>(p.gc + cg * BT * MS + r * MS + m4);
-  }
-  // chunks in which some slot decays by more than e^-BWD_DECAY_CLAMP over one of the two 32-row halves: the
-  // backward's factored products (e^(gc_i - ref) e^(ref - gc_j) as two operands, ref = the start of
-  // j's half) leave the bf16 / fp32 range there.  One slot per lane of the first wave.
-  if (tid < 64) {
-    const float* g = p.gc + cg * BT * MS;
-    const int m = tid;
-    const float g31 = g[(R > 32 ? 31 : R - 1) * MS + m];
-    const bool b = (g31 < -BWD_DECAY_CLAMP) | (g[(R - 1) * MS + m] - g31 < -BWD_DECAY_CLAMP);
-    const bool any = __any(b);
-    if (tid == 0) big[cg] = any ? 1 : 0;
-  }
-}
-
 template <int D, int G, int NW, int TK>
 int launch_out(const MP& p, hipStream_t st) {
   static std::once_flag once;
@@ -1490,26 +1417,16 @@ int prefill_mfma_impl(const NhaPrefillArgs* a, int phase) {
   return run_mfma<256>(p, phase, st);
 }
 
-// Runs the state pass of `a` in the segment form and exports it; gc [T_tot][H][M], hkc
-// [NT][H][K][M], hkct [NT][H][M][K], hvct [NT][H][V][M] receive fp32 copies, hkb [NT][H][M][K] and
-// hvb [NT][H][M][V] bf16 copies with their low parts hkl, hvl (hkc, hkct, hvct may be NULL together), big [NT][H] the flag of
-// chunks with a decay beyond e^-80
-int prefill_mfma_export_states(const NhaPrefillArgs* a, float* gc, float* hkc, float* hkct, float* hvct, void* hkb, void* hvb,
-                               void* hkl, void* hvl, int* big) {
-  const MP p = make_mp(a);
+// The state pass of `a` in the segment form (the backward's): `out` receives the parameter block whose tables it filled --
+// segment-local chunk-start states, segment-start states, decays and gate cumsums.
+int prefill_mfma_segment_states(const NhaPrefillArgs* a, MP* out) {
+  const MP p = *out = make_mp(a);
   hipStream_t st = (hipStream_t)a->stream;
   if (p.NT > 65535) {
     set_error("nha_prefill_bwd(mfma): more than 65535 chunks (%d) in one call", p.NT);
     return NHA_ERR_UNSUPPORTED;
   }
-  const int rcs = a->K == 64 ? run_state_pass<64>(p, true, st) : a->K == 128 ? run_state_pass<128>(p, true, st) : run_state_pass<256>(p, true, st);
-  if (rcs != NHA_OK) return rcs;
-  const dim3 grid(a->NT, a->H);
-  if (a->K == 64) hipLaunchKernelGGL((export_states_kernel<64>), grid, dim3(256), 0, st, p, gc, hkc, hkct, hvct, (bf16_t*)hkb, (bf16_t*)hvb, (bf16_t*)hkl, (bf16_t*)hvl, big);
-  else if (a->K == 128) hipLaunchKernelGGL((export_states_kernel<128>), grid, dim3(256), 0, st, p, gc, hkc, hkct, hvct, (bf16_t*)hkb, (bf16_t*)hvb, (bf16_t*)hkl, (bf16_t*)hvl, big);
-  else hipLaunchKernelGGL((export_states_kernel<256>), grid, dim3(256), 0, st, p, gc, hkc, hkct, hvct, (bf16_t*)hkb, (bf16_t*)hvb, (bf16_t*)hkl, (bf16_t*)hvl, big);
-  NHA_CHECK_LAUNCH("nha_prefill_bwd(state export)");
-  return NHA_OK;
+  return a->K == 64 ? run_state_pass<64>(p, true, st) : a->K == 128 ? run_state_pass<128>(p, true, st) : run_state_pass<256>(p, true, st);
 }
 
 }  // namespace nha

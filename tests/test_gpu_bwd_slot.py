@@ -1,0 +1,36 @@
+"""The one-launch slot branch of the bf16 backward (prefill_bwd_slot.hip) against reverse-mode differentiation of the fp64
+recurrence, at the places where its tiling can go wrong.
+
+Tolerances are those of test_gpu_prefill_bwd.py: o, do and the gradients are bf16 (2^-9 = 2e-3 per rounding), and a gradient
+sums products of two or three such roundings with independent signs, so 1e-2 in relative L2; tables made from fp32
+intermediates are kept to 16 bits of mantissa and add nothing to that."""
+import pytest
+import torch
+
+from tests.test_gpu_prefill_bwd import BF, run_bwd_case
+from tests.util import prefill_inputs
+
+pytestmark = pytest.mark.gpu
+
+# one row, the last row of the first half, the first of the second, a whole chunk, one row of a second chunk, three chunks
+CU = [0, 1, 33, 66, 130, 195, 340]
+
+
+@pytest.mark.parametrize("shift", [0, 32, 70])
+@pytest.mark.parametrize("NG", [1, 3])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_slot_branch_edges(D, NG, shift):
+    """Ragged chunks, one and several query heads per kv-head, sequences shorter than the shift, a shift past a chunk."""
+    H = 2
+    d = prefill_inputs(8100 + D + NG + shift, 1, CU[-1], H * NG, H, D, D, 64, dtype=BF, qk_scale=D ** -0.5, with_state=True, N=len(CU) - 1)
+    run_bwd_case(f"slot D{D} NG{NG} shift{shift}", d, wl=40, shift=shift, dtype=BF, cu=CU, with_dht=True)
+
+
+@pytest.mark.parametrize("gate_mean", [-2.0, -5.0])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_slot_branch_strong_gates(D, gate_mean):
+    """Chunks whose decay leaves the factored form's range (about e^-70 within a half at -2: some chunks; all at -5) are
+    taken by the launch that forms the decay pair by pair; the LSE's own cotangent included."""
+    d = prefill_inputs(8200 + D, 1, CU[-1], 4, 2, D, D, 64, dtype=BF, qk_scale=D ** -0.5, gate_div=1.0, gate_mean=gate_mean,
+                       with_state=True, N=len(CU) - 1)
+    run_bwd_case(f"slot strong {gate_mean} D{D}", d, wl=40, shift=0, dtype=BF, cu=CU, with_lse=True)
