@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define NHA_ABI_VERSION 10
+#define NHA_ABI_VERSION 11
 
 enum { NHA_DTYPE_F32 = 0, NHA_DTYPE_BF16 = 1 };
 enum {
@@ -236,6 +236,28 @@ size_t nha_decode_scratch_bytes(void);
 int nha_decode_step(const NhaDecodeArgs* a);
 /* count[b] += 1 for b < B (ring mode bookkeeping between steps). */
 int nha_decode_advance(int32_t* count, int32_t B, void* stream);
+
+/* Hand-over of prompts to decode rings, one launch: ring slot r of sequence n takes the newest token j of the sequence
+ * with j % W == r, or zeros where there is none; count[n] is the sequence's length; the states are copied.
+ * src[x]: rows of row_bytes[x] bytes, one per token of the packed sequences; ring[x]: [N][W] rows.  x = 0..3: window
+ * keys, slot keys, values, log gates.  state[x], state_out[x]: state_bytes[x] bytes per sequence (may be 0).
+ * cu_seqlens [N+1] on the device, or NULL for N sequences of T tokens.  Sources, destinations and byte counts are
+ * multiples of 16. */
+typedef struct NhaRingFillArgs {
+  const void* src[4];
+  void* ring[4];
+  int32_t row_bytes[4];
+  const void* state[2];
+  void* state_out[2];
+  int64_t state_bytes[2];
+  const int32_t* cu_seqlens;
+  int32_t* count;
+  int64_t tokens;   /* rows of every src: a boundary past them leaves its slots zero */
+  int32_t N, T, W;
+  void* stream;
+} NhaRingFillArgs;
+
+int nha_ring_fill(const NhaRingFillArgs* a);
 
 /* ------------------------------------------------------------------------------------------
  * Varlen chunk tables (HOST pointers, pure integer, no GPU).  Replaces fla's

@@ -15,7 +15,7 @@ NHA_DTYPE_F32, NHA_DTYPE_BF16 = 0, 1
 NHA_IMPL_AUTO, NHA_IMPL_SIMPLE, NHA_IMPL_MFMA = 0, 1, 2
 NHA_DECODE_WINDOW, NHA_DECODE_LOGITS, NHA_DECODE_RING = 0, 1, 2
 NHA_OK, NHA_ERR_INVALID, NHA_ERR_UNSUPPORTED, NHA_ERR_SCRATCH, NHA_ERR_LAUNCH = 0, -1, -2, -3, -4
-ABI_VERSION = 10
+ABI_VERSION = 11
 NHA_NOALLOC_SCRATCH_BYTES = 32 << 20   # workspace of nha_prefill_fwd_noalloc (include/nha_hip.h)
 NHA_FMAP_NONE, NHA_FMAP_SWISH, NHA_FMAP_RELU = 0, 1, 2
 
@@ -164,6 +164,15 @@ class NhaShortConvBwdArgs(C.Structure):
     ]
 
 
+class NhaRingFillArgs(C.Structure):
+    _fields_ = [
+        ("src", C.c_void_p * 4), ("ring", C.c_void_p * 4), ("row_bytes", C.c_int32 * 4),
+        ("state", C.c_void_p * 2), ("state_out", C.c_void_p * 2), ("state_bytes", C.c_int64 * 2),
+        ("cu_seqlens", C.c_void_p), ("count", C.c_void_p), ("tokens", C.c_int64), ("N", C.c_int32), ("T", C.c_int32), ("W", C.c_int32),
+        ("stream", C.c_void_p),
+    ]
+
+
 _PACK_CODES = {C.c_int32: "i", C.c_int64: "q", C.c_float: "f", C.c_void_p: "P", C.c_size_t: "N"}
 
 
@@ -215,6 +224,8 @@ def load() -> C.CDLL:
     lib.decode_step_packed = C.CFUNCTYPE(C.c_int, C.c_char_p)(("nha_decode_step", lib))
     lib.nha_decode_advance.restype = C.c_int
     lib.nha_decode_advance.argtypes = [C.c_void_p, C.c_int32, C.c_void_p]
+    lib.nha_ring_fill.restype = C.c_int
+    lib.nha_ring_fill.argtypes = [C.POINTER(NhaRingFillArgs)]
     lib.nha_layer_prologue.restype = C.c_int
     lib.nha_layer_prologue.argtypes = [C.POINTER(NhaLayerPrologueArgs)]
     lib.nha_layer_epilogue.restype = C.c_int

@@ -199,6 +199,23 @@ int nha_decode_step(const NhaDecodeArgs* a) { return decode_step_impl(a); }
 
 int nha_decode_advance(int32_t* count, int32_t B, void* stream) { return decode_advance_impl(count, B, stream); }
 
+int nha_ring_fill(const NhaRingFillArgs* a) {
+  NHA_CHECK_ARG(a != nullptr, "nha_ring_fill: null args");
+  NHA_CHECK_ARG(a->N > 0 && a->N <= 65535 && a->T >= 0 && a->W > 0 && a->W <= (1 << 30), "nha_ring_fill: bad dimension");
+  NHA_CHECK_ARG(a->count != nullptr, "nha_ring_fill: count is required");
+  uintptr_t all = 0;
+  for (int x = 0; x < 4; ++x) {
+    NHA_CHECK_ARG(a->src[x] && a->ring[x] && a->row_bytes[x] > 0, "nha_ring_fill: rows, rings and row sizes are required");
+    all |= reinterpret_cast<uintptr_t>(a->src[x]) | reinterpret_cast<uintptr_t>(a->ring[x]) | (uintptr_t)a->row_bytes[x];
+  }
+  for (int x = 0; x < 2; ++x) {
+    NHA_CHECK_ARG(a->state_bytes[x] == 0 || (a->state_bytes[x] > 0 && a->state[x] && a->state_out[x]), "nha_ring_fill: bad state");
+    all |= reinterpret_cast<uintptr_t>(a->state[x]) | reinterpret_cast<uintptr_t>(a->state_out[x]) | (uintptr_t)a->state_bytes[x];
+  }
+  NHA_CHECK_ARG((all & 15) == 0, "nha_ring_fill: addresses and sizes must be multiples of 16 bytes");
+  return ring_fill_impl(a);
+}
+
 int nha_layer_prologue(const NhaLayerPrologueArgs* a) {
   NHA_CHECK_ARG(a != nullptr, "nha_layer_prologue: null args");
   NHA_CHECK_ARG(a->T_tot > 0 && a->N > 0 && a->HQ > 0 && a->H > 0 && a->K > 0 && a->V > 0 && a->M > 0,

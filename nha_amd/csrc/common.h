@@ -141,6 +141,7 @@ int short_conv_bwd_parts(int T_tot);
 int short_conv_bwd_impl(const NhaShortConvBwdArgs* a);
 int decode_step_impl(const NhaDecodeArgs* a);
 int decode_advance_impl(int32_t* count, int32_t B, void* stream);
+int ring_fill_impl(const NhaRingFillArgs* a);
 bool decode_mfma_supported(const NhaDecodeArgs* a);
 int decode_mfma_impl(const NhaDecodeArgs* a);
 // decode_split.hip: the calls of decode_mfma_impl with too few (sequence, kv-head) pairs to fill the chip

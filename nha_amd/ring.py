@@ -6,6 +6,7 @@ reference (nha_fla/models/nha_cache.py:105-131, :143-154; models/qwen3_moe_nha/q
 slot and attends over the valid entries, reading state and window once per kv-head."""
 from __future__ import annotations
 
+import ctypes as C
 from dataclasses import dataclass
 from typing import Optional
 
@@ -54,18 +55,21 @@ class NHARingState:
         dev, W = k_swa.device, int(window)
         B, T, H, K = k_swa.shape
         V, M = v.shape[-1], g.shape[-1]
+        hk, hv = final_state
+        if cu_seqlens is not None and B != 1:
+            raise ValueError("cu_seqlens needs the packed layout [1, T_tot, ...]")
+        N = B if cu_seqlens is None else cu_seqlens.numel() - 1
+        if tuple(hk.shape) != (N, H, K, M) or tuple(hv.shape) != (N, H, M, V):
+            raise ValueError(f"final_state must be ([{N},{H},{K},{M}], [{N},{H},{M},{V}]), got {tuple(hk.shape)}, {tuple(hv.shape)}")
+        st = cls._fill((k_swa, k_gsa, v, g), hk, hv, W, cu_seqlens, N, T)
+        if st is not None:
+            return st
         if cu_seqlens is None:
             starts = torch.arange(B, device=dev, dtype=torch.long) * T
             lens = torch.full((B,), T, device=dev, dtype=torch.long)
         else:
-            if B != 1:
-                raise ValueError("cu_seqlens needs the packed layout [1, T_tot, ...]")
             cu = cu_seqlens.to(device=dev, dtype=torch.long)
             starts, lens = cu[:-1], cu[1:] - cu[:-1]
-        N = starts.numel()
-        hk, hv = final_state
-        if tuple(hk.shape) != (N, H, K, M) or tuple(hv.shape) != (N, H, M, V):
-            raise ValueError(f"final_state must be ([{N},{H},{K},{M}], [{N},{H},{M},{V}]), got {tuple(hk.shape)}, {tuple(hv.shape)}")
         r = torch.arange(W, device=dev, dtype=torch.long)
         last = (lens - 1)[:, None]
         tok = last - torch.remainder(last - r[None, :], W)            # newest token j <= L-1 with j % W == r
@@ -78,6 +82,35 @@ class NHARingState:
 
         return cls(hk.to(torch.float32).clone(), hv.to(torch.float32).clone(), gather(k_swa), gather(k_gsa), gather(v),
                    gather(g), lens.to(torch.int32))
+
+    @classmethod
+    def _fill(cls, rows, hk, hv, W: int, cu_seqlens, N: int, T: int) -> Optional["NHARingState"]:
+        """The hand-over in one launch, or None for what the kernel does not move: rows, states or addresses that are
+        not whole 16-byte pieces, states that are not fp32, tensors with a gradient to carry or on several devices."""
+        dev = rows[0].device
+        ts = (*rows, hk, hv)
+        if (torch.compiler.is_compiling() or N < 1 or N > 65535 or W < 1
+                or any(x.dim() != 4 or x.shape[:2] != rows[0].shape[:2] or x.numel() == 0 for x in rows)
+                or any(x.device != dev for x in ts) or dev.index != torch.cuda.current_device() or (torch.is_grad_enabled() and any(x.requires_grad for x in ts))
+                or hk.dtype != torch.float32 or hv.dtype != torch.float32):
+            return None
+        rows, states = [x.contiguous() for x in rows], [hk.contiguous(), hv.contiguous()]
+        rings = [x.new_empty(N, W, *x.shape[2:]) for x in rows]
+        out = [torch.empty_like(x) for x in states]
+        count = torch.empty(N, dtype=torch.int32, device=dev)
+        cu = None if cu_seqlens is None else cu_seqlens.to(device=dev, dtype=torch.int32).contiguous()
+        sizes = [x.shape[2] * x.shape[3] * x.element_size() for x in rows]
+        state_sizes = [x.numel() // N * 4 for x in states]
+        if any(b % 16 for b in (*sizes, *state_sizes)) or any(x.data_ptr() % 16 for x in (*rows, *states)):
+            return None
+        a = _lib.NhaRingFillArgs()
+        for x in range(4):
+            a.src[x], a.ring[x], a.row_bytes[x] = rows[x].data_ptr(), rings[x].data_ptr(), sizes[x]
+        for x in range(2):
+            a.state[x], a.state_out[x], a.state_bytes[x] = states[x].data_ptr(), out[x].data_ptr(), state_sizes[x]
+        a.cu_seqlens, a.count, a.N, a.T, a.tokens, a.W, a.stream = _ptr(cu), count.data_ptr(), N, T, rows[0].shape[0] * T, W, _stream(dev)
+        _lib.check(_lib.load().nha_ring_fill(C.byref(a)))
+        return cls(*out, *rings, count)
 
     @property
     def window(self) -> int:
