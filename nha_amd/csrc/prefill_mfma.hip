@@ -554,28 +554,32 @@ __global__ __launch_bounds__(256) void state_apply_kernel(const MP p) {
 // ==========================================================================================
 // One workgroup = one 64-row chunk x G query heads of one kv-head; its NW waves split the
 // 64 x G query rows into RQB blocks of 16 rows per wave.  Window K/V stream through four LDS
-// buffers of TK keys (two K, two V, double buffered); TK = 64 for D <= 128, 32 for D = 256.
+// buffers of TK keys (two K, two V, double buffered); TK = 64 for G > 1 at D <= 128, else 32.
 // The slot branch runs first on the same buffers: its four 64-row operand tiles (transposed
 // chunk-start k-state, k_gsa rows, chunk-start v-state, v rows) fit at once when TK = 64 and
 // in two stages when TK = 32.  The decay factors s_j[m] exp(gr[m] - gc_j[m]) that every wave
-// needs are computed once per workgroup into LDS, already in MFMA fragment order.
+// needs are computed once per workgroup into LDS, already in MFMA fragment order (G > 1).
 
-template <int D, int TK>
+// With one head per workgroup every wave owns one sub-block of query rows and no fragment is used by two waves: each
+// forms its own in registers, and the 44 KB that hold them otherwise let a second workgroup onto the CU.
+template <int D, int TK, int G>
 struct OutSmem {
   static constexpr int LDT = D + 16;
   static constexpr size_t tile_bytes = (size_t)TK * LDT * 2;
   static constexpr size_t bytes =
-      4 * tile_bytes + (size_t)BT * GLD * 4 + (size_t)BT * SLD * 2 + (size_t)(NSEA + NSEB) * 512 * 2;
+      4 * tile_bytes + (size_t)BT * GLD * 4 + (size_t)BT * SLD * 2 + (G > 1 ? (size_t)(NSEA + NSEB) * 512 * 2 : 0);
 };
 
 
 template <int D, int G, int NW, int TK>
-__global__ __launch_bounds__(64 * NW, 1) void mfma_out_kernel(const MP p) {
+__global__ __launch_bounds__(64 * NW, G == 1 ? 2 : 1) void mfma_out_kernel(const MP p) {
   constexpr int NTHR = 64 * NW;      // threads per workgroup
   constexpr int WPU = NW / G;        // waves per (chunk, head)
   constexpr int RQB = 4 / WPU;       // 16-row query blocks per wave
   static_assert(WPU >= 1 && WPU <= 4 && RQB * WPU == 4, "bad wave split");
   static_assert(TK == 64 || TK == 32, "bad tile size");
+  constexpr bool OWN = G == 1;       // decay fragments formed by the wave that uses them
+  static_assert(!OWN || RQB == 1, "a wave's own fragments serve one sub-block");
   constexpr int KS = D / 32;
   constexpr int DB = D / 16;
   constexpr int LDT = D + 16;
@@ -742,54 +746,62 @@ __global__ __launch_bounds__(64 * NW, 1) void mfma_out_kernel(const MP p) {
   // j of earlier sub-blocks, and bounded by the sub-block's own decay for its diagonal rows.
   // All LDS reads of an item are issued before the first exponential waits for one: read one at a
   // time, the 8 values of an item cost 24 LDS latencies in sequence.
-  for (int item = tid; item < (NSEA + NSEB) * 64; item += NTHR) {
-    const int f = item >> 6, ln = item & 63;
-    const int fl16 = ln & 15, fkb = ln >> 4;
-    bf16x8 out;
-    if (f < NSEA) {
-      const int Q = f < 4 ? 0 : f < 8 ? 1 : f < 16 ? 2 : 3;
-      const int rem = f - sea_base(Q);
-      const int pr = rem >> 2, mb = rem & 3;
-      const int m = 16 * mb + fl16;
-      const float gr = Q > 0 ? gcR[(16 * Q - 1) * GLD + m] : 0.f;
-      float gv[8];
-      bf16_t sv[8];
+  // sea_item: s_j[m] exp(gr[m] - gc_j[m]) with a slot per lane (rows j of blocks 2 pr and 2 pr + 1, slots of block mb)
+  auto sea_item = [&](int Q, int pr, int mb, int fl16, int fkb) {
+    const int m = 16 * mb + fl16;
+    const float gr = Q > 0 ? gcR[(16 * Q - 1) * GLD + m] : 0.f;
+    float gv[8];
+    bf16_t sv[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int j = 16 * (2 * pr + (e >> 2)) + 4 * fkb + (e & 3);   // j < 64 for every fragment
-        gv[e] = gcR[j * GLD + m];
-        sv[e] = sR[j * SLD + m];
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int jb = 2 * pr + (e >> 2);
-        const float val = bf16_to_f32(sv[e]) * fexp(fminf(gr - gv[e], DECAY_CLAMP));
-        out[e] = (__bf16)(jb <= Q ? val : 0.f);
-      }
-      *reinterpret_cast<NHA_LDS bf16x8*>(SEa + f * 512 + ln * 8) = out;
-    } else {
-      const int g2 = f - NSEA;
-      const int Q = g2 < 2 ? 0 : g2 < 6 ? 1 : g2 < 12 ? 2 : 3;
-      const int rem = g2 - seb_base(Q);
-      const int jb = rem >> 1, pr = rem & 1;
-      const int j = 16 * jb + fl16;
-      f32x4 gv[2], gr[2];
-      bf16x4 sv[2];
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int m0 = 32 * pr + 16 * hh + 4 * fkb;   // the lane's 4 consecutive slots of this half
-        gv[hh] = *reinterpret_cast<const NHA_LDS f32x4*>(gcR + j * GLD + m0);
-        gr[hh] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        if (Q > 0) gr[hh] = *reinterpret_cast<const NHA_LDS f32x4*>(gcR + (16 * Q - 1) * GLD + m0);
-        sv[hh] = *reinterpret_cast<const NHA_LDS bf16x4*>(sR + j * SLD + m0);
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        out[e] = (__bf16)((float)sv[e >> 2][e & 3] * fexp(fminf(gr[e >> 2][e & 3] - gv[e >> 2][e & 3], DECAY_CLAMP)));
-      *reinterpret_cast<NHA_LDS bf16x8*>(SEb + g2 * 512 + ln * 8) = out;
+    for (int e = 0; e < 8; ++e) {
+      const int j = 16 * (2 * pr + (e >> 2)) + 4 * fkb + (e & 3);   // j < 64 for every fragment
+      gv[e] = gcR[j * GLD + m];
+      sv[e] = sR[j * SLD + m];
     }
+    bf16x8 out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int jb = 2 * pr + (e >> 2);
+      const float val = bf16_to_f32(sv[e]) * fexp(fminf(gr - gv[e], DECAY_CLAMP));
+      out[e] = (__bf16)(jb <= Q ? val : 0.f);
+    }
+    return out;
+  };
+  // seb_item: the same with a row j of block jb per lane (slots of half pr)
+  auto seb_item = [&](int Q, int jb, int pr, int fl16, int fkb) {
+    const int j = 16 * jb + fl16;
+    f32x4 gv[2], gr[2];
+    bf16x4 sv[2];
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+      const int m0 = 32 * pr + 16 * hh + 4 * fkb;   // the lane's 4 consecutive slots of this half
+      gv[hh] = *reinterpret_cast<const NHA_LDS f32x4*>(gcR + j * GLD + m0);
+      gr[hh] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      if (Q > 0) gr[hh] = *reinterpret_cast<const NHA_LDS f32x4*>(gcR + (16 * Q - 1) * GLD + m0);
+      sv[hh] = *reinterpret_cast<const NHA_LDS bf16x4*>(sR + j * SLD + m0);
+    }
+    bf16x8 out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      out[e] = (__bf16)((float)sv[e >> 2][e & 3] * fexp(fminf(gr[e >> 2][e & 3] - gv[e >> 2][e & 3], DECAY_CLAMP)));
+    return out;
+  };
+  if constexpr (!OWN) {
+    for (int item = tid; item < (NSEA + NSEB) * 64; item += NTHR) {
+      const int f = item >> 6, ln = item & 63;
+      if (f < NSEA) {
+        const int Q = f < 4 ? 0 : f < 8 ? 1 : f < 16 ? 2 : 3;
+        const int rem = f - sea_base(Q);
+        *reinterpret_cast<NHA_LDS bf16x8*>(SEa + f * 512 + ln * 8) = sea_item(Q, rem >> 2, rem & 3, ln & 15, ln >> 4);
+      } else {
+        const int g2 = f - NSEA;
+        const int Q = g2 < 2 ? 0 : g2 < 6 ? 1 : g2 < 12 ? 2 : 3;
+        const int rem = g2 - seb_base(Q);
+        *reinterpret_cast<NHA_LDS bf16x8*>(SEb + g2 * 512 + ln * 8) = seb_item(Q, rem >> 1, rem & 1, ln & 15, ln >> 4);
+      }
+    }
+    __syncthreads();
   }
-  __syncthreads();
 
   // per-lane softmax state for the RQB queries (l16 + 16*(qb0+qb)) this lane serves
   float mrun[RQB], lg[RQB];
@@ -865,7 +877,9 @@ __global__ __launch_bounds__(64 * NW, 1) void mfma_out_kernel(const MP p) {
 #pragma unroll
       for (int pr = 0; pr < 2; ++pr)
         if (2 * pr <= Q) {
-          const bf16x8 se = *reinterpret_cast<const NHA_LDS bf16x8*>(SEa + (sea_base(Q) + 4 * pr + mb) * 512 + lane * 8);
+          bf16x8 se;
+          if constexpr (OWN) se = sea_item(Q, pr, mb, l16, kb);
+          else se = *reinterpret_cast<const NHA_LDS bf16x8*>(SEa + (sea_base(Q) + 4 * pr + mb) * 512 + lane * 8);
           oki[mb] = mfma16(se, bA[pr], oki[mb]);
         }
     }
@@ -946,7 +960,9 @@ __global__ __launch_bounds__(64 * NW, 1) void mfma_out_kernel(const MP p) {
         if (jb <= Q) {
 #pragma unroll
           for (int pr = 0; pr < 2; ++pr) {
-            const bf16x8 se = *reinterpret_cast<const NHA_LDS bf16x8*>(SEb + (seb_base(Q) + 2 * jb + pr) * 512 + lane * 8);
+            bf16x8 se;
+            if constexpr (OWN) se = seb_item(Q, jb, pr, l16, kb);
+            else se = *reinterpret_cast<const NHA_LDS bf16x8*>(SEb + (seb_base(Q) + 2 * jb + pr) * 512 + lane * 8);
             av[jb] = mfma16(se, bpr[qb][pr], av[jb]);
           }
           if (jb == Q) {
@@ -1262,7 +1278,7 @@ template <int D, int G, int NW, int TK>
 int launch_out(const MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  const size_t lds = OutSmem<D, TK>::bytes;
+  const size_t lds = OutSmem<D, TK, G>::bytes;
   std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)mfma_out_kernel<D, G, NW, TK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));
@@ -1321,7 +1337,11 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
   if (phases != 1) {
     // G query heads of one kv-head share a workgroup.  D <= 128: 64-key tiles, 8 waves of 32 (G = 4)
     // or 16 (G = 2) query rows, two per SIMD; D = 256: 32-key tiles and 16-row waves to fit the
-    // register file and LDS
+    // register file and LDS.  One head (G = 1): 32-key tiles, four waves and two (D = 128) or three
+    // (D = 64) workgroups per CU, which 64-key tiles or decay fragments in LDS do not leave room for:
+    // 16 heads, 8192 tokens, W = 2048: D = 64 291 -> 147 us, D = 128 434 -> 269 us (with 64-key tiles 165, 375);
+    // 5003 packed tokens, W = 300: 93 -> 46, 119 -> 70.  Two heads of a pair as two such workgroups tie with
+    // G = 2 (8 / 4 heads of 128: 64 against 67 us at W = 150, 407 against 379 at W = 1500)
     int rc;
 #ifdef NHA_AB_SWITCHES   // measurement builds only (-DNHA_AB_SWITCHES): run the kernels the LDS-direct ones replaced
     static const bool ring_off = getenv("NHA_PREFILL_NO_RING") != nullptr;
@@ -1335,7 +1355,7 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
     } else if constexpr (D <= 128) {
       if (p.NG % 4 == 0) rc = launch_out<D, 4, 8, 64>(p, st);
       else if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 64>(p, st);
-      else rc = launch_out<D, 1, 4, 64>(p, st);
+      else rc = launch_out<D, 1, 4, 32>(p, st);
     } else {
       if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 32>(p, st);
       else rc = launch_out<D, 1, 4, 32>(p, st);
