@@ -167,6 +167,7 @@ int bwd_window_mfma_dq(const NhaPrefillBwdArgs* a, const float* delta, void* ld)
 // prefill_bwd_ring.hip: the window gradients with LDS-direct operands for four query heads per kv-head at
 // K = V = 128; `ld` [T_tot, HQ] pairs of floats is written by the dq call and read by the dk / dv call
 bool bwd_ring_supported(const NhaPrefillBwdArgs* a);
+bool bwd_ring_dkv_supported(const NhaPrefillBwdArgs* a);
 int bwd_ring_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld);
 int bwd_ring_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs);
 int bwd_window_mfma_dkv(const NhaPrefillBwdArgs* a, const float* delta, const float* dvs, const void* ld);

@@ -603,6 +603,20 @@ bool bwd_ring_supported(const NhaPrefillBwdArgs* a) {
   return (int64_t)a->T_tot * a->HQ * 128 * 2 < ((int64_t)1 << 32);
 }
 
+// key groups of 128 instead of 256: windows of less than 160 keys
+static bool short_groups(const NhaPrefillBwdArgs* a) { return a->wl >= 0 && a->wl < 160; }
+
+// A workgroup of ring_dkv_kernel walks all queries that see its key group, four heads of them, whatever the size of the
+// call.  Where its groups would fill half of the chip or less, bwd_dkv_kernel's groups of 64 keys are up to four times as
+// many and each walks fewer queries: 1700 tokens, 32 / 8 heads, W = 256 (56 groups) 114 -> 62 us; 4000 tokens, W = 1000
+// (128) 308 -> 236; 3000 tokens, 32 / 4 heads, W = 512 (48) 333 -> 188.  Beyond, the groups of 64 pass one round of
+// places (two per CU) and pull every q / do row four times as often: 5000 tokens, 32 / 8 heads, W = 512 (160) 187 against
+// 217 us; 4000 tokens, W = 128 (256) 51 against 57.
+bool bwd_ring_dkv_supported(const NhaPrefillBwdArgs* a) {
+  const int64_t groups = (int64_t)a->H * (short_groups(a) ? (a->NT + 1) / 2 : (a->NT + 3) / 4);
+  return bwd_ring_supported(a) && groups > 128;
+}
+
 int bwd_ring_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld) {
   DqP p;
   p.q = (const bf16_t*)a->q_swa; p.k = (const bf16_t*)a->k_swa; p.v = (const bf16_t*)a->v; p.dout = (const bf16_t*)a->dout;
@@ -641,7 +655,7 @@ int bwd_ring_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs)
     return NHA_ERR_LAUNCH;
   }
   // one launch row per chunk, rounded up to whole key groups (4 chunks of 256 keys, 2 of 128)
-  if (p.wl >= 0 && p.wl < 160)
+  if (short_groups(a))
     hipLaunchKernelGGL(ring_dkv_kernel<128>, dim3(p.H, 2 * ((p.NT + 1) / 2)), dim3(512), KV_BYTES, (hipStream_t)a->stream, p);
   else
     hipLaunchKernelGGL(ring_dkv_kernel<256>, dim3(p.H, 4 * ((p.NT + 3) / 4)), dim3(512), KV_BYTES, (hipStream_t)a->stream, p);
