@@ -55,6 +55,7 @@ struct MP {
   float* dtot;   // [NSLOT][H][MS]   total decay of a segment
   int* flags;    // [NT][H][4]       per 16-slot block: bit q = sub-block q decays past DECAY_CLAMP
   int T_tot, N, NT, HQ, H, NG, wl, shift;
+  int seg_sh;    // a segment is 1 << seg_sh chunks
   int sinks;     // window-only launches (prefill_ring.hip, SINK): zero-logit keys in front of every sequence
   float scale;
 };
@@ -119,10 +120,10 @@ __device__ __forceinline__ bf16x8 lds_frag_tr(const lbf16* tile, int ld, int r0a
   return __builtin_bit_cast(bf16x8, t);
 }
 
-// the slot recurrence is cut into segments of SEG chunks (two-level state pass)
+// the slot recurrence is cut into segments of 1 << sh <= SEG chunks (two-level state pass; prefill_mfma.hip: plan_scratch)
 constexpr int SEG = 8;
 
-__device__ __forceinline__ int seg_slot(const int32_t* coff, int n, int it) { return coff[n] / SEG + it / SEG + n; }
+__device__ __forceinline__ int seg_slot(const int32_t* coff, int n, int it, int sh) { return (coff[n] >> sh) + (it >> sh) + n; }
 
 // decay-factor fragments of the slot branch, built once per workgroup in MFMA operand order
 constexpr int NSEA = 24;   // fragments s*decay with rows = slots  (A operand of the logit update)

@@ -94,7 +94,7 @@ struct SlotP {
   float *xg, *dsi;                             // [T,H,64] (row token)
   float *ek, *ev;                              // [NT][H][D][64]
   float *dks, *dvs;                            // [T,H,D] (source token)
-  int HQ, H, NG, NT, shift;
+  int HQ, H, NG, NT, shift, seg_sh;
   float scale;
 };
 
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
   const int bos = p.cu[n], eos = p.cu[n + 1], c0 = bos + it * BT;
   const int R = (eos - c0) < BT ? (eos - c0) : BT;
   const int64_t cg = (int64_t)chunk * H + h;
-  const int64_t sl = (int64_t)seg_slot(p.coff, n, it) * H + h;
+  const int64_t sl = (int64_t)seg_slot(p.coff, n, it, p.seg_sh) * H + h;
   const float* const gc = p.gc + cg * BT * MS;   // rows past R repeat the last one
   int vlo = p.shift - it * BT;   // rows before vlo have no source token
   vlo = vlo < 0 ? 0 : vlo;
@@ -675,7 +675,7 @@ int bwd_slot_branch(const NhaPrefillBwdArgs* a, const mf::MP& m, float* delta, f
   p.hk = m.hkT; p.hv = m.hvc; p.hsk = m.hseg_k; p.hsv = m.hseg_v; p.dcum = m.dcum; p.gc = m.gc;
   p.cu = a->cu_seqlens; p.cidx = a->chunk_indices; p.coff = a->chunk_offsets;
   p.dq = (bf16_t*)a->dq_gsa; p.delta = delta; p.xg = xg; p.dsi = dsi; p.ek = ek; p.ev = ev; p.dks = dks; p.dvs = dvs;
-  p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H; p.NT = a->NT; p.shift = a->shift; p.scale = a->scale;
+  p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H; p.NT = a->NT; p.shift = a->shift; p.seg_sh = m.seg_sh; p.scale = a->scale;
   hipStream_t st = (hipStream_t)a->stream;
   if (a->K == 64) return launch<64>(p, st);
   if (a->K == 128) return launch<128>(p, st);

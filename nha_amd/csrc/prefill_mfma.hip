@@ -60,7 +60,7 @@ __device__ __forceinline__ void tile_r2l(lbf16* lds, const TileRegs<ROWS, D, NTH
 // state pass, two levels
 // ==========================================================================================
 // The slot recurrence is sequential over the chunks of a sequence, so it is cut into segments of
-// SEG chunks.  Level 1 (mfma_state_local_kernel, one workgroup per (segment, kv-head), one wave
+// 1, 2, 4 or SEG = 8 chunks (plan_scratch).  Level 1 (mfma_state_local_kernel, one workgroup per (segment, kv-head), one wave
 // per 16-slot block) runs the recurrence of chunk_fused.py:30-113 from a ZERO state over its
 // segment and stores, per chunk, the local chunk-start states, the gate cumsum table and the
 // decay accumulated since the segment start; per segment, the local end state and total decay.
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void mfma_state_local_kernel(const MP p) {
   const bf16_t* xsrc = (isv ? p.v : p.k_gsa) + dcol0;
   bf16_t* hloc = isv ? p.hvc : p.hkT;
   float* hend = isv ? p.hend_v : p.hend_k;
-  // segment k of the call -> (sequence n, segment kseg of it): a running count of ceil(chunks / SEG) over the
+  // segment k of the call -> (sequence n, segment kseg of it): a running count of ceil(chunks / segment) over the
   // sequences, 256 at a time (one per thread, prefix over the workgroup)
   __shared__ int seg_wave[4], seg_hit[2];
   int n = 0, kseg = 0;
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void mfma_state_local_kernel(const MP p) {
     int base = 0;
     for (int n0 = 0; n0 < p.N; n0 += 256) {
       const int i = n0 + tid;
-      const int segs = i < p.N ? (p.coff[i + 1] - p.coff[i] + SEG - 1) / SEG : 0;
+      const int segs = i < p.N ? (p.coff[i + 1] - p.coff[i] + (1 << p.seg_sh) - 1) >> p.seg_sh : 0;
       int incl = segs;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
@@ -134,12 +134,12 @@ __global__ __launch_bounds__(256) void mfma_state_local_kernel(const MP p) {
     n = seg_hit[0];
     kseg = seg_hit[1];
   }
-  const int it0 = kseg * SEG;
+  const int it0 = kseg << p.seg_sh;
   const int chunk0 = p.coff[n] + it0;
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int L = eos - bos;
   const int nchunks = (L + BT - 1) / BT;
-  const int nloc = (nchunks - it0) < SEG ? (nchunks - it0) : SEG;
+  const int nloc = (nchunks - it0) < (1 << p.seg_sh) ? (nchunks - it0) : 1 << p.seg_sh;
   const int m = wave * 16 + l16;   // this lane's slot
 
   f32x4 hx[NB];
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(256) void mfma_state_local_kernel(const MP p) {
     }
   }
   // segment end: local state (fp32, [m][d]) and total decay
-  const int64_t sl = (int64_t)seg_slot(p.coff, n, it0) * H + h;
+  const int64_t sl = (int64_t)seg_slot(p.coff, n, it0, p.seg_sh) * H + h;
 #pragma unroll
   for (int b = 0; b < NB; ++b)
     *reinterpret_cast<float4*>(hend + (sl * MS + m) * D + dcol0 + 16 * b + 4 * kb) = make_float4(hx[b][0], hx[b][1], hx[b][2], hx[b][3]);
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const MP p) {
   const int m = em / D, d = em % D;
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int nchunks = (eos - bos + BT - 1) / BT;
-  const int nseg = (nchunks + SEG - 1) / SEG;
+  const int nseg = (nchunks + (1 << p.seg_sh) - 1) >> p.seg_sh;
   float4 hcur = make_float4(0.f, 0.f, 0.f, 0.f);
   if (p.h0k) {
     if (isv) {
@@ -329,7 +329,7 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const MP p) {
   const float* __restrict__ hend = isv ? p.hend_v : p.hend_k;
   float* __restrict__ hseg = isv ? p.hseg_v : p.hseg_k;
   const float* __restrict__ dtot = p.dtot;
-  const int slot0 = p.coff[n] / SEG + n;
+  const int slot0 = (p.coff[n] >> p.seg_sh) + n;
   struct Grp {
     float4 he[SCAN_AHEAD];
     float dt[SCAN_AHEAD];
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(256) void state_final_kernel(const MP p) {
   const int m = em / D, d = em % D;
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int nchunks = (eos - bos + BT - 1) / BT;
-  const int nseg = (nchunks + SEG - 1) / SEG;
+  const int nseg = (nchunks + (1 << p.seg_sh) - 1) >> p.seg_sh;
   float hcur[4] = {0.f, 0.f, 0.f, 0.f};
   if (p.h0k) {
     if (isv) {
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(256) void state_final_kernel(const MP p) {
   const float* hend = isv ? p.hend_v : p.hend_k;
   bf16_t* hloc = isv ? p.hvc : p.hkT;
   const int chunk0 = p.coff[n];
-  const int slot0 = chunk0 / SEG + n;
+  const int slot0 = (chunk0 >> p.seg_sh) + n;
   struct Small {      // what the chain itself needs of a segment
     float dc[SEG];
     float dt;
@@ -430,7 +430,7 @@ __global__ __launch_bounds__(256) void state_final_kernel(const MP p) {
 #pragma unroll
     for (int jc = 0; jc < SEG; ++jc) {
       r.dc[jc] = 0.f;
-      if (sg * SEG + jc < nchunks) r.dc[jc] = p.dcum[((int64_t)(chunk0 + sg * SEG + jc) * H + h) * MS + m];
+      if (jc < (1 << p.seg_sh) && (sg << p.seg_sh) + jc < nchunks) r.dc[jc] = p.dcum[((int64_t)(chunk0 + (sg << p.seg_sh) + jc) * H + h) * MS + m];
     }
     r.dt = p.dtot[sl * MS + m];
     r.he = *reinterpret_cast<const float4*>(hend + (sl * MS + m) * D + d);
@@ -442,9 +442,9 @@ __global__ __launch_bounds__(256) void state_final_kernel(const MP p) {
 #pragma unroll
     for (int jc = 0; jc < SEG; ++jc) {
       r.v[jc] = make_uint2(0, 0);
-      if (sg * SEG + jc < nchunks && amax * sm.dc[jc] >= CARRY_FLOOR) {
+      if (jc < (1 << p.seg_sh) && (sg << p.seg_sh) + jc < nchunks && amax * sm.dc[jc] >= CARRY_FLOOR) {
         r.need |= 1u << jc;
-        r.v[jc] = *reinterpret_cast<const uint2*>(hloc + (((int64_t)(chunk0 + sg * SEG + jc) * H + h) * MS + m) * D + d);
+        r.v[jc] = *reinterpret_cast<const uint2*>(hloc + (((int64_t)(chunk0 + (sg << p.seg_sh) + jc) * H + h) * MS + m) * D + d);
       }
     }
   };
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(256) void state_final_kernel(const MP p) {
 #pragma unroll
     for (int jc = 0; jc < SEG; ++jc) {
       if (l_cur.need & (1u << jc)) {
-        const int64_t cg = (int64_t)(chunk0 + sg * SEG + jc) * H + h;
+        const int64_t cg = (int64_t)(chunk0 + (sg << p.seg_sh) + jc) * H + h;
         const uint32_t w[2] = {l_cur.v[jc].x, l_cur.v[jc].y};
         bf16x4 o4;
 #pragma unroll
@@ -502,14 +502,14 @@ __global__ __launch_bounds__(256) void state_apply_kernel(const MP p) {
     int lo = 0, hi = p.N - 1;
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
-      if (p.coff[mid] / SEG + mid <= slot) lo = mid; else hi = mid - 1;
+      if ((p.coff[mid] >> p.seg_sh) + mid <= slot) lo = mid; else hi = mid - 1;
     }
     n = lo;
   }
-  const int it0 = (slot - (p.coff[n] / SEG + n)) * SEG;
+  const int it0 = (slot - ((p.coff[n] >> p.seg_sh) + n)) << p.seg_sh;
   const int nchunks = p.coff[n + 1] - p.coff[n];
   if (it0 >= nchunks) return;
-  const int nloc = (nchunks - it0) < SEG ? (nchunks - it0) : SEG;
+  const int nloc = (nchunks - it0) < (1 << p.seg_sh) ? (nchunks - it0) : 1 << p.seg_sh;
   const int e4 = blockIdx.z * 256 + threadIdx.x;
   const bool isv = e4 >= MS * D / 4;
   const int em = (isv ? e4 - MS * D / 4 : e4) * 4;
@@ -1302,8 +1302,9 @@ int run_state_pass(const MP& p, bool segment_form, hipStream_t st) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
-  // at most NT / SEG + N segments: every sequence but for its last segment fills SEG chunks
-  const int64_t l1_grid = (int64_t)(p.NT / SEG + p.N) * p.H * 2 * (D / DW);
+  // at most NT / segment + N segments: every sequence but for its last segment fills them
+  const int nslot = (p.NT >> p.seg_sh) + p.N;
+  const int64_t l1_grid = (int64_t)nslot * p.H * 2 * (D / DW);
   if (l1_grid > 0x7fffffff) {
     set_error("nha_prefill_fwd(mfma): too many segments for one launch (%lld workgroups)", (long long)l1_grid);
     return NHA_ERR_UNSUPPORTED;
@@ -1313,12 +1314,12 @@ int run_state_pass(const MP& p, bool segment_form, hipStream_t st) {
   // the forward's chunk states: inside the scan while a sequence has about eight segments or fewer (a thread's
   // chain there costs a memory latency per segment: 15 us at 4 segments, 21 us at 16 on one box), after it beyond
   // (two launches without a chain: 16-18 us whatever the length)
-  const bool in_scan = !segment_form && (int64_t)p.NT <= (int64_t)8 * SEG * p.N;
+  const bool in_scan = !segment_form && (int64_t)p.NT <= ((int64_t)8 * p.N << p.seg_sh);
   if (in_scan) {
     hipLaunchKernelGGL((state_final_kernel<D>), dim3(p.N * p.H, 2 * MS * D / 1024), dim3(256), 0, st, p);
   } else {
     hipLaunchKernelGGL((state_scan_kernel<D>), dim3(p.N * p.H, 2 * MS * D / 1024), dim3(256), 0, st, p);
-    if (!segment_form) hipLaunchKernelGGL((state_apply_kernel<D>), dim3(p.NT / SEG + p.N + 1, p.H, 2 * MS * D / 1024), dim3(256), 0, st, p);
+    if (!segment_form) hipLaunchKernelGGL((state_apply_kernel<D>), dim3(nslot + 1, p.H, 2 * MS * D / 1024), dim3(256), 0, st, p);
   }
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma state pass, level 2)");
   return NHA_OK;
@@ -1377,10 +1378,11 @@ bool prefill_mfma_supported(const NhaPrefillArgs* a) {
 namespace {
 struct ScratchPlan {
   size_t hkT, hvc, gc, dcum, hend_k, hend_v, hseg_k, hseg_v, dtot, flags, total;
+  int seg_sh;
 };
-ScratchPlan plan_scratch(const NhaPrefillArgs* a) {
+ScratchPlan plan_scratch(const NhaPrefillArgs* a, int seg_sh) {
   const size_t per = (size_t)a->NT * a->H;
-  const size_t nslot = (size_t)a->NT / SEG + a->N + 1;
+  const size_t nslot = ((size_t)a->NT >> seg_sh) + a->N + 1;
   const size_t seg = aligned(nslot * a->H * MS * a->K * 4);
   ScratchPlan s;
   size_t off = 0;
@@ -1395,7 +1397,29 @@ ScratchPlan plan_scratch(const NhaPrefillArgs* a) {
   s.dtot = off; off += aligned(nslot * a->H * MS * 4);
   s.flags = off; off += aligned(per * 4 * 4);
   s.total = off;
+  s.seg_sh = seg_sh;
   return s;
+}
+
+// Chunks per segment: 8, where the chip is full.  Level 1 walks its segment at 2.4 us per chunk whatever else runs, so a
+// call that leaves places on the chip empty takes shorter segments, as long as all its workgroups are resident at once
+// (two per CU at head sizes 128 and 256, three at 64, by registers); level 2 then combines more of them, at about 0.25 us
+// each: hence the weights 11 : 1.  Level 1 / state pass at 1000 tokens, 8 kv-heads of 128: 25.4 / 31.6 us with 8 chunks,
+// 15.9 / 21.3 with 4, 9.0 / 20.3 with 1; 4 heads of 256 25.4 / 31.9, 16.7 / 21.9, 9.7 / 21.3.  More workgroups than places
+// lose: 2 x 2048 tokens, 8 heads of 128 take 35 us with 8 chunks, 30 with 4 and 43 with 1.
+// A call whose workspace fits the library's own array with 8 chunks keeps fitting it.
+ScratchPlan plan_scratch(const NhaPrefillArgs* a) {
+  const ScratchPlan full = plan_scratch(a, 3);
+  const int z = a->K >= 256 ? 4 : 2, places = a->K >= 128 ? 512 : 768;
+  const int64_t chunks = ((int64_t)a->NT + a->N - 1) / a->N;
+  int best = 3;
+  for (int sh = 2; sh >= 0; --sh) {
+    if ((((int64_t)a->NT >> sh) + a->N) * a->H * z > places) break;
+    if ((11 << sh) + (chunks >> sh) >= (11 << best) + (chunks >> best)) break;
+    if (full.total <= (size_t)NHA_NOALLOC_SCRATCH_BYTES && plan_scratch(a, sh).total > (size_t)NHA_NOALLOC_SCRATCH_BYTES) break;
+    best = sh;
+  }
+  return best == 3 ? full : plan_scratch(a, best);
 }
 }  // namespace
 
@@ -1425,6 +1449,7 @@ MP make_mp(const NhaPrefillArgs* a) {
   p.flags = (int*)(sc + sp.flags);
   p.T_tot = a->T_tot; p.N = a->N; p.NT = a->NT; p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H;
   p.wl = a->wl; p.shift = a->shift; p.scale = a->scale;
+  p.seg_sh = sp.seg_sh;
   return p;
 }
 }  // namespace
