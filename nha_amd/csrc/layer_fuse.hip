@@ -26,7 +26,6 @@ struct LP {
 
 constexpr int TOK_PER_WG = 4;     // one wave per token
 constexpr int ROWS_PER_WAVE = 4;  // epilogue rows a wave walks with its weight slice in registers
-constexpr int BWD_ROWS = 32;      // epilogue backward: rows per workgroup (one partial weight gradient each)
 
 template <typename T> __device__ __forceinline__ float rnd(float x);
 template <> __device__ __forceinline__ float rnd<float>(float x) { return x; }
@@ -384,11 +383,108 @@ struct EPB {
   void* dout;
   const float* w;
   float *dw_part, *db_part;
-  int rows, dim;
+  int rows, dim, rows_wg;
   float eps;
 };
 
-// Backward of y = silu(o) * rstd * w + b for BWD_ROWS rows per workgroup.  Thread `tid` owns the
+// rows of a workgroup (and of one row of the partial sums): fewer for small calls, which would leave CUs idle
+__host__ __device__ constexpr int bwd_rows(int rows) { return rows <= 8192 ? 8 : 32; }
+
+// Backward of y = silu(o) * rstd * w + b, dim <= 512 NV: one wave per row, the rows of a workgroup dealt to its four waves,
+// the next row's two reads requested before this row's sums are formed.  Lane l owns the columns (64 n + l) * 8 .. + 8 of
+// every row; the waves' shares of the weight and bias gradients are added through LDS in a fixed order.
+// Bound: HBM (o, dy in, do out).  With the row spread over a workgroup every row was two barriers and a memory latency,
+// 1.4 us, and half the threads idle at dim = 1024: 1400 rows of 1024 44 -> 9 us, 16384 rows 47 -> 21 us;
+// 16384 rows of 2048 66 -> 51 us.
+template <typename T, int NV>
+__global__ __launch_bounds__(256) void layer_epilogue_bwd_wave_kernel(EPB p) {
+  extern __shared__ float sums[];   // [3 waves][dw, db][dim]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float w[NV][8], dw[NV][8], db[NV][8];
+  Raw<T, 8> xn[NV], dn[NV];
+#pragma unroll
+  for (int n = 0; n < NV; ++n) {
+    const int u = (64 * n + lane) * 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[n][e] = 1.f, dw[n][e] = 0.f, db[n][e] = 0.f;
+    if (p.w && u < p.dim) ldv<float, 8>(p.w + u, w[n]);
+  }
+  const int r0 = blockIdx.x * p.rows_wg;
+  const int r1 = r0 + p.rows_wg < p.rows ? r0 + p.rows_wg : p.rows;
+  auto request = [&](int r) {
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const int u = (64 * n + lane) * 8;
+      if (r < r1 && u < p.dim) {
+        xn[n].load((const T*)p.o + (size_t)r * p.dim + u);
+        dn[n].load((const T*)p.dy + (size_t)r * p.dim + u);
+      }
+    }
+  };
+  request(r0 + wave);
+  for (int r = r0 + wave; r < r1; r += 4) {
+    float ss = 0.f, dot = 0.f, a[NV][8], x[NV][8], d[NV][8];
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      xn[n].unpack(x[n]);
+      dn[n].unpack(d[n]);
+      if ((64 * n + lane) * 8 >= p.dim)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[n][e] = d[n][e] = 0.f;
+    }
+    request(r + 4);
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        a[n][e] = rnd<T>(silu_f(x[n][e]));
+        ss += a[n][e] * a[n][e];
+        dot += d[n][e] * w[n][e] * a[n][e];
+      }
+    ss = wave_sum(ss);
+    dot = wave_sum(dot);
+    const float rstd = rsqrtf(ss / (float)p.dim + p.eps);
+    const float coef = dot * rstd * rstd * rstd / (float)p.dim;  // rstd * mean(dn * n), n = a * rstd
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const int u = (64 * n + lane) * 8;
+      float g[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        dw[n][e] += d[n][e] * a[n][e] * rstd;
+        db[n][e] += d[n][e];
+        const float da = rstd * d[n][e] * w[n][e] - coef * a[n][e];
+        g[e] = da * silu_grad_f(x[n][e]);
+      }
+      if (u < p.dim) stv<T, 8>((T*)p.dout + (size_t)r * p.dim + u, g);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NV; ++n) {
+    const int u = (64 * n + lane) * 8;
+    if (wave > 0 && u < p.dim) {
+      stv<float, 8>(sums + (size_t)(2 * wave - 2) * p.dim + u, dw[n]);
+      stv<float, 8>(sums + (size_t)(2 * wave - 1) * p.dim + u, db[n]);
+    }
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int n = 0; n < NV; ++n) {
+    const int u = (64 * n + lane) * 8;
+    if (u >= p.dim) continue;
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        dw[n][e] += sums[(size_t)(2 * k) * p.dim + u + e];
+        db[n][e] += sums[(size_t)(2 * k + 1) * p.dim + u + e];
+      }
+    if (p.dw_part) stv<float, 8>(p.dw_part + (size_t)blockIdx.x * p.dim + u, dw[n]);
+    if (p.db_part) stv<float, 8>(p.db_part + (size_t)blockIdx.x * p.dim + u, db[n]);
+  }
+}
+
+// The same for longer rows, a row per workgroup at a time.  Thread `tid` owns the
 // columns (n * 256 + tid) * 8 .. + 8, n < NV, of every row, so its share of the weight and bias
 // gradients accumulates in registers and leaves as one row of the partial-sum arrays
 // dw_part / db_part [gridDim.x, dim] (summed over the first axis by the caller: a fixed order).
@@ -404,8 +500,8 @@ __global__ __launch_bounds__(256) void layer_epilogue_bwd_kernel(EPB p) {
     for (int e = 0; e < 8; ++e) w[n][e] = 1.f, dw[n][e] = 0.f, db[n][e] = 0.f;
     if (p.w && u < p.dim) ldv<float, 8>(p.w + u, w[n]);
   }
-  const int r0 = blockIdx.x * BWD_ROWS;
-  for (int rr = 0; rr < BWD_ROWS; ++rr) {
+  const int r0 = blockIdx.x * p.rows_wg;
+  for (int rr = 0; rr < p.rows_wg; ++rr) {
     const int r = r0 + rr;
     if (r >= p.rows) break;  // uniform over the workgroup
     const T* src = (const T*)p.o + (size_t)r * p.dim;
@@ -465,8 +561,10 @@ __global__ __launch_bounds__(256) void layer_epilogue_bwd_kernel(EPB p) {
 
 template <typename T>
 int launch_epilogue_bwd(const EPB& p, hipStream_t st) {
-  const dim3 grid((p.rows + BWD_ROWS - 1) / BWD_ROWS);
-  if (p.dim <= 2048) hipLaunchKernelGGL((layer_epilogue_bwd_kernel<T, 1>), grid, dim3(256), 0, st, p);
+  const dim3 grid((p.rows + p.rows_wg - 1) / p.rows_wg);
+  const size_t lds = (size_t)6 * p.dim * sizeof(float);   // at most 48 KB
+  if (p.dim <= 1024) hipLaunchKernelGGL((layer_epilogue_bwd_wave_kernel<T, 2>), grid, dim3(256), lds, st, p);
+  else if (p.dim <= 2048) hipLaunchKernelGGL((layer_epilogue_bwd_wave_kernel<T, 4>), grid, dim3(256), lds, st, p);
   else if (p.dim <= 4096) hipLaunchKernelGGL((layer_epilogue_bwd_kernel<T, 2>), grid, dim3(256), 0, st, p);
   else hipLaunchKernelGGL((layer_epilogue_bwd_kernel<T, 4>), grid, dim3(256), 0, st, p);
   return 0;
@@ -842,7 +940,7 @@ int layer_epilogue_bwd_impl(const NhaLayerEpilogueBwdArgs* a) {
   }
   EPB p;
   p.o = a->o; p.dy = a->dy; p.dout = a->dout; p.w = a->weight; p.dw_part = a->dweight_partial; p.db_part = a->dbias_partial;
-  p.rows = a->rows; p.dim = a->dim; p.eps = a->eps;
+  p.rows = a->rows; p.dim = a->dim; p.rows_wg = bwd_rows(a->rows); p.eps = a->eps;
   hipStream_t st = (hipStream_t)a->stream;
   if (a->dtype == NHA_DTYPE_BF16) launch_epilogue_bwd<bf16_t>(p, st);
   else launch_epilogue_bwd<float>(p, st);
