@@ -478,6 +478,10 @@ int nha_layer_prologue_bwd(const NhaLayerPrologueBwdArgs* a);
 int32_t nha_layer_epilogue_bwd_parts(int32_t rows);
 int nha_layer_epilogue_bwd(const NhaLayerEpilogueBwdArgs* a);
 
+/* Share of the slot branch in the softmax mass (nha_fla/layers/nha.py:288-298): the sum over n tokens x heads of
+ * e^lse_gsa / (e^lse_swa + e^lse_gsa) as `parts` partial sums, one per workgroup, which the caller adds up. */
+int nha_gsa_share(const float* lse_swa, const float* lse_gsa, int64_t n, float* partial, int32_t parts, void* stream);
+
 /* Depthwise causal short convolution with optional SiLU over packed tokens: what the layer applies to its
  * q / k / v projections when use_short_conv is set (nha_fla/layers/nha.py:121-140, :186-206; the module
  * itself, fla.modules.ShortConvolution, is a dependency outside the reference tree):

@@ -236,6 +236,8 @@ def load() -> C.CDLL:
     lib.nha_layer_epilogue_bwd.argtypes = [C.POINTER(NhaLayerEpilogueBwdArgs)]
     lib.nha_layer_epilogue_bwd_parts.restype = C.c_int32
     lib.nha_layer_epilogue_bwd_parts.argtypes = [C.c_int32]
+    lib.nha_gsa_share.restype = C.c_int
+    lib.nha_gsa_share.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_int32, C.c_void_p]
     lib.nha_hybrid_prologue.restype = C.c_int
     lib.nha_hybrid_prologue.argtypes = [C.POINTER(NhaHybridPrologueArgs)]
     lib.nha_zero_sink_rescale.restype = C.c_int

@@ -352,6 +352,12 @@ int nha_layer_epilogue_bwd(const NhaLayerEpilogueBwdArgs* a) {
   return layer_epilogue_bwd_impl(a);
 }
 
+int nha_gsa_share(const float* lse_swa, const float* lse_gsa, int64_t n, float* partial, int32_t parts, void* stream) {
+  NHA_CHECK_ARG(lse_swa && lse_gsa && partial, "nha_gsa_share: lse_swa, lse_gsa and partial are required");
+  NHA_CHECK_ARG(n > 0 && parts > 0 && parts <= 65535, "nha_gsa_share: bad dimension");
+  return gsa_share_impl(lse_swa, lse_gsa, n, partial, parts, stream);
+}
+
 static int check_short_conv(const char* who, const void* x, const void* w, int T_tot, int N, int C, int KS, int act, int dtype) {
   NHA_CHECK_ARG(T_tot > 0 && N > 0 && C > 0, "%s: non-positive dimension", who);
   NHA_CHECK_ARG(dtype == NHA_DTYPE_F32 || dtype == NHA_DTYPE_BF16, "%s: bad dtype %d", who, dtype);

@@ -559,6 +559,22 @@ __global__ __launch_bounds__(256) void layer_epilogue_bwd_kernel(EPB p) {
   }
 }
 
+// Share of the slot branch in the softmax mass, e^gsa / (e^swa + e^gsa) over n pairs of log-sum-exps: one partial sum per
+// workgroup.  The layer records the mean of every training forward; as tensor operations that was ten launches.
+__global__ __launch_bounds__(256) void gsa_share_kernel(const float* __restrict__ swa, const float* __restrict__ gsa, int64_t n, float* part) {
+  __shared__ float red[4];
+  float sum = 0.f;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const float a = swa[i], b = gsa[i], m = fmaxf(a, b);
+    const float ea = expf(a - m), eb = expf(b - m);
+    sum += eb / (ea + eb);
+  }
+  sum = wave_sum(sum);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
 template <typename T>
 int launch_epilogue_bwd(const EPB& p, hipStream_t st) {
   const dim3 grid((p.rows + p.rows_wg - 1) / p.rows_wg);
@@ -897,7 +913,13 @@ int layer_prologue_bwd_impl(const NhaLayerPrologueBwdArgs* a) {
   return NHA_OK;
 }
 
-int layer_epilogue_bwd_parts(int rows) { return (rows + BWD_ROWS - 1) / BWD_ROWS; }
+int layer_epilogue_bwd_parts(int rows) { return (rows + bwd_rows(rows) - 1) / bwd_rows(rows); }
+
+int gsa_share_impl(const float* swa, const float* gsa, int64_t n, float* part, int parts, void* stream) {
+  hipLaunchKernelGGL(gsa_share_kernel, dim3(parts), dim3(256), 0, (hipStream_t)stream, swa, gsa, n, part);
+  NHA_CHECK_LAUNCH("nha_gsa_share");
+  return NHA_OK;
+}
 
 int short_conv_bwd_parts(int T_tot) { return (T_tot + SC_RUN - 1) / SC_RUN; }
 

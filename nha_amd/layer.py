@@ -22,7 +22,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops as _ops
-from .ops import chunk_nha, nha_layer_epilogue, nha_layer_prologue
+from .ops import chunk_nha, gsa_share, nha_layer_epilogue, nha_layer_prologue
 
 
 class RMSNorm(nn.Module):
@@ -349,9 +349,12 @@ class NativeHybridAttention(nn.Module):
                 max_seqlen=max_seqlen,
             )
             if self.training:
-                lse_max = torch.maximum(lse_swa, lse_gsa)
-                w_swa, w_gsa = torch.exp(lse_swa - lse_max), torch.exp(lse_gsa - lse_max)
-                self._store_compression_stats(w_swa, w_gsa)
+                if getattr(self._store_compression_stats, '__func__', None) is _STORE_STATS:
+                    self._append_compression_stats(gsa_share(lse_swa, lse_gsa))
+                else:                                    # a record of the caller's own takes the two weights
+                    lse_max = torch.maximum(lse_swa, lse_gsa)
+                    w_swa, w_gsa = torch.exp(lse_swa - lse_max), torch.exp(lse_gsa - lse_max)
+                    self._store_compression_stats(w_swa, w_gsa)
                 if self.gsa_aux_loss_enable:
                     output, gsa_aux_loss = self._apply_gsa_aux_loss(output, lse_swa, lse_gsa)
                     self._store_gsa_aux_loss(gsa_aux_loss)
@@ -393,10 +396,15 @@ class NativeHybridAttention(nn.Module):
     @torch.no_grad()
     def _store_compression_stats(self, w_swa: torch.Tensor, w_gsa: torch.Tensor):
         """GSA vs SWA share of the softmax mass (nha_fla/layers/nha.py:288-298)."""
-        gsa_ratio = (w_gsa / (w_swa + w_gsa)).mean().item()
+        self._append_compression_stats((w_gsa / (w_swa + w_gsa)).mean().item())
+
+    def _append_compression_stats(self, gsa_ratio: float):
         if not hasattr(self, '_compression_stats'):
             self._compression_stats = []
         self._compression_stats.append({'gsa_ratio': gsa_ratio, 'swa_ratio': 1.0 - gsa_ratio})
+
+
+_STORE_STATS = NativeHybridAttention._store_compression_stats
 
 
 class _AttachLossGrad(torch.autograd.Function):

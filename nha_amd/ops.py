@@ -385,6 +385,20 @@ def nha_layer_epilogue(o, weight: Optional[torch.Tensor], bias: Optional[torch.T
     return _epilogue_fwd(o, w, b, float(eps))
 
 
+@torch.compiler.disable
+def gsa_share(lse_swa: torch.Tensor, lse_gsa: torch.Tensor) -> float:
+    """Mean over tokens and heads of e^lse_gsa / (e^lse_swa + e^lse_gsa) (fp32 tensors of one shape): one launch, then one
+    copy of its partial sums to the host, which adds them."""
+    _need_cuda(lse_swa, lse_gsa)
+    if lse_swa.dtype != torch.float32 or lse_gsa.dtype != torch.float32 or lse_swa.shape != lse_gsa.shape:
+        raise ValueError("gsa_share takes two float32 tensors of one shape")
+    a, b = lse_swa.detach().contiguous(), lse_gsa.detach().contiguous()
+    n = a.numel()
+    part = torch.empty(min(256, (n + 255) // 256), dtype=torch.float32, device=a.device)
+    _lib.check(_lib.load().nha_gsa_share(a.data_ptr(), b.data_ptr(), n, part.data_ptr(), part.numel(), _stream(a.device)))
+    return sum(part.tolist()) / n
+
+
 def _short_conv_args(x, cu):
     T_tot = x.shape[0] * x.shape[1]
     N = (cu.numel() - 1) if cu is not None else x.shape[0]

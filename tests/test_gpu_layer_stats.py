@@ -1,5 +1,5 @@
-"""The epilogue's backward with a wave per row (dim <= 2048) at the edges of its columns and row groups, against the
-fp64 formula."""
+"""The epilogue's backward with a wave per row (dim <= 2048) at the edges of its columns and row groups, and the slot
+branch's share of the softmax mass, against the fp64 formulas."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -26,3 +26,14 @@ def test_epilogue_backward_rows(dtype, rows, dim):
     for name, g, r in zip(("do", "dweight", "dbias"), got, ref):
         rel = ((g.double().cpu() - r).norm() / r.norm()).item()
         assert rel <= bar, f"{name}: relative L2 error {rel:.3e}"
+
+
+@pytest.mark.parametrize("n", [1, 255, 65536, 300001])
+def test_gsa_share(n):
+    from nha_amd.ops import gsa_share
+    gen = torch.Generator().manual_seed(n)
+    a, b = 30 * torch.randn(n, generator=gen), 30 * torch.randn(n, generator=gen)
+    if n > 1:
+        a[0], b[1] = float("-inf"), float("-inf")
+    ref = torch.sigmoid(b.double() - a.double()).mean().item()
+    assert abs(gsa_share(a.cuda(), b.cuda()) - ref) <= 1e-5      # fp32 exponentials and sums of up to 1200 terms
