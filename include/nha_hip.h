@@ -478,6 +478,22 @@ int nha_layer_prologue_bwd(const NhaLayerPrologueBwdArgs* a);
 int32_t nha_layer_epilogue_bwd_parts(int32_t rows);
 int nha_layer_epilogue_bwd(const NhaLayerEpilogueBwdArgs* a);
 
+/* Weight gradients of up to four projections of one input, bf16 with fp32 sums: dw[q] [O[q], I] = dy[q]^T x, x [T, I],
+ * dy[q] [T, O[q]], I and O[q] multiples of 8, all 16-byte aligned; rows * I below 2^31.  scratch: at least
+ * nha_wgrad_scratch_bytes(a) bytes (0: bad arguments), which reads n, T, I and O only. */
+typedef struct NhaWgradArgs {
+  const void* x;
+  const void* dy[4];
+  void* dw[4];
+  void* scratch;
+  size_t scratch_bytes;
+  void* stream;
+  int32_t O[4];
+  int32_t n, T, I;
+} NhaWgradArgs;
+size_t nha_wgrad_scratch_bytes(const NhaWgradArgs* a);
+int nha_wgrad(const NhaWgradArgs* a);
+
 /* Share of the slot branch in the softmax mass (nha_fla/layers/nha.py:288-298): the sum over n tokens x heads of
  * e^lse_gsa / (e^lse_swa + e^lse_gsa) as `parts` partial sums, one per workgroup, which the caller adds up. */
 int nha_gsa_share(const float* lse_swa, const float* lse_gsa, int64_t n, float* partial, int32_t parts, void* stream);

@@ -164,6 +164,12 @@ class NhaShortConvBwdArgs(C.Structure):
     ]
 
 
+class NhaWgradArgs(C.Structure):
+    _fields_ = [("x", C.c_void_p), ("dy", C.c_void_p * 4), ("dw", C.c_void_p * 4), ("scratch", C.c_void_p),
+                ("scratch_bytes", C.c_size_t), ("stream", C.c_void_p), ("O", C.c_int32 * 4), ("n", C.c_int32),
+                ("T", C.c_int32), ("I", C.c_int32)]
+
+
 class NhaRingFillArgs(C.Structure):
     _fields_ = [
         ("src", C.c_void_p * 4), ("ring", C.c_void_p * 4), ("row_bytes", C.c_int32 * 4),
@@ -236,6 +242,10 @@ def load() -> C.CDLL:
     lib.nha_layer_epilogue_bwd.argtypes = [C.POINTER(NhaLayerEpilogueBwdArgs)]
     lib.nha_layer_epilogue_bwd_parts.restype = C.c_int32
     lib.nha_layer_epilogue_bwd_parts.argtypes = [C.c_int32]
+    lib.nha_wgrad_scratch_bytes.restype = C.c_size_t
+    lib.nha_wgrad_scratch_bytes.argtypes = [C.POINTER(NhaWgradArgs)]
+    lib.nha_wgrad.restype = C.c_int
+    lib.nha_wgrad.argtypes = [C.POINTER(NhaWgradArgs)]
     lib.nha_gsa_share.restype = C.c_int
     lib.nha_gsa_share.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_int32, C.c_void_p]
     lib.nha_hybrid_prologue.restype = C.c_int

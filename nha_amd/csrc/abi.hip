@@ -352,6 +352,41 @@ int nha_layer_epilogue_bwd(const NhaLayerEpilogueBwdArgs* a) {
   return layer_epilogue_bwd_impl(a);
 }
 
+static int check_wgrad(const NhaWgradArgs* a, bool pointers) {
+  NHA_CHECK_ARG(a != nullptr, "nha_wgrad: null args");
+  NHA_CHECK_ARG(a->n >= 1 && a->n <= 4 && a->T > 0 && a->T <= (1 << 30) && a->I > 0 && a->I % 8 == 0, "nha_wgrad: bad dimension");
+  int64_t rows = 0;
+  for (int q = 0; q < a->n; ++q) {
+    NHA_CHECK_ARG(a->O[q] > 0 && a->O[q] % 8 == 0, "nha_wgrad: O must be positive multiples of 8");
+    rows += a->O[q];
+    if (pointers) {
+      NHA_CHECK_ARG(a->dy[q] && a->dw[q], "nha_wgrad: dy and dw are required");
+      NHA_CHECK_ARG(((reinterpret_cast<uintptr_t>(a->dy[q]) | reinterpret_cast<uintptr_t>(a->dw[q])) & 15) == 0,
+                    "nha_wgrad: tensors must be 16-byte aligned");
+    }
+  }
+  NHA_CHECK_ARG(rows * a->I < ((int64_t)1 << 31), "nha_wgrad: the weights are too large");
+  if (pointers) {
+    NHA_CHECK_ARG(a->x && a->scratch, "nha_wgrad: x and scratch are required");
+    NHA_CHECK_ARG(((reinterpret_cast<uintptr_t>(a->x) | reinterpret_cast<uintptr_t>(a->scratch)) & 15) == 0,
+                  "nha_wgrad: tensors must be 16-byte aligned");
+  }
+  return NHA_OK;
+}
+
+size_t nha_wgrad_scratch_bytes(const NhaWgradArgs* a) { return check_wgrad(a, false) == NHA_OK ? wgrad_scratch_bytes(a) : 0; }
+
+int nha_wgrad(const NhaWgradArgs* a) {
+  const int rc = check_wgrad(a, true);
+  if (rc != NHA_OK) return rc;
+  const size_t need = wgrad_scratch_bytes(a);
+  if (a->scratch_bytes < need) {
+    set_error("nha_wgrad: scratch has %zu bytes, %zu needed", a->scratch_bytes, need);
+    return NHA_ERR_SCRATCH;
+  }
+  return wgrad_impl(a);
+}
+
 int nha_gsa_share(const float* lse_swa, const float* lse_gsa, int64_t n, float* partial, int32_t parts, void* stream) {
   NHA_CHECK_ARG(lse_swa && lse_gsa && partial, "nha_gsa_share: lse_swa, lse_gsa and partial are required");
   NHA_CHECK_ARG(n > 0 && parts > 0 && parts <= 65535, "nha_gsa_share: bad dimension");

@@ -131,6 +131,8 @@ int layer_prologue_impl(const NhaLayerPrologueArgs* a);
 int layer_epilogue_impl(const NhaLayerEpilogueArgs* a);
 int layer_prologue_bwd_impl(const NhaLayerPrologueBwdArgs* a);
 int layer_epilogue_bwd_parts(int rows);
+size_t wgrad_scratch_bytes(const NhaWgradArgs* a);
+int wgrad_impl(const NhaWgradArgs* a);
 int gsa_share_impl(const float* swa, const float* gsa, int64_t n, float* part, int parts, void* stream);
 int layer_epilogue_bwd_impl(const NhaLayerEpilogueBwdArgs* a);
 int hybrid_prologue_impl(const NhaHybridPrologueArgs* a);

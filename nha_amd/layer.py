@@ -22,7 +22,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops as _ops
-from .ops import chunk_nha, gsa_share, nha_layer_epilogue, nha_layer_prologue
+from .ops import chunk_nha, gsa_share, linear, nha_layer_epilogue, nha_layer_prologue, shared_input_linears
 
 
 class RMSNorm(nn.Module):
@@ -301,15 +301,13 @@ class NativeHybridAttention(nn.Module):
             indices, cu_seqlens, max_seqlen = get_unpad_data(attention_mask[:, -q_len:])
             hidden_states = hidden_states.reshape(batch_size * q_len, -1)[indices].unsqueeze(0)
         conv_state_q = conv_state_k = conv_state_v = None
+        q, k, v, f = shared_input_linears(hidden_states, (self.q_proj, self.k_proj, self.v_proj, self.f_proj))
         if self.use_short_conv:
             if last_state is not None:
                 conv_state_q, conv_state_k, conv_state_v = last_state['conv_state']
-            q, conv_state_q = self.q_conv1d(self.q_proj(hidden_states), conv_state_q, use_cache, cu_seqlens)
-            k, conv_state_k = self.k_conv1d(self.k_proj(hidden_states), conv_state_k, use_cache, cu_seqlens)
-            v, conv_state_v = self.v_conv1d(self.v_proj(hidden_states), conv_state_v, use_cache, cu_seqlens)
-        else:
-            q, k, v = self.q_proj(hidden_states), self.k_proj(hidden_states), self.v_proj(hidden_states)
-        f = self.f_proj(hidden_states)
+            q, conv_state_q = self.q_conv1d(q, conv_state_q, use_cache, cu_seqlens)
+            k, conv_state_k = self.k_conv1d(k, conv_state_k, use_cache, cu_seqlens)
+            v, conv_state_v = self.v_conv1d(v, conv_state_v, use_cache, cu_seqlens)
         q = q.unflatten(-1, (-1, self.head_k_dim))
         k = k.unflatten(-1, (-1, self.head_k_dim))
         v = v.unflatten(-1, (-1, self.head_v_dim))
@@ -369,8 +367,8 @@ class NativeHybridAttention(nn.Module):
             )
         o = output[:, :, :, :self.head_v_dim].flatten(-2)
         if fused:
-            o = F.linear(nha_layer_epilogue(o, self.g_norm.weight, self.g_norm.bias, self.norm_eps),
-                         self.o_proj.weight, self.o_proj.bias)
+            o = linear(nha_layer_epilogue(o, self.g_norm.weight, self.g_norm.bias, self.norm_eps),
+                       self.o_proj.weight, self.o_proj.bias)
         else:
             o = rms_norm_linear(F.silu(o), self.g_norm.weight, self.g_norm.bias, self.o_proj.weight, self.o_proj.bias,
                                 eps=self.norm_eps)

@@ -385,6 +385,101 @@ def nha_layer_epilogue(o, weight: Optional[torch.Tensor], bias: Optional[torch.T
     return _epilogue_fwd(o, w, b, float(eps))
 
 
+def nha_wgrad(x: torch.Tensor, dys) -> list:
+    """dy^T x for every dy [T, O] of `dys` (at most four), x [T, I]: the weight gradients of projections of one input, bf16."""
+    lib = _lib.load()
+    T, width = x.shape
+    outs = [torch.empty(dy.shape[1], width, dtype=x.dtype, device=x.device) for dy in dys]
+    a = _lib.NhaWgradArgs(x=_ptr(x), n=len(outs), T=T, I=width, stream=_stream(x.device))
+    for i, (dy, dw) in enumerate(zip(dys, outs)):
+        a.dy[i], a.dw[i], a.O[i] = _ptr(dy), _ptr(dw), dy.shape[1]
+    nbytes = lib.nha_wgrad_scratch_bytes(C.byref(a))
+    if nbytes == 0:
+        _lib.check(_lib.NHA_ERR_INVALID)
+    scratch = _workspace(nbytes, x.device, a.stream or 0)
+    a.scratch, a.scratch_bytes = _ptr(scratch), scratch.numel()
+    _lib.check(lib.nha_wgrad(C.byref(a)))
+    return outs
+
+
+def _wgrad_supported(x: torch.Tensor, dys) -> bool:
+    """Rows of 16-byte pieces, bf16.  A single gradient of few tokens stays with the library: 1024 x 1024 from 4096 tokens
+    takes it 29 us against 34, from 6000 45 against 39, from 16384 104 against 54.  Several at once are faster from any
+    number (1024 columns, outputs of 3 x 1024 + 256 from 300 tokens: 28 us against 78 for four library calls)."""
+    T, width = x.shape
+    return (x.dtype == torch.bfloat16 and 0 < T <= 1 << 30 and width % 8 == 0 and x.data_ptr() % 16 == 0 and len(dys) <= 4
+            and all(dy.dtype == x.dtype and dy.shape[1] % 8 == 0 and dy.data_ptr() % 16 == 0 for dy in dys)
+            and sum(dy.shape[1] for dy in dys) * width < 1 << 31 and (len(dys) > 1 or T >= 6000))
+
+
+class _SharedInputLinear(torch.autograd.Function):
+    """F.linear of one input with several weights.  Backward: the input's gradient summed inside the products (each added
+    to the one before it, no tensors in between), the weights' gradients in one launch (nha_wgrad)."""
+
+    @staticmethod
+    def forward(ctx, x, *weights):
+        ctx.save_for_backward(x, *weights)
+        return tuple(torch.nn.functional.linear(x, w) for w in weights)
+
+    @staticmethod
+    def backward(ctx, *dys):
+        x, *weights = ctx.saved_tensors
+        rows = [dy.reshape(-1, dy.shape[-1]) for dy in dys]
+        xr = x.reshape(-1, x.shape[-1])
+        need = [i for i, n in enumerate(ctx.needs_input_grad[1:]) if n]
+        dx, dws = None, [None] * len(weights)
+        if torch.is_grad_enabled():                        # a second derivative is wanted: operations that have one
+            if ctx.needs_input_grad[0]:
+                dx = sum(dy @ w for dy, w in zip(rows, weights)).view(x.shape)
+            for i in need:
+                dws[i] = rows[i].t() @ xr
+            return (dx, *dws)
+        if ctx.needs_input_grad[0]:
+            dx = rows[0] @ weights[0]
+            for dy, w in zip(rows[1:], weights[1:]):
+                dx.addmm_(dy, w)
+            dx = dx.view(x.shape)
+        picked, xc = [rows[i].contiguous() for i in need], xr.contiguous()
+        if need and _wgrad_supported(xc, picked):
+            for i, dw in zip(need, nha_wgrad(xc, picked)):
+                dws[i] = dw
+        else:
+            for i in need:
+                dws[i] = rows[i].t() @ xr
+        return (dx, *dws)
+
+
+_LINEAR_FORWARD = torch.nn.Linear.forward
+
+
+def _linears(x: torch.Tensor, weights):
+    """F.linear of x with every weight through one autograd node, or None where something besides reverse-mode autograd
+    looks at the call (autocast, tracing, modes, transforms, subclasses) or there is nothing to differentiate."""
+    if (x.is_cuda and x.dtype == torch.bfloat16 and torch.is_grad_enabled() and not torch.compiler.is_compiling()
+            and not torch.is_autocast_enabled("cuda") and all(w.dtype == x.dtype and w.device == x.device for w in weights)
+            and any(t.requires_grad for t in (x, *weights)) and _plain_autograd((x, *weights))):
+        return _SharedInputLinear.apply(x, *weights)
+    return None
+
+
+def shared_input_linears(x: torch.Tensor, modules):
+    """[m(x) for m in modules]; nn.Linear modules without bias, hooks or a forward of their own as one autograd node."""
+    if (torch.nn.Linear.forward is _LINEAR_FORWARD and not torch.nn.modules.module._has_any_global_hook()
+            and all(type(m) is torch.nn.Linear and "forward" not in m.__dict__ and m.bias is None
+                    and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+                    for m in modules)):
+        outs = _linears(x, [m.weight for m in modules])
+        if outs is not None:
+            return outs
+    return tuple(m(x) for m in modules)
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
+    """F.linear, its weight gradient by nha_wgrad where that is the faster one."""
+    outs = None if bias is not None else _linears(x, [weight])
+    return torch.nn.functional.linear(x, weight, bias) if outs is None else outs[0]
+
+
 @torch.compiler.disable
 def gsa_share(lse_swa: torch.Tensor, lse_gsa: torch.Tensor) -> float:
     """Mean over tokens and heads of e^lse_gsa / (e^lse_swa + e^lse_gsa) (fp32 tensors of one shape): one launch, then one

@@ -1,0 +1,79 @@
+"""nha_wgrad (weight gradients of projections of one input) against the fp64 product, and the layer's shared projections
+against its modules called one by one.  fp32 sums and one rounding to bf16 (8 significant bits), which is 2^-8 of the value at
+most: relative L2 4e-3."""
+import ctypes as C
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# one token; one past a step of 64; columns of one 16-byte piece, around a tile of 256; splits that do not divide the tokens
+@pytest.mark.parametrize("T,width,outs", [(1, 8, [8]), (65, 256, [256, 8]), (777, 520, [264, 248, 8]), (129, 248, [512]),
+                                          (4099, 264, [256, 256, 64, 8]), (20000, 128, [136])])
+def test_wgrad(T, width, outs):
+    from nha_amd.ops import nha_wgrad
+    gen = torch.Generator(device="cuda").manual_seed(T + width)
+    x = torch.randn(T, width, generator=gen, device="cuda").bfloat16()
+    dys = [torch.randn(T, o, generator=gen, device="cuda").bfloat16() for o in outs]
+    for dy, dw in zip(dys, nha_wgrad(x, dys)):
+        ref = dy.double().t() @ x.double()
+        rel = ((dw.double() - ref).norm() / ref.norm()).item()
+        assert rel <= 4e-3, f"{tuple(dw.shape)}: relative L2 error {rel:.3e}"
+
+
+def test_wgrad_refuses():
+    from nha_amd import _lib
+    lib = _lib.load()
+    a = _lib.NhaWgradArgs(n=1, T=64, I=12)
+    a.O[0] = 8
+    assert lib.nha_wgrad_scratch_bytes(C.byref(a)) == 0
+    a.I, a.n = 16, 5
+    assert lib.nha_wgrad_scratch_bytes(C.byref(a)) == 0
+    a.n = 1
+    assert lib.nha_wgrad_scratch_bytes(C.byref(a)) > 0 and lib.nha_wgrad(C.byref(a)) != 0      # no tensors
+
+
+def _layer(**kw):
+    from nha_amd.layer import NativeHybridAttention
+    torch.manual_seed(4)
+    return NativeHybridAttention(hidden_size=256, num_heads=4, num_kv_heads=2, num_slots=64, layer_idx=0, window_size=40,
+                                 **kw).cuda().bfloat16()
+
+
+@pytest.mark.parametrize("case", ["plain", "frozen", "short conv", "strided input"])
+def test_layer_projections(case):
+    layer = _layer(use_short_conv=case == "short conv")
+    x = torch.randn(2, 90, 512 if case == "strided input" else 256, device="cuda").bfloat16()[..., :256].requires_grad_()
+    if case == "frozen":
+        layer.k_proj.weight.requires_grad_(False)
+    leaves = [x, *(p for p in layer.parameters() if p.requires_grad)]
+    dy = torch.randn(2, 90, 256, device="cuda").bfloat16()
+
+    def run():
+        y = layer(x)[0]
+        return y, torch.autograd.grad(y, leaves, dy)
+    y, grads = run()
+    seen = []
+    for m in (layer.q_proj, layer.f_proj):                 # a hook: the modules are called
+        m.register_forward_hook(lambda *a: seen.append(1))
+    y2, grads2 = run()
+    assert len(seen) == 2 and torch.equal(y, y2)
+    for g, r in zip(grads, grads2):
+        # dx adds four products in bf16 one way and inside the products the other: up to four roundings of 2^-8, independent of each other and of one quarter to all of the sum
+        assert g.shape == r.shape and g.dtype == r.dtype
+        assert ((g.double() - r.double()).norm() / r.double().norm()).item() <= 1e-2
+
+
+def test_second_derivative_of_the_projections():
+    from nha_amd.ops import shared_input_linears
+    lin = [torch.nn.Linear(64, o, bias=False).cuda().bfloat16() for o in (32, 16)]
+    x = torch.randn(20, 64, device="cuda").bfloat16().requires_grad_()
+    got, ref = [], []
+    for out, call in ((got, lambda: shared_input_linears(x, lin)), (ref, lambda: [m(x) for m in lin])):
+        a, b = call()
+        dx = torch.autograd.grad((a.float().pow(2).sum() + b.float().pow(2).sum()), x, create_graph=True)[0]
+        out.extend(torch.autograd.grad(dx.float().pow(2).sum(), [x, *(m.weight for m in lin)]))
+    for g, r in zip(got, ref):
+        assert ((g.double() - r.double()).norm() / r.double().norm()).item() <= 1e-2
