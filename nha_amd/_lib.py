@@ -20,6 +20,7 @@ NHA_NOALLOC_SCRATCH_BYTES = 32 << 20   # workspace of nha_prefill_fwd_noalloc (i
 NHA_FMAP_NONE, NHA_FMAP_SWISH, NHA_FMAP_RELU = 0, 1, 2
 
 EXPORTS = (
+    "nha_ring_fill", "nha_wgrad", "nha_wgrad_scratch_bytes", "nha_gsa_share",
     "nha_prefill_scratch_bytes", "nha_prefill_fwd", "nha_prefill_fwd_noalloc", "nha_prefill_bwd_scratch_bytes", "nha_prefill_bwd",
     "nha_decode_scratch_bytes", "nha_decode_step", "nha_decode_advance", "nha_layer_prologue", "nha_layer_epilogue",
     "nha_layer_prologue_bwd", "nha_layer_epilogue_bwd", "nha_layer_epilogue_bwd_parts",

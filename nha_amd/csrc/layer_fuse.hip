@@ -383,22 +383,21 @@ struct EPB {
   void* dout;
   const float* w;
   float *dw_part, *db_part;
-  int rows, dim, rows_wg;
+  int rows, dim;
   float eps;
 };
 
-// rows of a workgroup (and of one row of the partial sums): fewer for small calls, which would leave CUs idle
-__host__ __device__ constexpr int bwd_rows(int rows) { return rows <= 8192 ? 8 : 32; }
+constexpr int BWD_ROWS = 32;   // rows per workgroup (one partial weight gradient each)
 
-// Backward of y = silu(o) * rstd * w + b, dim <= 512 NV: one wave per row, the rows of a workgroup dealt to its four waves,
+// Backward of y = silu(o) * rstd * w + b, dim <= 512 NV: one wave per row, the rows of a workgroup dealt to its NW waves,
 // the next row's two reads requested before this row's sums are formed.  Lane l owns the columns (64 n + l) * 8 .. + 8 of
 // every row; the waves' shares of the weight and bias gradients are added through LDS in a fixed order.
 // Bound: HBM (o, dy in, do out).  With the row spread over a workgroup every row was two barriers and a memory latency,
-// 1.4 us, and half the threads idle at dim = 1024: 1400 rows of 1024 44 -> 9 us, 16384 rows 47 -> 21 us;
-// 16384 rows of 2048 66 -> 51 us.
-template <typename T, int NV>
-__global__ __launch_bounds__(256) void layer_epilogue_bwd_wave_kernel(EPB p) {
-  extern __shared__ float sums[];   // [3 waves][dw, db][dim]
+// 1.4 us, and half the threads idle at dim = 1024: 1400 rows of 1024 44 -> 13 us, 16384 rows 47 -> 25 us;
+// 700 rows of 2048 43 -> 25 us, 16384 rows 66 -> 52 us.
+template <typename T, int NV, int NW>
+__global__ __launch_bounds__(64 * NW) void layer_epilogue_bwd_wave_kernel(EPB p) {
+  extern __shared__ float sums[];   // [NW - 1 waves][dw, db][dim]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float w[NV][8], dw[NV][8], db[NV][8];
   Raw<T, 8> xn[NV], dn[NV];
@@ -409,8 +408,8 @@ __global__ __launch_bounds__(256) void layer_epilogue_bwd_wave_kernel(EPB p) {
     for (int e = 0; e < 8; ++e) w[n][e] = 1.f, dw[n][e] = 0.f, db[n][e] = 0.f;
     if (p.w && u < p.dim) ldv<float, 8>(p.w + u, w[n]);
   }
-  const int r0 = blockIdx.x * p.rows_wg;
-  const int r1 = r0 + p.rows_wg < p.rows ? r0 + p.rows_wg : p.rows;
+  const int r0 = blockIdx.x * BWD_ROWS;
+  const int r1 = r0 + BWD_ROWS < p.rows ? r0 + BWD_ROWS : p.rows;
   auto request = [&](int r) {
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
@@ -422,7 +421,7 @@ __global__ __launch_bounds__(256) void layer_epilogue_bwd_wave_kernel(EPB p) {
     }
   };
   request(r0 + wave);
-  for (int r = r0 + wave; r < r1; r += 4) {
+  for (int r = r0 + wave; r < r1; r += NW) {
     float ss = 0.f, dot = 0.f, a[NV][8], x[NV][8], d[NV][8];
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
@@ -432,7 +431,7 @@ __global__ __launch_bounds__(256) void layer_epilogue_bwd_wave_kernel(EPB p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[n][e] = d[n][e] = 0.f;
     }
-    request(r + 4);
+    request(r + NW);
 #pragma unroll
     for (int n = 0; n < NV; ++n)
 #pragma unroll
@@ -473,7 +472,7 @@ __global__ __launch_bounds__(256) void layer_epilogue_bwd_wave_kernel(EPB p) {
   for (int n = 0; n < NV; ++n) {
     const int u = (64 * n + lane) * 8;
     if (u >= p.dim) continue;
-    for (int k = 0; k < 3; ++k)
+    for (int k = 0; k < NW - 1; ++k)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         dw[n][e] += sums[(size_t)(2 * k) * p.dim + u + e];
@@ -500,8 +499,8 @@ __global__ __launch_bounds__(256) void layer_epilogue_bwd_kernel(EPB p) {
     for (int e = 0; e < 8; ++e) w[n][e] = 1.f, dw[n][e] = 0.f, db[n][e] = 0.f;
     if (p.w && u < p.dim) ldv<float, 8>(p.w + u, w[n]);
   }
-  const int r0 = blockIdx.x * p.rows_wg;
-  for (int rr = 0; rr < p.rows_wg; ++rr) {
+  const int r0 = blockIdx.x * BWD_ROWS;
+  for (int rr = 0; rr < BWD_ROWS; ++rr) {
     const int r = r0 + rr;
     if (r >= p.rows) break;  // uniform over the workgroup
     const T* src = (const T*)p.o + (size_t)r * p.dim;
@@ -577,10 +576,10 @@ __global__ __launch_bounds__(256) void gsa_share_kernel(const float* __restrict_
 
 template <typename T>
 int launch_epilogue_bwd(const EPB& p, hipStream_t st) {
-  const dim3 grid((p.rows + p.rows_wg - 1) / p.rows_wg);
-  const size_t lds = (size_t)6 * p.dim * sizeof(float);   // at most 48 KB
-  if (p.dim <= 1024) hipLaunchKernelGGL((layer_epilogue_bwd_wave_kernel<T, 2>), grid, dim3(256), lds, st, p);
-  else if (p.dim <= 2048) hipLaunchKernelGGL((layer_epilogue_bwd_wave_kernel<T, 4>), grid, dim3(256), lds, st, p);
+  const dim3 grid((p.rows + BWD_ROWS - 1) / BWD_ROWS);
+  // LDS of the waves' sums: at most 56 and 48 KB
+  if (p.dim <= 1024) hipLaunchKernelGGL((layer_epilogue_bwd_wave_kernel<T, 2, 8>), grid, dim3(512), (size_t)14 * p.dim * sizeof(float), st, p);
+  else if (p.dim <= 2048) hipLaunchKernelGGL((layer_epilogue_bwd_wave_kernel<T, 4, 4>), grid, dim3(256), (size_t)6 * p.dim * sizeof(float), st, p);
   else if (p.dim <= 4096) hipLaunchKernelGGL((layer_epilogue_bwd_kernel<T, 2>), grid, dim3(256), 0, st, p);
   else hipLaunchKernelGGL((layer_epilogue_bwd_kernel<T, 4>), grid, dim3(256), 0, st, p);
   return 0;
@@ -913,7 +912,7 @@ int layer_prologue_bwd_impl(const NhaLayerPrologueBwdArgs* a) {
   return NHA_OK;
 }
 
-int layer_epilogue_bwd_parts(int rows) { return (rows + bwd_rows(rows) - 1) / bwd_rows(rows); }
+int layer_epilogue_bwd_parts(int rows) { return (rows + BWD_ROWS - 1) / BWD_ROWS; }
 
 int gsa_share_impl(const float* swa, const float* gsa, int64_t n, float* part, int parts, void* stream) {
   hipLaunchKernelGGL(gsa_share_kernel, dim3(parts), dim3(256), 0, (hipStream_t)stream, swa, gsa, n, part);
@@ -962,7 +961,7 @@ int layer_epilogue_bwd_impl(const NhaLayerEpilogueBwdArgs* a) {
   }
   EPB p;
   p.o = a->o; p.dy = a->dy; p.dout = a->dout; p.w = a->weight; p.dw_part = a->dweight_partial; p.db_part = a->dbias_partial;
-  p.rows = a->rows; p.dim = a->dim; p.rows_wg = bwd_rows(a->rows); p.eps = a->eps;
+  p.rows = a->rows; p.dim = a->dim; p.eps = a->eps;
   hipStream_t st = (hipStream_t)a->stream;
   if (a->dtype == NHA_DTYPE_BF16) launch_epilogue_bwd<bf16_t>(p, st);
   else launch_epilogue_bwd<float>(p, st);

@@ -7,7 +7,7 @@ import torch.nn.functional as F
 pytestmark = pytest.mark.gpu
 
 
-# one row; a ragged group; dims at the edges of 512 columns per step; both sides of 8192 rows (8 and 32 rows per group)
+# one row; a ragged group; dims at the edges of 512 columns per step and of 1024 (eight waves or four); many groups
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rows,dim", [(1, 8), (9, 512), (45, 520), (8192, 64), (8195, 1024), (61, 1032), (70, 2048), (8225, 1544)])
 def test_epilogue_backward_rows(dtype, rows, dim):
