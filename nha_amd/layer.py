@@ -22,7 +22,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops as _ops
-from .ops import chunk_nha, gsa_share, linear, nha_layer_epilogue, nha_layer_prologue, shared_input_linears
+from .ops import chunk_nha, gsa_share_begin, gsa_share_end, linear, nha_layer_epilogue, nha_layer_prologue, shared_input_linears
 
 
 class RMSNorm(nn.Module):
@@ -335,6 +335,7 @@ class NativeHybridAttention(nn.Module):
             # rotary on the kv-head keys: identical across the heads of a group, so rotating before the
             # (implicit, in-kernel) group expansion equals the reference's repeat-then-rotate
             q_swa, k_swa = self.rotary(q, k, seqlen_offset=seqlen_offset, cu_seqlens=cu_seqlens)
+        share = None
         if mode == 'chunk':
             output, lse_swa, lse_gsa = chunk_nha(
                 q_swa=q_swa, k_swa=k_swa, q_gsa=q_gsa, k_gsa=k_gsa, v=v, s=s, g=g,
@@ -348,7 +349,7 @@ class NativeHybridAttention(nn.Module):
             )
             if self.training:
                 if getattr(self._store_compression_stats, '__func__', None) is _STORE_STATS:
-                    self._append_compression_stats(gsa_share(lse_swa, lse_gsa))
+                    share = gsa_share_begin(lse_swa, lse_gsa)     # read below, once the rest of the call is queued
                 else:                                    # a record of the caller's own takes the two weights
                     lse_max = torch.maximum(lse_swa, lse_gsa)
                     w_swa, w_gsa = torch.exp(lse_swa - lse_max), torch.exp(lse_gsa - lse_max)
@@ -374,6 +375,8 @@ class NativeHybridAttention(nn.Module):
                                 eps=self.norm_eps)
         if attention_mask is not None:
             o = pad_input(o.squeeze(0), indices, batch_size, q_len)
+        if share is not None:
+            self._append_compression_stats(gsa_share_end(share))
         return o, None, past_key_values
 
     def _apply_gsa_aux_loss(self, output: torch.Tensor, lse_swa: torch.Tensor, lse_gsa: torch.Tensor):

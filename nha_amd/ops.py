@@ -481,9 +481,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) 
 
 
 @torch.compiler.disable
-def gsa_share(lse_swa: torch.Tensor, lse_gsa: torch.Tensor) -> float:
-    """Mean over tokens and heads of e^lse_gsa / (e^lse_swa + e^lse_gsa) (fp32 tensors of one shape): one launch, then one
-    copy of its partial sums to the host, which adds them."""
+def gsa_share_begin(lse_swa: torch.Tensor, lse_gsa: torch.Tensor):
+    """Starts forming the mean over tokens and heads of e^lse_gsa / (e^lse_swa + e^lse_gsa) (fp32 tensors of one shape) on
+    the current stream: one launch and a copy of its partial sums to the host.  gsa_share_end waits for the value, so work
+    queued between the two runs under the wait."""
     _need_cuda(lse_swa, lse_gsa)
     if lse_swa.dtype != torch.float32 or lse_gsa.dtype != torch.float32 or lse_swa.shape != lse_gsa.shape:
         raise ValueError("gsa_share takes two float32 tensors of one shape")
@@ -491,7 +492,23 @@ def gsa_share(lse_swa: torch.Tensor, lse_gsa: torch.Tensor) -> float:
     n = a.numel()
     part = torch.empty(min(256, (n + 255) // 256), dtype=torch.float32, device=a.device)
     _lib.check(_lib.load().nha_gsa_share(a.data_ptr(), b.data_ptr(), n, part.data_ptr(), part.numel(), _stream(a.device)))
-    return sum(part.tolist()) / n
+    host = torch.empty(part.numel(), dtype=torch.float32, pin_memory=True)
+    host.copy_(part, non_blocking=True)
+    done = torch.cuda.Event()
+    done.record(torch.cuda.current_stream(a.device))
+    return done, host, n
+
+
+@torch.compiler.disable
+def gsa_share_end(pending) -> float:
+    done, host, n = pending
+    done.synchronize()
+    return sum(host.tolist()) / n
+
+
+def gsa_share(lse_swa: torch.Tensor, lse_gsa: torch.Tensor) -> float:
+    """Mean over tokens and heads of e^lse_gsa / (e^lse_swa + e^lse_gsa)."""
+    return gsa_share_end(gsa_share_begin(lse_swa, lse_gsa))
 
 
 def _short_conv_args(x, cu):
