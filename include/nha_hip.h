@@ -478,9 +478,14 @@ int nha_layer_prologue_bwd(const NhaLayerPrologueBwdArgs* a);
 int32_t nha_layer_epilogue_bwd_parts(int32_t rows);
 int nha_layer_epilogue_bwd(const NhaLayerEpilogueBwdArgs* a);
 
+/* The prologue and its backward on q, k, v, f (and dq, dk, dv, df) whose rows lie row_stride elements apart: the columns of
+ * one matrix that a single projection of the input writes.  row_stride: a multiple of 8, no shorter than a row. */
+int nha_layer_prologue_rows(const NhaLayerPrologueArgs* a, int64_t row_stride);
+int nha_layer_prologue_bwd_rows(const NhaLayerPrologueBwdArgs* a, int64_t row_stride);
+
 /* Weight gradients of up to four projections of one input, bf16 with fp32 sums: dw[q] [O[q], I] = dy[q]^T x, x [T, I],
  * dy[q] [T, O[q]], I and O[q] multiples of 8, all 16-byte aligned; rows * I below 2^31.  scratch: at least
- * nha_wgrad_scratch_bytes(a) bytes (0: bad arguments), which reads n, T, I and O only. */
+ * nha_wgrad_scratch_bytes(a) bytes (0: bad arguments), which reads n, T, I, O and ldy only. */
 typedef struct NhaWgradArgs {
   const void* x;
   const void* dy[4];
@@ -490,6 +495,7 @@ typedef struct NhaWgradArgs {
   void* stream;
   int32_t O[4];
   int32_t n, T, I;
+  int32_t ldy;      /* elements between the rows of every dy; 0: O[q] */
 } NhaWgradArgs;
 size_t nha_wgrad_scratch_bytes(const NhaWgradArgs* a);
 int nha_wgrad(const NhaWgradArgs* a);

@@ -20,7 +20,7 @@ NHA_NOALLOC_SCRATCH_BYTES = 32 << 20   # workspace of nha_prefill_fwd_noalloc (i
 NHA_FMAP_NONE, NHA_FMAP_SWISH, NHA_FMAP_RELU = 0, 1, 2
 
 EXPORTS = (
-    "nha_ring_fill", "nha_wgrad", "nha_wgrad_scratch_bytes", "nha_gsa_share",
+    "nha_ring_fill", "nha_wgrad", "nha_wgrad_scratch_bytes", "nha_gsa_share", "nha_layer_prologue_rows", "nha_layer_prologue_bwd_rows",
     "nha_prefill_scratch_bytes", "nha_prefill_fwd", "nha_prefill_fwd_noalloc", "nha_prefill_bwd_scratch_bytes", "nha_prefill_bwd",
     "nha_decode_scratch_bytes", "nha_decode_step", "nha_decode_advance", "nha_layer_prologue", "nha_layer_epilogue",
     "nha_layer_prologue_bwd", "nha_layer_epilogue_bwd", "nha_layer_epilogue_bwd_parts",
@@ -168,7 +168,7 @@ class NhaShortConvBwdArgs(C.Structure):
 class NhaWgradArgs(C.Structure):
     _fields_ = [("x", C.c_void_p), ("dy", C.c_void_p * 4), ("dw", C.c_void_p * 4), ("scratch", C.c_void_p),
                 ("scratch_bytes", C.c_size_t), ("stream", C.c_void_p), ("O", C.c_int32 * 4), ("n", C.c_int32),
-                ("T", C.c_int32), ("I", C.c_int32)]
+                ("T", C.c_int32), ("I", C.c_int32), ("ldy", C.c_int32)]
 
 
 class NhaRingFillArgs(C.Structure):
@@ -243,6 +243,10 @@ def load() -> C.CDLL:
     lib.nha_layer_epilogue_bwd.argtypes = [C.POINTER(NhaLayerEpilogueBwdArgs)]
     lib.nha_layer_epilogue_bwd_parts.restype = C.c_int32
     lib.nha_layer_epilogue_bwd_parts.argtypes = [C.c_int32]
+    lib.nha_layer_prologue_rows.restype = C.c_int
+    lib.nha_layer_prologue_rows.argtypes = [C.POINTER(NhaLayerPrologueArgs), C.c_int64]
+    lib.nha_layer_prologue_bwd_rows.restype = C.c_int
+    lib.nha_layer_prologue_bwd_rows.argtypes = [C.POINTER(NhaLayerPrologueBwdArgs), C.c_int64]
     lib.nha_wgrad_scratch_bytes.restype = C.c_size_t
     lib.nha_wgrad_scratch_bytes.argtypes = [C.POINTER(NhaWgradArgs)]
     lib.nha_wgrad.restype = C.c_int

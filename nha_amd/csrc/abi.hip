@@ -216,7 +216,7 @@ int nha_ring_fill(const NhaRingFillArgs* a) {
   return ring_fill_impl(a);
 }
 
-int nha_layer_prologue(const NhaLayerPrologueArgs* a) {
+static int run_layer_prologue(const NhaLayerPrologueArgs* a, int64_t row_stride) {
   NHA_CHECK_ARG(a != nullptr, "nha_layer_prologue: null args");
   NHA_CHECK_ARG(a->T_tot > 0 && a->N > 0 && a->HQ > 0 && a->H > 0 && a->K > 0 && a->V > 0 && a->M > 0,
                 "nha_layer_prologue: non-positive dimension");
@@ -234,7 +234,17 @@ int nha_layer_prologue(const NhaLayerPrologueArgs* a) {
   const void* ptrs[] = {a->q, a->k, a->v, a->f, a->q_swa, a->k_swa, a->q_gsa, a->k_gsa, a->v_out, a->s, a->g};
   for (const void* p : ptrs)
     NHA_CHECK_ARG((reinterpret_cast<uintptr_t>(p) & 15) == 0, "nha_layer_prologue: tensors must be 16-byte aligned");
-  return layer_prologue_impl(a);
+  const int64_t widest = (int64_t)(a->HQ > a->H ? a->HQ : a->H) * a->K;
+  NHA_CHECK_ARG(row_stride == 0 || (row_stride % 8 == 0 && row_stride >= widest && row_stride >= (int64_t)a->H * a->V && row_stride >= (int64_t)a->H * a->M),
+                "nha_layer_prologue_rows: the row stride must be a multiple of 8 and no shorter than a row");
+  return layer_prologue_impl(a, row_stride);
+}
+
+int nha_layer_prologue(const NhaLayerPrologueArgs* a) { return run_layer_prologue(a, 0); }
+
+int nha_layer_prologue_rows(const NhaLayerPrologueArgs* a, int64_t row_stride) {
+  NHA_CHECK_ARG(row_stride > 0, "nha_layer_prologue_rows: bad row stride");
+  return run_layer_prologue(a, row_stride);
 }
 
 int nha_hybrid_prologue(const NhaHybridPrologueArgs* a) {
@@ -316,7 +326,7 @@ int nha_layer_epilogue(const NhaLayerEpilogueArgs* a) {
   return layer_epilogue_impl(a);
 }
 
-int nha_layer_prologue_bwd(const NhaLayerPrologueBwdArgs* a) {
+static int run_layer_prologue_bwd(const NhaLayerPrologueBwdArgs* a, int64_t row_stride) {
   NHA_CHECK_ARG(a != nullptr, "nha_layer_prologue_bwd: null args");
   NHA_CHECK_ARG(a->T_tot > 0 && a->N > 0 && a->HQ > 0 && a->H > 0 && a->K > 0 && a->V > 0 && a->M > 0,
                 "nha_layer_prologue_bwd: non-positive dimension");
@@ -336,7 +346,17 @@ int nha_layer_prologue_bwd(const NhaLayerPrologueBwdArgs* a) {
                         a->dq, a->dk, a->dv, a->df};
   for (const void* p : ptrs)
     NHA_CHECK_ARG((reinterpret_cast<uintptr_t>(p) & 15) == 0, "nha_layer_prologue_bwd: tensors must be 16-byte aligned");
-  return layer_prologue_bwd_impl(a);
+  const int64_t widest = (int64_t)(a->HQ > a->H ? a->HQ : a->H) * a->K;
+  NHA_CHECK_ARG(row_stride == 0 || (row_stride % 8 == 0 && row_stride >= widest && row_stride >= (int64_t)a->H * a->V && row_stride >= (int64_t)a->H * a->M),
+                "nha_layer_prologue_bwd_rows: the row stride must be a multiple of 8 and no shorter than a row");
+  return layer_prologue_bwd_impl(a, row_stride);
+}
+
+int nha_layer_prologue_bwd(const NhaLayerPrologueBwdArgs* a) { return run_layer_prologue_bwd(a, 0); }
+
+int nha_layer_prologue_bwd_rows(const NhaLayerPrologueBwdArgs* a, int64_t row_stride) {
+  NHA_CHECK_ARG(row_stride > 0, "nha_layer_prologue_bwd_rows: bad row stride");
+  return run_layer_prologue_bwd(a, row_stride);
 }
 
 int32_t nha_layer_epilogue_bwd_parts(int32_t rows) { return rows > 0 ? layer_epilogue_bwd_parts(rows) : 0; }
@@ -366,6 +386,8 @@ static int check_wgrad(const NhaWgradArgs* a, bool pointers) {
     }
   }
   NHA_CHECK_ARG(rows * a->I < ((int64_t)1 << 31), "nha_wgrad: the weights are too large");
+  for (int q = 0; q < a->n; ++q)
+    NHA_CHECK_ARG(a->ldy == 0 || (a->ldy >= a->O[q] && a->ldy % 8 == 0), "nha_wgrad: ldy must be a multiple of 8 and no shorter than a row");
   if (pointers) {
     NHA_CHECK_ARG(a->x && a->scratch, "nha_wgrad: x and scratch are required");
     NHA_CHECK_ARG(((reinterpret_cast<uintptr_t>(a->x) | reinterpret_cast<uintptr_t>(a->scratch)) & 15) == 0,

@@ -127,9 +127,9 @@ static inline int next_pow2_i(int x) {
 // host-side error plumbing (thread-local message)
 void set_error(const char* fmt, ...);
 
-int layer_prologue_impl(const NhaLayerPrologueArgs* a);
+int layer_prologue_impl(const NhaLayerPrologueArgs* a, int64_t row_stride);
 int layer_epilogue_impl(const NhaLayerEpilogueArgs* a);
-int layer_prologue_bwd_impl(const NhaLayerPrologueBwdArgs* a);
+int layer_prologue_bwd_impl(const NhaLayerPrologueBwdArgs* a, int64_t row_stride);
 int layer_epilogue_bwd_parts(int rows);
 size_t wgrad_scratch_bytes(const NhaWgradArgs* a);
 int wgrad_impl(const NhaWgradArgs* a);

@@ -18,6 +18,7 @@ struct LP {
   const float* inv_freq;
   const int32_t* cu;
   int T_tot, N, T, HQ, H, K, V, M, fm, off;
+  int64_t lq, lk, lv, lf;   // elements between the rows of q, k, v, f and of their gradients
   float inv_norm;
   // backward only: cotangents of the seven outputs, gradients of the four inputs
   const void *dq_swa, *dk_swa, *dq_gsa, *dk_gsa, *dv_out, *ds, *dg;
@@ -146,11 +147,11 @@ __global__ __launch_bounds__(256) void layer_prologue_kernel(LP p) {
   const int t = token_angles(p, cs, wave, lane, &live);
   if (!live) return;
   const size_t tq = (size_t)t * p.HQ * p.K, tk = (size_t)t * p.H * p.K;
-  rope_rows<T, VEC>((const T*)p.q + tq, (T*)p.q_swa + tq, p.q_gsa ? (T*)p.q_gsa + tq : nullptr, p.HQ, p.K, cs, p.fm, lane);
-  rope_rows<T, VEC>((const T*)p.k + tk, (T*)p.k_swa + tk, p.k_gsa ? (T*)p.k_gsa + tk : nullptr, p.H, p.K, cs, p.fm, lane);
+  rope_rows<T, VEC>((const T*)p.q + (size_t)t * p.lq, (T*)p.q_swa + tq, p.q_gsa ? (T*)p.q_gsa + tq : nullptr, p.HQ, p.K, cs, p.fm, lane);
+  rope_rows<T, VEC>((const T*)p.k + (size_t)t * p.lk, (T*)p.k_swa + tk, p.k_gsa ? (T*)p.k_gsa + tk : nullptr, p.H, p.K, cs, p.fm, lane);
   {
     const int n = p.H * p.V;
-    const T* src = (const T*)p.v + (size_t)t * n;
+    const T* src = (const T*)p.v + (size_t)t * p.lv;
     T* dst = (T*)p.v_out + (size_t)t * n;
     for (int u = lane * VEC; u < n; u += 64 * VEC) {
       float x[VEC];
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(256) void layer_prologue_kernel(LP p) {
   }
   {
     const int n = p.H * p.M;
-    const T* src = (const T*)p.f + (size_t)t * n;
+    const T* src = (const T*)p.f + (size_t)t * p.lf;
     T* dg = (T*)p.g + (size_t)t * n;
     T* ds = (T*)p.s + (size_t)t * n;
     for (int u = lane * VEC; u < n; u += 64 * VEC) {
@@ -233,15 +234,15 @@ __global__ __launch_bounds__(256) void layer_prologue_bwd_kernel(LP p) {
   const int t = token_angles(p, cs, wave, lane, &live);
   if (!live) return;
   const size_t tq = (size_t)t * p.HQ * p.K, tk = (size_t)t * p.H * p.K;
-  rope_rows_bwd<T, VEC>((const T*)p.q + tq, (const T*)p.dq_swa + tq, p.dq_gsa ? (const T*)p.dq_gsa + tq : nullptr,
-                        (T*)p.dq + tq, p.HQ, p.K, cs, p.fm, lane);
-  rope_rows_bwd<T, VEC>((const T*)p.k + tk, (const T*)p.dk_swa + tk, p.dk_gsa ? (const T*)p.dk_gsa + tk : nullptr,
-                        (T*)p.dk + tk, p.H, p.K, cs, p.fm, lane);
+  rope_rows_bwd<T, VEC>((const T*)p.q + (size_t)t * p.lq, (const T*)p.dq_swa + tq, p.dq_gsa ? (const T*)p.dq_gsa + tq : nullptr,
+                        (T*)p.dq + (size_t)t * p.lq, p.HQ, p.K, cs, p.fm, lane);
+  rope_rows_bwd<T, VEC>((const T*)p.k + (size_t)t * p.lk, (const T*)p.dk_swa + tk, p.dk_gsa ? (const T*)p.dk_gsa + tk : nullptr,
+                        (T*)p.dk + (size_t)t * p.lk, p.H, p.K, cs, p.fm, lane);
   {
     const int n = p.H * p.V;
-    const T* src = (const T*)p.v + (size_t)t * n;
+    const T* src = (const T*)p.v + (size_t)t * p.lv;
     const T* dsrc = (const T*)p.dv_out + (size_t)t * n;
-    T* dst = (T*)p.dv + (size_t)t * n;
+    T* dst = (T*)p.dv + (size_t)t * p.lv;
     for (int u = lane * VEC; u < n; u += 64 * VEC) {
       float x[VEC], d[VEC];
       ldv<T, VEC>(src + u, x);
@@ -254,10 +255,10 @@ __global__ __launch_bounds__(256) void layer_prologue_bwd_kernel(LP p) {
   {
     // g = logsigmoid(f)/n, s = 1 - exp(g):  df = (dg - ds * exp(g)) / n * sigmoid(-f)
     const int n = p.H * p.M;
-    const T* src = (const T*)p.f + (size_t)t * n;
+    const T* src = (const T*)p.f + (size_t)t * p.lf;
     const T* pdg = (const T*)p.dg + (size_t)t * n;
     const T* pds = (const T*)p.ds + (size_t)t * n;
-    T* dst = (T*)p.df + (size_t)t * n;
+    T* dst = (T*)p.df + (size_t)t * p.lf;
     for (int u = lane * VEC; u < n; u += 64 * VEC) {
       float x[VEC], dg[VEC], ds[VEC];
       ldv<T, VEC>(src + u, x);
@@ -863,7 +864,7 @@ int launch_short_conv(const SC& p, int KS, bool bwd, hipStream_t st) {
 
 }  // namespace
 
-int layer_prologue_impl(const NhaLayerPrologueArgs* a) {
+int layer_prologue_impl(const NhaLayerPrologueArgs* a, int64_t row_stride) {
   LP p = {};
   p.q = a->q; p.k = a->k; p.v = a->v; p.f = a->f;
   p.q_swa = a->q_swa; p.k_swa = a->k_swa;
@@ -876,6 +877,10 @@ int layer_prologue_impl(const NhaLayerPrologueArgs* a) {
   p.HQ = a->HQ; p.H = a->H; p.K = a->K; p.V = a->V; p.M = a->M;
   p.fm = a->feature_map; p.off = a->seqlen_offset;
   p.inv_norm = 1.f / a->gate_logit_normalizer;
+  p.lq = row_stride ? row_stride : (int64_t)a->HQ * a->K;
+  p.lk = row_stride ? row_stride : (int64_t)a->H * a->K;
+  p.lv = row_stride ? row_stride : (int64_t)a->H * a->V;
+  p.lf = row_stride ? row_stride : (int64_t)a->H * a->M;
   hipStream_t st = (hipStream_t)a->stream;
   if (a->dtype == NHA_DTYPE_BF16) launch_prologue<bf16_t>(p, st);
   else launch_prologue<float>(p, st);
@@ -887,7 +892,7 @@ int layer_prologue_impl(const NhaLayerPrologueArgs* a) {
   return NHA_OK;
 }
 
-int layer_prologue_bwd_impl(const NhaLayerPrologueBwdArgs* a) {
+int layer_prologue_bwd_impl(const NhaLayerPrologueBwdArgs* a, int64_t row_stride) {
   LP p = {};
   p.q = a->q; p.k = a->k; p.v = a->v; p.f = a->f;
   p.dq_swa = a->dq_swa; p.dk_swa = a->dk_swa;
@@ -901,6 +906,10 @@ int layer_prologue_bwd_impl(const NhaLayerPrologueBwdArgs* a) {
   p.HQ = a->HQ; p.H = a->H; p.K = a->K; p.V = a->V; p.M = a->M;
   p.fm = a->feature_map; p.off = a->seqlen_offset;
   p.inv_norm = 1.f / a->gate_logit_normalizer;
+  p.lq = row_stride ? row_stride : (int64_t)a->HQ * a->K;
+  p.lk = row_stride ? row_stride : (int64_t)a->H * a->K;
+  p.lv = row_stride ? row_stride : (int64_t)a->H * a->V;
+  p.lf = row_stride ? row_stride : (int64_t)a->H * a->M;
   hipStream_t st = (hipStream_t)a->stream;
   if (a->dtype == NHA_DTYPE_BF16) launch_prologue_bwd<bf16_t>(p, st);
   else launch_prologue_bwd<float>(p, st);

@@ -29,6 +29,7 @@ struct WG {
   const bf16_t* dy[4];
   bf16_t* dw[4];
   int O[4], row0[4], tile0[4];   // first row of each output among all of them, first of its column tiles
+  int ldy[4];
   int n, T, I, otiles, itiles, split, tsplit, rows;
   float* part;                   // [split][rows][I]
 };
@@ -44,7 +45,7 @@ __global__ __launch_bounds__(NTHR, 2) void wgrad_kernel(const WG p) {
   const int it = v % p.itiles, ot = (v / p.itiles) % p.otiles, sp = v / (p.itiles * p.otiles);
   int q = 0;
   while (q + 1 < p.n && ot >= p.tile0[q + 1]) ++q;
-  const int O = p.O[q], o0 = (ot - p.tile0[q]) * TW, i0 = it * TW;
+  const int O = p.O[q], ldy = p.ldy[q], o0 = (ot - p.tile0[q]) * TW, i0 = it * TW;
   const int t0 = sp * p.tsplit, t1 = t0 + p.tsplit < p.T ? t0 + p.tsplit : p.T;
   const int steps = (t1 - t0 + TK - 1) / TK;   // every split holds tokens
   const bf16_t* const xs = p.x + i0;
@@ -59,7 +60,7 @@ __global__ __launch_bounds__(NTHR, 2) void wgrad_kernel(const WG p) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         rx[u] = *reinterpret_cast<const uint4*>(xs + (int64_t)(ts + 16 * u + row) * p.I + col);
-        ry[u] = *reinterpret_cast<const uint4*>(ys + (int64_t)(ts + 16 * u + row) * O + col);
+        ry[u] = *reinterpret_cast<const uint4*>(ys + (int64_t)(ts + 16 * u + row) * ldy + col);
       }
     } else {
 #pragma unroll
@@ -67,7 +68,7 @@ __global__ __launch_bounds__(NTHR, 2) void wgrad_kernel(const WG p) {
         const int t = ts + 16 * u + row;
         rx[u] = ry[u] = make_uint4(0, 0, 0, 0);
         if (t < t1 && i0 + col < p.I) rx[u] = *reinterpret_cast<const uint4*>(xs + (int64_t)t * p.I + col);
-        if (t < t1 && o0 + col < O) ry[u] = *reinterpret_cast<const uint4*>(ys + (int64_t)t * O + col);
+        if (t < t1 && o0 + col < O) ry[u] = *reinterpret_cast<const uint4*>(ys + (int64_t)t * ldy + col);
       }
     }
   };
@@ -161,6 +162,7 @@ int plan(const NhaWgradArgs* a, WG& p) {
   p.otiles = p.rows = 0;
   for (int q = 0; q < a->n; ++q) {
     p.O[q] = a->O[q];
+    p.ldy[q] = a->ldy ? a->ldy : a->O[q];
     p.row0[q] = p.rows;
     p.tile0[q] = p.otiles;
     p.rows += a->O[q];

@@ -22,7 +22,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops as _ops
-from .ops import chunk_nha, gsa_share_begin, gsa_share_end, linear, nha_layer_epilogue, nha_layer_prologue, shared_input_linears
+from .ops import chunk_nha, gsa_share_begin, gsa_share_end, layer_front_supported, linear, nha_layer_epilogue, nha_layer_prologue, \
+    shared_input_linears
 
 
 class RMSNorm(nn.Module):
@@ -301,27 +302,37 @@ class NativeHybridAttention(nn.Module):
             indices, cu_seqlens, max_seqlen = get_unpad_data(attention_mask[:, -q_len:])
             hidden_states = hidden_states.reshape(batch_size * q_len, -1)[indices].unsqueeze(0)
         conv_state_q = conv_state_k = conv_state_v = None
-        q, k, v, f = shared_input_linears(hidden_states, (self.q_proj, self.k_proj, self.v_proj, self.f_proj))
-        if self.use_short_conv:
-            if last_state is not None:
-                conv_state_q, conv_state_k, conv_state_v = last_state['conv_state']
-            q, conv_state_q = self.q_conv1d(q, conv_state_q, use_cache, cu_seqlens)
-            k, conv_state_k = self.k_conv1d(k, conv_state_k, use_cache, cu_seqlens)
-            v, conv_state_v = self.v_conv1d(v, conv_state_v, use_cache, cu_seqlens)
-        q = q.unflatten(-1, (-1, self.head_k_dim))
-        k = k.unflatten(-1, (-1, self.head_k_dim))
-        v = v.unflatten(-1, (-1, self.head_v_dim))
-        f = f.unflatten(-1, (-1, self.num_slots))
         seqlen_offset = 0
         if last_state is not None and 'seqlen_offset' in last_state:
             seqlen_offset = last_state['seqlen_offset']
-        fused = self._fused_glue(q) and f.dtype == q.dtype
+        projections = (self.q_proj, self.k_proj, self.v_proj, self.f_proj)
+        dims = (self.num_heads, self.num_kv_heads, self.head_k_dim, self.head_v_dim, self.num_slots)
+        # projections and prologue as one node: training, plain modules, nothing between the two
+        front = (not self.use_short_conv and self.feature_map is not None and self._fused_glue(hidden_states)
+                 and layer_front_supported(hidden_states, projections, dims))
+        fused = front
+        if not fused:
+            q, k, v, f = shared_input_linears(hidden_states, projections)
+            if self.use_short_conv:
+                if last_state is not None:
+                    conv_state_q, conv_state_k, conv_state_v = last_state['conv_state']
+                q, conv_state_q = self.q_conv1d(q, conv_state_q, use_cache, cu_seqlens)
+                k, conv_state_k = self.k_conv1d(k, conv_state_k, use_cache, cu_seqlens)
+                v, conv_state_v = self.v_conv1d(v, conv_state_v, use_cache, cu_seqlens)
+            q = q.unflatten(-1, (-1, self.head_k_dim))
+            k = k.unflatten(-1, (-1, self.head_k_dim))
+            v = v.unflatten(-1, (-1, self.head_v_dim))
+            f = f.unflatten(-1, (-1, self.num_slots))
+            fused = self._fused_glue(q) and f.dtype == q.dtype
         if fused:
-            if self._inv_freq is None or self._inv_freq.device != q.device:
-                self._inv_freq = self.rotary.inv_freq(q.device)
+            device = hidden_states.device
+            if self._inv_freq is None or self._inv_freq.device != device:
+                self._inv_freq = self.rotary.inv_freq(device)
             fm = None if self.feature_map is None else ('swish' if isinstance(self.feature_map, SwishFeatureMap) else 'relu')
+            source = dict(q=None, k=None, v=None, f=None, projections=(hidden_states, projections, dims)) if front \
+                else dict(q=q, k=k, v=v, f=f)
             q_swa, k_swa, q_gsa, k_gsa, v, s, g = nha_layer_prologue(
-                q, k, v, f, self._inv_freq, feature_map=fm, gate_logit_normalizer=self.gate_logit_normalizer,
+                **source, inv_freq=self._inv_freq, feature_map=fm, gate_logit_normalizer=self.gate_logit_normalizer,
                 seqlen_offset=seqlen_offset, cu_seqlens=cu_seqlens)
         else:
             if self.feature_map is not None:

@@ -23,6 +23,14 @@ def test_wgrad(T, width, outs):
         assert rel <= 4e-3, f"{tuple(dw.shape)}: relative L2 error {rel:.3e}"
 
 
+def test_wgrad_row_stride():
+    from nha_amd.ops import nha_wgrad
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    x, both = (torch.randn(333, n, generator=gen, device="cuda").bfloat16() for n in (72, 344))
+    dense = nha_wgrad(x, [both[:, :264].contiguous(), both[:, 264:].contiguous()])
+    assert all(torch.equal(a, b) for a, b in zip(dense, nha_wgrad(x, [both[:, :264], both[:, 264:]])))
+
+
 def test_wgrad_refuses():
     from nha_amd import _lib
     lib = _lib.load()
@@ -42,24 +50,28 @@ def _layer(**kw):
                                  **kw).cuda().bfloat16()
 
 
-@pytest.mark.parametrize("case", ["plain", "frozen", "short conv", "strided input"])
+@pytest.mark.parametrize("case", ["plain", "frozen", "short conv", "strided input", "padding mask", "frozen input"])
 def test_layer_projections(case):
     layer = _layer(use_short_conv=case == "short conv")
     x = torch.randn(2, 90, 512 if case == "strided input" else 256, device="cuda").bfloat16()[..., :256].requires_grad_()
     if case == "frozen":
         layer.k_proj.weight.requires_grad_(False)
-    leaves = [x, *(p for p in layer.parameters() if p.requires_grad)]
+    if case == "frozen input":
+        x = x.detach()
+    kw = dict(attention_mask=(torch.arange(90)[None] >= torch.tensor([[0], [27]])).cuda()) if case == "padding mask" else {}
+    leaves = [t for t in (x, *layer.parameters()) if t.requires_grad]
     dy = torch.randn(2, 90, 256, device="cuda").bfloat16()
 
     def run():
-        y = layer(x)[0]
+        y = layer(x, **kw)[0]
         return y, torch.autograd.grad(y, leaves, dy)
     y, grads = run()
     seen = []
     for m in (layer.q_proj, layer.f_proj):                 # a hook: the modules are called
         m.register_forward_hook(lambda *a: seen.append(1))
     y2, grads2 = run()
-    assert len(seen) == 2 and torch.equal(y, y2)
+    # one product or four: the same sums in another order, one rounding of 2^-8 in q, k, v and f
+    assert len(seen) == 2 and ((y.double() - y2.double()).norm() / y2.double().norm()).item() <= 1e-2
     for g, r in zip(grads, grads2):
         # dx adds four products in bf16 one way and inside the products the other: up to four roundings of 2^-8, independent of each other and of one quarter to all of the sum
         assert g.shape == r.shape and g.dtype == r.dtype
