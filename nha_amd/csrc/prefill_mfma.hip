@@ -554,31 +554,31 @@ __global__ __launch_bounds__(256) void state_apply_kernel(const MP p) {
 // ==========================================================================================
 // One workgroup = one 64-row chunk x G query heads of one kv-head; its NW waves split the
 // 64 x G query rows into RQB blocks of 16 rows per wave.  Window K/V stream through four LDS
-// buffers of TK keys (two K, two V, double buffered); TK = 64 for G > 1 at D <= 128, else 32.
+// buffers of TK keys (two K, two V, double buffered), TK = 64 or 32 (run_mfma).
 // The slot branch runs first on the same buffers: its four 64-row operand tiles (transposed
 // chunk-start k-state, k_gsa rows, chunk-start v-state, v rows) fit at once when TK = 64 and
 // in two stages when TK = 32.  The decay factors s_j[m] exp(gr[m] - gc_j[m]) that every wave
-// needs are computed once per workgroup into LDS, already in MFMA fragment order (G > 1).
+// needs are computed once per workgroup into LDS, already in MFMA fragment order; OWN: by the wave that uses them.
 
-// With one head per workgroup every wave owns one sub-block of query rows and no fragment is used by two waves: each
-// forms its own in registers, and the 44 KB that hold them otherwise let a second workgroup onto the CU.
-template <int D, int TK, int G>
+// OWN: with four waves per head every wave owns one sub-block of query rows and shares its fragments with the waves of the
+// other heads at most: each forms its own in registers, and the 44 KB that hold them otherwise let a second workgroup onto
+// the CU (two heads: at 128 registers, four waves per SIMD).
+template <int D, int TK, bool OWN>
 struct OutSmem {
   static constexpr int LDT = D + 16;
   static constexpr size_t tile_bytes = (size_t)TK * LDT * 2;
   static constexpr size_t bytes =
-      4 * tile_bytes + (size_t)BT * GLD * 4 + (size_t)BT * SLD * 2 + (G > 1 ? (size_t)(NSEA + NSEB) * 512 * 2 : 0);
+      4 * tile_bytes + (size_t)BT * GLD * 4 + (size_t)BT * SLD * 2 + (OWN ? 0 : (size_t)(NSEA + NSEB) * 512 * 2);
 };
 
 
-template <int D, int G, int NW, int TK>
-__global__ __launch_bounds__(64 * NW, G == 1 ? 2 : 1) void mfma_out_kernel(const MP p) {
+template <int D, int G, int NW, int TK, bool OWN>
+__global__ __launch_bounds__(64 * NW, OWN ? NW / 2 : 1) void mfma_out_kernel(const MP p) {
   constexpr int NTHR = 64 * NW;      // threads per workgroup
   constexpr int WPU = NW / G;        // waves per (chunk, head)
   constexpr int RQB = 4 / WPU;       // 16-row query blocks per wave
   static_assert(WPU >= 1 && WPU <= 4 && RQB * WPU == 4, "bad wave split");
   static_assert(TK == 64 || TK == 32, "bad tile size");
-  constexpr bool OWN = G == 1;       // decay fragments formed by the wave that uses them
   static_assert(!OWN || RQB == 1, "a wave's own fragments serve one sub-block");
   constexpr int KS = D / 32;
   constexpr int DB = D / 16;
@@ -1274,17 +1274,17 @@ int launch_repair(const MP& p, hipStream_t st) {
   return NHA_OK;
 }
 
-template <int D, int G, int NW, int TK>
+template <int D, int G, int NW, int TK, bool OWN>
 int launch_out(const MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  const size_t lds = OutSmem<D, TK, G>::bytes;
-  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)mfma_out_kernel<D, G, NW, TK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+  const size_t lds = OutSmem<D, TK, OWN>::bytes;
+  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)mfma_out_kernel<D, G, NW, TK, OWN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL((mfma_out_kernel<D, G, NW, TK>), dim3(p.H * (p.NG / G), p.NT), dim3(64 * NW), lds, st, p);
+  hipLaunchKernelGGL((mfma_out_kernel<D, G, NW, TK, OWN>), dim3(p.H * (p.NG / G), p.NT), dim3(64 * NW), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma output pass)");
   return NHA_OK;
 }
@@ -1341,8 +1341,9 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
     // register file and LDS.  One head (G = 1): 32-key tiles, four waves and two (D = 128) or three
     // (D = 64) workgroups per CU, which 64-key tiles or decay fragments in LDS do not leave room for:
     // 16 heads, 8192 tokens, W = 2048: D = 64 291 -> 147 us, D = 128 434 -> 269 us (with 64-key tiles 165, 375);
-    // 5003 packed tokens, W = 300: 93 -> 46, 119 -> 70.  Two heads of a pair as two such workgroups tie with
-    // G = 2 (8 / 4 heads of 128: 64 against 67 us at W = 150, 407 against 379 at W = 1500)
+    // 5003 packed tokens, W = 300: 93 -> 46, 119 -> 70.  G = 2: where there is more than a workgroup for
+    // every CU, two fit one as well (8 / 4 heads, 4 x 8000 tokens, W = 1500: D = 128 378 -> 330-353 us, with 32-key tiles; D = 64
+    // 244 -> 198); below, one with the fragments shared is faster (3000 tokens, 188 workgroups: 25 against 31, 17.5 against 19)
     int rc;
 #ifdef NHA_AB_SWITCHES   // measurement builds only (-DNHA_AB_SWITCHES): run the kernels the LDS-direct ones replaced
     static const bool ring_off = getenv("NHA_PREFILL_NO_RING") != nullptr;
@@ -1354,12 +1355,13 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
     } else if (!ring_off && prefill_ring256_supported(p, D)) {
       rc = prefill_ring256_launch(p, st);
     } else if constexpr (D <= 128) {
-      if (p.NG % 4 == 0) rc = launch_out<D, 4, 8, 64>(p, st);
-      else if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 64>(p, st);
-      else rc = launch_out<D, 1, 4, 32>(p, st);
+      if (p.NG % 4 == 0) rc = launch_out<D, 4, 8, 64, false>(p, st);
+      else if (p.NG % 2 == 0 && (int64_t)p.HQ / 2 * p.NT > 256) rc = launch_out<D, 2, 8, D == 128 ? 32 : 64, true>(p, st);
+      else if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 64, false>(p, st);
+      else rc = launch_out<D, 1, 4, 32, true>(p, st);
     } else {
-      if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 32>(p, st);
-      else rc = launch_out<D, 1, 4, 32>(p, st);
+      if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 32, false>(p, st);
+      else rc = launch_out<D, 1, 4, 32, true>(p, st);
     }
     if (rc != NHA_OK) return rc;
     return launch_repair<D>(p, st);

@@ -1,6 +1,7 @@
 """Rules that pick a split by the size of the call, on both sides of each line: chunks per segment of the bf16 state pass
-(1 to 8), key groups of the window's dk / dv (64 per workgroup below, 128 or 256 above), against the fp32 kernels, which
-share no code with them.  The bf16 kernels see the same rounded inputs, so the tolerances are those of the parity tests:
+(1 to 8), key groups of the window's dk / dv (64 per workgroup below, 128 or 256 above), where the output pass keeps its
+decay fragments; against the fp32 kernels, which share no code with them.  The bf16 kernels see the same rounded inputs, so
+the tolerances are those of the parity tests:
 outputs 2e-2 absolute + 1e-2 relative per element, gradients 1e-2 relative L2 (two or three bf16 roundings of 2^-9 each).
 dg is a reverse cumulative sum over the sequence whose terms carry independent roundings while the sum itself stays as
 large as the few rows the gates remember: its error grows with the square root of the length, from the 1e-2 that the
@@ -52,3 +53,17 @@ def test_backward_groups(D, T, wl):
             n = NG if g.shape[2] > H else 1
             check_grad(f"d{k} D{D} T{T} wl{wl} kv-head {h}", g[:, :, n * h:n * (h + 1)], r.cpu(), BF,
                        rel_bar=1e-2 * max(1.0, (T / 340) ** 0.5) if k == "g" else 1e-2)
+
+
+# two query heads per kv-head: 224 and 264 workgroups of the output pass, either side of the 256 CUs
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [1786, 2100])
+def test_output_pass_pairs(D, T):
+    from nha_amd import chunk_nha
+    H = 8
+    d = prefill_inputs(9200 + D + T, 1, T, 2 * H, H, D, D, 64, dtype=BF, qk_scale=D ** -0.5, gate_div=1.0, gate_mean=-1.0)
+    c = [d[k].cuda() for k in KEYS]
+    got = chunk_nha(*c, window_size_left=150)
+    ref = chunk_nha(*(x.float() for x in c), window_size_left=150, impl="simple")
+    for name, x, y in zip(("o", "lse_swa", "lse_gsa"), got, ref):
+        assert_close(f"{name} D{D} T{T}", x, y, BF)
