@@ -538,7 +538,8 @@ def _one_node(x: torch.Tensor, weights) -> bool:
 
 def _plain_modules(modules) -> bool:
     """nn.Linear modules without bias, hooks or a forward of their own."""
-    return (torch.nn.Linear.forward is _LINEAR_FORWARD and not torch.nn.modules.module._has_any_global_hook()
+    return (not torch.compiler.is_compiling() and torch.nn.Linear.forward is _LINEAR_FORWARD
+            and not torch.nn.modules.module._has_any_global_hook()
             and all(type(m) is torch.nn.Linear and "forward" not in m.__dict__ and m.bias is None
                     and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
                     for m in modules))
