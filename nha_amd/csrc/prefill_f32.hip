@@ -48,10 +48,10 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __bui
 __device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 // e^x to about an ulp: 2^t of the rounded t = x log2(e), corrected to first order for what rounding t lost (an fma recovers
 // it exactly).  v_exp_f32 of the rounded product alone is off by |x| 2^-24, the library's expf takes twice the instructions
-// for ranges that do not occur here; below e^-200 everything is 0, -inf and -inf - -inf included.
+// for ranges that do not occur here; below e^-200 everything is 0, -inf included.  NaN stays NaN (fmaxf would drop it).
 __device__ __forceinline__ float exp_f32(float x) {
   constexpr float HI = 1.44269502f, LO = 1.92596299e-8f, LN2 = 0.693147181f;   // HI + LO = log2(e)
-  x = fmaxf(x, -200.f);
+  x = __builtin_elementwise_maximum(x, -200.f);
   const float t = x * HI, lost = fmaf(x, HI, -t) + x * LO, e = __builtin_amdgcn_exp2f(t);
   return fmaf(e, lost * LN2, e);
 }

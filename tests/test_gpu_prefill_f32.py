@@ -35,3 +35,29 @@ def test_f32_strong_gates(mean):
     d["g"][:, 40:75, :, 5] = mean
     d["s"] = 1 - d["g"].exp()
     run_case(f"one fast slot {mean}", d, wl=20, shift=5, dtype=F32, impl=None)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("name", ["q_swa", "k_swa", "q_gsa", "k_gsa", "v", "s", "g", "h0k", "h0v"])
+def test_f32_nan_reaches_every_output_that_depends_on_it(name, D):
+    """NaN in one row of an operand: every output that is NaN in the recurrence is NaN here (a maximum or a clamp drops
+    NaN where it is not looked after), and tokens of the 16-row blocks before it are untouched."""
+    from nha_amd import chunk_nha
+    from oracle import nha_ref as R
+    from tests.test_gpu_prefill import KEYS
+    at, T, wl = 70, 200, 20
+    d = prefill_inputs(D, 1, T, 4, 2, D, D, 64, dtype=F32, with_state=True)
+    if name in ("h0k", "h0v"):
+        d["h0"][name == "h0v"][:, 1, 3] = float("nan")
+        at = 0
+    else:
+        d[name][:, at] = float("nan")
+    ref = R.prefill_ref(*[d[k] for k in KEYS], window_size_left=wl, gsa_kv_shift=0, initial_state=d["h0"])
+    o, lse_swa, lse_gsa, (hkt, hvt) = chunk_nha(*[d[k].cuda() for k in KEYS], window_size_left=wl, window_size_right=0,
+                                                initial_state=tuple(x.cuda() for x in d["h0"]), output_final_state=True)
+    assert any(x.isnan().any() for x in ref)
+    for what, got, want in zip(("o", "lse_swa", "lse_gsa", "hk", "hv"), (o, lse_swa, lse_gsa, hkt, hvt), ref):
+        got, want = got.cpu(), want.reshape(got.shape)
+        assert not (want.isnan() & ~got.isnan()).any(), what
+        if what in ("o", "lse_swa", "lse_gsa"):
+            assert got[:, :at // 16 * 16].isfinite().all(), what
