@@ -268,7 +268,8 @@ __global__ __launch_bounds__(64 * NW, 2) void decode_split_kernel(const SplitArg
       mx = fmaxf(mx, across<1 << SH>(mx));
       mx = fmaxf(mx, across<2 << SH>(mx));
       mx = fmaxf(mx, across<4 << SH>(mx));
-      const float mnew = fmaxf(mrun, mx), alpha = fexp2(mrun - mnew), e = fexp2(v - mnew);
+      const float mnew = fmaxf(mrun, mx), ref = mnew == -INFINITY ? 0.f : mnew;   // eight slots may all weigh nothing
+      const float alpha = fexp2(mrun - ref), e = fexp2(v - ref);
       float sum = e;
       sum += across<1 << SH>(sum);
       sum += across<2 << SH>(sum);
@@ -301,6 +302,7 @@ __global__ __launch_bounds__(64 * NW, 2) void decode_split_kernel(const SplitArg
     }
 #pragma unroll
     for (int g = 0; g < G; ++g) st_f<CPL>(os + g * D + CPL * lane, O[g]);
+    if (lrun != lrun) mrun = INFINITY;   // a maximum does not carry NaN: without this the merge would pass the part over
   }
   ml[(2 * wave) * G + (lane >> (SH + 3))] = mrun;      // -inf and 0 where the wave had no slot task
   ml[(2 * wave + 1) * G + (lane >> (SH + 3))] = lrun;
@@ -438,6 +440,7 @@ __global__ __launch_bounds__(64 * NW, 2) void decode_split_kernel(const SplitArg
       }
     }
     wsum = sum_over_rows(wsum);
+    if (wsum != wsum) wmax = INFINITY;   // as for the slots: the merge gives NaN
     // O^T[v = 16*vt + 4*qd + r][head l16] -> wave-private fp32 [G][D] over this wave's V tile
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     lfloat* Ow = (lfloat*)(NHA_LDS void*)X;

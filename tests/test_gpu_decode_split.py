@@ -61,3 +61,48 @@ def test_split_step_in_a_graph_without_scratch_of_its_own():
         torch.cuda.synchronize()
         assert torch.equal(o, want) and torch.equal(hk, whk) and torch.equal(hv, whv)
         assert torch.equal(fused_recurrent_nha_decode(**a)[0], want)
+
+
+@pytest.mark.parametrize("B,NG,H,K,W", [(1, 4, 2, 128, 200), (3, 2, 1, 256, 40), (2, 8, 2, 64, 20), (40, 4, 4, 128, 64)])
+@pytest.mark.parametrize("where", ["q", "sq", "slots of one task", "keys of one task", "values"])
+def test_split_step_keeps_nan(B, NG, H, K, W, where):
+    """NaN in all that one part of a pair's work sees reaches the pair's output (the part's maximum does not carry it), and
+    no other pair's."""
+    from nha_amd import NHARingState, ring_decode_step
+    dt, HQ, M, nan = torch.bfloat16, NG * H, 64, float("nan")
+    gen = torch.Generator().manual_seed(W)
+    ring = [randn(gen, B, W, H, d, dtype=dt) for d in (K, K, K)] + [-randn(gen, B, W, H, M, dtype=dt).abs()]
+    hk, hv = randn(gen, B, H, K, M, dtype=torch.float32), randn(gen, B, H, M, K, dtype=torch.float32)
+    new = [randn(gen, B, h, K, dtype=dt) for h in (HQ, HQ, H, H, H)] + [-randn(gen, B, H, M, dtype=dt).abs()]
+    count = torch.full((B,), 2 * W, dtype=torch.int32)
+    if where == "q":
+        new[0][0, 0] = nan
+    elif where == "sq":
+        new[1][0, 0] = nan
+    elif where == "slots of one task":
+        hk[0, 0, :, 8:16] = nan
+    elif where == "keys of one task":
+        ring[0][0, :32, 0] = nan
+        new[2][0, 0] = nan
+    else:
+        ring[2][0, W // 2, 0] = nan
+    want = R.decode_ring_ref(*new, *ring, count, hk, hv)[0]
+    st = NHARingState(*[x.clone().cuda() for x in (hk, hv, *ring, count)])
+    o = ring_decode_step(st, *[x.cuda() for x in new]).cpu()
+    assert want.isnan().any() and torch.equal(o.isnan(), want.isnan())
+
+
+def test_split_step_with_a_task_of_slots_that_weigh_nothing():
+    """The eight slots of one task at logit -inf: their weight is 0, the rest of the softmax stands."""
+    from nha_amd import NHARingState, ring_decode_step
+    B, HQ, H, K, W, M, dt = 2, 4, 1, 128, 100, 64, torch.bfloat16
+    gen = torch.Generator().manual_seed(5)
+    ring = [randn(gen, B, W, H, d, dtype=dt) for d in (K, K, K)] + [-randn(gen, B, W, H, M, dtype=dt).abs()]
+    hk, hv = randn(gen, B, H, K, M, dtype=torch.float32), randn(gen, B, H, M, K, dtype=torch.float32)
+    hk[..., 16:24] = -float("inf")
+    new = [randn(gen, B, h, K, dtype=dt) for h in (HQ, HQ, H, H, H)] + [-randn(gen, B, H, M, dtype=dt).abs()]
+    new[0] = new[0].abs() + 0.01
+    count = torch.full((B,), 2 * W, dtype=torch.int32)
+    want = R.decode_ring_ref(*new, *ring, count, hk, hv)[0]
+    st = NHARingState(*[x.clone().cuda() for x in (hk, hv, *ring, count)])
+    assert_close("o", ring_decode_step(st, *[x.cuda() for x in new]), want, dt)
