@@ -15,6 +15,7 @@ is a HIP kernel behind the C ABI.  There is no CPU / eager fallback.
 from __future__ import annotations
 
 import ctypes as C
+import threading
 import weakref
 from typing import Optional, Tuple
 
@@ -100,6 +101,7 @@ def _workspace(nbytes: int, dev, stream: int) -> torch.Tensor:
 # scratch of the decode steps (arrival counters, partial results): one small buffer per (device, stream), zero when it is
 # made; a step leaves its counters zero again, so it serves every decode call of the stream
 _DECODE_SCRATCH: dict = {}
+_DECODE_SCRATCH_LOCK = threading.Lock()
 
 
 def decode_scratch(dev, stream: int) -> torch.Tensor:
@@ -107,9 +109,11 @@ def decode_scratch(dev, stream: int) -> torch.Tensor:
         return torch.zeros(_lib.load().nha_decode_scratch_bytes(), dtype=torch.uint8, device=dev)
     ws = _DECODE_SCRATCH.get((dev, stream))
     if ws is None:
-        while len(_DECODE_SCRATCH) >= _WORKSPACE_MAX_STREAMS:
-            _DECODE_SCRATCH.pop(next(iter(_DECODE_SCRATCH)))
-        ws = _DECODE_SCRATCH[(dev, stream)] = torch.zeros(_lib.load().nha_decode_scratch_bytes(), dtype=torch.uint8, device=dev)
+        ws = torch.zeros(_lib.load().nha_decode_scratch_bytes(), dtype=torch.uint8, device=dev)
+        with _DECODE_SCRATCH_LOCK:                     # threads with new streams of their own
+            while len(_DECODE_SCRATCH) >= _WORKSPACE_MAX_STREAMS:
+                _DECODE_SCRATCH.pop(next(iter(_DECODE_SCRATCH)))
+            _DECODE_SCRATCH[(dev, stream)] = ws
     return ws
 
 
@@ -118,9 +122,10 @@ def release_workspaces() -> int:
     the bytes they held.  The buffers are grow-only: one large prefill otherwise keeps its scratch for the life of the
     process, out of reach of `torch.cuda.empty_cache()`.  Work already queued keeps its buffer alive through the
     caching allocator's stream ordering, so this is safe to call between steps."""
-    held = sum(ws.numel() for pool in (_WORKSPACE, _DECODE_SCRATCH) for ws in pool.values())
-    _WORKSPACE.clear()
-    _DECODE_SCRATCH.clear()
+    with _DECODE_SCRATCH_LOCK:
+        held = sum(ws.numel() for pool in (_WORKSPACE, _DECODE_SCRATCH) for ws in pool.values())
+        _WORKSPACE.clear()
+        _DECODE_SCRATCH.clear()
     return held
 
 

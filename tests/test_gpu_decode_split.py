@@ -106,3 +106,29 @@ def test_split_step_with_a_task_of_slots_that_weigh_nothing():
     want = R.decode_ring_ref(*new, *ring, count, hk, hv)[0]
     st = NHARingState(*[x.clone().cuda() for x in (hk, hv, *ring, count)])
     assert_close("o", ring_decode_step(st, *[x.cuda() for x in new]), want, dt)
+
+
+def test_split_steps_on_more_streams_than_scratch_is_kept_for():
+    """Four threads, each taking the window form through new streams of its own: 24 in all, more than the pool keeps."""
+    import threading
+    from nha_amd import fused_recurrent_nha_decode, ops
+    B, HQ, H, K, W, M, dt = 2, 8, 2, 128, 200, 64, torch.bfloat16
+    gen = torch.Generator().manual_seed(9)
+    r = lambda *s: randn(gen, *s, dtype=dt).cuda()
+    a = dict(q=r(B, 1, HQ, K), sq=r(B, 1, HQ, K), k=r(B, 1, H, K), v=r(B, 1, H, K), g=-r(B, 1, H, M).abs() / 8, sw_k=r(B, W, H, K),
+             sw_v=r(B, W, H, K), initial_state=(r(B, H, K, M).float(), r(B, H, M, K).float()), output_final_state=True)
+    want = fused_recurrent_nha_decode(**a)[0]
+    torch.cuda.synchronize()
+    got, streams = [], [[torch.cuda.Stream() for _ in range(6)] for _ in range(4)]
+
+    def work(mine):
+        for s in mine:
+            with torch.cuda.stream(s):
+                for _ in range(5):
+                    o = fused_recurrent_nha_decode(**a)[0]
+                s.synchronize()
+                got.append(torch.equal(o, want))
+    threads = [threading.Thread(target=work, args=(x,)) for x in streams]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert got == [True] * 24 and len(ops._DECODE_SCRATCH) <= ops._WORKSPACE_MAX_STREAMS
