@@ -84,13 +84,15 @@ __global__ __launch_bounds__(256) void f32_state_local_kernel(const FP p) {
   for (int i = 1; i < 16; ++i) g[i] += g[i - 1];
   const float t0 = __shfl(g[15], l16, 64), t1 = __shfl(g[15], 16 + l16, 64), t2 = __shfl(g[15], 32 + l16, 64), t3 = __shfl(g[15], 48 + l16, 64);
   const float before = qd == 0 ? 0.f : qd == 1 ? t0 : qd == 2 ? t0 + t1 : t0 + t1 + t2;
-  const float last = t0 + t1 + t2 + t3;
+  // A row's decay to the end of the chunk is summed from the gates after it, not taken as a difference of two cumsums that
+  // were each rounded at the chunk's whole magnitude: error of the final states against 64 bits at 512 tokens, 4 heads of 64,
+  // gates logsigmoid(N(0,1)): 9.3e-7 with the difference, 7.6e-7 in the generic kernels, 1.9e-7 like this.
+  const float after = qd == 3 ? 0.f : qd == 2 ? t3 : qd == 1 ? t2 + t3 : t1 + t2 + t3, own = g[15];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    g[i] += before;
+    s[i] *= exp_f32(own - g[i] + after);
     const int j = 16 * qd + i;
-    if (blockIdx.y == 0 && j < rows) p.gc[((int64_t)(bos + it * BT + j) * p.H + h) * MS + m] = g[i];
-    s[i] *= exp_f32(last - g[i]);
+    if (blockIdx.y == 0 && j < rows) p.gc[((int64_t)(bos + it * BT + j) * p.H + h) * MS + m] = g[i] + before;
   }
   const float* x = blockIdx.y == 0 ? p.k_gsa : p.v;
   float* u = (blockIdx.y == 0 ? p.hkc : p.hvc) + ((int64_t)chunk * p.H + h) * MS * D;

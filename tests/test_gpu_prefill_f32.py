@@ -61,3 +61,21 @@ def test_f32_nan_reaches_every_output_that_depends_on_it(name, D):
         assert not (want.isnan() & ~got.isnan()).any(), what
         if what in ("o", "lse_swa", "lse_gsa"):
             assert got[:, :at // 16 * 16].isfinite().all(), what
+
+
+@pytest.mark.parametrize("T,D,div,mean", [(512, 64, 1.0, 0.0), (700, 256, 8.0, 0.0), (896, 128, 1.0, -1.0)])
+def test_f32_states_are_no_less_exact_than_the_generic_kernels(T, D, div, mean):
+    """Error of the final states against 64 bits, beside that of the generic kernels: decays formed from cumsums rounded at
+    the chunk's magnitude were 1.2 times theirs; a quarter of an fp32 rounding is left for the order of the sums."""
+    from nha_amd import chunk_nha
+    from oracle import nha_ref as R
+    from tests.test_gpu_prefill import KEYS
+    d = prefill_inputs(1, 1, T, 4, 4, D, D, 64, dtype=F32, gate_div=div, gate_mean=mean, qk_scale=D ** -0.5, with_state=True)
+    ref = R.prefill_ref(*[d[k] for k in KEYS], window_size_left=63, gsa_kv_shift=0, initial_state=d["h0"])[3:]
+    errs = {}
+    for impl in ("simple", None):
+        got = chunk_nha(*[d[k].cuda() for k in KEYS], window_size_left=63, window_size_right=0, impl=impl,
+                        initial_state=tuple(x.cuda() for x in d["h0"]), output_final_state=True)[3]
+        errs[impl] = [((a.double().cpu() - b).norm() / b.norm()).item() for a, b in zip(got, ref)]
+    print(errs)
+    assert all(a <= b + 2.0 ** -26 for a, b in zip(errs[None], errs["simple"])), errs
