@@ -247,6 +247,13 @@ __global__ __launch_bounds__(64 * NW, 2) void decode_split_kernel(const SplitArg
         eg[s] = has_pop ? e : 1.f;
         sg[s] = has_pop ? (spop ? sg[s] : 1.f - e) : 0.f;
       }
+      // a ring that is not full pops nothing: its row holds no token yet and may hold anything, NaN included, which a zero
+      // strength would not keep out
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) {
+        kp[c] = has_pop ? kp[c] : 0.f;
+        vp[c] = has_pop ? vp[c] : 0.f;
+      }
 #pragma unroll
       for (int c = 0; c < CPL; ++c) {
 #pragma unroll

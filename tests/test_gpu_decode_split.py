@@ -132,3 +132,26 @@ def test_split_steps_on_more_streams_than_scratch_is_kept_for():
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert got == [True] * 24 and len(ops._DECODE_SCRATCH) <= ops._WORKSPACE_MAX_STREAMS
+
+
+# pairs that are split, that keep one workgroup of four waves, and that keep the kernel of large calls
+@pytest.mark.parametrize("B,NG,H,K,W", [(3, 4, 2, 128, 200), (3, 8, 1, 64, 33), (2, 1, 2, 256, 300), (80, 4, 4, 128, 64), (3, 3, 64, 64, 40),
+                                        (160, 4, 4, 64, 48)])
+@pytest.mark.parametrize("value", ["nan", "inf"])
+def test_ring_rows_without_a_token_are_not_looked_at(B, NG, H, K, W, value):
+    """A ring that is not full pops nothing: rows past its count may hold anything (fresh memory, an earlier request's), and
+    the step is that of a ring with zeros there."""
+    from nha_amd import NHARingState, ring_decode_step
+    dt, HQ, M = torch.bfloat16, NG * H, 64
+    gen = torch.Generator().manual_seed(W + B)
+    clean = [randn(gen, B, W, H, d, dtype=dt) for d in (K, K, K)] + [-randn(gen, B, W, H, M, dtype=dt).abs()]
+    hk, hv = randn(gen, B, H, K, M, dtype=torch.float32, scale=0.3), randn(gen, B, H, M, K, dtype=torch.float32, scale=0.3)
+    count = torch.tensor([0, 1, W - 1] * B, dtype=torch.int32)[:B]
+    empty = (torch.arange(W)[None] >= count[:, None])[..., None, None]
+    clean = [x.masked_fill(empty, 0) for x in clean]
+    st = NHARingState(*[x.clone().cuda() for x in (hk, hv, *[x.masked_fill(empty, float(value)) for x in clean], count)])
+    new = [randn(gen, B, h, K, dtype=dt) for h in (HQ, HQ, H, H, H)] + [-randn(gen, B, H, M, dtype=dt).abs()]
+    o = ring_decode_step(st, *[x.cuda() for x in new])
+    ro, hk, hv, ring = R.decode_ring_ref(*new, *clean, count, hk, hv)
+    for name, a, b in (("o", o, ro), ("hk", st.hk, hk), ("hv", st.hv, hv)):
+        assert_close(name, a, b, dt)
