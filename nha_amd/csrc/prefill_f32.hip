@@ -17,7 +17,9 @@
 // Everything is computed transposed (a query per lane), with operands loaded from global memory in MFMA layout: A = a
 // row of keys / slots per lane (16 bytes of consecutive columns, four products per load; both operands number the
 // contraction the same way, so its order is free), and the accumulator of a score product is the B operand of the next
-// product as it stands.  No LDS, no barriers.
+// product as it stands.  No LDS, no barriers.  A unit whose output is not finite is formed a second time without the rows that
+// a query does not see (f32_out_rows); the look at the output costs nothing measurable (567 / 560 us without / with, at
+// B=2, T=4096, 32/8 heads of 128).
 #include "common.h"
 
 namespace nha {
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(256) void f32_state_local_kernel(const FP p) {
   const int m0 = 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = m0 + l16;
   const int chunk = blockIdx.x / p.H, h = blockIdx.x % p.H;
   const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
-  const int bos = p.cu[n] + 0, eos = p.cu[n + 1];
+  const int bos = p.cu[n], eos = p.cu[n + 1];
   const int rows = min(BT, eos - bos - it * BT), base = it * BT - p.shift;   // row j absorbs token bos + base + j
   const int jlo = base < 0 ? -base : 0;                                      // first row with a source token
   float g[16], s[16];
@@ -110,6 +112,9 @@ __global__ __launch_bounds__(256) void f32_state_local_kernel(const FP p) {
       const int j = max(min(16 * qd + i, rows - 1), jlo);
       b[i] = x[((int64_t)(bos + base + j) * p.H + h) * D + 16 * c + l16];
     }
+    if (jlo > 0 || rows < BT)   // rows that absorb nothing: zero, not the row that was read in their place (0 inf is NaN)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) b[i] = 16 * qd + i >= jlo && 16 * qd + i < rows ? b[i] : 0.f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc = mfma4(s[i], b[i], acc);   // [slot 4 (l/16) + r][column l%16]
@@ -163,20 +168,19 @@ __global__ __launch_bounds__(256) void f32_state_scan_kernel(const FP p) {
     for (int e = 0; e < 4; ++e) p.hkt[(sh * D + c4 + e) * MS + m] = st[e];
 }
 
-template <int D, int WPB>
-__global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
+// 16 rows (block `sub` of a chunk) of one query head.  A product takes its 16 rows of keys, values or strengths for all 16
+// queries, the ones that a query does not see (later rows, rows before its window, rows that absorb no token) with weight
+// zero: exact for finite values only.  Returns whether an output is not finite, with nothing of the unit settled then;
+// EXACT leaves such rows out, query by query and row by row, and always settles it.
+template <int D, bool EXACT>
+__device__ __forceinline__ bool f32_out_rows(const FP& p, int chunk, int h, int gq, int sub) {
   constexpr int KK = D / 16;   // 16-column pieces of a row
   const int lane = threadIdx.x & 63, l16 = lane & 15, qd = lane >> 4;
-  int unit = blockIdx.x * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int gq = unit % p.NG; unit /= p.NG;       // the heads of a group and the rows of a chunk share keys: neighbours
-  const int sub = unit & 3; unit >>= 2;
-  const int h = unit % p.H, chunk = unit / p.H;
-  if (chunk >= p.NT) return;
   const int hq = h * p.NG + gq;
   const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int cb = bos + it * BT, rows = min(BT, eos - cb);
-  if (16 * sub >= rows) return;
+  if (16 * sub >= rows) return false;
   const int t0 = cb + 16 * sub, t = t0 + l16, tq = min(t, eos - 1);   // the lane's query; rows past the end are not stored
   f32x4 O[KK];
 #pragma unroll
@@ -224,6 +228,17 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
 #pragma unroll
       for (int c = 0; c < KK; ++c) O[c] = mfma4(v.a[r][c], w[r], O[c]);
   };
+  // value of accumulator row jj (of 16) for the lane's query
+  auto of_row = [&](const f32x4& w, int jj) { return __shfl(jj & 2 ? (jj & 1 ? w[3] : w[2]) : (jj & 1 ? w[1] : w[0]), 16 * (jj >> 2) + l16, 64); };
+  // the same sum over the rows jj that the lane's query sees; row(jj) = where row jj starts
+  auto read_seen = [&](auto row, auto seen, const f32x4& w) {
+    for (int jj = 0; jj < 16; ++jj) {
+      const float x = of_row(w, jj);
+      if (!seen(jj)) continue;
+#pragma unroll
+      for (int c = 0; c < KK; ++c) O[c] += ld4(row(jj) + 16 * c + 4 * qd) * x;
+    }
+  };
 
   // ---- window: keys max(bos, t - wl) .. t, newest 16 first (every query meets its own key in the first block) --------
   load_q(p.q_swa);
@@ -233,7 +248,9 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
   Rows kr = keys(t0);
   for (int kb = t0; kb > lo - 16; kb -= 16) {
     // the values of this block and the keys of the next are under way while its scores are formed
-    const Cols vc = fetch_cols([&](int r) { return p.v + ((int64_t)max(bos, min(kb + 4 * qd + r, eos - 1)) * p.H + h) * D; });
+    auto vrow = [&](int j) { return p.v + ((int64_t)max(bos, min(kb + j, eos - 1)) * p.H + h) * D; };
+    Cols vc;
+    if constexpr (!EXACT) vc = fetch_cols([&](int r) { return vrow(4 * qd + r); });
     const Rows kn = keys(kb - 16);
     f32x4 s = scores(kr);
     kr = kn;
@@ -256,7 +273,8 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
       s[r] = exp_f32(s[r] - mw);
       lw += s[r];
     }
-    read(vc, s);
+    if constexpr (EXACT) read_seen(vrow, [&](int jj) { return kb + jj <= tq && kb + jj >= mylo; }, s);
+    else read(vc, s);
   }
   lw = rows_sum(lw);
 
@@ -284,9 +302,29 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) L[b][r] *= exp_f32(gi[b][r]);
   }
-  const bool pairwise = __any(growth > GROWTH_MAX);
-  f32x4 A;   // intra-chunk scores [row][query] of the 16 rows of `sub`
+  const bool pairwise = EXACT || __any(growth > GROWTH_MAX);
+  f32x4 A;   // intra-chunk scores [row][query] of 16 rows, at last of those of `sub`
+  // the logits' share of the 16 rows of J, each with its own decay
+  auto add_pairs = [&](int J) {
+    for (int jj = 0; jj < 16; ++jj) {
+      const int j = 16 * J + jj;
+      const float a = of_row(A, jj);
+      if (live(j) == 0.f) continue;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const f32x4 sv = ld4(p.s + ((int64_t)src(j) * p.H + h) * MS + 16 * b + 4 * qd), gj = ld4(gcb + (int64_t)j * gs + 16 * b + 4 * qd);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (J < sub || jj <= l16) L[b][r] += a * sv[r] * exp_f32(gi[b][r] - gj[r]);
+      }
+    }
+  };
   for (int J = 0; J <= sub; ++J) {
+    if constexpr (EXACT) {
+      A = scores(fetch(p.k_gsa + ((int64_t)src(16 * J + l16) * p.H + h) * D));
+      add_pairs(J);
+      continue;
+    }
     float sv[4][4], gv[4][4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -313,23 +351,13 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
       for (int b = 0; b < 4; ++b) L2[b] = mfma4(sv[r][b] * live(j) * exp_f32(ga[b] - gv[r][b]), A[r], L2[b]);
     }
   }
+  if constexpr (!EXACT) {
 #pragma unroll
-  for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < 4; ++b)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) L[b][r] += L2[b][r] * exp_f32(gi[b][r] - gr[b][r]);
-  if (pairwise)
-    for (int jj = 0; jj < 16; ++jj) {
-      const int j = 16 * sub + jj;
-      const float a = __shfl(jj & 2 ? (jj & 1 ? A[3] : A[2]) : (jj & 1 ? A[1] : A[0]), 16 * (jj >> 2) + l16, 64);
-      if (live(j) == 0.f) continue;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const f32x4 sv = ld4(p.s + ((int64_t)src(j) * p.H + h) * MS + 16 * b + 4 * qd), gj = ld4(gcb + (int64_t)j * gs + 16 * b + 4 * qd);
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (jj <= l16) L[b][r] += a * sv[r] * exp_f32(gi[b][r] - gj[r]);
-      }
-    }
+      for (int r = 0; r < 4; ++r) L[b][r] += L2[b][r] * exp_f32(gi[b][r] - gr[b][r]);
+    if (pairwise) add_pairs(sub);
+  }
 
   // ---- one softmax over [slots | window] ----------------------------------------------------------------------------
   float mg = -INFINITY, lg = 0.f;
@@ -369,9 +397,11 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
     read(fetch_cols([&](int r) { return p.hvc + (ch * MS + 16 * b + 4 * qd + r) * D; }), w);
   }
   for (int J = 0; J <= sub; ++J) {
-    const Cols vc = fetch_cols([&](int r) { return p.v + ((int64_t)src(16 * J + 4 * qd + r) * p.H + h) * D; });
+    auto vrow = [&](int j) { return p.v + ((int64_t)src(16 * J + j) * p.H + h) * D; };
+    Cols vc;
+    if constexpr (!EXACT) vc = fetch_cols([&](int r) { return vrow(4 * qd + r); });
     f32x4 w = {0.f, 0.f, 0.f, 0.f};   // weights [row][query]
-    if (J < sub || !pairwise) {
+    if (!EXACT && (J < sub || !pairwise)) {
       const int j = 16 * J + l16;
       const float* srow = p.s + ((int64_t)src(j) * p.H + h) * MS + 4 * qd;
       const float* grow = gcb + (int64_t)min(j, rows - 1) * gs + 4 * qd;
@@ -385,7 +415,7 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
       }
     } else {
       for (int jj = 0; jj < 16; ++jj) {
-        const int j = 16 * sub + jj;
+        const int j = 16 * J + jj;
         if (live(j) == 0.f) continue;
         float x = 0.f;
 #pragma unroll
@@ -393,7 +423,7 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
           const f32x4 sv = ld4(p.s + ((int64_t)src(j) * p.H + h) * MS + 16 * b + 4 * qd), gj = ld4(gcb + (int64_t)j * gs + 16 * b + 4 * qd);
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            if (jj <= l16) x += L[b][r] * sv[r] * exp_f32(gi[b][r] - gj[r]);
+            if (J < sub || jj <= l16) x += L[b][r] * sv[r] * exp_f32(gi[b][r] - gj[r]);
         }
         x = rows_sum(x);
 #pragma unroll
@@ -405,11 +435,32 @@ __global__ __launch_bounds__(64 * WPB) void f32_out_kernel(const FP p) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (4 * qd + r > l16) w[r] = 0.f;
-    read(vc, w);
+    if constexpr (EXACT) read_seen(vrow, [&](int jj) { return live(16 * J + jj) != 0.f && (J < sub || jj <= l16); }, w);
+    else read(vc, w);
+  }
+  if constexpr (!EXACT) {
+    float z = 0.f;   // NaN if an output is not finite
+#pragma unroll
+    for (int c = 0; c < KK; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z = fmaf(O[c][e], 0.f, z);
+    if (__any(t < eos && z != 0.f)) return true;
   }
   if (t < eos)
 #pragma unroll
     for (int c = 0; c < KK; ++c) *reinterpret_cast<f32x4*>(p.o + ((int64_t)t * p.HQ + hq) * D + 16 * c + 4 * qd) = O[c];
+  return false;
+}
+
+// (two waves per SIMD up to head size 128: the rare form's registers do not cost the second)
+template <int D, int WPB>
+__global__ __launch_bounds__(64 * WPB, D <= 128 ? 2 : 1) void f32_out_kernel(const FP p) {
+  int unit = blockIdx.x * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int gq = unit % p.NG; unit /= p.NG;       // the heads of a group and the rows of a chunk share keys: neighbours
+  const int sub = unit & 3; unit >>= 2;
+  const int h = unit % p.H, chunk = unit / p.H;
+  if (chunk >= p.NT) return;
+  if (f32_out_rows<D, false>(p, chunk, h, gq, sub)) f32_out_rows<D, true>(p, chunk, h, gq, sub);
 }
 
 template <int D>

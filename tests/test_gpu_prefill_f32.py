@@ -79,3 +79,29 @@ def test_f32_states_are_no_less_exact_than_the_generic_kernels(T, D, div, mean):
         errs[impl] = [((a.double().cpu() - b).norm() / b.norm()).item() for a, b in zip(got, ref)]
     print(errs)
     assert all(a <= b + 2.0 ** -26 for a, b in zip(errs[None], errs["simple"])), errs
+
+
+# (window, shift): slots that absorb every token at once, the window's hand-over, a gap between window and slots (the last
+# `shift` tokens are absorbed by nobody; the one at 195 is one of them)
+@pytest.mark.parametrize("D,wl,shift", [(64, 20, 0), (128, 19, 20), (64, 5, 37), (256, 20, 0)])
+@pytest.mark.parametrize("at", [70, 111, 195])
+@pytest.mark.parametrize("name,value", [(n, "nan") for n in ("q_swa", "k_swa", "q_gsa", "k_gsa", "v", "s", "g")] +
+                         [(n, "inf") for n in ("k_swa", "k_gsa", "v", "s")])
+def test_f32_rows_that_a_token_does_not_see(name, value, at, D, wl, shift):
+    """A row that is not finite reaches exactly the outputs that depend on it: not earlier tokens of its 16-row block, nor
+    tokens that it has left the window of, nor, where no slot has absorbed it, any later one.  (The products take 16 rows at
+    once, the unseen ones with weight zero, and zero times NaN or inf is NaN.)"""
+    from nha_amd import chunk_nha
+    from oracle import nha_ref as R
+    from tests.test_gpu_prefill import KEYS
+    from tests.util import assert_close
+    d = prefill_inputs(D + at, 1, 200, 4, 2, D, D, 64, dtype=F32, qk_scale=0.5, with_state=True)
+    d[name][:, at, 1, :] = float(value)
+    ref = R.prefill_ref(*[d[k] for k in KEYS], window_size_left=wl, gsa_kv_shift=shift, initial_state=d["h0"])
+    o, lse_swa, lse_gsa, (hkt, hvt) = chunk_nha(*[d[k].cuda() for k in KEYS], window_size_left=wl, window_size_right=0, gsa_kv_shift=shift,
+                                                initial_state=tuple(x.cuda() for x in d["h0"]), output_final_state=True)
+    assert any(not x.isfinite().all() for x in ref) or at == 195
+    for what, got, want in zip(("o", "lse_swa", "lse_gsa", "hk", "hv"), (o, lse_swa, lse_gsa, hkt, hvt), ref):
+        got, want = got.cpu(), want.reshape(got.shape)
+        assert torch.equal(got.isfinite(), want.isfinite()), (what, got.isfinite().sum().item(), want.isfinite().sum().item())
+        assert_close(what, got.masked_fill(~got.isfinite(), 0), want.masked_fill(~want.isfinite(), 0), F32)
