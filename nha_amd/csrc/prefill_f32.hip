@@ -485,8 +485,13 @@ size_t aligned(size_t x) { return (x + 255) & ~(size_t)255; }
 
 }  // namespace
 
+// Rows are read and written 16 bytes at a time; tensors that start elsewhere (a view into a buffer) keep the generic kernels,
+// which read single floats there.
 bool prefill_f32_supported(const NhaPrefillArgs* a) {
-  return a->dtype == NHA_DTYPE_F32 && a->K == a->V && (a->K == 64 || a->K == 128 || a->K == 256) && a->M == MS &&
+  uintptr_t at = 0;
+  for (const void* x : {a->q_swa, a->k_swa, a->q_gsa, a->k_gsa, a->v, a->s, (const void*)a->o, (const void*)a->h0v, (const void*)a->hvt, (const void*)a->scratch})
+    at |= reinterpret_cast<uintptr_t>(x);
+  return (at & 15) == 0 && a->dtype == NHA_DTYPE_F32 && a->K == a->V && (a->K == 64 || a->K == 128 || a->K == 256) && a->M == MS &&
          (int64_t)a->NT * a->H * 4 * (a->HQ / a->H) < ((int64_t)1 << 31);
 }
 

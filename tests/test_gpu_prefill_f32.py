@@ -105,3 +105,25 @@ def test_f32_rows_that_a_token_does_not_see(name, value, at, D, wl, shift):
         got, want = got.cpu(), want.reshape(got.shape)
         assert torch.equal(got.isfinite(), want.isfinite()), (what, got.isfinite().sum().item(), want.isfinite().sum().item())
         assert_close(what, got.masked_fill(~got.isfinite(), 0), want.masked_fill(~want.isfinite(), 0), F32)
+
+
+@pytest.mark.parametrize("name", ["q_swa", "k_swa", "q_gsa", "k_gsa", "v", "s", "g", "h0k", "h0v"])
+def test_f32_operands_off_a_16_byte_boundary(name):
+    """A contiguous view one float into its buffer: the matrix-core kernels, which read 16 bytes at a time, leave the call to
+    the generic ones wherever they would read it so."""
+    from nha_amd import chunk_nha
+    from tests.test_gpu_prefill import KEYS
+    d = prefill_inputs(3, 1, 90, 4, 2, 64, 64, 64, dtype=F32, qk_scale=0.5, with_state=True)
+    c = {k: x.cuda() for k, x in d.items() if k in KEYS}
+    c["h0k"], c["h0v"] = (x.cuda() for x in d["h0"])
+    buf = torch.empty(c[name].numel() + 1, dtype=F32, device="cuda")
+    call = lambda impl: chunk_nha(*[c[k] for k in KEYS], window_size_left=20, window_size_right=0, impl=impl,
+                                  initial_state=(c["h0k"], c["h0v"]), output_final_state=True)
+    flat = lambda out: [*out[:3], *out[3]]
+    fast, want = flat(call(None)), flat(call("simple"))
+    assert not torch.equal(fast[0], want[0])              # two kernels, two orders of sums
+    c[name] = buf[1:].view(c[name].shape).copy_(c[name])
+    assert c[name].is_contiguous() and c[name].data_ptr() % 16
+    if name in ("g", "h0k"):                              # single floats in both
+        want = fast
+    assert all(torch.equal(x, y) for x, y in zip(flat(call(None)), want))
