@@ -155,3 +155,28 @@ def test_ring_rows_without_a_token_are_not_looked_at(B, NG, H, K, W, value):
     ro, hk, hv, ring = R.decode_ring_ref(*new, *clean, count, hk, hv)
     for name, a, b in (("o", o, ro), ("hk", st.hk, hk), ("hv", st.hv, hv)):
         assert_close(name, a, b, dt)
+
+
+@pytest.mark.parametrize("name", ["q", "k", "v", "g", "s"])
+def test_window_step_on_operands_off_a_16_byte_boundary(name):
+    """A contiguous view one element into its buffer goes to the kernel that reads single elements: the output is its, bit for
+    bit, at a size that is split otherwise."""
+    from nha_amd import fused_recurrent_nha_decode, ops
+    B, HQ, H, K, W, M, dt = 2, 8, 2, 128, 200, 64, torch.bfloat16
+    gen = torch.Generator().manual_seed(4)
+    r = lambda *s: randn(gen, *s, dtype=dt).cuda()
+    a = dict(q=r(B, 1, HQ, K), sq=r(B, 1, HQ, K), k=r(B, 1, H, K), v=r(B, 1, H, K), g=-r(B, 1, H, M).abs() / 8, s=r(B, 1, H, M).abs(),
+             sw_k=r(B, W, H, K), sw_v=r(B, W, H, K), initial_state=(r(B, H, K, M).float(), r(B, H, M, K).float()), output_final_state=True)
+    o, state = fused_recurrent_nha_decode(**a)
+    small = torch.zeros(16, dtype=torch.uint8, device="cuda")
+    keep, ops.decode_scratch = ops.decode_scratch, lambda dev, stream: small      # too small to be split over workgroups
+    try:
+        unsplit, want = fused_recurrent_nha_decode(**a)
+    finally:
+        ops.decode_scratch = keep
+    assert not torch.equal(state[0], want[0]) or not torch.equal(o, unsplit)      # two kernels, two orders of sums
+    x = a[name]
+    a[name] = torch.empty(x.numel() + 1, dtype=dt, device="cuda")[1:].view(x.shape).copy_(x)
+    assert a[name].is_contiguous() and a[name].data_ptr() % 16
+    got, (hk, hv) = fused_recurrent_nha_decode(**a)
+    assert torch.equal(got, unsplit) and torch.equal(hk, want[0]) and torch.equal(hv, want[1])
