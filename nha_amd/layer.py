@@ -22,7 +22,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops as _ops
-from .ops import chunk_nha, gsa_share_begin, gsa_share_end, layer_front_supported, linear, nha_layer_epilogue, nha_layer_prologue, \
+from .ops import chunk_nha, gsa_share_begin, gsa_share_end, layer_front_projections, linear, nha_layer_epilogue, nha_layer_prologue, \
     shared_input_linears
 
 
@@ -308,9 +308,10 @@ class NativeHybridAttention(nn.Module):
         projections = (self.q_proj, self.k_proj, self.v_proj, self.f_proj)
         dims = (self.num_heads, self.num_kv_heads, self.head_k_dim, self.head_v_dim, self.num_slots)
         # projections and prologue as one node: training, plain modules, nothing between the two
-        front = (not self.use_short_conv and self.feature_map is not None and self._fused_glue(hidden_states)
-                 and layer_front_supported(hidden_states, projections, dims))
-        fused = front
+        front = None
+        if not self.use_short_conv and self.feature_map is not None and self._fused_glue(hidden_states):
+            front = layer_front_projections(hidden_states, projections, dims)
+        fused = front is not None
         if not fused:
             q, k, v, f = shared_input_linears(hidden_states, projections)
             if self.use_short_conv:
@@ -329,8 +330,7 @@ class NativeHybridAttention(nn.Module):
             if self._inv_freq is None or self._inv_freq.device != device:
                 self._inv_freq = self.rotary.inv_freq(device)
             fm = None if self.feature_map is None else ('swish' if isinstance(self.feature_map, SwishFeatureMap) else 'relu')
-            source = dict(q=None, k=None, v=None, f=None, projections=(hidden_states, projections, dims)) if front \
-                else dict(q=q, k=k, v=v, f=f)
+            source = dict(q=None, k=None, v=None, f=None, projections=front) if front is not None else dict(q=q, k=k, v=v, f=f)
             q_swa, k_swa, q_gsa, k_gsa, v, s, g = nha_layer_prologue(
                 **source, inv_freq=self._inv_freq, feature_map=fm, gate_logit_normalizer=self.gate_logit_normalizer,
                 seqlen_offset=seqlen_offset, cu_seqlens=cu_seqlens)

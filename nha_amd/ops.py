@@ -312,19 +312,18 @@ def nha_layer_prologue(q, k, v, f, inv_freq, *, feature_map: Optional[str], gate
     tensor).  Returns (q_swa, k_swa, q_gsa, k_gsa, v, s, g); without a feature map q_gsa / k_gsa
     are q / k themselves.  Differentiable with respect to q, k, v, f (one launch backward too).
 
-    projections: (x [B,T,hidden], the q, k, v, f projection modules, (HQ, H, K, V, M)) in the place of q, k, v, f, for calls
-    that layer_front_supported accepts and a feature map.  The weights side by side are one product instead of four, and one
-    for the input's gradient: layer step of 1400 tokens (host-bound) 1010 -> 865 us, of 16384 tokens 1778 -> 1731."""
-    if projections is not None:
-        x, modules, dims = projections
-        if cu_seqlens is not None and x.shape[0] != 1:
-            raise ValueError("cu_seqlens needs the packed layout [1, T_tot, ...]")
-        cu = None if cu_seqlens is None else cu_seqlens.to(device=x.device, dtype=torch.int32).contiguous()
-        return _LayerFrontFunction.apply(x, *(m.weight for m in modules), inv_freq.detach().to(torch.float32).contiguous(),
-                                         tuple(dims), _FMAP[feature_map], float(gate_logit_normalizer), int(seqlen_offset), cu)
-    _need_cuda(q, k, v, f, inv_freq, cu_seqlens)
+    projections: (x [B,T,hidden], the q, k, v, f projection modules, (HQ, H, K, V, M)) in the place of q, k, v, f: one autograd
+    node with the projections (_layer_front) where layer_front_supported accepts them and there is a feature map, the modules'
+    own outputs elsewhere."""
     if feature_map not in _FMAP:
         raise NotImplementedError(f"Feature map `{feature_map}` has no fused prologue.")
+    if projections is not None:
+        x, modules, (HQ, H, K, V, M) = projections
+        if _FMAP[feature_map] and (isinstance(projections, _FrontProjections) or layer_front_supported(*projections)):
+            return _layer_front(x, modules, (HQ, H, K, V, M), inv_freq, feature_map=feature_map,
+                                gate_logit_normalizer=gate_logit_normalizer, seqlen_offset=seqlen_offset, cu_seqlens=cu_seqlens)
+        q, k, v, f = (y.unflatten(-1, d) for y, d in zip(shared_input_linears(x, modules), ((HQ, K), (H, K), (H, V), (H, M))))
+    _need_cuda(q, k, v, f, inv_freq, cu_seqlens)
     _dtype_code(q)
     q, k, v, f = (x.contiguous() for x in (q, k, v, f))
     inv_freq = inv_freq.detach().to(torch.float32).contiguous()
@@ -338,6 +337,21 @@ def nha_layer_prologue(q, k, v, f, inv_freq, *, feature_map: Optional[str], gate
         return outs[0], outs[1], q, k, outs[2], outs[3], outs[4]
     q_swa, k_swa, q_gsa, k_gsa, v_out, s, g = _prologue_fwd(*args)
     return q_swa, k_swa, (q_gsa if fm else q), (k_gsa if fm else k), v_out, s, g
+
+
+def _layer_front(x, modules, dims, inv_freq, *, feature_map: str, gate_logit_normalizer: float, seqlen_offset: int = 0,
+                 cu_seqlens: Optional[torch.Tensor] = None):
+    """nha_layer_prologue on the outputs of the q, k, v, f projection `modules` of x [B,T,hidden], projections and prologue as
+    one node; for calls that layer_front_supported accepts.  dims: (HQ, H, K, V, M).  The weights side by side are one product
+    instead of four, and one for the input's gradient: layer step of 1400 tokens (host-bound) 1010 -> 865 us, of 16384
+    tokens 1778 -> 1731."""
+    if cu_seqlens is not None and x.shape[0] != 1:
+        raise ValueError("cu_seqlens needs the packed layout [1, T_tot, ...]")
+    if inv_freq.numel() != dims[2] // 2 or inv_freq.device != x.device:
+        raise ValueError(f"inv_freq must hold K/2 = {dims[2] // 2} entries on {x.device}, got {inv_freq.numel()} on {inv_freq.device}")
+    cu = None if cu_seqlens is None else cu_seqlens.to(device=x.device, dtype=torch.int32).contiguous()
+    return _LayerFrontFunction.apply(x, *(m.weight for m in modules), inv_freq.detach().to(torch.float32).contiguous(),
+                                     tuple(dims), _FMAP[feature_map], float(gate_logit_normalizer), int(seqlen_offset), cu)
 
 
 def _epilogue_fwd(o, w, b, eps: float):
@@ -567,6 +581,16 @@ def layer_front_supported(x: torch.Tensor, modules, dims) -> bool:
     weights = [m.weight for m in modules]
     return (all(tuple(w.shape) == (n, x.shape[-1]) and n % 8 == 0 for w, n in zip(weights, (HQ * K, H * K, H * V, H * M)))
             and _one_node(x, weights))
+
+
+class _FrontProjections(tuple):
+    """(x, modules, dims) that layer_front_supported has accepted."""
+
+
+def layer_front_projections(x: torch.Tensor, modules, dims) -> Optional[_FrontProjections]:
+    """What the next nha_layer_prologue call takes as its projections without looking them over a second time, or None for
+    what layer_front_supported refuses."""
+    return _FrontProjections((x, modules, dims)) if layer_front_supported(x, modules, dims) else None
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:

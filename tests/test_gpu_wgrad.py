@@ -89,3 +89,46 @@ def test_second_derivative_of_the_projections():
         out.extend(torch.autograd.grad(dx.float().pow(2).sum(), [x, *(m.weight for m in lin)]))
     for g, r in zip(got, ref):
         assert ((g.double() - r.double()).norm() / r.double().norm()).item() <= 1e-2
+
+
+def _front_call(modules, x, inv, fmap="swish", cu=None):
+    from nha_amd.ops import nha_layer_prologue
+    return nha_layer_prologue(None, None, None, None, inv, feature_map=fmap, gate_logit_normalizer=8, cu_seqlens=cu,
+                              projections=(x, modules, (4, 2, 64, 64, 64)))
+
+
+@pytest.mark.parametrize("case", ["one node", "no grad", "no feature map", "bias", "hook", "fp32"])
+def test_prologue_on_projections(case):
+    """The form that takes the projections gives what the plain form gives on the modules' outputs, also for calls that cannot
+    be one node."""
+    from nha_amd.ops import nha_layer_prologue
+    torch.manual_seed(6)
+    dt = torch.float32 if case == "fp32" else torch.bfloat16
+    modules = [torch.nn.Linear(128, n, bias=case == "bias").cuda().to(dt) for n in (256, 128, 128, 128)]
+    x = torch.randn(2, 50, 128, device="cuda").to(dt).requires_grad_()
+    inv = 10000.0 ** (-torch.arange(0, 64, 2, device="cuda").float() / 64)
+    fmap = None if case == "no feature map" else "swish"
+    seen = []
+    if case == "hook":
+        modules[1].register_forward_hook(lambda *a: seen.append(1))
+    with torch.set_grad_enabled(case != "no grad"):
+        got = _front_call(modules, x, inv, fmap)
+        raw = [m(x).unflatten(-1, (h, 64)) for m, h in zip(modules, (4, 2, 2, 2))]
+        want = nha_layer_prologue(*raw, inv, feature_map=fmap, gate_logit_normalizer=8)
+    for a, b in zip(got, want):    # one product or four: another order of sums, one rounding of the projection (2^-8 in bf16)
+        assert a.shape == b.shape and a.dtype == b.dtype and a.requires_grad == b.requires_grad
+        assert ((a.double() - b.double()).norm() / b.double().norm()).item() <= (1e-2 if dt == torch.bfloat16 else 1e-5)
+    assert len(seen) == 2 * (case == "hook")
+
+
+def test_prologue_on_projections_refuses():
+    modules = [torch.nn.Linear(128, n, bias=False).cuda().bfloat16() for n in (256, 128, 128, 128)]
+    x = torch.randn(2, 50, 128, device="cuda").bfloat16().requires_grad_()
+    inv = 10000.0 ** (-torch.arange(0, 64, 2, device="cuda").float() / 64)
+    for bad in (inv[:16], inv.cpu(), torch.cat([inv, inv])):
+        with pytest.raises((ValueError, RuntimeError)):
+            _front_call(modules, x, bad)
+    with pytest.raises(ValueError):
+        _front_call(modules, x, inv, cu=torch.tensor([0, 30, 100], dtype=torch.int32, device="cuda"))
+    with pytest.raises(NotImplementedError):
+        _front_call(modules, x, inv, fmap="t2r")
