@@ -15,6 +15,7 @@ is a HIP kernel behind the C ABI.  There is no CPU / eager fallback.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import threading
 import weakref
 from typing import Optional, Tuple
@@ -234,6 +235,37 @@ def nha_prefill_bwd(q_swa, k_swa, q_gsa, k_gsa, v, s, g, o, lse_swa, lse_gsa, do
     return (*outs, dh0k, dh0v)
 
 
+class _Refusal(torch.autograd.Function):
+    """The first n of the tensors, as functions of the others that have no derivative."""
+
+    @staticmethod
+    def forward(ctx, n, *tensors):
+        return tuple(t.detach() for t in tensors[:n])
+
+    @staticmethod
+    def backward(ctx, *grads):
+        raise RuntimeError("the NHA kernels have first derivatives only: this gradient cannot be differentiated twice")
+
+
+def _first_derivatives_only(backward):
+    """For an autograd node whose backward is a kernel.  Under create_graph its gradients hang on everything that they were
+    formed from, through a node that raises: a second derivative that passes through here is refused, also one that reaches
+    its input by another way too (a residual connection), where torch's once_differentiable, whose node hangs on nothing, is
+    passed by and the sum comes out without the terms of this node."""
+    @functools.wraps(backward)
+    def wrapped(ctx, *grads):
+        with torch.no_grad():
+            outs = backward(ctx, *grads)
+        if torch.is_grad_enabled():
+            roots = [t for t in (*grads, *ctx.saved_tensors) if t is not None and t.requires_grad]
+            formed = [t for t in outs if t is not None]
+            if roots and formed:
+                new = iter(_Refusal.apply(len(formed), *formed, *roots))
+                outs = tuple(None if t is None else next(new) for t in outs)
+        return outs
+    return wrapped
+
+
 _FMAP = {None: _lib.NHA_FMAP_NONE, "none": _lib.NHA_FMAP_NONE, "swish": _lib.NHA_FMAP_SWISH, "relu": _lib.NHA_FMAP_RELU}
 
 
@@ -291,6 +323,7 @@ class _LayerPrologueFunction(torch.autograd.Function):
         return outs if fm else (outs[0], outs[1], outs[4], outs[5], outs[6])
 
     @staticmethod
+    @_first_derivatives_only
     def backward(ctx, *grads):
         q, k, v, f, inv_freq = ctx.saved_tensors
         fm, normalizer, offset = ctx.meta
@@ -378,6 +411,7 @@ class _LayerEpilogueFunction(torch.autograd.Function):
         return _epilogue_fwd(o, w, b, eps)
 
     @staticmethod
+    @_first_derivatives_only
     def backward(ctx, dy):
         lib = _lib.load()
         o, w = ctx.saved_tensors
@@ -505,6 +539,7 @@ class _LayerFrontFunction(torch.autograd.Function):
         return outs
 
     @staticmethod
+    @_first_derivatives_only
     def backward(ctx, *grads):
         x, wq, wk, wv, wf, raw, inv_freq = ctx.saved_tensors
         (HQ, H, K, V, M), fm, normalizer, offset = ctx.meta
@@ -528,10 +563,10 @@ class _LayerFrontFunction(torch.autograd.Function):
             dx = (rows @ torch.cat(weights)).view(x.shape)
         need = [i for i in range(4) if ctx.needs_input_grad[1 + i]]
         picked, xc = [dys[i] for i in need], xr.contiguous()
-        if need and not torch.is_grad_enabled() and _wgrad_supported(xc, picked):
+        if need and _wgrad_supported(xc, picked):
             for i, dw in zip(need, nha_wgrad(xc, picked)):
                 dws[i] = dw
-        else:                                              # operations that have a derivative of their own, or other shapes
+        else:
             for i in need:
                 dws[i] = dys[i].t() @ xr
         return (dx, *dws, None, None, None, None, None, None)
@@ -658,6 +693,7 @@ class _ShortConvFunction(torch.autograd.Function):
         return y
 
     @staticmethod
+    @_first_derivatives_only
     def backward(ctx, dy):
         lib = _lib.load()
         x, w, b, cu = ctx.saved_tensors
@@ -873,7 +909,7 @@ class _ChunkNHAFunction(torch.autograd.Function):
         return o, lse_swa, lse_gsa, hkt, hvt
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
+    @_first_derivatives_only
     def backward(ctx, do, dlse_swa, dlse_gsa, dhkt, dhvt):
         *args, o, lse_swa, lse_gsa, h0k, h0v = ctx.saved_tensors
         if do is None:

@@ -73,3 +73,44 @@ def test_hooks_edits_and_second_derivatives():
     gr = torch.autograd.grad(o.float().sum(), leaves[4], create_graph=True)[0]
     with pytest.raises(RuntimeError):
         gr.float().sum().backward()
+
+
+NODES = ["operator", "prologue", "projections and prologue", "epilogue", "short convolution", "layer", "layer, short convolution"]
+
+
+@pytest.mark.parametrize("residual", [False, True])
+@pytest.mark.parametrize("node", NODES)
+def test_second_derivatives_through_the_kernels_are_refused(node, residual):
+    """The kernels have first derivatives only: a gradient taken with create_graph leads to an error, never to a second
+    derivative without the terms that pass through them, whether the input is reached through them alone or past them too."""
+    from nha_amd import chunk_nha, ops
+    from nha_amd.layer import NativeHybridAttention
+    torch.manual_seed(2)
+    r = lambda *s: torch.randn(*s, device="cuda").bfloat16()
+    inv = 10000.0 ** (-torch.arange(0, 64, 2, device="cuda").float() / 64)
+    x, w = r(1, 90, 128).requires_grad_(), r(128).requires_grad_()
+    total = lambda ts: sum(t.float().pow(2).sum() for t in ts)
+    if node.startswith("layer"):
+        m = NativeHybridAttention(hidden_size=128, num_heads=2, num_slots=64, layer_idx=0, window_size=40, use_short_conv="short" in node)
+        out = total(m.cuda().bfloat16()(x)[:1])
+    elif node in ("prologue", "operator"):
+        q, k, v, f = (y.view(1, 90, 2, 64) for y in (x, x * 2, x * 3, x * 4))
+        out = total(ops.nha_layer_prologue(q, k, v, f, inv, feature_map="swish", gate_logit_normalizer=8)) if node == "prologue" \
+            else total(chunk_nha(q, k, q, k, v, r(1, 90, 2, 64).sigmoid(), -r(1, 90, 2, 64).abs(), window_size_left=40)[:1])
+    elif node == "projections and prologue":
+        mods = [torch.nn.Linear(128, 128, bias=False).cuda().bfloat16() for _ in range(4)]
+        out = total(ops.nha_layer_prologue(None, None, None, None, inv, feature_map="swish", gate_logit_normalizer=8,
+                                           projections=(x, mods, (2, 2, 64, 64, 64))))
+    elif node == "epilogue":
+        out = total([ops.nha_layer_epilogue(x, w, None, 1e-5)])
+    else:
+        out = total([ops.nha_short_conv(x, r(128, 4).requires_grad_(), None, activation="silu")])
+    if residual:
+        out = out + x.float().pow(3).sum()
+    plain = torch.autograd.grad(out, x, retain_graph=True)[0]
+    dx = torch.autograd.grad(out, x, create_graph=True)[0]
+    assert dx.requires_grad
+    # the layer's projections add four products in another order where a graph is wanted: a rounding of 2^-8 each
+    assert torch.equal(dx, plain) if node != "layer, short convolution" else (dx - plain).float().norm() <= 1e-2 * plain.float().norm()
+    with pytest.raises(RuntimeError, match="differentiated twice"):
+        torch.autograd.grad(dx.float().pow(2).sum(), x)
