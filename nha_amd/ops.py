@@ -88,21 +88,24 @@ _WORKSPACE: dict = {}
 _WORKSPACE_MAX_STREAMS = 16      # entries kept; the one used longest ago leaves first (streams come and go)
 
 
+_POOL_LOCK = threading.Lock()    # of both pools: several threads take, evict and release (autograd's backward thread is one)
+
+
 def _workspace(nbytes: int, dev, stream: int) -> torch.Tensor:
     key = (str(dev), stream)
-    ws = _WORKSPACE.pop(key, None)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
-    _WORKSPACE[key] = ws             # re-inserted: the dict's order is the order of last use
-    while len(_WORKSPACE) > _WORKSPACE_MAX_STREAMS:
-        _WORKSPACE.pop(next(iter(_WORKSPACE)))
+    with _POOL_LOCK:
+        ws = _WORKSPACE.pop(key, None)
+        if ws is None or ws.numel() < nbytes:
+            ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
+        _WORKSPACE[key] = ws             # re-inserted: the dict's order is the order of last use
+        while len(_WORKSPACE) > _WORKSPACE_MAX_STREAMS:
+            _WORKSPACE.pop(next(iter(_WORKSPACE)))
     return ws
 
 
 # scratch of the decode steps (arrival counters, partial results): one small buffer per (device, stream), zero when it is
 # made; a step leaves its counters zero again, so it serves every decode call of the stream
 _DECODE_SCRATCH: dict = {}
-_DECODE_SCRATCH_LOCK = threading.Lock()
 
 
 def decode_scratch(dev, stream: int) -> torch.Tensor:
@@ -111,7 +114,7 @@ def decode_scratch(dev, stream: int) -> torch.Tensor:
     ws = _DECODE_SCRATCH.get((dev, stream))
     if ws is None:
         ws = torch.zeros(_lib.load().nha_decode_scratch_bytes(), dtype=torch.uint8, device=dev)
-        with _DECODE_SCRATCH_LOCK:                     # threads with new streams of their own
+        with _POOL_LOCK:                               # threads with new streams of their own
             while len(_DECODE_SCRATCH) >= _WORKSPACE_MAX_STREAMS:
                 _DECODE_SCRATCH.pop(next(iter(_DECODE_SCRATCH)))
             _DECODE_SCRATCH[(dev, stream)] = ws
@@ -123,7 +126,7 @@ def release_workspaces() -> int:
     the bytes they held.  The buffers are grow-only: one large prefill otherwise keeps its scratch for the life of the
     process, out of reach of `torch.cuda.empty_cache()`.  Work already queued keeps its buffer alive through the
     caching allocator's stream ordering, so this is safe to call between steps."""
-    with _DECODE_SCRATCH_LOCK:
+    with _POOL_LOCK:
         held = sum(ws.numel() for pool in (_WORKSPACE, _DECODE_SCRATCH) for ws in pool.values())
         _WORKSPACE.clear()
         _DECODE_SCRATCH.clear()
