@@ -464,8 +464,10 @@ def nha_wgrad(x: torch.Tensor, dys) -> list:
     nbytes = lib.nha_wgrad_scratch_bytes(C.byref(a))
     if nbytes == 0:
         _lib.check(_lib.NHA_ERR_INVALID)
-    scratch = _workspace(nbytes, x.device, a.stream or 0)
-    a.scratch, a.scratch_bytes = _ptr(scratch), scratch.numel()
+    # of the call's own: it holds the partial sums between two launches, and another thread of this stream may queue a call that
+    # uses the stream's shared workspace between them
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    a.scratch, a.scratch_bytes = _ptr(scratch), nbytes
     _lib.check(lib.nha_wgrad(C.byref(a)))
     return outs
 

@@ -31,6 +31,15 @@ def test_wgrad_row_stride():
     assert all(torch.equal(a, b) for a, b in zip(dense, nha_wgrad(x, [both[:, :264], both[:, 264:]])))
 
 
+def test_wgrad_scratch_is_its_own(monkeypatch):
+    """The partial sums lie between two launches: not in the workspace that every call of a stream shares, which another thread
+    may queue a call on in between."""
+    from nha_amd import ops
+    monkeypatch.setattr(ops, "_workspace", lambda *a: pytest.fail("shared workspace"))
+    x, dy = (torch.randn(500, n, device="cuda").bfloat16() for n in (64, 32))
+    assert ops.nha_wgrad(x, [dy])[0].shape == (32, 64)
+
+
 def test_wgrad_refuses():
     from nha_amd import _lib
     lib = _lib.load()
