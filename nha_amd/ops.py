@@ -453,12 +453,22 @@ def nha_layer_epilogue(o, weight: Optional[torch.Tensor], bias: Optional[torch.T
 
 
 def nha_wgrad(x: torch.Tensor, dys) -> list:
-    """dy^T x for every dy [T, O] of `dys` (at most four, one row stride for all where they are not dense), x [T, I]: the
-    weight gradients of projections of one input, bf16."""
+    """dy^T x for every dy [T, O] of `dys` (at most four), x [T, I]: the weight gradients of projections of one input, bf16."""
     lib = _lib.load()
+    if not 1 <= len(dys) <= 4 or x.dim() != 2 or any(dy.dim() != 2 or dy.shape[0] != x.shape[0] for dy in dys):
+        raise ValueError(f"nha_wgrad takes x [T, I] and one to four dy [T, O], got {[tuple(t.shape) for t in (x, *dys)]}")
+    if any(t.dtype != torch.bfloat16 or not t.is_cuda or t.device != x.device for t in (x, *dys)):
+        raise TypeError("nha_wgrad takes bfloat16 tensors on one GPU")
+    x = x.contiguous()
     T, width = x.shape
+    # columns of one matrix are read where they are; rows that lie otherwise are made dense
+    ldy = 0
+    if not all(dy.is_contiguous() for dy in dys):
+        ldy = dys[0].stride(0)
+        if ldy % 8 or any(dy.stride() != (ldy, 1) or dy.shape[1] > ldy for dy in dys):
+            dys, ldy = [dy.contiguous() for dy in dys], 0
     outs = [torch.empty(dy.shape[1], width, dtype=x.dtype, device=x.device) for dy in dys]
-    a = _lib.NhaWgradArgs(x=_ptr(x), n=len(outs), T=T, I=width, ldy=0 if all(dy.is_contiguous() for dy in dys) else dys[0].stride(0), stream=_stream(x.device))
+    a = _lib.NhaWgradArgs(x=_ptr(x), n=len(outs), T=T, I=width, ldy=ldy, stream=_stream(x.device))
     for i, (dy, dw) in enumerate(zip(dys, outs)):
         a.dy[i], a.dw[i], a.O[i] = _ptr(dy), _ptr(dw), dy.shape[1]
     nbytes = lib.nha_wgrad_scratch_bytes(C.byref(a))

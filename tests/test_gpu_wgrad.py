@@ -31,6 +31,31 @@ def test_wgrad_row_stride():
     assert all(torch.equal(a, b) for a, b in zip(dense, nha_wgrad(x, [both[:, :264], both[:, 264:]])))
 
 
+@pytest.mark.parametrize("case", ["dense beside columns", "columns beside dense", "two matrices", "expanded", "every second column", "x of a matrix"])
+def test_wgrad_rows_of_different_strides(case):
+    """Gradients whose rows do not lie one common stride apart, 16-byte pieces within them, are the same as dense ones."""
+    from nha_amd.ops import nha_wgrad
+    r = lambda *s: torch.randn(*s, device="cuda").bfloat16()
+    x, wide, other = r(130, 72), r(130, 344), r(130, 64)
+    dys = {"dense beside columns": [r(130, 64), wide[:, :264]], "columns beside dense": [wide[:, 264:], r(130, 64)],
+           "two matrices": [wide[:, :64], other[:, 8:16]], "expanded": [r(1, 64).expand(130, 64), wide[:, :8]],
+           "every second column": [wide[:, ::2][:, :64]], "x of a matrix": [r(130, 64)]}[case]
+    if case == "x of a matrix":
+        x = r(130, 144)[:, ::2]
+    dense = nha_wgrad(x.contiguous(), [dy.contiguous() for dy in dys])
+    assert all(torch.equal(a, b) for a, b in zip(dense, nha_wgrad(x, dys)))
+
+
+def test_wgrad_refuses_tensors_that_do_not_fit():
+    from nha_amd.ops import nha_wgrad
+    x, dy = torch.randn(64, 32, device="cuda").bfloat16(), torch.randn(60, 16, device="cuda").bfloat16()
+    for bad in ([dy], [], [dy] * 5):
+        with pytest.raises(ValueError):
+            nha_wgrad(x, bad)
+    with pytest.raises(TypeError):
+        nha_wgrad(x, [x.float()])
+
+
 def test_wgrad_scratch_is_its_own(monkeypatch):
     """The partial sums lie between two launches: not in the workspace that every call of a stream shares, which another thread
     may queue a call on in between."""
