@@ -8,7 +8,7 @@
 //
 // Bound: LDS.  A workgroup of eight waves (128 x 64 of the tile each, two per SIMD) reads 197 KB and writes 64 KB of LDS
 // per 64 tokens, as many clocks as its matrix products take.  16384 tokens, 1024 columns, outputs of 3 x 1024 + 256: 138 us
-// with the sum (0.87 PFLOP/s) against 415 us for four library products, which run 64 x 64 tiles without a split; one output
+// with the sum (0.81 PFLOP/s) against 415 us for four library products, which run 64 x 64 tiles without a split; one output
 // of 1024: 54 against 104 us; 2048 columns, 2048 + 2 x 512 + 256: 250 against 468 us.
 #include "mfma_common.h"
 
@@ -140,8 +140,8 @@ __global__ __launch_bounds__(256) void wgrad_sum_kernel(const WG p) {
   Elem<bf16_t>::st8(p.dw[q] + (int64_t)(r - p.row0[q]) * p.I + c, s);
 }
 
-// Token splits: a round of the chip is 256 workgroups; a step of 64 tokens costs STEP and a workgroup's start and end FIXED,
-// a split's round trip in fp32 its bytes.
+// Token splits: a round of the chip is 256 workgroups; a step of 64 tokens costs 1.4 us and a workgroup's start and end 6,
+// a split's round trip in fp32 its bytes (4 written and 4 read per element) at 4.5 TB/s.
 int wgrad_split(int tiles, int T, int64_t elements) {
   const int steps = (T + TK - 1) / TK;
   int best = 1;

@@ -483,13 +483,18 @@ def nha_wgrad(x: torch.Tensor, dys) -> list:
 
 
 def _wgrad_supported(x: torch.Tensor, dys) -> bool:
-    """Rows of 16-byte pieces, bf16.  A single gradient of few tokens stays with the library: 1024 x 1024 from 4096 tokens
-    takes it 29 us against 34, from 6000 45 against 39, from 16384 104 against 54.  Several at once are faster from any
-    number (1024 columns, outputs of 3 x 1024 + 256 from 300 tokens: 28 us against 78 for four library calls)."""
+    """Rows of 16-byte pieces, bf16, and sizes at which nha_wgrad is the faster one.  A single gradient of few tokens stays with
+    the library: 1024 x 1024 from 4096 tokens takes it 30 us against 34, from 6000 45 against 39, from 16384 102 against 54;
+    2048 x 2048 from 6000 72 against 67.  Several at once are faster from any number (1024 columns, outputs of 3 x 1024 + 512
+    from 300 tokens: 28 us against 76 for four library calls).  Large weights are the library's, whose tiles of 256 columns fill
+    the chip without a split there: a single 3072 x 3072 from 16384 tokens 303 us against 325; 3072 columns, 3072 + 2 x 768 + 512
+    (15.7 M elements) from 1024 tokens 77 against 59, from 16384 703 against 488, but 4096 columns, 4096 + 2 x 1024 + 512 (27 M)
+    80 against 100 and 916 against 902, and 3 x 4096 + 512 (52 M) 124 against 193 and 1512 against 1707."""
     T, width = x.shape
+    elements = sum(dy.shape[1] for dy in dys) * width
     return (x.dtype == torch.bfloat16 and 0 < T <= 1 << 30 and width % 8 == 0 and x.data_ptr() % 16 == 0 and len(dys) <= 4
             and all(dy.dtype == x.dtype and dy.shape[1] % 8 == 0 and dy.data_ptr() % 16 == 0 for dy in dys)
-            and sum(dy.shape[1] for dy in dys) * width < 1 << 31 and (len(dys) > 1 or T >= 6000))
+            and (elements <= 1 << 24 if len(dys) > 1 else elements <= 1 << 22 and T >= 6000))
 
 
 class _SharedInputLinear(torch.autograd.Function):

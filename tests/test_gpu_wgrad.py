@@ -112,6 +112,23 @@ def test_layer_projections(case):
         assert ((g.double() - r.double()).norm() / r.double().norm()).item() <= 1e-2
 
 
+def test_wide_layer_projections():
+    """Weights past the size that nha_wgrad takes: the node's gradients are the library's."""
+    from nha_amd.ops import nha_layer_prologue
+    torch.manual_seed(8)
+    modules = [torch.nn.Linear(4096, n, bias=False).cuda().bfloat16() for n in (4096, 1024, 1024, 512)]
+    inv = 10000.0 ** (-torch.arange(0, 128, 2, device="cuda").float() / 128)
+    x = torch.randn(2, 40, 4096, device="cuda").bfloat16().requires_grad_()
+    leaves, grads = [x, *(m.weight for m in modules)], []
+    kw = dict(feature_map="swish", gate_logit_normalizer=8)
+    for one in (True, False):
+        out = nha_layer_prologue(None, None, None, None, inv, projections=(x, modules, (32, 8, 128, 128, 64)), **kw) if one else \
+            nha_layer_prologue(*(m(x).unflatten(-1, (h, -1)) for m, h in zip(modules, (32, 8, 8, 8))), inv, **kw)
+        grads.append(torch.autograd.grad([t.float().pow(2).sum() for t in out], leaves))
+    for a, b in zip(*grads):      # q, k, v, f from one product or four, dx of one or four: roundings of 2^-8
+        assert ((a.double() - b.double()).norm() / b.double().norm()).item() <= 1e-2
+
+
 def test_second_derivative_of_the_projections():
     from nha_amd.ops import shared_input_linears
     lin = [torch.nn.Linear(64, o, bias=False).cuda().bfloat16() for o in (32, 16)]
