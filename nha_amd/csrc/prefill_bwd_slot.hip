@@ -417,8 +417,10 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
 #pragma unroll
         for (int blk = 0; blk < 4; ++blk)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)   // A is zero for rows before j
-            cU[blk][e] += bf16_to_f32(AT[j * TLD + 16 * blk + 4 * kb + e]) * sj * expf(fminf(gi[blk][e] - gj, 0.f));
+          for (int e = 0; e < 4; ++e) {
+            const float w = bf16_to_f32(AT[j * TLD + 16 * blk + 4 * kb + e]) * sj * expf(gi[blk][e] - gj);
+            cU[blk][e] += 16 * blk + 4 * kb + e >= j ? w : 0.f;   // (for rows before j the factor grows, out of range even)
+          }
       }
     if constexpr (KEEP) row_delta(orow, hq, lane);
 #pragma unroll
@@ -516,7 +518,7 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const int i = 16 * blk + 4 * kb + e;
-              if (i >= col) c[blk][e] += ep[i * MS + m] * sr * expf(fminf(gc[i * MS + m] - gr, 0.f));
+              if (i >= col) c[blk][e] += ep[i * MS + m] * sr * expf(gc[i * MS + m] - gr);
             }
         }
       for (int i = 0; i < R; ++i) {
@@ -524,8 +526,10 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)   // gi: the gate rows of r = 16 rb + 4 kb + e
-            accS[rb][e] += bf16_to_f32(AT[(16 * rb + 4 * kb + e) * TLD + i]) * x * expf(fminf(g - gi[rb][e], 0.f));
+          for (int e = 0; e < 4; ++e) {   // gi: the gate rows of r = 16 rb + 4 kb + e
+            const float w = bf16_to_f32(AT[(16 * rb + 4 * kb + e) * TLD + i]) * x * expf(g - gi[rb][e]);
+            accS[rb][e] += i >= 16 * rb + 4 * kb + e ? w : 0.f;
+          }
       }
     }
     if constexpr (EXACT) __syncthreads();

@@ -34,3 +34,14 @@ def test_slot_branch_strong_gates(D, gate_mean):
     d = prefill_inputs(8200 + D, 1, CU[-1], 4, 2, D, D, 64, dtype=BF, qk_scale=D ** -0.5, gate_div=1.0, gate_mean=gate_mean,
                        with_state=True, N=len(CU) - 1)
     run_bwd_case(f"slot strong {gate_mean} D{D}", d, wl=40, shift=0, dtype=BF, cu=CU, with_lse=True)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_slot_branch_growing_gates_beside_strong_ones(D):
+    """Slots that grow (log gates up to +0.01) in chunks that others make strongly decaying: the decay of a pair is formed as it
+    is, above 1 too."""
+    d = prefill_inputs(8300 + D, 1, CU[-1], 4, 2, D, D, 64, dtype=BF, qk_scale=D ** -0.5, gate_div=1.0, gate_mean=-5.0,
+                       with_state=True, N=len(CU) - 1)
+    d["g"][..., 8:] = (d["g"][..., 8:] / -400).clamp(0, 0.01)
+    d["s"][..., 8:] = (d["s"][..., 8:] / 20)
+    run_bwd_case(f"slot growing D{D}", d, wl=40, shift=0, dtype=BF, cu=CU, with_lse=True)
