@@ -138,7 +138,11 @@ struct Operands {
 };
 
 // EXACT: the chunks in which some slot decays by more than e^-BWD_DECAY_CLAMP within a 32-row half (the growing factor of the
-// split decay would leave the range), with the decay of every pair formed on its own in fp32; the other launch skips them.
+// split decay would leave the range); the other launch skips them.  Pairs of rows in different 16-row blocks take the cumsum
+// at the start of the later row's block as their reference, both factors then shrink (Tb: X and Xp against their own block);
+// pairs within a block have their decay formed one by one in fp32.  With all pairs of the chunk one by one this launch was slower
+// than the VALU kernels that it replaced: backward of 4000 tokens, every chunk strongly decaying, 32/8 heads of 128 1985 us with
+// those, 2702 with all pairs, 1142 like this; 3000 tokens, 4 heads of 256 525 / 802 / 413; 5000, 16 of 64 1040 / 1735 / 720.
 // DW: the output columns x of a workgroup.  Half of the 256 of the largest head: a workgroup of all would hold 128 sums per
 // lane next to its operands and tiles of 66 KB; the products over all columns (A, B, U, P0, delta) are formed twice instead,
 // from the other columns of q and do in the room of the state tiles and operands streamed two steps at a time.
@@ -172,6 +176,7 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
   lbf16* const Z = sm + L::S + (vs ? L::TILE : 0);               // its other columns (until the state tiles are written)
   lbf16* const T0h = sm + L::X0 + (vs ? 2 * L::TAB : 0), * const T0l = T0h + L::TAB;   // X0 or Xp0
   lbf16* const T1h = sm + L::X1 + (vs ? 2 * L::HTAB : 0), * const T1l = T1h + L::HTAB;
+  lbf16* const Tbh = sm + (vs ? L::Y : L::X1), * const Tbl = Tbh + L::TAB;   // EXACT has neither Y nor X1
   lbf16* const AT = sm + L::A + (vs ? L::TAB : 0);               // A or B
   lbf16* const Ch = sm + L::C + (vs ? 2 * L::TAB : 0), * const Cl = Ch + L::TAB;
   lfloat* const rdelta = (lfloat*)(NHA_LDS void*)(sm + L::ROW), * const rlse = rdelta + BT, * const rlg = rlse + BT, * const rdlg = rlg + BT;
@@ -284,11 +289,12 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
     for (int ks = 0; ks < (KEEP ? KS : 2); ++ks) load_operands(ks, ks, lane0);
     FENCE;
     if (!EXACT && !mine()) return;
+    if constexpr (!EXACT)
 #pragma unroll
     for (int e = 0; e < 8; e += 4) {
       f32x4 yv;
 #pragma unroll
-      for (int x = 0; x < 4; ++x) yv[x] = live && !EXACT ? sv[e + x] * __expf((j >= 32 ? ref[e + x] : 0.f) - g[e + x]) : 0.f;
+      for (int x = 0; x < 4; ++x) yv[x] = live ? sv[e + x] * __expf((j >= 32 ? ref[e + x] : 0.f) - g[e + x]) : 0.f;
       put4_pair(sm + L::Y, sm + L::Y + L::TAB, j * TLD + m8 + e, yv);
     }
     store_head(head, lane0);
@@ -388,40 +394,76 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
     const float g31 = ld_at<float>(gc + 31 * MS, col * 4);
     lds_barrier();
     // ---- u (k side) or dp (v side) of rows 16 blk + 4 kb + e, slot col, to the other side ------------------------------
-    bf16x8 yf[2][2];
-#pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      yf[hf][0] = lds_frag_tr(Yh, TLD, 32 * hf, 32 * hf + 16, 16 * w, lane);
-      yf[hf][1] = lds_frag_tr(Yl, TLD, 32 * hf, 32 * hf + 16, 16 * w, lane);
-    }
-#pragma unroll
-    for (int blk = 0; blk < 4; ++blk) {
-      f32x4 c[2];
+    if constexpr (!EXACT) {
+      bf16x8 yf[2][2];
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
-        c[hf] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        if (EXACT || 2 * hf > blk) continue;   // rows of the first half see none of the second
-        const bf16x8 x = lds_frag_tr(AT, TLD, 32 * hf, 32 * hf + 16, 16 * blk, lane);
-        c[hf] = mfma16(x, yf[hf][0], mfma16(x, yf[hf][1], c[hf]));
+        yf[hf][0] = lds_frag_tr(Yh, TLD, 32 * hf, 32 * hf + 16, 16 * w, lane);
+        yf[hf][1] = lds_frag_tr(Yl, TLD, 32 * hf, 32 * hf + 16, 16 * w, lane);
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float e0 = __expf(gi[blk][e]), e1 = blk >= 2 ? __expf(gi[blk][e] - g31) : 0.f;
-        cU[blk][e] = e0 * (cU[blk][e] + c[0][e]) + e1 * c[1][e];
-      }
-      FENCE;
-    }
-    if constexpr (EXACT)
-      for (int j = vlo; j < R; ++j) {
-        const float sj = bf16_to_f32(p.s[(((int64_t)c0 + j - p.shift) * H + h) * MS + col]), gj = gc[j * MS + col];
+      for (int blk = 0; blk < 4; ++blk) {
+        f32x4 c[2];
 #pragma unroll
-        for (int blk = 0; blk < 4; ++blk)
+        for (int hf = 0; hf < 2; ++hf) {
+          c[hf] = (f32x4){0.f, 0.f, 0.f, 0.f};
+          if (2 * hf > blk) continue;   // rows of the first half see none of the second
+          const bf16x8 x = lds_frag_tr(AT, TLD, 32 * hf, 32 * hf + 16, 16 * blk, lane);
+          c[hf] = mfma16(x, yf[hf][0], mfma16(x, yf[hf][1], c[hf]));
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float e0 = __expf(gi[blk][e]), e1 = blk >= 2 ? __expf(gi[blk][e] - g31) : 0.f;
+          cU[blk][e] = e0 * (cU[blk][e] + c[0][e]) + e1 * c[1][e];
+        }
+        FENCE;
+      }
+    } else {
+      float sj[4][4];   // strengths of the rows 16 blk + 4 kb + e
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int j = 16 * blk + 4 * kb + e;
+          const bool on = j >= vlo && j < R;
+          const float x = bf16_to_f32(p.s[((int64_t)(on ? c0 + j - p.shift : bos) * H + h) * MS + col]);
+          sj[blk][e] = on ? x : 0.f;
+        }
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk) {
+        f32x4 c = {0.f, 0.f, 0.f, 0.f};
+        const float ref = blk ? ld_at<float>(gc + (16 * blk - 1) * MS, col * 4) : 0.f;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {   // earlier blocks against ref
+          if (2 * hf >= blk) continue;
+          bf16x8 yh, yl;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int bj = 2 * hf + (e >> 2);
+            const float y = bj < blk ? sj[bj][e & 3] * expf(ref - gi[bj][e & 3]) : 0.f;
+            yh[e] = (__bf16)y;
+            yl[e] = (__bf16)(y - (float)yh[e]);
+          }
+          const bf16x8 x = lds_frag_tr(AT, TLD, 32 * hf, 32 * hf + 16, 16 * blk, lane);
+          c = mfma16(x, yh, mfma16(x, yl, c));
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) cU[blk][e] = expf(gi[blk][e]) * cU[blk][e] + (blk ? expf(gi[blk][e] - ref) * c[e] : 0.f);
+#pragma unroll 4
+        for (int jj = 0; jj < 16; ++jj) {   // the block itself (A is zero for rows before j, whose factor may leave the range)
+          const int j = 16 * blk + jj;
+          const bool on = j >= vlo && j < R;
+          const float s = bf16_to_f32(p.s[((int64_t)(on ? c0 + j - p.shift : bos) * H + h) * MS + col]), gj = gc[j * MS + col];
+          const bf16x4 a = *reinterpret_cast<const NHA_LDS bf16x4*>(AT + j * TLD + 16 * blk + 4 * kb);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float w = bf16_to_f32(AT[j * TLD + 16 * blk + 4 * kb + e]) * sj * expf(gi[blk][e] - gj);
-            cU[blk][e] += 16 * blk + 4 * kb + e >= j ? w : 0.f;   // (for rows before j the factor grows, out of range even)
+            const float x = (float)a[e] * s * expf(gi[blk][e] - gj);
+            cU[blk][e] += on && 4 * kb + e >= jj ? x : 0.f;
           }
+        }
+        FENCE;
       }
+    }
     if constexpr (KEEP) row_delta(orow, hq, lane);
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) {
@@ -451,15 +493,21 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
         for (int e = 0; e < 4; ++e) du[e] += dg[e] * __expf(u[e] - lg[e]);
       }
       f32x4 t0, t1;
+      float own[4];
+      if constexpr (EXACT)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) own[e] = blk ? gi[blk][e] - ld_at<float>(gc + (16 * blk - 1) * MS, col * 4) : gi[blk][e];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float x = i0 + e < R ? (vs ? pm[e] : p.scale * du[e]) : 0.f;
-        t0[e] = x * __expf(gi[blk][e]);
-        if (blk >= 2) t1[e] = x * __expf(gi[blk][e] - g31);
+        t0[e] = x * (EXACT ? expf(gi[blk][e]) : __expf(gi[blk][e]));
+        if constexpr (EXACT) t1[e] = x * expf(own[e]);
+        else if (blk >= 2) t1[e] = x * __expf(gi[blk][e] - g31);
         if constexpr (EXACT) ep[(i0 + e) * MS + col] = x;   // undecayed, for the pairwise sums (N takes the place afterwards)
       }
       put4_pair(T0h, T0l, col * TLD + i0, t0);
-      if (!EXACT && blk >= 2) put4_pair(T1h, T1l, col * HLD + i0 - 32, t1);
+      if constexpr (EXACT) put4_pair(Tbh, Tbl, col * TLD + i0, t1);
+      else if (blk >= 2) put4_pair(T1h, T1l, col * HLD + i0 - 32, t1);
       if (vs == (blk >= 2)) xg[blk & 1] += du * u + pm * dp;
       FENCE;
     }
@@ -510,26 +558,86 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
       }
     } else {
       const int tl = it * BT + col - p.shift;
-      if (col < R && tl >= 0)
-        for (int m = 0; m < MS; ++m) {
-          const float sr = bf16_to_f32(p.s[((int64_t)(bos + tl) * H + h) * MS + m]), gr = gc[col * MS + m];
+      const bool on = col < R && tl >= 0;
+      const bf16_t* const sr = p.s + ((int64_t)(on ? bos + tl : bos) * H + h) * MS;
+      // rows i of later blocks than r's: against the start of their block
 #pragma unroll
-          for (int blk = 0; blk < 4; ++blk)
+      for (int ks = 0; ks < 2; ++ks) {
+        float y[8], g[8];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int i = 16 * blk + 4 * kb + e;
-              if (i >= col) c[blk][e] += ep[i * MS + m] * sr * expf(gc[i * MS + m] - gr);
-            }
+        for (int q = 0; q < 2; ++q) {
+          const int m = 32 * ks + 16 * q + 4 * kb;
+          const bf16x4 sv = *reinterpret_cast<const bf16x4*>(sr + m);
+          const f32x4 gv = *reinterpret_cast<const f32x4*>(gc + col * MS + m);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[4 * q + e] = on ? (float)sv[e] : 0.f, g[4 * q + e] = gv[e];
         }
-      for (int i = 0; i < R; ++i) {
-        const float x = ep[i * MS + col], g = gc[i * MS + col];
 #pragma unroll
-        for (int rb = 0; rb < 4; ++rb)
+        for (int blk = 1; blk < 4; ++blk) {
+          if (blk <= w) continue;
+          const f32x4 ra = *reinterpret_cast<const f32x4*>(gc + (16 * blk - 1) * MS + 32 * ks + 4 * kb);
+          const f32x4 rb = *reinterpret_cast<const f32x4*>(gc + (16 * blk - 1) * MS + 32 * ks + 16 + 4 * kb);
+          bf16x8 yh, yl;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {   // gi: the gate rows of r = 16 rb + 4 kb + e
-            const float w = bf16_to_f32(AT[(16 * rb + 4 * kb + e) * TLD + i]) * x * expf(g - gi[rb][e]);
-            accS[rb][e] += i >= 16 * rb + 4 * kb + e ? w : 0.f;
+          for (int e = 0; e < 8; ++e) {
+            const float v = y[e] * expf((e < 4 ? ra[e & 3] : rb[e & 3]) - g[e]);
+            yh[e] = (__bf16)v;
+            yl[e] = (__bf16)(v - (float)yh[e]);
           }
+          const bf16x8 xh = lds_frag_tr(Tbh, TLD, 32 * ks, 32 * ks + 16, 16 * blk, lane);
+          const bf16x8 xl = lds_frag_tr(Tbl, TLD, 32 * ks, 32 * ks + 16, 16 * blk, lane);
+          c[blk] = mfma16(xh, yh, mfma16(xh, yl, mfma16(xl, yh, c[blk])));
+        }
+        FENCE;
+      }
+      // rows i of r's block, four slots at a time
+      f32x4 own = {0.f, 0.f, 0.f, 0.f};
+      for (int m = 0; m < MS; m += 4) {
+        const bf16x4 sv = *reinterpret_cast<const bf16x4*>(sr + m);
+        const f32x4 gr = *reinterpret_cast<const f32x4*>(gc + col * MS + m);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = 16 * w + 4 * kb + e;
+          const f32x4 x = *reinterpret_cast<const f32x4*>(ep + i * MS + m), g = *reinterpret_cast<const f32x4*>(gc + i * MS + m);
+          float z = 0.f;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) z += x[u] * (float)sv[u] * expf(g[u] - gr[u]);
+          own[e] += on && i >= col ? z : 0.f;
+        }
+      }
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk)
+        if (blk == w) c[blk] = own;
+      // ds_intra of rows r = 16 rb + 4 kb + e
+#pragma unroll
+      for (int bi = 1; bi < 4; ++bi) {
+        bf16x8 xh = col_frag(Tbh, TLD, col, 32 * (bi >> 1), kb), xl = col_frag(Tbl, TLD, col, 32 * (bi >> 1), kb);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if ((e >> 2) != (bi & 1)) xh[e] = xl[e] = (__bf16)0.f;   // the other block of the half
+        const float ref = ld_at<float>(gc + (16 * bi - 1) * MS, col * 4);
+#pragma unroll
+        for (int rb = 0; rb < bi; ++rb) {
+          const bf16x8 af = col_frag(AT, TLD, 16 * rb + l16, 32 * (bi >> 1), kb);
+          const f32x4 z = mfma16(af, xh, mfma16(af, xl, (f32x4){0.f, 0.f, 0.f, 0.f}));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) accS[rb][e] += z[e] * expf(ref - gi[rb][e]);
+        }
+        FENCE;
+      }
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) {
+#pragma unroll 4
+        for (int ii = 0; ii < 16; ++ii) {
+          const int i = 16 * rb + ii;
+          const float x = ep[i * MS + col], g = gc[i * MS + col];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float z = bf16_to_f32(AT[(16 * rb + 4 * kb + e) * TLD + i]) * x * expf(g - gi[rb][e]);
+            accS[rb][e] += ii >= 4 * kb + e ? z : 0.f;
+          }
+        }
+        FENCE;
       }
     }
     if constexpr (EXACT) __syncthreads();
