@@ -43,7 +43,7 @@ constexpr int HLD = 36;    // row stride of the tables that hold rows 32..63 onl
 
 __device__ __forceinline__ float logaddexp_f(float a, float b) {
   const float mx = fmaxf(a, b);
-  return mx + logf(__expf(a - mx) + __expf(b - mx));
+  return mx + logf(expf(a - mx) + expf(b - mx));
 }
 
 // 8 rows of column n of a transposed table tab[n][row]: rows r0 + 4 kb + e and r0 + 16 + 4 kb + e (the numbering of a
@@ -484,13 +484,13 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
       f32x4 u = vs ? other[blk] : cU[blk], dp = vs ? cU[blk] : other[blk], pm, du;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        pm[e] = __expf(u[e] - lt[e]);
+        pm[e] = EXACT ? expf(u[e] - lt[e]) : __expf(u[e] - lt[e]);
         du[e] = pm[e] * (dp[e] - dl[e]);
       }
       if (p.dlse_gsa) {
         const f32x4 lg = *reinterpret_cast<const NHA_LDS f32x4*>(rlg + i0), dg = *reinterpret_cast<const NHA_LDS f32x4*>(rdlg + i0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) du[e] += dg[e] * __expf(u[e] - lg[e]);
+        for (int e = 0; e < 4; ++e) du[e] += dg[e] * (EXACT ? expf(u[e] - lg[e]) : __expf(u[e] - lg[e]));
       }
       f32x4 t0, t1;
       float own[4];
