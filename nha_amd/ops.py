@@ -602,17 +602,23 @@ def _front_columns(raw: torch.Tensor, dims):
 _LINEAR_FORWARD = torch.nn.Linear.forward
 
 
+def _for_one_node(x: torch.Tensor) -> bool:
+    """Whether it is worth looking over the modules: not in inference (10 us of host time per layer call), nor where the look
+    itself would be compiled."""
+    return torch.is_grad_enabled() and not torch.compiler.is_compiling() and x.is_cuda and x.dtype == torch.bfloat16
+
+
 def _one_node(x: torch.Tensor, weights) -> bool:
     """Whether a node of our own may stand for F.linear of x with every weight: something to differentiate, and nothing
     besides reverse-mode autograd that looks at the call (autocast, tracing, modes, transforms, subclasses)."""
-    return (x.is_cuda and x.dtype == torch.bfloat16 and torch.is_grad_enabled() and not torch.compiler.is_compiling()
-            and not torch.is_autocast_enabled("cuda") and all(w.dtype == x.dtype and w.device == x.device for w in weights)
+    return (_for_one_node(x) and not torch.is_autocast_enabled("cuda")
+            and all(w.dtype == x.dtype and w.device == x.device for w in weights)
             and any(t.requires_grad for t in (x, *weights)) and _plain_autograd((x, *weights)))
 
 
 def _plain_modules(modules) -> bool:
     """nn.Linear modules without bias, hooks or a forward of their own."""
-    return (not torch.compiler.is_compiling() and torch.nn.Linear.forward is _LINEAR_FORWARD
+    return (torch.nn.Linear.forward is _LINEAR_FORWARD
             and not torch.nn.modules.module._has_any_global_hook()
             and all(type(m) is torch.nn.Linear and "forward" not in m.__dict__ and m.bias is None
                     and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
@@ -621,7 +627,7 @@ def _plain_modules(modules) -> bool:
 
 def shared_input_linears(x: torch.Tensor, modules):
     """[m(x) for m in modules], as one autograd node where it may be one."""
-    weights = [m.weight for m in modules] if _plain_modules(modules) else None
+    weights = [m.weight for m in modules] if _for_one_node(x) and _plain_modules(modules) else None
     if weights is not None and _one_node(x, weights):
         return _SharedInputLinear.apply(x, *weights)
     return tuple(m(x) for m in modules)
@@ -631,7 +637,7 @@ def layer_front_supported(x: torch.Tensor, modules, dims) -> bool:
     """Whether nha_layer_prologue takes (x, modules, dims) as its projections: plain modules whose products with x
     [B, T, hidden] and the prologue may be one autograd node.  dims: query heads, kv-heads, key size, value size, slots."""
     HQ, H, K, V, M = dims
-    if not _plain_modules(modules) or x.dim() != 3 or x.numel() == 0 or K % 2 or K > 1024:
+    if not _for_one_node(x) or not _plain_modules(modules) or x.dim() != 3 or x.numel() == 0 or K % 2 or K > 1024:
         return False
     weights = [m.weight for m in modules]
     return (all(tuple(w.shape) == (n, x.shape[-1]) and n % 8 == 0 for w, n in zip(weights, (HQ * K, H * K, H * V, H * M)))

@@ -129,6 +129,16 @@ def test_wide_layer_projections():
         assert ((a.double() - b.double()).norm() / b.double().norm()).item() <= 1e-2
 
 
+@pytest.mark.parametrize("case", ["no grad", "fp32"])
+def test_calls_that_cannot_be_one_node_look_at_no_module(case, monkeypatch):
+    from nha_amd import ops
+    layer, seen = _layer().to(torch.float32 if case == "fp32" else torch.bfloat16), []
+    monkeypatch.setattr(ops, "_plain_modules", lambda m: seen.append(m) or False)
+    x = torch.randn(1, 50, 256, device="cuda", dtype=layer.q_proj.weight.dtype)
+    with torch.set_grad_enabled(case != "no grad"):
+        assert layer(x)[0].isfinite().all() and not seen
+
+
 def test_second_derivative_of_the_projections():
     from nha_amd.ops import shared_input_linears
     lin = [torch.nn.Linear(64, o, bias=False).cuda().bfloat16() for o in (32, 16)]
