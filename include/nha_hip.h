@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define NHA_ABI_VERSION 11
+#define NHA_ABI_VERSION 12
 
 enum { NHA_DTYPE_F32 = 0, NHA_DTYPE_BF16 = 1 };
 enum {
@@ -233,6 +233,9 @@ typedef struct NhaDecodeArgs {
 
 /* Bytes of NhaDecodeArgs.scratch, the same for every call. */
 size_t nha_decode_scratch_bytes(void);
+/* 1 if nha_decode_step(a), given scratch, spreads a (sequence, kv-head) pair over several workgroups; 0: it leaves the scratch
+ * alone.  Looks at sizes, types and addresses only, not at a->scratch. */
+int nha_decode_uses_scratch(const NhaDecodeArgs* a);
 int nha_decode_step(const NhaDecodeArgs* a);
 /* count[b] += 1 for b < B (ring mode bookkeeping between steps). */
 int nha_decode_advance(int32_t* count, int32_t B, void* stream);

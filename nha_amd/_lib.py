@@ -15,14 +15,14 @@ NHA_DTYPE_F32, NHA_DTYPE_BF16 = 0, 1
 NHA_IMPL_AUTO, NHA_IMPL_SIMPLE, NHA_IMPL_MFMA = 0, 1, 2
 NHA_DECODE_WINDOW, NHA_DECODE_LOGITS, NHA_DECODE_RING = 0, 1, 2
 NHA_OK, NHA_ERR_INVALID, NHA_ERR_UNSUPPORTED, NHA_ERR_SCRATCH, NHA_ERR_LAUNCH = 0, -1, -2, -3, -4
-ABI_VERSION = 11
+ABI_VERSION = 12
 NHA_NOALLOC_SCRATCH_BYTES = 32 << 20   # workspace of nha_prefill_fwd_noalloc (include/nha_hip.h)
 NHA_FMAP_NONE, NHA_FMAP_SWISH, NHA_FMAP_RELU = 0, 1, 2
 
 EXPORTS = (
     "nha_ring_fill", "nha_wgrad", "nha_wgrad_scratch_bytes", "nha_gsa_share", "nha_layer_prologue_rows", "nha_layer_prologue_bwd_rows",
     "nha_prefill_scratch_bytes", "nha_prefill_fwd", "nha_prefill_fwd_noalloc", "nha_prefill_bwd_scratch_bytes", "nha_prefill_bwd",
-    "nha_decode_scratch_bytes", "nha_decode_step", "nha_decode_advance", "nha_layer_prologue", "nha_layer_epilogue",
+    "nha_decode_scratch_bytes", "nha_decode_uses_scratch", "nha_decode_step", "nha_decode_advance", "nha_layer_prologue", "nha_layer_epilogue",
     "nha_layer_prologue_bwd", "nha_layer_epilogue_bwd", "nha_layer_epilogue_bwd_parts",
     "nha_short_conv", "nha_short_conv_bwd", "nha_short_conv_bwd_parts", "nha_hybrid_prologue", "nha_zero_sink_rescale", "nha_sink_window_fwd", "nha_sink_window_scratch_bytes",
     "nha_varlen_num_chunks", "nha_varlen_indices", "nha_last_error", "nha_abi_version",
@@ -193,6 +193,12 @@ def packer(cls):
 
 
 pack_decode = packer(NhaDecodeArgs)
+_PACK_SCRATCH = struct.Struct("@PN").pack      # the last two fields
+
+
+def with_scratch(args: bytes, scratch: int, nbytes: int) -> bytes:
+    """The block of pack_decode with another scratch."""
+    return args[:-16] + _PACK_SCRATCH(scratch, nbytes)
 
 
 class NhaError(RuntimeError):
@@ -229,6 +235,9 @@ def load() -> C.CDLL:
     lib.nha_decode_step.argtypes = [C.POINTER(NhaDecodeArgs)]
     # the same entry for an argument block packed by pack_decode
     lib.decode_step_packed = C.CFUNCTYPE(C.c_int, C.c_char_p)(("nha_decode_step", lib))
+    lib.nha_decode_uses_scratch.restype = C.c_int
+    lib.nha_decode_uses_scratch.argtypes = [C.POINTER(NhaDecodeArgs)]
+    lib.decode_uses_scratch_packed = C.CFUNCTYPE(C.c_int, C.c_char_p)(("nha_decode_uses_scratch", lib))
     lib.nha_decode_advance.restype = C.c_int
     lib.nha_decode_advance.argtypes = [C.c_void_p, C.c_int32, C.c_void_p]
     lib.nha_ring_fill.restype = C.c_int

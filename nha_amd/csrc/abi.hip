@@ -195,6 +195,10 @@ int nha_prefill_bwd(const NhaPrefillBwdArgs* a) {
 
 size_t nha_decode_scratch_bytes(void) { return decode_scratch_bytes(); }
 
+int nha_decode_uses_scratch(const NhaDecodeArgs* a) {
+  return a && a->B > 0 && a->H > 0 && a->HQ > 0 && a->W > 0 && a->HQ % a->H == 0 && decode_mfma_supported(a) && decode_split_uses_scratch(a);
+}
+
 int nha_decode_step(const NhaDecodeArgs* a) { return decode_step_impl(a); }
 
 int nha_decode_advance(int32_t* count, int32_t B, void* stream) { return decode_advance_impl(count, B, stream); }

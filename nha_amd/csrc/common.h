@@ -150,6 +150,7 @@ int decode_mfma_impl(const NhaDecodeArgs* a);
 // decode_split.hip: the calls of decode_mfma_impl with too few (sequence, kv-head) pairs to fill the chip
 size_t decode_scratch_bytes();
 bool decode_split_wanted(const NhaDecodeArgs* a);
+bool decode_split_uses_scratch(const NhaDecodeArgs* a);
 int decode_split_impl(const NhaDecodeArgs* a);
 size_t prefill_simple_scratch_bytes(const NhaPrefillArgs* a);
 // phase: 0 = whole op, 1 = state pass only, 2 = output pass only (scratch filled by an earlier state pass)

@@ -630,13 +630,19 @@ int dispatch(const NhaDecodeArgs* a, int G, int P) {
 // heads per kv-head.
 size_t decode_scratch_bytes() { return MAX_SPLIT * 4 + (size_t)CUS * (8 * 256 + 2 * 8) * 4; }
 
-bool decode_split_wanted(const NhaDecodeArgs* a) {
+// Workgroups per pair at these addresses too; 0 as in split_of.
+static int split_at(const NhaDecodeArgs* a) {
   // decode_mfma_kernel reads these (and writes o) element by element, so they may start anywhere; here they move in pieces of
   // up to 16 bytes
   uintptr_t at = reinterpret_cast<uintptr_t>(a->o);
   for (const void* x : {a->q, a->k_pop, a->v_pop, a->g_pop, a->s_pop}) at |= reinterpret_cast<uintptr_t>(x);
-  if (at & 15) return false;
-  const int P = split_of(a);
+  return (at & 15) ? 0 : split_of(a);
+}
+
+bool decode_split_uses_scratch(const NhaDecodeArgs* a) { return split_at(a) > 1; }
+
+bool decode_split_wanted(const NhaDecodeArgs* a) {
+  const int P = split_at(a);
   return P == 1 || (P > 1 && a->scratch && a->scratch_bytes >= decode_scratch_bytes());
 }
 

@@ -33,9 +33,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import _lib
 from .cache import NHARingCache
-from .ops import (chunk_nha, fused_chunk_nha_prefill, hybrid_prologue_supported, nha_hybrid_prologue,
+from .ops import (chunk_nha, fused_chunk_nha_prefill, hybrid_prologue_supported, new_decode_scratch, nha_hybrid_prologue,
                   nha_zero_sink_rescale_, zero_sink_attention, zero_sink_attention_supported)
 
 GATE_LOGIT_NORMALIZER = 8          # qwennha.py:62, llamanha.py:96
@@ -366,7 +365,7 @@ class RecordedDecodeStep:
         self.pos = torch.zeros(batch, 1, dtype=torch.long, device=p.device)
         st = cache.states[block.layer_idx]
         if st.scratch is None:
-            st.scratch = torch.zeros(_lib.load().nha_decode_scratch_bytes(), dtype=torch.uint8, device=p.device)
+            st.scratch = new_decode_scratch(p.device)
         count0 = st.count.clone()
         snap = [t.clone() for t in (st.hk, st.hv, st.ring_k, st.ring_kg, st.ring_v, st.ring_g)]
         tokens = (cache._layer_tokens.get(block.layer_idx, 0), cache.former_tokens, cache._seen_tokens)

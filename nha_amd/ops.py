@@ -108,17 +108,33 @@ def _workspace(nbytes: int, dev, stream: int) -> torch.Tensor:
 _DECODE_SCRATCH: dict = {}
 
 
-def decode_scratch(dev, stream: int) -> torch.Tensor:
-    if torch.cuda.is_current_stream_capturing():       # a recording keeps its own, zeroed at every replay
-        return torch.zeros(_lib.load().nha_decode_scratch_bytes(), dtype=torch.uint8, device=dev)
+def new_decode_scratch(dev) -> torch.Tensor:
+    return torch.zeros(_lib.load().nha_decode_scratch_bytes(), dtype=torch.uint8, device=dev)
+
+
+def decode_scratch(dev, stream: int) -> Optional[torch.Tensor]:
+    if torch.cuda.is_current_stream_capturing():       # a recording keeps its own (run_decode)
+        return None
     ws = _DECODE_SCRATCH.get((dev, stream))
     if ws is None:
-        ws = torch.zeros(_lib.load().nha_decode_scratch_bytes(), dtype=torch.uint8, device=dev)
+        ws = new_decode_scratch(dev)
         with _POOL_LOCK:                               # threads with new streams of their own
             while len(_DECODE_SCRATCH) >= _WORKSPACE_MAX_STREAMS:
                 _DECODE_SCRATCH.pop(next(iter(_DECODE_SCRATCH)))
             _DECODE_SCRATCH[(dev, stream)] = ws
     return ws
+
+
+def run_decode(args: bytes, dev, scratch: Optional[torch.Tensor]) -> None:
+    """The step of an argument block from pack_decode.  Without scratch (in a recording) one is made, zeroed at every replay,
+    if the call needs it: the fill takes a replay 1.5 to 3 us."""
+    lib = _lib.load()
+    if scratch is None and lib.decode_uses_scratch_packed(args):
+        scratch = new_decode_scratch(dev)
+        args = _lib.with_scratch(args, scratch.data_ptr(), scratch.numel())
+    rc = lib.decode_step_packed(args)
+    if rc:
+        _lib.check(rc)
 
 
 def release_workspaces() -> int:
@@ -1206,10 +1222,8 @@ def fused_recurrent_nha_decode(
     args = _lib.pack_decode(
         _lib.NHA_DECODE_WINDOW, _dtype_code(q_), B, HQ, H, K, V, M, W, float(scale), p(q_), p(sq_), p(k_), p(v_), p(g_), p(s_),
         p(swk_), p(swv_), p(cos), p(sin), c_sb, c_sw, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, p(hk0), p(hv0), p(hkt), p(hvt), p(o),
-        stream, 0, p(scratch), scratch.numel())
-    rc = _lib.load().decode_step_packed(args)
-    if rc:
-        _lib.check(rc)
+        stream, 0, p(scratch), 0 if scratch is None else scratch.numel())
+    run_decode(args, dev, scratch)
     return o, (hkt, hvt)
 
 

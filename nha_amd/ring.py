@@ -13,7 +13,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .ops import _dtype_code, _need_cuda, _ptr, _stream, decode_scratch
+from .ops import _dtype_code, _need_cuda, _ptr, _stream, decode_scratch, run_decode
 
 
 @dataclass
@@ -158,10 +158,8 @@ def ring_decode_step(state: NHARingState, q: torch.Tensor, sq: torch.Tensor, k_n
         0, 0, 0, 0, 0, 0, state.ring_k.data_ptr(), state.ring_kg.data_ptr(), state.ring_v.data_ptr(), state.ring_g.data_ptr(),
         k_new.data_ptr(), kg_new.data_ptr(), v_new.data_ptr(), g_new.data_ptr(), state.count.data_ptr(), hk, hv, hk, hv,
         o.data_ptr(), stream, state.count_alt.data_ptr() if advance else 0,      # the kernel writes count + 1 there
-        scratch.data_ptr(), scratch.numel())
-    rc = _lib.load().decode_step_packed(args)
-    if rc:
-        _lib.check(rc)
+        *((0, 0) if scratch is None else (scratch.data_ptr(), scratch.numel())))
+    run_decode(args, dev, scratch)
     if advance:      # the two counter arrays trade places
         state.count, state.count_alt = state.count_alt, state.count
     return o

@@ -180,3 +180,30 @@ def test_window_step_on_operands_off_a_16_byte_boundary(name):
     assert a[name].is_contiguous() and a[name].data_ptr() % 16
     got, (hk, hv) = fused_recurrent_nha_decode(**a)
     assert torch.equal(got, unsplit) and torch.equal(hk, want[0]) and torch.equal(hv, want[1])
+
+
+@pytest.mark.parametrize("B,W,fills", [(3, 200, 1), (130, 64, 0)])
+def test_recorded_steps_take_scratch_where_they_use_it(B, W, fills, monkeypatch):
+    """A recording makes (and so fills, at every replay) scratch for the steps that use it only; its replays are the eager step."""
+    from nha_amd import NHARingState, ops, ring_decode_step
+    HQ, H, K, M, dt = 8, 2, 128, 64, torch.bfloat16
+    gen = torch.Generator().manual_seed(W)
+    r = lambda *s: randn(gen, *s, dtype=dt).cuda()
+    first = [randn(gen, B, H, *s, dtype=torch.float32, scale=0.3).cuda() for s in ((K, M), (M, K))] + [r(B, W, H, K) for _ in range(3)] + \
+        [-r(B, W, H, M).abs(), torch.full((B,), 2 * W + 1, dtype=torch.int32, device="cuda")]
+    new = [r(B, HQ, K), r(B, HQ, K), r(B, H, K), r(B, H, K), r(B, H, K), -r(B, H, M).abs()]
+    eager = NHARingState(*[x.clone() for x in first])
+    want = ring_decode_step(eager, *new, advance=False)
+    st, made, make = NHARingState(*[x.clone() for x in first]), [], ops.new_decode_scratch
+    monkeypatch.setattr(ops, "new_decode_scratch", lambda dev: made.append(1) or make(dev))
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        o = ring_decode_step(st, *new, advance=False)
+    assert len(made) == fills
+    for _ in range(3):
+        for x, y in zip((st.hk, st.hv, st.ring_k, st.ring_kg, st.ring_v, st.ring_g), first):
+            x.copy_(y)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, want) and torch.equal(st.hk, eager.hk) and torch.equal(st.ring_v, eager.ring_v)
