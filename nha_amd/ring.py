@@ -13,7 +13,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .ops import _dtype_code, _need_cuda, _ptr, _stream, decode_scratch, run_decode
+from .ops import _dtype_code, _need_cuda, _plain_autograd, _ptr, _stream, decode_scratch, run_decode
 
 
 @dataclass
@@ -86,10 +86,11 @@ class NHARingState:
     @classmethod
     def _fill(cls, rows, hk, hv, W: int, cu_seqlens, N: int, T: int) -> Optional["NHARingState"]:
         """The hand-over in one launch, or None for what the kernel does not move: rows, states or addresses that are
-        not whole 16-byte pieces, states that are not fp32, tensors with a gradient to carry or on several devices."""
+        not whole 16-byte pieces, states that are not fp32, tensors with a gradient to carry or on several devices, calls that
+        something besides autograd looks at (fake tensors, modes, forward-mode levels)."""
         dev = rows[0].device
         ts = (*rows, hk, hv)
-        if (torch.compiler.is_compiling() or N < 1 or N > 65535 or W < 1
+        if (torch.compiler.is_compiling() or not _plain_autograd((*ts, cu_seqlens)) or N < 1 or N > 65535 or W < 1
                 or any(x.dim() != 4 or x.shape[:2] != rows[0].shape[:2] or x.numel() == 0 for x in rows)
                 or any(x.device != dev for x in ts) or dev.index != torch.cuda.current_device() or (torch.is_grad_enabled() and any(x.requires_grad for x in ts))
                 or hk.dtype != torch.float32 or hv.dtype != torch.float32):
