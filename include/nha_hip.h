@@ -87,8 +87,9 @@ typedef struct NhaPrefillArgs {
   void* stream;
 } NhaPrefillArgs;
 
-/* Bytes of device scratch nha_prefill_fwd needs for these dims (chunk-start slot states, gate
- * cumsums, staging).  Only the integer/dtype/impl fields of `a` are read. */
+/* Bytes of device scratch nha_prefill_fwd runs fastest with at these dims (chunk-start slot states, gate
+ * cumsums, staging).  Only the integer/dtype/impl fields of `a` are read.  A workspace of this many bytes for a
+ * call serves every call of fewer tokens with the same heads, head sizes and number of sequences. */
 size_t nha_prefill_scratch_bytes(const NhaPrefillArgs* a);
 int nha_prefill_fwd(const NhaPrefillArgs* a);
 

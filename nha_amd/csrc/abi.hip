@@ -139,7 +139,7 @@ static int prefill_fwd_phase(const NhaPrefillArgs* a, int phase) {
               a->V, a->M, a->HQ / a->H);
     return NHA_ERR_UNSUPPORTED;
   }
-  const size_t need = mfma ? prefill_mfma_scratch_bytes(a) : prefill_simple_scratch_bytes(a);
+  const size_t need = mfma ? prefill_mfma_least_scratch_bytes(a) : prefill_simple_scratch_bytes(a);
   if (a->scratch_bytes < need) {
     set_error("nha_prefill_fwd: scratch has %zu bytes, %zu needed", a->scratch_bytes, need);
     return NHA_ERR_SCRATCH;
@@ -156,7 +156,7 @@ int nha_prefill_fwd_noalloc(const NhaPrefillArgs* a) {
               a->V, a->M, a->HQ / a->H);
     return NHA_ERR_UNSUPPORTED;
   }
-  const size_t need = mfma ? prefill_mfma_scratch_bytes(a) : prefill_simple_scratch_bytes(a);
+  const size_t need = mfma ? prefill_mfma_least_scratch_bytes(a) : prefill_simple_scratch_bytes(a);
   if (need > (size_t)NHA_NOALLOC_SCRATCH_BYTES) {
     set_error("nha_prefill_fwd_noalloc: this call needs %zu bytes of scratch, the library's array holds %zu "
               "(use nha_prefill_fwd with a workspace of nha_prefill_scratch_bytes() bytes)", need, (size_t)NHA_NOALLOC_SCRATCH_BYTES);
@@ -185,7 +185,7 @@ int nha_prefill_bwd(const NhaPrefillBwdArgs* a) {
     set_error("nha_prefill_bwd: built for K, V <= 256 (multiples of 8) and M <= 64, got K=%d V=%d M=%d", a->K, a->V, a->M);
     return NHA_ERR_UNSUPPORTED;
   }
-  const size_t need = prefill_bwd_scratch_bytes(a);
+  const size_t need = prefill_bwd_least_scratch_bytes(a);
   if (a->scratch_bytes < need) {
     set_error("nha_prefill_bwd: scratch has %zu bytes, %zu needed", a->scratch_bytes, need);
     return NHA_ERR_SCRATCH;

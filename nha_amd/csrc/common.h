@@ -159,12 +159,15 @@ int prefill_simple_impl(const NhaPrefillArgs* a, int phase);
 bool prefill_f32_supported(const NhaPrefillArgs* a);
 int prefill_f32_impl(const NhaPrefillArgs* a, int phase);
 bool prefill_mfma_supported(const NhaPrefillArgs* a);
+// what a call runs fastest with, and what it runs with at all (prefill_mfma.hip: plan_call)
 size_t prefill_mfma_scratch_bytes(const NhaPrefillArgs* a);
+size_t prefill_mfma_least_scratch_bytes(const NhaPrefillArgs* a);
 int prefill_mfma_impl(const NhaPrefillArgs* a, int phase);
 int bwd_slot_inter_slabs(const NhaPrefillBwdArgs* a);
 int bwd_slot_inter(const NhaPrefillBwdArgs* a, const float* gc, const float* ek, const float* ev, const float* dks, float* dvs, float* dsp);
 bool prefill_bwd_supported(const NhaPrefillBwdArgs* a);
 size_t prefill_bwd_scratch_bytes(const NhaPrefillBwdArgs* a);
+size_t prefill_bwd_least_scratch_bytes(const NhaPrefillBwdArgs* a);
 int prefill_bwd_impl(const NhaPrefillBwdArgs* a);
 bool bwd_window_mfma_supported(const NhaPrefillBwdArgs* a);
 int bwd_window_mfma_dq(const NhaPrefillBwdArgs* a, const float* delta, void* ld);

@@ -961,7 +961,8 @@ struct BwdPlan {
   bool use_mfma;   // the slot branch runs on the matrix cores
   int nbk, nbv;
 };
-BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f) {
+// fwd_bytes: the room of the forward's state pass
+BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f, size_t fwd_bytes) {
   BwdPlan s = {};
   // bf16 shapes the matrix-core state pass covers
   s.use_mfma = prefill_mfma_supported(&f);
@@ -975,7 +976,7 @@ BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f) {
   };
   const size_t states_k = (size_t)a->NT * a->H * a->K * a->M * 4, states_v = (size_t)a->NT * a->H * a->V * a->M * 4;
   const size_t tqm = (size_t)a->T_tot * a->HQ * a->M * 4, thm = (size_t)a->T_tot * a->H * a->M * 4;
-  s.fwd = take(s.use_mfma ? prefill_mfma_scratch_bytes(&f) : prefill_simple_scratch_bytes(&f));
+  s.fwd = take(fwd_bytes);
   s.hkT = take((size_t)a->N * a->H * a->K * a->M * 4);
   s.hvT = take((size_t)a->N * a->H * a->M * a->V * 4);
   if (!s.use_mfma) {
@@ -1013,10 +1014,17 @@ NhaPrefillArgs forward_args(const NhaPrefillBwdArgs* a) {
   return f;
 }
 
+BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, bool least, NhaPrefillArgs* f) {
+  *f = forward_args(a);
+  f->scratch_bytes = !prefill_mfma_supported(f) ? prefill_simple_scratch_bytes(f) : least ? prefill_mfma_least_scratch_bytes(f) : prefill_mfma_scratch_bytes(f);
+  return plan_bwd(a, *f, f->scratch_bytes);
+}
+
 template <typename T>
 int run_bwd(const NhaPrefillBwdArgs* a) {
-  NhaPrefillArgs f = forward_args(a);
-  const BwdPlan sp = plan_bwd(a, f);
+  NhaPrefillArgs f;
+  BwdPlan sp = plan_bwd(a, false, &f);
+  if (sp.total > a->scratch_bytes) sp = plan_bwd(a, true, &f);   // a workspace sized for another call: long segments
   char* sc = (char*)a->scratch;
   f.hkt = (float*)(sc + sp.hkT);
   f.hvt = (float*)(sc + sp.hvT);
@@ -1032,13 +1040,11 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
   f.scratch = sc + sp.fwd;
   if (sp.use_mfma) {
     f.impl = NHA_IMPL_MFMA;
-    f.scratch_bytes = prefill_mfma_scratch_bytes(&f);
     rc = prefill_mfma_segment_states(&f, &states);
     if (rc == NHA_OK)
       rc = bwd_slot_branch(a, states, (float*)(sc + sp.delta), (float*)(sc + sp.xg), (float*)(sc + sp.dsi), (float*)(sc + sp.ek),
                            (float*)(sc + sp.ev), (float*)(sc + sp.dks), (float*)(sc + sp.dvs));
   } else {
-    f.scratch_bytes = prefill_simple_scratch_bytes(&f);
     rc = prefill_simple_impl(&f, 1);   // the state pass only
   }
   if (rc != NHA_OK) return rc;
@@ -1125,8 +1131,12 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
 }  // namespace
 
 size_t prefill_bwd_scratch_bytes(const NhaPrefillBwdArgs* a) {
-  NhaPrefillArgs f = forward_args(a);
-  return plan_bwd(a, f).total;
+  NhaPrefillArgs f;
+  return plan_bwd(a, false, &f).total;
+}
+size_t prefill_bwd_least_scratch_bytes(const NhaPrefillBwdArgs* a) {
+  NhaPrefillArgs f;
+  return plan_bwd(a, true, &f).total;
 }
 
 bool prefill_bwd_supported(const NhaPrefillBwdArgs* a) { return a->K <= 256 && a->V <= 256 && a->M <= 64 && a->K % 8 == 0 && a->V % 8 == 0; }

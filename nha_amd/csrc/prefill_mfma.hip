@@ -1423,9 +1423,18 @@ ScratchPlan plan_scratch(const NhaPrefillArgs* a) {
   }
   return best == 3 ? full : plan_scratch(a, best);
 }
+
+// The plan of a call: the best one that a->scratch_bytes holds.  Short segments take up to three times the room, so a workspace
+// that was sized for a longer call may be too small for a shorter one's best plan; eight chunks fit it always.
+ScratchPlan plan_call(const NhaPrefillArgs* a) {
+  ScratchPlan s = plan_scratch(a);
+  while (s.seg_sh < 3 && s.total > a->scratch_bytes) s = plan_scratch(a, s.seg_sh + 1);
+  return s;
+}
 }  // namespace
 
 size_t prefill_mfma_scratch_bytes(const NhaPrefillArgs* a) { return plan_scratch(a).total; }
+size_t prefill_mfma_least_scratch_bytes(const NhaPrefillArgs* a) { return plan_scratch(a, 3).total; }
 
 namespace {
 MP make_mp(const NhaPrefillArgs* a) {
@@ -1437,7 +1446,7 @@ MP make_mp(const NhaPrefillArgs* a) {
   p.lse_swa = a->lse_swa; p.lse_gsa = a->lse_gsa;
   p.h0k = a->h0k; p.h0v = a->h0v; p.hkt = a->hkt; p.hvt = a->hvt;
   p.cu = a->cu_seqlens; p.cidx = a->chunk_indices; p.coff = a->chunk_offsets;
-  const ScratchPlan sp = plan_scratch(a);
+  const ScratchPlan sp = plan_call(a);
   char* sc = (char*)a->scratch;
   p.hkT = (bf16_t*)(sc + sp.hkT);
   p.hvc = (bf16_t*)(sc + sp.hvc);
