@@ -1017,7 +1017,7 @@ def chunk_nha(
     assert q_swa.dim() == 4, "Expected [B, T, H, D] for input"
     _need_cuda(q_swa, k_swa, q_gsa, k_gsa, v, s, g)
     if q_swa.dtype == torch.float16:
-        # float16 tensors: computed in float32 (every float16 value is one) by the generic kernels, o returned in float16
+        # float16 tensors: computed in float32 (every float16 value is one) by the kernels of that type, o returned in float16
         out = chunk_nha(*(x.float() for x in (q_swa, k_swa, q_gsa, k_gsa, v, s, g)), cu_seqlens=cu_seqlens, max_seqlen=max_seqlen,
                         scale=scale, window_size_left=window_size_left, window_size_right=window_size_right, head_first=head_first,
                         gsa_kv_shift=gsa_kv_shift, initial_state=initial_state, output_final_state=output_final_state, impl=impl)
