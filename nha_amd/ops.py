@@ -266,6 +266,16 @@ class _Refusal(torch.autograd.Function):
         raise RuntimeError("the NHA kernels have first derivatives only: this gradient cannot be differentiated twice")
 
 
+class _SavedOnce:
+    """A node's context whose saved tensors are unpacked once (torch.utils.checkpoint gives them out once)."""
+
+    def __init__(self, ctx):
+        self._ctx, self.saved_tensors = ctx, ctx.saved_tensors
+
+    def __getattr__(self, name):
+        return getattr(self._ctx, name)
+
+
 def _first_derivatives_only(backward):
     """For an autograd node whose backward is a kernel.  Under create_graph its gradients hang on everything that they were
     formed from, through a node that raises: a second derivative that passes through here is refused, also one that reaches
@@ -273,14 +283,16 @@ def _first_derivatives_only(backward):
     passed by and the sum comes out without the terms of this node."""
     @functools.wraps(backward)
     def wrapped(ctx, *grads):
+        if not torch.is_grad_enabled():
+            return backward(ctx, *grads)
+        ctx = _SavedOnce(ctx)
         with torch.no_grad():
             outs = backward(ctx, *grads)
-        if torch.is_grad_enabled():
-            roots = [t for t in (*grads, *ctx.saved_tensors) if t is not None and t.requires_grad]
-            formed = [t for t in outs if t is not None]
-            if roots and formed:
-                new = iter(_Refusal.apply(len(formed), *formed, *roots))
-                outs = tuple(None if t is None else next(new) for t in outs)
+        roots = [t for t in (*grads, *ctx.saved_tensors) if t is not None and t.requires_grad]
+        formed = [t for t in outs if t is not None]
+        if roots and formed:
+            new = iter(_Refusal.apply(len(formed), *formed, *roots))
+            outs = tuple(None if t is None else next(new) for t in outs)
         return outs
     return wrapped
 

@@ -78,39 +78,63 @@ def test_hooks_edits_and_second_derivatives():
 NODES = ["operator", "prologue", "projections and prologue", "epilogue", "short convolution", "layer", "layer, short convolution"]
 
 
-@pytest.mark.parametrize("residual", [False, True])
-@pytest.mark.parametrize("node", NODES)
-def test_second_derivatives_through_the_kernels_are_refused(node, residual):
-    """The kernels have first derivatives only: a gradient taken with create_graph leads to an error, never to a second
-    derivative without the terms that pass through them, whether the input is reached through them alone or past them too."""
+def _node(node):
+    """A function of one tensor [1, 90, 128] to the scalar of one node's outputs."""
     from nha_amd import chunk_nha, ops
     from nha_amd.layer import NativeHybridAttention
     torch.manual_seed(2)
     r = lambda *s: torch.randn(*s, device="cuda").bfloat16()
     inv = 10000.0 ** (-torch.arange(0, 64, 2, device="cuda").float() / 64)
-    x, w = r(1, 90, 128).requires_grad_(), r(128).requires_grad_()
     total = lambda ts: sum(t.float().pow(2).sum() for t in ts)
+    kw = dict(feature_map="swish", gate_logit_normalizer=8)
+    heads = lambda x: [y.view(1, 90, 2, 64) for y in (x, x * 2, x * 3, x * 4)]
     if node.startswith("layer"):
         m = NativeHybridAttention(hidden_size=128, num_heads=2, num_slots=64, layer_idx=0, window_size=40, use_short_conv="short" in node)
-        out = total(m.cuda().bfloat16()(x)[:1])
-    elif node in ("prologue", "operator"):
-        q, k, v, f = (y.view(1, 90, 2, 64) for y in (x, x * 2, x * 3, x * 4))
-        out = total(ops.nha_layer_prologue(q, k, v, f, inv, feature_map="swish", gate_logit_normalizer=8)) if node == "prologue" \
-            else total(chunk_nha(q, k, q, k, v, r(1, 90, 2, 64).sigmoid(), -r(1, 90, 2, 64).abs(), window_size_left=40)[:1])
-    elif node == "projections and prologue":
+        m = m.cuda().bfloat16()
+        return lambda x: total(m(x)[:1])
+    if node == "operator":
+        s, g = r(1, 90, 2, 64).sigmoid(), -r(1, 90, 2, 64).abs()
+        return lambda x: total((lambda q, k, v, f: chunk_nha(q, k, q, k, v, s, g, window_size_left=40)[:1])(*heads(x)))
+    if node == "prologue":
+        return lambda x: total(ops.nha_layer_prologue(*heads(x), inv, **kw))
+    if node == "projections and prologue":
         mods = [torch.nn.Linear(128, 128, bias=False).cuda().bfloat16() for _ in range(4)]
-        out = total(ops.nha_layer_prologue(None, None, None, None, inv, feature_map="swish", gate_logit_normalizer=8,
-                                           projections=(x, mods, (2, 2, 64, 64, 64))))
-    elif node == "epilogue":
-        out = total([ops.nha_layer_epilogue(x, w, None, 1e-5)])
-    else:
-        out = total([ops.nha_short_conv(x, r(128, 4).requires_grad_(), None, activation="silu")])
+        return lambda x: total(ops.nha_layer_prologue(None, None, None, None, inv, projections=(x, mods, (2, 2, 64, 64, 64)), **kw))
+    w, taps = r(128).requires_grad_(), r(128, 4).requires_grad_()
+    if node == "epilogue":
+        return lambda x: total([ops.nha_layer_epilogue(x, w, None, 1e-5)])
+    return lambda x: total([ops.nha_short_conv(x, taps, None, activation="silu")])
+
+
+def _same(node, a, b):
+    # the layer's projections add four products in another order where a graph is wanted: a rounding of 2^-8 each
+    return torch.equal(a, b) if node != "layer, short convolution" else (a - b).float().norm() <= 1e-2 * b.float().norm()
+
+
+@pytest.mark.parametrize("residual", [False, True])
+@pytest.mark.parametrize("node", NODES)
+def test_second_derivatives_through_the_kernels_are_refused(node, residual):
+    """The kernels have first derivatives only: a gradient taken with create_graph leads to an error, never to a second
+    derivative without the terms that pass through them, whether the input is reached through them alone or past them too."""
+    f = _node(node)
+    x = torch.randn(1, 90, 128, device="cuda").bfloat16().requires_grad_()
+    out = f(x)
     if residual:
         out = out + x.float().pow(3).sum()
     plain = torch.autograd.grad(out, x, retain_graph=True)[0]
     dx = torch.autograd.grad(out, x, create_graph=True)[0]
-    assert dx.requires_grad
-    # the layer's projections add four products in another order where a graph is wanted: a rounding of 2^-8 each
-    assert torch.equal(dx, plain) if node != "layer, short convolution" else (dx - plain).float().norm() <= 1e-2 * plain.float().norm()
+    assert dx.requires_grad and _same(node, dx, plain)
     with pytest.raises(RuntimeError, match="differentiated twice"):
         torch.autograd.grad(dx.float().pow(2).sum(), x)
+
+
+@pytest.mark.parametrize("create_graph", [False, True])
+@pytest.mark.parametrize("node", NODES)
+def test_first_derivatives_under_checkpointing(node, create_graph):
+    """Saved tensors that are formed anew in the backward are unpacked once, with and without a graph of the gradients."""
+    from torch.utils.checkpoint import checkpoint
+    f = _node(node)
+    x = torch.randn(1, 90, 128, device="cuda").bfloat16().requires_grad_()
+    plain = torch.autograd.grad(f(x), x)[0]
+    dx = torch.autograd.grad(checkpoint(f, x, use_reentrant=False), x, create_graph=create_graph)[0]
+    assert _same(node, dx, plain)
