@@ -15,12 +15,18 @@
 //   dP^T = V dO^T) and K once more for the transposing read (A operand of dQ^T += K^T dS^T).  It also
 //   leaves (-lse / scale, -delta) per (token, q-head) as pairs for the kernel below, whose score and
 //   dP accumulators start from them.
-// ring_dkv_kernel: one workgroup of 8 waves = 256 keys of one kv-head (a key per lane and 16-key block, 32 keys per wave,
-//   K and V rows in registers); the q / do rows of every query head of the group stream through the ring
-//   in items of 32 queries: four tiles (q and do as row fragments for S = Q K^T and dP = dO V^T, and once
-//   more for the transposing read: dV^T += dO^T P, dK^T += Q^T dS) plus the 32 (lse, delta) pairs.
+// ring_dkv_kernel: one workgroup of 8 waves = 256 keys of one kv-head (a key per lane and 16-key block, 32 keys per wave, K
+//   rows in registers, V rows in LDS); the q / do rows of every query head of the group stream through the ring in items of
+//   32 queries: a tile of each plus the 32 (lse, delta) pairs.  One layout of a tile serves both reads, the row fragments of
+//   S = Q K^T and dP = dO V^T and the transposing read of dV^T += dO^T P and dK^T += Q^T dS: the planes of 32-byte rows
+//   give a wave's 16-byte reads of 16 rows the LDS's full rate too.
 //   The first and the last units of a head are triangles over the waves (causal edge, window edge) that
 //   complement each other: such units are held in LDS two at a time and every wave works on its own.
+//   Bound: the products and, beside them, LDS reads and exponentials of two waves per SIMD (48 % of the matrix rate over the
+//   launch).  B=2, T=8192, 32/8 heads, W=2048: 1149 us with K and V in registers (no room to read ahead; the row
+//   fragments read once per 16-key block), each tile in LDS twice and the exponentials between the products; 950 with
+//   V in LDS, one tile and one stream of products; 934 with two items per barrier.  Transposed fragments one, three or four
+//   products ahead instead of two: the same.
 #include "common.h"
 #include "mfma_common.h"
 
@@ -258,9 +264,10 @@ struct DkvP {
   float scale;
 };
 
-constexpr int KV_ITEM = 4 * UB + 1024;   // q rows | do rows | q transposing | do transposing | 32 (lse, delta) pairs
-constexpr int KV_QR = 0, KV_OR = UB, KV_QT = 2 * UB, KV_OT = 3 * UB, KV_LD = 4 * UB;
-constexpr int KV_BYTES = NR * KV_ITEM;
+// an item: q tile | do tile | 32 (lse, delta) pairs; a tile in 1 KB blocks of 16 rows x 32 columns, two planes of 32-byte rows
+// each, which both the row fragments and the transposing reads take without bank conflicts
+constexpr int KV_Q = 0, KV_O = UB, KV_LD = 2 * UB, KV_ITEM = 2 * UB + 256;
+template <int KEYS> constexpr int KV_BYTES = NR * KV_ITEM + KEYS * D * 2;   // ring, then the V rows of the workgroup's keys
 
 __device__ __forceinline__ void g2l4(const void* gbase, uint32_t voff_bytes, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff_bytes), "s"(gbase), "s"(lds_base) : "memory");
@@ -275,7 +282,7 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
   constexpr int NKB = KEYS / 16 / 8;       // 16-key blocks per wave
   constexpr int CPG = KEYS / 64;           // chunks per key group
   constexpr int UPG = KEYS / 32;           // 32-query units that a key group spans
-  constexpr int KV_LPW = 4;   // tile loads per wave and item (32 blocks of 1 KB, 8 waves)
+  constexpr int KV_LPW = 2;                // tile loads per wave and item (16 blocks of 1 KB, 8 waves)
   extern __shared__ __align__(1024) unsigned char smem_[];
   lbyte* const lds = (lbyte*)smem_;
   const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
@@ -304,7 +311,7 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
   const int nun = (qend - c0 + 31) / 32;   // >= 1
   const int total = NG * nun;
 
-  // block (16-row half wave / 4, 32-column block wave % 4) of each of the four tiles of an item
+  // block (16-row half wave / 4, 32-column block wave % 4) of both tiles of an item
   const int rh = wave >> 2, cq = wave & 3;
   // item (g, u): rows [c0 + 32 u, c0 + 32 u + 32) of query head h NG + g; rows past eos are read from row
   // eos - 1 (always masked, always finite)
@@ -313,23 +320,16 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
     // cost registers the accumulators need
     int ln = threadIdx.x & 63;
     asm volatile("" : "+v"(ln));
-    const int lrow16 = ln & 15, lpk = ln >> 4;
-    const int lrowv = (ln & 31) >> 1, lpv = 2 * (ln >> 5) + (ln & 1);
     const int hq = h * NG + g;
     const int q0 = c0 + 32 * u;
     const bf16_t* const qbase = p.q + ((int64_t)bos * HQ + hq) * D;
     const bf16_t* const obase = p.dout + ((int64_t)bos * HQ + hq) * D;
-    int rr = q0 + 16 * rh + lrow16;
-    rr = rr < eos ? rr : eos - 1;
-    int rt = q0 + 16 * rh + lrowv;
+    int rt = q0 + 16 * rh + ((ln & 31) >> 1);
     rt = rt < eos ? rt : eos - 1;
-    const uint32_t offr = ((uint32_t)(rr - bos) * (uint32_t)(HQ * D) + (uint32_t)(4 * cq + lpk) * 8) * 2;
-    const uint32_t offt = ((uint32_t)(rt - bos) * (uint32_t)(HQ * D) + (uint32_t)(4 * cq + lpv) * 8) * 2;
+    const uint32_t off = ((uint32_t)(rt - bos) * (uint32_t)(HQ * D) + (uint32_t)(4 * cq + 2 * (ln >> 5) + (ln & 1)) * 8) * 2;
     const uint32_t dst = lds0 + slot * KV_ITEM + rh * HB + cq * 1024;
-    g2l16(qbase, offr, dst + KV_QR);
-    g2l16(obase, offr, dst + KV_OR);
-    g2l16(qbase, offt, dst + KV_QT);
-    g2l16(obase, offt, dst + KV_OT);
+    g2l16(qbase, off, dst + KV_Q);
+    g2l16(obase, off, dst + KV_O);
     if (wave == 0) {
       int r = q0 + (ln >> 1);
       r = r < eos ? r : eos - 1;
@@ -385,31 +385,35 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
     }
     advance(pw);
   };
+  // This lane's keys (one per 16-key block of the wave) and their K / V rows (B operands: K[key][32 ks + 8 kb ..]).  The V rows
+  // lie in LDS, in the order in which their wave reads them; K and V both in registers would leave none to read ahead with.
+  const int kbase = 16 * NKB * wave;               // first key of the wave, relative to c0
+  const uint32_t vrows = (uint32_t)(NR * KV_ITEM + wave * (NKB * KS * 1024));
+#pragma unroll
+  for (int kk = 0; kk < NKB; ++kk) {
+    const int tk = c0 + kbase + 16 * kk + l16;
+    const uint32_t row = (uint32_t)((tk < eos ? tk : eos - 1) - bos) * (uint32_t)(H * D);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      g2l16(p.v + ((int64_t)bos * H + h) * D, (row + 32 * ks + 8 * kb) * 2, lds0 + vrows + (kk * KS + ks) * 1024);
+  }
   int issued = 0;
   for (; issued < NR - 1 && issued < total; ++issued) issue_next(issued);
 
-  // this lane's keys (one per 16-key block of the wave) and their K / V rows (B operands: K[key][32 ks + 8 kb ..])
-  const int kbase = 16 * NKB * wave;               // first key of the wave, relative to c0
-  bf16x8 kfr[NKB][KS], vfr[NKB][KS];
+  bf16x8 kfr[NKB][KS];
 #pragma unroll
   for (int kk = 0; kk < NKB; ++kk) {
     const int tk = c0 + kbase + 16 * kk + l16;
     const int64_t jk = (int64_t)(tk < eos ? tk : eos - 1) * H + h;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      kfr[kk][ks] = as_bf16x8(*reinterpret_cast<const uint4*>(p.k + jk * D + 32 * ks + 8 * kb));
-      vfr[kk][ks] = as_bf16x8(*reinterpret_cast<const uint4*>(p.v + jk * D + 32 * ks + 8 * kb));
-    }
+    for (int ks = 0; ks < KS; ++ks) kfr[kk][ks] = as_bf16x8(*reinterpret_cast<const uint4*>(p.k + jk * D + 32 * ks + 8 * kb));
   }
-  // the K / V rows are in their registers before the loop starts: left to the compiler, the wait for them sits
+  // the K rows are in their registers before the loop starts: left to the compiler, the wait for them sits
   // at their first use inside the loop, as a wait for every load in flight, the LDS-direct ones included
 #pragma unroll
   for (int kk = 0; kk < NKB; ++kk)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      asm volatile("" : "+v"(kfr[kk][ks]));
-      asm volatile("" : "+v"(vfr[kk][ks]));
-    }
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(kfr[kk][ks]));
   f32x4 dK[DB][NKB], dV[DB][NKB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -418,9 +422,13 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
       dK[db][kk] = (f32x4){0.f, 0.f, 0.f, 0.f};
       dV[db][kk] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
-  uint32_t kaddr, vaddr;   // set per item (see issue_item)
-  auto rfrag = [&](uint32_t a, int kk, int ks) -> bf16x8 {
-    return *reinterpret_cast<const NHA_LDS bf16x8*>(lds + (a + kaddr) + kk * HB + ks * 1024);
+  uint32_t kaddr, vaddr, faddr;   // set per item (see issue_item)
+  // row fragment of a tile at byte address a: rows 16 qb + l16, columns 32 ks + 8 kb ..
+  auto rfrag = [&](uint32_t a, int qb, int ks) -> bf16x8 {
+    return *reinterpret_cast<const NHA_LDS bf16x8*>(lds + (a + kaddr) + qb * HB + ks * 1024);
+  };
+  auto vfrag = [&](int kk, int ks) -> bf16x8 {
+    return *reinterpret_cast<const NHA_LDS bf16x8*>(lds + faddr + (kk * KS + ks) * 1024);
   };
   auto tfrag = [&](uint32_t a, int db) -> bf16x8 {
     const lbyte* pa = lds + (a + vaddr) + (db >> 1) * 1024 + (db & 1) * 512;
@@ -435,9 +443,16 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
   auto no_work = [&](int u) { return (32 * u + 31 < kbase) || (p.wl >= 0 && 32 * u > kbase + 16 * NKB - 1 + p.wl); };
   Walk cw = {0, rot0, 0};
   for (int k = 0; k < total;) {
+    // a step is a unit and its complement, of which a wave takes the one it has work in, or up to two units in a row
     const int prim = cw.u;
-    const int need = prim < npair ? 2 : 1;   // items of this step: k .. k + need - 1
+    const bool pair = prim < npair;
     advance(cw);
+    int need = pair ? 2 : 1, next = -1;   // items of this step: k .. k + need - 1
+    if (!pair && k + 1 < total && cw.u >= npair) {
+      next = cw.u;
+      need = 2;
+      advance(cw);
+    }
     // they have landed (this wave's part; wave 0 carries one more load per item), then everybody's; the
     // requests after them stay in flight
     const int younger = issued - (k + need);
@@ -453,116 +468,115 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
     lds_barrier();
     // every wave is past the items before k: their slots take the next requests
     for (; issued < total && issued < k + NR; ++issued) issue_next(issued & (NR - 1));
-    int u = prim;
-    uint32_t base = (uint32_t)((k & (NR - 1)) * KV_ITEM);
-    if (need == 2 && no_work(prim)) {
+    int u = prim, slot = k;
+    if (pair && no_work(prim)) {
       u = prim + K0;
-      base = (uint32_t)(((k + 1) & (NR - 1)) * KV_ITEM);
+      slot = k + 1;
     }
     k += need;
-    int lc = threadIdx.x & 63;
-    asm volatile("" : "+v"(lc));
-    const int l16 = lc & 15, kb = lc >> 4;
-    kaddr = (uint32_t)(lc * 16);
-    vaddr = (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
-    if (!no_work(u)) {
-      const bool edge = (32 * u < kbase + 16 * NKB - 1) || (p.wl >= 0 && 32 * u + 31 > kbase + p.wl) || (c0 + 32 * u + 32 > eos);
-      // ---- phase 1: S = Q K^T and dP = dO V^T, one 16-key block at a time (two blocks of scores beside both
-      //      gradient accumulators do not fit the register file, so the q / do row fragments are read once per
-      //      block); step i = (contraction step i / 2, 16-query block i % 2).  PD1 / PD2: how many steps ahead
-      //      of its product a fragment is requested from LDS; what the register file allows here (as two
-      //      launches, one gradient each, there is room for 2-3 steps and both blocks of scores: 873 + 709 us
-      //      against 1178 us for this kernel) ----
-      constexpr int N1 = 2 * KS;
-      constexpr int GS = 1;
-      constexpr int PD1 = NKB == 2 ? 0 : 1;
-      constexpr int PD2 = 1;
-      bf16x8 Pb[NKB], dSb[NKB];
-      bf16x8 ot[DB], qt[DB];
-#pragma unroll
-      for (int g0 = 0; g0 < NKB; g0 += GS) {
-        f32x4 S[2][GS], dP[2][GS];
-        bf16x8 qa[N1], oa[N1];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < PD1; ++i) {
-          qa[i] = rfrag(base + KV_QR, i & 1, i >> 1);
-          oa[i] = rfrag(base + KV_OR, i & 1, i >> 1);
-        }
-        // rows of the accumulators are the queries 16 qb + 4 kb + r, the column is this lane's key of block
-        // g0 + j; they start from (-lse / scale, -delta) of their rows
+    do {
+      const uint32_t base = (uint32_t)((slot & (NR - 1)) * KV_ITEM);
+      int lc = threadIdx.x & 63;
+      asm volatile("" : "+v"(lc));
+      const int l16 = lc & 15, kb = lc >> 4;
+      kaddr = (uint32_t)((kb >> 1) * 512 + l16 * 32 + (kb & 1) * 16);
+      vaddr = (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
+      faddr = vrows + (uint32_t)(lc * 16);
+      if (!no_work(u)) {
+        const bool edge = (32 * u < kbase + 16 * NKB - 1) || (p.wl >= 0 && 32 * u + 31 > kbase + p.wl) || (c0 + 32 * u + 32 > eos);
+        // One stream of products: S = Q K^T, dP = dO V^T beside the exponentials of S, dV^T[d][key] += dO^T[d][q] P[q][key]
+        // beside dS, dK^T[d][key] += Q^T[d][q] dS[q][key]; what a step multiplies was requested from LDS a step (1 KB row
+        // fragments) or two (transposed ones) before.
+        constexpr int PT = 2;       // transposed fragments are requested this many products ahead
+        constexpr int NQ = 2 * NKB;   // quads of scores: (16-query block q & 1, 16-key block q >> 1)
+        f32x4 S[NQ], dP[NQ];
+        bf16x8 qa[KS][2], oa[KS][2], va[KS][NKB], ot[DB], qt[DB];
+        // rows of the accumulators are the queries 16 qb + 4 kb + r, the column is this lane's key of its block; they start from
+        // (-lse / scale, -delta) of their rows
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
+          qa[0][qb] = rfrag(base + KV_Q, qb, 0);
           const NHA_LDS f32x4* lp = reinterpret_cast<const NHA_LDS f32x4*>(lds + base + KV_LD + (16 * qb + 4 * kb) * 8);
           const f32x4 a0 = lp[0], a1 = lp[1];   // the pairs of rows r = 0, 1 and r = 2, 3
 #pragma unroll
-          for (int j = 0; j < GS; ++j) {
-            S[qb][j] = (f32x4){a0[0], a0[2], a1[0], a1[2]};
-            dP[qb][j] = (f32x4){a0[1], a0[3], a1[1], a1[3]};
+          for (int kk = 0; kk < NKB; ++kk) {
+            S[qb + 2 * kk] = (f32x4){a0[0], a0[2], a1[0], a1[2]};
+            dP[qb + 2 * kk] = (f32x4){a0[1], a0[3], a1[1], a1[3]};
           }
+        }
+        auto read_do = [&](int ks) {
+#pragma unroll
+          for (int qb = 0; qb < 2; ++qb) oa[ks][qb] = rfrag(base + KV_O, qb, ks);
+#pragma unroll
+          for (int kk = 0; kk < NKB; ++kk) va[ks][kk] = vfrag(kk, ks);
+        };
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (ks + 1 < KS) {
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) qa[ks + 1][qb] = rfrag(base + KV_Q, qb, ks + 1);
+          } else {
+            read_do(0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) S[q] = mfma16(qa[ks][q & 1], kfr[q >> 1][ks], S[q]);
         }
         __builtin_amdgcn_sched_barrier(0);
+        if (edge) {
 #pragma unroll
-        for (int i = 0; i < N1; ++i) {
-          const int qb = i & 1, ks = i >> 1;
-          if (i + PD1 < N1) {
-            qa[i + PD1] = rfrag(base + KV_QR, (i + PD1) & 1, (i + PD1) >> 1);
-            oa[i + PD1] = rfrag(base + KV_OR, (i + PD1) & 1, (i + PD1) >> 1);
-          }
-#pragma unroll
-          for (int j = 0; j < GS; ++j) {
-            S[qb][j] = mfma16(qa[i], kfr[g0 + j][ks], S[qb][j]);
-            dP[qb][j] = mfma16(oa[i], vfr[g0 + j][ks], dP[qb][j]);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        // the first transposed fragments of phase 2 are requested before the last exponentials
-        if (g0 + GS == NKB) {
-#pragma unroll
-          for (int i = 0; i < PD2; ++i) {
-            ot[i] = tfrag(base + KV_OT, i);
-            qt[i] = tfrag(base + KV_QT, i);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int j = 0; j < GS; ++j) {
-          const int kk = g0 + j;
-          f32x4 P[2], dS[2];
-#pragma unroll
-          for (int qb = 0; qb < 2; ++qb)
+          for (int q = 0; q < NQ; ++q)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              float x = S[qb][j][r] * cs;
-              if (edge) {
-                const int y = 32 * u + 16 * qb + 4 * kb + r, xk = kbase + 16 * kk + l16;
-                const bool ok = (xk <= y) && (p.wl < 0 || y - xk <= p.wl) && (c0 + y < eos);
-                if (!ok) x = -INFINITY;
-              }
-              const float pr = fexp2(x);
-              P[qb][r] = pr;
-              dS[qb][r] = pr * dP[qb][j][r];
+              const int y = 32 * u + 16 * (q & 1) + 4 * kb + r, xk = kbase + 16 * (q >> 1) + l16;
+              const bool ok = (xk <= y) && (p.wl < 0 || y - xk <= p.wl) && (c0 + y < eos);
+              if (!ok) S[q][r] = -INFINITY;
             }
-          Pb[kk] = pack8(P[0], P[1]);
-          dSb[kk] = pack8(dS[0], dS[1]);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      // ---- phase 2: dV^T[d][key] += dO^T[d][q] P[q][key];  dK^T[d][key] += Q^T[d][q] dS[q][key] ----
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        if (db + PD2 < DB) {
-          ot[db + PD2] = tfrag(base + KV_OT, db + PD2);
-          qt[db + PD2] = tfrag(base + KV_QT, db + PD2);
         }
 #pragma unroll
-        for (int kk = 0; kk < NKB; ++kk) {
-          dV[db][kk] = mfma16(ot[db], Pb[kk], dV[db][kk]);
-          dK[db][kk] = mfma16(qt[db], dSb[kk], dK[db][kk]);
+        for (int ks = 0; ks < KS; ++ks) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (ks + 1 < KS) {
+            read_do(ks + 1);
+          } else {
+#pragma unroll
+            for (int i = 0; i < PT; ++i) ot[i] = tfrag(base + KV_O, i);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) dP[q] = mfma16(oa[ks][q & 1], va[ks][q >> 1], dP[q]);
+          if (ks < NQ)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[ks][r] = fexp2(S[ks][r] * cs);
         }
-        __builtin_amdgcn_sched_barrier(0);
+        bf16x8 Pb[NKB], dSb[NKB];
+#pragma unroll
+        for (int kk = 0; kk < NKB; ++kk) Pb[kk] = pack8(S[2 * kk], S[2 * kk + 1]);
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (db + PT < DB) ot[db + PT] = tfrag(base + KV_O, db + PT);
+          else qt[db + PT - DB] = tfrag(base + KV_Q, db + PT - DB);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int kk = 0; kk < NKB; ++kk) dV[db][kk] = mfma16(ot[db], Pb[kk], dV[db][kk]);
+          if (db >= 1 && db <= NQ) S[db - 1] *= dP[db - 1];
+          if (db >= 1 && db <= NQ && db % 2 == 0) dSb[db / 2 - 1] = pack8(S[db - 2], S[db - 1]);
+        }
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (db + PT < DB) qt[db + PT] = tfrag(base + KV_Q, db + PT);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int kk = 0; kk < NKB; ++kk) dK[db][kk] = mfma16(qt[db], dSb[kk], dK[db][kk]);
+        }
       }
-    }
+      u = next;
+      next = -1;
+      ++slot;
+    } while (u >= 0);
   }
 #pragma unroll
   for (int kk = 0; kk < NKB; ++kk) {
@@ -646,19 +660,19 @@ int bwd_ring_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs)
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(once, [&] {
-    attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<256>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES);
+    attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<256>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES<256>);
     if (attr_err == hipSuccess)
-      attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES);
+      attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES<128>);
   });
   if (attr_err != hipSuccess) {
-    set_error("nha_prefill_bwd: cannot reserve %d bytes of LDS: %s", KV_BYTES, hipGetErrorString(attr_err));
+    set_error("nha_prefill_bwd: cannot reserve %d bytes of LDS: %s", KV_BYTES<256>, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
   // one launch row per chunk, rounded up to whole key groups (4 chunks of 256 keys, 2 of 128)
   if (short_groups(a))
-    hipLaunchKernelGGL(ring_dkv_kernel<128>, dim3(p.H, 2 * ((p.NT + 1) / 2)), dim3(512), KV_BYTES, (hipStream_t)a->stream, p);
+    hipLaunchKernelGGL(ring_dkv_kernel<128>, dim3(p.H, 2 * ((p.NT + 1) / 2)), dim3(512), KV_BYTES<128>, (hipStream_t)a->stream, p);
   else
-    hipLaunchKernelGGL(ring_dkv_kernel<256>, dim3(p.H, 4 * ((p.NT + 3) / 4)), dim3(512), KV_BYTES, (hipStream_t)a->stream, p);
+    hipLaunchKernelGGL(ring_dkv_kernel<256>, dim3(p.H, 4 * ((p.NT + 3) / 4)), dim3(512), KV_BYTES<256>, (hipStream_t)a->stream, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(window dk, dv, ring)");
   return NHA_OK;
 }
