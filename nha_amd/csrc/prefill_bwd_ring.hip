@@ -5,21 +5,24 @@
 // delta = do . o of the whole op per (token, q-head), window logits w = scale q.k:
 //   pi = e^(w - lse),  dw = pi (do.v - delta),
 //   dq_swa_q = scale sum_j dw k_j,   dk_swa_j = scale sum_q dw q_q,   dv_j += sum_q pi do_q.
-// Every streamed operand goes from global memory straight into LDS (global_load_lds_dwordx4) through a
-// ring of four buffers; LDS layouts as in prefill_ring.hip (row-fragment tiles read as consecutive
-// bytes, tiles for the transposing read in two planes of 32-byte rows).
+// Every streamed operand goes from global memory straight into LDS (global_load_lds_dwordx4) through a ring of buffers.  One
+// layout of a tile serves row fragments and transposing reads: 1 KB blocks of 16 rows x 32 columns, each two planes of
+// 32-byte rows, from which a wave's 16-byte reads of 16 rows run at the LDS's full rate too.
 //
 // ring_dq_kernel: one workgroup of 8 waves = one 64-token chunk x 4 query heads of one kv-head (a query
 //   per lane, 32 queries per wave), so the K / V rows of the window are fetched once for the four heads,
-//   in units of 32 keys.  A unit is three tiles: K and V as row fragments (A operands of S^T = K Q^T and
-//   dP^T = V dO^T) and K once more for the transposing read (A operand of dQ^T += K^T dS^T).  It also
+//   in units of 32 keys: a K tile (row fragments for S^T = K Q^T, transposed for dQ^T += K^T dS^T) and a V tile (row
+//   fragments for dP^T = V dO^T).  Two units share a barrier, and the products of the two interleave with what
+//   lies between them: exponentials beside dP, dS of the first unit beside the scores of the second, dS of the second
+//   beside dQ of the first.  It also
 //   leaves (-lse / scale, -delta) per (token, q-head) as pairs for the kernel below, whose score and
 //   dP accumulators start from them.
+//   Bound: as below, 56 % of the matrix rate.  B=2, T=8192, 32/8 heads, W=2048: 625 us unit by unit with K in LDS twice and
+//   the compiler's schedule, 597 like this, 591 with a stretch's first fragments requested during the stretch before.
 // ring_dkv_kernel: one workgroup of 8 waves = 256 keys of one kv-head (a key per lane and 16-key block, 32 keys per wave, K
 //   rows in registers, V rows in LDS); the q / do rows of every query head of the group stream through the ring in items of
 //   32 queries: a tile of each plus the 32 (lse, delta) pairs.  One layout of a tile serves both reads, the row fragments of
-//   S = Q K^T and dP = dO V^T and the transposing read of dV^T += dO^T P and dK^T += Q^T dS: the planes of 32-byte rows
-//   give a wave's 16-byte reads of 16 rows the LDS's full rate too.
+//   S = Q K^T and dP = dO V^T and the transposing read of dV^T += dO^T P and dK^T += Q^T dS.
 //   The first and the last units of a head are triangles over the waves (causal edge, window edge) that
 //   complement each other: such units are held in LDS two at a time and every wave works on its own.
 //   Bound: the products and, beside them, LDS reads and exponentials of two waves per SIMD (48 % of the matrix rate over the
@@ -61,11 +64,11 @@ constexpr int KS = D / 32;            // contraction steps of the score products
 constexpr int DB = D / 16;            // 16-row blocks of dQ^T
 constexpr int UB = 32 * D * 2;        // bytes of a 32-row tile
 constexpr int HB = UB / 2;
-constexpr int NR = 4;                 // ring slots
-constexpr int UNIT = 3 * UB;          // K rows | V rows | K for the transposing read
-constexpr int KR = 0, VR = UB, KT = 2 * UB;
-constexpr int LPW = 3;                // LDS-direct loads per wave and unit (24 blocks of 1 KB, 8 waves)
-constexpr int BYTES = NR * UNIT;
+constexpr int NR = 4;                 // ring slots of ring_dkv_kernel
+constexpr int NRU = 8;                // ring slots of ring_dq_kernel
+constexpr int UNIT = 2 * UB;          // K tile | V tile
+constexpr int LPW = 2;                // LDS-direct loads per wave and unit (16 blocks of 1 KB, 8 waves)
+constexpr int BYTES = NRU * UNIT;
 constexpr int RQB = 2;                // 16-row query blocks per wave
 
 __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
@@ -93,30 +96,26 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
   // before its sequence; units 0 and 1 are the chunk's own rows and may run past eos
   int lowest = bos;
   if (p.wl >= 0 && c0 - p.wl > bos) lowest = c0 - p.wl;
-  const int nunits = (c0 + 64 - lowest + 31) / 32;   // >= 2
+  // an even number: the loop takes them in twos, and (c0 - bos) / 32 is even, so the one added does not start before its
+  // sequence either (the window masks it)
+  const int nunits = ((c0 + 64 - lowest + 31) / 32 + 1) & ~1;
 
-  // block b = wave + 8 i of a unit: tile b / 8, 16-row half (b % 8) / KS, 32-column block b % KS
-  const int lrow16 = lane & 15, lpk = lane >> 4;                             // row fragments: piece lane / 16 of row lane % 16
-  const int lrowv = (lane & 31) >> 1, lpv = 2 * (lane >> 5) + (lane & 1);    // transposing read: two planes of 32-byte rows
+  // a unit's blocks of 16 rows x 32 columns, one of each tile per wave: half wave / KS, columns 32 (wave % KS) ..
+  const int rh = wave / KS, cq = wave % KS;
   const bf16_t* const kbase = p.k + ((int64_t)bos * H + h) * D;
   const bf16_t* const vbase = p.v + ((int64_t)bos * H + h) * D;
+  const uint32_t pcol = (uint32_t)(4 * cq + 2 * (lane >> 5) + (lane & 1)) * 8;
   // rows past eos (units 0 and 1 only) are read from row eos - 1: always masked, always finite
   auto issue_unit = [&](int u) {
-    const int key0 = c0 + 32 - 32 * u;
-    const int slot = u & (NR - 1);
-#pragma unroll
-    for (int i = 0; i < LPW; ++i) {
-      const int b = wave + 8 * i;
-      const int tile = b >> 3, rh = (b & 7) / KS, cq = b % KS;
-      const bool tr = tile == 2;
-      int row = key0 + 16 * rh + (tr ? lrowv : lrow16);
-      row = row < eos ? row : eos - 1;
-      const uint32_t off = ((uint32_t)(row - bos) * (uint32_t)(H * D) + (uint32_t)(4 * cq + (tr ? lpv : lpk)) * 8) * 2;
-      g2l16(tile == 1 ? vbase : kbase, off, lds0 + slot * UNIT + tile * UB + rh * HB + cq * 1024);
-    }
+    int row = c0 + 32 - 32 * u + 16 * rh + ((lane & 31) >> 1);
+    row = row < eos ? row : eos - 1;
+    const uint32_t off = ((uint32_t)(row - bos) * (uint32_t)(H * D) + pcol) * 2;
+    const uint32_t dst = lds0 + (u & (NRU - 1)) * UNIT + rh * HB + cq * 1024;
+    g2l16(kbase, off, dst);
+    g2l16(vbase, off, dst + UB);
   };
 #pragma unroll
-  for (int u = 0; u < NR - 1; ++u)
+  for (int u = 0; u < NRU - 2; ++u)
     if (u < nunits) issue_unit(u);
 
   // query-side fragments: q pre-scaled by scale * log2(e) (the rounding the forward's scores saw), do as it is
@@ -160,13 +159,13 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
 #pragma unroll
     for (int qb = 0; qb < RQB; ++qb) dQ[db][qb] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  const uint32_t kaddr = (uint32_t)(lane * 16);
+  const uint32_t kaddr = (uint32_t)((kb >> 1) * 512 + l16 * 32 + (kb & 1) * 16);
   const uint32_t vaddr = (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
-  // row fragment (rows 16 kk + l16 of a tile, columns 32 ks + 8 kb ..) of a row-fragment tile at byte address a
+  // row fragment of a tile at byte address a: rows 16 kk + l16, columns 32 ks + 8 kb ..
   auto rfrag = [&](uint32_t a, int kk, int ks) -> bf16x8 {
     return *reinterpret_cast<const NHA_LDS bf16x8*>(lds + (a + kaddr) + kk * HB + ks * 1024);
   };
-  // transposed fragment of the third tile: X[4 kb + e][16 db + l16] (e < 4) and X[16 + 4 kb + e - 4][..]
+  // transposed fragment: X[4 kb + e][16 db + l16] (e < 4) and X[16 + 4 kb + e - 4][..]
   auto tfrag = [&](uint32_t a, int db) -> bf16x8 {
     const lbyte* pa = lds + (a + vaddr) + (db >> 1) * 1024 + (db & 1) * 512;
     struct { s16x4 a, b; } t;
@@ -176,67 +175,108 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
   };
   auto is_edge = [&](int u) -> bool { return (63 - 32 * u > 0) || (p.wl >= 0 && 32 - 32 * u < 63 - p.wl); };
 
-  for (int u = 0; u < nunits; ++u) {
-    // unit u has landed (this wave's part), then everybody's; units u+1, u+2 may stay in flight
-    if (u + 2 < nunits) wait_vm<2 * LPW>();
-    else if (u + 1 < nunits) wait_vm<LPW>();
-    else wait_vm<0>();
-    lds_barrier();
-    // every wave is past unit u-1: its slot takes unit u+3
-    if (u + NR - 1 < nunits) issue_unit(u + NR - 1);
-    const uint32_t base = (uint32_t)((u & (NR - 1)) * UNIT);
-    f32x4 S[2][RQB], dP[2][RQB];
+  // The products of a unit as stretches that other work runs beside; scores (16-key block kk, 16-query block qb) at 2 kk + qb.
+  // A stretch is given its first fragments, and its last product is preceded by `tail`, the request for the next stretch's.
+  constexpr int NQ = 2 * RQB;
+  struct Unit {
+    f32x4 S[NQ], dP[NQ];
+    bf16x8 dS[RQB];
+  };
+  struct Frags {
+    bf16x8 x[2];
+  };
+  constexpr int PT = 2;   // transposed fragments are requested this many products ahead
+  auto row_frags = [&](uint32_t a, int ks) { return Frags{{rfrag(a, 0, ks), rfrag(a, 1, ks)}}; };
+  auto columns = [&](uint32_t a) { return Frags{{tfrag(a, 0), tfrag(a, 1)}}; };
+  auto scores = [&](Unit& t, uint32_t base, const Frags& first, auto beside, auto tail) {   // S = K Q^T - lse
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+    for (int q = 0; q < NQ; ++q) t.S[q] = (f32x4){nlse[q & 1], nlse[q & 1], nlse[q & 1], nlse[q & 1]};
+    Frags ka[KS];
+    ka[0] = first;
 #pragma unroll
-      for (int qb = 0; qb < RQB; ++qb) {
-        S[kk][qb] = (f32x4){nlse[qb], nlse[qb], nlse[qb], nlse[qb]};
-        dP[kk][qb] = (f32x4){-dl[qb], -dl[qb], -dl[qb], -dl[qb]};
-      }
+    for (int ks = 0; ks < KS; ++ks) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (ks + 1 < KS) ka[ks + 1] = row_frags(base, ks + 1);
+      else tail();
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        const bf16x8 ka = rfrag(base + KR, kk, ks), va = rfrag(base + VR, kk, ks);
-#pragma unroll
-        for (int qb = 0; qb < RQB; ++qb) {
-          S[kk][qb] = mfma16(ka, qf[qb][ks], S[kk][qb]);
-          dP[kk][qb] = mfma16(va, df[qb][ks], dP[kk][qb]);
-        }
-      }
-    if (is_edge(u)) {
-      const int xbase = 32 - 32 * u;
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-        for (int qb = 0; qb < RQB; ++qb) {
-          const int y = 16 * (qb0 + qb) + l16;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int x = xbase + 16 * kk + 4 * kb + r;
-            const bool ok = (x <= y) && (p.wl < 0 || x >= y - p.wl);
-            if (!ok) S[kk][qb][r] = -INFINITY;
-          }
-        }
+      for (int q = 0; q < NQ; ++q) t.S[q] = mfma16(ka[ks].x[q >> 1], qf[q & 1][ks], t.S[q]);
+      beside(ks);
     }
-    bf16x8 dSb[RQB];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto mask = [&](Unit& t, int u) {
+    if (!is_edge(u)) return;
+    const int xbase = 32 - 32 * u;
 #pragma unroll
-    for (int qb = 0; qb < RQB; ++qb) {
-      f32x4 d0, d1;
+    for (int q = 0; q < NQ; ++q) {
+      const int y = 16 * (qb0 + (q & 1)) + l16;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        d0[r] = fexp2(S[0][qb][r]) * dP[0][qb][r];
-        d1[r] = fexp2(S[1][qb][r]) * dP[1][qb][r];
+        const int x = xbase + 16 * (q >> 1) + 4 * kb + r;
+        const bool ok = (x <= y) && (p.wl < 0 || x >= y - p.wl);
+        if (!ok) t.S[q][r] = -INFINITY;
       }
-      dSb[qb] = pack8(d0, d1);
     }
-    // dQ^T[d][q] += K^T[d][key] dS^T[key][q]
+  };
+  auto dprob = [&](Unit& t, uint32_t base, const Frags& first, auto tail) {   // dP = V dO^T - delta, the exponentials beside it
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) t.dP[q] = (f32x4){-dl[q & 1], -dl[q & 1], -dl[q & 1], -dl[q & 1]};
+    Frags va[KS];
+    va[0] = first;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (ks + 1 < KS) va[ks + 1] = row_frags(base + UB, ks + 1);
+      else tail();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) t.dP[q] = mfma16(va[ks].x[q >> 1], df[q & 1][ks], t.dP[q]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t.S[ks][r] = fexp2(t.S[ks][r]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto form_ds = [&](Unit& t, int qb) {
+    t.dS[qb] = pack8(t.S[qb] * t.dP[qb], t.S[2 + qb] * t.dP[2 + qb]);
+  };
+  auto dquery = [&](Unit& t, uint32_t base, const Frags& first, auto beside, auto tail) {   // dQ^T[d][q] += K^T[d][key] dS^T[key][q]
+    bf16x8 kt[DB] = {first.x[0], first.x[1]};
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
-      const bf16x8 kt = tfrag(base + KT, db);
+      __builtin_amdgcn_sched_barrier(0);
+      if (db + PT < DB) kt[db + PT] = tfrag(base, db + PT);
+      else if (db + 1 == DB) tail();
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int qb = 0; qb < RQB; ++qb) dQ[db][qb] = mfma16(kt, dSb[qb], dQ[db][qb]);
+      for (int qb = 0; qb < RQB; ++qb) dQ[db][qb] = mfma16(kt[db], t.dS[qb], dQ[db][qb]);
+      beside(db);
     }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  for (int u = 0; u < nunits; u += 2) {
+    // units u and u + 1 have landed (this wave's part), then everybody's; the four after them may stay in flight
+    if (u + 4 < nunits) wait_vm<4 * LPW>();
+    else if (u + 2 < nunits) wait_vm<2 * LPW>();
+    else wait_vm<0>();
+    lds_barrier();
+    // every wave is past units u - 1 and u - 2: their slots take the next two
+    if (u + NRU - 2 < nunits) {
+      issue_unit(u + NRU - 2);
+      issue_unit(u + NRU - 1);
+    }
+    const uint32_t b0 = (uint32_t)((u & (NRU - 1)) * UNIT), b1 = b0 + UNIT;   // (u is even, so is NRU)
+    Unit t0, t1;
+    Frags k0 = row_frags(b0, 0), v0, k1, v1, c0f, c1f;
+    scores(t0, b0, k0, [](int) {}, [&] { v0 = row_frags(b0 + UB, 0); });
+    mask(t0, u);
+    dprob(t0, b0, v0, [&] { k1 = row_frags(b1, 0); });
+    scores(t1, b1, k1, [&](int ks) { if (ks >= 1 && ks <= RQB) form_ds(t0, ks - 1); }, [&] { v1 = row_frags(b1 + UB, 0); });
+    mask(t1, u + 1);
+    dprob(t1, b1, v1, [&] { c0f = columns(b0); });
+    dquery(t0, b0, c0f, [&](int db) { if (db >= 1 && db <= RQB) form_ds(t1, db - 1); }, [&] { c1f = columns(b1); });
+    dquery(t1, b1, c1f, [](int) {}, [] {});
   }
 #pragma unroll
   for (int qb = 0; qb < RQB; ++qb) {
@@ -264,8 +304,7 @@ struct DkvP {
   float scale;
 };
 
-// an item: q tile | do tile | 32 (lse, delta) pairs; a tile in 1 KB blocks of 16 rows x 32 columns, two planes of 32-byte rows
-// each, which both the row fragments and the transposing reads take without bank conflicts
+// an item: q tile | do tile | 32 (lse, delta) pairs
 constexpr int KV_Q = 0, KV_O = UB, KV_LD = 2 * UB, KV_ITEM = 2 * UB + 256;
 template <int KEYS> constexpr int KV_BYTES = NR * KV_ITEM + KEYS * D * 2;   // ring, then the V rows of the workgroup's keys
 
