@@ -15,6 +15,7 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 #define NHA_LDS __attribute__((address_space(3)))
 typedef NHA_LDS bf16_t lbf16;
 typedef NHA_LDS float lfloat;
+typedef NHA_LDS unsigned char lbyte;
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void lds_st16(lbf16* p, uint4 v) { *reinterpret_cast<NHA_LDS u32x4*>(p) = (u32x4){v.x, v.y, v.z, v.w}; }
@@ -74,8 +75,6 @@ __device__ __forceinline__ bf16x8 pack8(f32x4 a, f32x4 b) {
   return r;
 }
 
-// workgroup barrier that orders LDS traffic only: outstanding global loads (tile prefetches) stay
-// in flight across it
 // Tile of a workgroup in a launch of (kv-heads x groups-per-kv-head, chunks) tiles.  Workgroups are dispatched
 // in the order L = y * gridDim.x + x and workgroup L runs on XCD L % 8, each XCD with its own L2: XCD k takes
 // the k-th eighth of the tile sequence (kv-head, chunk, group of the kv-head), fastest last, so that what an
@@ -91,6 +90,63 @@ __device__ __forceinline__ void xcd_tile(int ngrp, int nchunks, int& vx, int& vy
   vx = (rest / nchunks) * ngrp + g;
 }
 
+// Two chunks of a sequence per workgroup: launch index -> (head x, sequence n, first chunk it of the pair); false for the
+// workgroups beyond the last pair.  The launch (pair_grid) has room for the most pairs that NT chunks in N sequences can make;
+// the pairs are counted without gaps, so that the working workgroups come first: left strewn over the launch order, those that
+// leave at once give the shader engines unequal shares of the others (2 x 4000 tokens, 4 heads: 256 pairs on 256 CUs took two
+// rounds).  As in xcd_tile XCD k takes the k-th eighth of the sequence (kv-head, pair, head of the kv-head's ngrp), the
+// pairs from the last to the first.  Each wave counts for itself, 64 sequences at a time.
+__device__ __forceinline__ bool pair_tile(const int32_t* coff, int N, int heads, int ngrp, int& x, int& n, int& it) {
+  const int lane = threadIdx.x & 63, L = blockIdx.x;
+  auto pairs = [&](int n0) { return n0 + lane < N ? (coff[n0 + lane + 1] - coff[n0 + lane] + 1) >> 1 : 0; };
+  auto prefix = [&](int c) {   // over the wave, inclusive (DPP: rows of 16 lanes, then across the rows)
+    c += __builtin_amdgcn_update_dpp(0, c, 0x111, 0xf, 0xf, false);
+    c += __builtin_amdgcn_update_dpp(0, c, 0x112, 0xf, 0xf, false);
+    c += __builtin_amdgcn_update_dpp(0, c, 0x114, 0xf, 0xf, false);
+    c += __builtin_amdgcn_update_dpp(0, c, 0x118, 0xf, 0xf, false);
+    c += __builtin_amdgcn_update_dpp(0, c, 0x142, 0xa, 0xf, false);
+    c += __builtin_amdgcn_update_dpp(0, c, 0x143, 0xc, 0xf, false);
+    return c;
+  };
+  int c = pairs(0), incl = prefix(c), total = __builtin_amdgcn_readlane(incl, 63);
+  for (int n0 = 64; n0 < N; n0 += 64) total += __builtin_amdgcn_readlane(prefix(pairs(n0)), 63);
+  const int work = heads * total, per = work >> 3;
+  if (L >= work) return false;
+  const int v = L < 8 * per ? (L & 7) * per + (L >> 3) : L, g = v % ngrp, rest = v / ngrp;
+  x = (rest / total) * ngrp + g;
+  const int k = total - 1 - rest % total;
+  int base = 0;
+  for (int n0 = 0; n0 < N; n0 += 64) {
+    if (n0) c = pairs(n0), incl = prefix(c);
+    const int first = base + incl - c;
+    const uint64_t hit = __ballot(k >= first && k < first + c);
+    if (hit) {
+      const int at = __builtin_ctzll(hit);
+      n = n0 + at;
+      it = 2 * (k - __builtin_amdgcn_readlane(first, at));
+      return true;
+    }
+    base += __builtin_amdgcn_readlane(incl, 63);
+  }
+  return false;
+}
+static inline dim3 pair_grid(int heads, int NT, int N) { return dim3((unsigned)heads * ((unsigned)(NT + N) / 2)); }
+
+// 16 bytes per lane from global memory into LDS at lds_base + 16 * lane (lds_base wave-uniform).
+// Issued outside the compiler's memory model: every wait on these loads is written by hand.
+__device__ __forceinline__ void g2l16(const void* gbase, uint32_t voff_bytes, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff_bytes), "s"(gbase), "s"(lds_base) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void g2l4(const void* gbase, uint32_t voff_bytes, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff_bytes), "s"(gbase), "s"(lds_base) : "memory");
+}
+
+// workgroup barrier that orders LDS traffic only: outstanding global loads (tile prefetches) stay
+// in flight across it
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // max over the four 16-lane rows of a wave (lanes l, l^16, l^32, l^48), VALU only
@@ -119,6 +175,45 @@ __device__ __forceinline__ bf16x8 lds_frag_tr(const lbf16* tile, int ld, int r0a
   t.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)pb);
   return __builtin_bit_cast(bf16x8, t);
 }
+
+// A 32-row bf16 tile in LDS that LDS-direct loads fill and both row fragments and transposing reads take without bank
+// conflicts.  Blocks of 8 rows x 64 columns (1 KB, one load of a wave, eight neighbouring lanes a whole 128-byte line of a row);
+// the 16-byte piece c of row r lies at piece c ^ f(r) of its 128 bytes.  f takes all eight values over the even rows of 16 and
+// over the odd ones (a fragment's 16 pieces meet every bank once), and f / 2 all four over the even rows of eight (so do the
+// 32 bytes of eight rows that half a wave's transposing read takes).
+// What neighbouring lanes cover decides the rate of the loads, one line a cycle: out of L2 a CU pulls 38 GB/s in 16-byte pieces of
+// 16 rows, 74 in 32-byte pieces, 135 in 64-byte and 133 in 128-byte rows, all 256 together 9.4, 18.0, 20.5 and 30.1 TB/s.
+template <int D>
+struct SwzTile {
+  static constexpr int ROWB = D / 64 * 1024;   // bytes of eight rows
+  static constexpr int HALF = 2 * ROWB;        // and of 16
+  const lbyte* lds;
+  uint32_t row_at, col_at;
+  static __device__ __forceinline__ int f(int r) { return ((r >> 1) & 3) * 2 + ((r >> 3) & 1); }
+  __device__ __forceinline__ SwzTile(const lbyte* l, int lane) : lds(l) {
+    const int l16 = lane & 15, kb = lane >> 4, r = 4 * kb + (l16 >> 2);
+    row_at = (uint32_t)((l16 >> 3) * ROWB + (l16 & 7) * 128 + (kb ^ f(l16)) * 16);
+    col_at = (uint32_t)((r >> 3) * ROWB + (r & 7) * 128 + (((l16 >> 1) & 1) ^ f(r)) * 16 + (l16 & 1) * 8);
+  }
+  // loads: where block (eight rows rb, 64 columns cb) lies, and the first of the eight columns that a lane takes of row
+  // 8 rb + lane / 8
+  static __device__ __forceinline__ uint32_t block(int rb, int cb) { return (uint32_t)(rb * ROWB + cb * 1024); }
+  static __device__ __forceinline__ uint32_t load_col(int rb, int cb, int lane) {
+    return (uint32_t)(64 * cb + 8 * ((lane & 7) ^ f(8 * (rb & 1) + (lane >> 3))));
+  }
+  // row fragment of the tile at byte address a (a multiple of 128): row 16 rh + l16, columns 32 ks + 8 kb ..
+  __device__ __forceinline__ bf16x8 row(uint32_t a, int rh, int ks) const {
+    return *reinterpret_cast<const NHA_LDS bf16x8*>(lds + ((a + row_at) ^ ((ks & 1) * 64)) + rh * HALF + (ks >> 1) * 1024);
+  }
+  // transposed fragment: X[4 kb + e][16 c + l16] (e < 4) and X[16 + 4 kb + e - 4][..]
+  __device__ __forceinline__ bf16x8 col(uint32_t a, int c) const {
+    const lbyte* pa = lds + ((a + col_at) ^ ((c & 3) * 32)) + (c >> 2) * 1024;
+    struct { s16x4 a, b; } t;
+    t.a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)pa);
+    t.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)(pa + HALF));
+    return __builtin_bit_cast(bf16x8, t);
+  }
+};
 
 // the slot recurrence is cut into segments of 1 << sh <= SEG chunks (two-level state pass; prefill_mfma.hip: plan_scratch)
 constexpr int SEG = 8;

@@ -39,16 +39,6 @@ namespace nha {
 namespace {
 using namespace mf;
 
-typedef NHA_LDS unsigned char lbyte;
-
-__device__ __forceinline__ void g2l16(const void* gbase, uint32_t voff_bytes, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff_bytes), "s"(gbase), "s"(lds_base) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 struct DqP {
   const bf16_t *q, *k, *v, *dout;          // q_swa [T,HQ,D]; k_swa, v [T,H,D]; dout [T,HQ,D]
   const float *lse_swa, *lse_gsa, *delta;  // [T,HQ]
@@ -307,10 +297,6 @@ struct DkvP {
 // an item: q tile | do tile | 32 (lse, delta) pairs
 constexpr int KV_Q = 0, KV_O = UB, KV_LD = 2 * UB, KV_ITEM = 2 * UB + 256;
 template <int KEYS> constexpr int KV_BYTES = NR * KV_ITEM + KEYS * D * 2;   // ring, then the V rows of the workgroup's keys
-
-__device__ __forceinline__ void g2l4(const void* gbase, uint32_t voff_bytes, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff_bytes), "s"(gbase), "s"(lds_base) : "memory");
-}
 
 // KEYS: keys per workgroup, 256 or 128 (a wave holds KEYS / 8 of them).  With 256 every q / do fragment read from LDS
 // feeds two matrix products, with 128 one: long windows, which are bound by those reads, take 256 (headline shape:

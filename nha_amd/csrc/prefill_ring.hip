@@ -37,7 +37,6 @@ namespace nha {
 namespace {
 using namespace mf;
 
-typedef NHA_LDS unsigned char lbyte;
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // nothing crosses: the instruction order of the loop is the source order
@@ -52,15 +51,6 @@ __device__ __forceinline__ unsigned cvt2(float a, float b) {
   return __builtin_bit_cast(unsigned, t);
 }
 
-// 16 bytes per lane from global memory into LDS at lds_base + 16 * lane (lds_base wave-uniform).
-// Issued outside the compiler's memory model: every wait on these loads is written by hand.
-__device__ __forceinline__ void g2l16(const void* gbase, uint32_t voff_bytes, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff_bytes), "s"(gbase), "s"(lds_base) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 // 16 bytes per lane from global memory into registers, outside the compiler's memory model like the loads above: the
 // wait the compiler writes for a load of its own does not know of the LDS-direct requests behind it and waits for
 // all of them.  The value is there after wait_vm<N> with at most N younger requests pending; until then nothing may

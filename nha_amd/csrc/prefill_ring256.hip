@@ -33,7 +33,6 @@ namespace nha {
 namespace {
 using namespace mf;
 
-typedef NHA_LDS unsigned char lbyte;
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 #define NHA_FENCE() __builtin_amdgcn_sched_barrier(0)
@@ -44,16 +43,6 @@ __device__ __forceinline__ unsigned cvt2(float a, float b) {
   t[0] = (__bf16)a;
   t[1] = (__bf16)b;
   return __builtin_bit_cast(unsigned, t);
-}
-
-// 16 bytes per lane from global memory into LDS at lds_base + 16 * lane (lds_base wave-uniform).
-// Issued outside the compiler's memory model: every wait on these loads is written by hand.
-__device__ __forceinline__ void g2l16(const void* gbase, uint32_t voff_bytes, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff_bytes), "s"(gbase), "s"(lds_base) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
 template <int NCH>
@@ -75,38 +64,6 @@ struct Cfg {
   static constexpr int BYTES = GC2 + (NCH - 1) * 16384;
 };
 
-// Two chunks per workgroup: launch index -> (query head, chunk).  The grid has a workgroup per (query head, chunk);
-// those of a sequence's odd chunks leave at once.  The even chunk indices come first in the launch order (in sequences
-// of even chunk counts they are the working ones), from the last chunk to the first, and as in xcd_tile XCD k (launch
-// index % 8) takes the k-th eighth of each class, so that neighbouring pairs of a kv-head meet in one L2.
-__device__ __forceinline__ void pair_tile(int ngrp, int nchunks, int& vx, int& chunk) {
-  const int nev = (nchunks + 1) >> 1, nod = nchunks >> 1;
-  const int L = blockIdx.y * gridDim.x + blockIdx.x;
-  const int tot_e = gridDim.x * nev, tot_o = gridDim.x * nod;
-  // each class is dealt to the XCDs in eighths; the up to seven workgroups a class has beyond a multiple of 8 keep
-  // their place at its end
-  int v, nn, par;
-  const int pe = tot_e >> 3, po = tot_o >> 3;
-  if (L < 8 * (pe + po)) {
-    const int k = L & 7, w = L >> 3;
-    if (w < pe) {
-      v = k * pe + w, nn = nev, par = 0;
-    } else {
-      v = k * po + (w - pe), nn = nod, par = 1;
-    }
-  } else {
-    const int r = L - 8 * (pe + po);   // < (tot_e & 7) + (tot_o & 7)
-    if (r < (tot_e & 7)) {
-      v = 8 * pe + r, nn = nev, par = 0;
-    } else {
-      v = 8 * po + r - (tot_e & 7), nn = nod, par = 1;
-    }
-  }
-  const int g = v % ngrp, rest = v / ngrp;
-  vx = (rest / nn) * ngrp + g;
-  chunk = 2 * (nn - 1 - rest % nn) + par;
-}
-
 // LDS layouts as in prefill_ring.hip: a 32-row buffer is cut into 16-row x 32-column blocks of 1 KB
 // (half h, column block c at h * HB + c * 1024).  K layout: 16-byte piece c of row r at 256 c + 16 r (a wave's
 // row fragments are 1 KB of consecutive bytes).  V layout: two planes of 16 rows x 32 bytes (columns 0..15, then 16..31).
@@ -121,23 +78,20 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, kb = lane >> 4;
   const int H = p.H, HQ = p.HQ, NG = p.NG;
-  // grid = (query head, chunk), tiles dealt so that an XCD works on neighbouring chunks of one kv-head
-  // (xcd_tile); chunks from the last to the first
-  int vx, chunk;
+  // tiles dealt so that an XCD works on neighbouring chunks of one kv-head (xcd_tile, pair_tile); chunks from the last to the first
+  int vx, chunk, n, it;
   if constexpr (NCH == 1) {
     int vy;
     xcd_tile(NG, p.NT, vx, vy);
     chunk = p.NT - 1 - vy;
+    n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
   } else {
-    pair_tile(NG, p.NT, vx, chunk);
+    if (!pair_tile(p.coff, p.N, p.HQ, NG, vx, n, it)) return;
+    chunk = p.coff[n] + it;
   }
   const int hq = vx, h = hq / NG;
   const int ch = wave >> 2;                    // this wave's chunk of the workgroup's NCH
   const int Q = wave & 3;                      // its 16-row sub-block of that chunk
-  const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
-  // two chunks per workgroup: the workgroup of a sequence's even chunk takes that chunk and the next one of the
-  // same sequence, if there is one; the workgroups of the odd chunks leave at once
-  if (NCH == 2 && (it & 1)) return;
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int c0 = bos + it * BT;                // first row of the workgroup (its first chunk)
   const int rows_wg = (eos - c0) < NCH * BT ? (eos - c0) : NCH * BT;
@@ -828,7 +782,7 @@ int prefill_ring256_launch(const mf::MP& p, hipStream_t st) {
   if (2 * (int64_t)p.NT < 3 * (int64_t)p.N)
     hipLaunchKernelGGL(ring256_out_kernel<1>, dim3(p.HQ, p.NT), dim3(256), Cfg<1>::BYTES, st, p);
   else
-    hipLaunchKernelGGL(ring256_out_kernel<2>, dim3(p.HQ, p.NT), dim3(512), Cfg<2>::BYTES, st, p);
+    hipLaunchKernelGGL(ring256_out_kernel<2>, pair_grid(p.HQ, p.NT, p.N), dim3(512), Cfg<2>::BYTES, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma output pass, ring, head size 256)");
   return NHA_OK;
 }
