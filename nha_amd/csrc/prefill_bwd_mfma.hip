@@ -421,7 +421,9 @@ __global__ __launch_bounds__(256) void bwd_dkv_kernel(const WP p) {
 // ------------------------------------------------------------------------------------------
 // Slot branch, the parts that involve the state gradient carried in from later chunks (the rest: prefill_bwd_slot.hip)
 // ------------------------------------------------------------------------------------------
-constexpr int TLD = 72;   // bf16 row stride of the 64 x 64 tables in LDS
+// bf16 row stride of tables of 64 columns in LDS.  They are read 16 bytes per lane of 16 rows and transposed: 4.15 and 3.3
+// cycles per wave instruction at 80 (a workgroup of eight waves), 8.1 and 4.4 at 72.
+constexpr int TLD = 80;
 
 struct SP2 {
   const bf16_t *kg, *v, *s;          // k_gsa, v [T,H,D]; s [T,H,64]
@@ -461,7 +463,7 @@ __device__ __forceinline__ void split4_bf16(const float4 x, lbf16* hi, lbf16* lo
 // state and column range; the gate kernel adds the slabs).
 template <int D, int DW>
 __global__ __launch_bounds__(256) void bwd_slot_inter_kernel(const SP2 p) {
-  constexpr int DB = DW / 16, LDT = DW + 16, TILE = BT * LDT, ELD = BT + 8, NH = D / DW;
+  constexpr int DB = DW / 16, LDT = DW + 16, TILE = BT * LDT, ELD = TLD, NH = D / DW;
   extern __shared__ __align__(16) unsigned char smem[];
   lbf16* const Yt = (lbf16*)smem;        // [64 rows r][DW]  k' / v'
   lbf16* const Et = Yt + TILE;           // [DW x][ELD]      E[x][m], high part
@@ -687,7 +689,7 @@ int bwd_window_mfma_dkv(const NhaPrefillBwdArgs* a, const float* delta, const fl
 template <int D>
 static int launch_slot_inter(const SP2& p, int NT, hipStream_t st) {
   constexpr int DWI = D > 128 ? 128 : D;   // columns per workgroup
-  const size_t lds = (size_t)BT * (DWI + 16) * 2 + (size_t)2 * DWI * (BT + 8) * 2 + (size_t)2 * BT * TLD * 2;
+  const size_t lds = (size_t)BT * (DWI + 16) * 2 + (size_t)2 * DWI * TLD * 2 + (size_t)2 * BT * TLD * 2;
   static std::atomic<bool> configured{false};   // the attribute call is idempotent: a second thread may repeat it
   if (!configured) {
     hipError_t e = hipFuncSetAttribute((const void*)bwd_slot_inter_kernel<D, DWI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -38,8 +38,12 @@ using namespace mf;
 // keeps the scheduler from collecting the operand reads of a whole unrolled stage in registers
 #define FENCE __builtin_amdgcn_sched_barrier(0)
 
-constexpr int TLD = 72;    // row stride (bf16) of the 64 x 64 tables
-constexpr int HLD = 36;    // row stride of the tables that hold rows 32..63 only
+// Row strides (bf16).  The tables are read and written 8 bytes per lane, along rows and transposed; the tiles are read 16
+// bytes per lane of 16 rows and transposed.  LDS cycles of a wave instruction with eight waves at it: tile rows 8.1 at D + 8,
+// 4.15 at D + 16; tiles transposed 4.4 / 3.3; tables written transposed 8.1 at 72, 6.4 at 68, read so 3.3 / 4.5, transposing
+// read 4.4 / 4.5.  68 is what leaves room for the tiles' D + 16.
+constexpr int TLD = 68;    // 64 x 64 tables
+constexpr int HLD = 36;    // tables that hold rows 32..63 only
 
 __device__ __forceinline__ float logaddexp_f(float a, float b) {
   const float mx = fmaxf(a, b);
@@ -99,17 +103,17 @@ struct SlotP {
 };
 
 template <int DW> struct SlotLds {
-  static constexpr int LDT = DW + 8, TILE = BT * LDT, TAB = BT * TLD, HTAB = BT * HLD;
+  static constexpr int LDT = DW + 16, TILE = BT * LDT, TAB = BT * TLD, HTAB = BT * HLD;
   static constexpr int Q = 0, O = Q + TILE;     // bf16 offsets
   static constexpr int X0 = O + TILE;           // X0 hi, lo, Xp0 hi, lo   [64 m][TLD]; u / dp in transit
   static constexpr int A = X0 + 4 * TAB;        // A, B [64 j][TLD], then X1 hi, lo, Xp1 hi, lo [64 m][HLD]
   static constexpr int X1 = A + 2 * TAB;
   static constexpr int C = A;                   // ck hi, lo, cv hi, lo [64 r][TLD], once A, B, X1, Xp1 are done with
-  static constexpr int S = A + 4 * TAB;         // k-state [64 m][LDT], k' [64 j][LDT]; first the other columns of q and do
+  static constexpr int S = X1 + 4 * HTAB;        // k-state [64 m][LDT], k' [64 j][LDT]; first the other columns of q and do
   static constexpr int ROW = S + 2 * TILE;                      // floats: delta, lse, lse_gsa, dlse_gsa of the 64 rows
   static constexpr int Y = ROW + 2 * 4 * BT;                    // Y hi, lo [64 j][TLD]
   static constexpr size_t BYTES = (size_t)(Y + 2 * TAB) * 2;
-  static_assert(2 * TAB + 4 * HTAB == 4 * TAB, "ck and cv fit where A, B, X1 and Xp1 were");
+  static_assert(2 * TAB <= 4 * HTAB, "ck and cv fit where A, B, X1 and Xp1 were");
   static_assert(BYTES <= 160 * 1024, "LDS");
 };
 
