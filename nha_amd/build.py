@@ -8,7 +8,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libnha_hip.so")
-SOURCES = ["abi.hip", "decode.hip", "decode_mfma.hip", "decode_split.hip", "prefill_simple.hip", "prefill_f32.hip", "prefill_mfma.hip", "prefill_ring.hip", "prefill_ring256.hip", "prefill_bwd.hip", "prefill_bwd_mfma.hip", "prefill_bwd_slot.hip", "prefill_bwd_ring.hip",
+SOURCES = ["abi.hip", "decode.hip", "decode_mfma.hip", "decode_split.hip", "prefill_simple.hip", "prefill_f32.hip", "prefill_mfma.hip", "prefill_ring.hip", "prefill_ring256.hip", "prefill_bwd.hip", "prefill_bwd_mfma.hip", "prefill_bwd_slot.hip", "prefill_bwd_ring.hip", "prefill_bwd_ring256.hip",
            "layer_fuse.hip", "wgrad.hip", "hybrid_fuse.hip", "ring_fill.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -23,7 +23,8 @@ FLAGS = [
 # canonicalised by an extra VALU instruction in the softmax inner loop.  decode_split.hip goes without it: its merge asks
 # which partial sums are NaN, and its steps take the same time (12.5 us at 24 pairs, W = 2048)
 EXTRA = {"prefill_mfma.hip": ["-fno-honor-nans"], "prefill_ring.hip": ["-fno-honor-nans"], "prefill_ring256.hip": ["-fno-honor-nans"], "decode_mfma.hip": ["-fno-honor-nans"],
-         "prefill_bwd_mfma.hip": ["-fno-honor-nans"], "prefill_bwd_slot.hip": ["-fno-honor-nans"], "prefill_bwd_ring.hip": ["-fno-honor-nans"]}
+         "prefill_bwd_mfma.hip": ["-fno-honor-nans"], "prefill_bwd_slot.hip": ["-fno-honor-nans"], "prefill_bwd_ring.hip": ["-fno-honor-nans"],
+         "prefill_bwd_ring256.hip": ["-fno-honor-nans"]}
 
 
 STAMP = os.path.join(HERE, "build", "sources.sha256")

@@ -177,6 +177,11 @@ bool bwd_ring_supported(const NhaPrefillBwdArgs* a);
 bool bwd_ring_dkv_supported(const NhaPrefillBwdArgs* a);
 int bwd_ring_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld);
 int bwd_ring_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs);
+// prefill_bwd_ring256.hip: the same for K = V = 256, any number of query heads per kv-head
+bool bwd_ring256_dq_supported(const NhaPrefillBwdArgs* a);
+bool bwd_ring256_dkv_supported(const NhaPrefillBwdArgs* a);
+int bwd_ring256_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld);
+int bwd_ring256_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs);
 int bwd_window_mfma_dkv(const NhaPrefillBwdArgs* a, const float* delta, const float* dvs, const void* ld);
 
 }  // namespace nha

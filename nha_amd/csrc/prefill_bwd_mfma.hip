@@ -33,6 +33,7 @@ struct WP {
   const bf16_t *q, *k, *v, *dout;          // q_swa [T,HQ,D]; k_swa, v [T,H,D]; dout [T,HQ,D]
   const float *lse_swa, *lse_gsa, *delta;  // [T,HQ]
   const float* dvs;                        // [T,H,D] slot-branch part of dv
+  float2* ld;                              // [T,HQ] out of the dq kernel, where the dk / dv kernel wants it: (-lse log2(e), -delta)
   bf16_t *dq, *dk, *dv;
   const int32_t *cu, *cidx;
   int HQ, H, NG, wl;
@@ -156,6 +157,7 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(const WP p) {
   const float lse2 = valid ? logaddexp_f(p.lse_swa[tq], p.lse_gsa[tq]) * LOG2E : 0.f;
   const float dl = valid ? p.delta[tq] : 0.f;
   const float cs = p.scale * LOG2E;
+  if (p.ld && valid && kb == 0) p.ld[tq] = make_float2(-lse2, -dl);
   f32x4 dQ[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) dQ[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -652,6 +654,7 @@ int launch_dkv(const WP& p, int NT, hipStream_t st) {
 
 WP make_wp(const NhaPrefillBwdArgs* a, const float* delta, const float* dvs) {
   WP p;
+  p.ld = nullptr;
   p.q = (const bf16_t*)a->q_swa; p.k = (const bf16_t*)a->k_swa; p.v = (const bf16_t*)a->v;
   p.dout = (const bf16_t*)a->dout;
   p.lse_swa = a->lse_swa; p.lse_gsa = a->lse_gsa; p.delta = delta; p.dvs = dvs;
@@ -670,7 +673,9 @@ bool bwd_window_mfma_supported(const NhaPrefillBwdArgs* a) {
 
 int bwd_window_mfma_dq(const NhaPrefillBwdArgs* a, const float* delta, void* ld) {
   if (bwd_ring_supported(a)) return bwd_ring_dq(a, delta, (float2*)ld);
-  const WP p = make_wp(a, delta, nullptr);
+  if (bwd_ring256_dq_supported(a)) return bwd_ring256_dq(a, delta, (float2*)ld);
+  WP p = make_wp(a, delta, nullptr);
+  if (bwd_ring256_dkv_supported(a)) p.ld = (float2*)ld;
   hipStream_t st = (hipStream_t)a->stream;
   if (a->K == 64) return launch_dq<64, 64>(p, a->NT, st);
   if (a->K == 128) return launch_dq<128, 64>(p, a->NT, st);
@@ -679,6 +684,7 @@ int bwd_window_mfma_dq(const NhaPrefillBwdArgs* a, const float* delta, void* ld)
 
 int bwd_window_mfma_dkv(const NhaPrefillBwdArgs* a, const float* delta, const float* dvs, const void* ld) {
   if (bwd_ring_dkv_supported(a)) return bwd_ring_dkv(a, (const float2*)ld, dvs);
+  if (bwd_ring256_dkv_supported(a)) return bwd_ring256_dkv(a, (const float2*)ld, dvs);
   const WP p = make_wp(a, delta, dvs);
   hipStream_t st = (hipStream_t)a->stream;
   if (a->K == 64) return launch_dkv<64, 64, false>(p, a->NT, st);

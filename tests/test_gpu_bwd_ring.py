@@ -1,7 +1,7 @@
-"""Window gradients from the LDS-direct kernels (four or eight query heads per kv-head at K = V = 128, more key groups than 128)
-against the fp32 call (generic kernels) on the same bf16-rounded inputs: ragged packed sequences that end inside a 32-row unit,
-a chunk and a group of four chunks, windows below and above the 160 keys where the key groups change size, odd and even numbers
-of units, longer than every sequence and unbounded."""
+"""Window gradients from the LDS-direct kernels (K = V = 128: four or eight query heads per kv-head, more key groups than 128;
+K = V = 256: any grouping, more than 256 chunks x kv-heads) against the fp32 call (generic kernels) on the same bf16-rounded
+inputs: ragged packed sequences that end inside a 32-row unit, a chunk and a group of chunks, windows below and above those where
+the kernels and their key groups change, odd and even numbers of units, longer than every sequence and unbounded."""
 import pytest
 import torch
 
@@ -11,22 +11,38 @@ from tests.util import prefill_inputs
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("NG", [4, 8])
-@pytest.mark.parametrize("wl", [-1, 0, 31, 64, 159, 160, 383, 500, 2000])
-def test_window_gradients_of_many_key_groups(wl, NG):
+def compare(cu, wl, H, NG, D, keys):
     from nha_amd import chunk_nha
-    H, D, M = 32, 128, 64
-    cu = [0, 1, 40, 104, 361, 1190]
-    print("case", wl, NG, flush=True)
-    assert H * (sum((b - a + 63) // 64 for a, b in zip(cu, cu[1:])) // 4) > 128     # otherwise other kernels take dk and dv
-    d = prefill_inputs(9100 + wl + NG, 1, cu[-1], H * NG, H, D, D, M, dtype=BF, qk_scale=1.0)
+    d = prefill_inputs(9100 + wl + NG, 1, cu[-1], H * NG, H, D, D, 64, dtype=BF, qk_scale=1.0)
     do = torch.randn(1, cu[-1], H * NG, D, generator=torch.Generator().manual_seed(wl + 5)).to(BF)
-    grads = []
+    outs, grads = [], []
     for dt in (BF, torch.float32):
         x = [d[k].cuda().to(dt).requires_grad_(True) for k in KEYS]
         o = chunk_nha(*x, cu_seqlens=torch.tensor(cu, dtype=torch.int32).cuda(), scale=D ** -0.5, window_size_left=wl, gsa_kv_shift=0)[0]
         o.backward(do.cuda().to(dt))
+        outs.append(o.detach())
         grads.append([t.grad for t in x])
+    check_grad(f"wl={wl} o", outs[0], outs[1].double().cpu(), BF)
     for k, gb, gf in zip(KEYS, *grads):
-        if k in ("q_swa", "k_swa", "v"):
+        if k in keys:
             check_grad(f"wl={wl} d{k}", gb, gf.double().cpu(), BF)
+
+
+@pytest.mark.parametrize("H,NG,D", [(32, 4, 128), (32, 8, 128), (16, 1, 256), (13, 3, 256)])
+@pytest.mark.parametrize("wl", [-1, 0, 31, 64, 159, 160, 192, 383, 384, 500, 2000])
+def test_window_gradients_of_many_key_groups(wl, H, NG, D):
+    cu = [0, 1, 40, 104, 361, 1190]
+    print("case", wl, H, NG, D, flush=True)
+    # otherwise other kernels take dk and dv
+    chunks = sum((b - a + 63) // 64 for a, b in zip(cu, cu[1:]))
+    assert H * chunks > 256 if D == 256 else H * (chunks // 4) > 128
+    compare(cu, wl, H, NG, D, ("q_swa", "k_swa", "v"))
+
+
+@pytest.mark.parametrize("wl", [40, 400])
+def test_more_sequences_than_lanes(wl):
+    """The workgroups of two chunks count the pairs of 64 sequences at a time: 150 of them, empty ones among them."""
+    lens = [(37 * i) % 131 for i in range(150)]
+    cu = torch.tensor([0, *lens]).cumsum(0).tolist()
+    print("case", wl, flush=True)
+    compare(cu, wl, 4, 1, 256, KEYS)
