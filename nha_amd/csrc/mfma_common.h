@@ -176,38 +176,40 @@ __device__ __forceinline__ bf16x8 lds_frag_tr(const lbf16* tile, int ld, int r0a
   return __builtin_bit_cast(bf16x8, t);
 }
 
-// A 32-row bf16 tile in LDS that LDS-direct loads fill and both row fragments and transposing reads take without bank
-// conflicts.  Blocks of 8 rows x 64 columns (1 KB, one load of a wave, eight neighbouring lanes a whole 128-byte line of a row);
-// the 16-byte piece c of row r lies at piece c ^ f(r) of its 128 bytes.  f takes all eight values over the even rows of 16 and
-// over the odd ones (a fragment's 16 pieces meet every bank once), and f / 2 all four over the even rows of eight (so do the
-// 32 bytes of eight rows that half a wave's transposing read takes).
-// What neighbouring lanes cover decides the rate of the loads, one line a cycle: out of L2 a CU pulls 38 GB/s in 16-byte pieces of
-// 16 rows, 74 in 32-byte pieces, 135 in 64-byte and 133 in 128-byte rows, all 256 together 9.4, 18.0, 20.5 and 30.1 TB/s.
+// A 32-row bf16 tile in LDS that LDS-direct loads fill and both row fragments and transposing reads take at the LDS's full rate.
+// Blocks of 16 rows x 32 columns (1 KB, one load of a wave, four neighbouring lanes 64 consecutive bytes of a row); the
+// 16-byte piece c of row r lies at piece c ^ f(r) of its 64 bytes, f(r) = -(r / 4) mod 4.  Cycles of a wave instruction (eight waves):
+// row fragment 4.1, transposing read 3.2; with f(r) = r / 4, 8.1 and 4.5.
+// What neighbouring lanes cover decides the rate of the loads: out of L2 a CU pulls 38 GB/s in 16-byte pieces of 16 rows, 74 in 32-byte
+// pieces, 135 in 64-byte and 133 in 128-byte rows; all 256 together 9.4, 18.0, 20.5 and 30.1 TB/s.
 template <int D>
-struct SwzTile {
-  static constexpr int ROWB = D / 64 * 1024;   // bytes of eight rows
-  static constexpr int HALF = 2 * ROWB;        // and of 16
+struct LineTile {
+  static constexpr int HALF = D / 32 * 1024;   // bytes of 16 rows
+  static __device__ __forceinline__ int f(int r) { return -(r >> 2) & 3; }
+  // loads: where the block of rows 16 rh .. and columns 32 cb .. lies; the row of it that a lane takes eight columns of, and the
+  // first of them
+  static __device__ __forceinline__ uint32_t block(int rh, int cb) { return (uint32_t)(rh * HALF + cb * 1024); }
+  static __device__ __forceinline__ int load_row(int lane) { return lane >> 2; }
+  static __device__ __forceinline__ uint32_t load_col(int cb, int lane) { return (uint32_t)(32 * cb + 8 * ((lane & 3) ^ f(lane >> 2))); }
+  // reads: byte offsets of a lane's part of a row fragment and of a transposing read of even / odd 16-column blocks
+  static __device__ __forceinline__ uint32_t row_at(int lane) {
+    const int l16 = lane & 15, kb = lane >> 4;
+    return (uint32_t)(l16 * 64 + (kb ^ f(l16)) * 16);
+  }
+  static __device__ __forceinline__ uint32_t col_at(int lane) {
+    const int l16 = lane & 15, r = 4 * (lane >> 4) + (l16 >> 2);
+    return (uint32_t)(r * 64 + (((l16 >> 1) & 1) ^ f(r)) * 16 + (l16 & 1) * 8);
+  }
   const lbyte* lds;
-  uint32_t row_at, col_at;
-  static __device__ __forceinline__ int f(int r) { return ((r >> 1) & 3) * 2 + ((r >> 3) & 1); }
-  __device__ __forceinline__ SwzTile(const lbyte* l, int lane) : lds(l) {
-    const int l16 = lane & 15, kb = lane >> 4, r = 4 * kb + (l16 >> 2);
-    row_at = (uint32_t)((l16 >> 3) * ROWB + (l16 & 7) * 128 + (kb ^ f(l16)) * 16);
-    col_at = (uint32_t)((r >> 3) * ROWB + (r & 7) * 128 + (((l16 >> 1) & 1) ^ f(r)) * 16 + (l16 & 1) * 8);
-  }
-  // loads: where block (eight rows rb, 64 columns cb) lies, and the first of the eight columns that a lane takes of row
-  // 8 rb + lane / 8
-  static __device__ __forceinline__ uint32_t block(int rb, int cb) { return (uint32_t)(rb * ROWB + cb * 1024); }
-  static __device__ __forceinline__ uint32_t load_col(int rb, int cb, int lane) {
-    return (uint32_t)(64 * cb + 8 * ((lane & 7) ^ f(8 * (rb & 1) + (lane >> 3))));
-  }
-  // row fragment of the tile at byte address a (a multiple of 128): row 16 rh + l16, columns 32 ks + 8 kb ..
+  uint32_t ra, ca;
+  __device__ __forceinline__ LineTile(const lbyte* l, int lane) : lds(l), ra(row_at(lane)), ca(col_at(lane)) {}
+  // row fragment of the tile at byte address a (a multiple of 64): row 16 rh + l16, columns 32 ks + 8 kb ..
   __device__ __forceinline__ bf16x8 row(uint32_t a, int rh, int ks) const {
-    return *reinterpret_cast<const NHA_LDS bf16x8*>(lds + ((a + row_at) ^ ((ks & 1) * 64)) + rh * HALF + (ks >> 1) * 1024);
+    return *reinterpret_cast<const NHA_LDS bf16x8*>(lds + (a + ra) + rh * HALF + ks * 1024);
   }
   // transposed fragment: X[4 kb + e][16 c + l16] (e < 4) and X[16 + 4 kb + e - 4][..]
   __device__ __forceinline__ bf16x8 col(uint32_t a, int c) const {
-    const lbyte* pa = lds + ((a + col_at) ^ ((c & 3) * 32)) + (c >> 2) * 1024;
+    const lbyte* pa = lds + ((a + ca) ^ ((c & 1) * 32)) + (c >> 1) * 1024;
     struct { s16x4 a, b; } t;
     t.a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)pa);
     t.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)(pa + HALF));

@@ -22,7 +22,7 @@ namespace {
 using namespace mf;
 
 constexpr int D = 256, KS = D / 32, DB = D / 16;
-constexpr int UB = 32 * D * 2;        // a 32-row tile (SwzTile)
+constexpr int UB = 32 * D * 2;        // a 32-row tile (LineTile)
 constexpr int ROWS = 128;             // rows (queries or keys) of a workgroup
 
 struct WinP {
@@ -40,16 +40,15 @@ struct WinP {
 
 // The workgroup's 128 rows of a [*, heads, D] tensor into LDS as four tiles of 32 rows from byte address `at` on, by all waves (eight
 // loads each): a wave's own fragments loaded from global memory are 16-byte pieces of 16 rows, the slowest pattern there is
-// (SwzTile), and came twice, for both waves of a pair.  Rows past the end repeat row `last`.
+// (LineTile), and came twice, for both waves of a pair.  Rows past the end repeat row `last`.
 __device__ __forceinline__ void load_rows(const bf16_t* src, int64_t stride, int first, int last, uint32_t at, int wave, int lane) {
-  const int rb = wave >> 2, cb = wave & 3;
-  const uint32_t col = SwzTile<D>::load_col(rb, cb, lane);
+  const uint32_t col = LineTile<D>::load_col(wave, lane);
 #pragma unroll
   for (int i = 0; i < ROWS / 16; ++i) {
-    int r = 16 * i + 8 * rb + (lane >> 3);
+    int r = 16 * i + LineTile<D>::load_row(lane);
     r = first + r < last ? r : last - first;
     g2l16(src + (int64_t)first * stride, ((uint32_t)r * (uint32_t)stride + col) * 2,
-          at + SwzTile<D>::block(rb, cb) + (i >> 1) * UB + (i & 1) * SwzTile<D>::HALF);
+          at + wave * 1024 + (i >> 1) * UB + (i & 1) * LineTile<D>::HALF);
   }
 }
 
@@ -85,15 +84,15 @@ __global__ __launch_bounds__(512, 1) void ring256_dq_kernel(const WinP p) {
   auto issue_unit = [&](int u) {
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));
-    const int rb = wave >> 2, cb = wave & 3;   // a wave loads the blocks (rb, cb) and (rb + 2, cb) of both tiles
-    const uint32_t dst = lds0 + (u & (DQ_NR - 1)) * DQ_UNIT + SwzTile<D>::block(rb, cb), pcol = SwzTile<D>::load_col(rb, cb, lane);
+    // a wave loads 32 columns of both tiles
+    const uint32_t dst = lds0 + (u & (DQ_NR - 1)) * DQ_UNIT + wave * 1024, pcol = LineTile<D>::load_col(wave, lane);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      int r = top - 32 * (u + 1) + 16 * i + 8 * rb + (lane >> 3);
+      int r = top - 32 * (u + 1) + 16 * i + LineTile<D>::load_row(lane);
       r = r < eos ? r : eos - 1;
       const uint32_t off = ((uint32_t)(r - bos) * (uint32_t)(H * D) + pcol) * 2;
-      g2l16(kbase, off, dst + i * SwzTile<D>::HALF);
-      g2l16(vbase, off, dst + UB + i * SwzTile<D>::HALF);
+      g2l16(kbase, off, dst + i * LineTile<D>::HALF);
+      g2l16(vbase, off, dst + UB + i * LineTile<D>::HALF);
     }
   };
   // q and do rows through the ring's slots: q where the first two units go, do where the next two go
@@ -115,7 +114,7 @@ __global__ __launch_bounds__(512, 1) void ring256_dq_kernel(const WinP p) {
   }
   bf16x8 qf[2][KS], df[2][KS];
   {
-    const SwzTile<D> rd(lds, lane);
+    const LineTile<D> rd(lds, lane);
     wait_vm<0>();
     lds_barrier();
 #pragma unroll
@@ -149,7 +148,7 @@ __global__ __launch_bounds__(512, 1) void ring256_dq_kernel(const WinP p) {
     const uint32_t base = (uint32_t)((t & (DQ_NR - 1)) * DQ_UNIT);
     int lc = threadIdx.x & 63;
     asm volatile("" : "+v"(lc));   // what follows from the lane's number is derived anew: there are no registers to keep it
-    const SwzTile<D> rd(lds, lc);
+    const LineTile<D> rd(lds, lc);
     const int l16 = lc & 15, kb = lc >> 4;
     lbyte* const ex = lds + DQ_EX + pair * 2048 + lc * 8;   // + 8192 (unit parity) + 1024 (half) + 512 (16-query block)
     f32x4 S[2], dP[2];
@@ -292,15 +291,14 @@ __global__ __launch_bounds__(512, 1) void ring256_dkv_kernel(const WinP p) {
     const int hq = h * NG + iw.g, q0 = c0 + 32 * iw.u;
     const bf16_t* const qbase = p.q + ((int64_t)bos * HQ + hq) * D;
     const bf16_t* const obase = p.dout + ((int64_t)bos * HQ + hq) * D;
-    const int rb = wave >> 2, cb = wave & 3;
-    const uint32_t dst = lds0 + islot * KV_ITEM + SwzTile<D>::block(rb, cb), pcol = SwzTile<D>::load_col(rb, cb, ln);
+    const uint32_t dst = lds0 + islot * KV_ITEM + wave * 1024, pcol = LineTile<D>::load_col(wave, ln);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      int r = q0 + 16 * i + 8 * rb + (ln >> 3);
+      int r = q0 + 16 * i + LineTile<D>::load_row(ln);
       r = r < eos ? r : eos - 1;
       const uint32_t off = ((uint32_t)(r - bos) * (uint32_t)(HQ * D) + pcol) * 2;
-      g2l16(qbase, off, dst + KV_Q + i * SwzTile<D>::HALF);
-      g2l16(obase, off, dst + KV_O + i * SwzTile<D>::HALF);
+      g2l16(qbase, off, dst + KV_Q + i * LineTile<D>::HALF);
+      g2l16(obase, off, dst + KV_O + i * LineTile<D>::HALF);
     }
     if (wave == 0) {
       int r = q0 + (ln >> 1);
@@ -316,7 +314,7 @@ __global__ __launch_bounds__(512, 1) void ring256_dkv_kernel(const WinP p) {
   load_rows(p.v + (int64_t)h * D, (int64_t)H * D, c0, eos - 1, lds0 + 4 * UB, wave, lane);
   bf16x8 own[2][KS];
   {
-    const SwzTile<D> rd(lds, lane);
+    const LineTile<D> rd(lds, lane);
     wait_vm<0>();
     lds_barrier();
 #pragma unroll
@@ -362,7 +360,7 @@ __global__ __launch_bounds__(512, 1) void ring256_dkv_kernel(const WinP p) {
     if (mine && !no_work(u)) {
       int lc = threadIdx.x & 63;
       asm volatile("" : "+v"(lc));
-      const SwzTile<D> rd(lds, lc);
+      const LineTile<D> rd(lds, lc);
       const int kb = lc >> 4;
       const uint32_t rt = base + (second ? KV_O : KV_Q), tt = base + (second ? KV_Q : KV_O);
       lbyte* const pb = lds + KV_P + (second ? (t + 1) & 1 : t & 1) * 16384 + pair * 4096 + lc * 16;

@@ -19,16 +19,11 @@
 //    comparisons and no rescaling of the accumulators.  A row whose window sum leaves that range
 //    (overflowed, or below 2^-100) is flagged for mfma_repair_kernel, which recomputes it exactly.
 //
-// LDS layouts (no padding, which a 1 KB wave load cannot produce; the 16-byte pieces of a wave load may
-// come from anywhere, so any order of pieces inside a 1 KB block is free): a 32-row unit is cut into
-// 16-row x 32-column blocks of 1 KB.  "K layout" (row fragments, ds_read_b128): the 16-byte piece c of
-// row r sits at 256 c + 16 r, which is exactly 16 x the number of the lane that reads it as its MFMA
-// operand, so a wave reads a block as 1 KB of consecutive bytes (with 64-byte rows and the piece index
-// XORed with (row / 4) % 4 a read took 12 LDS cycles instead of 4: SQ_LDS_BANK_CONFLICT 3.9e7 -> 5.1e6,
-// SQ_LDS_IDX_ACTIVE 1.12e8 -> 7.8e7 cycles per launch at the T = 8192 shape).  "V layout" (transposing
-// ds_read_b64_tr_b16, which takes 16 columns = 32 bytes of each of 16 rows per wave instruction): the
-// block is two planes of 16 rows x 32 bytes, columns 0..15 then columns 16..31, so that the 512 bytes
-// of one instruction are contiguous (with 64-byte rows: SQ_LDS_BANK_CONFLICT 9.8e7 -> 3.9e7).
+// LDS layout of units, queries and slot tiles: LineTile (mfma_common.h), 64 consecutive bytes of a row per four lanes of a load.
+// Bound: matrix and vector instructions of two waves per SIMD at long windows (51 % of the matrix rate, 40 % of the vector issue at
+// T = 16384, W = 2048), operands arriving with nothing else resident on the CU at short ones.  With K units, query and
+// k-state rows loaded in 16-byte pieces and V in 32-byte ones: 505 -> 497 us at B=2, T=8192, 32/8 heads, W=2048, 1090 -> 1079 at
+// T=16384, 172.5 -> 171.5 at W=64, 19.6 -> 18.2 at 331 tokens (32/4 heads).
 #include "mfma_common.h"
 
 #include <mutex>
@@ -51,18 +46,6 @@ __device__ __forceinline__ unsigned cvt2(float a, float b) {
   return __builtin_bit_cast(unsigned, t);
 }
 
-// 16 bytes per lane from global memory into registers, outside the compiler's memory model like the loads above: the
-// wait the compiler writes for a load of its own does not know of the LDS-direct requests behind it and waits for
-// all of them.  The value is there after wait_vm<N> with at most N younger requests pending; until then nothing may
-// read or move the register, so its first use is claim_reg, placed behind that wait and a scheduling fence (a copy
-// the register allocator makes for the claim then comes after the wait as well).
-__device__ __forceinline__ u32x4 gload16(const void* ptr) {
-  u32x4 x;
-  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(x) : "v"(ptr) : "memory");
-  return x;
-}
-__device__ __forceinline__ void claim_reg(u32x4& x) { asm volatile("" : "+v"(x)::"memory"); }
-
 template <int D>
 struct RingCfg {
   static constexpr int KS = D / 32;            // 32-column blocks per row == contraction steps of q.k
@@ -72,10 +55,11 @@ struct RingCfg {
   static constexpr int NR = 512 / D;           // ring slots (64 KB of K and V units together)
   static constexpr int LPW = KS / 2;           // LDS-direct loads per wave for a unit (K and V) or a 64-row tile
   static constexpr int RING_K = 0, RING_V = NR * UB;
-  static constexpr int TA = 2 * NR * UB;       // chunk-start k-state [m][d], K layout
-  static constexpr int TB = TA + 2 * UB;       // k_gsa rows, K layout
-  static constexpr int TC = TB + 2 * UB;       // chunk-start v-state [m][d], V layout
-  static constexpr int TD = TC + 2 * UB;       // v rows, V layout
+  static constexpr int TA = 2 * NR * UB;       // chunk-start k-state [m][d]
+  static constexpr int TB = TA + 2 * UB;       // k_gsa rows
+  static constexpr int TC = TB + 2 * UB;       // chunk-start v-state [m][d]
+  static constexpr int TD = TC + 2 * UB;       // v rows
+  static constexpr int QT = TA;                // first the window queries, 32 rows of each of the eight waves
   static constexpr int GC = TD + 2 * UB;       // gate cumsum fp32 [64][64], pieces XORed with row % 16
   static constexpr int SS = GC + 16384;        // s bf16 [64][64], pieces XORed with row % 8
   static constexpr int BYTES = SS + 8192;
@@ -126,10 +110,8 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   const int nunits = (c0 + 64 - lowest + 31) / 32;   // >= 2
 
   // ---- load descriptors of this wave: LDS-direct load i of a unit / a 64-row tile ------------------
-  // block index b = wave + 8 i; K layout: the lane's 16 bytes are piece lane / 16 of row lane % 16 of the block
-  const int lrow16 = lane & 15, lswz = lane >> 4;
-  // V layout: the lane's 16 bytes are piece lane % 2 of plane lane / 32, row (lane % 32) / 2
-  const int lrowv = (lane & 31) >> 1, lpv = 2 * (lane >> 5) + (lane & 1);
+  // block index b = wave + 8 i of a unit's K tile, then its V tile
+  const int lrow = LineTile<D>::load_row(lane);
   uint32_t u_off[LPW];          // byte offset from the unit's first row (token rows, stride H*D)
   uint32_t u_lds[LPW];          // LDS address of the block inside ring slot 0
   bool u_isv[LPW];
@@ -140,7 +122,7 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
     const int bb = isv ? b - 2 * KS : b;
     const int rh = bb / KS, cq = bb % KS;
     u_isv[i] = isv;
-    u_off[i] = ((uint32_t)(16 * rh + (isv ? lrowv : lrow16)) * (uint32_t)(H * D) + (uint32_t)(4 * cq + (isv ? lpv : lswz)) * 8) * 2;
+    u_off[i] = ((uint32_t)(16 * rh + lrow) * (uint32_t)(H * D) + LineTile<D>::load_col(cq, lane)) * 2;
     u_lds[i] = lds0 + (isv ? C::RING_V : C::RING_K) + rh * HB + cq * 1024;
   }
   // request unit u; rows past eos (units 0 and 1 only) are read from row eos - 1: always masked, always finite
@@ -153,23 +135,22 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
       const bool isv = b >= 2 * KS;
       const int bb = isv ? b - 2 * KS : b;
       const int rh = bb / KS, cq = bb % KS;
-      int row = key0 + 16 * rh + (isv ? lrowv : lrow16);
+      int row = key0 + 16 * rh + lrow;
       row = row < eos ? row : eos - 1;
-      const uint32_t off = ((uint32_t)(row - bos) * (uint32_t)(H * D) + (uint32_t)(4 * cq + (isv ? lpv : lswz)) * 8) * 2;
+      const uint32_t off = ((uint32_t)(row - bos) * (uint32_t)(H * D) + LineTile<D>::load_col(cq, lane)) * 2;
       const bf16_t* base = (isv ? p.v : p.k_swa) + ((int64_t)bos * H + h) * D;
       g2l16(base, off, u_lds[i] + slot * UB);
     }
   };
-  // 64-row tile of the slot branch: kind 0 = K layout, 1 = V layout; rows of `src` with `stride` elements,
-  // row r of the tile is global row rowmap(r)
-  auto issue_tile = [&](int lds_tile, bool vlay, const bf16_t* src, uint32_t stride, auto rowmap) {
+  // 64-row tile of the slot branch; rows of `src` with `stride` elements, row r of the tile is global row rowmap(r)
+  auto issue_tile = [&](int lds_tile, const bf16_t* src, uint32_t stride, auto rowmap) {
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
       const int b = wave + 8 * i;            // < 4 KS
       const int unit = b / (2 * KS), bb = b % (2 * KS);
       const int rh = bb / KS, cq = bb % KS;
-      const int r = 32 * unit + 16 * rh + (vlay ? lrowv : lrow16);
-      const uint32_t off = ((uint32_t)rowmap(r) * stride + (uint32_t)(4 * cq + (vlay ? lpv : lswz)) * 8) * 2;
+      const int r = 32 * unit + 16 * rh + lrow;
+      const uint32_t off = ((uint32_t)rowmap(r) * stride + LineTile<D>::load_col(cq, lane)) * 2;
       g2l16(src, off, lds0 + lds_tile + unit * UB + rh * HB + cq * 1024);
     }
   };
@@ -177,14 +158,15 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   // ---- requests, in the order of their first use: the query fragments and unit 0 (first scores), then the other
   //      first units.  A CU serves the loads of its waves in the order they were issued: the barrier keeps the
   //      other units of the early waves from queueing in front of the last wave's queries and unit 0 ----
-  u32x4 qraw[RQB][KS];
+  // the wave's 32 query rows, whole lines into the room of the slot operands (which are requested once they have been read);
+  // rows past the end of the sequence read its last row and are zeroed afterwards
+  const uint32_t qtile = (uint32_t)(C::QT + wave * UB);
 #pragma unroll
-  for (int qb = 0; qb < RQB; ++qb) {
-    // rows past the end of the sequence read its last row (the waits below count the loads) and are zeroed afterwards
-    const int irow = 16 * (qb0 + qb) + l16;
-    const bf16_t* qp = p.q_swa + ((int64_t)(c0 + (irow < rows ? irow : rows - 1)) * HQ + hq) * D + 8 * kb;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qraw[qb][ks] = gload16(qp + 32 * ks);
+  for (int i = 0; i < RQB * KS; ++i) {
+    int r = 16 * (qb0 + i / KS) + lrow;
+    r = r < rows ? r : rows - 1;
+    g2l16(p.q_swa + ((int64_t)c0 * HQ + hq) * D, ((uint32_t)r * (uint32_t)(HQ * D) + LineTile<D>::load_col(i % KS, lane)) * 2,
+          lds0 + qtile + LineTile<D>::block(i / KS, i % KS));
   }
   issue_unit_checked(0);
   __builtin_amdgcn_s_barrier();
@@ -201,6 +183,7 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   }
   NHA_FENCE();
 
+  const uint32_t kaddr = LineTile<D>::row_at(lane), vaddr = LineTile<D>::col_at(lane);
   // window-query fragments, pre-scaled by scale * log2(e): scores come out of the matrix core in the
   // units the exponential wants
   bf16x8 qs[RQB][KS];
@@ -209,8 +192,8 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
     const int irow = 16 * (qb0 + qb) + l16;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      claim_reg(qraw[qb][ks]);
-      const u32x4 x = irow < rows ? qraw[qb][ks] : (u32x4){0u, 0u, 0u, 0u};
+      u32x4 x = *reinterpret_cast<const NHA_LDS u32x4*>(lds + qtile + kaddr + qb * HB + ks * 1024);
+      if (irow >= rows) x = (u32x4){0u, 0u, 0u, 0u};
       const uint32_t w[4] = {x[0], x[1], x[2], x[3]};
       bf16x8 r;
 #pragma unroll
@@ -247,10 +230,10 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
       const int c = (lane & 7) ^ (r & 7);
       g2l16(p.s + ((int64_t)bos * H + h) * MS, ((uint32_t)tok(r) * (uint32_t)(H * MS) + (uint32_t)c * 8) * 2, lds0 + C::SS + wave * 1024);
     }
-    issue_tile(C::TA, false, p.hkT + cg * MS * D, (uint32_t)D, ident);
-    issue_tile(C::TB, false, p.k_gsa + ((int64_t)bos * H + h) * D, (uint32_t)(H * D), tok);
-    issue_tile(C::TC, true, p.hvc + cg * MS * D, (uint32_t)D, ident);
-    issue_tile(C::TD, true, p.v + ((int64_t)bos * H + h) * D, (uint32_t)(H * D), tok);
+    issue_tile(C::TA, p.hkT + cg * MS * D, (uint32_t)D, ident);
+    issue_tile(C::TB, p.k_gsa + ((int64_t)bos * H + h) * D, (uint32_t)(H * D), tok);
+    issue_tile(C::TC, p.hvc + cg * MS * D, (uint32_t)D, ident);
+    issue_tile(C::TD, p.v + ((int64_t)bos * H + h) * D, (uint32_t)(H * D), tok);
   };
 
   // ---- window loop state ------------------------------------------------------------------------
@@ -274,15 +257,13 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   // the reference is taken from unit 0 when a score there exceeds 2^THR, and kept from then on
   constexpr float THR = 8.f;
 
-  const uint32_t kaddr = (uint32_t)(lane * 16);
-  const uint32_t vaddr = (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
-  // row fragment (rows 16 kk + l16 of a unit, columns 32 ks + 8 kb ..) of a K-layout unit at byte address a
+  // row fragment (rows 16 kk + l16 of a unit, columns 32 ks + 8 kb ..) of a tile at byte address a - kaddr
   auto kfrag = [&](uint32_t a, int kk, int ks) -> bf16x8 {
     return *reinterpret_cast<const NHA_LDS bf16x8*>(lds + a + kk * HB + ks * 1024);
   };
-  // transposed fragment of a V-layout unit: X[4 kb + e][16 db + l16] (e < 4) and X[16 + 4 kb + e - 4][..]
+  // transposed fragment of a tile at byte address a - vaddr: X[4 kb + e][16 db + l16] (e < 4) and X[16 + 4 kb + e - 4][..]
   auto vfrag = [&](uint32_t a, int db) -> bf16x8 {
-    const lbyte* pa = lds + a + (db >> 1) * 1024 + (db & 1) * 512;
+    const lbyte* pa = lds + (a ^ ((db & 1) * 32)) + (db >> 1) * 1024;
     struct { s16x4 a, b; } t;
     t.a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)pa);
     t.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)(pa + HB));
@@ -535,7 +516,8 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   // blocks jb <= Q, zero elsewhere: query sub-block Q (16 rows) references the gate cumsum gr_Q of the
   // row before it (0 for Q = 0), so the exponent is <= 0 for rows of earlier blocks and bounded by the
   // block's own decay on the diagonal.  Rows whose source token does not exist (before the sequence,
-  // past its end) carry no weight.  Stored as 32-row units in the V layout (64 columns): the logit
+  // past its end) carry no weight.  Stored as 32-row units (64 columns) in blocks of 16 rows x 32
+  // columns, two planes of 32-byte rows each: the logit
   // update reads them transposed (rows = slots), the slot-read weights row by row (rows = tokens).
   // Units: E_0 -> 0, E_1 -> 1, E_2 -> 2,3, E_3 -> 4,5; a thread makes 8 consecutive slots of a row.
   for (int item = tid; item < 6 * 256; item += 512) {
@@ -581,9 +563,10 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   wait_vm<0>();   // the four tiles
   __syncthreads();
 
+  const uint32_t taddr = (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
   // E_Q transposed: rows = slots 16 mb + l16, contraction over the tokens 32 pr + {4 kb + e, 16 + 4 kb + e - 4}
   auto etab_tr = [&](int Q, int pr, int mb) -> bf16x8 {
-    const lbyte* pa = lds + C::ETAB + ((Q < 2 ? Q : 2 * Q - 2) + pr) * 4096 + (mb >> 1) * 1024 + (mb & 1) * 512 + vaddr;
+    const lbyte* pa = lds + C::ETAB + ((Q < 2 ? Q : 2 * Q - 2) + pr) * 4096 + (mb >> 1) * 1024 + (mb & 1) * 512 + taddr;
     struct { s16x4 a, b; } t;
     t.a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)pa);
     t.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)(pa + 2048));
@@ -777,7 +760,7 @@ int launch_ring(const MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   // the window-only launch has no slot operands: the ring is all the LDS it uses
-  const size_t lds = SINK ? (size_t)RingCfg<D>::TA : (size_t)RingCfg<D>::BYTES;
+  const size_t lds = SINK ? (size_t)(RingCfg<D>::QT + 8 * RingCfg<D>::UB) : (size_t)RingCfg<D>::BYTES;   // the window queries end where the tiles do
   std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring_out_kernel<D, SINK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));

@@ -64,9 +64,7 @@ struct Cfg {
   static constexpr int BYTES = GC2 + (NCH - 1) * 16384;
 };
 
-// LDS layouts as in prefill_ring.hip: a 32-row buffer is cut into 16-row x 32-column blocks of 1 KB
-// (half h, column block c at h * HB + c * 1024).  K layout: 16-byte piece c of row r at 256 c + 16 r (a wave's
-// row fragments are 1 KB of consecutive bytes).  V layout: two planes of 16 rows x 32 bytes (columns 0..15, then 16..31).
+// LDS layout of a 32-row buffer: LineTile.
 template <int NCH>
 __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   using C = Cfg<NCH>;
@@ -109,16 +107,15 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   const int nunits = (c0 + BT * NCH - lowest + 31) / 32;   // >= 2 NCH
 
   // ---- LDS-direct loads: block b = wave + NW i of a buffer; per lane a row of the block and a 16-byte piece
-  const int lrow16 = lane & 15, lswz = lane >> 4;          // K layout
-  const int lrowv = (lane & 31) >> 1, lpv = 2 * (lane >> 5) + (lane & 1);         // V layout
+  const int lrow = LineTile<D>::load_row(lane);
   // one 32-row buffer from rows of `src` (row stride in elements): row r of the buffer is global row rowmap(r)
-  auto issue_buffer = [&](uint32_t lds_buf, bool vlay, const bf16_t* src, uint32_t stride, auto rowmap) {
+  auto issue_buffer = [&](uint32_t lds_buf, const bf16_t* src, uint32_t stride, auto rowmap) {
 #pragma unroll
     for (int i = 0; i < LPB; ++i) {
       const int b = wave + NW * i;           // < 16
       const int rh = b / KS, cq = b % KS;
-      const int r = 16 * rh + (vlay ? lrowv : lrow16);
-      const uint32_t off = ((uint32_t)rowmap(r) * stride + (uint32_t)(4 * cq + (vlay ? lpv : lswz)) * 8) * 2;
+      const int r = 16 * rh + lrow;
+      const uint32_t off = ((uint32_t)rowmap(r) * stride + LineTile<D>::load_col(cq, lane)) * 2;
       g2l16(src, off, lds0 + lds_buf + rh * HB + cq * 1024);
     }
   };
@@ -130,35 +127,34 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     const int last = eos - 1 - bos;
     return [=](int r) { return key0 + r < last ? key0 + r : last; };
   };
-  auto issue_k = [&](int u) { issue_buffer(C::RING_K + (u % NR) * UB, false, kbase, (uint32_t)(H * D), unit_row(u)); };
-  auto issue_v = [&](int u) { issue_buffer(C::RING_V + (u % NR) * UB, true, vbase, (uint32_t)(H * D), unit_row(u)); };
+  auto issue_k = [&](int u) { issue_buffer(C::RING_K + (u % NR) * UB, kbase, (uint32_t)(H * D), unit_row(u)); };
+  auto issue_v = [&](int u) { issue_buffer(C::RING_V + (u % NR) * UB, vbase, (uint32_t)(H * D), unit_row(u)); };
   // units >= 2 NCH lie wholly before the workgroup's rows (never past eos): fixed per-lane offsets from a wave-uniform row pointer
-  uint32_t koff[LPB], voff[LPB], boff[LPB];
+  uint32_t uoff[LPB], boff[LPB];
 #pragma unroll
   for (int i = 0; i < LPB; ++i) {
     const int b = wave + NW * i;
     const int rh = b / KS, cq = b % KS;
-    koff[i] = ((uint32_t)(16 * rh + lrow16) * (uint32_t)(H * D) + (uint32_t)(4 * cq + lswz) * 8) * 2;
-    voff[i] = ((uint32_t)(16 * rh + lrowv) * (uint32_t)(H * D) + (uint32_t)(4 * cq + lpv) * 8) * 2;
+    uoff[i] = ((uint32_t)(16 * rh + lrow) * (uint32_t)(H * D) + LineTile<D>::load_col(cq, lane)) * 2;
     boff[i] = lds0 + rh * HB + cq * 1024;
   }
   auto issue_k_fast = [&](int u, uint32_t slot_off) {
     if (NCH > 1 && u < 2 * NCH) {
-      issue_buffer(C::RING_K + slot_off, false, kbase, (uint32_t)(H * D), unit_row(u));
+      issue_buffer(C::RING_K + slot_off, kbase, (uint32_t)(H * D), unit_row(u));
       return;
     }
     const bf16_t* src = p.k_swa + (((int64_t)c0 + XB0 - 32 * u) * H + h) * D;
 #pragma unroll
-    for (int i = 0; i < LPB; ++i) g2l16(src, koff[i], boff[i] + C::RING_K + slot_off);
+    for (int i = 0; i < LPB; ++i) g2l16(src, uoff[i], boff[i] + C::RING_K + slot_off);
   };
   auto issue_v_fast = [&](int u, uint32_t slot_off) {
     if (NCH > 1 && u < 2 * NCH) {
-      issue_buffer(C::RING_V + slot_off, true, vbase, (uint32_t)(H * D), unit_row(u));
+      issue_buffer(C::RING_V + slot_off, vbase, (uint32_t)(H * D), unit_row(u));
       return;
     }
     const bf16_t* src = p.v + (((int64_t)c0 + XB0 - 32 * u) * H + h) * D;
 #pragma unroll
-    for (int i = 0; i < LPB; ++i) g2l16(src, voff[i], boff[i] + C::RING_V + slot_off);
+    for (int i = 0; i < LPB; ++i) g2l16(src, uoff[i], boff[i] + C::RING_V + slot_off);
   };
 
   // The slot branch runs chunk by chunk (its tables and tiles are one chunk's): cc is the chunk it is at, and these
@@ -200,7 +196,8 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   auto s_at = [&](int j, int m) -> const lbf16* { return (const lbf16*)(lds + C::SS + j * 128 + (((m >> 3) ^ (j & 7)) * 16) + (m & 7) * 2); };
   // decay tables E_Q[j][m] = s_j[m] exp(min(gr_Q[m] - gc_j[m], DECAY_CLAMP)) for the rows j of the 16-row
   // blocks jb <= Q, zero elsewhere (gr_Q: gate cumsum of the row before sub-block Q, 0 for Q = 0); rows
-  // whose source token does not exist carry no weight.  32-row units in the V layout (64 columns):
+  // whose source token does not exist carry no weight.  32-row units (64 columns) in blocks of 16 rows x 32
+  // columns, two planes of 32-byte rows each, which is what the transposing read takes:
   // E_0 -> unit 0, E_1 -> 1, E_2 -> 2,3, E_3 -> 4,5; a thread makes 8 consecutive slots of a row.
   auto build_decay_tables = [&]() {
     for (int item = tid; item < 6 * 256; item += 64 * NW) {
@@ -285,17 +282,16 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   constexpr float THR = 8.f;           // the reference moves (prologue, slot branch) when a score tops it by more than 2^THR
   constexpr float BIG = 96.f;          // scores this far above the reference leave the matrix-core path
 
-  const uint32_t kaddr = (uint32_t)(lane * 16);
-  const uint32_t vaddr = (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
-  // row fragment (rows 16 kk + l16 of a buffer, columns 32 ks + 8 kb ..) of a K-layout buffer at byte address a
+  const uint32_t kaddr = LineTile<D>::row_at(lane), vaddr = LineTile<D>::col_at(lane);
+  // row fragment (rows 16 kk + l16 of a buffer, columns 32 ks + 8 kb ..) of a buffer at byte address a
   auto kfrag = [&](uint32_t a, int kk, int ks) -> bf16x8 {
     const lbyte* base = lds + (a + kaddr);     // one address per buffer; the fragment is a constant offset from it
     return *reinterpret_cast<const NHA_LDS bf16x8*>(base + (kk * HB + ks * 1024));
   };
-  // transposed fragment of a V-layout buffer: X[4 kb + e][16 db + l16] (e < 4) and X[16 + 4 kb + e - 4][..]
+  // transposed fragment of a buffer: X[4 kb + e][16 db + l16] (e < 4) and X[16 + 4 kb + e - 4][..]
   auto vfrag = [&](uint32_t a, int db) -> bf16x8 {
-    const lbyte* base = lds + (a + vaddr);
-    const lbyte* pa = base + ((db >> 1) * 1024 + (db & 1) * 512);
+    const lbyte* base = lds + ((a + vaddr) ^ ((db & 1) * 32));   // two addresses per buffer
+    const lbyte* pa = base + (db >> 1) * 1024;
     struct { s16x4 a, b; } t;
     t.a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)pa);
     t.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)(pa + HB));
@@ -391,9 +387,9 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   // unit buffer, so the in-flight counts of the loop stay what they are); the two v-state halves follow
   // after the loop, and shorter windows request everything then.
   const bf16_t* const t_kg = p.k_gsa + ((int64_t)bos * H + h) * D;
-  auto issue_ta = [&](uint32_t off, int half) { issue_buffer(off, false, p.hkT + (cg + (int64_t)cc * H) * MS * D, (uint32_t)D, [=](int r) { return 32 * half + r; }); };
-  auto issue_tb = [&](uint32_t off, int half) { issue_buffer(off, false, t_kg, (uint32_t)(H * D), [&](int r) { return tok(32 * half + r); }); };
-  auto issue_tc = [&](uint32_t off, int half) { issue_buffer(off, true, p.hvc + (cg + (int64_t)cc * H) * MS * D, (uint32_t)D, [=](int r) { return 32 * half + r; }); };
+  auto issue_ta = [&](uint32_t off, int half) { issue_buffer(off, p.hkT + (cg + (int64_t)cc * H) * MS * D, (uint32_t)D, [=](int r) { return 32 * half + r; }); };
+  auto issue_tb = [&](uint32_t off, int half) { issue_buffer(off, t_kg, (uint32_t)(H * D), [&](int r) { return tok(32 * half + r); }); };
+  auto issue_tc = [&](uint32_t off, int half) { issue_buffer(off, p.hvc + (cg + (int64_t)cc * H) * MS * D, (uint32_t)D, [=](int r) { return 32 * half + r; }); };
   const bool early = nunits >= 5;
   uint32_t oA0 = C::RING_K, oA1 = C::RING_K + UB, oB0 = C::RING_K + 2 * UB, oB1 = C::RING_V;   // where the halves lie
   uint32_t oC0 = C::RING_V + UB, oC1 = C::RING_V + 2 * UB;
@@ -568,7 +564,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     const int etu = Q < 2 ? Q : 2 * Q - 2;   // first table unit of this wave's sub-block
     // E_Q transposed: rows = slots 16 mb + l16, contraction over the tokens 32 pr + {4 kb + e, 16 + 4 kb + e - 4}
     auto etab_tr = [&](int pr, int mb) -> bf16x8 {
-      const lbyte* pa = lds + C::ETAB + (etu + pr) * 4096 + (mb >> 1) * 1024 + (mb & 1) * 512 + vaddr;
+      const lbyte* pa = lds + C::ETAB + (etu + pr) * 4096 + (mb >> 1) * 1024 + (mb & 1) * 512 + (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
       struct { s16x4 a, b; } t;
       t.a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)pa);
       t.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)(pa + 2048));
@@ -597,7 +593,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     lds_barrier();
 #pragma unroll
     for (int half = 0; half < 2; ++half)
-      issue_buffer(half ? oA1 : oA0, true, vbase, (uint32_t)(H * D), [&](int r) { return tok(32 * half + r); });
+      issue_buffer(half ? oA1 : oA0, vbase, (uint32_t)(H * D), [&](int r) { return tok(32 * half + r); });
     bf16x8 bp[2], bpr[2];   // slot probabilities x exp(gc_i) and x exp(gc_i - gr), B operands
     if (mine) {
       // intra-chunk scores AT[j][i] = sum_d k_gsa[j][d] q[i][d] for row blocks jb <= Q, masked j <= i
@@ -690,7 +686,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     if (ahead) {
 #pragma unroll
       for (int half = 0; half < 2; ++half)
-        issue_buffer(half ? oB1 : oB0, false, t_kg, (uint32_t)(H * D), [&](int r) { return tok_from(c0 + BT - p.shift, 32 * half + r); });
+        issue_buffer(half ? oB1 : oB0, t_kg, (uint32_t)(H * D), [&](int r) { return tok_from(c0 + BT - p.shift, 32 * half + r); });
     }
     bf16x8 bAv[2];
     if (mine) {
