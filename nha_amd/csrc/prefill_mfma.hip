@@ -191,40 +191,29 @@ __global__ __launch_bounds__(256) void mfma_state_local_kernel(const MP p) {
     float gcv[16], sg[16];
     const bf16x8 gq01 = lds_frag_tr(Gt, SLD, 0, 16, 16 * wave, lane), gq23 = lds_frag_tr(Gt, SLD, 32, 48, 16 * wave, lane);
     const bf16x8 sq01 = lds_frag_tr(St, SLD, 0, 16, 16 * wave, lane), sq23 = lds_frag_tr(St, SLD, 32, 48, 16 * wave, lane);
-    {
-      float run[4], base = 0.f;
+    // the chunk's last cumsum: rows without a source token and past the end have gate 0, so it is the sum of all
+    float glast = 0.f;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float a = 0.f;
+    for (int q = 0; q < 4; ++q) {
+      float a = 0.f;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          a += (float)(q < 2 ? gq01[4 * q + r] : gq23[4 * (q - 2) + r]);
-          gcv[4 * q + r] = a;
-        }
-        run[q] = a;
+      for (int r = 0; r < 4; ++r) {
+        a += (float)(q < 2 ? gq01[4 * q + r] : gq23[4 * (q - 2) + r]);
+        gcv[4 * q + r] = a;
+      }
+      // the sums of the four 16-lane rows, for every lane (lane swaps: sixteen LDS permutes took 1.3k of a chunk's 7.7k cycles)
+      const unsigned u = __float_as_uint(a);
+      const auto x = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+      const auto y0 = __builtin_amdgcn_permlane32_swap(x[0], x[0], false, false), y1 = __builtin_amdgcn_permlane32_swap(x[1], x[1], false, false);
+      const float row[4] = {__uint_as_float(y0[0]), __uint_as_float(y1[0]), __uint_as_float(y0[1]), __uint_as_float(y1[1])};
+      float off = glast;
+#pragma unroll
+      for (int k2 = 0; k2 < 4; ++k2) {
+        if (k2 < kb) off += row[k2];
+        glast += row[k2];
       }
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float off = base;
-#pragma unroll
-        for (int k2 = 0; k2 < 4; ++k2) {
-          const float a = __shfl(run[q], l16 + 16 * k2, 64);
-          base += a;
-          if (k2 < kb) off += a;
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) gcv[4 * q + r] += off;
-      }
-    }
-    float glast;
-    {
-      const int tl = rows - 1;
-      const int src_kb = (tl & 15) >> 2, e = 4 * (tl >> 4) + (tl & 3);
-      float cand = 0.f;
-#pragma unroll
-      for (int x = 0; x < 16; ++x)
-        if (x == e) cand = gcv[x];
-      glast = __shfl(cand, l16 + 16 * src_kb, 64);
+      for (int r = 0; r < 4; ++r) gcv[4 * q + r] += off;
     }
     const int64_t cg = (int64_t)chunk * H + h;
     if (lead) {
