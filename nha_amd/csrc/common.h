@@ -163,8 +163,9 @@ bool prefill_mfma_supported(const NhaPrefillArgs* a);
 size_t prefill_mfma_scratch_bytes(const NhaPrefillArgs* a);
 size_t prefill_mfma_least_scratch_bytes(const NhaPrefillArgs* a);
 int prefill_mfma_impl(const NhaPrefillArgs* a, int phase);
-int bwd_slot_inter_slabs(const NhaPrefillBwdArgs* a);
-int bwd_slot_inter(const NhaPrefillBwdArgs* a, const float* gc, const float* ek, const float* ev, const float* dks, float* dvs, float* dsp);
+// prefill_bwd_mfma.hip: the parts of dk_gsa, dv and ds that involve the carried state gradient, and the chunks' gate sums
+int bwd_slot_inter(const NhaPrefillBwdArgs* a, const float* gc, const float* ek, const float* ev, const float* dks, float* dvs, const float* xg,
+                   float* dsi, float* gtot);
 bool prefill_bwd_supported(const NhaPrefillBwdArgs* a);
 size_t prefill_bwd_scratch_bytes(const NhaPrefillBwdArgs* a);
 size_t prefill_bwd_least_scratch_bytes(const NhaPrefillBwdArgs* a);

@@ -966,8 +966,8 @@ BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f, size_t fwd
   BwdPlan s = {};
   // bf16 shapes the matrix-core state pass covers
   s.use_mfma = prefill_mfma_supported(&f);
-  s.nbk = s.use_mfma ? bwd_slot_inter_slabs(a) : (a->K + CB - 1) / CB;
-  s.nbv = s.use_mfma ? bwd_slot_inter_slabs(a) : (a->V + CB - 1) / CB;
+  s.nbk = s.use_mfma ? 0 : (a->K + CB - 1) / CB;   // (the matrix-core path keeps these sums on the chip)
+  s.nbv = s.use_mfma ? 0 : (a->V + CB - 1) / CB;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
@@ -1112,13 +1112,13 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
   }
   hipLaunchKernelGGL(bwd_state_scan_kernel, dim3(a->N * a->H, ((K + V) * M + 255) / 256), dim3(256), 0, st, p);
   if (sp.use_mfma) {
-    rc = bwd_slot_inter(a, states.gc, p.ek, p.ev, p.dks, p.dvs, p.dsp);
+    rc = bwd_slot_inter(a, states.gc, p.ek, p.ev, p.dks, p.dvs, p.xg, p.dsi, p.gtot);
     if (rc != NHA_OK) return rc;
   } else {
     hipLaunchKernelGGL((bwd_state_inter_kernel<T>), dim3(a->NT, a->H * nbmax, 2), dim3(256), lds_s3, st, p);
+    hipLaunchKernelGGL((bwd_gate_local_kernel<T>), dim3(a->NT, a->H), dim3(256), 0, st, p);
   }
   NHA_CHECK_LAUNCH("nha_prefill_bwd(state gradients)");
-  hipLaunchKernelGGL((bwd_gate_local_kernel<T>), dim3(a->NT, a->H), dim3(256), 0, st, p);
   hipLaunchKernelGGL((bwd_gate_scan_kernel<T>), dim3(a->N * a->H), dim3(64), 0, st, p);
   hipLaunchKernelGGL((bwd_gate_final_kernel<T>), dim3(a->NT, a->H), dim3(256), 0, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(gate scan)");

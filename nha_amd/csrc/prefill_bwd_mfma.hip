@@ -433,9 +433,10 @@ struct SP2 {
   const float *ek, *ev;              // [NT][H][D][64] x2
   const float* dks;                  // [T][H][D] intra-chunk part of dk_gsa (source-token index)
   float* dvs;                        // the same of the slot-branch dv; completed here
-  float* dsp;                        // [2 * slabs][T][H][64] inter-chunk part of ds per state and column range
+  const float* xg;                   // [T][H][64] first part of the dg summand
+  float *dsi, *gtot;                 // [T][H][64] intra-chunk part of ds, then the chunk's reverse cumulative sums; [NT][H][64] their totals
+  bf16_t* ds;                        // [T,H,64]
   bf16_t* dkg;                       // dk_gsa [T,H,D]
-  int T_tot;
   const int32_t *cu, *cidx;
   int H, shift;
 };
@@ -455,17 +456,21 @@ __device__ __forceinline__ void split4_bf16(const float4 x, lbf16* hi, lbf16* lo
   *reinterpret_cast<NHA_LDS bf16x4*>(lo + idx) = l;
 }
 
-// bwd_slot_inter_kernel, grid (H, NT, 2 D / DW): the parts that involve E_c, the state gradient carried
+// bwd_slot_inter_kernel, grid (H, NT): the parts that involve E_c, the state gradient carried
 // into the END of chunk c (z even: k-state, rows k', output dk_gsa; z odd: v-state, rows v', output
 // dvs), with dec_r[m] = e^(gl[m] - gc_r[m]):
 //   out[r][x] = intra part + sum_m (s_r[m] dec_r[m]) E[x][m]         as out^T = E sE^T
-//   dsp[r][m] = dec_r[m] sum_x y_r[x] E[x][m]                         as Y E
-// A workgroup takes DW of the D columns x (z / 2 picks them): at head size 256 two workgroups of half the
-// columns fit a CU where one of all columns does not, and each writes its own partial of dsp (one slab per
-// state and column range; the gate kernel adds the slabs).
+//   ds[r][m] += dec_r[m] sum_x y_r[x] E[x][m]                         as Y E
+// z / 2 picks DW of the D columns x: at head size 256 a part of half the columns leaves room for two workgroups on a CU.
+// A workgroup takes the parts of its chunk one after the other (the next one's operands requested during the products), keeps
+// their sums for ds, and goes on with the gates: ds complete, and the chunk's reverse cumulative sums of the dg summand
+// xg - s ds with their total.  Bound: HBM.  With a workgroup per part, the sums handed on through memory and the gates in a
+// launch of their own: B=2, T=8192, 32/8 heads of 128 98 + 31 -> 93 us; B=8, T=2048, 4 heads of 256 119 + 28 -> 98; 5003 packed
+// tokens, 16 heads of 64 44 + 22 -> 44; 300 tokens, 4 heads of 256 (20 workgroups in place of 80) 20.5 -> 19.6 together.
 template <int D, int DW>
-__global__ __launch_bounds__(256) void bwd_slot_inter_kernel(const SP2 p) {
-  constexpr int DB = DW / 16, LDT = DW + 16, TILE = BT * LDT, ELD = TLD, NH = D / DW;
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void bwd_slot_inter_kernel(const SP2 p) {
+  constexpr int DB = DW / 16, LDT = DW + 16, TILE = BT * LDT, ELD = TLD, NH = D / DW, NZ = 2 * NH;
+  constexpr int NY = BT * DW / 8 / 256, NE = DW * BT / 4 / 256, NS = BT * BT / 4 / 256;
   extern __shared__ __align__(16) unsigned char smem[];
   lbf16* const Yt = (lbf16*)smem;        // [64 rows r][DW]  k' / v'
   lbf16* const Et = Yt + TILE;           // [DW x][ELD]      E[x][m], high part
@@ -476,59 +481,65 @@ __global__ __launch_bounds__(256) void bwd_slot_inter_kernel(const SP2 p) {
   const int l16 = lane & 15, kb = lane >> 4;
   const int H = p.H;
   const int h = blockIdx.x, chunk = blockIdx.y;
-  const bool isv = (blockIdx.z & 1) != 0;
-  const int xh = blockIdx.z >> 1, x0 = xh * DW;   // this workgroup's columns
   const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int c0 = bos + it * BT;
   const int R = (eos - c0) < BT ? (eos - c0) : BT;
-  const bf16_t* ysrc = isv ? p.v : p.kg;
   int vlo = p.shift - it * BT;
   vlo = vlo < 0 ? 0 : vlo;
-  Tile<BT, DW> ry;
+  const float* const gcb = p.gc + ((int64_t)chunk * H + h) * BT * BT;
+  struct Part {
+    uint4 y[NY];
+    float4 e[NE];
+  };
+  auto request = [&](Part& t, int z) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // addresses derived anew for every part: there are no registers to keep them
+    const bool isv = (z & 1) != 0;
+    const int x0 = (z >> 1) * DW;
+    const bf16_t* const ysrc = isv ? p.v : p.kg;
 #pragma unroll
-  for (int u = 0; u < Tile<BT, DW>::NPC; ++u) {
-    const int c = tid + 256 * u;
-    const int row = c / (DW / 8), cc = (c % (DW / 8)) * 8;
-    uint4 x = make_uint4(0, 0, 0, 0);
-    if (row >= vlo && row < R) x = *reinterpret_cast<const uint4*>(ysrc + (((int64_t)c0 + row - p.shift) * H + h) * D + x0 + cc);
-    ry.r[u] = x;
-  }
-  const float* ep = (isv ? p.ev : p.ek) + (((int64_t)chunk * H + h) * D + x0) * BT;
-  const float* gcb = p.gc + ((int64_t)chunk * H + h) * BT * BT;
+    for (int u = 0; u < NY; ++u) {
+      const int c = tid + 256 * u;
+      const int row = c / (DW / 8), cc = (c % (DW / 8)) * 8;
+      t.y[u] = make_uint4(0, 0, 0, 0);
+      if (row >= vlo && row < R) t.y[u] = *reinterpret_cast<const uint4*>(ysrc + (((int64_t)c0 + row - p.shift) * H + h) * D + x0 + cc);
+    }
+    const float4* const ep4 = reinterpret_cast<const float4*>((isv ? p.ev : p.ek) + (((int64_t)chunk * H + h) * D + x0) * BT);
+#pragma unroll
+    for (int u = 0; u < NE; ++u) t.e[u] = ep4[tid + 256 * u];
+  };
+  auto place = [&](const Part& t) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+#pragma unroll
+    for (int u = 0; u < NY; ++u) {
+      const int c = tid + 256 * u;
+      lds_st16(Yt + c / (DW / 8) * LDT + (c % (DW / 8)) * 8, t.y[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < NE; ++u) {
+      const int e = 4 * (tid + 256 * u);
+      split4_bf16(t.e[u], Et, El, (e >> 6) * ELD + (e & 63));
+    }
+  };
+  Part part;
+  request(part, 0);
   {
-    // all global loads of a batch are issued before the first conversion waits for one; the first batch
-    // of E and the gate rows are requested before the Y tile is stored
-    constexpr int NE = DW * BT / 4 / 256, EB = NE < 8 ? NE : 8;
-    const float4* ep4 = reinterpret_cast<const float4*>(ep);
-    constexpr int NS = BT * BT / 4 / 256;
     float4 gl[NS], gr[NS];
     uint2 sr[NS];
 #pragma unroll
-    for (int b0 = 0; b0 < NE; b0 += EB) {
-      float4 buf[EB];
-#pragma unroll
-      for (int u = 0; u < EB; ++u) buf[u] = ep4[tid + 256 * (b0 + u)];
-      if (b0 == 0) {
-#pragma unroll
-        for (int u = 0; u < NS; ++u) {
-          const int e = 4 * (tid + 256 * u), r = e >> 6, m = e & 63;
-          gl[u] = gr[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-          sr[u] = make_uint2(0, 0);
-          if (r >= vlo && r < R) {
-            sr[u] = *reinterpret_cast<const uint2*>(p.s + (((int64_t)c0 + r - p.shift) * H + h) * BT + m);
-            gl[u] = *reinterpret_cast<const float4*>(gcb + (BT - 1) * BT + m);
-            gr[u] = *reinterpret_cast<const float4*>(gcb + r * BT + m);
-          }
-        }
-        ry.store(Yt, tid);
-      }
-#pragma unroll
-      for (int u = 0; u < EB; ++u) {
-        const int e = 4 * (tid + 256 * (b0 + u));
-        split4_bf16(buf[u], Et, El, (e >> 6) * ELD + (e & 63));
+    for (int u = 0; u < NS; ++u) {
+      const int e = 4 * (tid + 256 * u), r = e >> 6, m = e & 63;
+      gl[u] = gr[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      sr[u] = make_uint2(0, 0);
+      if (r >= vlo && r < R) {
+        sr[u] = *reinterpret_cast<const uint2*>(p.s + (((int64_t)c0 + r - p.shift) * H + h) * BT + m);
+        gl[u] = *reinterpret_cast<const float4*>(gcb + (BT - 1) * BT + m);
+        gr[u] = *reinterpret_cast<const float4*>(gcb + r * BT + m);
       }
     }
+    place(part);
 #pragma unroll
     for (int u = 0; u < NS; ++u) {
       const int e = 4 * (tid + 256 * u), r = e >> 6, m = e & 63;
@@ -544,78 +555,128 @@ __global__ __launch_bounds__(256) void bwd_slot_inter_kernel(const SP2 p) {
   }
   lds_barrier();
   const int col = 16 * wave + l16;
-  // the gate rows of the last products' decay, requested before the products
-  const float glast = gcb[(BT - 1) * BT + col];
-  float grow[4][4];
+  // the gates' own rows: four consecutive rows 4 rg + q, four slots gm ..; and the gate rows of the decay of ds
+  const int rg = tid >> 4, gm = (tid & 15) * 4;
+  float4 gi[4], gx[4];
+  uint2 gsv[4];
+  float glast, grow[4][4];
+  auto request_gates = [&]() {
+    glast = gcb[(BT - 1) * BT + col];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) grow[rb][q] = gcb[(16 * rb + 4 * kb + q) * BT + col];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = 4 * rg + q;
+      gi[q] = gx[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+      gsv[q] = make_uint2(0, 0);
+      if (r >= vlo && r < R) {
+        const int64_t rt = (((int64_t)c0 + r) * H + h) * BT + gm;
+        gi[q] = *reinterpret_cast<const float4*>(p.dsi + rt);
+        gx[q] = *reinterpret_cast<const float4*>(p.xg + rt);
+        gsv[q] = *reinterpret_cast<const uint2*>(p.s + (((int64_t)c0 + r - p.shift) * H + h) * BT + gm);
+      }
+    }
+  };
+  const bool has = col >= vlo && col < R;
+  f32x4 dsa[4];   // ds / dec: rows r = 16 rb + 4 kb + q, slot col
+#pragma unroll
+  for (int rb = 0; rb < 4; ++rb) dsa[rb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int z = 0; z < NZ; ++z) {
+    const bool isv = (z & 1) != 0;
+    const int64_t oi = (((int64_t)c0 + col - p.shift) * H + h) * D + (z >> 1) * DW;
+    // the partial sums the first products are added to, then the next part's operands: requested before the products
+    const float* const old = isv ? p.dvs : p.dks;
+    float4 pve[DB];
+    if (has) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db) pve[db] = *reinterpret_cast<const float4*>(old + oi + 16 * db + 4 * kb);
+    }
+    if (z + 1 < NZ) request(part, z + 1);
+    else request_gates();
+    // out^T[x][r = col] = sum_m E[x][m] sE[r][m]: A = E rows (plain), B = sE rows (plain), contraction m in 2 steps
+    f32x4 accO[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) accO[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const bf16x8 bs = lds_frag(St, TLD, col, 32 * ks + 8 * kb), bsl = lds_frag(Sl, TLD, col, 32 * ks + 8 * kb);
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        const bf16x8 eh = lds_frag(Et, ELD, 16 * db + l16, 32 * ks + 8 * kb);
+        accO[db] = mfma16(eh, bs, mfma16(eh, bsl, mfma16(lds_frag(El, ELD, 16 * db + l16, 32 * ks + 8 * kb), bs, accO[db])));
+      }
+    }
+    if (has) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        const float o0 = accO[db][0] + pve[db].x, o1 = accO[db][1] + pve[db].y, o2 = accO[db][2] + pve[db].z, o3 = accO[db][3] + pve[db].w;
+        if (isv) {
+          *reinterpret_cast<float4*>(p.dvs + oi + 16 * db + 4 * kb) = make_float4(o0, o1, o2, o3);
+        } else {
+          bf16x4 pk;
+          pk[0] = (__bf16)o0; pk[1] = (__bf16)o1; pk[2] = (__bf16)o2; pk[3] = (__bf16)o3;
+          *reinterpret_cast<bf16x4*>(p.dkg + oi + 16 * db + 4 * kb) = pk;
+        }
+      }
+    }
+    // ds[r][m = col] / dec += sum_x y_r[x] E[x][m]: A = y rows (two 8-byte reads, contraction index
+    // permuted like the transposing read), B = E via the transposing read
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) {
+#pragma unroll
+      for (int xs = 0; xs < DW / 32; ++xs) {
+        struct { bf16x4 a, b; } t;
+        t.a = *reinterpret_cast<const NHA_LDS bf16x4*>(Yt + (16 * rb + l16) * LDT + 32 * xs + 4 * kb);
+        t.b = *reinterpret_cast<const NHA_LDS bf16x4*>(Yt + (16 * rb + l16) * LDT + 32 * xs + 16 + 4 * kb);
+        const bf16x8 ya = __builtin_bit_cast(bf16x8, t);
+        dsa[rb] = mfma16(ya, lds_frag_tr(Et, ELD, 32 * xs, 32 * xs + 16, 16 * wave, lane),
+                         mfma16(ya, lds_frag_tr(El, ELD, 32 * xs, 32 * xs + 16, 16 * wave, lane), dsa[rb]));
+      }
+    }
+    if (z + 1 == NZ) break;
+    lds_barrier();   // (waits for this wave's reads)
+    place(part);
+    lds_barrier();
+  }
+  // through LDS to the thread that has the row's four slots
+  constexpr int GLD = BT + 4;
+  lfloat* const dl = (lfloat*)(NHA_LDS void*)Yt, * const gs = dl + BT * GLD;   // [64 r][GLD], [16 groups of rows][64]
+  static_assert((BT * GLD + 16 * BT) * 4 <= (TILE + 2 * DW * ELD) * 2, "the rows of ds fit where the tiles were");
+  lds_barrier();
 #pragma unroll
   for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = 16 * rb + 4 * kb + q;
-      grow[rb][q] = gcb[r * BT + col];
-    }
-  // the partial sums the first products are added to: requested before the products where the registers
-  // allow (head sizes up to 128)
-  const bool has = col >= vlo && col < R;
-  const int64_t oi = (((int64_t)c0 + col - p.shift) * H + h) * D + x0;
-  const float* const part = isv ? p.dvs : p.dks;
-  constexpr bool EARLY = DW <= 128;
-  float4 pve[EARLY ? DB : 1];
-  if (EARLY && has) {
+    for (int q = 0; q < 4; ++q) dl[(16 * rb + 4 * kb + q) * GLD + col] = dsa[rb][q] * __expf(glast - grow[rb][q]);
+  lds_barrier();
+  f32x4 sum[4], run = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int db = 0; db < DB; ++db) pve[EARLY ? db : 0] = *reinterpret_cast<const float4*>(part + oi + 16 * db + 4 * kb);
+  for (int q = 3; q >= 0; --q) {
+    const int r = 4 * rg + q;
+    if (r >= vlo && r < R) {
+      const f32x4 d = (f32x4){gi[q].x, gi[q].y, gi[q].z, gi[q].w} + *reinterpret_cast<const NHA_LDS f32x4*>(dl + r * GLD + gm);
+      const f32x4 sv = {__uint_as_float(gsv[q].x << 16), __uint_as_float(gsv[q].x & 0xffff0000u), __uint_as_float(gsv[q].y << 16),
+                        __uint_as_float(gsv[q].y & 0xffff0000u)};
+      run += (f32x4){gx[q].x, gx[q].y, gx[q].z, gx[q].w} - sv * d;
+      bf16x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (__bf16)d[e];
+      *reinterpret_cast<bf16x4*>(p.ds + (((int64_t)c0 + r - p.shift) * H + h) * BT + gm) = o;
+    }
+    sum[q] = run;   // over the later rows of the group
   }
-  // out^T[x][r = col] = sum_m E[x][m] sE[r][m]: A = E rows (plain), B = sE rows (plain), contraction m in 2 steps
-  f32x4 accO[DB];
+  *reinterpret_cast<NHA_LDS f32x4*>(gs + rg * BT + gm) = run;
+  lds_barrier();
+  f32x4 later = {0.f, 0.f, 0.f, 0.f};
+  for (int g = 15; g > rg; --g) later += *reinterpret_cast<const NHA_LDS f32x4*>(gs + g * BT + gm);
 #pragma unroll
-  for (int db = 0; db < DB; ++db) accO[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const bf16x8 bs = lds_frag(St, TLD, col, 32 * ks + 8 * kb), bsl = lds_frag(Sl, TLD, col, 32 * ks + 8 * kb);
-#pragma unroll
-    for (int db = 0; db < DB; ++db) {
-      const bf16x8 eh = lds_frag(Et, ELD, 16 * db + l16, 32 * ks + 8 * kb);
-      accO[db] = mfma16(eh, bs, mfma16(eh, bsl, mfma16(lds_frag(El, ELD, 16 * db + l16, 32 * ks + 8 * kb), bs, accO[db])));
-    }
+  for (int q = 0; q < 4; ++q) {
+    const int r = 4 * rg + q;
+    if (r >= vlo && r < R) *reinterpret_cast<f32x4*>(p.dsi + (((int64_t)c0 + r) * H + h) * BT + gm) = sum[q] + later;
   }
-  if (has) {
-#pragma unroll
-    for (int db = 0; db < DB; ++db) {
-      const float4 pv = EARLY ? pve[EARLY ? db : 0] : *reinterpret_cast<const float4*>(part + oi + 16 * db + 4 * kb);
-      const float o0 = accO[db][0] + pv.x, o1 = accO[db][1] + pv.y, o2 = accO[db][2] + pv.z, o3 = accO[db][3] + pv.w;
-      if (isv) {
-        *reinterpret_cast<float4*>(p.dvs + oi + 16 * db + 4 * kb) = make_float4(o0, o1, o2, o3);
-      } else {
-        bf16x4 pk;
-        pk[0] = (__bf16)o0; pk[1] = (__bf16)o1; pk[2] = (__bf16)o2; pk[3] = (__bf16)o3;
-        *reinterpret_cast<bf16x4*>(p.dkg + oi + 16 * db + 4 * kb) = pk;
-      }
-    }
-  }
-  // dsp[r][m = col] = dec_r[m] sum_x y_r[x] E[x][m]: A = y rows (two 8-byte reads, contraction index
-  // permuted like the transposing read), B = E via the transposing read
-#pragma unroll
-  for (int rb = 0; rb < 4; ++rb) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int xs = 0; xs < DW / 32; ++xs) {
-      struct { bf16x4 a, b; } t;
-      t.a = *reinterpret_cast<const NHA_LDS bf16x4*>(Yt + (16 * rb + l16) * LDT + 32 * xs + 4 * kb);
-      t.b = *reinterpret_cast<const NHA_LDS bf16x4*>(Yt + (16 * rb + l16) * LDT + 32 * xs + 16 + 4 * kb);
-      const bf16x8 ya = __builtin_bit_cast(bf16x8, t);
-      acc = mfma16(ya, lds_frag_tr(Et, ELD, 32 * xs, 32 * xs + 16, 16 * wave, lane),
-                   mfma16(ya, lds_frag_tr(El, ELD, 32 * xs, 32 * xs + 16, 16 * wave, lane), acc));
-    }
-    // C[r = 16 rb + 4 kb + q][m = col]
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = 16 * rb + 4 * kb + q;
-      if (r < R) {
-        const float dec = __expf(glast - grow[rb][q]);
-        p.dsp[(((int64_t)((isv ? NH : 0) + xh) * p.T_tot + c0 + r) * H + h) * BT + col] = acc[q] * dec;
-      }
-    }
-  }
+  if (rg == 0) *reinterpret_cast<f32x4*>(p.gtot + ((int64_t)chunk * H + h) * BT + gm) = run + later;
 }
 
 template <int D, int TK>
@@ -705,19 +766,18 @@ static int launch_slot_inter(const SP2& p, int NT, hipStream_t st) {
     }
     configured = true;
   }
-  hipLaunchKernelGGL((bwd_slot_inter_kernel<D, DWI>), dim3(p.H, NT, 2 * (D / DWI)), dim3(256), lds, st, p);
+  hipLaunchKernelGGL((bwd_slot_inter_kernel<D, DWI>), dim3(p.H, NT), dim3(256), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(slot branch, carried state gradient)");
   return NHA_OK;
 }
 
-// partial-ds slabs per state that bwd_slot_inter_kernel writes: one per column range of a workgroup
-int bwd_slot_inter_slabs(const NhaPrefillBwdArgs* a) { return a->K > 128 ? a->K / 128 : 1; }
-
-int bwd_slot_inter(const NhaPrefillBwdArgs* a, const float* gc, const float* ek, const float* ev, const float* dks, float* dvs, float* dsp) {
+int bwd_slot_inter(const NhaPrefillBwdArgs* a, const float* gc, const float* ek, const float* ev, const float* dks, float* dvs, const float* xg,
+                   float* dsi, float* gtot) {
   SP2 p;
   p.kg = (const bf16_t*)a->k_gsa; p.v = (const bf16_t*)a->v; p.s = (const bf16_t*)a->s;
-  p.gc = gc; p.ek = ek; p.ev = ev; p.dks = dks; p.dvs = dvs; p.dsp = dsp;
-  p.dkg = (bf16_t*)a->dk_gsa; p.T_tot = a->T_tot;
+  p.gc = gc; p.ek = ek; p.ev = ev; p.dks = dks; p.dvs = dvs;
+  p.xg = xg; p.dsi = dsi; p.gtot = gtot; p.ds = (bf16_t*)a->ds;
+  p.dkg = (bf16_t*)a->dk_gsa;
   p.cu = a->cu_seqlens; p.cidx = a->chunk_indices;
   p.H = a->H; p.shift = a->shift;
   hipStream_t st = (hipStream_t)a->stream;
