@@ -185,20 +185,36 @@ _PACK_CODES = {C.c_int32: "i", C.c_int64: "q", C.c_float: "f", C.c_void_p: "P", 
 
 def packer(cls):
     """`pack(*values)` of a `struct.Struct` with the fields of the ctypes structure `cls` in their order (NULL is 0): an
-    argument block as bytes in about 1 us, where setting 40 ctypes fields one by one takes 4."""
-    s = struct.Struct("@" + "".join(_PACK_CODES[t] for _, t in cls._fields_))
+    argument block as bytes in about 1 us, where setting 40 ctypes fields one by one takes 4.  An array field takes as
+    many values as it has entries."""
+    code = lambda t: _PACK_CODES[t] if t in _PACK_CODES else _PACK_CODES[t._type_] * t._length_
+    s = struct.Struct("@" + "".join(code(t) for _, t in cls._fields_))
     assert s.size <= C.sizeof(cls) < s.size + 8      # the structure's own tail padding is not part of the format
     pad = C.sizeof(cls) - s.size
     return s.pack if not pad else struct.Struct(s.format + "%dx" % pad).pack
 
 
 pack_decode = packer(NhaDecodeArgs)
+pack_prefill = packer(NhaPrefillArgs)
+pack_prefill_bwd = packer(NhaPrefillBwdArgs)
+pack_hybrid_prologue = packer(NhaHybridPrologueArgs)
+pack_ring_fill = packer(NhaRingFillArgs)
 _PACK_SCRATCH = struct.Struct("@PN").pack      # the last two fields
 
 
 def with_scratch(args: bytes, scratch: int, nbytes: int) -> bytes:
     """The block of pack_decode with another scratch."""
     return args[:-16] + _PACK_SCRATCH(scratch, nbytes)
+
+
+def i32(x: int) -> int:
+    """x as a ctypes int32 field holds it: a whole number out of range wraps (struct would refuse it)."""
+    return x if -0x80000000 <= x <= 0x7fffffff else C.c_int32(x).value
+
+
+def f32(x: float) -> float:
+    """x as a ctypes float field holds it: infinite beyond float32's range (struct would refuse it)."""
+    return C.c_float(x).value
 
 
 class NhaError(RuntimeError):
@@ -225,6 +241,13 @@ def load() -> C.CDLL:
     lib.nha_prefill_fwd.argtypes = [C.POINTER(NhaPrefillArgs)]
     lib.nha_prefill_fwd_noalloc.restype = C.c_int
     lib.nha_prefill_fwd_noalloc.argtypes = [C.POINTER(NhaPrefillArgs)]
+    # the same entries for argument blocks packed by pack_prefill and its like
+    lib.prefill_scratch_bytes_packed = C.CFUNCTYPE(C.c_size_t, C.c_char_p)(("nha_prefill_scratch_bytes", lib))
+    lib.prefill_fwd_packed = C.CFUNCTYPE(C.c_int, C.c_char_p)(("nha_prefill_fwd", lib))
+    lib.prefill_bwd_scratch_bytes_packed = C.CFUNCTYPE(C.c_size_t, C.c_char_p)(("nha_prefill_bwd_scratch_bytes", lib))
+    lib.prefill_bwd_packed = C.CFUNCTYPE(C.c_int, C.c_char_p)(("nha_prefill_bwd", lib))
+    lib.hybrid_prologue_packed = C.CFUNCTYPE(C.c_int, C.c_char_p)(("nha_hybrid_prologue", lib))
+    lib.ring_fill_packed = C.CFUNCTYPE(C.c_int, C.c_char_p)(("nha_ring_fill", lib))
     lib.nha_prefill_bwd_scratch_bytes.restype = C.c_size_t
     lib.nha_prefill_bwd_scratch_bytes.argtypes = [C.POINTER(NhaPrefillBwdArgs)]
     lib.nha_prefill_bwd.restype = C.c_int

@@ -197,14 +197,14 @@ class HybridNHAAttention(nn.Module):
         a copy held by the module (rebuilt when a weight's storage or version changes): inference memory for the
         attention projections doubles, four launches become one."""
         mods = [self.q_proj, self.k_proj, self.v_proj] + ([self.g_proj] if with_gates else [])
-        key = tuple((m.weight.data_ptr(), m.weight._version, m.weight.dtype, m.weight.device,
-                     None if m.bias is None else (m.bias.data_ptr(), m.bias._version)) for m in mods)
+        wb = [(m.weight, m.bias) for m in mods]      # read once: a module's attribute takes a look-up in three dictionaries
+        key = tuple([(w.data_ptr(), w._version, w.dtype, w.device, None if b is None else (b.data_ptr(), b._version)) for w, b in wb])
         if self._fused_key != key:
-            w = torch.cat([m.weight.detach() for m in mods], 0)
+            w = torch.cat([wt.detach() for wt, _ in wb], 0)
             b = None
-            if any(m.bias is not None for m in mods):
-                b = torch.cat([m.bias.detach() if m.bias is not None else
-                               torch.zeros(m.weight.shape[0], dtype=w.dtype, device=w.device) for m in mods], 0)
+            if any(bt is not None for _, bt in wb):
+                b = torch.cat([bt.detach() if bt is not None else
+                               torch.zeros(wt.shape[0], dtype=w.dtype, device=w.device) for wt, bt in wb], 0)
             self._fused_key, self._fused_wb = key, (w, b)
         w, b = self._fused_wb
         return F.linear(x, w, b)
@@ -257,7 +257,7 @@ class HybridNHAAttention(nn.Module):
                  and not (hidden_states.dtype == torch.float32 and torch.is_autocast_enabled()))
         if fused:
             y = self._fused_projection(hidden_states, with_gates=nha)
-            o0, o1, o2 = HQ * D, HQ * D + H * D, HQ * D + 2 * H * D
+            qy, ky, vy, fy = y.split([HQ * D, H * D, H * D, y.shape[-1] - (HQ + 2 * H) * D], -1)
             cos = sin = pos = inv = None
             if position_embeddings is not None:
                 cos, sin = self._tables(hidden_states, position_ids, position_embeddings, past_key_value, T)
@@ -267,7 +267,7 @@ class HybridNHAAttention(nn.Module):
                     start = past_key_value.layer_tokens(self.layer_idx) if past_key_value is not None else 0
                     pos = torch.arange(start, start + T, device=hidden_states.device)[None].expand(B, T)
             q, sq, k, sk, v, g, s = nha_hybrid_prologue(
-                y[..., :o0], y[..., o0:o1], y[..., o1:o2], y[..., o2:] if nha else None, cos, sin, positions=pos, inv_freq=inv,
+                qy, ky, vy, fy if nha else None, cos, sin, positions=pos, inv_freq=inv,
                 num_heads=HQ,
                 num_kv_heads=H, head_dim=D, num_slots=M, q_weight=self.q_norm.weight if self.qk_norm else None,
                 k_weight=self.k_norm.weight if self.qk_norm else None,

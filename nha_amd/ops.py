@@ -170,42 +170,47 @@ def nha_prefill(q_swa, k_swa, q_gsa, k_gsa, v, s, g, cu_host: np.ndarray, *, wl:
                 h0=None, want_state: bool = False, want_lse: bool = True, impl=None):
     """Packed prefill on token-major tensors ``[T_tot, heads, dim]`` (one nha_prefill_fwd call).
     Returns (o, lse_swa, lse_gsa, hkt, hvt)."""
+    return _prefill((q_swa, k_swa, q_gsa, k_gsa, v, s, g), q_swa.shape[:1], cu_host, wl, shift, scale, h0, want_state, want_lse, impl)
+
+
+def _at(t: Optional[torch.Tensor]) -> int:
+    return 0 if t is None else t.data_ptr()
+
+
+def _prefill(args, lead, cu_host: np.ndarray, wl: int, shift: int, scale: float, h0, want_state: bool, want_lse: bool, impl):
+    """nha_prefill on contiguous tensors ``[..., heads, dim]`` whose leading sizes number the same tokens; o and the
+    logsumexps come back with the leading sizes `lead`.  Small calls are bound by this function: with the argument block
+    packed (not 35 ctypes fields set) and no views made of operands and results, chunk_nha on 512 tokens of 4 fp32 heads of 64
+    takes 34 us where it took 44, the host's share of it 31 where it was 47."""
     lib = _lib.load()
-    T_tot, HQ, K = q_swa.shape
-    H, V, M = k_swa.shape[1], v.shape[-1], s.shape[-1]
-    dev = q_swa.device
+    q_swa, k_swa, v, s = args[0], args[1], args[4], args[5]
+    HQ, K = q_swa.shape[-2:]
+    T_tot = q_swa.shape[0] if q_swa.dim() == 3 else q_swa.shape[0] * q_swa.shape[1]
+    H, V, M = k_swa.shape[-2], v.shape[-1], s.shape[-1]
+    dev, dt = q_swa.device, q_swa.dtype
     N = cu_host.size - 1
     cu_d, idx_d, off_d, NT = prefill_tables(cu_host, dev)
-    o = torch.empty(T_tot, HQ, V, dtype=q_swa.dtype, device=dev)
-    lse_swa = torch.empty(T_tot, HQ, dtype=torch.float32, device=dev) if want_lse else None
-    lse_gsa = torch.empty(T_tot, HQ, dtype=torch.float32, device=dev) if want_lse else None
+    o = torch.empty(*lead, HQ, V, dtype=dt, device=dev)
+    lse_swa = torch.empty(*lead, HQ, dtype=torch.float32, device=dev) if want_lse else None
+    lse_gsa = torch.empty(*lead, HQ, dtype=torch.float32, device=dev) if want_lse else None
     hkt = torch.empty(N, H, K, M, dtype=torch.float32, device=dev) if want_state else None
     hvt = torch.empty(N, H, M, V, dtype=torch.float32, device=dev) if want_state else None
     h0k = h0v = None
     if h0 is not None and h0[0] is not None:
-        h0k = h0[0].to(torch.float32).contiguous()
-        h0v = h0[1].to(torch.float32).contiguous()
+        h0k, h0v = _as(h0[0], torch.float32), _as(h0[1], torch.float32)
         if tuple(h0k.shape) != (N, H, K, M) or tuple(h0v.shape) != (N, H, M, V):
             raise ValueError(f"initial_state must be ([{N},{H},{K},{M}], [{N},{H},{M},{V}]) (kv-head count), "
                              f"got {tuple(h0k.shape)} / {tuple(h0v.shape)}")
-    a = _lib.NhaPrefillArgs()
-    a.q_swa, a.k_swa, a.q_gsa, a.k_gsa = _ptr(q_swa), _ptr(k_swa), _ptr(q_gsa), _ptr(k_gsa)
-    a.v, a.s, a.g, a.o = _ptr(v), _ptr(s), _ptr(g), _ptr(o)
-    a.lse_swa, a.lse_gsa = _ptr(lse_swa), _ptr(lse_gsa)
-    a.h0k, a.h0v, a.hkt, a.hvt = _ptr(h0k), _ptr(h0v), _ptr(hkt), _ptr(hvt)
-    a.cu_seqlens, a.chunk_indices, a.chunk_offsets = _ptr(cu_d), _ptr(idx_d), _ptr(off_d)
-    a.T_tot, a.N, a.NT, a.HQ, a.H, a.K, a.V, a.M = T_tot, N, NT, HQ, H, K, V, M
-    a.wl, a.shift = int(wl), int(shift)
-    a.dtype = _dtype_code(q_swa)
-    a.impl = _IMPL[impl]
-    a.scale = float(scale)
-    a.stream = _stream(dev)
-    nbytes = lib.nha_prefill_scratch_bytes(C.byref(a))
+    stream = _stream(dev)
+    head = (*(x.data_ptr() for x in args), o.data_ptr(), _at(lse_swa), _at(lse_gsa), _at(h0k), _at(h0v), _at(hkt), _at(hvt),
+            cu_d.data_ptr(), idx_d.data_ptr(), off_d.data_ptr())
+    dims = (T_tot, N, NT, HQ, H, K, V, M, _lib.i32(int(wl)), _lib.i32(int(shift)), _dtype_code(q_swa), _IMPL[impl],
+            _lib.f32(float(scale)), stream)
+    nbytes = lib.prefill_scratch_bytes_packed(_lib.pack_prefill(*head, 0, 0, *dims))
     if nbytes == 0:
         _lib.check(_lib.NHA_ERR_INVALID)
-    scratch = _workspace(nbytes, dev, a.stream or 0)
-    a.scratch, a.scratch_bytes = _ptr(scratch), scratch.numel()
-    _lib.check(lib.nha_prefill_fwd(C.byref(a)))
+    scratch = _workspace(nbytes, dev, stream)
+    _lib.check(lib.prefill_fwd_packed(_lib.pack_prefill(*head, scratch.data_ptr(), scratch.numel(), *dims)))
     return o, lse_swa, lse_gsa, hkt, hvt
 
 
@@ -214,43 +219,43 @@ def nha_prefill_bwd(q_swa, k_swa, q_gsa, k_gsa, v, s, g, o, lse_swa, lse_gsa, do
                     want_dh0: bool = False):
     """Packed prefill backward on token-major tensors (one nha_prefill_bwd call).  Returns
     (dq_swa, dk_swa, dq_gsa, dk_gsa, dv, ds, dg, dh0k, dh0v) -- the last two None unless wanted."""
+    return _prefill_bwd((q_swa, k_swa, q_gsa, k_gsa, v, s, g), o, lse_swa, lse_gsa, dout, cu_host, wl, shift, scale, h0, dlse_swa,
+                        dlse_gsa, dht, want_dh0)
+
+
+def _prefill_bwd(args, o, lse_swa, lse_gsa, dout, cu_host: np.ndarray, wl: int, shift: int, scale: float, h0, dlse_swa, dlse_gsa,
+                 dht, want_dh0: bool):
+    """nha_prefill_bwd on contiguous tensors ``[..., heads, dim]`` whose leading sizes number the same tokens; a gradient has
+    its tensor's shape."""
     lib = _lib.load()
-    T_tot, HQ, K = q_swa.shape
-    H, V, M = k_swa.shape[1], v.shape[-1], s.shape[-1]
+    q_swa, k_swa, v, s = args[0], args[1], args[4], args[5]
+    HQ, K = q_swa.shape[-2:]
+    T_tot = q_swa.shape[0] if q_swa.dim() == 3 else q_swa.shape[0] * q_swa.shape[1]
+    H, V, M = k_swa.shape[-2], v.shape[-1], s.shape[-1]
     dev = q_swa.device
     N = cu_host.size - 1
     cu_d, idx_d, off_d, NT = prefill_tables(cu_host, dev)
-    f32 = lambda x: None if x is None else x.to(torch.float32).contiguous()
+    f32 = lambda x: _as(x, torch.float32)
     h0k, h0v = (None, None) if h0 is None or h0[0] is None else (f32(h0[0]), f32(h0[1]))
     dhkt, dhvt = (None, None) if dht is None else dht
     if (dhkt is None) != (dhvt is None):      # one final state unused downstream: its cotangent is zero
         dhkt = torch.zeros(N, H, K, M, dtype=torch.float32, device=dev) if dhkt is None else dhkt
         dhvt = torch.zeros(N, H, M, V, dtype=torch.float32, device=dev) if dhvt is None else dhvt
     dhkt, dhvt, dlse_swa, dlse_gsa = f32(dhkt), f32(dhvt), f32(dlse_swa), f32(dlse_gsa)
-    dout = dout.to(q_swa.dtype).contiguous()
-    outs = [torch.empty_like(x) for x in (q_swa, k_swa, q_gsa, k_gsa, v, s, g)]
+    dout = _as(dout, q_swa.dtype)
+    outs = [torch.empty_like(x) for x in args]
     dh0k = torch.empty(N, H, K, M, dtype=torch.float32, device=dev) if want_dh0 else None
     dh0v = torch.empty(N, H, M, V, dtype=torch.float32, device=dev) if want_dh0 else None
-    a = _lib.NhaPrefillBwdArgs()
-    a.q_swa, a.k_swa, a.q_gsa, a.k_gsa = _ptr(q_swa), _ptr(k_swa), _ptr(q_gsa), _ptr(k_gsa)
-    a.v, a.s, a.g = _ptr(v), _ptr(s), _ptr(g)
-    a.o, a.lse_swa, a.lse_gsa = _ptr(o), _ptr(lse_swa), _ptr(lse_gsa)
-    a.h0k, a.h0v = _ptr(h0k), _ptr(h0v)
-    a.dout, a.dlse_swa, a.dlse_gsa, a.dhkt, a.dhvt = _ptr(dout), _ptr(dlse_swa), _ptr(dlse_gsa), _ptr(dhkt), _ptr(dhvt)
-    a.dq_swa, a.dk_swa, a.dq_gsa, a.dk_gsa, a.dv, a.ds, a.dg = [_ptr(x) for x in outs]
-    a.dh0k, a.dh0v = _ptr(dh0k), _ptr(dh0v)
-    a.cu_seqlens, a.chunk_indices, a.chunk_offsets = _ptr(cu_d), _ptr(idx_d), _ptr(off_d)
-    a.T_tot, a.N, a.NT, a.HQ, a.H, a.K, a.V, a.M = T_tot, N, NT, HQ, H, K, V, M
-    a.wl, a.shift = int(wl), int(shift)
-    a.dtype = _dtype_code(q_swa)
-    a.scale = float(scale)
-    a.stream = _stream(dev)
-    nbytes = lib.nha_prefill_bwd_scratch_bytes(C.byref(a))
+    stream = _stream(dev)
+    head = (*(x.data_ptr() for x in args), o.data_ptr(), lse_swa.data_ptr(), lse_gsa.data_ptr(), _at(h0k), _at(h0v), dout.data_ptr(),
+            _at(dlse_swa), _at(dlse_gsa), _at(dhkt), _at(dhvt), *(x.data_ptr() for x in outs), _at(dh0k), _at(dh0v),
+            cu_d.data_ptr(), idx_d.data_ptr(), off_d.data_ptr())
+    dims = (T_tot, N, NT, HQ, H, K, V, M, _lib.i32(int(wl)), _lib.i32(int(shift)), _dtype_code(q_swa), _lib.f32(float(scale)), stream)
+    nbytes = lib.prefill_bwd_scratch_bytes_packed(_lib.pack_prefill_bwd(*head, 0, 0, *dims))
     if nbytes == 0:
         _lib.check(_lib.NHA_ERR_INVALID)
-    scratch = _workspace(nbytes, dev, a.stream or 0)     # shared with the forward: calls on one stream are ordered
-    a.scratch, a.scratch_bytes = _ptr(scratch), nbytes
-    _lib.check(lib.nha_prefill_bwd(C.byref(a)))
+    scratch = _workspace(nbytes, dev, stream)     # shared with the forward: calls on one stream are ordered
+    _lib.check(lib.prefill_bwd_packed(_lib.pack_prefill_bwd(*head, scratch.data_ptr(), nbytes, *dims)))
     return (*outs, dh0k, dh0v)
 
 
@@ -867,14 +872,13 @@ def nha_hybrid_prologue(q, k, v, f, cos, sin, *, num_heads: int, num_kv_heads: i
     new = lambda h, d: torch.empty(B, T, h, d, dtype=dt, device=dev)
     qo, sqo, ko, sko, vo, go = new(HQ, D), new(HQ, D), new(H, D), new(H, D), new(H, D), new(H, M)
     so = new(H, M) if want_s else None
-    a = _lib.NhaHybridPrologueArgs(
-        q=_ptr(q), k=_ptr(k), v=_ptr(v), f=_ptr(f), q_stride=qs, k_stride=ks, v_stride=vs, f_stride=fs,
-        q_weight=_ptr(None if q_weight is None else q_weight.contiguous()),
-        k_weight=_ptr(None if k_weight is None else k_weight.contiguous()), cos=_ptr(cos), sin=_ptr(sin),
-        cs_batch_stride=cs_stride, positions=_ptr(positions), inv_freq=_ptr(inv_freq), mask=_ptr(mask), q_out=_ptr(qo), sq_out=_ptr(sqo),
-        k_out=_ptr(ko), sk_out=_ptr(sko), v_out=_ptr(vo), g_out=_ptr(go), s_out=_ptr(so), B=B, T=T, HQ=HQ, H=H, D=D, M=M,
-        dtype=_dtype_code(q), eps=float(eps), gate_logit_normalizer=float(gate_logit_normalizer), stream=_stream(dev))
-    _lib.check(_lib.load().nha_hybrid_prologue(C.byref(a)))
+    qw, kw = (None if w is None else w.contiguous() for w in (q_weight, k_weight))
+    args = _lib.pack_hybrid_prologue(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), _at(f), qs, ks, vs, fs, _at(qw), _at(kw), _at(cos), _at(sin), cs_stride,
+        _at(positions), _at(inv_freq), _at(mask), qo.data_ptr(), sqo.data_ptr(), ko.data_ptr(), sko.data_ptr(), vo.data_ptr(),
+        go.data_ptr(), _at(so), B, T, HQ, H, D, M, _dtype_code(q), _lib.f32(float(eps)), _lib.f32(float(gate_logit_normalizer)),
+        _stream(dev))
+    _lib.check(_lib.load().hybrid_prologue_packed(args))
     return qo, sqo, ko, sko, vo, go, so
 
 
@@ -950,11 +954,10 @@ class _ChunkNHAFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q_swa, k_swa, q_gsa, k_gsa, v, s, g, h0k, h0v, cu_host, wl, shift, scale, want_state, impl):
         args = (q_swa, k_swa, q_gsa, k_gsa, v, s, g)
-        ctx.shapes = [x.shape for x in args]
         args = [x.contiguous() for x in args]      # saved as they are: a view made here would hide later edits from autograd
         h0 = None if h0k is None else (h0k, h0v)
-        o, lse_swa, lse_gsa, hkt, hvt = nha_prefill(*(_flat(x) for x in args), cu_host, wl=wl, shift=shift, scale=scale, h0=h0,
-                                                    want_state=want_state, impl=impl)
+        o, lse_swa, lse_gsa, hkt, hvt = _prefill(args, (q_swa.shape[0] * q_swa.shape[1],), cu_host, wl, shift, scale, h0, want_state,
+                                                 True, impl)
         ctx.save_for_backward(*args, o, lse_swa, lse_gsa, h0k, h0v)
         ctx.cu_host, ctx.wl, ctx.shift, ctx.scale = cu_host.copy(), wl, shift, scale    # it may be the caller's memory
         ctx.set_materialize_grads(False)
@@ -970,13 +973,12 @@ class _ChunkNHAFunction(torch.autograd.Function):
             do = torch.zeros_like(o)
         want_dh0 = h0k is not None and (ctx.needs_input_grad[7] or ctx.needs_input_grad[8])
         dht = None if dhkt is None and dhvt is None else (dhkt, dhvt)
-        grads = nha_prefill_bwd(*(_flat(x) for x in args), o, lse_swa, lse_gsa, do, ctx.cu_host, wl=ctx.wl,
-                                shift=ctx.shift, scale=ctx.scale, h0=None if h0k is None else (h0k, h0v), dlse_swa=dlse_swa,
-                                dlse_gsa=dlse_gsa, dht=dht, want_dh0=want_dh0)
+        grads = _prefill_bwd([x.contiguous() for x in args], o, lse_swa, lse_gsa, do, ctx.cu_host, ctx.wl, ctx.shift, ctx.scale,
+                             None if h0k is None else (h0k, h0v), dlse_swa, dlse_gsa, dht, want_dh0)
         dh0k, dh0v = grads[7], grads[8]
         if dh0k is not None:
             dh0k, dh0v = dh0k.to(h0k.dtype), dh0v.to(h0v.dtype)
-        return (*(x.view(shape) for x, shape in zip(grads, ctx.shapes)), dh0k, dh0v, None, None, None, None, None, None)
+        return (*grads[:7], dh0k, dh0v, None, None, None, None, None, None)
 
 
 def _plain_autograd(tensors) -> bool:
@@ -1056,11 +1058,11 @@ def chunk_nha(
     h0 = (None, None) if initial_state is None or initial_state[0] is None else tuple(initial_state)
     # empty sequences (a fully padded batch row after unpadding yields a repeated cu_seqlens entry): the
     # kernels see the packing without them; their final state is their initial state
-    lens = np.diff(cu_host)
-    if (lens < 0).any():
-        raise ValueError("cu_seqlens must be non-decreasing")
     keep = None
-    if (lens == 0).any():
+    lens = None if cu_seqlens is None else np.diff(cu_host)
+    if lens is not None and (lens < 0).any():
+        raise ValueError("cu_seqlens must be non-decreasing")
+    if lens is not None and (lens == 0).any():
         keep = torch.from_numpy(np.nonzero(lens > 0)[0]).to(q_swa.device)
         n_all = lens.size
         cu_host = np.concatenate([[0], np.cumsum(lens[lens > 0])]).astype(np.int32)
@@ -1069,7 +1071,7 @@ def chunk_nha(
             h0 = (h0[0][keep], h0[1][keep])
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (*args, *h0)):
         # the autograd node itself where nothing else has to see the call: the registered operator's dispatch costs a
-        # training step 110 us of host time (390 against 280 us, where the GPU takes 210 to 270 for 1700 tokens)
+        # training step 110 us of host time, where the GPU takes 210 to 270 for 1700 tokens
         if impl is not None or _plain_autograd((*args, *h0)):
             o, lse_swa, lse_gsa, hkt, hvt = _ChunkNHAFunction.apply(
                 *args, h0[0], h0[1], cu_host, int(window_size_left), int(gsa_kv_shift), float(scale), output_final_state, impl)
@@ -1079,18 +1081,16 @@ def chunk_nha(
                 *(_flat(x) for x in args), torch.from_numpy(np.ascontiguousarray(cu_host, dtype=np.int32)), int(window_size_left),
                 int(gsa_kv_shift), float(scale), h0[0], h0[1], bool(output_final_state))
     else:
-        o, lse_swa, lse_gsa, hkt, hvt = nha_prefill(
-            *(_flat(x) for x in args), cu_host, wl=window_size_left, shift=gsa_kv_shift, scale=scale,
-            h0=None if h0[0] is None else h0, want_state=output_final_state, impl=impl)
+        o, lse_swa, lse_gsa, hkt, hvt = _prefill([x.contiguous() for x in args], (B, T), cu_host, window_size_left, gsa_kv_shift, scale,
+                                                 None if h0[0] is None else h0, output_final_state, True, impl)
     if keep is not None and output_final_state:
         def spread(part, init):
             full = torch.zeros(n_all, *part.shape[1:], dtype=part.dtype, device=part.device) if init is None \
                 else init.to(part.dtype).clone()
             return full.index_copy(0, keep, part)
         hkt, hvt = spread(hkt, h0_all[0]), spread(hvt, h0_all[1])
-    o = o.view(B, T, HQ, -1)
-    lse_swa = lse_swa.view(B, T, HQ)
-    lse_gsa = lse_gsa.view(B, T, HQ)
+    if o.dim() == 3:
+        o, lse_swa, lse_gsa = o.view(B, T, HQ, -1), lse_swa.view(B, T, HQ), lse_gsa.view(B, T, HQ)
     if output_final_state:
         return o, lse_swa, lse_gsa, (hkt, hvt)
     return o, lse_swa, lse_gsa
@@ -1138,10 +1138,9 @@ def fused_chunk_nha_prefill(
         scale = K ** -0.5
     cu_host = np.arange(0, (B + 1) * T, T, dtype=np.int32)
     dt = q.dtype
-    args = [_flat(x.to(dt)) for x in (rotary_q, rotary_k, q, k, v, s, g)]
-    o, _, _, hkt, hvt = nha_prefill(*args, cu_host, wl=W - 1, shift=W, scale=scale, h0=initial_state,
-                                    want_state=output_final_state, want_lse=False, impl=impl)
-    return o.view(B, T, HQ, -1), (hkt, hvt)
+    args = [_as(x, dt) for x in (rotary_q, rotary_k, q, k, v, s, g)]
+    o, _, _, hkt, hvt = _prefill(args, (B, T), cu_host, W - 1, W, scale, initial_state, output_final_state, False, impl)
+    return o, (hkt, hvt)
 
 
 def _decode_state(initial_state, output_final_state, NG, B, H, K, V, M, dev):

@@ -6,7 +6,6 @@ reference (nha_fla/models/nha_cache.py:105-131, :143-154; models/qwen3_moe_nha/q
 slot and attends over the valid entries, reading state and window once per kv-head."""
 from __future__ import annotations
 
-import ctypes as C
 from dataclasses import dataclass
 from typing import Optional
 
@@ -104,13 +103,10 @@ class NHARingState:
         state_sizes = [x.numel() // N * 4 for x in states]
         if any(b % 16 for b in (*sizes, *state_sizes)) or any(x.data_ptr() % 16 for x in (*rows, *states)):
             return None
-        a = _lib.NhaRingFillArgs()
-        for x in range(4):
-            a.src[x], a.ring[x], a.row_bytes[x] = rows[x].data_ptr(), rings[x].data_ptr(), sizes[x]
-        for x in range(2):
-            a.state[x], a.state_out[x], a.state_bytes[x] = states[x].data_ptr(), out[x].data_ptr(), state_sizes[x]
-        a.cu_seqlens, a.count, a.N, a.T, a.tokens, a.W, a.stream = _ptr(cu), count.data_ptr(), N, T, rows[0].shape[0] * T, W, _stream(dev)
-        _lib.check(_lib.load().nha_ring_fill(C.byref(a)))
+        at = lambda xs: [x.data_ptr() for x in xs]
+        args = _lib.pack_ring_fill(*at(rows), *at(rings), *sizes, *at(states), *at(out), *state_sizes, 0 if cu is None else cu.data_ptr(),
+                                   count.data_ptr(), rows[0].shape[0] * T, N, T, _lib.i32(W), _stream(dev))
+        _lib.check(_lib.load().ring_fill_packed(args))
         return cls(*out, *rings, count)
 
     @property
