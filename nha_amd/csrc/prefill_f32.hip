@@ -5,19 +5,20 @@
 //   state_local : per (chunk, kv-head, state) the chunk's own contribution  U = K^T (S exp(gc_last - gc)), [m][d], and the
 //                 chunk-local gate cumsum gc
 //   state_scan  : h_c+1 = exp(gc_last) h_c + U_c element by element over the chunks of a sequence; U_c is replaced by h_c
-//   out         : one WAVE per (16 rows of a chunk, query head): window, slot logits, slot read, one softmax
+//   out         : one WAVE per (16 rows of a chunk, query head): window, slot logits, slot read, one softmax; four waves where
+//                 there are few such units
 //
 // The generic kernels walk a sequence's chunks in one workgroup per 16 slots, every row's loads waited for one by one
 // (115 us per chunk), and their output pass redoes the slot algebra per token; here the chunks are independent but for
 // an element-wise scan, and everything else is matrix products.  Bound: launches and latencies at prompt sizes (B=1, T=512, 4
-// heads of 64, W=64: 1028 -> 34 us of kernels), the fp32 matrix rate beyond (per call, generic kernels / these: B=1, T=2048,
+// heads of 64, W=64: 1028 -> 23 us of kernels), the fp32 matrix rate beyond (per call, generic kernels / these: B=1, T=2048,
 // 8/2 heads of 128, W=64 8.2 ms / 62 us; B=2, T=4096, 32/8 heads 30.7 / 0.57 ms = 46 TFLOP/s; B=1, T=4096, 16 heads of 64,
 // W=1024 16.9 / 0.29 ms = 67 TFLOP/s; a library matrix product reaches 150).
 //
 // Everything is computed transposed (a query per lane), with operands loaded from global memory in MFMA layout: A = a
 // row of keys / slots per lane (16 bytes of consecutive columns, four products per load; both operands number the
 // contraction the same way, so its order is free), and the accumulator of a score product is the B operand of the next
-// product as it stands.  No LDS, no barriers.  A unit whose output is not finite is formed a second time without the rows that
+// product as it stands.  No LDS, no barriers (but for the exchange between four waves of a unit).  A unit whose output is not finite is formed a second time without the rows that
 // a query does not see (f32_out_rows); the look at the output costs nothing measurable (567 / 560 us without / with, at
 // B=2, T=4096, 32/8 heads of 128).
 #include "common.h"
@@ -463,6 +464,302 @@ __global__ __launch_bounds__(64 * WPB, D <= 128 ? 2 : 1) void f32_out_kernel(con
   if (f32_out_rows<D, false>(p, chunk, h, gq, sub)) f32_out_rows<D, true>(p, chunk, h, gq, sub);
 }
 
+// The same unit by a workgroup of four waves, for calls with fewer units than the card has room for: a unit alone is one chain
+// of dependent loads and products (q, window blocks one after the other, logits, the rows of the chunk twice).  Wave w takes
+// every fourth block of window keys and the 16 slots from 16 w on, each with a softmax of its own, and row block w of the
+// chunk: its scores for the slots of all waves, and its values with the weights that the four waves' slots give it.  What
+// the waves exchange goes through LDS: scores, weights relative to each wave's maximum, at last 3/4 of the outputs.
+// Kernel at 512 tokens, 4 heads of 64, W = 64 (128 units): 22.9 -> 12.5 us,
+// W = 512 45.0 -> 17.4; 8 heads of 128, W = 64 (256 units) 32.7 -> 16.7; 4 heads of 256 59.5 -> 29.7.  (With the values and
+// weights of the slot part requested before the window too: 13.2 and 256 registers, one workgroup per CU.)
+template <int D>
+__global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void f32_out_split_kernel(const FP p) {
+  constexpr int KK = D / 16, OWN = KK / 4;
+  constexpr bool EARLY = D == 64;   // the rows of the slot part are under way during the window; wider ones have no room for them
+  __shared__ f32x4 lds[12 * OWN > 20 ? 12 * OWN : 20][64];
+  __shared__ f32x4 stat[4][16];
+  f32x4(*const As)[64] = lds;                                        // [row block][lane]
+  f32x4(*const Ws)[4][64] = reinterpret_cast<f32x4(*)[4][64]>(lds + 4);   // [row block][wave][lane]
+  f32x4(*const Os)[3][OWN][64] = reinterpret_cast<f32x4(*)[3][OWN][64]>(lds);   // [owner][other wave][piece][lane]
+  const int lane = threadIdx.x & 63, l16 = lane & 15, qd = lane >> 4, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int unit = blockIdx.x;
+  const int gq = unit % p.NG; unit /= p.NG;
+  const int sub = unit & 3; unit >>= 2;
+  const int h = unit % p.H, chunk = unit / p.H, hq = h * p.NG + gq;
+  const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
+  const int bos = p.cu[n], eos = p.cu[n + 1];
+  const int cb = bos + it * BT, rows = min(BT, eos - cb);
+  if (16 * sub >= rows) return;
+  const int t0 = cb + 16 * sub, t = t0 + l16, tq = min(t, eos - 1);
+  const int64_t ch = (int64_t)chunk * p.H + h;
+  const float* gcb = p.gc + ((int64_t)cb * p.H + h) * MS;
+  const int gs = p.H * MS, base = it * BT - p.shift;
+  auto src = [&](int j) { return bos + max(0, min(base + j, eos - bos - 1)); };
+  auto live = [&](int j) { return base + j >= 0 && j < rows ? 1.f : 0.f; };
+  struct Rows { f32x4 a[KK]; };
+  struct Cols { float a[4][KK]; };
+  auto fetch = [&](const float* x) {
+    Rows k;
+#pragma unroll
+    for (int c = 0; c < KK; ++c) k.a[c] = ld4(x + 16 * c + 4 * qd);
+    return k;
+  };
+  auto fetch_cols = [&](auto row) {
+    Cols v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float* x = row(r) + l16;
+#pragma unroll
+      for (int c = 0; c < KK; ++c) v.a[r][c] = x[16 * c];
+    }
+    return v;
+  };
+  auto scores = [&](const Rows& k, const Rows& q) {
+    f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < KK; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        acc0 = mfma4(k.a[c][e], q.a[c][e] * p.scale, acc0);
+        acc1 = mfma4(k.a[c][e + 1], q.a[c][e + 1] * p.scale, acc1);
+      }
+    return acc0 + acc1;
+  };
+  f32x4 O[KK];
+#pragma unroll
+  for (int c = 0; c < KK; ++c) O[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  auto read = [&](const Cols& v, const f32x4& x) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int c = 0; c < KK; ++c) O[c] = mfma4(v.a[r][c], x[r], O[c]);
+  };
+  auto of_row = [&](const f32x4& x, int jj) { return __shfl(jj & 2 ? (jj & 1 ? x[3] : x[2]) : (jj & 1 ? x[1] : x[0]), 16 * (jj >> 2) + l16, 64); };
+
+  // ---- operands ----------------------------------------------------------------------------------------------------
+  auto krow = [&](int kb) { return p.k_swa + ((int64_t)max(bos, min(kb + l16, eos - 1)) * p.H + h) * D; };
+  const Rows q = fetch(p.q_swa + ((int64_t)tq * p.HQ + hq) * D);
+  Rows kr = fetch(krow(t0 - 16 * w));
+  Rows qg, hk, kg;
+  auto slot_rows = [&] {
+    qg = fetch(p.q_gsa + ((int64_t)tq * p.HQ + hq) * D);
+    hk = fetch(p.hkc + (ch * MS + 16 * w + l16) * D);
+    kg = fetch(p.k_gsa + ((int64_t)src(16 * w + l16) * p.H + h) * D);
+  };
+  const int last = min(16 * sub + 15, rows - 1), ref = max(16 * sub - 1, 0), m4 = 16 * w + 4 * qd, m1 = 16 * w + l16;
+  const f32x4 gi = ld4(gcb + (int64_t)(tq - cb) * gs + m4);
+  f32x4 gr = ld4(gcb + (int64_t)ref * gs + m4);
+  float ga = gcb[(int64_t)ref * gs + m1];
+  const float gl = gcb[(int64_t)last * gs + m1];
+  // strengths and gate sums of the chunk's rows: a slot per lane for the logits (here), a row per lane for the weights (later)
+  float sa[4][4], gv[4][4];
+  f32x4 sw[4], gw[4];
+#pragma unroll
+  for (int J = 0; J < 4; ++J) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = 16 * J + 4 * qd + r;
+      sa[J][r] = p.s[((int64_t)src(j) * p.H + h) * MS + m1];
+      gv[J][r] = gcb[(int64_t)min(j, rows - 1) * gs + m1];
+    }
+  }
+  if constexpr (EARLY) slot_rows();
+  if (!sub) {
+    gr = (f32x4){0.f, 0.f, 0.f, 0.f};
+    ga = 0.f;
+  }
+
+  // ---- window: every fourth block of 16 keys, newest first.  A query may meet no key here: what it does not see counts 0,
+  // whatever its maximum --------------------------------------------------------------------------------------------
+  const int lo = p.wl < 0 ? bos : max(bos, t0 - p.wl), mylo = p.wl < 0 ? bos : max(bos, t - p.wl);
+  float mw = -INFINITY, lw = 0.f;
+  for (int kb = t0 - 16 * w; kb > lo - 16; kb -= 64) {
+    const Cols vc = fetch_cols([&](int r) { return p.v + ((int64_t)max(bos, min(kb + 4 * qd + r, eos - 1)) * p.H + h) * D; });
+    const Rows kn = fetch(krow(kb - 64));
+    f32x4 s = scores(kr, q);
+    kr = kn;
+    float mx = -INFINITY;
+    bool seen[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = kb + 4 * qd + r;
+      seen[r] = j <= tq && j >= mylo;
+      mx = fmaxf(mx, seen[r] ? s[r] : -INFINITY);
+    }
+    mx = rows_max(mx);
+    const float mn = fmaxf(mw, mx);
+    if (__any(mn != mw)) {
+      const float alpha = mn == mw ? 1.f : exp_f32(mw - mn);
+      lw *= alpha;
+#pragma unroll
+      for (int c = 0; c < KK; ++c) O[c] *= alpha;
+      mw = mn;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      s[r] = seen[r] ? exp_f32(s[r] - mw) : 0.f;
+      lw += s[r];
+    }
+    read(vc, s);
+  }
+  lw = rows_sum(lw);
+
+  // ---- slot logits L[m][query], m = 16 w + 4 (l/16) + r ------------------------------------------------------------
+  if constexpr (!EARLY) slot_rows();
+#pragma unroll
+  for (int J = 0; J < 4; ++J) {
+    const int j = 16 * J + l16;
+    sw[J] = ld4(p.s + ((int64_t)src(j) * p.H + h) * MS + m4);
+    gw[J] = ld4(gcb + (int64_t)min(j, rows - 1) * gs + m4);
+  }
+  f32x4 L = scores(hk, qg), L2 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int r = 0; r < 4; ++r) L[r] *= exp_f32(gi[r]);
+  if (w <= sub) {
+    f32x4 A = scores(kg, qg);
+    if (w == sub)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * qd + r > l16) A[r] = 0.f;
+    As[w][lane] = A;
+  }
+  __syncthreads();
+  const bool pairwise = __any(ga - gl > GROWTH_MAX);
+  const int fast = pairwise ? sub : sub + 1;   // row blocks whose decays are factored
+#pragma unroll
+  for (int J = 0; J < 4; ++J)
+    if (J < fast) {
+      const f32x4 A = As[J][lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) L2 = mfma4(sa[J][r] * live(16 * J + 4 * qd + r) * exp_f32(ga - gv[J][r]), A[r], L2);
+    }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) L[r] += L2[r] * exp_f32(gi[r] - gr[r]);
+  auto pair_row = [&](int jj, f32x4* sv, f32x4* gj) {
+    const int j = 16 * sub + jj;
+    *sv = ld4(p.s + ((int64_t)src(j) * p.H + h) * MS + m4);
+    *gj = ld4(gcb + (int64_t)j * gs + m4);
+    return live(j) != 0.f;
+  };
+  if (pairwise) {
+    const f32x4 A = As[sub][lane];
+    for (int jj = 0; jj < rows - 16 * sub && jj < 16; ++jj) {
+      const float a = of_row(A, jj);
+      f32x4 sv, gj;
+      if (!pair_row(jj, &sv, &gj)) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (jj <= l16) L[r] += a * sv[r] * exp_f32(gi[r] - gj[r]);
+    }
+  }
+
+  // ---- softmax over this wave's slots and keys, its slots' read, the weights that its slots give the chunk's rows ------
+  float mg = rows_max(fmaxf(fmaxf(L[0], L[1]), fmaxf(L[2], L[3]))), lg = 0.f;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    L[r] = exp_f32(L[r] - mg);
+    lg += L[r];
+  }
+  lg = rows_sum(lg);
+  const float mt = fmaxf(mg, mw), eg = exp_f32(mg - mt), ew = exp_f32(mw - mt);
+#pragma unroll
+  for (int c = 0; c < KK; ++c) O[c] *= ew;
+  f32x4 wr;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    L[r] *= eg;
+    wr[r] = L[r] * exp_f32(gi[r]);
+    L2[r] = L[r] * exp_f32(gi[r] - gr[r]);
+  }
+#pragma unroll
+  for (int J = 0; J < 4; ++J)
+    if (J < fast) {
+      f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x = mfma4(sw[J][r] * live(16 * J + l16) * exp_f32(gr[r] - gw[J][r]), L2[r], x);
+      Ws[J][w][lane] = x;
+    }
+  if (pairwise) {
+    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+    for (int jj = 0; jj < rows - 16 * sub && jj < 16; ++jj) {
+      f32x4 sv, gj;
+      if (!pair_row(jj, &sv, &gj)) continue;
+      float y = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (jj <= l16) y += L[r] * sv[r] * exp_f32(gi[r] - gj[r]);
+      y = rows_sum(y);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (jj == 4 * qd + r) x[r] = y;
+    }
+    Ws[sub][w][lane] = x;
+  }
+  if (qd == 0) stat[w][l16] = (f32x4){mw, lw, mg, lg};
+  read(fetch_cols([&](int r) { return p.hvc + (ch * MS + 16 * w + 4 * qd + r) * D; }), wr);
+  const Cols vj = fetch_cols([&](int r) { return p.v + ((int64_t)src(16 * w + 4 * qd + r) * p.H + h) * D; });
+  __syncthreads();
+
+  // ---- the four softmaxes as one -----------------------------------------------------------------------------------
+  f32x4 st[4];
+  float MW = -INFINITY, LW = 0.f, MG = -INFINITY, LG = 0.f;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    st[x] = stat[x][l16];
+    MW = fmaxf(MW, st[x][0]);
+    MG = fmaxf(MG, st[x][2]);
+  }
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    LW += st[x][1] * exp_f32(st[x][0] - MW);
+    LG += st[x][3] * exp_f32(st[x][2] - MG);
+  }
+  const float MT = fmaxf(MG, MW), inv = 1.f / (LG * exp_f32(MG - MT) + LW * exp_f32(MW - MT));
+  float part[4];   // wave x's outputs and weights are relative to its own maximum
+#pragma unroll
+  for (int x = 0; x < 4; ++x) part[x] = exp_f32(fmaxf(st[x][2], st[x][0]) - MT) * inv;
+  const float mine = exp_f32(mt - MT) * inv;
+#pragma unroll
+  for (int c = 0; c < KK; ++c) O[c] *= mine;
+  if (w <= sub) {
+    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int y = 0; y < 4; ++y) x += Ws[w][y][lane] * part[y];
+    if (w == sub)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * qd + r > l16) x[r] = 0.f;
+    read(vj, x);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < KK; ++c)   // (unrolled over all pieces: O is indexed by constants only)
+    if (c / OWN != w) Os[c / OWN][(w - c / OWN - 1) & 3][c % OWN][lane] = O[c];
+  __syncthreads();
+  f32x4 out[OWN];
+#pragma unroll
+  for (int c = 0; c < KK; ++c)
+    if (c / OWN == w) out[c % OWN] = O[c];
+  float z = 0.f;   // NaN if an output is not finite
+#pragma unroll
+  for (int c = 0; c < OWN; ++c) {
+    out[c] += Os[w][0][c][lane] + Os[w][1][c][lane] + Os[w][2][c][lane];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) z = fmaf(out[c][e], 0.f, z);
+  }
+  if (__syncthreads_or(t < eos && z != 0.f)) {
+    if (w == 0) f32_out_rows<D, true>(p, chunk, h, gq, sub);
+    return;
+  }
+  if (t >= eos) return;
+  if (w == 0 && qd == 0) {
+    if (p.lse_gsa) p.lse_gsa[(int64_t)t * p.HQ + hq] = MG + logf(LG);
+    if (p.lse_swa) p.lse_swa[(int64_t)t * p.HQ + hq] = MW + logf(LW);
+  }
+#pragma unroll
+  for (int c = 0; c < OWN; ++c) *reinterpret_cast<f32x4*>(p.o + ((int64_t)t * p.HQ + hq) * D + 16 * (w * OWN + c) + 4 * qd) = out[c];
+}
+
 template <int D>
 int run(const FP& p, int phase, hipStream_t st) {
   if (phase != 2) {
@@ -474,7 +771,12 @@ int run(const FP& p, int phase, hipStream_t st) {
   if (phase != 1) {
     // Workgroups of four waves (neighbouring units share keys through L1) once there are four per CU, of one wave before.
     const int64_t units = (int64_t)p.NT * p.H * 4 * p.NG;
-    if (units >= 1024) hipLaunchKernelGGL((f32_out_kernel<D, 4>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, st, p);
+    // Four waves per unit up to two such workgroups per CU (kernel, a wave / four waves per unit): W = 64, 32 units 22.8 / 12.3,
+    // 256 units 23.8 / 12.8, 512 units 26.4 / 20.7, 1024 units 28.1 / 36.0 us (heads of 64); 512 units of 128 36.6 / 26.8,
+    // 1024 42.5 / 49.2; 512 of 256 68.7 / 63.8, 1024 72.8 / 120.9.  The rows of the chunk and their decays are worked off once
+    // more per wave, so the split costs where the CUs are full anyway.
+    if (units <= 512) hipLaunchKernelGGL((f32_out_split_kernel<D>), dim3((unsigned)units), dim3(256), 0, st, p);
+    else if (units >= 1024) hipLaunchKernelGGL((f32_out_kernel<D, 4>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, st, p);
     else hipLaunchKernelGGL((f32_out_kernel<D, 1>), dim3((unsigned)units), dim3(64), 0, st, p);
     NHA_CHECK_LAUNCH("nha_prefill_fwd(fp32 output pass)");
   }

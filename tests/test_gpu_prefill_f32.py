@@ -127,3 +127,29 @@ def test_f32_operands_off_a_16_byte_boundary(name):
     if name in ("g", "h0k"):                              # single floats in both
         want = fast
     assert all(torch.equal(x, y) for x, y in zip(flat(call(None)), want))
+
+
+@pytest.mark.parametrize("T,D,HQ,H,wl,shift,mean", [(1, 64, 4, 4, 0, 0, 0.0), (17, 64, 6, 2, 63, 64, 0.0), (200, 64, 4, 4, -1, 16, -8.0),
+                                                    (79, 128, 5, 1, 16, 0, 0.0), (145, 256, 2, 2, 100, 3, -4.0)])
+@pytest.mark.parametrize("bad", [None, "v", "k_swa", "s"])
+def test_f32_four_waves_or_one_per_unit(T, D, HQ, H, wl, shift, mean, bad):
+    """A sequence alone (units of 16 rows and a head below 512: four waves each) and the same one many times over (one wave
+    each), against the oracle; with a row of NaN in `bad`, the outputs that are finite in the recurrence are finite."""
+    from nha_amd import chunk_nha
+    from oracle import nha_ref as R
+    from tests.test_gpu_prefill import KEYS
+    from tests.util import assert_close
+    d = prefill_inputs(T + D, 1, T, HQ, H, D, D, 64, dtype=F32, qk_scale=0.5, gate_div=1.0, gate_mean=mean, with_state=True)
+    if bad:
+        d[bad][:, T // 2] = float("nan")
+    ref = R.prefill_ref(*[d[k] for k in KEYS], window_size_left=wl, gsa_kv_shift=shift, initial_state=d["h0"])[:3]
+    units = (T + 63) // 64 * 4 * HQ
+    for B in (1, 512 // units + 1):
+        assert (B * units <= 512) == (B == 1)
+        out = chunk_nha(*[d[k].cuda().expand(B, -1, -1, -1) for k in KEYS], window_size_left=wl, window_size_right=0, gsa_kv_shift=shift,
+                        initial_state=tuple(x.cuda().expand(B, -1, -1, -1) for x in d["h0"]))
+        for what, got, want in zip(("o", "lse_swa", "lse_gsa"), out, ref):
+            assert torch.equal(got.nan_to_num(7.0), got[:1].nan_to_num(7.0).expand_as(got))      # every copy the same
+            got, want = got[:1].cpu(), want.reshape(got[:1].shape)
+            assert torch.equal(got.isfinite(), want.isfinite()), (what, B)
+            assert_close(what, got.masked_fill(~got.isfinite(), 0), want.masked_fill(~want.isfinite(), 0), F32)
