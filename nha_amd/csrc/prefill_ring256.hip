@@ -7,8 +7,7 @@
 //  * One workgroup = NCH consecutive 64-row chunks of a sequence for one query head, 4 NCH waves of 16 query
 //    rows: the accumulators of 16 rows x 256 columns are 64 registers, those of 32 rows would not leave room
 //    for the fragments.  Launched with NCH = 2: the two chunks walk one window (20 units at a window of 512
-//    where two workgroups of one chunk fetch 18 each) with two waves per SIMD; the slot branch, whose tiles
-//    and tables are one chunk's, runs chunk by chunk.
+//    where two workgroups of one chunk fetch 18 each) with two waves per SIMD.
 //  * A unit of 32 keys is 16 KB of K and 16 KB of V.  K and V units live in two rings of three buffers
 //    with their own schedules: iteration u forms the scores of unit u + 1 and the products of unit u, so
 //    after its barrier the K buffer of unit u + 1 and the V buffer of unit u - 1 are free and take K of
@@ -16,11 +15,12 @@
 //  * Fragments are read from LDS a few matrix instructions before their use and not earlier: sixteen K
 //    and sixteen V fragments held at once (128 registers) would push the accumulators out of the
 //    register file.
-//  * The slot-branch operands (four 64 x 256 tiles, 128 KB) do not fit beside the rings: they pass
-//    through the ring buffers.  The two halves of the chunk-start k-state and the first half of the
-//    chunk's k_gsa rows are requested into the K buffers the last iterations of the loop retire, the
-//    second half of the rows into the V buffer the last iteration retires, the halves of the v-state after
-//    the loop; the chunk's v rows replace the k-state once the slot logits are formed.
+//  * The slot branch passes its tiles (k-state, k_gsa rows, v-state, v rows: 32 KB each a chunk) through four ring buffers, one
+//    kind at a time for both chunks together, so that all eight waves work on their own rows; the second chunk's decay tables
+//    take the two buffers left.  The k-states are requested into the buffers that the last iterations of the loop retire, every
+//    further tile when all waves are done with the one before, and what needs no tile (tables, softmax, weights) is computed
+//    while it is on its way.  (Chunk by chunk, with half of the waves idle, the branch took 34 of a workgroup's 100 thousand
+//    cycles, now 21: 213 -> 205 us, 93.0 -> 89.5.)
 //  * The softmax reference of a row is fixed by the prologue (the chunk's own keys): rescaling 64
 //    accumulator registers inside the loop costs the loop its registers whether or not the branch is
 //    taken.  A unit whose maximum tops the reference by 2^96 hands the wave's 16 rows to the exact pass
@@ -157,20 +157,12 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     for (int i = 0; i < LPB; ++i) g2l16(src, uoff[i], boff[i] + C::RING_V + slot_off);
   };
 
-  // The slot branch runs chunk by chunk (its tables and tiles are one chunk's): cc is the chunk it is at, and these
-  // are that chunk's first row whose source token exists, its number of rows and the source token of its row 0
-  int cc = 0;
-  int vlo = (p.shift - it * BT) < 0 ? 0 : (p.shift - it * BT);
-  int rows_c = rows_wg < BT ? rows_wg : BT;
-  int grow_s = c0 - p.shift;
-  uint32_t gco = C::GC;   // where that chunk's gate cumsums lie
   auto tok_from = [&](int gs, int r) {   // source token of row r of a chunk whose row 0 has source token gs, kept inside the sequence
     int t = gs + r;
     t = t < bos ? bos : t;
     t = t < eos ? t : eos - 1;
     return t - bos;
   };
-  auto tok = [&](int r) { return tok_from(grow_s, r); };   // rows outside [vlo, rows_c) carry no weight
   // gate cumsums of chunk c of the workgroup (16 blocks of 4 rows; rows past the chunk's last were never written by the
   // state pass and stay unused) and the s rows of its source tokens
   auto issue_gc = [&](int c_, uint32_t dst) {
@@ -192,14 +184,18 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     }
   };
 
-  auto gc_at = [&](int j, int m) -> const lfloat* { return (const lfloat*)(lds + gco + j * 256 + (((m >> 2) ^ (j & 15)) * 16) + (m & 3) * 4); };
+  auto gc_at = [&](uint32_t gco, int j, int m) -> const lfloat* { return (const lfloat*)(lds + gco + j * 256 + (((m >> 2) ^ (j & 15)) * 16) + (m & 3) * 4); };
   auto s_at = [&](int j, int m) -> const lbf16* { return (const lbf16*)(lds + C::SS + j * 128 + (((m >> 3) ^ (j & 7)) * 16) + (m & 7) * 2); };
   // decay tables E_Q[j][m] = s_j[m] exp(min(gr_Q[m] - gc_j[m], DECAY_CLAMP)) for the rows j of the 16-row
   // blocks jb <= Q, zero elsewhere (gr_Q: gate cumsum of the row before sub-block Q, 0 for Q = 0); rows
   // whose source token does not exist carry no weight.  32-row units (64 columns) in blocks of 16 rows x 32
   // columns, two planes of 32-byte rows each, which is what the transposing read takes:
   // E_0 -> unit 0, E_1 -> 1, E_2 -> 2,3, E_3 -> 4,5; a thread makes 8 consecutive slots of a row.
-  auto build_decay_tables = [&]() {
+  // (of chunk c_ of the workgroup, from its gate cumsums at gco and the s rows at SS, to two places)
+  auto build_decay_tables = [&](int c_, uint32_t gco, uint32_t to03, uint32_t to45) {
+    // first row whose source token exists, number of rows; rows outside carry no weight
+    const int vlo = (p.shift - (it + c_) * BT) < 0 ? 0 : (p.shift - (it + c_) * BT);
+    const int rows_c = rows_wg - c_ * BT < BT ? rows_wg - c_ * BT : BT;
     for (int item = tid; item < 6 * 256; item += 64 * NW) {
       const int U = item >> 8, r32 = (item >> 3) & 31, m = (item & 7) * 8;
       const int Qt = U == 0 ? 0 : U == 1 ? 1 : U < 4 ? 2 : 3;
@@ -213,15 +209,15 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
         f32x4 gv[2], gr[2];
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
-          gv[hh] = *reinterpret_cast<const NHA_LDS f32x4*>(gc_at(j, m + 4 * hh));
+          gv[hh] = *reinterpret_cast<const NHA_LDS f32x4*>(gc_at(gco, j, m + 4 * hh));
           gr[hh] = (f32x4){0.f, 0.f, 0.f, 0.f};
-          if (Qt > 0) gr[hh] = *reinterpret_cast<const NHA_LDS f32x4*>(gc_at(16 * Qt - 1, m + 4 * hh));
+          if (Qt > 0) gr[hh] = *reinterpret_cast<const NHA_LDS f32x4*>(gc_at(gco, 16 * Qt - 1, m + 4 * hh));
         }
         const bf16x8 sv = *reinterpret_cast<const NHA_LDS bf16x8*>(s_at(j, m));
 #pragma unroll
         for (int e = 0; e < 8; ++e) out[e] = (__bf16)((float)sv[e] * fexp(fminf(gr[e >> 2][e & 3] - gv[e >> 2][e & 3], DECAY_CLAMP)));
       }
-      *reinterpret_cast<NHA_LDS bf16x8*>(lds + C::ETAB + U * 4096 + (r32 >> 4) * 2048 + (m >> 5) * 1024 + ((m >> 4) & 1) * 512 + (r32 & 15) * 32 + (m & 15) * 2) = out;
+      *reinterpret_cast<NHA_LDS bf16x8*>(lds + (U < 4 ? to03 : to45 - 4 * 4096) + U * 4096 + (r32 >> 4) * 2048 + (m >> 5) * 1024 + ((m >> 4) & 1) * 512 + (r32 & 15) * 32 + (m & 15) * 2) = out;
     }
   };
   // ---- requests: the gate blocks (the decay tables are built from them while the units are still on their
@@ -229,7 +225,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   //      query fragments -------------------------------------
   const bool second = rows_wg > BT;   // the workgroup has a second chunk
   issue_gc(0, C::GC);
-  issue_s(grow_s);
+  issue_s(c0 - p.shift);
   if (NCH == 2 && second) issue_gc(1, C::GC2);
   issue_k(0);
   issue_v(0);
@@ -252,7 +248,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   if (2 < nunits) wait_vm<5 * LPB + KS>();
   else wait_vm<4 * LPB + KS>();
   lds_barrier();
-  build_decay_tables();
+  build_decay_tables(0, C::GC, C::ETAB, C::ETAB + 4 * 4096);
   NHA_FENCE();
   {
 #pragma unroll
@@ -381,18 +377,22 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     return P;
   };
 
-  // The slot-branch tiles (k-state, k_gsa rows, v-state as two 32-row halves each) take ring buffers as the
-  // window loop retires them: with at least five units the last three K buffers and the last V buffer to
-  // come free receive four of the six halves while the loop still runs (a half is as many loads as a
-  // unit buffer, so the in-flight counts of the loop stay what they are); the two v-state halves follow
-  // after the loop, and shorter windows request everything then.
+  // The slot branch takes four tiles of 64 rows per chunk (k-state, k_gsa rows, v-state, v rows), one after the other and those of
+  // all NCH chunks together, each as two 32-row halves in ring buffers.  With at least five units the buffers that the window
+  // loop retires last take the halves of the k-states while it still runs (a half is as many loads as a unit buffer, so the
+  // in-flight counts of the loop stay what they are); shorter windows request them afterwards.
   const bf16_t* const t_kg = p.k_gsa + ((int64_t)bos * H + h) * D;
-  auto issue_ta = [&](uint32_t off, int half) { issue_buffer(off, p.hkT + (cg + (int64_t)cc * H) * MS * D, (uint32_t)D, [=](int r) { return 32 * half + r; }); };
-  auto issue_tb = [&](uint32_t off, int half) { issue_buffer(off, t_kg, (uint32_t)(H * D), [&](int r) { return tok(32 * half + r); }); };
-  auto issue_tc = [&](uint32_t off, int half) { issue_buffer(off, p.hvc + (cg + (int64_t)cc * H) * MS * D, (uint32_t)D, [=](int r) { return 32 * half + r; }); };
+  auto issue_ta = [&](uint32_t off, int c_, int half) { issue_buffer(off, p.hkT + (cg + (int64_t)c_ * H) * MS * D, (uint32_t)D, [=](int r) { return 32 * half + r; }); };
+  auto issue_tb = [&](uint32_t off, int c_, int half, const bf16_t* src) {   // rows of the source tokens of a chunk
+    issue_buffer(off, src, (uint32_t)(H * D), [&](int r) { return tok_from(c0 + c_ * BT - p.shift, 32 * half + r); });
+  };
+  auto issue_tc = [&](uint32_t off, int c_, int half) { issue_buffer(off, p.hvc + (cg + (int64_t)c_ * H) * MS * D, (uint32_t)D, [=](int r) { return 32 * half + r; }); };
   const bool early = nunits >= 5;
-  uint32_t oA0 = C::RING_K, oA1 = C::RING_K + UB, oB0 = C::RING_K + 2 * UB, oB1 = C::RING_V;   // where the halves lie
-  uint32_t oC0 = C::RING_V + UB, oC1 = C::RING_V + 2 * UB;
+  const int last_c = NCH == 2 && second ? 1 : 0;   // (a workgroup of one chunk requests that chunk's twice)
+  uint32_t oT[NCH][2];   // where the halves of a chunk's tile lie: the K buffers, and a V buffer
+  oT[0][0] = C::RING_K, oT[0][1] = C::RING_K + UB;
+  if constexpr (NCH == 2) oT[1][0] = C::RING_K + 2 * UB, oT[1][1] = C::RING_V;
+  uint32_t oE2 = C::RING_V + UB, oE2b = C::RING_V + 2 * UB;   // the two buffers left, which take the second chunk's decay tables
   // ring positions as rotating buffer offsets: s0 = buffer of unit u, s1 of unit u+1, s2 of unit u+2
   uint32_t s0 = 0, s1 = UB, s2 = 2 * UB;
   for (int u = 0; u + 1 < nunits; ++u) {
@@ -431,23 +431,23 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     lds_barrier();
     if (u + 2 < nunits) {
       issue_v_fast(u + 2, s2);
-    } else if (early) {
-      oB1 = C::RING_V + s2;
-      issue_tb(oB1, 1);
+    } else if (NCH == 2 && early) {
+      oT[NCH - 1][1] = C::RING_V + s2;
+      issue_ta(oT[NCH - 1][1], last_c, 1);
     }
     if (u + 4 < nunits) {
       issue_k_fast(u + 4, s1);   // unit u+4 takes the buffer of unit u+1
     } else if (early) {
       const uint32_t off = C::RING_K + s1;
       if (u + 4 == nunits) {
-        oA0 = off;
-        issue_ta(off, 0);
+        oT[0][0] = off;
+        issue_ta(off, 0, 0);
       } else if (u + 3 == nunits) {
-        oA1 = off;
-        issue_ta(off, 1);
-      } else {
-        oB0 = off;
-        issue_tb(off, 0);
+        oT[0][1] = off;
+        issue_ta(off, 0, 1);
+      } else if (NCH == 2) {
+        oT[NCH - 1][0] = off;
+        issue_ta(off, last_c, 0);
       }
     }
     NHA_FENCE();
@@ -516,215 +516,201 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   }
 
   // ================= slot branch, folded into the running softmax =================================
-  // One chunk at a time: the tables and tiles in LDS are one chunk's.  Every wave requests its share of the loads,
-  // helps with the tables and keeps the barriers; the products are those of the waves whose rows the chunk holds.
+  // Every wave its own rows, the waves of both chunks side by side; the next tile is requested when every wave is done with
+  // the one before, and what needs no tile is computed while it is on its way.
   // every request of this wave has landed, every wave is done with the rings
   wait_vm<0>();
   lds_barrier();
+  if (!early) {
+    issue_ta(oT[0][0], 0, 0);
+    issue_ta(oT[0][1], 0, 1);
+    if (NCH == 2 && second) {
+      issue_ta(oT[NCH - 1][0], NCH - 1, 0);
+      issue_ta(oT[NCH - 1][1], NCH - 1, 1);
+    }
+  } else {
+    oE2 = C::RING_V + s2, oE2b = C::RING_V + s0;   // (after the loop's last rotation)
+  }
   // the window's own log-sum-exp, before the slots join the running softmax
   if (p.lse_swa && kb == 0 && irow < rows) p.lse_swa[(int64_t)(c0 + yrow) * HQ + hq] = (__builtin_amdgcn_logf(Lw[0]) - nm) * LN2;
-  float psum = 0.f;
-#pragma unroll 1
-  for (cc = 0; cc < NCH; ++cc) {
-    if (cc == 0) {
-      if (!early) {
-        issue_ta(oA0, 0);
-        issue_ta(oA1, 1);
-        issue_tb(oB0, 0);
-        issue_tb(oB1, 1);
-      } else {   // the V buffers of the last two units (s0, s2 after the loop's last rotation) are the free ones
-        oC0 = C::RING_V + s2;
-        oC1 = C::RING_V + s0;
+  auto issue_all = [&](auto issue) {
+#pragma unroll
+    for (int c_ = 0; c_ < NCH; ++c_)
+      if (c_ == 0 || second) {
+        issue(oT[c_][0], c_, 0);
+        issue(oT[c_][1], c_, 1);
       }
-      issue_tc(oC0, 0);
-      issue_tc(oC1, 1);
-    } else {
-      // the second chunk: its tiles are requested once the first chunk is done with the buffers, and its decay tables
-      // built, from the gate blocks that came in during the window loop, once the first chunk is done with the tables
-      if (!second) break;
-      lds_barrier();
-      vlo = (p.shift - (it + 1) * BT) < 0 ? 0 : (p.shift - (it + 1) * BT);
-      rows_c = rows_wg - BT;
-      grow_s = c0 + BT - p.shift;
-      gco = C::GC2;
-      // the tiles go where the first chunk's were; the k_gsa rows are already on their way (requested when the first
-      // chunk had read its own)
-      issue_ta(oA0, 0);
-      issue_ta(oA1, 1);
-      issue_tc(oC0, 0);
-      issue_tc(oC1, 1);
-      build_decay_tables();
-    }
-    const bool mine = ch == cc;
-
-    // k-state and k_gsa rows have landed (the two v-state halves may still fly)
-    wait_vm<2 * LPB>();
-    __syncthreads();
-
-    const int etu = Q < 2 ? Q : 2 * Q - 2;   // first table unit of this wave's sub-block
-    // E_Q transposed: rows = slots 16 mb + l16, contraction over the tokens 32 pr + {4 kb + e, 16 + 4 kb + e - 4}
-    auto etab_tr = [&](int pr, int mb) -> bf16x8 {
-      const lbyte* pa = lds + C::ETAB + (etu + pr) * 4096 + (mb >> 1) * 1024 + (mb & 1) * 512 + (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
-      struct { s16x4 a, b; } t;
-      t.a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)pa);
-      t.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)(pa + 2048));
-      return __builtin_bit_cast(bf16x8, t);
-    };
-    // E_Q by rows: row = token 16 jb + l16, contraction over the slots 32 pr + {4 kb + e, 16 + 4 kb + e - 4}
-    auto etab_row = [&](int jb, int pr) -> bf16x8 {
-      const lbyte* pa = lds + C::ETAB + (etu + (jb >> 1)) * 4096 + (jb & 1) * 2048 + pr * 1024 + l16 * 32 + 8 * kb;
-      struct { bf16x4 a, b; } t;
-      t.a = *reinterpret_cast<const NHA_LDS bf16x4*>(pa);
-      t.b = *reinterpret_cast<const NHA_LDS bf16x4*>(pa + 512);
-      return __builtin_bit_cast(bf16x8, t);
-    };
-
-    // inter-chunk slot logits: okT[m][i] = sum_d hkT[m][d] q[i][d]
-    f32x4 ok[4];
-    if (mine) {
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) ok[mb] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int mb = 0; mb < 4; ++mb) ok[mb] = mfma16(kfrag(((mb >> 1) ? oA1 : oA0), mb & 1, ks), qg[ks], ok[mb]);
-    }
-    // every wave is done with the k-state tile: the v rows take its buffers and land during what follows
+  };
+  auto landed = [&]() {
+    wait_vm<0>();
     lds_barrier();
+  };
+  if (!early) landed();
+  const bool mine = ch == 0 || second;
+  const uint32_t t0_ = oT[0][0], t1_ = oT[0][1];
+  const uint32_t tile0 = NCH == 2 && ch ? oT[NCH - 1][0] : t0_, tile1 = NCH == 2 && ch ? oT[NCH - 1][1] : t1_;   // halves of the wave's tile
+  const uint32_t gco = NCH == 2 && ch ? C::GC2 : C::GC;
+  // first table unit of this wave's sub-block (units 0 .. 3 lie in one piece, 4 and 5 in another)
+  const uint32_t etab = Q == 3 ? (NCH == 2 && ch ? oE2b : C::ETAB + 4 * 4096) : (NCH == 2 && ch ? oE2 : C::ETAB) + (Q < 2 ? Q : 2) * 4096;
+  // E_Q transposed: rows = slots 16 mb + l16, contraction over the tokens 32 pr + {4 kb + e, 16 + 4 kb + e - 4}
+  auto etab_tr = [&](int pr, int mb) -> bf16x8 {
+    const lbyte* pa = lds + etab + pr * 4096 + (mb >> 1) * 1024 + (mb & 1) * 512 + (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
+    struct { s16x4 a, b; } t;
+    t.a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)pa);
+    t.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)(pa + 2048));
+    return __builtin_bit_cast(bf16x8, t);
+  };
+  // E_Q by rows: row = token 16 jb + l16, contraction over the slots 32 pr + {4 kb + e, 16 + 4 kb + e - 4}
+  auto etab_row = [&](int jb, int pr) -> bf16x8 {
+    const lbyte* pa = lds + etab + (jb >> 1) * 4096 + (jb & 1) * 2048 + pr * 1024 + l16 * 32 + 8 * kb;
+    struct { bf16x4 a, b; } t;
+    t.a = *reinterpret_cast<const NHA_LDS bf16x4*>(pa);
+    t.b = *reinterpret_cast<const NHA_LDS bf16x4*>(pa + 512);
+    return __builtin_bit_cast(bf16x8, t);
+  };
+
+  // inter-chunk slot logits: okT[m][i] = sum_d hkT[m][d] q[i][d]
+  f32x4 ok[4];
+  if (mine) {
 #pragma unroll
-    for (int half = 0; half < 2; ++half)
-      issue_buffer(half ? oA1 : oA0, vbase, (uint32_t)(H * D), [&](int r) { return tok(32 * half + r); });
-    bf16x8 bp[2], bpr[2];   // slot probabilities x exp(gc_i) and x exp(gc_i - gr), B operands
-    if (mine) {
-      // intra-chunk scores AT[j][i] = sum_d k_gsa[j][d] q[i][d] for row blocks jb <= Q, masked j <= i
-      bf16x8 bA[2];
-      {
-        f32x4 at[4];
+    for (int mb = 0; mb < 4; ++mb) ok[mb] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int jb = 0; jb < 4; ++jb) at[jb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
+      for (int mb = 0; mb < 4; ++mb) ok[mb] = mfma16(kfrag(((mb >> 1) ? tile1 : tile0), mb & 1, ks), qg[ks], ok[mb]);
+  }
+  // every wave is done with the k-states: the k_gsa rows, and meanwhile the second chunk's tables
+  lds_barrier();
+  issue_all([&](uint32_t o, int c_, int half) { issue_tb(o, c_, half, t_kg); });
+  if (NCH == 2 && second) build_decay_tables(1, C::GC2, oE2, oE2b);
+  landed();
+  bf16x8 bA[2];
+  if (mine) {
+    // intra-chunk scores AT[j][i] = sum_d k_gsa[j][d] q[i][d] for row blocks jb <= Q, masked j <= i
+    f32x4 at[4];
 #pragma unroll
-          for (int jb = 0; jb < 4; ++jb)
-            if (jb <= Q) at[jb] = mfma16(kfrag(((jb >> 1) ? oB1 : oB0), jb & 1, ks), qg[ks], at[jb]);
+    for (int jb = 0; jb < 4; ++jb) at[jb] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int jb = 0; jb < 4; ++jb)
-          if (jb == Q) {
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (4 * kb + r > l16) at[jb][r] = 0.f;
-          }
-        bA[0] = pack8(at[0], at[1]);
-        bA[1] = pack8(at[2], at[3]);
+      for (int jb = 0; jb < 4; ++jb)
+        if (jb <= Q) at[jb] = mfma16(kfrag(((jb >> 1) ? tile1 : tile0), jb & 1, ks), qg[ks], at[jb]);
+#pragma unroll
+    for (int jb = 0; jb < 4; ++jb)
+      if (jb == Q) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (4 * kb + r > l16) at[jb][r] = 0.f;
       }
-      // okT_intra[m][i] = sum_j s_j[m] exp(gr[m] - gc_j[m]) AT[j][i]
-      f32x4 oki[4];
+    bA[0] = pack8(at[0], at[1]);
+    bA[1] = pack8(at[2], at[3]);
+  }
+  // done with the k_gsa rows: the v-states, and meanwhile the softmax
+  lds_barrier();
+  issue_all([&](uint32_t o, int c_, int half) { issue_tc(o, c_, half); });
+  float psum = 0.f;
+  bf16x8 bp[2], bpr[2];   // slot probabilities x exp(gc_i) and x exp(gc_i - gr), B operands
+  if (mine) {
+    // okT_intra[m][i] = sum_j s_j[m] exp(gr[m] - gc_j[m]) AT[j][i]
+    f32x4 oki[4];
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        oki[mb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int mb = 0; mb < 4; ++mb) {
+      oki[mb] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int pr = 0; pr < 2; ++pr)
-          if (2 * pr <= Q) oki[mb] = mfma16(etab_tr(pr, mb), bA[pr], oki[mb]);
+      for (int pr = 0; pr < 2; ++pr)
+        if (2 * pr <= Q) oki[mb] = mfma16(etab_tr(pr, mb), bA[pr], oki[mb]);
+    }
+    // combine; the slot logits join the running softmax as one more set of keys
+    const int rref = 16 * Q - 1;
+    f32x4 egi[4], egr[4];   // exp(gc_i[m]) and exp(gc_i[m] - gr[m]) in accumulator layout
+    float xmax = -INFINITY;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
+      const f32x4 gi = *reinterpret_cast<const NHA_LDS f32x4*>(gc_at(gco, irow, 16 * mb + 4 * kb));
+      f32x4 gr4 = (f32x4){0.f, 0.f, 0.f, 0.f};
+      if (Q > 0) gr4 = *reinterpret_cast<const NHA_LDS f32x4*>(gc_at(gco, rref, 16 * mb + 4 * kb));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        egi[mb][r] = fexp(gi[r]);
+        egr[mb][r] = fexp(gi[r] - gr4[r]);
+        ok[mb][r] = (ok[mb][r] * egi[mb][r] + oki[mb][r] * egr[mb][r]) * cs;   // slot logit, log2 units
+        xmax = fmaxf(xmax, ok[mb][r]);
       }
-      // combine; the slot logits join the running softmax as one more set of keys
-      const int rref = 16 * Q - 1;
-      f32x4 egi[4], egr[4];   // exp(gc_i[m]) and exp(gc_i[m] - gr[m]) in accumulator layout
-      float xmax = -INFINITY;
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        const f32x4 gi = *reinterpret_cast<const NHA_LDS f32x4*>(gc_at(irow, 16 * mb + 4 * kb));
-        f32x4 gr4 = (f32x4){0.f, 0.f, 0.f, 0.f};
-        if (Q > 0) gr4 = *reinterpret_cast<const NHA_LDS f32x4*>(gc_at(rref, 16 * mb + 4 * kb));
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          egi[mb][r] = fexp(gi[r]);
-          egr[mb][r] = fexp(gi[r] - gr4[r]);
-          ok[mb][r] = (ok[mb][r] * egi[mb][r] + oki[mb][r] * egr[mb][r]) * cs;   // slot logit, log2 units
-          xmax = fmaxf(xmax, ok[mb][r]);
-        }
-      }
-      const float ms = max_over_rows(xmax);   // the slots' own maximum
-      if (__any(ms + nm > THR)) rescale_acc(fmaxf(ms + nm, 0.f));
-      if (p.lse_gsa) {
-        float pown = 0.f;
-#pragma unroll
-        for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) pown += fexp2(ok[mb][r] - ms);
-        pown += __shfl_xor(pown, 16, 64);
-        pown += __shfl_xor(pown, 32, 64);
-        if (kb == 0 && irow < rows) p.lse_gsa[(int64_t)(c0 + yrow) * HQ + hq] = (__builtin_amdgcn_logf(pown) + ms) * LN2;
-      }
+    }
+    const float ms = max_over_rows(xmax);   // the slots' own maximum
+    if (__any(ms + nm > THR)) rescale_acc(fmaxf(ms + nm, 0.f));
+    if (p.lse_gsa) {
+      float pown = 0.f;
 #pragma unroll
       for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          ok[mb][r] = fexp2(ok[mb][r] + nm);   // unnormalised slot probabilities
-          psum += ok[mb][r];
-        }
-      psum += __shfl_xor(psum, 16, 64);
-      psum += __shfl_xor(psum, 32, 64);
+        for (int r = 0; r < 4; ++r) pown += fexp2(ok[mb][r] - ms);
+      pown += __shfl_xor(pown, 16, 64);
+      pown += __shfl_xor(pown, 32, 64);
+      if (kb == 0 && irow < rows) p.lse_gsa[(int64_t)(c0 + yrow) * HQ + hq] = (__builtin_amdgcn_logf(pown) + ms) * LN2;
+    }
 #pragma unroll
-      for (int pr = 0; pr < 2; ++pr) {
-        f32x4 x0, x1, y0, y1;
+    for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          x0[r] = ok[2 * pr][r] * egi[2 * pr][r];
-          x1[r] = ok[2 * pr + 1][r] * egi[2 * pr + 1][r];
-          y0[r] = ok[2 * pr][r] * egr[2 * pr][r];
-          y1[r] = ok[2 * pr + 1][r] * egr[2 * pr + 1][r];
+      for (int r = 0; r < 4; ++r) {
+        ok[mb][r] = fexp2(ok[mb][r] + nm);   // unnormalised slot probabilities
+        psum += ok[mb][r];
+      }
+    psum += __shfl_xor(psum, 16, 64);
+    psum += __shfl_xor(psum, 32, 64);
+#pragma unroll
+    for (int pr = 0; pr < 2; ++pr) {
+      f32x4 x0, x1, y0, y1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x0[r] = ok[2 * pr][r] * egi[2 * pr][r];
+        x1[r] = ok[2 * pr + 1][r] * egi[2 * pr + 1][r];
+        y0[r] = ok[2 * pr][r] * egr[2 * pr][r];
+        y1[r] = ok[2 * pr + 1][r] * egr[2 * pr + 1][r];
+      }
+      bp[pr] = pack8(x0, x1);
+      bpr[pr] = pack8(y0, y1);
+    }
+  }
+  landed();
+  // slot read, inter-chunk part: O^T[d][i] += sum_m hv[m][d] (p[i][m] exp(gc_i[m]))
+  if (mine) {
+#pragma unroll
+    for (int pr = 0; pr < 2; ++pr)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) O[db] = mfma16(vfrag((pr ? tile1 : tile0), db), bp[pr], O[db]);
+  }
+  // done with the v-states: the v rows, and meanwhile their weights
+  lds_barrier();
+  issue_all([&](uint32_t o, int c_, int half) { issue_tb(o, c_, half, vbase); });
+  bf16x8 bAv[2];
+  if (mine) {
+    // intra-chunk part: AvT[j][i] = sum_m s_j[m] exp(gr[m]-gc_j[m]) (p[i][m] exp(gc_i[m]-gr[m])), j <= i
+    f32x4 av[4];
+#pragma unroll
+    for (int jb = 0; jb < 4; ++jb) {
+      av[jb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      if (jb <= Q) {
+#pragma unroll
+        for (int pr = 0; pr < 2; ++pr) av[jb] = mfma16(etab_row(jb, pr), bpr[pr], av[jb]);
+        if (jb == Q) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (4 * kb + r > l16) av[jb][r] = 0.f;
         }
-        bp[pr] = pack8(x0, x1);
-        bpr[pr] = pack8(y0, y1);
       }
     }
-    // the v-state halves have landed (this wave's part, then everybody's); the v rows behind them may fly
-    wait_vm<2 * LPB>();
-    lds_barrier();
-    // every wave has read the chunk's k_gsa rows: the second chunk's take their buffers now
-    const bool ahead = NCH == 2 && cc == 0 && second;
-    if (ahead) {
+    bAv[0] = pack8(av[0], av[1]);
+    bAv[1] = pack8(av[2], av[3]);
+  }
+  landed();
+  if (mine) {
 #pragma unroll
-      for (int half = 0; half < 2; ++half)
-        issue_buffer(half ? oB1 : oB0, t_kg, (uint32_t)(H * D), [&](int r) { return tok_from(c0 + BT - p.shift, 32 * half + r); });
-    }
-    bf16x8 bAv[2];
-    if (mine) {
-      // slot read, inter-chunk part: O^T[d][i] += sum_m hv[m][d] (p[i][m] exp(gc_i[m]))
+    for (int pr = 0; pr < 2; ++pr)
+      if (2 * pr <= Q) {
 #pragma unroll
-      for (int pr = 0; pr < 2; ++pr)
-#pragma unroll
-        for (int db = 0; db < DB; ++db) O[db] = mfma16(vfrag((pr ? oC1 : oC0), db), bp[pr], O[db]);
-      // intra-chunk part: AvT[j][i] = sum_m s_j[m] exp(gr[m]-gc_j[m]) (p[i][m] exp(gc_i[m]-gr[m])), j <= i
-      f32x4 av[4];
-#pragma unroll
-      for (int jb = 0; jb < 4; ++jb) {
-        av[jb] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        if (jb <= Q) {
-#pragma unroll
-          for (int pr = 0; pr < 2; ++pr) av[jb] = mfma16(etab_row(jb, pr), bpr[pr], av[jb]);
-          if (jb == Q) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (4 * kb + r > l16) av[jb][r] = 0.f;
-          }
-        }
+        for (int db = 0; db < DB; ++db) O[db] = mfma16(vfrag((pr ? tile1 : tile0), db), bAv[pr], O[db]);
       }
-      bAv[0] = pack8(av[0], av[1]);
-      bAv[1] = pack8(av[2], av[3]);
-    }
-    // the v rows have landed (this wave's part, then everybody's); the second chunk's k_gsa rows behind them may fly
-    if (ahead) wait_vm<2 * LPB>();
-    else wait_vm<0>();
-    lds_barrier();
-    if (mine) {
-#pragma unroll
-      for (int pr = 0; pr < 2; ++pr)
-        if (2 * pr <= Q) {
-#pragma unroll
-          for (int db = 0; db < DB; ++db) O[db] = mfma16(vfrag((pr ? oA1 : oA0), db), bAv[pr], O[db]);
-        }
-    }
   }
 
   // ---- epilogue: 16-byte stores (the lanes of an even 16-lane row keep block db, those of the odd
