@@ -12,6 +12,11 @@
 //    with their own schedules: iteration u forms the scores of unit u + 1 and the products of unit u, so
 //    after its barrier the K buffer of unit u + 1 and the V buffer of unit u - 1 are free and take K of
 //    unit u + 4 and V of unit u + 2; both have two iterations to land.
+//    An iteration that does nothing else has its loads between the products and steps two pointers; with each request's
+//    address formed anew it took 2400 cycles, now 2100, 1056 of them matrix instructions (kernel, 32768 tokens packed, 4 heads,
+//    W = 512: 205 -> 198 us; 8 x 2048 tokens 89.5 -> 86.6).
+//  * Query rows go through LDS in whole lines (a fragment as it lies in memory is 16 bytes of 16 rows: 56 cycles a load, a line
+//    load 16), unscaled, the scores taking the scale as they take the reference (198 -> 193 us; 86.6 -> 85.0).
 //  * Fragments are read from LDS a few matrix instructions before their use and not earlier: sixteen K
 //    and sixteen V fragments held at once (128 registers) would push the accumulators out of the
 //    register file.
@@ -28,6 +33,7 @@
 #include "mfma_common.h"
 
 #include <mutex>
+#include <type_traits>
 
 namespace nha {
 namespace {
@@ -127,8 +133,8 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     const int last = eos - 1 - bos;
     return [=](int r) { return key0 + r < last ? key0 + r : last; };
   };
-  auto issue_k = [&](int u) { issue_buffer(C::RING_K + (u % NR) * UB, kbase, (uint32_t)(H * D), unit_row(u)); };
-  auto issue_v = [&](int u) { issue_buffer(C::RING_V + (u % NR) * UB, vbase, (uint32_t)(H * D), unit_row(u)); };
+  auto issue_k = [&](int u, uint32_t slot_off) { issue_buffer(C::RING_K + slot_off, kbase, (uint32_t)(H * D), unit_row(u)); };
+  auto issue_v = [&](int u, uint32_t slot_off) { issue_buffer(C::RING_V + slot_off, vbase, (uint32_t)(H * D), unit_row(u)); };
   // units >= 2 NCH lie wholly before the workgroup's rows (never past eos): fixed per-lane offsets from a wave-uniform row pointer
   uint32_t uoff[LPB], boff[LPB];
 #pragma unroll
@@ -138,24 +144,6 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     uoff[i] = ((uint32_t)(16 * rh + lrow) * (uint32_t)(H * D) + LineTile<D>::load_col(cq, lane)) * 2;
     boff[i] = lds0 + rh * HB + cq * 1024;
   }
-  auto issue_k_fast = [&](int u, uint32_t slot_off) {
-    if (NCH > 1 && u < 2 * NCH) {
-      issue_buffer(C::RING_K + slot_off, kbase, (uint32_t)(H * D), unit_row(u));
-      return;
-    }
-    const bf16_t* src = p.k_swa + (((int64_t)c0 + XB0 - 32 * u) * H + h) * D;
-#pragma unroll
-    for (int i = 0; i < LPB; ++i) g2l16(src, uoff[i], boff[i] + C::RING_K + slot_off);
-  };
-  auto issue_v_fast = [&](int u, uint32_t slot_off) {
-    if (NCH > 1 && u < 2 * NCH) {
-      issue_buffer(C::RING_V + slot_off, vbase, (uint32_t)(H * D), unit_row(u));
-      return;
-    }
-    const bf16_t* src = p.v + (((int64_t)c0 + XB0 - 32 * u) * H + h) * D;
-#pragma unroll
-    for (int i = 0; i < LPB; ++i) g2l16(src, uoff[i], boff[i] + C::RING_V + slot_off);
-  };
 
   auto tok_from = [&](int gs, int r) {   // source token of row r of a chunk whose row 0 has source token gs, kept inside the sequence
     int t = gs + r;
@@ -220,50 +208,35 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
       *reinterpret_cast<NHA_LDS bf16x8*>(lds + (U < 4 ? to03 : to45 - 4 * 4096) + U * 4096 + (r32 >> 4) * 2048 + (m >> 5) * 1024 + ((m >> 4) & 1) * 512 + (r32 & 15) * 32 + (m & 15) * 2) = out;
     }
   };
-  // ---- requests: the gate blocks (the decay tables are built from them while the units are still on their
-  //      way; the second chunk's gate cumsums wait in a place of their own), K and V of the first units, then the
-  //      query fragments -------------------------------------
+  // ---- requests: the gate blocks and the window queries, these through the rings in whole lines (a fragment loaded from global
+  //      memory as it is, 16 bytes of 16 rows, takes three times as long); then K and V of the first units, under way while the
+  //      decay tables are built, and the second chunk's gate cumsums, which wait in a place of their own ------------------
   const bool second = rows_wg > BT;   // the workgroup has a second chunk
   issue_gc(0, C::GC);
   issue_s(c0 - p.shift);
-  if (NCH == 2 && second) issue_gc(1, C::GC2);
-  issue_k(0);
-  issue_v(0);
-  issue_k(1);
-  issue_v(1);
-  if (2 < nunits) issue_k_fast(2, 2 * UB);
-  // window-query fragments, pre-scaled by scale * log2(e)
-  bf16x8 qs[KS];
-  uint4 qraw[KS];
-  {
-    // rows past the end of the sequence read the last row (the number of loads must not depend on the lane:
-    // the wait below counts them) and are zeroed afterwards
-    const bf16_t* qp = p.q_swa + ((int64_t)(c0 + (yrow < rows_wg ? yrow : rows_wg - 1)) * HQ + hq) * D + 8 * kb;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qraw[ks] = *reinterpret_cast<const uint4*>(qp + 32 * ks);
-  }
-  NHA_FENCE();
-  // the gate blocks were requested first: they have landed once no more than the requests made after them
-  // are outstanding (four or five unit buffers and the query loads)
-  if (2 < nunits) wait_vm<5 * LPB + KS>();
-  else wait_vm<4 * LPB + KS>();
+  for (int j = 0; j < NW / 2; ++j)    // rows past the end of the sequence: its last, never stored
+    issue_buffer(j * UB, p.q_swa + ((int64_t)c0 * HQ + hq) * D, (uint32_t)(HQ * D), [&](int r) { return 32 * j + r < rows_wg ? 32 * j + r : rows_wg - 1; });
+  const uint32_t kaddr = LineTile<D>::row_at(lane), vaddr = LineTile<D>::col_at(lane);
+  // row fragment (rows 16 kk + l16 of a buffer, columns 32 ks + 8 kb ..) of a buffer at byte address a
+  auto kfrag = [&](uint32_t a, int kk, int ks) -> bf16x8 {
+    const lbyte* base = lds + (a + kaddr);     // one address per buffer; the fragment is a constant offset from it
+    return *reinterpret_cast<const NHA_LDS bf16x8*>(base + (kk * HB + ks * 1024));
+  };
+  wait_vm<0>();
   lds_barrier();
+  bf16x8 qs[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) qs[ks] = kfrag(wave * HB, 0, ks);
+  lds_barrier();
+  issue_k(0, 0);
+  issue_v(0, 0);
+  issue_k(1, UB);
+  issue_v(1, UB);
+  if (2 < nunits) issue_k(2, 2 * UB);
+  if (NCH == 2 && second) issue_gc(1, C::GC2);
   build_decay_tables(0, C::GC, C::ETAB, C::ETAB + 4 * 4096);
   NHA_FENCE();
-  {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const uint4 x = irow < rows ? qraw[ks] : make_uint4(0, 0, 0, 0);
-      const uint32_t w[4] = {x.x, x.y, x.z, x.w};
-      bf16x8 r;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float f = __uint_as_float((e & 1) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16));
-        r[e] = (__bf16)(f * cs);
-      }
-      qs[ks] = r;
-    }
-  }
 
   // ---- window loop state ------------------------------------------------------------------------
   f32x4 O[DB];
@@ -271,19 +244,12 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   for (int db = 0; db < DB; ++db) O[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
   f32x4 Lw = {0.f, 0.f, 0.f, 0.f};
   float nm = 0.f;                      // minus the running reference maximum, log2 units
-  f32x4 nmv = {0.f, 0.f, 0.f, 0.f};    // nm broadcast: the accumulator the score products start from
   bf16x8 ones;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.0f;
   constexpr float THR = 8.f;           // the reference moves (prologue, slot branch) when a score tops it by more than 2^THR
   constexpr float BIG = 96.f;          // scores this far above the reference leave the matrix-core path
 
-  const uint32_t kaddr = LineTile<D>::row_at(lane), vaddr = LineTile<D>::col_at(lane);
-  // row fragment (rows 16 kk + l16 of a buffer, columns 32 ks + 8 kb ..) of a buffer at byte address a
-  auto kfrag = [&](uint32_t a, int kk, int ks) -> bf16x8 {
-    const lbyte* base = lds + (a + kaddr);     // one address per buffer; the fragment is a constant offset from it
-    return *reinterpret_cast<const NHA_LDS bf16x8*>(base + (kk * HB + ks * 1024));
-  };
   // transposed fragment of a buffer: X[4 kb + e][16 db + l16] (e < 4) and X[16 + 4 kb + e - 4][..]
   auto vfrag = [&](uint32_t a, int db) -> bf16x8 {
     const lbyte* base = lds + ((a + vaddr) ^ ((db & 1) * 32));   // two addresses per buffer
@@ -312,7 +278,6 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   auto rescale_acc = [&](float delta) {
     const float alpha = fexp2(-delta);
     nm -= delta;
-    nmv = (f32x4){nm, nm, nm, nm};
 #pragma unroll
     for (int r = 0; r < 4; ++r) Lw[r] *= alpha;
 #pragma unroll
@@ -341,13 +306,17 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   wait_vm<0>();
   lds_barrier();
   {
-    Sc[0] = nmv;
-    Sc[1] = nmv;
+    Sc[0] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    Sc[1] = Sc[0];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       Sc[0] = mfma16(kfrag(C::RING_K, 0, ks), qs[ks], Sc[0]);
       Sc[1] = mfma16(kfrag(C::RING_K, 1, ks), qs[ks], Sc[1]);
     }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Sc[kk][r] *= cs;
     mask_unit(Sc, 0);   // unit 0 is always an edge unit
     const float x = max8(Sc);
     if (__any(x > THR)) rescale(Sc, x);
@@ -357,17 +326,24 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   // older than everything the loop's waits leave in flight)
   lds_barrier();
   if (NCH == 2 && second) issue_s(c0 + BT - p.shift);
-  if (3 < nunits) issue_k_fast(3, 0);
+  if (3 < nunits) issue_k(3, 0);
 
-  // slot-branch query fragments (requested while the last unit is worked on)
-  bf16x8 qg[KS];
+  // slot-branch queries, requested while the last unit is worked on: whole lines, as 1 KB blocks of 16 rows x 32 columns, put
+  // into fragment order through LDS when they are taken
+  uint4 qraw[KS];
   auto load_qg = [&]() {
-    const bf16_t* qp = p.q_gsa + ((int64_t)(c0 + yrow) * HQ + hq) * D + 8 * kb;
+    const int y = BT * ch + 16 * Q + lrow;
+    const bf16_t* qp = p.q_gsa + ((int64_t)(c0 + (y < rows_wg ? y : rows_wg - 1)) * HQ + hq) * D;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qraw[ks] = *reinterpret_cast<const uint4*>(qp + LineTile<D>::load_col(ks, lane));
+  };
+  bf16x8 qg[KS];
+  auto take_qg = [&](uint32_t buf) {   // (two blocks per wave: what a wave writes there it alone reads)
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      uint4 x = make_uint4(0, 0, 0, 0);
-      if (irow < rows) x = *reinterpret_cast<const uint4*>(qp + 32 * ks);
-      qg[ks] = as_bf16x8(x);
+      const uint32_t at = buf + wave * 2048 + (ks & 1) * 1024;
+      *reinterpret_cast<NHA_LDS u32x4*>(lds + (at + lane * 16)) = __builtin_bit_cast(u32x4, qraw[ks]);
+      qg[ks] = *reinterpret_cast<const NHA_LDS bf16x8*>(lds + (at + kaddr));
     }
   };
   auto pack_p = [&]() -> bf16x8 {
@@ -395,7 +371,11 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   uint32_t oE2 = C::RING_V + UB, oE2b = C::RING_V + 2 * UB;   // the two buffers left, which take the second chunk's decay tables
   // ring positions as rotating buffer offsets: s0 = buffer of unit u, s1 of unit u+1, s2 of unit u+2
   uint32_t s0 = 0, s1 = UB, s2 = 2 * UB;
-  for (int u = 0; u + 1 < nunits; ++u) {
+  // K of unit u + 4 and V of unit u + 2
+  const bf16_t *kp = p.k_swa + (((int64_t)c0 + XB0 - 32 * 4) * H + h) * D, *vp = p.v + (((int64_t)c0 + XB0 - 32 * 2) * H + h) * D;
+  const int64_t upr = (int64_t)32 * H * D;
+  auto step = [&](int u, auto body_) {
+    constexpr bool BODY = decltype(body_)::value;
     const uint32_t k_n = C::RING_K + s1;    // K of unit u+1
     const uint32_t v_c = C::RING_V + s0;    // V of unit u
     // ---- phase A: scores of unit u+1 on the matrix core (two accumulators in turn), exponentials of
@@ -409,7 +389,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     for (int i = 0; i < 2 * KS; ++i) {
       const int ks = i >> 1, kk = i & 1;
       if (i + PD < 2 * KS) kfr[i + PD] = kfrag(k_n, (i + PD) & 1, (i + PD) >> 1);
-      Sn[kk] = mfma16(kfr[i], qs[ks], ks == 0 ? nmv : Sn[kk]);
+      Sn[kk] = mfma16(kfr[i], qs[ks], ks == 0 ? (f32x4){0.f, 0.f, 0.f, 0.f} : Sn[kk]);
       if (kk == 1) {
         Sc[ks >> 2][ks & 3] = fexp2(Sc[ks >> 2][ks & 3]);
         NHA_PIN(Sc[ks >> 2][ks & 3]);
@@ -420,7 +400,9 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     NHA_FENCE();
     // K of unit u+2 and V of unit u (requested two iterations ago) have landed for this wave, then for
     // everybody.  What may stay in flight: the requests of the previous iteration.
-    if (u >= 1) {
+    if constexpr (BODY) {
+      wait_vm<2 * LPB>();
+    } else if (u >= 1) {
       if (early) {                    // every iteration requests two buffers' worth, V side first
         if (u + 2 == nunits) wait_vm<LPB>();   // last iteration: also V of the last unit; the tile half behind it may fly
         else wait_vm<2 * LPB>();
@@ -429,32 +411,48 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
       }
     }
     lds_barrier();
-    if (u + 2 < nunits) {
-      issue_v_fast(u + 2, s2);
-    } else if (NCH == 2 && early) {
-      oT[NCH - 1][1] = C::RING_V + s2;
-      issue_ta(oT[NCH - 1][1], last_c, 1);
-    }
-    if (u + 4 < nunits) {
-      issue_k_fast(u + 4, s1);   // unit u+4 takes the buffer of unit u+1
-    } else if (early) {
-      const uint32_t off = C::RING_K + s1;
-      if (u + 4 == nunits) {
-        oT[0][0] = off;
-        issue_ta(off, 0, 0);
-      } else if (u + 3 == nunits) {
-        oT[0][1] = off;
-        issue_ta(off, 0, 1);
-      } else if (NCH == 2) {
-        oT[NCH - 1][0] = off;
-        issue_ta(off, last_c, 0);
+    if constexpr (!BODY) {
+      if (u + 2 < nunits) {
+        issue_v(u + 2, s2);
+      } else if (NCH == 2 && early) {
+        oT[NCH - 1][1] = C::RING_V + s2;
+        issue_ta(oT[NCH - 1][1], last_c, 1);
+      }
+      if (u + 4 < nunits) {
+        issue_k(u + 4, s1);   // unit u+4 takes the buffer of unit u+1
+      } else if (early) {
+        const uint32_t off = C::RING_K + s1;
+        if (u + 4 == nunits) {
+          oT[0][0] = off;
+          issue_ta(off, 0, 0);
+        } else if (u + 3 == nunits) {
+          oT[0][1] = off;
+          issue_ta(off, 0, 1);
+        } else if (NCH == 2) {
+          oT[NCH - 1][0] = off;
+          issue_ta(off, last_c, 0);
+        }
       }
     }
+    auto request = [&](int i) {   // in the common form the loads stand between the products of phase B, V first
+      if constexpr (BODY) {
+        if (i < LPB) g2l16(vp, uoff[i], boff[i] + C::RING_V + s2);
+        else g2l16(kp, uoff[i - LPB], boff[i - LPB] + C::RING_K + s1);
+      }
+    };
     NHA_FENCE();
     // ---- phase B: value products of unit u on the matrix core, row maximum of unit u+1 on the VALU;
     //      V fragment db is read PD products ahead ----
     float m0 = 0.f, m1 = 0.f;
     auto max_step = [&](int s2) {
+      if (s2 == 0 || s2 == 2) {   // to log2 units, relative to the reference
+        const int kk = s2 >> 1;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          Sn[kk][r] = fmaf(Sn[kk][r], cs, nm);
+          NHA_PIN(Sn[kk][r]);
+        }
+      }
       if (s2 == 0) m0 = fmaxf(Sn[0][0], Sn[0][1]);
       if (s2 == 1) m1 = fmaxf(Sn[0][2], Sn[0][3]);
       if (s2 == 2) m0 = fmaxf(fmaxf(m0, Sn[1][0]), Sn[1][1]);
@@ -472,6 +470,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     for (int db = 0; db < DB; ++db) {
       if (db + PD < DB) vfr[db + PD] = vfrag(v_c, db + PD);
       O[db] = mfma16(vfr[db], Pq, O[db]);
+      if (db % (DB / (2 * LPB)) == 0) request(db / (DB / (2 * LPB)));
       if (db % 3 == 0 && db / 3 < 5) max_step(db / 3);
       NHA_FENCE();
     }
@@ -492,14 +491,25 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     }
     Sc[0] = Sn[0];
     Sc[1] = Sn[1];
+    kp -= upr;
+    vp -= upr;
     const uint32_t t0 = s0;
     s0 = s1;
     s1 = s2;
     s2 = t0;
-  }
+  };
+  // Most iterations request the next units and nothing else; their scalar instructions are those of two running pointers.
+  int u = 0;
+#pragma unroll 1
+  do {
+    step(u, std::false_type{});
+    ++u;
+    if (u >= 2 * NCH - 2)
+#pragma unroll 1
+      for (; u + 4 < nunits; ++u) step(u, std::true_type{});
+  } while (u + 1 < nunits);
   // ---- the last unit: no further scores; the slot-branch queries are requested meanwhile ----
   {
-    const int u = nunits - 1;
     const uint32_t v_c = C::RING_V + (u % NR) * UB;
     bf16x8 vf[DB];
 #pragma unroll
@@ -533,6 +543,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   }
   // the window's own log-sum-exp, before the slots join the running softmax
   if (p.lse_swa && kb == 0 && irow < rows) p.lse_swa[(int64_t)(c0 + yrow) * HQ + hq] = (__builtin_amdgcn_logf(Lw[0]) - nm) * LN2;
+  take_qg(oE2);
   auto issue_all = [&](auto issue) {
 #pragma unroll
     for (int c_ = 0; c_ < NCH; ++c_)
