@@ -50,7 +50,8 @@ struct BP {
   float *dsp;             // [nbk+nbv][T_tot][H][M]  inter-chunk part of ds per column block
   float *dvs;             // [T_tot][H][V]     slot-branch dv, indexed by SOURCE token
   const float* gcx;       // [NT][H][BT][M]    the gate cumsums by chunk (matrix-core slot branch), or NULL: gc
-  float *gtot;            // [NT][H][M]        chunk sums of the dg summand, then sums of all later chunks
+  float *gtot;            // [NT][H][M]        chunk sums of the dg summand, then (if `scanned`) sums of all later chunks
+  bool scanned;
   float *dks;             // [T_tot][H][K]     intra-chunk part of dk_gsa, indexed by SOURCE token
   float *ek, *ev;         // [NT][H][K][M], [NT][H][V][M]  N_c, then E_c (see the state-gradient kernels)
   int T_tot, N, NT, HQ, H, K, V, M, wl, shift, nbk, nbv, xNG;   // xNG: heads of a group that xg still keeps apart
@@ -654,9 +655,10 @@ __global__ __launch_bounds__(256) void bwd_state_inter_kernel(const BP p) {
 }
 
 // ------------------------------------------------------------------------------------------
-// ds and dg.  dg is a reverse cumulative sum over the rows of a sequence; three small launches:
-// per chunk the summand, ds and the chunk-local sums (bwd_gate_local_kernel), per sequence the
-// sums of all later chunks plus the end term (bwd_gate_scan_kernel), per chunk the final values
+// ds and dg.  dg is a reverse cumulative sum over the rows of a sequence: per chunk the summand, ds and
+// the chunk-local sums (bwd_gate_local_kernel; on the matrix-core path bwd_slot_inter_kernel forms them),
+// where BP::scanned says so per sequence the sums of all later chunks plus the end term
+// (bwd_gate_scan_kernel), per chunk the final values
 // (bwd_gate_final_kernel, which also zeroes the gradients of the tokens that never reach the
 // slots: the last `shift` of a sequence).
 // ------------------------------------------------------------------------------------------
@@ -823,15 +825,39 @@ __global__ __launch_bounds__(256) void bwd_gate_final_kernel(const BP p) {
   const int c0 = bos + it * BT;
   const int R = (eos - c0) < BT ? (eos - c0) : BT;
   if (M == BT) {
+    __shared__ float4 part[16][16];
     // four consecutive slots of four rows per thread, their 16-byte reads requested together
     const int m = (threadIdx.x & 15) * 4, r0 = threadIdx.x >> 4;
-    const float4 gt = *reinterpret_cast<const float4*>(p.gtot + ((int64_t)chunk * H + h) * M + m);
+    float4 gt = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (!p.scanned) {   // the sums of the later chunks: every sixteenth per group of threads, two at a time
+      const int last = p.coff[n + 1];
+      const float* g = p.gtot + (int64_t)h * M + m;
+      const int64_t step = (int64_t)H * M;
+      for (int c = chunk + 1 + r0; c < last; c += 32) {
+        const float4 a = *reinterpret_cast<const float4*>(g + c * step);
+        const float4 b = *reinterpret_cast<const float4*>(g + (c + 16 < last ? c + 16 : c) * step);
+        const float on = c + 16 < last ? 1.f : 0.f;
+        gt.x += a.x + on * b.x; gt.y += a.y + on * b.y; gt.z += a.z + on * b.z; gt.w += a.w + on * b.w;
+      }
+    } else {
+      gt = *reinterpret_cast<const float4*>(p.gtot + ((int64_t)chunk * H + h) * M + m);
+    }
     float4 v[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int r = r0 + 16 * q, t = c0 + r;
       v[q] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (r < R && t - p.shift >= bos) v[q] = *reinterpret_cast<const float4*>(p.dsi + ((int64_t)t * H + h) * M + m);
+    }
+    if (!p.scanned) {
+      part[r0][threadIdx.x & 15] = gt;
+      __syncthreads();
+      gt = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int g = 0; g < 16; ++g) {
+        const float4 a = part[g][threadIdx.x & 15];
+        gt.x += a.x; gt.y += a.y; gt.z += a.z; gt.w += a.w;
+      }
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -1067,6 +1093,11 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
   p.ck = (float*)(sc + sp.ck); p.cv = (float*)(sc + sp.cv);
   p.dsi = (float*)(sc + sp.dsi); p.dsp = (float*)(sc + sp.dsp); p.dvs = (float*)(sc + sp.dvs);
   p.gtot = (float*)(sc + sp.gtot);
+  // Without gradients of the final states the last pass of the gates can add up a chunk's later chunks itself, half of NT^2 H
+  // rows of 256 bytes in all at worst, and one launch is saved (scan and last pass / last pass alone: 5003 tokens of 16 heads
+  // 15.6 / 8.5 us, 8 x 2048 of 4 11.9 / 8.0, 2 x 8192 of 8 19.5 / 14.3; NT^2 H = 2^21: 32768 tokens of 8 heads 43.1 / 30.1, 65536 of
+  // 2 44.7 / 18.9).  The sum grows with the square of the length and the scan does not: beyond what is measured, the scan.
+  p.scanned = a->dhkt || a->dhvt || a->M != BT || (int64_t)a->NT * a->NT * a->H > (1 << 21);
   p.dks = (float*)(sc + sp.dks); p.ek = (float*)(sc + sp.ek); p.ev = (float*)(sc + sp.ev);
   p.T_tot = a->T_tot; p.N = a->N; p.NT = a->NT; p.HQ = a->HQ; p.H = a->H; p.K = a->K; p.V = a->V; p.M = a->M;
   p.wl = a->wl; p.shift = a->shift; p.nbk = sp.nbk; p.nbv = sp.nbv; p.scale = a->scale;
@@ -1119,7 +1150,7 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
     hipLaunchKernelGGL((bwd_gate_local_kernel<T>), dim3(a->NT, a->H), dim3(256), 0, st, p);
   }
   NHA_CHECK_LAUNCH("nha_prefill_bwd(state gradients)");
-  hipLaunchKernelGGL((bwd_gate_scan_kernel<T>), dim3(a->N * a->H), dim3(64), 0, st, p);
+  if (p.scanned) hipLaunchKernelGGL((bwd_gate_scan_kernel<T>), dim3(a->N * a->H), dim3(64), 0, st, p);
   hipLaunchKernelGGL((bwd_gate_final_kernel<T>), dim3(a->NT, a->H), dim3(256), 0, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(gate scan)");
   if (wmfma) return bwd_window_mfma_dkv(a, p.delta, p.dvs, sc + sp.ld);

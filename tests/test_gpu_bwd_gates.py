@@ -1,0 +1,36 @@
+"""Gate gradients: the sums of a chunk's later chunks by the last pass itself, and by a scan over the sequence (taken where
+the final states have gradients; zero ones change nothing)."""
+import numpy as np
+import pytest
+import torch
+
+from tests.util import prefill_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lens,shift", [((1,), 0), ((64, 65), 0), ((16 * 64, 17 * 64), 5), ((33 * 64 + 7, 30, 31 * 64), 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_sum_over_later_chunks_is_the_scan(lens, shift, dtype):
+    from nha_amd.ops import nha_prefill, nha_prefill_bwd
+    from tests.test_gpu_prefill import KEYS
+    cu = np.cumsum((0, *lens)).astype(np.int32)
+    T, N, HQ, H, D = int(cu[-1]), len(lens), 4, 2, 64
+    d = prefill_inputs(T, 1, T, HQ, H, D, D, 64, dtype=dtype, qk_scale=0.5)
+    xs = [d[k][0].cuda().contiguous() for k in KEYS]
+    kw = dict(wl=31, shift=shift, scale=D ** -0.5)
+    o, lw, lg, _, _ = nha_prefill(*xs, cu, **kw)
+    do = torch.randn(T, HQ, D, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
+    zero = tuple(torch.zeros(N, H, 64, 64, device="cuda") for _ in range(2))
+    a = nha_prefill_bwd(*xs, o, lw, lg, do, cu, **kw)
+    b = nha_prefill_bwd(*xs, o, lw, lg, do, cu, dht=zero, **kw)
+    for i in range(7):
+        if i != 6:
+            assert torch.equal(a[i], b[i])
+    x, y = a[6].double(), b[6].double()
+    # two orders of up to 34 fp32 sums whose terms are no larger than twice the largest result, then each side's rounding to the
+    # dtype (half a unit in the last place: 2^-8 of the value in bf16, 2^-24 in fp32)
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    bound = 2 * 34 * 2.0 ** -24 * 2 * y.abs().amax() + 2 * half * torch.maximum(x.abs(), y.abs())
+    assert ((x - y).abs() <= bound).all()
+    assert x.abs().sum() > 0 or T <= shift
