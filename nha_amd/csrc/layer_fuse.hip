@@ -5,7 +5,9 @@
 //   epilogue: rms_norm(silu(o)) * weight (+ bias), the input of the output projection
 //             (nha_fla/layers/nha.py:278).
 // Both are HBM-bound streaming kernels: one wave per token (four tokens per workgroup), 16-byte
-// accesses, every input element read once and every output element written once.  Intermediate results are rounded to
+// accesses, every input element read once and every output element written once (8 x 2048 tokens, 4 heads of 256, 64 slots:
+// prologue 49 us, its backward 75, 403 MB at the rate of a copy; 65 and 91 with the library's log1p and exponentials for the
+// gates, eight of them to a lane and half of the lanes idle, bound by the vector units).  Intermediate results are rounded to
 // the tensor dtype at the points where the reference's chain of tensor ops rounds them.
 #include "common.h"
 
@@ -36,13 +38,53 @@ template <> __device__ __forceinline__ float rnd<bf16_t>(float x) { return bf16_
 __device__ __forceinline__ float silu_f(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 __device__ __forceinline__ float feature_f(float x, int fm) { return fm == 1 ? silu_f(x) : (fm == 2 ? fmaxf(x, 0.f) : x); }
 
+// ls = log(1 / (1 + e^-x)), rounded to T
+template <typename T> __device__ __forceinline__ float logsigmoid_f(float x);
+template <> __device__ __forceinline__ float logsigmoid_f<float>(float x) { return fminf(x, 0.f) - log1pf(expf(-fabsf(x))); }
+// bf16: u = e^-|x| with the rounding of x log2(e) made good, log(1 + u) = 2 atanh(u / (2 + u)) by its series to the 15th power of
+// at most 1/3: 3 ulp of float32, a thousandth of the rounding that follows, for a third of the library's instructions
+template <> __device__ __forceinline__ float logsigmoid_f<bf16_t>(float x) {
+  const float a = -fabsf(x), t = a * 1.44269502f, lost = fmaf(a, 1.44269502f, -t) + a * 1.92596299e-8f;
+  const float e = __builtin_amdgcn_exp2f(t), u = a < -87.f ? e : fmaf(e, lost * 0.693147181f, e);   // (-inf: lost is NaN)
+  const float s = u * __builtin_amdgcn_rcpf(2.f + u), q = s * s;
+  float r = fmaf(q, 2.f / 15.f, 2.f / 13.f);
+  r = fmaf(q, r, 2.f / 11.f);
+  r = fmaf(q, r, 2.f / 9.f);
+  r = fmaf(q, r, 2.f / 7.f);
+  r = fmaf(q, r, 2.f / 5.f);
+  r = fmaf(q, r, 2.f / 3.f);
+  r = fmaf(q, r, 2.f);
+  return rnd<bf16_t>(fminf(x, 0.f) - s * r);
+}
+// e^x, x <= 0 (a log gate; bf16: off by |x| 2^-24, then rounded to 8 bits)
+template <typename T> __device__ __forceinline__ float exp_gate_f(float x);
+template <> __device__ __forceinline__ float exp_gate_f<float>(float x) { return expf(x); }
+template <> __device__ __forceinline__ float exp_gate_f<bf16_t>(float x) {
+  return __builtin_amdgcn_exp2f(fmaf(x, 1.44269502f, x * 1.92596299e-8f));
+}
+
 template <typename T, int VEC> __device__ __forceinline__ void ldv(const T* p, float* o) {
-  if constexpr (VEC == 8) Elem<T>::ld8(p, o);
-  else o[0] = Elem<T>::ld(p);
+  if constexpr (VEC == 8) {
+    Elem<T>::ld8(p, o);
+  } else if constexpr (VEC == 4) {
+    struct alignas(4 * sizeof(T)) { T e[4]; } x = *reinterpret_cast<const decltype(x)*>(p);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = Elem<T>::ld(&x.e[e]);
+  } else {
+    o[0] = Elem<T>::ld(p);
+  }
 }
 template <typename T, int VEC> __device__ __forceinline__ void stv(T* p, const float* v) {
-  if constexpr (VEC == 8) Elem<T>::st8(p, v);
-  else Elem<T>::st(p, v[0]);
+  if constexpr (VEC == 8) {
+    Elem<T>::st8(p, v);
+  } else if constexpr (VEC == 4) {
+    struct alignas(4 * sizeof(T)) { T e[4]; } x;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) Elem<T>::st(&x.e[e], v[e]);
+    *reinterpret_cast<decltype(x)*>(p) = x;
+  } else {
+    Elem<T>::st(p, v[0]);
+  }
 }
 
 // VEC elements as loaded (conversion deferred, so a prefetched row costs half the registers in bf16)
@@ -139,6 +181,25 @@ __device__ __forceinline__ int token_angles(const LP& p, float* cs, int wave, in
 }
 
 template <typename T, int VEC>
+__device__ __forceinline__ void gate_rows(const LP& p, int t, int lane) {
+  const int n = p.H * p.M;
+  const T* src = (const T*)p.f + (size_t)t * p.lf;
+  T* dg = (T*)p.g + (size_t)t * n;
+  T* ds = (T*)p.s + (size_t)t * n;
+  for (int u = lane * VEC; u < n; u += 64 * VEC) {
+    float x[VEC], g[VEC], s[VEC];
+    ldv<T, VEC>(src + u, x);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      g[e] = rnd<T>(logsigmoid_f<T>(x[e]) * p.inv_norm);
+      s[e] = 1.f - rnd<T>(exp_gate_f<T>(g[e]));
+    }
+    stv<T, VEC>(dg + u, g);
+    stv<T, VEC>(ds + u, s);
+  }
+}
+
+template <typename T, int VEC>
 __global__ __launch_bounds__(256) void layer_prologue_kernel(LP p) {
   extern __shared__ float cs_all[];  // per wave: cos[K/2], sin[K/2]
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -161,24 +222,9 @@ __global__ __launch_bounds__(256) void layer_prologue_kernel(LP p) {
       stv<T, VEC>(dst + u, x);
     }
   }
-  {
-    const int n = p.H * p.M;
-    const T* src = (const T*)p.f + (size_t)t * p.lf;
-    T* dg = (T*)p.g + (size_t)t * n;
-    T* ds = (T*)p.s + (size_t)t * n;
-    for (int u = lane * VEC; u < n; u += 64 * VEC) {
-      float x[VEC], g[VEC], s[VEC];
-      ldv<T, VEC>(src + u, x);
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        const float ls = rnd<T>(fminf(x[e], 0.f) - log1pf(expf(-fabsf(x[e]))));
-        g[e] = rnd<T>(ls * p.inv_norm);
-        s[e] = 1.f - rnd<T>(expf(g[e]));
-      }
-      stv<T, VEC>(dg + u, g);
-      stv<T, VEC>(ds + u, s);
-    }
-  }
+  // a row of gates of at most 256 is four to a lane: eight would leave half of the wave idle
+  if (VEC == 8 && p.H * p.M <= 256) gate_rows<T, 4>(p, t, lane);
+  else gate_rows<T, VEC>(p, t, lane);
 }
 
 // d silu(x) / dx and the derivative of the feature map
@@ -225,6 +271,28 @@ __device__ __forceinline__ void rope_rows_bwd(const T* src, const T* dswa, const
   }
 }
 
+// g = logsigmoid(f)/n, s = 1 - exp(g):  df = (dg - ds * exp(g)) / n * sigmoid(-f)
+template <typename T, int VEC>
+__device__ __forceinline__ void gate_rows_bwd(const LP& p, int t, int lane) {
+  const int n = p.H * p.M;
+  const T* src = (const T*)p.f + (size_t)t * p.lf;
+  const T* pdg = (const T*)p.dg + (size_t)t * n;
+  const T* pds = (const T*)p.ds + (size_t)t * n;
+  T* dst = (T*)p.df + (size_t)t * p.lf;
+  for (int u = lane * VEC; u < n; u += 64 * VEC) {
+    float x[VEC], dg[VEC], ds[VEC];
+    ldv<T, VEC>(src + u, x);
+    ldv<T, VEC>(pdg + u, dg);
+    ldv<T, VEC>(pds + u, ds);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      const float eg = rnd<T>(exp_gate_f<T>(rnd<T>(logsigmoid_f<T>(x[e]) * p.inv_norm)));
+      dg[e] = (dg[e] - ds[e] * eg) * p.inv_norm / (1.f + expf(x[e]));
+    }
+    stv<T, VEC>(dst + u, dg);
+  }
+}
+
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void layer_prologue_bwd_kernel(LP p) {
   extern __shared__ float cs_all[];
@@ -252,27 +320,8 @@ __global__ __launch_bounds__(256) void layer_prologue_bwd_kernel(LP p) {
       stv<T, VEC>(dst + u, d);
     }
   }
-  {
-    // g = logsigmoid(f)/n, s = 1 - exp(g):  df = (dg - ds * exp(g)) / n * sigmoid(-f)
-    const int n = p.H * p.M;
-    const T* src = (const T*)p.f + (size_t)t * p.lf;
-    const T* pdg = (const T*)p.dg + (size_t)t * n;
-    const T* pds = (const T*)p.ds + (size_t)t * n;
-    T* dst = (T*)p.df + (size_t)t * p.lf;
-    for (int u = lane * VEC; u < n; u += 64 * VEC) {
-      float x[VEC], dg[VEC], ds[VEC];
-      ldv<T, VEC>(src + u, x);
-      ldv<T, VEC>(pdg + u, dg);
-      ldv<T, VEC>(pds + u, ds);
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        const float ls = rnd<T>(fminf(x[e], 0.f) - log1pf(expf(-fabsf(x[e]))));
-        const float eg = rnd<T>(expf(rnd<T>(ls * p.inv_norm)));
-        dg[e] = (dg[e] - ds[e] * eg) * p.inv_norm / (1.f + expf(x[e]));
-      }
-      stv<T, VEC>(dst + u, dg);
-    }
-  }
+  if (VEC == 8 && p.H * p.M <= 256) gate_rows_bwd<T, 4>(p, t, lane);
+  else gate_rows_bwd<T, VEC>(p, t, lane);
 }
 
 struct EP {
