@@ -20,7 +20,7 @@
 // recurrence over chunks): forward state pass (chunk-start states, gate cumsums) -> bwd_q_kernel (per token: the
 // vectors du, p) -> bwd_intra_kernel (per chunk: intra-chunk matrices and the intra part of ds)
 // -> bwd_dqg_kernel (per token: dq_gsa) -> bwd_state_{direct,scan,inter}_kernel (state gradients as a linear recurrence over
-// chunks: dk_gsa, slot-branch dv, inter-chunk part of ds, dh0) -> bwd_gate_*_kernel (reverse scan: ds, dg)
+// chunks: dk_gsa, slot-branch dv, inter-chunk part of ds, dh0) -> bwd_gate_*_kernel (reverse sums: ds, dg)
 // -> bwd_kv_window_kernel (per key: dk_swa, dv).  For bf16 tensors with K == V in {64,128,256} the
 // window parts (dq_swa, dk_swa, dv) run on the matrix cores instead (prefill_bwd_mfma.hip).
 #include "mfma_common.h"
@@ -389,7 +389,8 @@ __global__ __launch_bounds__(512) void bwd_intra_kernel(const BP p) {
 // the last parallel over chunks:
 //   bwd_state_direct_kernel   N_c and the intra-chunk part of dk' / dv'   (per chunk, CB columns)
 //   bwd_state_scan_kernel     the recurrence, element-wise over chunks (E_c replaces N_c; dh0)
-//   bwd_state_inter_kernel    the parts of dk' / dv' / ds that involve E_c (per chunk, CB columns)
+//   bwd_state_inter_kernel    the parts of dk' / dv' / ds that involve E_c (per chunk, CB columns; bf16 matrix-core calls:
+//                             bwd_slot_inter_kernel, which goes on with the gates)
 // blockIdx.z = 0: k-state (columns d; q_gsa / k_gsa rows, weights dus, matrix ck, output dk_gsa);
 // 1: v-state (columns c; do / v rows, weights p, matrix cv, output dvs).  eg holds N then E as
 // [NT][H][X][M] per state.

@@ -18,13 +18,13 @@
 // Bound: latency between short products -- one workgroup of eight waves fits a CU (LDS), a head is eight barriers with 4 to
 // 100 MFMAs per wave between them, about 24k cycles of which the MFMAs are 4k.  As five launches with the tables handed on
 // through HBM (A, B, du, p, ck, cv: 112 KB per head and chunk) plus one that exported the states as bf16 pairs, the same
-// work took 914 us at B=2, T=8192, 32/8 heads of 128 (now 459, and 7 for the launch that looks for strongly decaying
-// chunks), 366 at B=8, T=2048, 4/4 heads of 256 (now 237 + 7) and 191 at 5003 packed tokens, 16/16 heads of 64 (now 100 + 5).
+// work took 914 us at B=2, T=8192, 32/8 heads of 128 (now 429, and 7 for the launch that looks for strongly decaying
+// chunks), 366 at B=8, T=2048, 4/4 heads of 256 (now 230 + 7) and 191 at 5003 packed tokens, 16/16 heads of 64 (now 96 + 5).
 //
 // Registers are the scarce thing: sums over the heads (64 at DW = 128) and the operands (48) stay, so whatever spills waits,
 // with every load before it, for memory.  Hence: nothing derived from the lane's number lives across the loop over heads;
-// wave-uniform bases with 32-bit offsets; Y read from LDS in both forms; stores only after the last load.  (459 us was 709
-// with the spills of the first version.)
+// wave-uniform bases with 32-bit offsets; Y read from LDS in both forms; stores only after the last load.  (709 us with the
+// spills of the first version.)  Operands staged through LDS in whole lines, which other kernels gain from, change nothing here.
 //
 // Precision: dg is a difference of nearly equal sums, so every table made from fp32 values (X, Xp, Y, ck, cv, the chunk-start
 // states) is a bf16 pair hi + lo and its products are hi hi + hi lo + lo hi (single bf16 tables put 1-5 % on dg).
