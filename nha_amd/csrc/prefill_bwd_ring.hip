@@ -6,8 +6,8 @@
 //   pi = e^(w - lse),  dw = pi (do.v - delta),
 //   dq_swa_q = scale sum_j dw k_j,   dk_swa_j = scale sum_q dw q_q,   dv_j += sum_q pi do_q.
 // Every streamed operand goes from global memory straight into LDS (global_load_lds_dwordx4) through a ring of buffers.  One
-// layout of a tile serves row fragments and transposing reads: 1 KB blocks of 16 rows x 32 columns, each two planes of
-// 32-byte rows, from which a wave's 16-byte reads of 16 rows run at the LDS's full rate too.
+// layout of a tile serves row fragments and transposing reads: 1 KB blocks of 16 rows x 32 columns, of 64-byte rows with their
+// pieces exchanged (LineTile) in ring_dq_kernel, two planes of 32-byte rows in ring_dkv_kernel (with LineTile 905 -> 920 us).
 //
 // ring_dq_kernel: one workgroup of 8 waves = one 64-token chunk x 4 query heads of one kv-head (a query
 //   per lane, 32 queries per wave), so the K / V rows of the window are fetched once for the four heads,
@@ -18,7 +18,8 @@
 //   leaves (-lse / scale, -delta) per (token, q-head) as pairs for the kernel below, whose score and
 //   dP accumulators start from them.
 //   Bound: as below, 56 % of the matrix rate.  B=2, T=8192, 32/8 heads, W=2048: 625 us unit by unit with K in LDS twice and
-//   the compiler's schedule, 597 like this, 591 with a stretch's first fragments requested during the stretch before.
+//   the compiler's schedule, 597 like this, 591 with a stretch's first fragments requested during the stretch before, 575 (582 on that card) with the
+//   query and do rows loaded in whole lines: 2 x 4096 tokens, W=256 114 -> 110, 500 tokens 25.7 -> 23.7, 1700 tokens, W=64 19.5 -> 19.8.
 // ring_dkv_kernel: one workgroup of 8 waves = 256 keys of one kv-head (a key per lane and 16-key block, 32 keys per wave, K
 //   rows in registers, V rows in LDS); the q / do rows of every query head of the group stream through the ring in items of
 //   32 queries: a tile of each plus the 32 (lse, delta) pairs.  One layout of a tile serves both reads, the row fragments of
@@ -94,10 +95,10 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
   const int rh = wave / KS, cq = wave % KS;
   const bf16_t* const kbase = p.k + ((int64_t)bos * H + h) * D;
   const bf16_t* const vbase = p.v + ((int64_t)bos * H + h) * D;
-  const uint32_t pcol = (uint32_t)(4 * cq + 2 * (lane >> 5) + (lane & 1)) * 8;
+  const uint32_t pcol = LineTile<D>::load_col(cq, lane);
   // rows past eos (units 0 and 1 only) are read from row eos - 1: always masked, always finite
   auto issue_unit = [&](int u) {
-    int row = c0 + 32 - 32 * u + 16 * rh + ((lane & 31) >> 1);
+    int row = c0 + 32 - 32 * u + 16 * rh + LineTile<D>::load_row(lane);
     row = row < eos ? row : eos - 1;
     const uint32_t off = ((uint32_t)(row - bos) * (uint32_t)(H * D) + pcol) * 2;
     const uint32_t dst = lds0 + (u & (NRU - 1)) * UNIT + rh * HB + cq * 1024;
@@ -108,7 +109,26 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
   for (int u = 0; u < NRU - 2; ++u)
     if (u < nunits) issue_unit(u);
 
-  // query-side fragments: q pre-scaled by scale * log2(e) (the rounding the forward's scores saw), do as it is
+  // query-side fragments: q pre-scaled by scale * log2(e) (the rounding the forward's scores saw), do as it is.  The rows come in
+  // whole lines, as 1 KB blocks of 16 rows x 32 columns (a fragment as it lies in memory, 16 bytes of 16 rows, takes three
+  // times as long to load), and are put into fragment order through the two ring slots that no unit has been requested into.
+  uint4 qraw[RQB][KS], draw[RQB][KS];
+#pragma unroll
+  for (int qb = 0; qb < RQB; ++qb) {
+    int r = 16 * (qb0 + qb) + LineTile<D>::load_row(lane);
+    r = r < rows ? r : rows - 1;
+    const int64_t at = ((int64_t)(c0 + r) * HQ + hq) * D;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      qraw[qb][ks] = *reinterpret_cast<const uint4*>(p.q + at + LineTile<D>::load_col(ks, lane));
+      draw[qb][ks] = *reinterpret_cast<const uint4*>(p.dout + at + LineTile<D>::load_col(ks, lane));
+    }
+  }
+  const uint32_t own = (NRU - 2) * UNIT + wave * 4096, kaddr = LineTile<D>::row_at(lane);
+  auto turned = [&](const uint4& x, int slot) {   // (what a wave writes there it alone reads)
+    *reinterpret_cast<NHA_LDS u32x4*>(lds + (own + slot * 1024 + lane * 16)) = __builtin_bit_cast(u32x4, x);
+    return *reinterpret_cast<const NHA_LDS u32x4*>(lds + (own + slot * 1024 + kaddr));
+  };
   bf16x8 qf[RQB][KS], df[RQB][KS];
   float nlse[RQB], dl[RQB];
 #pragma unroll
@@ -116,22 +136,18 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
     const int irow = 16 * (qb0 + qb) + l16;
     const bool valid = irow < rows;
     const int64_t tq = (int64_t)(c0 + (valid ? irow : 0)) * HQ + hq;
+    const uint32_t on = valid ? ~0u : 0u;   // (a mask: a choice between loaded registers may become a branch)
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      uint4 x = make_uint4(0, 0, 0, 0), y = x;
-      if (valid) {
-        x = *reinterpret_cast<const uint4*>(p.q + tq * D + 32 * ks + 8 * kb);
-        y = *reinterpret_cast<const uint4*>(p.dout + tq * D + 32 * ks + 8 * kb);
-      }
-      const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+      const u32x4 x = turned(qraw[qb][ks], (2 * ks) & 3) & on;
       bf16x8 r;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float f = __uint_as_float((e & 1) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16));
+        const float f = __uint_as_float((e & 1) ? (x[e >> 1] & 0xffff0000u) : (x[e >> 1] << 16));
         r[e] = (__bf16)(f * cs);
       }
       qf[qb][ks] = r;
-      df[qb][ks] = as_bf16x8(y);
+      df[qb][ks] = __builtin_bit_cast(bf16x8, turned(draw[qb][ks], (2 * ks + 1) & 3) & on);
     }
     float ls = 0.f, lg = 0.f;
     if (valid) {
@@ -149,15 +165,14 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
 #pragma unroll
     for (int qb = 0; qb < RQB; ++qb) dQ[db][qb] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  const uint32_t kaddr = (uint32_t)((kb >> 1) * 512 + l16 * 32 + (kb & 1) * 16);
-  const uint32_t vaddr = (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
+  const uint32_t vaddr = LineTile<D>::col_at(lane);
   // row fragment of a tile at byte address a: rows 16 kk + l16, columns 32 ks + 8 kb ..
   auto rfrag = [&](uint32_t a, int kk, int ks) -> bf16x8 {
     return *reinterpret_cast<const NHA_LDS bf16x8*>(lds + (a + kaddr) + kk * HB + ks * 1024);
   };
   // transposed fragment: X[4 kb + e][16 db + l16] (e < 4) and X[16 + 4 kb + e - 4][..]
   auto tfrag = [&](uint32_t a, int db) -> bf16x8 {
-    const lbyte* pa = lds + (a + vaddr) + (db >> 1) * 1024 + (db & 1) * 512;
+    const lbyte* pa = lds + ((a + vaddr) ^ ((db & 1) * 32)) + (db >> 1) * 1024;
     struct { s16x4 a, b; } t;
     t.a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)pa);
     t.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NHA_LDS s16x4*)(pa + HB));
