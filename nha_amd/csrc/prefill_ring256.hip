@@ -215,7 +215,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   issue_gc(0, C::GC);
   issue_s(c0 - p.shift);
 #pragma unroll
-  for (int j = 0; j < NW / 2; ++j)    // rows past the end of the sequence: its last, never stored
+  for (int j = 0; j < NW / 2; ++j)    // rows past the end of the sequence: its last, zeroed once they are in their registers
     issue_buffer(j * UB, p.q_swa + ((int64_t)c0 * HQ + hq) * D, (uint32_t)(HQ * D), [&](int r) { return 32 * j + r < rows_wg ? 32 * j + r : rows_wg - 1; });
   const uint32_t kaddr = LineTile<D>::row_at(lane), vaddr = LineTile<D>::col_at(lane);
   // row fragment (rows 16 kk + l16 of a buffer, columns 32 ks + 8 kb ..) of a buffer at byte address a
@@ -227,7 +227,11 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   lds_barrier();
   bf16x8 qs[KS];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) qs[ks] = kfrag(wave * HB, 0, ks);
+  for (int ks = 0; ks < KS; ++ks) {
+    // rows that do not exist score 0: scores of a copied row could top the reference below and flag rows of another sequence
+    const u32x4 x = __builtin_bit_cast(u32x4, kfrag(wave * HB, 0, ks));
+    qs[ks] = __builtin_bit_cast(bf16x8, irow < rows ? x : (u32x4){0u, 0u, 0u, 0u});
+  }
   lds_barrier();
   issue_k(0, 0);
   issue_v(0, 0);
@@ -483,7 +487,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     // is ever taken.  fp32 sums and bf16 probabilities hold 2^BIG above it; a score beyond that sends the
     // wave's 16 rows to the exact pass (mfma_repair_kernel recomputes flagged sub-blocks) and is clamped.
     if (__any(m0 > BIG)) {
-      if (lane == 0) atomicOr(p.flags + (cg + (int64_t)ch * H) * 4, 1 << Q);
+      if (lane == 0 && 16 * Q < rows) atomicOr(p.flags + (cg + (int64_t)ch * H) * 4, 1 << Q);   // (a chunk that is not there has no flags)
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
