@@ -565,13 +565,14 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
         }
         __builtin_amdgcn_sched_barrier(0);
         if (edge) {
+          const float none = cs < 0.f ? INFINITY : -INFINITY;   // -inf once it has been multiplied by cs below
 #pragma unroll
           for (int q = 0; q < NQ; ++q)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const int y = 32 * u + 16 * (q & 1) + 4 * kb + r, xk = kbase + 16 * (q >> 1) + l16;
               const bool ok = (xk <= y) && (p.wl < 0 || y - xk <= p.wl) && (c0 + y < eos);
-              if (!ok) S[q][r] = -INFINITY;
+              if (!ok) S[q][r] = none;
             }
         }
 #pragma unroll

@@ -11,14 +11,15 @@ from tests.util import prefill_inputs
 pytestmark = pytest.mark.gpu
 
 
-def compare(cu, wl, H, NG, D, keys):
+def compare(cu, wl, H, NG, D, keys, scale=None):
     from nha_amd import chunk_nha
     d = prefill_inputs(9100 + wl + NG, 1, cu[-1], H * NG, H, D, D, 64, dtype=BF, qk_scale=1.0)
     do = torch.randn(1, cu[-1], H * NG, D, generator=torch.Generator().manual_seed(wl + 5)).to(BF)
     outs, grads = [], []
     for dt in (BF, torch.float32):
         x = [d[k].cuda().to(dt).requires_grad_(True) for k in KEYS]
-        o = chunk_nha(*x, cu_seqlens=torch.tensor(cu, dtype=torch.int32).cuda(), scale=D ** -0.5, window_size_left=wl, gsa_kv_shift=0)[0]
+        o = chunk_nha(*x, cu_seqlens=torch.tensor(cu, dtype=torch.int32).cuda(),
+                      scale=D ** -0.5 if scale is None else scale, window_size_left=wl, gsa_kv_shift=0)[0]
         o.backward(do.cuda().to(dt))
         outs.append(o.detach())
         grads.append([t.grad for t in x])
@@ -46,3 +47,11 @@ def test_more_sequences_than_lanes(wl):
     cu = torch.tensor([0, *lens]).cumsum(0).tolist()
     print("case", wl, flush=True)
     compare(cu, wl, 4, 1, 256, KEYS)
+
+
+@pytest.mark.parametrize("H,NG,D", [(32, 4, 128), (16, 1, 256)])
+@pytest.mark.parametrize("wl", [-1, 64, 200, 500])
+def test_negative_scale(wl, H, NG, D):
+    """The weights of the keys outside the window are zero whatever the sign of the scale."""
+    print("case", wl, H, NG, D, flush=True)
+    compare([0, 1, 40, 104, 361, 1190], wl, H, NG, D, KEYS, scale=-D ** -0.5)
