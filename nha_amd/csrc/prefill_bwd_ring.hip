@@ -667,7 +667,9 @@ static bool short_groups(const NhaPrefillBwdArgs* a) { return a->wl >= 0 && a->w
 // (128) 308 -> 236; 3000 tokens, 32 / 4 heads, W = 512 (48) 333 -> 188.  Beyond, the groups of 64 pass one round of
 // places (two per CU) and pull every q / do row four times as often: 5000 tokens, 32 / 8 heads, W = 512 (160) 187 against
 // 217 us; 4000 tokens, W = 128 (256) 51 against 57.
+// A scale of (almost) zero goes to bwd_dkv_kernel too: the scores here start from -lse / scale.
 bool bwd_ring_dkv_supported(const NhaPrefillBwdArgs* a) {
+  if (!(fabsf(a->scale) > 1e-30f)) return false;
   const int64_t groups = (int64_t)a->H * (short_groups(a) ? (a->NT + 1) / 2 : (a->NT + 3) / 4);
   return bwd_ring_supported(a) && groups > 128;
 }

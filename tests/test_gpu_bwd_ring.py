@@ -55,3 +55,11 @@ def test_negative_scale(wl, H, NG, D):
     """The weights of the keys outside the window are zero whatever the sign of the scale."""
     print("case", wl, H, NG, D, flush=True)
     compare([0, 1, 40, 104, 361, 1190], wl, H, NG, D, KEYS, scale=-D ** -0.5)
+
+
+@pytest.mark.parametrize("scale", [0.0, 1e-42, -1e-42, 1e-28])
+@pytest.mark.parametrize("wl", [64, 500])
+def test_scale_of_zero(wl, scale):
+    """All keys of the window weigh the same; dk_swa is zero, or nearly so, and finite."""
+    print("case", wl, scale, flush=True)
+    compare([0, 1, 40, 104, 361, 1190], wl, 32, 4, 128, ("k_swa", "v"), scale=scale)
