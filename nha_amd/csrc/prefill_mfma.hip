@@ -609,7 +609,12 @@ __global__ __launch_bounds__(64 * NW, OWN ? NW / 2 : 1) void mfma_out_kernel(con
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int c0 = bos + it * BT;
   const int rows = (eos - c0) < BT ? (eos - c0) : BT;
-  const float cs = p.scale * LOG2E;   // logits are kept unscaled; p = exp2(cs * (s - m))
+  // logits are kept unscaled; p = exp2(cs * (s - m)) with cs > 0: the sign of the scale is the queries', and where it is 0 they are
+  const float cs = p.scale == 0.f ? LOG2E : fabsf(p.scale) * LOG2E;
+  const uint32_t qkeep = p.scale == 0.f ? 0u : ~0u, qsign = p.scale < 0.f ? 0x80008000u : 0u;
+  auto query = [&](const uint4& x) {
+    return as_bf16x8(make_uint4((x.x & qkeep) ^ qsign, (x.y & qkeep) ^ qsign, (x.z & qkeep) ^ qsign, (x.w & qkeep) ^ qsign));
+  };
   const int64_t cg = (int64_t)chunk * H + h;
 
   // ---- window tile schedule: tile i covers keys [c0 + 64 - TK (i+1), c0 + 64 - TK i) ----------
@@ -811,7 +816,7 @@ __global__ __launch_bounds__(64 * NW, OWN ? NW / 2 : 1) void mfma_out_kernel(con
     for (int ks = 0; ks < KS; ++ks) {
       uint4 x = make_uint4(0, 0, 0, 0);
       if (irow < rows) x = *reinterpret_cast<const uint4*>(qp + 32 * ks);
-      qs[qb][ks] = as_bf16x8(x);
+      qs[qb][ks] = query(x);
     }
   }
   // ---- phase 1a: slot logits and the slot "tile" of the softmax, one 16-row block at a time ----
@@ -826,7 +831,7 @@ __global__ __launch_bounds__(64 * NW, OWN ? NW / 2 : 1) void mfma_out_kernel(con
       for (int ks = 0; ks < KS; ++ks) {
         uint4 x = make_uint4(0, 0, 0, 0);
         if (irow < rows) x = *reinterpret_cast<const uint4*>(qp + 32 * ks);
-        qf[ks] = as_bf16x8(x);
+        qf[ks] = query(x);
       }
     }
     // inter-chunk slot logits: okT[m][i] = sum_d hkT[m][d] q[i][d]
