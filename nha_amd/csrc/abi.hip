@@ -91,6 +91,14 @@ static int check_prefill_bwd(const NhaPrefillBwdArgs* a, bool pointers) {
   return NHA_OK;
 }
 
+// Kernels add a token's index to the window in 32 bits.  No call holds 2^30 tokens, so that a longer window sees what this one sees.
+template <class Args>
+static Args with_window_in_range(const Args* a) {
+  Args b = *a;
+  if (b.wl > (1 << 30)) b.wl = 1 << 30;
+  return b;
+}
+
 static bool use_mfma(const NhaPrefillArgs* a) {
   if (a->impl == NHA_IMPL_SIMPLE) return false;
   return prefill_mfma_supported(a);
@@ -144,7 +152,8 @@ static int prefill_fwd_phase(const NhaPrefillArgs* a, int phase) {
     set_error("nha_prefill_fwd: scratch has %zu bytes, %zu needed", a->scratch_bytes, need);
     return NHA_ERR_SCRATCH;
   }
-  return run_prefill(a, mfma, phase);
+  const NhaPrefillArgs b = with_window_in_range(a);
+  return run_prefill(&b, mfma, phase);
 }
 
 int nha_prefill_fwd_noalloc(const NhaPrefillArgs* a) {
@@ -167,7 +176,7 @@ int nha_prefill_fwd_noalloc(const NhaPrefillArgs* a) {
   if (rc != NHA_OK) return rc;
   // nothing in the scratch has to start at zero: the state pass writes every table the output pass
   // reads (rows past a sequence's end are never read), so the previous call's contents are harmless
-  NhaPrefillArgs b = *a;
+  NhaPrefillArgs b = with_window_in_range(a);
   b.scratch = ptr;
   b.scratch_bytes = (size_t)NHA_NOALLOC_SCRATCH_BYTES;
   return run_prefill(&b, mfma, 0);
@@ -190,7 +199,8 @@ int nha_prefill_bwd(const NhaPrefillBwdArgs* a) {
     set_error("nha_prefill_bwd: scratch has %zu bytes, %zu needed", a->scratch_bytes, need);
     return NHA_ERR_SCRATCH;
   }
-  return prefill_bwd_impl(a);
+  const NhaPrefillBwdArgs b = with_window_in_range(a);
+  return prefill_bwd_impl(&b);
 }
 
 size_t nha_decode_scratch_bytes(void) { return decode_scratch_bytes(); }

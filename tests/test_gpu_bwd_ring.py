@@ -63,3 +63,19 @@ def test_scale_of_zero(wl, scale):
     """All keys of the window weigh the same; dk_swa is zero, or nearly so, and finite."""
     print("case", wl, scale, flush=True)
     compare([0, 1, 40, 104, 361, 1190], wl, 32, 4, 128, ("k_swa", "v"), scale=scale)
+
+
+@pytest.mark.parametrize("H,NG,D,dt", [(32, 4, 128, BF), (2, 4, 128, BF), (16, 1, 256, BF), (2, 1, 256, BF), (4, 1, 64, BF), (4, 1, 64, torch.float32)])
+@pytest.mark.parametrize("wl", [2**31 - 1, 2**31 - 1000, 2**30])
+def test_longest_windows_are_unbounded(wl, H, NG, D, dt):
+    from nha_amd import chunk_nha
+    print("case", wl, H, NG, D, dt, flush=True)
+    cu = torch.tensor([0, 1, 40, 104, 361, 1190], dtype=torch.int32).cuda()
+    d = prefill_inputs(5, 1, 1190, H * NG, H, D, D, 64, dtype=dt)
+    do = torch.randn(1, 1190, H * NG, D, generator=torch.Generator().manual_seed(2)).to(dt).cuda()
+    res = []
+    for w in (-1, wl):
+        x = [d[k].cuda().requires_grad_(True) for k in KEYS]
+        out = chunk_nha(*x, cu_seqlens=cu, window_size_left=w, gsa_kv_shift=0)
+        res.append([*out, *torch.autograd.grad(out[0], x, do)])
+    assert all(torch.equal(p, q) for p, q in zip(*res))
