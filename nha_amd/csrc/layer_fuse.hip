@@ -38,30 +38,38 @@ template <> __device__ __forceinline__ float rnd<bf16_t>(float x) { return bf16_
 __device__ __forceinline__ float silu_f(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 __device__ __forceinline__ float feature_f(float x, int fm) { return fm == 1 ? silu_f(x) : (fm == 2 ? fmaxf(x, 0.f) : x); }
 
+// The gates' functions in fp32.  For bf16 tensors they are formed here, for half of the library's instructions: correct to a little more
+// than a unit in the last place of fp32, subnormal results included, and, what is checked for every bf16 argument, the library's
+// number once it is rounded to bf16.
+
+// e^x: 2^n 2^f with |f| <= 1/2 and the rounding of x log2(e) made good
+__device__ __forceinline__ float exp_f(float x) {
+  x = x < -150.f ? -150.f : x;   // (a NaN stays one)
+  x = x > 100.f ? 100.f : x;
+  const float n = rintf(x * 1.44269502f);
+  const float f = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -n));
+  return ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+}
 // ls = log(1 / (1 + e^-x)), rounded to T
 template <typename T> __device__ __forceinline__ float logsigmoid_f(float x);
 template <> __device__ __forceinline__ float logsigmoid_f<float>(float x) { return fminf(x, 0.f) - log1pf(expf(-fabsf(x))); }
-// bf16: u = e^-|x| with the rounding of x log2(e) made good, log(1 + u) = 2 atanh(u / (2 + u)) by its series to the 15th power of
-// at most 1/3: 3 ulp of float32, a thousandth of the rounding that follows, for a third of the library's instructions
+// bf16: u = e^-|x|, log(1 + u) = 2 atanh(s) by its series to the 15th power of s = u / (2 + u) <= 1/3, s with its remainder made good
 template <> __device__ __forceinline__ float logsigmoid_f<bf16_t>(float x) {
-  const float a = -fabsf(x), t = a * 1.44269502f, lost = fmaf(a, 1.44269502f, -t) + a * 1.92596299e-8f;
-  const float e = __builtin_amdgcn_exp2f(t), u = a < -87.f ? e : fmaf(e, lost * 0.693147181f, e);   // (-inf: lost is NaN)
-  const float s = u * __builtin_amdgcn_rcpf(2.f + u), q = s * s;
+  const float u = exp_f(-fabsf(x)), d = 2.f + u, dlo = (2.f - d) + u, rc = __builtin_amdgcn_rcpf(d);
+  const float s0 = u * rc, s = fmaf(fmaf(-s0, dlo, fmaf(-s0, d, u)), rc, s0), q = s * s;
   float r = fmaf(q, 2.f / 15.f, 2.f / 13.f);
   r = fmaf(q, r, 2.f / 11.f);
   r = fmaf(q, r, 2.f / 9.f);
   r = fmaf(q, r, 2.f / 7.f);
   r = fmaf(q, r, 2.f / 5.f);
   r = fmaf(q, r, 2.f / 3.f);
-  r = fmaf(q, r, 2.f);
-  return rnd<bf16_t>(fminf(x, 0.f) - s * r);
+  const float l = fmaf(s * q, r, 2.f * s);
+  return rnd<bf16_t>(fminf(x, 0.f) - (u < 2.98e-8f ? u : l));   // (2^-25: log(1 + u) = u, and s would lose bits of a subnormal u)
 }
-// e^x, x <= 0 (a log gate; bf16: off by |x| 2^-24, then rounded to 8 bits)
+// e^x of a log gate
 template <typename T> __device__ __forceinline__ float exp_gate_f(float x);
 template <> __device__ __forceinline__ float exp_gate_f<float>(float x) { return expf(x); }
-template <> __device__ __forceinline__ float exp_gate_f<bf16_t>(float x) {
-  return __builtin_amdgcn_exp2f(fmaf(x, 1.44269502f, x * 1.92596299e-8f));
-}
+template <> __device__ __forceinline__ float exp_gate_f<bf16_t>(float x) { return exp_f(x); }
 
 template <typename T, int VEC> __device__ __forceinline__ void ldv(const T* p, float* o) {
   if constexpr (VEC == 8) {

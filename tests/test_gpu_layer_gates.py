@@ -36,3 +36,21 @@ def test_gates_of_every_bf16_logit(H, normalizer):
     want = torch.sigmoid(-x) / normalizer
     ok = want > 2.0 ** -120
     assert ((dg - want).abs()[ok] <= 2.0 ** -8 * 1.01 * want[ok]).all()
+
+
+@pytest.mark.parametrize("H", [4, 8])
+@pytest.mark.parametrize("normalizer", [1.0, 8.0, 16.0, 0.5, 3.0, -1.0])
+def test_gates_are_the_rounded_values(H, normalizer):
+    """Every bf16 logit, subnormal results and NaN included: the values of the 64-bit chain, each step rounded to bf16 once."""
+    from nha_amd.ops import nha_layer_prologue
+    M, K = 64, 16
+    f = torch.arange(65536, dtype=torch.int32).to(torch.uint16).view(torch.bfloat16).view(1, -1, H, M).cuda()
+    z = torch.zeros(1, f.shape[1], H, K, dtype=torch.bfloat16, device="cuda")
+    out = nha_layer_prologue(z, z, z, f, torch.ones(K // 2, device="cuda"), feature_map="swish", gate_logit_normalizer=normalizer)
+    s, g = out[5].double(), out[6].double()
+    r = lambda x: x.to(torch.bfloat16).double()
+    x = f.double()
+    want = r(r(x.clamp(max=0) - torch.log1p(torch.exp(-x.abs()))) / normalizer)
+    same = lambda a, b: torch.equal(a.nan_to_num(7.0, torch.inf, -torch.inf), b.nan_to_num(7.0, torch.inf, -torch.inf))
+    assert same(g, want) and torch.equal(g.isnan(), x.isnan())
+    assert same(s, r(1 - r(torch.exp(g)))) and torch.equal(s.isnan(), x.isnan())
