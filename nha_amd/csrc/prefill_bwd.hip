@@ -836,9 +836,10 @@ __global__ __launch_bounds__(256) void bwd_gate_final_kernel(const BP p) {
       const int64_t step = (int64_t)H * M;
       for (int c = chunk + 1 + r0; c < last; c += 32) {
         const float4 a = *reinterpret_cast<const float4*>(g + c * step);
-        const float4 b = *reinterpret_cast<const float4*>(g + (c + 16 < last ? c + 16 : c) * step);
-        const float on = c + 16 < last ? 1.f : 0.f;
-        gt.x += a.x + on * b.x; gt.y += a.y + on * b.y; gt.z += a.z + on * b.z; gt.w += a.w + on * b.w;
+        const bool two = c + 16 < last;
+        const float4 b = *reinterpret_cast<const float4*>(g + (two ? c + 16 : c) * step);
+        // (chosen, not multiplied by 0: the sum of a chunk may be infinite)
+        gt.x += a.x + (two ? b.x : 0.f); gt.y += a.y + (two ? b.y : 0.f); gt.z += a.z + (two ? b.z : 0.f); gt.w += a.w + (two ? b.w : 0.f);
       }
     } else {
       gt = *reinterpret_cast<const float4*>(p.gtot + ((int64_t)chunk * H + h) * M + m);

@@ -34,3 +34,25 @@ def test_sum_over_later_chunks_is_the_scan(lens, shift, dtype):
     bound = 2 * 34 * 2.0 ** -24 * 2 * y.abs().amax() + 2 * half * torch.maximum(x.abs(), y.abs())
     assert ((x - y).abs() <= bound).all()
     assert x.abs().sum() > 0 or T <= shift
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_infinite_sum_of_a_later_chunk(dtype):
+    """The gate gradients of a sequence's last chunk add up to more than float32 holds: those before are infinite, not NaN."""
+    from nha_amd.ops import nha_prefill, nha_prefill_bwd
+    cu = np.array([0, 192], np.int32)
+    T, H, D, M = 192, 2, 64, 64
+    one = torch.ones(T, H, D, dtype=dtype, device="cuda")
+    strength = torch.zeros(T, H, M, dtype=dtype, device="cuda")
+    strength[..., 0] = 1
+    xs = [one] * 5 + [strength, torch.zeros_like(strength)]
+    kw = dict(wl=31, shift=0, scale=1.0)
+    o, lw, lg, _, _ = nha_prefill(*xs, cu, **kw)
+    # slot 0 alone is written and read: its logit is 64 (t + 1) in row t, exact in every step, with the cotangent c = 2^111, and dg of row r is
+    # 64 c r (T - r): 3e37 at the last row, 1.4e39 at the first of the last chunk (row 128), 1.1e39 at row 48, whose own chunk adds
+    # -2.5e38 to the infinite sum (from rows further up it would be -inf)
+    dl = torch.full((T, H), 2.0 ** 111, device="cuda")
+    zero = tuple(torch.zeros(1, H, 64, 64, device="cuda") for _ in range(2))
+    a, b = (nha_prefill_bwd(*xs, o, lw, lg, torch.zeros_like(o), cu, dlse_gsa=dl, dht=dht, **kw)[6][..., 0].float() for dht in (None, zero))
+    assert (b[48:129] == torch.inf).all() and b[188:].isfinite().all()
+    assert (a[48:129] == torch.inf).all() and torch.equal(a[188:], b[188:])
