@@ -91,14 +91,18 @@ __device__ __forceinline__ void xcd_tile(int ngrp, int nchunks, int& vx, int& vy
 }
 
 // Two chunks of a sequence per workgroup: launch index -> (head x, sequence n, first chunk it of the pair); false for the
-// workgroups beyond the last pair.  The launch (pair_grid) has room for the most pairs that NT chunks in N sequences can make;
-// the pairs are counted without gaps, so that the working workgroups come first: left strewn over the launch order, those that
-// leave at once give the shader engines unequal shares of the others (2 x 4000 tokens, 4 heads: 256 pairs on 256 CUs took two
-// rounds).  As in xcd_tile XCD k takes the k-th eighth of the sequence (kv-head, pair, head of the kv-head's ngrp), the
-// pairs from the last to the first.  Each wave counts for itself, 64 sequences at a time.
+// workgroups without one.  The launch (pair_grid) has room for the most pairs that NT chunks in N sequences can make.
+// As in xcd_tile XCD k takes the k-th eighth of the sequence (kv-head, pair, head of the kv-head's ngrp), the
+// pairs from the last to the first.
+// Up to 64 sequences the pairs are counted without gaps, so that the working workgroups come first: left strewn over the launch
+// order, those that leave at once give the shader engines unequal shares of the others (2 x 4000 tokens, 4 heads: 256 pairs on 256
+// CUs took two rounds).  Each wave counts for itself, a sequence per lane.
+// More sequences are not counted, which takes longer the more there are (chunk_nha without / with gradients, 4 heads, W = 512, counted / searched:
+// 1000 sequences of 130 tokens 1803 / 1605 and 9435 / 8785 us, 3000 of them 6452 / 5055 and 32437 / 27475): sequence n has the places (coff[n] + n) / 2 to
+// (coff[n + 1] + n + 1) / 2, its pairs and where it has an even number of chunks now and then one more (every third place of
+// two-chunk sequences, so no engine's in particular), and is found by a search in steps of 64.
 __device__ __forceinline__ bool pair_tile(const int32_t* coff, int N, int heads, int ngrp, int& x, int& n, int& it) {
   const int lane = threadIdx.x & 63, L = blockIdx.x;
-  auto pairs = [&](int n0) { return n0 + lane < N ? (coff[n0 + lane + 1] - coff[n0 + lane] + 1) >> 1 : 0; };
   auto prefix = [&](int c) {   // over the wave, inclusive (DPP: rows of 16 lanes, then across the rows)
     c += __builtin_amdgcn_update_dpp(0, c, 0x111, 0xf, 0xf, false);
     c += __builtin_amdgcn_update_dpp(0, c, 0x112, 0xf, 0xf, false);
@@ -108,27 +112,34 @@ __device__ __forceinline__ bool pair_tile(const int32_t* coff, int N, int heads,
     c += __builtin_amdgcn_update_dpp(0, c, 0x143, 0xc, 0xf, false);
     return c;
   };
-  int c = pairs(0), incl = prefix(c), total = __builtin_amdgcn_readlane(incl, 63);
-  for (int n0 = 64; n0 < N; n0 += 64) total += __builtin_amdgcn_readlane(prefix(pairs(n0)), 63);
+  int c = 0, incl = 0, total;
+  if (N <= 64) {
+    c = lane < N ? (coff[lane + 1] - coff[lane] + 1) >> 1 : 0;
+    incl = prefix(c);
+    total = __builtin_amdgcn_readlane(incl, 63);
+  } else {
+    total = (coff[N] + N) >> 1;
+  }
   const int work = heads * total, per = work >> 3;
   if (L >= work) return false;
   const int v = L < 8 * per ? (L & 7) * per + (L >> 3) : L, g = v % ngrp, rest = v / ngrp;
   x = (rest / total) * ngrp + g;
   const int k = total - 1 - rest % total;
-  int base = 0;
-  for (int n0 = 0; n0 < N; n0 += 64) {
-    if (n0) c = pairs(n0), incl = prefix(c);
-    const int first = base + incl - c;
-    const uint64_t hit = __ballot(k >= first && k < first + c);
-    if (hit) {
-      const int at = __builtin_ctzll(hit);
-      n = n0 + at;
-      it = 2 * (k - __builtin_amdgcn_readlane(first, at));
-      return true;
-    }
-    base += __builtin_amdgcn_readlane(incl, 63);
+  if (N <= 64) {
+    n = __builtin_ctzll(__ballot(k >= incl - c && k < incl));
+    it = 2 * (k - __builtin_amdgcn_readlane(incl - c, n));
+    return true;
   }
-  return false;
+  int step = 64;
+  while (step * 64 < N) step *= 64;
+  n = 0;   // the first place of sequence n is at k or before, and that of n + 64 step is not
+  for (; step; step >>= 6) {
+    const int i = n + lane * step;
+    const uint64_t before = __ballot(i < N && (coff[i < N ? i : 0] + i) >> 1 <= k);
+    n += (__popcll(before) - 1) * step;
+  }
+  it = 2 * (k - ((coff[n] + n) >> 1));
+  return it < coff[n + 1] - coff[n];
 }
 static inline dim3 pair_grid(int heads, int NT, int N) { return dim3((unsigned)heads * ((unsigned)(NT + N) / 2)); }
 

@@ -40,13 +40,15 @@ def test_window_gradients_of_many_key_groups(wl, H, NG, D):
     compare(cu, wl, H, NG, D, ("q_swa", "k_swa", "v"))
 
 
+@pytest.mark.parametrize("N,H", [(64, 4), (65, 4), (150, 4), (4097, 1)])
 @pytest.mark.parametrize("wl", [40, 400])
-def test_more_sequences_than_lanes(wl):
-    """The workgroups of two chunks count the pairs of 64 sequences at a time: 150 of them, empty ones among them."""
-    lens = [(37 * i) % 131 for i in range(150)]
+def test_more_sequences_than_lanes(wl, N, H):
+    """The workgroups of two chunks count the pairs of up to 64 sequences and search among more, in steps of 64 and of 4096; empty ones among
+    them, one to three chunks."""
+    lens = [(37 * i) % 131 for i in range(N)] if N < 4096 else [(65, 1, 0, 130, 2, 66)[i % 6] for i in range(N)]
     cu = torch.tensor([0, *lens]).cumsum(0).tolist()
-    print("case", wl, flush=True)
-    compare(cu, wl, 4, 1, 256, KEYS)
+    print("case", wl, N, H, flush=True)
+    compare(cu, wl, H, 1, 256, KEYS)
 
 
 @pytest.mark.parametrize("H,NG,D", [(32, 4, 128), (16, 1, 256)])
