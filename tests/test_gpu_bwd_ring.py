@@ -1,7 +1,8 @@
 """Window gradients from the LDS-direct kernels (K = V = 128: four or eight query heads per kv-head, more key groups than 128;
-K = V = 256: any grouping, more than 256 chunks x kv-heads) against the fp32 call (generic kernels) on the same bf16-rounded
-inputs: ragged packed sequences that end inside a 32-row unit, a chunk and a group of chunks, windows below and above those where
-the kernels and their key groups change, odd and even numbers of units, longer than every sequence and unbounded."""
+K = V = 256: any grouping, more than 256 chunks x kv-heads, few empty halves of 128-row workgroups) against the fp32 call (generic
+kernels) on the same bf16-rounded inputs: ragged packed sequences that end inside a 32-row unit, a chunk and a group of chunks,
+windows below and above those where the kernels and their key groups change, odd and even numbers of units, longer than every
+sequence and unbounded."""
 import pytest
 import torch
 
@@ -29,10 +30,14 @@ def compare(cu, wl, H, NG, D, keys, scale=None):
             check_grad(f"wl={wl} d{k}", gb, gf.double().cpu(), BF)
 
 
-@pytest.mark.parametrize("H,NG,D", [(32, 4, 128), (32, 8, 128), (16, 1, 256), (13, 3, 256)])
+# 1, 1, 1, 5 and 13 chunks: seven in eight halves of 128-row workgroups are taken as filled (too few for some of the 256-wide kernels); 1, 1, 1, 5
+# and 12, four on average: all
+CU, CU256 = [0, 1, 40, 104, 361, 1190], [0, 1, 40, 104, 361, 1126]
+
+
+@pytest.mark.parametrize("H,NG,D,cu", [(32, 4, 128, CU), (32, 8, 128, CU), (16, 1, 256, CU), (13, 3, 256, CU), (16, 1, 256, CU256), (13, 3, 256, CU256)])
 @pytest.mark.parametrize("wl", [-1, 0, 31, 64, 159, 160, 192, 383, 384, 500, 2000])
-def test_window_gradients_of_many_key_groups(wl, H, NG, D):
-    cu = [0, 1, 40, 104, 361, 1190]
+def test_window_gradients_of_many_key_groups(wl, H, NG, D, cu):
     print("case", wl, H, NG, D, flush=True)
     # otherwise other kernels take dk and dv
     chunks = sum((b - a + 63) // 64 for a, b in zip(cu, cu[1:]))
@@ -40,23 +45,24 @@ def test_window_gradients_of_many_key_groups(wl, H, NG, D):
     compare(cu, wl, H, NG, D, ("q_swa", "k_swa", "v"))
 
 
-@pytest.mark.parametrize("N,H", [(64, 4), (65, 4), (150, 4), (4097, 1)])
+@pytest.mark.parametrize("N,H", [(64, 4), (68, 4), (152, 4), (4100, 1)])
 @pytest.mark.parametrize("wl", [40, 400])
 def test_more_sequences_than_lanes(wl, N, H):
-    """The workgroups of two chunks count the pairs of up to 64 sequences and search among more, in steps of 64 and of 4096; empty ones among
-    them, one to three chunks."""
-    lens = [(37 * i) % 131 for i in range(N)] if N < 4096 else [(65, 1, 0, 130, 2, 66)[i % 6] for i in range(N)]
+    """The workgroups of two chunks count the pairs of up to 64 sequences and search among more, in steps of 64 and of 4096: one to three chunks
+    each, two on average (taken as filled; the 256-wide window gradients of others fall to kernels of 64 rows), empty ones among them."""
+    lens = [(65, 1, 130, 66)[i % 4] for i in range(N)]
+    lens[N // 2:N // 2] = [0, 0]
     cu = torch.tensor([0, *lens]).cumsum(0).tolist()
     print("case", wl, N, H, flush=True)
     compare(cu, wl, H, 1, 256, KEYS)
 
 
-@pytest.mark.parametrize("H,NG,D", [(32, 4, 128), (16, 1, 256)])
+@pytest.mark.parametrize("H,NG,D,cu", [(32, 4, 128, CU), (16, 1, 256, CU), (16, 1, 256, CU256)])
 @pytest.mark.parametrize("wl", [-1, 64, 200, 500])
-def test_negative_scale(wl, H, NG, D):
+def test_negative_scale(wl, H, NG, D, cu):
     """The weights of the keys outside the window are zero whatever the sign of the scale."""
     print("case", wl, H, NG, D, flush=True)
-    compare([0, 1, 40, 104, 361, 1190], wl, H, NG, D, KEYS, scale=-D ** -0.5)
+    compare(cu, wl, H, NG, D, KEYS, scale=-D ** -0.5)
 
 
 @pytest.mark.parametrize("scale", [0.0, 1e-42, -1e-42, 1e-28])
@@ -64,7 +70,7 @@ def test_negative_scale(wl, H, NG, D):
 def test_scale_of_zero(wl, scale):
     """All keys of the window weigh the same; dk_swa is zero, or nearly so, and finite."""
     print("case", wl, scale, flush=True)
-    compare([0, 1, 40, 104, 361, 1190], wl, 32, 4, 128, ("k_swa", "v"), scale=scale)
+    compare(CU, wl, 32, 4, 128, ("k_swa", "v"), scale=scale)
 
 
 @pytest.mark.parametrize("H,NG,D,dt", [(32, 4, 128, BF), (2, 4, 128, BF), (16, 1, 256, BF), (2, 1, 256, BF), (4, 1, 64, BF), (4, 1, 64, torch.float32)])
@@ -72,9 +78,9 @@ def test_scale_of_zero(wl, scale):
 def test_longest_windows_are_unbounded(wl, H, NG, D, dt):
     from nha_amd import chunk_nha
     print("case", wl, H, NG, D, dt, flush=True)
-    cu = torch.tensor([0, 1, 40, 104, 361, 1190], dtype=torch.int32).cuda()
-    d = prefill_inputs(5, 1, 1190, H * NG, H, D, D, 64, dtype=dt)
-    do = torch.randn(1, 1190, H * NG, D, generator=torch.Generator().manual_seed(2)).to(dt).cuda()
+    cu = torch.tensor(CU256, dtype=torch.int32).cuda()
+    d = prefill_inputs(5, 1, CU256[-1], H * NG, H, D, D, 64, dtype=dt)
+    do = torch.randn(1, CU256[-1], H * NG, D, generator=torch.Generator().manual_seed(2)).to(dt).cuda()
     res = []
     for w in (-1, wl):
         x = [d[k].cuda().requires_grad_(True) for k in KEYS]
