@@ -6,7 +6,7 @@
 //             (nha_fla/layers/nha.py:278).
 // Both are HBM-bound streaming kernels: one wave per token (four tokens per workgroup), 16-byte
 // accesses, every input element read once and every output element written once (8 x 2048 tokens, 4 heads of 256, 64 slots:
-// prologue 49 us, its backward 75, 403 MB at the rate of a copy; 65 and 91 with the library's log1p and exponentials for the
+// prologue 51 us, its backward 78, 403 MB at the rate of a copy; 65 and 91 with the library's log1p and exponentials for the
 // gates, eight of them to a lane and half of the lanes idle, bound by the vector units).  Intermediate results are rounded to
 // the tensor dtype at the points where the reference's chain of tensor ops rounds them.
 #include "common.h"

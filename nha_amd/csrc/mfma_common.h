@@ -92,15 +92,16 @@ __device__ __forceinline__ void xcd_tile(int ngrp, int nchunks, int& vx, int& vy
 
 // Two chunks of a sequence per workgroup: launch index -> (head x, sequence n, first chunk it of the pair); false for the
 // workgroups without one.  The launch (pair_grid) has room for the most pairs that NT chunks in N sequences can make.
-// As in xcd_tile XCD k takes the k-th eighth of the sequence (kv-head, pair, head of the kv-head's ngrp), the
-// pairs from the last to the first.
+// As in xcd_tile XCD k takes the k-th eighth of the sequence (kv-head, pair, head of the kv-head's ngrp), the pairs from the last
+// to the first.
 // Up to 64 sequences the pairs are counted without gaps, so that the working workgroups come first: left strewn over the launch
 // order, those that leave at once give the shader engines unequal shares of the others (2 x 4000 tokens, 4 heads: 256 pairs on 256
 // CUs took two rounds).  Each wave counts for itself, a sequence per lane.
-// More sequences are not counted, which takes longer the more there are (chunk_nha without / with gradients, 4 heads, W = 512, counted / searched:
-// 1000 sequences of 130 tokens 1803 / 1605 and 9435 / 8785 us, 3000 of them 6452 / 5055 and 32437 / 27475): sequence n has the places (coff[n] + n) / 2 to
-// (coff[n + 1] + n + 1) / 2, its pairs and where it has an even number of chunks now and then one more (every third place of
-// two-chunk sequences, so no engine's in particular), and is found by a search in steps of 64.
+// More sequences are not counted, which takes longer the more there are (chunk_nha without / with gradients, 4 heads, W = 512,
+// counted / searched: 1000 sequences of 130 tokens 1803 / 1605 and 9435 / 8785 us, 3000 of them 6452 / 5055 and 32437 / 27475):
+// sequence n has the places (coff[n] + n) / 2 to (coff[n + 1] + n + 1) / 2, its pairs and where it has an even number of chunks now
+// and then one more (every third place of two-chunk sequences, so no engine's in particular), and is found by a search in steps of
+// 64.
 __device__ __forceinline__ bool pair_tile(const int32_t* coff, int N, int heads, int ngrp, int& x, int& n, int& it) {
   const int lane = threadIdx.x & 63, L = blockIdx.x;
   auto prefix = [&](int c) {   // over the wave, inclusive (DPP: rows of 16 lanes, then across the rows)

@@ -665,7 +665,7 @@ __global__ __launch_bounds__(256) void bwd_state_inter_kernel(const BP p) {
 // ------------------------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_gate_local_kernel(const BP p) {
-  // M == 64 (the matrix-core path): thread = (group rg of 4 consecutive rows, 4 consecutive slots), 16-byte
+  // M == 64: thread = (group rg of 4 consecutive rows, 4 consecutive slots), 16-byte
   // reads, all of a thread's rows requested together; the reverse cumulative sum is a suffix sum over the
   // thread's rows plus the sums of the later groups through LDS.  Other M: thread = (group of 16 rows, slot).
   __shared__ float gs[16][BT];
@@ -1018,7 +1018,10 @@ BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f, size_t fwd
   }
   s.xg = take(s.use_mfma ? thm : tqm);
   s.delta = take((size_t)a->T_tot * a->HQ * 4);
-  s.ld = take((size_t)a->T_tot * a->HQ * 8);   // (-lse / scale, -delta) pairs of the LDS-direct window kernels
+  // What the LDS-direct dk / dv kernels start their sums from, a pair per (token, query head).  Head size 128: (-lse / scale,
+  // -delta), from ring_dq_kernel to ring_dkv_kernel.  Head size 256: (-lse log2(e), -delta), from ring256_dq_kernel or
+  // bwd_dq_kernel to ring256_dkv_kernel.
+  s.ld = take((size_t)a->T_tot * a->HQ * 8);
   s.dsi = take(thm);
   s.dsp = take(thm * (s.nbk + s.nbv));
   s.dvs = take((size_t)a->T_tot * a->H * a->V * 4);

@@ -5,8 +5,9 @@
 // the window logits w[q][j] = scale q_swa_q . k_swa_j (j in [max(bos, q - wl), q]) give
 //   pi = e^(w - lse),  dpi = do_q . v_j,  dw = pi (dpi - delta),
 //   dq_swa_q = scale sum_j dw k_swa_j,   dk_swa_j = scale sum_q dw q_swa_q,   dv_j += sum_q pi do_q.
-// Two kernels, for what prefill_bwd_ring.hip and prefill_bwd_ring256.hip do not take, each in the orientation whose accumulator layout feeds its next MFMA without moving
-// data between lanes (v_mfma_f32_16x16x32_bf16: A[i][8(l/16)+e], B[8(l/16)+e][j], C[4(l/16)+r][l%16]):
+// Two kernels, for what prefill_bwd_ring.hip and prefill_bwd_ring256.hip do not take, each in the orientation whose
+// accumulator layout feeds its next MFMA without moving data between lanes (v_mfma_f32_16x16x32_bf16: A[i][8(l/16)+e],
+// B[8(l/16)+e][j], C[4(l/16)+r][l%16]):
 //   bwd_dq_kernel   one workgroup per (64 queries, q-head); K/V tiles stream through LDS;
 //                   S^T = K Q^T and dP^T = V dO^T put a query per lane, dQ^T += K^T dS^T
 //   bwd_dkv_kernel  one workgroup per (64 keys, kv-head); Q/dO tiles of every q-head of the group

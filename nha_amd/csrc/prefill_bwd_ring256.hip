@@ -495,32 +495,34 @@ static bool served(const NhaPrefillBwdArgs* a) {
   return a->K == 256 && a->V == 256 && (int64_t)a->T_tot * a->HQ * 256 * 2 < ((int64_t)1 << 32);
 }
 
-// A sequence with an odd number of chunks leaves half of its last workgroup of 128 rows empty, which calls of short sequences feel.  Whether
-// `percent` of the halves have rows: equally long sequences are taken as such (c of 2 ceil(c / 2) halves at c chunks each); of others, the
-// shorter ones weighing more than their rows, three in four as odd.
+// A sequence with an odd number of chunks leaves half of its last workgroup of 128 rows empty, which calls of short sequences feel.
+// Whether `percent` of the halves have rows: equally long sequences are taken as such (c of 2 ceil(c / 2) halves at c chunks each);
+// of others, the shorter ones weighing more than their rows, three in four as odd.
 static bool filled(const NhaPrefillBwdArgs* a, int percent) {
   const int64_t NT = a->NT, N = a->N;
   const int64_t halves = NT % N == 0 ? 2 * N * ((NT / N + 1) / 2) : NT + 3 * N / 4;
   return 100 * NT >= percent * halves;
 }
 
-// A workgroup of 128 rows begins with 128 KB that nothing hides (11 of bwd_dq_kernel's 64 rows wait on a CU shared by two), which long
-// windows pay back.  us, bwd_dq_kernel / ring256_dq_kernel, 4 heads: W = 64 13.3 / 17.7 at 1000 tokens and 49 / 52 at 3 x 5000;
-// W = 256 23 / 26 at 1000 and 129 / 128 at 30000 packed; W = 512 35.0 / 35.2 at 1000, 38 / 38 at 4000, 52 / 45 at 2 x 4000, 98 / 88
-// at 3 x 5000; W = 1024 56 / 50 at 1000, 80 / 66 at 2 x 4000.
-// Short sequences, W = 512: 120 of 130 tokens (75 % filled) 54 / 74, of 256 (100 %) 116 / 102, of 400 (88 %) 175 / 223, of 513 (90 %) 269 / 270, 8 of 700
-// (92 %) 46 / 37, 60 of 960 (94 %) 264 / 265; ragged, 500 of 300 on average (87 %) 500 / 570, 80 of 400 (90 %) 142 / 145, 60 of 600 (93 %) 160 / 157.
+// A workgroup of 128 rows begins with 128 KB that nothing hides (11 of bwd_dq_kernel's 64 rows wait on a CU shared by two), which
+// long windows pay back.  us, bwd_dq_kernel / ring256_dq_kernel, 4 heads: W = 64 13.3 / 17.7 at 1000 tokens and 49 / 52 at 3 x
+// 5000; W = 256 23 / 26 at 1000 and 129 / 128 at 30000 packed; W = 512 35.0 / 35.2 at 1000, 38 / 38 at 4000, 52 / 45 at 2 x 4000,
+// 98 / 88 at 3 x 5000; W = 1024 56 / 50 at 1000, 80 / 66 at 2 x 4000.
+// Short sequences, W = 512: 120 of 130 tokens (75 % filled) 54 / 74, of 256 (100 %) 116 / 102, of 400 (88 %) 175 / 223, of 513 (90
+// %) 269 / 270, 8 of 700 (92 %) 46 / 37, 60 of 960 (94 %) 264 / 265; ragged, 500 of 300 on average (87 %) 500 / 570, 80 of 400 (90
+// %) 142 / 145, 60 of 600 (93 %) 160 / 157.
 bool bwd_ring256_dq_supported(const NhaPrefillBwdArgs* a) { return served(a) && (a->wl < 0 || a->wl >= 384) && filled(a, 91); }
 
-// One workgroup of 128 keys fills a CU where bwd_dkv_kernel has four of 64 (two per CU), and walks all heads of its group: it
-// pays from half of the chip on, and with one head and short windows not yet.  us, bwd_dkv_kernel / ring256_dkv_kernel: 4 / 4 heads,
-// 2 x 4000 tokens (256 groups) W = 64 47 / 43, W = 256 69 / 52, W = 512 102 / 73, W = 1024 149 / 92; 2 x 6000 (376) 72 / 81,
-// 104 / 101, -, 235 / 178; 4000 tokens (128) 25 / 33, 36 / 43, 52 / 60, 82 / 83; 8 / 2 heads, 2 x 4000 (128) 50 / 69, 95 / 110, 153 / 178,
-// 262 / 264; 2 x 6000 (188) 86 / 74, 172 / 115, -, 506 / 270.
-// Short sequences: 4 / 4 heads, W = 512, 120 of 130 tokens 105 / 142, of 256 211 / 170, of 400 347 / 382, of 513 523 / 435; ragged, 240 of 150 on average
-// (79 % filled) 229 / 251, 160 of 200 (83 %) 217 / 215, 80 of 400 (90 %) 260 / 231.  8 / 2 heads, W = 512: 1000 of 130 836 / 1030, 120 of 300 (83 %)
-// 331 / 266; ragged, 300 of 100 (73 %) 212 / 214, 240 of 150 306 / 257.  8 / 2 heads, W = 64: 120 of 130 122 / 130, of 256 198 / 157, of 400 297 / 302,
-// of 600 443 / 375; ragged, 300 of 100 194 / 216, 80 of 400 201 / 217, 500 of 600 (93 %) 1807 / 1525.
+// One workgroup of 128 keys fills a CU where bwd_dkv_kernel has four of 64 (two per CU), and walks all heads of its group: it pays
+// from half of the chip on, and with one head and short windows not yet.  us, bwd_dkv_kernel / ring256_dkv_kernel: 4 / 4 heads, 2 x
+// 4000 tokens (256 groups) W = 64 47 / 43, W = 256 69 / 52, W = 512 102 / 73, W = 1024 149 / 92; 2 x 6000 (376) 72 / 81, 104 / 101,
+// -, 235 / 178; 4000 tokens (128) 25 / 33, 36 / 43, 52 / 60, 82 / 83; 8 / 2 heads, 2 x 4000 (128) 50 / 69, 95 / 110, 153 / 178, 262
+// / 264; 2 x 6000 (188) 86 / 74, 172 / 115, -, 506 / 270.
+// Short sequences: 4 / 4 heads, W = 512, 120 of 130 tokens 105 / 142, of 256 211 / 170, of 400 347 / 382, of 513 523 / 435; ragged,
+// 240 of 150 on average (79 % filled) 229 / 251, 160 of 200 (83 %) 217 / 215, 80 of 400 (90 %) 260 / 231.  8 / 2 heads, W = 512:
+// 1000 of 130 836 / 1030, 120 of 300 (83 %) 331 / 266; ragged, 300 of 100 (73 %) 212 / 214, 240 of 150 306 / 257.  8 / 2 heads, W =
+// 64: 120 of 130 122 / 130, of 256 198 / 157, of 400 297 / 302, of 600 443 / 375; ragged, 300 of 100 194 / 216, 80 of 400 201 /
+// 217, 500 of 600 (93 %) 1807 / 1525.
 bool bwd_ring256_dkv_supported(const NhaPrefillBwdArgs* a) {
   if (!served(a) || (int64_t)a->H * a->NT <= 256) return false;
   const bool wide = a->wl < 0 || a->wl >= 192;

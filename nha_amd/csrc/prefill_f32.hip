@@ -18,9 +18,9 @@
 // Everything is computed transposed (a query per lane), with operands loaded from global memory in MFMA layout: A = a
 // row of keys / slots per lane (16 bytes of consecutive columns, four products per load; both operands number the
 // contraction the same way, so its order is free), and the accumulator of a score product is the B operand of the next
-// product as it stands.  No LDS, no barriers (but for the exchange between four waves of a unit).  A unit whose output is not finite is formed a second time without the rows that
-// a query does not see (f32_out_rows); the look at the output costs nothing measurable (567 / 560 us without / with, at
-// B=2, T=4096, 32/8 heads of 128).
+// product as it stands.  LDS and barriers only where four waves of a unit exchange their parts.  A unit whose output is not
+// finite is formed a second time without the rows that a query does not see (f32_out_rows); the look at the output costs
+// nothing measurable (567 / 560 us without / with, at B=2, T=4096, 32/8 heads of 128).
 #include "common.h"
 
 namespace nha {

@@ -561,8 +561,8 @@ struct OutSmem {
 };
 
 
-// SIGN: a scale that is not above zero (in the ordinary kernel the few instructions for it took 2 to 4 % of short windows: 60 ragged documents of 300
-// tokens, 4 heads of 128, W = 64, 50.2 -> 52.5 us).
+// SIGN: a scale that is not above zero (in the ordinary kernel the few instructions for it took 2 to 4 % of short windows: 60
+// ragged documents of 300 tokens, 4 heads of 128, W = 64, 50.2 -> 52.5 us).
 template <int D, int G, int NW, int TK, bool OWN, bool SIGN>
 __global__ __launch_bounds__(64 * NW, OWN ? NW / 2 : 1) void mfma_out_kernel(const MP p) {
   constexpr int NTHR = 64 * NW;      // threads per workgroup

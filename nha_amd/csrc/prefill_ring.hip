@@ -759,8 +759,9 @@ template <int D, bool SINK>
 int launch_ring(const MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  // the window-only launch has no slot operands: the ring is all the LDS it uses
-  const size_t lds = SINK ? (size_t)(RingCfg<D>::QT + 8 * RingCfg<D>::UB) : (size_t)RingCfg<D>::BYTES;   // the window queries end where the tiles do
+  // the window-only launch has no slot operands: the ring and the eight waves' window queries behind it (128 KB at D = 128, 96 at
+  // 64; its registers leave room for one workgroup per CU as well)
+  const size_t lds = SINK ? (size_t)(RingCfg<D>::QT + 8 * RingCfg<D>::UB) : (size_t)RingCfg<D>::BYTES;
   std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring_out_kernel<D, SINK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));

@@ -205,7 +205,8 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) out[e] = (__bf16)((float)sv[e] * fexp(fminf(gr[e >> 2][e & 3] - gv[e >> 2][e & 3], DECAY_CLAMP)));
       }
-      *reinterpret_cast<NHA_LDS bf16x8*>(lds + (U < 4 ? to03 : to45 - 4 * 4096) + U * 4096 + (r32 >> 4) * 2048 + (m >> 5) * 1024 + ((m >> 4) & 1) * 512 + (r32 & 15) * 32 + (m & 15) * 2) = out;
+      const uint32_t unit = (U < 4 ? to03 : to45 - 4 * 4096) + U * 4096, block = (r32 >> 4) * 2048 + (m >> 5) * 1024;
+      *reinterpret_cast<NHA_LDS bf16x8*>(lds + unit + block + ((m >> 4) & 1) * 512 + (r32 & 15) * 32 + (m & 15) * 2) = out;
     }
   };
   // ---- requests: the gate blocks and the window queries, these through the rings in whole lines (a fragment loaded from global
