@@ -166,10 +166,18 @@ def _cu_to_host(cu: torch.Tensor) -> np.ndarray:
     return host
 
 
+def _token_major(q, k):
+    """The packed entries number tokens by the first of three sizes; with another number of them the results would be
+    allocated for other tokens than the kernels write."""
+    if q.dim() != 3 or k.dim() != 3:
+        raise ValueError(f"expected token-major tensors [T, heads, dim], got q_swa {tuple(q.shape)}, k_swa {tuple(k.shape)}")
+
+
 def nha_prefill(q_swa, k_swa, q_gsa, k_gsa, v, s, g, cu_host: np.ndarray, *, wl: int, shift: int, scale: float,
                 h0=None, want_state: bool = False, want_lse: bool = True, impl=None):
     """Packed prefill on token-major tensors ``[T_tot, heads, dim]`` (one nha_prefill_fwd call).
     Returns (o, lse_swa, lse_gsa, hkt, hvt)."""
+    _token_major(q_swa, k_swa)
     return _prefill((q_swa, k_swa, q_gsa, k_gsa, v, s, g), q_swa.shape[:1], cu_host, wl, shift, scale, h0, want_state, want_lse, impl)
 
 
@@ -219,6 +227,7 @@ def nha_prefill_bwd(q_swa, k_swa, q_gsa, k_gsa, v, s, g, o, lse_swa, lse_gsa, do
                     want_dh0: bool = False):
     """Packed prefill backward on token-major tensors (one nha_prefill_bwd call).  Returns
     (dq_swa, dk_swa, dq_gsa, dk_gsa, dv, ds, dg, dh0k, dh0v) -- the last two None unless wanted."""
+    _token_major(q_swa, k_swa)
     return _prefill_bwd((q_swa, k_swa, q_gsa, k_gsa, v, s, g), o, lse_swa, lse_gsa, dout, cu_host, wl, shift, scale, h0, dlse_swa,
                         dlse_gsa, dht, want_dh0)
 

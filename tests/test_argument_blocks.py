@@ -1,9 +1,11 @@
 """Argument blocks packed as bytes hold what the ctypes structures of the C interface hold, field by field (CPU)."""
 import ctypes as C
 
+import numpy as np
 import pytest
+import torch
 
-from nha_amd import _lib
+from nha_amd import _lib, ops
 
 BLOCKS = [(_lib.pack_prefill, _lib.NhaPrefillArgs), (_lib.pack_prefill_bwd, _lib.NhaPrefillBwdArgs),
           (_lib.pack_hybrid_prologue, _lib.NhaHybridPrologueArgs), (_lib.pack_ring_fill, _lib.NhaRingFillArgs),
@@ -34,3 +36,15 @@ def test_floats_out_of_range_are_infinite_as_in_a_ctypes_field(x):
     a = _lib.NhaPrefillArgs()
     a.scale = x
     assert _lib.f32(x) == a.scale
+
+
+@pytest.mark.parametrize("q,k", [((2, 64, 4, 64), (2, 64, 4, 64)), ((128, 4, 64), (2, 64, 4, 64)), ((4, 64), (4, 64))])
+@pytest.mark.parametrize("bwd", [False, True])
+def test_packed_entries_refuse_tensors_that_are_not_token_major(q, k, bwd):
+    """A batch dimension more, and o would have B rows where the kernels write B T (refused before anything is allocated)."""
+    q, k, cu = torch.zeros(q), torch.zeros(k), np.array([0, 64, 128], dtype=np.int32)
+    with pytest.raises(ValueError, match="token-major"):
+        if bwd:
+            ops.nha_prefill_bwd(q, k, q, k, k, k, k, q, None, None, q, cu, wl=63, shift=0, scale=0.125)
+        else:
+            ops.nha_prefill(q, k, q, k, k, k, k, cu, wl=63, shift=0, scale=0.125)
