@@ -45,9 +45,19 @@ def test_window_gradients_of_many_key_groups(wl, H, NG, D, cu):
     compare(cu, wl, H, NG, D, ("q_swa", "k_swa", "v"))
 
 
+@pytest.mark.parametrize("wl", [40, 400])
+def test_more_sequences_than_lanes(wl):
+    """150 ragged sequences of up to 130 tokens, empty ones among them: the forward's workgroups of two chunks search among them, the
+    window gradients fall to kernels of 64 rows."""
+    lens = [(37 * i) % 131 for i in range(150)]
+    cu = torch.tensor([0, *lens]).cumsum(0).tolist()
+    print("case", wl, flush=True)
+    compare(cu, wl, 4, 1, 256, KEYS)
+
+
 @pytest.mark.parametrize("N,H", [(64, 4), (68, 4), (152, 4), (4100, 1)])
 @pytest.mark.parametrize("wl", [40, 400])
-def test_more_sequences_than_lanes(wl, N, H):
+def test_pairs_of_many_sequences(wl, N, H):
     """The workgroups of two chunks count the pairs of up to 64 sequences and search among more, in steps of 64 and of 4096: one to three chunks
     each, two on average (taken as filled; the 256-wide window gradients of others fall to kernels of 64 rows), empty ones among them."""
     lens = [(65, 1, 130, 66)[i % 4] for i in range(N)]
