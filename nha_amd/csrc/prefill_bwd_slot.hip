@@ -15,16 +15,19 @@
 // every 64 x 64 table.  u and dp trade sides through LDS once per head; every table lies transposed ([column][row]), so
 // that an accumulator's four rows are one 8-byte write and both operand forms are reads of it (plain or transposing).
 //
-// Bound: latency between short products -- one workgroup of eight waves fits a CU (LDS), a head is eight barriers with 4 to
-// 100 MFMAs per wave between them, about 24k cycles of which the MFMAs are 4k.  As five launches with the tables handed on
-// through HBM (A, B, du, p, ck, cv: 112 KB per head and chunk) plus one that exported the states as bf16 pairs, the same
-// work took 914 us at B=2, T=8192, 32/8 heads of 128 (now 429, and 7 for the launch that looks for strongly decaying
-// chunks), 366 at B=8, T=2048, 4/4 heads of 256 (now 230 + 7) and 191 at 5003 packed tokens, 16/16 heads of 64 (now 96 + 5).
+// Bound, several query heads per kv-head: latency between short products -- one workgroup of eight waves fits a CU (LDS), a head
+// is eight barriers with 4 to 100 MFMAs per wave between them, about 21k cycles of which vector instructions are 11k and MFMAs 6k
+// per SIMD; a workgroup's first loads (20k cycles, all CUs at once and so at the rate of the memory) and its results come on top.
+// One query head per kv-head (ONE): bytes (B=8, T=2048, 4/4 heads of 256: 580 MB in 159 us, half of them the fp32 results).
+// Times: 415 us at B=2, T=8192, 32/8 heads of 128 (and 7 for the launch that looks for strongly decaying chunks), 159 + 7 at B=8,
+// T=2048, 4/4 heads of 256, 88 + 5 at 5003 packed tokens, 16/16 heads of 64.
 //
 // Registers are the scarce thing: sums over the heads (64 at DW = 128) and the operands (48) stay, so whatever spills waits,
 // with every load before it, for memory.  Hence: nothing derived from the lane's number lives across the loop over heads;
-// wave-uniform bases with 32-bit offsets; Y read from LDS in both forms; stores only after the last load.  (709 us with the
-// spills of the first version.)  Operands staged through LDS in whole lines, which other kernels gain from, change nothing here.
+// wave-uniform bases with 32-bit offsets; Y read from LDS in both forms; stores only after the last load; the rows of o in whole
+// lines, 8 of them to each wave, instead of in the layout of the products by half of the waves (456 -> 415 us at the first shape:
+// 16 registers and the spills with them, and the half that had no rows waited), and N with its slots along the registers, so that a
+// lane's four sums are one store.  Operands staged through LDS in whole lines, which other kernels gain from, change nothing here.
 //
 // Precision: dg is a difference of nearly equal sums, so every table made from fp32 values (X, Xp, Y, ck, cv, the chunk-start
 // states) is a bf16 pair hi + lo and its products are hi hi + hi lo + lo hi (single bf16 tables put 1-5 % on dg).
@@ -76,6 +79,12 @@ __device__ __forceinline__ void put4_pair(lbf16* hi, lbf16* lo, int idx, const f
   *reinterpret_cast<NHA_LDS bf16x4*>(lo + idx) = l;
 }
 
+// x of another lane of the row of 16
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+
 // element at a 32-bit byte offset of a base that is the same for the whole wave (one scalar and one vector register)
 template <class T, class B>
 __device__ __forceinline__ T ld_at(const B* base, unsigned bytes) {
@@ -102,15 +111,16 @@ struct SlotP {
   float scale;
 };
 
-template <int DW> struct SlotLds {
+template <int DW, bool ONE> struct SlotLds {
   static constexpr int LDT = DW + 16, TILE = BT * LDT, TAB = BT * TLD, HTAB = BT * HLD;
   static constexpr int Q = 0, O = Q + TILE;     // bf16 offsets
   static constexpr int X0 = O + TILE;           // X0 hi, lo, Xp0 hi, lo   [64 m][TLD]; u / dp in transit
   static constexpr int A = X0 + 4 * TAB;        // A, B [64 j][TLD], then X1 hi, lo, Xp1 hi, lo [64 m][HLD]
   static constexpr int X1 = A + 2 * TAB;
   static constexpr int C = A;                   // ck hi, lo, cv hi, lo [64 r][TLD], once A, B, X1, Xp1 are done with
-  static constexpr int S = X1 + 4 * HTAB;        // k-state [64 m][LDT], k' [64 j][LDT]; first the other columns of q and do
-  static constexpr int ROW = S + 2 * TILE;                      // floats: delta, lse, lse_gsa, dlse_gsa of the 64 rows
+  // k-state [64 m][LDT], k' [64 j][LDT]; first the other columns of q and do (ONE: where q and do were, once N and out are formed)
+  static constexpr int S = ONE ? Q : X1 + 4 * HTAB;
+  static constexpr int ROW = X1 + 4 * HTAB + (ONE ? 0 : 2 * TILE);   // floats: delta, lse, lse_gsa, dlse_gsa of the 64 rows
   static constexpr int Y = ROW + 2 * 4 * BT;                    // Y hi, lo [64 j][TLD]
   static constexpr size_t BYTES = (size_t)(Y + 2 * TAB) * 2;
   static_assert(2 * TAB <= 4 * HTAB, "ck and cv fit where A, B, X1 and Xp1 were");
@@ -147,14 +157,20 @@ struct Operands {
 // pairs within a block have their decay formed one by one in fp32.  With all pairs of the chunk one by one this launch was slower
 // than the VALU kernels that it replaced: backward of 4000 tokens, every chunk strongly decaying, 32/8 heads of 128 1985 us with
 // those, 2702 with all pairs, 1142 like this; 3000 tokens, 4 heads of 256 525 / 802 / 413; 5000, 16 of 64 1040 / 1735 / 720.
-// DW: the output columns x of a workgroup.  Half of the 256 of the largest head: a workgroup of all would hold 128 sums per
-// lane next to its operands and tiles of 66 KB; the products over all columns (A, B, U, P0, delta) are formed twice instead,
-// from the other columns of q and do in the room of the state tiles and operands streamed two steps at a time.
-template <int D, int DW, bool EXACT>
+// ONE: one query head per kv-head.  Nothing is summed over heads, so N and out leave the products as they are formed (no sums in
+// registers), and the tiles of dq take the place of q and do once those are done with: a workgroup has all columns, also the 256
+// of the largest head, and requests all of its operands at once (240 -> 159 us at B=8, T=2048, 4/4 heads of 256, where two
+// workgroups of 128 columns each had formed the tables; 96 -> 88 at 5003 packed tokens, 16/16 heads of 64).
+// DW: the output columns x of a workgroup.  With several heads half of the 256 of the largest head: a workgroup of all would hold
+// 128 sums per lane next to its operands and tiles of 66 KB; the products over all columns (A, B, U, P0, delta) are formed twice
+// instead, from the other columns of q and do in the room of the state tiles and operands streamed two steps at a time.
+template <int D, int DW, bool EXACT, bool ONE>
 __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
-  typedef SlotLds<DW> L;
+  static_assert(!ONE || (D == DW && !EXACT), "ONE: all columns, split decays");
+  typedef SlotLds<DW, ONE> L;
   constexpr int KS = D / 32, KW = DW / 32, DB = DW / 16, LDT = L::LDT;
   constexpr int NPC = BT * DW / 8 / 256;   // 16-byte pieces of a tile per thread of the side
+  constexpr int LO = D / 8, NO = D / 64;   // lanes to a row of o, pieces of a lane of the wave's 8 rows
   constexpr bool KEEP = D == DW;   // the operands, the same for every head, stay in registers
   extern __shared__ __align__(16) unsigned char smem[];
   lbf16* const sm = (lbf16*)smem;
@@ -197,7 +213,7 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
     float ls, lg, dl;
   };
   struct Rows {
-    uint4 o[KS];
+    uint4 o[NO];
   };
   auto load_head = [&](Head& t, int hq, int lane) {
     const int stid = 64 * w + lane;
@@ -218,28 +234,31 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
     }
   };
   auto load_o = [&](Rows& t, int hq, int lane) {
-    if (!vs) return;
-    const int row = 16 * w + (lane & 15);
     const bf16_t* const src = p.o + ((int64_t)c0 * HQ + hq) * D;
-    const unsigned at = ((row < R ? row : R - 1) * HQ * D + 8 * (lane >> 4)) * 2;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) t.o[ks] = ld_at<uint4>(src + step_col(ks), at);
+    for (int u = 0; u < NO; ++u) {
+      const int row = 8 * wave + 8 / NO * u + lane / LO;
+      t.o[u] = ld_at<uint4>(src, ((row < R ? row : R - 1) * HQ * D + 8 * (lane % LO)) * 2);
+    }
   };
-  auto row_delta = [&](const Rows& t, int hq, int lane) {   // the four lanes of a row split its columns
-    if (!vs) return;
-    const int kb = lane >> 4, col = 16 * w + (lane & 15);
-    float acc = 0.f;
+  auto row_delta = [&](const Rows& t, int hq, int lane) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const bf16x8 o8 = as_bf16x8(t.o[ks]), d8 = lds_frag(step_tile(ks), LDT, col, 8 * kb);
+    for (int u = 0; u < NO; ++u) {
+      const int row = 8 * wave + 8 / NO * u + lane / LO, c = 8 * (lane % LO);
+      const lbf16* const dp = KEEP || (c & DW) == (x0 & DW) ? sm + L::O + row * LDT + c % DW : sm + L::S + L::TILE + row * LDT + c % DW;
+      const bf16x8 o8 = as_bf16x8(t.o[u]), d8 = *reinterpret_cast<const NHA_LDS bf16x8*>(dp);
+      float acc = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc += (float)o8[e] * (float)d8[e];
-    }
-    acc += __shfl_xor(acc, 16, 64);
-    acc += __shfl_xor(acc, 32, 64);
-    if (kb == 0) {
-      rdelta[col] = acc;
-      if (col < R && x0 == 0) p.delta[(int64_t)(c0 + col) * HQ + hq] = acc;
+      acc += dpp_f<0xB1>(acc);    // lanes 1 and 2 apart, the other four of 8, of 16, of 32
+      acc += dpp_f<0x4E>(acc);
+      acc += dpp_f<0x141>(acc);
+      if (LO >= 16) acc += dpp_f<0x140>(acc);
+      if (LO >= 32) acc += __shfl_xor(acc, 16, 64);
+      if (lane % LO == 0) {
+        rdelta[row] = acc;
+        if (row < R && x0 == 0) p.delta[(int64_t)(c0 + row) * HQ + hq] = acc;
+      }
     }
   };
   auto store_head = [&](const Head& t, int lane) {
@@ -257,6 +276,16 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
       rdlg[lane] = t.dl;
     }
   };
+  Rows orow;
+  float gi[4][4], g31;   // gate cumsums of a lane's rows 16 blk + 4 kb + e (slot col)
+  auto load_gates = [&](int kb, int col) {
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) gi[blk][e] = ld_at<float>(gc + (16 * blk + e) * MS, (4 * kb * MS + col) * 4);
+    g31 = ld_at<float>(gc + 31 * MS, col * 4);
+  };
+  float e0[4][4], e1[2][4];   // their exponentials, of the rows 32.. also against the cumsum at row 31
   Operands opd[KEEP ? KS : 2];
   auto load_operands = [&](int x, int ks, int lane) {
     const int l16 = lane & 15, kb = lane >> 4, col = 16 * w + l16;
@@ -288,6 +317,7 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
     Elem<float>::ld8(gc + 31 * MS + m8, ref);
     Head head;
     load_head(head, h * NG, lane0);
+    if constexpr (ONE) load_o(orow, h, lane0);
     const float dc = p.dcum[cg * MS + col];
 #pragma unroll
     for (int ks = 0; ks < (KEEP ? KS : 2); ++ks) load_operands(ks, ks, lane0);
@@ -307,28 +337,72 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         opd[ks].form(col < R && tl >= 0, dc, y[ks], hh[ks], hl[ks]);
-        if (!vs) store_states(32 * ks, hh[ks], y[ks], lane0);
+        if (!ONE && !vs) store_states(32 * ks, hh[ks], y[ks], lane0);
       }
+    }
+    if constexpr (ONE) {
+      load_gates(kb, col);
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          e0[blk][e] = __expf(gi[blk][e]);
+          if (blk >= 2) e1[blk - 2][e] = __expf(gi[blk][e] - g31);
+        }
     }
     lds_barrier();
   }
-  f32x4 accN[DB], accO[DB], accS[4], xg[2];   // xg: of the rows 32.. on the v side, of the others on the k side
+  f32x4 accN[ONE ? 1 : DB], accO[ONE ? 1 : DB], accS[4], xg[2];   // xg: of the rows 32.. on the v side, of the others on the k side
 #pragma unroll
-  for (int d = 0; d < DB; ++d) accN[d] = accO[d] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int d = 0; d < (ONE ? 1 : DB); ++d) accN[d] = accO[d] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int rb = 0; rb < 4; ++rb) accS[rb] = (f32x4){0.f, 0.f, 0.f, 0.f};
   xg[0] = xg[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
   float* const ep = (vs ? p.ev : p.ek) + (cg * D + x0) * MS;            // N [x][m]
+  float* const op = (vs ? p.dvs : p.dks) + ((int64_t)(bos + tl0) * H + h) * D + x0;   // out, at the rows' source tokens
 
-  for (int a = 0; a < NG; ++a) {
+  // xg and ds_intra (the sum of both sides): rows 32.. from the v side, the others from the k side
+  lfloat* const sums = ONE ? (lfloat*)(NHA_LDS void*)(sm + L::Y) : transit;
+  auto swap_sums = [&](int lane) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      if (vs) {   // (swapped in place: a choice between two elements by reference would put the array in memory)
+        const f32x4 z = accS[b];
+        accS[b] = accS[2 + b];
+        accS[2 + b] = z;
+      }
+      *reinterpret_cast<NHA_LDS f32x4*>(sums + ((wave * 2 + b) * 64 + lane) * 4) = accS[2 + b];
+    }
+  };
+  auto store_sums = [&](int kb, int col, int lane) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const f32x4 z = accS[b] + *reinterpret_cast<const NHA_LDS f32x4*>(sums + (((wave ^ 4) * 2 + b) * 64 + lane) * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 16 * b + 4 * kb + e + (vs ? 32 : 0);
+        const unsigned at = (r * H * MS + col) * 4;
+        const float d = vs ? g31 - gi[2 + b][e] : -gi[b][e];
+        if (r < R) {
+          st_at(p.xg + ((int64_t)c0 * H + h) * MS, at, xg[b][e]);
+          st_at(p.dsi + ((int64_t)c0 * H + h) * MS, at, EXACT ? z[e] : z[e] * __expf(d));
+        }
+      }
+    }
+  };
+  auto store_sides = [&](int d, const f32x4& n, const f32x4& o, int lane) {
+    const int l16 = lane & 15, kb = lane >> 4, col = 16 * w + l16, tl = it * BT + col - p.shift;
+    st_at(ep + 16 * d * MS + 16 * w, (l16 * MS + 4 * kb) * 4, n);
+    if (col < R && tl >= 0) st_at(op + 16 * d, ((tl - tl0) * H * D + 4 * kb) * 4, o);
+  };
+  for (int a = 0; a < (ONE ? 1 : NG); ++a) {
     const int hq = h * NG + a;
     // what depends on the lane's number is derived anew for every head: hoisted out of the loop, the addresses and decay
     // factors of a whole head are kept across it -- in memory, there are no registers for them
     int lane = lane0;
     asm volatile("" : "+v"(lane));
     const int l16 = lane & 15, kb = lane >> 4, col = 16 * w + l16;
-    Rows orow;
-    load_o(orow, hq, lane);
+    if constexpr (!ONE) load_o(orow, hq, lane);
     if constexpr (!KEEP) row_delta(orow, hq, lane);
     FENCE;
     // ---- A or B (rows 16 blk + 4 kb + e, column j = col), U or P0 (slot m = col) --------------------------------------
@@ -339,7 +413,23 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
         if (16 * blk + 4 * kb + e < col) c[e] = 0.f;   // j <= i
       put4(AT + col * TLD + 16 * blk + 4 * kb, c);
     };
-    if constexpr (KEEP) {
+    if constexpr (ONE) {
+      f32x4 cA[4];
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk) cA[blk] = cU[blk] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int blk = 0; blk < 4; ++blk) {
+          const bf16x8 x = lds_frag(X, LDT, 16 * blk + l16, 32 * ks + 8 * kb);
+          cA[blk] = mfma16(x, y[ks], cA[blk]);
+          cU[blk] = mfma16(x, hh[ks], mfma16(x, hl[ks], cU[blk]));
+        }
+        if (ks % 2 == 1) FENCE;
+      }
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk) put_scores(blk, cA[blk]);
+    } else if constexpr (KEEP) {
 #pragma unroll
       for (int blk = 0; blk < 4; ++blk) {
         f32x4 cA = {0.f, 0.f, 0.f, 0.f};
@@ -389,13 +479,7 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
 #pragma unroll
       for (int blk = 0; blk < 4; ++blk) put_scores(blk, cA[blk]);
     }
-    // gate cumsums of this lane's rows 16 blk + 4 kb + e (slot col)
-    float gi[4][4];
-#pragma unroll
-    for (int blk = 0; blk < 4; ++blk)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) gi[blk][e] = ld_at<float>(gc + (16 * blk + e) * MS, (4 * kb * MS + col) * 4);
-    const float g31 = ld_at<float>(gc + 31 * MS, col * 4);
+    if constexpr (!ONE) load_gates(kb, col);
     lds_barrier();
     // ---- u (k side) or dp (v side) of rows 16 blk + 4 kb + e, slot col, to the other side ------------------------------
     if constexpr (!EXACT) {
@@ -417,8 +501,11 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float e0 = __expf(gi[blk][e]), e1 = blk >= 2 ? __expf(gi[blk][e] - g31) : 0.f;
-          cU[blk][e] = e0 * (cU[blk][e] + c[0][e]) + e1 * c[1][e];
+          if constexpr (!ONE) {
+            e0[blk][e] = __expf(gi[blk][e]);
+            if (blk >= 2) e1[blk - 2][e] = __expf(gi[blk][e] - g31);
+          }
+          cU[blk][e] = e0[blk][e] * (cU[blk][e] + c[0][e]) + (blk >= 2 ? e1[blk - 2][e] * c[1][e] : 0.f);
         }
         FENCE;
       }
@@ -504,9 +591,9 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float x = i0 + e < R ? (vs ? pm[e] : p.scale * du[e]) : 0.f;
-        t0[e] = x * (EXACT ? expf(gi[blk][e]) : __expf(gi[blk][e]));
+        t0[e] = x * (EXACT ? expf(gi[blk][e]) : e0[blk][e]);
         if constexpr (EXACT) t1[e] = x * expf(own[e]);
-        else if (blk >= 2) t1[e] = x * __expf(gi[blk][e] - g31);
+        else if (blk >= 2) t1[e] = x * e1[blk - 2][e];
         if constexpr (EXACT) ep[(i0 + e) * MS + col] = x;   // undecayed, for the pairwise sums (N takes the place afterwards)
       }
       put4_pair(T0h, T0l, col * TLD + i0, t0);
@@ -653,23 +740,51 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
         if (16 * blk + 4 * kb + e < col) c[blk][e] = 0.f;
       put4_pair(Ch, Cl, col * TLD + 16 * blk + 4 * kb, c[blk]);
     }
+    if constexpr (ONE) swap_sums(lane);
     lds_barrier();
-    // ---- N^T and out^T: X^T times the tables --------------------------------------------------------------------------
+    if constexpr (ONE) store_sums(kb, col, lane);
+    Head next = {};   // (a value on every path: left open, the registers count as live around the whole loop)
+    if (!ONE && KEEP && a + 1 < NG) load_head(next, hq + 1, lane);
+    FENCE;
+    // ---- N (rows m = 16 w + 4 kb + e, columns x = 16 d + l16) and out^T: the tables times X ------------------------------
+    if constexpr (ONE) {
+      bf16x8 bw[2], bwl[2], bc[2], bcl[2];
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      const bf16x8 bw = col_frag(T0h, TLD, col, 32 * hf, kb), bwl = col_frag(T0l, TLD, col, 32 * hf, kb);
-      const bf16x8 bc = col_frag(Ch, TLD, col, 32 * hf, kb), bcl = col_frag(Cl, TLD, col, 32 * hf, kb);
+      for (int hf = 0; hf < 2; ++hf) {
+        bw[hf] = col_frag(T0h, TLD, col, 32 * hf, kb), bwl[hf] = col_frag(T0l, TLD, col, 32 * hf, kb);
+        bc[hf] = col_frag(Ch, TLD, col, 32 * hf, kb), bcl[hf] = col_frag(Cl, TLD, col, 32 * hf, kb);
+      }
 #pragma unroll
       for (int d = 0; d < DB; ++d) {
-        const bf16x8 x = lds_frag_tr(X, LDT, 32 * hf, 32 * hf + 16, 16 * d, lane);
-        accN[d] = mfma16(x, bw, mfma16(x, bwl, accN[d]));
-        accO[d] = mfma16(x, bc, mfma16(x, bcl, accO[d]));
+        f32x4 n = {0.f, 0.f, 0.f, 0.f}, o = n;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+          const bf16x8 x = lds_frag_tr(X, LDT, 32 * hf, 32 * hf + 16, 16 * d, lane);
+          n = mfma16(bw[hf], x, mfma16(bwl[hf], x, n));
+          o = mfma16(x, bc[hf], mfma16(x, bcl[hf], o));
+        }
+        store_sides(d, n, o, lane);
         if (d % 2 == 1) FENCE;
       }
+      lds_barrier();   // q and do are done with
+      if (!vs)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) store_states(32 * ks, hh[ks], y[ks], lane);
+      lds_barrier();
+    } else {
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        const bf16x8 bw = col_frag(T0h, TLD, col, 32 * hf, kb), bwl = col_frag(T0l, TLD, col, 32 * hf, kb);
+        const bf16x8 bc = col_frag(Ch, TLD, col, 32 * hf, kb), bcl = col_frag(Cl, TLD, col, 32 * hf, kb);
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+          const bf16x8 x = lds_frag_tr(X, LDT, 32 * hf, 32 * hf + 16, 16 * d, lane);
+          accN[d] = mfma16(bw, x, mfma16(bwl, x, accN[d]));
+          accO[d] = mfma16(x, bc, mfma16(x, bcl, accO[d]));
+          if (d % 2 == 1) FENCE;
+        }
+      }
     }
-    FENCE;
-    Head next = {};   // (a value on every path: left open, the registers count as live around the whole loop)
-    if (KEEP && a + 1 < NG) load_head(next, hq + 1, lane);
     FENCE;
     // ---- dq^T: rows i = 16 w + l16, this side's half of the columns -----------------------------------------------------
     {
@@ -702,7 +817,7 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
         }
       }
     }
-    if (a + 1 < NG) {
+    if (!ONE && a + 1 < NG) {
       if constexpr (!KEEP) load_head(next, hq + 1, lane);
       lds_barrier();   // the tiles and tables are done with
       store_head(next, lane);
@@ -714,70 +829,41 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
     }
   }
   // ---- results (loads first: a load waits for the stores issued before it) ---------------------------------------------
-  const int l16 = lane0 & 15, kb = lane0 >> 4, col = 16 * w + l16;
-  if (x0 == 0) {   // xg and ds_intra (the sum of both sides): rows 32.. from the v side, the others from the k side
-    const int rb0 = vs ? 2 : 0;
-    float gi[2][4];
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) gi[b][e] = ld_at<float>(gc + (16 * (rb0 + b) + e) * MS, (4 * kb * MS + col) * 4);
-    const float g31 = vs ? ld_at<float>(gc + 31 * MS, col * 4) : 0.f;
-    lds_barrier();
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      if (vs) {   // (swapped in place: a choice between two elements by reference would put the array in memory)
-        const f32x4 z = accS[b];
-        accS[b] = accS[2 + b];
-        accS[2 + b] = z;
-      }
-      *reinterpret_cast<NHA_LDS f32x4*>(transit + ((wave * 2 + b) * 64 + lane0) * 4) = accS[2 + b];
+  if constexpr (!ONE) {
+    const int l16 = lane0 & 15, kb = lane0 >> 4, col = 16 * w + l16;
+    if (x0 == 0) {
+      load_gates(kb, col);
+      lds_barrier();
+      swap_sums(lane0);
+      lds_barrier();
+      store_sums(kb, col, lane0);
     }
-    lds_barrier();
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const f32x4 z = accS[b] + *reinterpret_cast<const NHA_LDS f32x4*>(transit + (((wave ^ 4) * 2 + b) * 64 + lane0) * 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int r = 16 * (rb0 + b) + 4 * kb + e;
-        const unsigned at = (r * H * MS + col) * 4;
-        if (r < R) {
-          st_at(p.xg + ((int64_t)c0 * H + h) * MS, at, xg[b][e]);
-          st_at(p.dsi + ((int64_t)c0 * H + h) * MS, at, EXACT ? z[e] : z[e] * __expf(g31 - gi[b][e]));
-        }
-      }
-    }
-  }
-  {   // N[x = 16 d + 4 kb + e][m = col]; out[row = col][x] at its source token
-    const int tl = it * BT + col - p.shift;
-    float* const op = (vs ? p.dvs : p.dks) + ((int64_t)(bos + tl0) * H + h) * D + x0;
-#pragma unroll
-    for (int d = 0; d < DB; ++d) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) st_at(ep + (16 * d + e) * MS, (4 * kb * MS + col) * 4, accN[d][e]);
-      if (col < R && tl >= 0) st_at(op + 16 * d, ((tl - tl0) * H * D + 4 * kb) * 4, accO[d]);
-    }
+    for (int d = 0; d < DB; ++d) store_sides(d, accN[d], accO[d], lane0);
   }
 }
 
-template <int D>
-int launch(const SlotP& p, hipStream_t st) {
-  constexpr int DW = D < 128 ? D : 128;
-  constexpr size_t lds = SlotLds<DW>::BYTES;
+template <int D, int DW, bool EXACT, bool ONE>
+int launch_one(const SlotP& p, hipStream_t st) {
+  constexpr size_t lds = SlotLds<DW, ONE>::BYTES;
   static std::atomic<bool> configured{false};   // the attribute call is idempotent: a second thread may repeat it
   if (!configured) {
-    hipError_t e1 = hipFuncSetAttribute((const void*)bwd_slot_kernel<D, DW, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipError_t e2 = hipFuncSetAttribute((const void*)bwd_slot_kernel<D, DW, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e1 != hipSuccess || e2 != hipSuccess) {
-      set_error("nha_prefill_bwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e1 != hipSuccess ? e1 : e2));
+    const hipError_t e = hipFuncSetAttribute((const void*)bwd_slot_kernel<D, DW, EXACT, ONE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) {
+      set_error("nha_prefill_bwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
       return NHA_ERR_LAUNCH;
     }
     configured = true;
   }
-  hipLaunchKernelGGL((bwd_slot_kernel<D, DW, false>), dim3(p.H * (D / DW), p.NT), dim3(512), lds, st, p);
-  hipLaunchKernelGGL((bwd_slot_kernel<D, DW, true>), dim3(p.H * (D / DW), p.NT), dim3(512), lds, st, p);
+  hipLaunchKernelGGL((bwd_slot_kernel<D, DW, EXACT, ONE>), dim3(p.H * (D / DW), p.NT), dim3(512), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(slot branch)");
   return NHA_OK;
+}
+template <int D>
+int launch(const SlotP& p, hipStream_t st) {
+  constexpr int DW = D < 128 ? D : 128;
+  const int rc = p.NG == 1 ? launch_one<D, D, false, true>(p, st) : launch_one<D, DW, false, false>(p, st);
+  return rc != NHA_OK ? rc : launch_one<D, DW, true, false>(p, st);
 }
 
 }  // namespace

@@ -45,3 +45,13 @@ def test_slot_branch_growing_gates_beside_strong_ones(D):
     d["g"][..., 8:] = (d["g"][..., 8:] / -400).clamp(0, 0.01)
     d["s"][..., 8:] = (d["s"][..., 8:] / 20)
     run_bwd_case(f"slot growing D{D}", d, wl=40, shift=0, dtype=BF, cu=CU, with_lse=True)
+
+
+@pytest.mark.parametrize("gate_mean", [0.0, -2.0])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_slot_branch_one_head_per_kv_head(D, gate_mean):
+    """One query head per kv-head has an instance of its own (all columns in one workgroup, nothing summed over heads): an odd
+    number of heads, the LSE's own cotangent, and at -2 chunks that are left to the launch for strongly decaying ones."""
+    d = prefill_inputs(8400 + D, 1, CU[-1], 3, 3, D, D, 64, dtype=BF, qk_scale=D ** -0.5, gate_div=1.0, gate_mean=gate_mean,
+                       with_state=True, N=len(CU) - 1)
+    run_bwd_case(f"slot one head {gate_mean} D{D}", d, wl=40, shift=33, dtype=BF, cu=CU, with_lse=True)
