@@ -295,26 +295,63 @@ __global__ __launch_bounds__(256) void mfma_state_local_kernel(const MP p) {
 // grid (N*H, 2*MS*D/1024): the first MS*D/4 groups are the k-state ([m][d]), the rest the v-state.
 constexpr int SCAN_AHEAD = 4;
 
+// What a workgroup of level 2 owns: 16 slots x 64 columns of one state, a slot and four consecutive columns per thread (256
+// consecutive bytes of a row of the scratch's [m][d] states per 16 threads).  The caller's k-states lie [d][m]: they pass through
+// LDS, 16 slots (64 bytes) of a row side by side.  With a thread's own four columns read and written there one by one, level 2 of a call
+// with initial and final states was bound by that (16 packed sequences, 4 heads of 256, 32768 tokens:
+// state_scan_kernel 31 -> 23 us, state_final_kernel 43 -> 38).
+template <int D>
+struct StatePart {
+  static constexpr int GROUPS = MS * D / 1024;   // workgroups per state
+  bool isv;
+  int m, d;
+  __device__ __forceinline__ StatePart(int group, int tid) {
+    isv = group >= GROUPS;
+    const int g = isv ? group - GROUPS : group;
+    m = 16 * (g / (D / 64)) + (tid >> 4);
+    d = 64 * (g % (D / 64)) + 4 * (tid & 15);
+  }
+  // tr: [64 d][17] floats of the workgroup; k: the sequence and head's [D][MS]
+  __device__ __forceinline__ float4 load_k(const float* k, lfloat* tr, int tid) const {
+    const int m0 = m & ~15, d0 = d & ~63;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int x = (tid >> 4) + 16 * i;
+      tr[x * 17 + (tid & 15)] = k[(d0 + x) * MS + m0 + (tid & 15)];
+    }
+    __syncthreads();
+    const lfloat* const t = tr + (d & 63) * 17 + (m & 15);
+    return make_float4(t[0], t[17], t[34], t[51]);
+  }
+  __device__ __forceinline__ void store_k(float* k, const float4& v, lfloat* tr, int tid) const {
+    const int m0 = m & ~15, d0 = d & ~63;
+    lfloat* const t = tr + (d & 63) * 17 + (m & 15);
+    __syncthreads();
+    t[0] = v.x; t[17] = v.y; t[34] = v.z; t[51] = v.w;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int x = (tid >> 4) + 16 * i;
+      k[(d0 + x) * MS + m0 + (tid & 15)] = tr[x * 17 + (tid & 15)];
+    }
+  }
+};
+
 template <int D>
 __global__ __launch_bounds__(256) void state_scan_kernel(const MP p) {
+  __shared__ float trs[64 * 17];
+  lfloat* const tr = (lfloat*)trs;
   const int H = p.H;
   const int n = blockIdx.x / H, h = blockIdx.x % H;
-  const int e4 = blockIdx.y * 256 + threadIdx.x;
-  const bool isv = e4 >= MS * D / 4;
-  const int em = (isv ? e4 - MS * D / 4 : e4) * 4;
-  const int m = em / D, d = em % D;
+  const StatePart<D> part(blockIdx.y, threadIdx.x);
+  const bool isv = part.isv;
+  const int m = part.m, d = part.d;
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int nchunks = (eos - bos + BT - 1) / BT;
   const int nseg = (nchunks + (1 << p.seg_sh) - 1) >> p.seg_sh;
+  const int64_t nh = (int64_t)n * H + h;
   float4 hcur = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (p.h0k) {
-    if (isv) {
-      hcur = *reinterpret_cast<const float4*>(p.h0v + (((int64_t)n * H + h) * MS + m) * D + d);
-    } else {
-      const float* src = p.h0k + (((int64_t)n * H + h) * D + d) * MS + m;
-      hcur = make_float4(src[0], src[MS], src[2 * MS], src[3 * MS]);
-    }
-  }
+  if (p.h0k) hcur = isv ? *reinterpret_cast<const float4*>(p.h0v + (nh * MS + m) * D + d) : part.load_k(p.h0k + nh * D * MS, tr, threadIdx.x);
   const float* __restrict__ hend = isv ? p.hend_v : p.hend_k;
   float* __restrict__ hseg = isv ? p.hseg_v : p.hseg_k;
   const float* __restrict__ dtot = p.dtot;
@@ -353,12 +390,8 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const MP p) {
     cur = nxt;
   }
   if (p.hkt) {
-    if (isv) {
-      *reinterpret_cast<float4*>(p.hvt + (((int64_t)n * H + h) * MS + m) * D + d) = hcur;
-    } else {
-      float* dst = p.hkt + (((int64_t)n * H + h) * D + d) * MS + m;
-      dst[0] = hcur.x; dst[MS] = hcur.y; dst[2 * MS] = hcur.z; dst[3 * MS] = hcur.w;
-    }
+    if (isv) *reinterpret_cast<float4*>(p.hvt + (nh * MS + m) * D + d) = hcur;
+    else part.store_k(p.hkt + nh * D * MS, hcur, tr, threadIdx.x);
   }
 }
 
@@ -382,24 +415,21 @@ constexpr float CARRY_FLOOR = 0x1p-100f;
 // grid (N*H, 2*MS*D/1024): the first MS*D/4 groups are the k-state ([m][d]), the rest the v-state.
 template <int D>
 __global__ __launch_bounds__(256) void state_final_kernel(const MP p) {
+  __shared__ float trs[64 * 17];
+  lfloat* const tr = (lfloat*)trs;
   const int H = p.H;
   const int n = blockIdx.x / H, h = blockIdx.x % H;
-  const int e4 = blockIdx.y * 256 + threadIdx.x;
-  const bool isv = e4 >= MS * D / 4;
-  const int em = (isv ? e4 - MS * D / 4 : e4) * 4;
-  const int m = em / D, d = em % D;
+  const StatePart<D> part(blockIdx.y, threadIdx.x);
+  const bool isv = part.isv;
+  const int m = part.m, d = part.d;
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int nchunks = (eos - bos + BT - 1) / BT;
   const int nseg = (nchunks + (1 << p.seg_sh) - 1) >> p.seg_sh;
+  const int64_t nh = (int64_t)n * H + h;
   float hcur[4] = {0.f, 0.f, 0.f, 0.f};
   if (p.h0k) {
-    if (isv) {
-      const float4 x = *reinterpret_cast<const float4*>(p.h0v + (((int64_t)n * H + h) * MS + m) * D + d);
-      hcur[0] = x.x; hcur[1] = x.y; hcur[2] = x.z; hcur[3] = x.w;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) hcur[i] = p.h0k[(((int64_t)n * H + h) * D + d + i) * MS + m];
-    }
+    const float4 x = isv ? *reinterpret_cast<const float4*>(p.h0v + (nh * MS + m) * D + d) : part.load_k(p.h0k + nh * D * MS, tr, threadIdx.x);
+    hcur[0] = x.x; hcur[1] = x.y; hcur[2] = x.z; hcur[3] = x.w;
   }
   const float* hend = isv ? p.hend_v : p.hend_k;
   bf16_t* hloc = isv ? p.hvc : p.hkT;
@@ -471,12 +501,9 @@ __global__ __launch_bounds__(256) void state_final_kernel(const MP p) {
     l_cur = l_nxt;
   }
   if (p.hkt) {
-    if (isv) {
-      *reinterpret_cast<float4*>(p.hvt + (((int64_t)n * H + h) * MS + m) * D + d) = make_float4(hcur[0], hcur[1], hcur[2], hcur[3]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) p.hkt[(((int64_t)n * H + h) * D + d + i) * MS + m] = hcur[i];
-    }
+    const float4 x = make_float4(hcur[0], hcur[1], hcur[2], hcur[3]);
+    if (isv) *reinterpret_cast<float4*>(p.hvt + (nh * MS + m) * D + d) = x;
+    else part.store_k(p.hkt + nh * D * MS, x, tr, threadIdx.x);
   }
 }
 
