@@ -15,7 +15,7 @@
 //   state pass  (mfma_state_kernel): per (sequence, kv-head, 16-slot block) sweep over 64-row chunks
 //               with the fp32 state held in MFMA accumulators (chunk_fused.py:30-113).
 //   output pass (mfma_out_kernel)  : per (chunk, kv-head, group of <=4 q-heads).
-#include "mfma_common.h"
+#include "prefill_exact.h"
 
 #include <mutex>
 #include <stdlib.h>
@@ -1143,151 +1143,24 @@ __global__ __launch_bounds__(64 * NW, OWN ? NW / 2 : 1) void mfma_out_kernel(con
 }
 
 // ==========================================================================================
-// exact recomputation of rows the output pass cannot factor
+// exact recomputation of the flagged rows (prefill_exact.h) after the output passes that do not do it themselves: grid (chunk, kv-head),
+// the q-heads of the group in turn; workgroups of unflagged chunks leave at once
 // ==========================================================================================
-// The output pass writes the intra-chunk decay exp(gc_i - gc_j) as exp(gc_i - gr) * exp(gr - gc_j)
-// with gr the gate cumsum at the start of j's 16-row sub-block, and caps the second exponent at
-// DECAY_CLAMP.  Where a slot forgets faster than that (flags from the state pass), the rows of
-// that sub-block are recomputed here token by token with the unfactored decay (<= 1), in fp32
-// VALU arithmetic, from the same chunk-start states and gate table: slot logits
-// (nha_fla/ops/nha/chunk_fused.py:186-222), window logits, one softmax (:233-240), both reads
-// (:242-283) and the branch LSEs (nha_fla/ops/nha/chunk.py:459-470).  grid (chunk, kv-head), the
-// q-heads of the group in turn; workgroups of unflagged chunks leave at once.
-template <int D>
-struct RepairSmem {
-  static constexpr int LDH = D + 1;
-  static constexpr size_t floats = (size_t)MS * LDH + (size_t)MS * D + (size_t)BT * MS + 2 * D + 2 * MS + 2 * BT + 256 + 4 + BT;
-};
-
 template <int D>
 __global__ __launch_bounds__(256) void mfma_repair_kernel(const MP p) {
-  constexpr int LDH = RepairSmem<D>::LDH;
   const int chunk = blockIdx.x, h = blockIdx.y;
-  const int H = p.H, HQ = p.HQ;
-  const int64_t cg = (int64_t)chunk * H + h;
-  const int* fl = p.flags + cg * 4;
+  const int* fl = p.flags + ((int64_t)chunk * p.H + h) * 4;
   const int bits = fl[0] | fl[1] | fl[2] | fl[3];
   if (bits == 0) return;
   extern __shared__ __align__(16) float rsm[];
-  float* hk = rsm;                // [MS][LDH] true chunk-start k-state, transposed
-  float* hv = hk + MS * LDH;      // [MS][D]   true chunk-start v-state
-  float* gcl = hv + MS * D;       // [BT][MS]  gate cumsum
-  float* qg = gcl + BT * MS;      // [D] scaled slot-branch query
-  float* qs = qg + D;             // [D] scaled window query
-  float* okl = qs + D;            // [MS] slot logits -> probabilities
-  float* gct = okl + MS;          // [MS] gate cumsum of the row
-  float* Aj = gct + MS;           // [BT]
-  float* Avj = Aj + BT;           // [BT]
-  float* pw = Avj + BT;           // [256]
-  float* red = pw + 256;          // [4]
-  int* src = (int*)(red + 4);     // [BT]
-  const int tid = threadIdx.x;
-  const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
-  const int bos = p.cu[n], eos = p.cu[n + 1];
-  const int c0 = bos + it * BT;
-  const int rows = (eos - c0) < BT ? (eos - c0) : BT;
-  for (int e = tid; e < MS * D; e += 256) {
-    const int m = e / D, d = e % D;
-    hk[m * LDH + d] = bf16_to_f32(p.hkT[(cg * MS + m) * D + d]);
-    hv[m * D + d] = bf16_to_f32(p.hvc[(cg * MS + m) * D + d]);
-  }
-  for (int e = tid; e < BT * MS; e += 256) gcl[e] = p.gc[cg * BT * MS + e];
-
-  for (int hq = h * p.NG; hq < (h + 1) * p.NG; ++hq)
-  for (int r = 0; r < rows; ++r) {
-    if (!((bits >> (r >> 4)) & 1)) continue;
-    const int t = c0 + r;
-    __syncthreads();   // state tables are in place; the previous row is finished
-    const bf16_t* qsw = p.q_swa + ((int64_t)t * HQ + hq) * D;
-    const bf16_t* qgs = p.q_gsa + ((int64_t)t * HQ + hq) * D;
-    for (int i = tid; i < D; i += 256) {
-      qg[i] = bf16_to_f32(qgs[i]) * p.scale;
-      qs[i] = bf16_to_f32(qsw[i]) * p.scale;
-    }
-    if (tid < MS) gct[tid] = gcl[r * MS + tid];
-    if (tid < BT) {
-      const int tl = it * BT + tid - p.shift;
-      src[tid] = (tid <= r && tl >= 0) ? bos + tl : -1;
-    }
-    __syncthreads();
-    if (tid < BT) {
-      const int sj = src[tid];
-      Aj[tid] = sj >= 0 ? dot_row<bf16_t>(qg, p.k_gsa + ((int64_t)sj * H + h) * D, D) : 0.f;
-    }
-    __syncthreads();
-    float lmax = -INFINITY;
-    if (tid < MS) {
-      const int m = tid;
-      float acc = 0.f;
-      for (int d = 0; d < D; ++d) acc += qg[d] * hk[m * LDH + d];
-      acc *= expf(gct[m]);
-      for (int j = 0; j <= r; ++j) {
-        const int sj = src[j];
-        if (sj >= 0) acc += Aj[j] * bf16_to_f32(p.s[((int64_t)sj * H + h) * MS + m]) * expf(gct[m] - gcl[j * MS + m]);
-      }
-      okl[m] = acc;
-      lmax = acc;
-    }
-    const float mg = block_max(lmax, red);
-    const float lg = block_sum(tid < MS ? expf(okl[tid] - mg) : 0.f, red);
-    const int lo = p.wl < 0 ? bos : (t - p.wl > bos ? t - p.wl : bos);
-    float wm = -INFINITY, wsum = 0.f;
-    for (int j = lo + tid; j <= t; j += 256) {
-      const float d = dot_row<bf16_t>(qs, p.k_swa + ((int64_t)j * H + h) * D, D);
-      if (d > wm) {
-        wsum = wsum * expf(wm - d) + 1.f;
-        wm = d;
-      } else {
-        wsum += expf(d - wm);
-      }
-    }
-    const float mw = block_max(wm, red);
-    const float lw = block_sum(wm == -INFINITY ? 0.f : wsum * expf(wm - mw), red);
-    if (tid == 0) {
-      if (p.lse_gsa) p.lse_gsa[(int64_t)t * HQ + hq] = mg + logf(lg);
-      if (p.lse_swa) p.lse_swa[(int64_t)t * HQ + hq] = mw + logf(lw);
-    }
-    const float mt = fmaxf(mg, mw);
-    const float inv = 1.f / (lg * expf(mg - mt) + lw * expf(mw - mt));
-    __syncthreads();
-    if (tid < MS) okl[tid] = expf(okl[tid] - mt) * inv;
-    __syncthreads();
-    if (tid < BT) {
-      const int sj = src[tid];
-      float acc = 0.f;
-      if (sj >= 0) {
-        const bf16_t* srow = p.s + ((int64_t)sj * H + h) * MS;
-        for (int m = 0; m < MS; ++m) acc += okl[m] * bf16_to_f32(srow[m]) * expf(gct[m] - gcl[tid * MS + m]);
-      }
-      Avj[tid] = acc;
-    }
-    __syncthreads();
-    float acc = 0.f;   // value column tid (D <= 256 == threads)
-    if (tid < D) {
-      for (int m = 0; m < MS; ++m) acc += okl[m] * expf(gct[m]) * hv[m * D + tid];
-      for (int j = 0; j <= r; ++j) {
-        const int sj = src[j];
-        if (sj >= 0) acc += Avj[j] * bf16_to_f32(p.v[((int64_t)sj * H + h) * D + tid]);
-      }
-    }
-    for (int jb = lo; jb <= t; jb += 256) {
-      const int j = jb + tid;
-      __syncthreads();
-      pw[tid] = j <= t ? expf(dot_row<bf16_t>(qs, p.k_swa + ((int64_t)j * H + h) * D, D) - mt) * inv : 0.f;
-      __syncthreads();
-      const int cnt = (t - jb + 1) < 256 ? (t - jb + 1) : 256;
-      if (tid < D)
-        for (int x = 0; x < cnt; ++x) acc += pw[x] * bf16_to_f32(p.v[((int64_t)(jb + x) * H + h) * D + tid]);
-    }
-    if (tid < D) p.o[((int64_t)t * HQ + hq) * D + tid] = f32_to_bf16(acc);
-  }
+  exact_rows<D, 1>(p, rsm, chunk, h, h * p.NG, p.NG, bits);
 }
 
 template <int D>
 int launch_repair(const MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  const size_t lds = RepairSmem<D>::floats * 4;
+  const size_t lds = ExactSmem<D, 1>::bytes;
   std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)mfma_repair_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));
@@ -1373,15 +1246,16 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
     // every CU, two fit one as well (8 / 4 heads, 4 x 8000 tokens, W = 1500: D = 128 378 -> 330-353 us, with 32-key tiles; D = 64
     // 244 -> 198); below, one with the fragments shared is faster (3000 tokens, 188 workgroups: 25 against 31, 17.5 against 19)
     int rc;
+    bool exact = false;   // the output pass has formed the flagged rows itself
 #ifdef NHA_AB_SWITCHES   // measurement builds only (-DNHA_AB_SWITCHES): run the kernels the LDS-direct ones replaced
     static const bool ring_off = getenv("NHA_PREFILL_NO_RING") != nullptr;
 #else
     constexpr bool ring_off = false;
 #endif
     if (!ring_off && prefill_ring_supported(p, D)) {
-      rc = prefill_ring_launch(p, D, st);
+      rc = prefill_ring_launch(p, D, &exact, st);
     } else if (!ring_off && prefill_ring256_supported(p, D)) {
-      rc = prefill_ring256_launch(p, st);
+      rc = prefill_ring256_launch(p, &exact, st);
     } else if constexpr (D <= 128) {
       if (p.NG % 4 == 0) rc = launch_out<D, 4, 8, 64, false>(p, st);
       else if (p.NG % 2 == 0 && (int64_t)p.HQ / 2 * p.NT > 256) rc = launch_out<D, 2, 8, D == 128 ? 32 : 64, true>(p, st);
@@ -1391,8 +1265,7 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
       if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 32, false>(p, st);
       else rc = launch_out<D, 1, 4, 32, true>(p, st);
     }
-    if (rc != NHA_OK) return rc;
-    return launch_repair<D>(p, st);
+    return rc != NHA_OK || exact ? rc : launch_repair<D>(p, st);
   }
   return NHA_OK;
 }

@@ -17,14 +17,14 @@
 //    nearest keys; 0 for rows that unit does not reach): fp32 sums relative to a fixed reference are
 //    exact while every score stays within 2^+-100 of it, and the loop carries no maxima, no
 //    comparisons and no rescaling of the accumulators.  A row whose window sum leaves that range
-//    (overflowed, or below 2^-100) is flagged for mfma_repair_kernel, which recomputes it exactly.
+//    (overflowed, or below 2^-100) is recomputed exactly at the end (prefill_exact.h).
 //
 // LDS layout of units, queries and slot tiles: LineTile (mfma_common.h), 64 consecutive bytes of a row per four lanes of a load.
 // Bound: matrix and vector instructions of two waves per SIMD at long windows (51 % of the matrix rate, 40 % of the vector issue at
 // T = 16384, W = 2048), operands arriving with nothing else resident on the CU at short ones.  With K units, query and
 // k-state rows loaded in 16-byte pieces and V in 32-byte ones: 505 -> 497 us at B=2, T=8192, 32/8 heads, W=2048, 1090 -> 1079 at
 // T=16384, 172.5 -> 171.5 at W=64, 19.6 -> 18.2 at 331 tokens (32/4 heads).
-#include "mfma_common.h"
+#include "prefill_exact.h"
 
 #include <mutex>
 
@@ -62,7 +62,8 @@ struct RingCfg {
   static constexpr int QT = TA;                // first the window queries, 32 rows of each of the eight waves
   static constexpr int GC = TD + 2 * UB;       // gate cumsum fp32 [64][64], pieces XORed with row % 16
   static constexpr int SS = GC + 16384;        // s bf16 [64][64], pieces XORed with row % 8
-  static constexpr int BYTES = SS + 8192;
+  static constexpr int FLAGS = SS + 8192;      // per wave: its 16-row blocks that the exact pass takes (a word of eight)
+  static constexpr int BYTES = FLAGS + 32;
   static constexpr int ETAB = 0;               // decay tables (6 units of 4 KB), over the ring once the window is done
   static constexpr int NSLOT_LOADS = 4 * LPW + 3;   // per wave: four tiles, two gate blocks, one s block
   static constexpr int EGI = ETAB + 6 * 4096;  // exp(gc_i[m]) fp32 [64][64], laid out like GC
@@ -70,11 +71,67 @@ struct RingCfg {
   static_assert(6 * 4096 + 2 * 16384 <= 2 * NR * UB, "decay tables must fit the ring");
 };
 
+// Exact rows for the window-only launch: key by key in fp32 with a running maximum, the sinks in view joining as keys of logit 0 and
+// value 0.  The two groups of 256 threads take two of the workgroup's four heads (hq0 ..) at a time.
+template <int D>
+__device__ __forceinline__ void sink_exact_rows(const MP& p, float* rsm, int chunk, int h, int hq0, int bits) {
+  constexpr int ROW = D + 256 + 4;
+  const int t = threadIdx.x & 255, group = threadIdx.x >> 8;
+  float* const qs = rsm + group * ROW;   // [D] scaled query
+  float* const pw = qs + D;              // [256]
+  float* const red = pw + 256;           // [4]
+  const int H = p.H, HQ = p.HQ;
+  const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
+  const int bos = p.cu[n], eos = p.cu[n + 1];
+  const int c0 = bos + it * BT;
+  const int rows = (eos - c0) < BT ? (eos - c0) : BT;
+  for (int hq = hq0 + group; hq < hq0 + 4; hq += 2)
+    for (int r = 0; r < rows; ++r) {
+      if (!((bits >> (r >> 4)) & 1)) continue;
+      const int tok = c0 + r;
+      __syncthreads();   // the previous row is finished
+      const bf16_t* qsw = p.q_swa + ((int64_t)tok * HQ + hq) * D;
+      for (int i = t; i < D; i += 256) qs[i] = bf16_to_f32(qsw[i]) * p.scale;
+      __syncthreads();
+      int n0 = p.wl - (tok - bos);
+      n0 = n0 < 0 ? 0 : (n0 > p.sinks ? p.sinks : n0);
+      const int lo = p.wl < 0 ? bos : (tok - p.wl > bos ? tok - p.wl : bos);
+      float wm = -INFINITY, wsum = 0.f;
+      for (int j = lo + t; j <= tok; j += 256) {
+        const float d = dot_row<bf16_t>(qs, p.k_swa + ((int64_t)j * H + h) * D, D);
+        if (d > wm) {
+          wsum = wsum * expf(wm - d) + 1.f;
+          wm = d;
+        } else {
+          wsum += expf(d - wm);
+        }
+      }
+      float mt = group_max(wm, red, t);
+      if (n0 > 0) mt = fmaxf(mt, 0.f);
+      const float lw = group_sum(wm == -INFINITY ? 0.f : wsum * expf(wm - mt), red, t) + (float)n0 * expf(-mt);
+      if (t == 0 && p.lse_swa) p.lse_swa[(int64_t)tok * HQ + hq] = mt + logf(lw);
+      const float inv = 1.f / lw;
+      float acc = 0.f;   // value column t (D <= 256 == threads of a group)
+      for (int jb = lo; jb <= tok; jb += 256) {
+        const int j = jb + t;
+        __syncthreads();
+        pw[t] = j <= tok ? expf(dot_row<bf16_t>(qs, p.k_swa + ((int64_t)j * H + h) * D, D) - mt) * inv : 0.f;
+        __syncthreads();
+        const int cnt = (tok - jb + 1) < 256 ? (tok - jb + 1) : 256;
+        if (t < D)
+          for (int x = 0; x < cnt; ++x) acc += pw[x] * bf16_to_f32(p.v[((int64_t)(jb + x) * H + h) * D + t]);
+      }
+      if (t < D) p.o[((int64_t)tok * HQ + hq) * D + t] = f32_to_bf16(acc);
+    }
+}
+
 // SINK: the window branch alone, with p.sinks zero-logit, zero-value keys in front of every sequence of which query t
 // (position in its sequence) still sees clamp(p.wl - t, 0, p.sinks): the "full attention" layers of the hybrid models
 // (nha_fla/models/qwen3_moe_nha/qwennha.py:323-336, :400-413).  No slot operands are requested, the slot branch and its
 // tables are skipped, and the sinks join the denominator in the epilogue with the weight 2^(-reference) each.
-template <int D, bool SINK = false>
+// EXACT: rows that leave the range of the kernel's arithmetic are formed again at the end (prefill_exact.h has when); without it
+// they are flagged for the exact pass after it.
+template <int D, bool SINK, bool EXACT>
 __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   using C = RingCfg<D>;
   constexpr int KS = C::KS, DB = C::DB, UB = C::UB, HB = C::HB, NR = C::NR, LPW = C::LPW;
@@ -102,6 +159,8 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   const int rows = (eos - c0) < BT ? (eos - c0) : BT;
   const float cs = p.scale * LOG2E;
   const int64_t cg = (int64_t)chunk * H + h;
+  int exact = 0;   // 16-row blocks of the chunk that decay too fast for the split decay (flags of the state pass)
+  if constexpr (!SINK && EXACT) exact = p.flags[cg * 4] | p.flags[cg * 4 + 1] | p.flags[cg * 4 + 2] | p.flags[cg * 4 + 3];
 
   // window units: unit u covers keys [c0 + 32 - 32 u, c0 + 64 - 32 u); c0 - bos is a multiple of 64, so no
   // unit starts before its sequence; units 0 and 1 are the chunk's own rows and may run past eos
@@ -485,10 +544,16 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   // a window sum outside 2^+-100 of the fixed reference (overflowed sums are +inf: beyond the upper bound):
   // products with the values may have left fp32, or bf16 probabilities may have been flushed to zero
   // that matter against the sum; the exact pass redoes the rows of the sub-block
+  int bad = 0;
 #pragma unroll
-  for (int qb = 0; qb < RQB; ++qb) {
-    const bool bad = (16 * (qb0 + qb) + l16 < rows) && (Lw[qb][0] >= 0x1p100f || Lw[qb][0] < 0x1p-100f);
-    if (__any(bad) && lane == 0) atomicOr(p.flags + cg * 4, 1 << (qb0 + qb));
+  for (int qb = 0; qb < RQB; ++qb)
+    if (__any(16 * (qb0 + qb) + l16 < rows && (Lw[qb][0] >= 0x1p100f || Lw[qb][0] < 0x1p-100f))) bad |= 1 << (qb0 + qb);
+  constexpr int FLAGS = SINK ? 0 : C::FLAGS;
+  if constexpr (SINK) lds_barrier();   // the ring is done with
+  if constexpr (EXACT) {
+    if (lane == 0) *reinterpret_cast<NHA_LDS int*>(lds + FLAGS + 4 * wave) = bad;
+  } else if (bad && lane == 0) {
+    atomicOr(p.flags + cg * 4, bad);
   }
   float lg[RQB];
   if constexpr (SINK) {
@@ -510,6 +575,11 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   if (nunits <= NR) wait_vm<4 * LPW>();
   else wait_vm<0>();
   lds_barrier();
+  if constexpr (EXACT) {
+#pragma unroll
+    for (int w = 0; w < 8; ++w) exact |= *reinterpret_cast<const NHA_LDS int*>(lds + C::FLAGS + 4 * w);
+    exact = __builtin_amdgcn_readfirstlane(exact);
+  }
   auto gc_at = [&](int j, int m) -> const lfloat* { return (const lfloat*)(lds + C::GC + j * 256 + (((m >> 2) ^ (j & 15)) * 16) + (m & 3) * 4); };
   auto s_at = [&](int j, int m) -> const lbf16* { return (const lbf16*)(lds + C::SS + j * 128 + (((m >> 3) ^ (j & 7)) * 16) + (m & 7) * 2); };
   // decay tables E_Q[j][m] = s_j[m] exp(min(gr_Q[m] - gc_j[m], DECAY_CLAMP)) for the rows j of the 16-row
@@ -753,87 +823,35 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
       if (irow < rows) *reinterpret_cast<uint4*>(op + dcol) = make_uint4(a[0], a[1], b[0], b[1]);
     }
   }
+  // ---- rows that have to be formed again, for the four heads of the workgroup -----------------------
+  if constexpr (!EXACT) return;
+  if constexpr (SINK) {
+    lds_barrier();
+#pragma unroll
+    for (int w = 0; w < 8; ++w) exact |= *reinterpret_cast<const NHA_LDS int*>(lds + 4 * w);
+    exact = __builtin_amdgcn_readfirstlane(exact);
+  }
+  if (exact == 0) return;
+  before_exact();
+  if constexpr (SINK) sink_exact_rows<D>(p, reinterpret_cast<float*>(smem_), chunk, h, h * NG + grp * 4, exact);
+  else if constexpr (EXACT) exact_rows<D, 2>(p, reinterpret_cast<float*>(smem_), chunk, h, h * NG + grp * 4, 4, exact);
 }
 
-template <int D, bool SINK>
+template <int D, bool SINK, bool EXACT>
 int launch_ring(const MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   // the window-only launch has no slot operands: the ring and the eight waves' window queries behind it (128 KB at D = 128, 96 at
   // 64; its registers leave room for one workgroup per CU as well)
   const size_t lds = SINK ? (size_t)(RingCfg<D>::QT + 8 * RingCfg<D>::UB) : (size_t)RingCfg<D>::BYTES;
-  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring_out_kernel<D, SINK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring_out_kernel<D, SINK, EXACT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL((ring_out_kernel<D, SINK>), dim3(p.H * (p.NG / 4), p.NT), dim3(512), lds, st, p);
+  hipLaunchKernelGGL((ring_out_kernel<D, SINK, EXACT>), dim3(p.H * (p.NG / 4), p.NT), dim3(512), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma output pass, ring)");
   return NHA_OK;
-}
-
-__global__ __launch_bounds__(256) void zero_flags_kernel(int* flags, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) flags[i] = 0;
-}
-
-// Exact rows for the window-only launch: the rows of 16-row blocks whose window sums left the range of their fixed
-// softmax reference (flags set by ring_out_kernel<D, true>) are recomputed key by key in fp32 with a running maximum,
-// the sinks in view joining as keys of logit 0 and value 0.  grid (chunk, kv-head); workgroups of unflagged chunks
-// read four words and leave.
-template <int D>
-__global__ __launch_bounds__(256) void sink_repair_kernel(const MP p) {
-  const int chunk = blockIdx.x, h = blockIdx.y;
-  const int H = p.H, HQ = p.HQ;
-  const int* fl = p.flags + ((int64_t)chunk * H + h) * 4;
-  const int bits = fl[0] | fl[1] | fl[2] | fl[3];
-  if (bits == 0) return;
-  __shared__ float qs[D];
-  __shared__ float pw[256];
-  __shared__ float red[4];
-  const int tid = threadIdx.x;
-  const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
-  const int bos = p.cu[n], eos = p.cu[n + 1];
-  const int c0 = bos + it * BT;
-  const int rows = (eos - c0) < BT ? (eos - c0) : BT;
-  for (int hq = h * p.NG; hq < (h + 1) * p.NG; ++hq)
-    for (int r = 0; r < rows; ++r) {
-      if (!((bits >> (r >> 4)) & 1)) continue;
-      const int t = c0 + r;
-      __syncthreads();   // the previous row is finished
-      const bf16_t* qsw = p.q_swa + ((int64_t)t * HQ + hq) * D;
-      for (int i = tid; i < D; i += 256) qs[i] = bf16_to_f32(qsw[i]) * p.scale;
-      __syncthreads();
-      int n0 = p.wl - (t - bos);
-      n0 = n0 < 0 ? 0 : (n0 > p.sinks ? p.sinks : n0);
-      const int lo = p.wl < 0 ? bos : (t - p.wl > bos ? t - p.wl : bos);
-      float wm = -INFINITY, wsum = 0.f;
-      for (int j = lo + tid; j <= t; j += 256) {
-        const float d = dot_row<bf16_t>(qs, p.k_swa + ((int64_t)j * H + h) * D, D);
-        if (d > wm) {
-          wsum = wsum * expf(wm - d) + 1.f;
-          wm = d;
-        } else {
-          wsum += expf(d - wm);
-        }
-      }
-      float mt = block_max(wm, red);
-      if (n0 > 0) mt = fmaxf(mt, 0.f);
-      const float lw = block_sum(wm == -INFINITY ? 0.f : wsum * expf(wm - mt), red) + (float)n0 * expf(-mt);
-      if (tid == 0 && p.lse_swa) p.lse_swa[(int64_t)t * HQ + hq] = mt + logf(lw);
-      const float inv = 1.f / lw;
-      float acc = 0.f;   // value column tid (D <= 256 == threads)
-      for (int jb = lo; jb <= t; jb += 256) {
-        const int j = jb + tid;
-        __syncthreads();
-        pw[tid] = j <= t ? expf(dot_row<bf16_t>(qs, p.k_swa + ((int64_t)j * H + h) * D, D) - mt) * inv : 0.f;
-        __syncthreads();
-        const int cnt = (t - jb + 1) < 256 ? (t - jb + 1) : 256;
-        if (tid < D)
-          for (int x = 0; x < cnt; ++x) acc += pw[x] * bf16_to_f32(p.v[((int64_t)(jb + x) * H + h) * D + tid]);
-      }
-      if (tid < D) p.o[((int64_t)t * HQ + hq) * D + tid] = f32_to_bf16(acc);
-    }
 }
 
 }  // namespace
@@ -846,12 +864,15 @@ bool prefill_ring_supported(const mf::MP& p, int D) {
   return (int64_t)p.T_tot * p.H * D * 2 < ((int64_t)1 << 32) && (int64_t)p.T_tot * p.H * MS * 2 < ((int64_t)1 << 32);
 }
 
-int prefill_ring_launch(const mf::MP& p, int D, hipStream_t st) {
-  return D == 64 ? launch_ring<64, false>(p, st) : launch_ring<128, false>(p, st);
+int prefill_ring_launch(const mf::MP& p, int D, bool* exact, hipStream_t st) {
+  // a workgroup takes 18 us and 0.85 per unit at D = 128
+  *exact = (double)p.NT * p.HQ / 4 / 256 * (18 + 0.85 * window_units(p, BT)) <= EXACT_INSIDE_US;
+  if (*exact) return D == 64 ? launch_ring<64, false, true>(p, st) : launch_ring<128, false, true>(p, st);
+  return D == 64 ? launch_ring<64, false, false>(p, st) : launch_ring<128, false, false>(p, st);
 }
 
-// Sliding-window attention with zero sinks (nha_sink_window_fwd): the window loop of ring_out_kernel alone.  The scratch
-// holds the flags of the 16-row blocks that go to the exact pass.
+// Sliding-window attention with zero sinks (nha_sink_window_fwd): the window loop of ring_out_kernel alone.  (What
+// goes to the exact pass stays on the chip: the scratch that callers bring is not used any more.)
 size_t sink_window_scratch_bytes(const NhaSinkWindowArgs* a) { return ((size_t)a->NT * a->H * 4 * sizeof(int) + 255) & ~(size_t)255; }
 
 int sink_window_impl(const NhaSinkWindowArgs* a) {
@@ -860,7 +881,6 @@ int sink_window_impl(const NhaSinkWindowArgs* a) {
   p.o = (bf16_t*)a->o;
   p.lse_swa = a->lse;
   p.cu = a->cu_seqlens; p.cidx = a->chunk_indices; p.coff = a->chunk_offsets;
-  p.flags = (int*)a->scratch;
   p.T_tot = a->T_tot; p.N = a->N; p.NT = a->NT; p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H;
   p.wl = a->window - 1; p.shift = 0; p.scale = a->scale; p.sinks = a->sinks;
   if (a->dtype != NHA_DTYPE_BF16 || !prefill_ring_supported(p, a->D) || p.NT > 65535) {
@@ -869,15 +889,7 @@ int sink_window_impl(const NhaSinkWindowArgs* a) {
     return NHA_ERR_UNSUPPORTED;
   }
   hipStream_t st = (hipStream_t)a->stream;
-  const int nflags = a->NT * a->H * 4;
-  hipLaunchKernelGGL(zero_flags_kernel, dim3((nflags + 255) / 256), dim3(256), 0, st, p.flags, nflags);
-  NHA_CHECK_LAUNCH("nha_sink_window_fwd(flags)");
-  const int rc = a->D == 64 ? launch_ring<64, true>(p, st) : launch_ring<128, true>(p, st);
-  if (rc != NHA_OK) return rc;
-  if (a->D == 64) hipLaunchKernelGGL((sink_repair_kernel<64>), dim3(p.NT, p.H), dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((sink_repair_kernel<128>), dim3(p.NT, p.H), dim3(256), 0, st, p);
-  NHA_CHECK_LAUNCH("nha_sink_window_fwd(exact rows)");
-  return NHA_OK;
+  return a->D == 64 ? launch_ring<64, true, true>(p, st) : launch_ring<128, true, true>(p, st);
 }
 
 }  // namespace nha

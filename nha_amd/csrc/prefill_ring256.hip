@@ -29,8 +29,8 @@
 //  * The softmax reference of a row is fixed by the prologue (the chunk's own keys): rescaling 64
 //    accumulator registers inside the loop costs the loop its registers whether or not the branch is
 //    taken.  A unit whose maximum tops the reference by 2^96 hands the wave's 16 rows to the exact pass
-//    (mfma_repair_kernel) and is clamped.
-#include "mfma_common.h"
+//    (prefill_exact.h) and is clamped.
+#include "prefill_exact.h"
 
 #include <mutex>
 #include <type_traits>
@@ -67,11 +67,13 @@ struct Cfg {
   static constexpr int SS = GC + 16384;        // s bf16 [64][64], pieces XORed with row % 8
   static constexpr int ETAB = SS + 8192;       // decay tables, 6 units of 4 KB
   static constexpr int GC2 = ETAB + 6 * 4096;  // gate cumsums of the second chunk (NCH == 2)
-  static constexpr int BYTES = GC2 + (NCH - 1) * 16384;
+  static constexpr int USED = GC2 + (NCH - 1) * 16384, EXACT = ExactSmem<D, NCH>::bytes;
+  static constexpr int BYTES = USED > EXACT ? USED : EXACT;
 };
 
 // LDS layout of a 32-row buffer: LineTile.
-template <int NCH>
+// EXACT: as in ring_out_kernel (prefill_ring.hip).
+template <int NCH, bool EXACT>
 __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   using C = Cfg<NCH>;
   constexpr int XB0 = 64 * NCH - 32;           // first key of unit 0, relative to the workgroup's first row
@@ -104,6 +106,17 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   const int64_t cg = (int64_t)chunk * H + h;   // (chunk, kv-head) of the first chunk; the second one is H further
   const int irow = 16 * Q + l16;               // this lane's query row inside its chunk
   const int yrow = BT * ch + irow;             // ... and inside the workgroup's rows
+  // per chunk of the workgroup, the 16-row blocks that are formed again at the end: those that decay too fast for the split decay
+  // (flags of the state pass), and in the waves' own words those whose scores leave the range of their softmax reference
+  int exact[NCH], bad = 0;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    exact[c] = 0;
+    if (EXACT && rows_wg > BT * c) {
+      const int* const f = p.flags + (cg + (int64_t)c * H) * 4;
+      exact[c] = f[0] | f[1] | f[2] | f[3];
+    }
+  }
   const int r0w = BT * ch + 16 * Q;            // first row of this wave
 
   // window units: unit u covers keys [c0 + XB0 - 32 u, c0 + XB0 + 32 - 32 u); c0 - bos is a multiple of 64, so no
@@ -486,9 +499,13 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     // The reference of the window stays where the prologue put it: moving it would mean rescaling 64
     // accumulator registers inside this loop, which costs the loop its registers whether or not the branch
     // is ever taken.  fp32 sums and bf16 probabilities hold 2^BIG above it; a score beyond that sends the
-    // wave's 16 rows to the exact pass (mfma_repair_kernel recomputes flagged sub-blocks) and is clamped.
+    // wave's 16 rows to the exact pass and is clamped.
     if (__any(m0 > BIG)) {
-      if (lane == 0 && 16 * Q < rows) atomicOr(p.flags + (cg + (int64_t)ch * H) * 4, 1 << Q);   // (a chunk that is not there has no flags)
+      if constexpr (EXACT) {
+        if (16 * Q < rows) bad = 1 << Q;   // (a chunk that is not there has no flags)
+      } else if (lane == 0 && 16 * Q < rows) {
+        atomicOr(p.flags + (cg + (int64_t)ch * H) * 4, 1 << Q);
+      }
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -751,6 +768,20 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
       if (irow < rows) *reinterpret_cast<uint4*>(op + dcol) = make_uint4(a[0], a[1], b[0], b[1]);
     }
   }
+  // ---- rows that have to be formed again (prefill_exact.h) ------------------------------------------
+  if constexpr (!EXACT) return;
+  lds_barrier();
+  if (lane == 0) *reinterpret_cast<NHA_LDS int*>(lds + 4 * wave) = bad;
+  lds_barrier();
+#pragma unroll
+  for (int w = 0; w < NW; ++w) exact[w >> 2] |= *reinterpret_cast<const NHA_LDS int*>(lds + 4 * w);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int bits = __builtin_amdgcn_readfirstlane(exact[c]);
+    if (bits == 0) continue;
+    before_exact();
+    exact_rows<D, NCH>(p, reinterpret_cast<float*>(smem_), chunk + c, h, hq, 1, bits);
+  }
 }
 
 }  // namespace
@@ -763,26 +794,30 @@ bool prefill_ring256_supported(const mf::MP& p, int D) {
   return (int64_t)p.T_tot * p.H * D * 2 < ((int64_t)1 << 32) && (int64_t)p.T_tot * p.H * MS * 2 < ((int64_t)1 << 32);
 }
 
-int prefill_ring256_launch(const mf::MP& p, hipStream_t st) {
+namespace {
+template <int NCH, bool EXACT>
+int launch_ring256(const mf::MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  std::call_once(once, [&] {
-    attr_err = hipFuncSetAttribute((const void*)ring256_out_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg<2>::BYTES);
-    if (attr_err == hipSuccess)
-      attr_err = hipFuncSetAttribute((const void*)ring256_out_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg<1>::BYTES);
-  });
+  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring256_out_kernel<NCH, EXACT>, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg<NCH>::BYTES); });
   if (attr_err != hipSuccess) {
-    set_error("nha_prefill_fwd(mfma): cannot reserve %d bytes of LDS: %s", Cfg<2>::BYTES, hipGetErrorString(attr_err));
+    set_error("nha_prefill_fwd(mfma): cannot reserve %d bytes of LDS: %s", Cfg<NCH>::BYTES, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
-  // two chunks per workgroup unless most sequences have a single chunk (fewer than three chunks per two sequences):
-  // there the second half of a two-chunk workgroup would mostly idle
-  if (2 * (int64_t)p.NT < 3 * (int64_t)p.N)
-    hipLaunchKernelGGL(ring256_out_kernel<1>, dim3(p.HQ, p.NT), dim3(256), Cfg<1>::BYTES, st, p);
-  else
-    hipLaunchKernelGGL(ring256_out_kernel<2>, pair_grid(p.HQ, p.NT, p.N), dim3(512), Cfg<2>::BYTES, st, p);
+  hipLaunchKernelGGL((ring256_out_kernel<NCH, EXACT>), NCH == 1 ? dim3(p.HQ, p.NT) : pair_grid(p.HQ, p.NT, p.N), dim3(256 * NCH), Cfg<NCH>::BYTES, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma output pass, ring, head size 256)");
   return NHA_OK;
+}
+}  // namespace
+
+int prefill_ring256_launch(const mf::MP& p, bool* exact, hipStream_t st) {
+  // two chunks per workgroup unless most sequences have a single chunk (fewer than three chunks per two sequences):
+  // there the second half of a two-chunk workgroup would mostly idle
+  const bool one = 2 * (int64_t)p.NT < 3 * (int64_t)p.N;
+  // a workgroup takes 18 us and 0.9 per unit
+  *exact = (double)p.NT / (one ? 1 : 2) * p.HQ / 256 * (18 + 0.9 * window_units(p, one ? BT : 2 * BT)) <= EXACT_INSIDE_US * 3 / 5;
+  if (one) return *exact ? launch_ring256<1, true>(p, st) : launch_ring256<1, false>(p, st);
+  return *exact ? launch_ring256<2, true>(p, st) : launch_ring256<2, false>(p, st);
 }
 
 }  // namespace nha

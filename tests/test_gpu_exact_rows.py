@@ -1,0 +1,47 @@
+"""Rows that leave the range of the output pass's arithmetic are formed again by the pass itself where it is short and by a launch
+after it where it is long (prefill_exact.h).  The same sequences, some of whose rows decay too fast, in one long call and each alone:
+the two forms share their arithmetic but not their instances, and calls of other sizes may cut their states into other segments, which
+rounds chunk-start states of bf16 (2^-9) differently; outputs 2e-2 absolute + 1e-2 relative per element as in the parity tests, which
+hold the short calls against the oracle."""
+import pytest
+import torch
+
+from tests.util import assert_close, prefill_inputs
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+KEYS = ["q_swa", "k_swa", "q_gsa", "k_gsa", "v", "s", "g"]
+
+
+# estimates of the output pass (us, of which 200 or, at head size 256, 120 are the line): 280, 230, 230 in one call, below 5 alone
+@pytest.mark.parametrize("D,HQ,H,N", [(128, 32, 8, 42), (64, 16, 4, 70), (256, 8, 2, 64)])
+def test_exact_rows_inside_and_after(D, HQ, H, N):
+    from nha_amd import chunk_nha
+    L = 700
+    d = prefill_inputs(9500 + D, 1, N * L, HQ, H, D, D, 64, dtype=BF, qk_scale=D ** -0.5)
+    for n in (0, 1, N - 1):                       # decays of e^-80 within 16 rows, in some slots of some rows
+        lo = n * L + 100 + 37 * (n % 3)
+        d["g"][:, lo:lo + 40, :, 3:20] = -5.0
+        d["s"][:, lo:lo + 40, :, 3:20] = 0.99
+    c = [d[k].cuda() for k in KEYS]
+    cu = torch.arange(0, N * L + 1, L, dtype=torch.int32, device="cuda")
+    got = chunk_nha(*c, cu_seqlens=cu, window_size_left=63, gsa_kv_shift=64)
+    for n in (0, 1, 2, N - 1):
+        alone = chunk_nha(*(x[:, n * L:(n + 1) * L] for x in c), window_size_left=63, gsa_kv_shift=64)
+        for name, x, y in zip(("o", "lse_swa", "lse_gsa"), got, alone):
+            assert_close(f"{name} D{D} sequence {n}", x[:, n * L:(n + 1) * L], y, BF)
+
+
+def test_exact_rows_of_one_head_in_pairs():
+    """Head size 256: the two halves of a workgroup take rows of the same head; windows of 256 and more keys, whose rows walk
+    them in different numbers of steps, an odd number of rows, the last of them alone."""
+    from nha_amd import chunk_nha
+    T, H = 619, 2
+    d = prefill_inputs(9600, 1, T, H, H, 256, 256, 64, dtype=BF, qk_scale=256 ** -0.5)
+    d["g"][:, 240:300, :, 3:20] = -5.0
+    d["g"][:, 600:, :, 3:20] = -5.0
+    c = [d[k].cuda() for k in KEYS]
+    got = chunk_nha(*c, window_size_left=255)
+    ref = chunk_nha(*(x.float() for x in c), window_size_left=255, impl="simple")
+    for name, x, y in zip(("o", "lse_swa", "lse_gsa"), got, ref):
+        assert_close(name, x, y, BF)
