@@ -3,13 +3,16 @@
 //
 // The contraction runs over the tokens, the outer axis of both operands, and the outputs are small: 1024 x 1024 from 16384
 // tokens is 16 tiles of 256 x 256, so the tokens are split over workgroups (wgrad_split), each leaves its tile's sum in
-// fp32 and a second launch adds the splits in a fixed order.  Both operands go to LDS as they lie ([token][column]) and
-// are read by the transposing LDS read, which hands a lane the tokens of one column.
+// fp32 and a second launch adds the splits in a fixed order.  Both operands go straight into LDS as they lie ([token][column],
+// LineTile), a ring of four units of 32 tokens, and are read by the transposing LDS read, which hands a lane the tokens of one column.
 //
-// Bound: LDS.  A workgroup of eight waves (128 x 64 of the tile each, two per SIMD) reads 197 KB and writes 64 KB of LDS
-// per 64 tokens, as many clocks as its matrix products take.  16384 tokens, 1024 columns, outputs of 3 x 1024 + 256: 138 us
-// with the sum (0.81 PFLOP/s) against 415 us for four library products, which run 64 x 64 tiles without a split; one output
-// of 1024: 54 against 104 us; 2048 columns, 2048 + 2 x 512 + 256: 250 against 468 us.
+// Bound: the matrix rate that this chip sustains (1.2 PFLOP/s, as a large library product) where the tiles
+// fill it, and the fp32 sums' way through memory where few outputs make many splits.  Eight waves hold 128 x 64 of a tile
+// each; a unit's fragments are in registers when its products begin and are replaced as they are done with.  Through registers and
+// padded rows, two buffers of 64 tokens, no read ahead: 16384 tokens, 1024 columns, outputs of 3 x 1024 + 256 127 us with the sum,
+// now 119 (0.93 PFLOP/s; four library products, which run 64 x 64 tiles without a split, 415); one output of 1024 53, 53 (library
+// 104); 2048 columns, 2048 + 2 x 512 + 256 217, 207 (468); 3072 columns, 3072 + 2 x 768 + 512 460, 440; 4096 tokens, 1024 columns,
+// 1024 + 2 x 256 + 128 44.5, 39.  A fifth unit in LDS: 123 and 40 where four take 119 and 39.
 #include "mfma_common.h"
 
 #include <atomic>
@@ -19,10 +22,13 @@ namespace {
 using namespace mf;
 
 constexpr int TW = 256;        // tile: columns of x and of dy
-constexpr int TK = 64;         // tokens per step
-constexpr int LDW = TW + 16;   // a row is 8 banks past the one before it: the 16 rows of a transposing read meet no conflict
+constexpr int TK = 32;         // tokens per unit
 constexpr int NTHR = 512;
-constexpr size_t LDS_BYTES = (size_t)4 * TK * LDW * 2;
+constexpr int NRING = 4;       // units in LDS
+typedef LineTile<TW> Tile;     // 32 tokens x 256 columns, 16 KB
+constexpr int TBYTES = 2 * Tile::HALF, UNIT = 2 * TBYTES;   // x, then dy
+constexpr size_t LDS_BYTES = (size_t)NRING * UNIT;
+#define FENCE __builtin_amdgcn_sched_barrier(0)
 
 struct WG {
   const bf16_t* x;
@@ -34,10 +40,11 @@ struct WG {
   float* part;                   // [split][rows][I]
 };
 
-__global__ __launch_bounds__(NTHR, 2) void wgrad_kernel(const WG p) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  lbf16* const tiles = (lbf16*)smem;   // x 0, x 1, dy 0, dy 1
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__global__ __launch_bounds__(NTHR, 1) void wgrad_kernel(const WG p) {
+  extern __shared__ __align__(1024) unsigned char smem[];
+  const lbyte* const lds = (const lbyte*)smem;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, kb = lane >> 4;
   // tiles dealt so that an XCD (workgroup id % 8) works on neighbouring tiles of one token range and their rows meet in its L2
   const int total = gridDim.x, per = total >> 3, L = blockIdx.x;
@@ -47,68 +54,100 @@ __global__ __launch_bounds__(NTHR, 2) void wgrad_kernel(const WG p) {
   while (q + 1 < p.n && ot >= p.tile0[q + 1]) ++q;
   const int O = p.O[q], ldy = p.ldy[q], o0 = (ot - p.tile0[q]) * TW, i0 = it * TW;
   const int t0 = sp * p.tsplit, t1 = t0 + p.tsplit < p.T ? t0 + p.tsplit : p.T;
-  const int steps = (t1 - t0 + TK - 1) / TK;   // every split holds tokens
-  const bf16_t* const xs = p.x + i0;
-  const bf16_t* const ys = p.dy[q] + o0;
-  const bool whole = i0 + TW <= p.I && o0 + TW <= O;
-  const int row = tid >> 5, col = (tid & 31) * 8;   // 16 rows per pass, four passes
+  const int units = (t1 - t0 + TK - 1) / TK;   // every split holds tokens
+  const bf16_t* const xs = p.x + (int64_t)t0 * p.I + i0;
+  const bf16_t* const ys = p.dy[q] + (int64_t)t0 * ldy + o0;
 
-  uint4 rx[4], ry[4];
-  auto load = [&](int s) {
-    const int ts = t0 + s * TK;
-    if (whole && ts + TK <= t1) {
+  // LDS-direct loads: block wave + 8 i of a tile's 16, a row and eight columns of it per lane.  Columns past the matrix are read from
+  // its last ones (their sums are not stored), tokens past the range from its last one (zeroed in the registers).
+  uint32_t xoff[2], yoff[2];   // bytes from the unit's first row
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        rx[u] = *reinterpret_cast<const uint4*>(xs + (int64_t)(ts + 16 * u + row) * p.I + col);
-        ry[u] = *reinterpret_cast<const uint4*>(ys + (int64_t)(ts + 16 * u + row) * ldy + col);
+  for (int i = 0; i < 2; ++i) {
+    const int r = 16 * i + Tile::load_row(lane), c = (int)Tile::load_col(wave, lane);
+    xoff[i] = (uint32_t)(r * p.I + (i0 + c < p.I ? c : p.I - 8 - i0)) * 2;
+    yoff[i] = (uint32_t)(r * ldy + (o0 + c < O ? c : O - 8 - o0)) * 2;
+  }
+  auto issue = [&](int u) {
+    const bf16_t* const xb = xs + (int64_t)u * TK * p.I;
+    const bf16_t* const yb = ys + (int64_t)u * TK * ldy;
+    const uint32_t to = lds0 + (u & (NRING - 1)) * UNIT + Tile::block(0, wave);
+    if (t0 + (u + 1) * TK <= t1) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        g2l16(xb, xoff[i], to + Tile::block(i, 0));
+        g2l16(yb, yoff[i], to + TBYTES + Tile::block(i, 0));
       }
     } else {
+      const int last = t1 - 1 - t0 - u * TK;   // < 31
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = ts + 16 * u + row;
-        rx[u] = ry[u] = make_uint4(0, 0, 0, 0);
-        if (t < t1 && i0 + col < p.I) rx[u] = *reinterpret_cast<const uint4*>(xs + (int64_t)t * p.I + col);
-        if (t < t1 && o0 + col < O) ry[u] = *reinterpret_cast<const uint4*>(ys + (int64_t)t * ldy + col);
+      for (int i = 0; i < 2; ++i) {
+        const int r = 16 * i + Tile::load_row(lane), back = r > last ? r - last : 0;
+        g2l16(xb, xoff[i] - (uint32_t)(back * p.I) * 2, to + Tile::block(i, 0));
+        g2l16(yb, yoff[i] - (uint32_t)(back * ldy) * 2, to + TBYTES + Tile::block(i, 0));
       }
     }
   };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      lds_st16(tiles + buf * TK * LDW + (16 * u + row) * LDW + col, rx[u]);
-      lds_st16(tiles + (2 + buf) * TK * LDW + (16 * u + row) * LDW + col, ry[u]);
-    }
-  };
+  // column fragments of the wave's 128 x 64 of the tile: x columns 16 a .., dy columns 16 b ..
   const int wi = (wave & 1) * 128, wo = (wave >> 1) * 64;
+  const Tile tile(lds, lane);
+  auto xfrag = [&](int u, int a) { return tile.col((uint32_t)((u & (NRING - 1)) * UNIT + wi * 32), a); };
+  auto yfrag = [&](int u, int b) { return tile.col((uint32_t)((u & (NRING - 1)) * UNIT + TBYTES + wo * 32), b); };
   f32x4 acc[8][4];
 #pragma unroll
   for (int a = 0; a < 8; ++a)
 #pragma unroll
     for (int b = 0; b < 4; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  load(0);
-  store(0);
-  if (steps > 1) load(1);
+
+  issue(0);
+  if (units > 1) issue(1);
+  if (units > 2) issue(2);
+  if (units > 2) wait_vm<8>();
+  else if (units > 1) wait_vm<4>();
+  else wait_vm<0>();
   lds_barrier();
-  for (int s = 0; s < steps; ++s) {
-    // the other buffer was read in step s - 1, which every wave has left
-    if (s + 1 < steps) store((s + 1) & 1);
-    if (s + 2 < steps) load(s + 2);
-    const lbf16* const X = tiles + (s & 1) * TK * LDW;
-    const lbf16* const Y = tiles + (2 + (s & 1)) * TK * LDW;
+  bf16x8 fx[8], fy[4];
 #pragma unroll
-    for (int k = 0; k < TK; k += 32) {
-      bf16x8 fy[4];
+  for (int b = 0; b < 4; ++b) fy[b] = yfrag(0, b);
 #pragma unroll
-      for (int b = 0; b < 4; ++b) fy[b] = lds_frag_tr(Y, LDW, k, k + 16, wo + 16 * b, lane);
-#pragma unroll
-      for (int a = 0; a < 8; ++a) {
-        const bf16x8 fx = lds_frag_tr(X, LDW, k, k + 16, wi + 16 * a, lane);
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = mfma16(fx, fy[b], acc[a][b]);
-      }
-    }
+  for (int a = 0; a < 8; ++a) fx[a] = xfrag(0, a);
+  // A unit's fragments are in registers when its products begin; those of the next one replace them as they are done with, a
+  // column block of x (four products) at a time.  One barrier per unit: behind it unit u + 1 has landed for everybody, and
+  // everybody has read unit u, so the slot of unit u - 1 takes unit u + 3.
+#pragma unroll 1
+  for (int u = 0; u + 1 < units; ++u) {
+    if (u + 2 < units) wait_vm<4>();
+    else wait_vm<0>();
     lds_barrier();
+    if (u + 3 < units) issue(u + 3);
+    FENCE;
+    bf16x8 ny[4];
+#pragma unroll
+    for (int a = 0; a < 8; ++a) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) acc[a][b] = mfma16(fx[a], fy[b], acc[a][b]);
+      FENCE;
+      fx[a] = xfrag(u + 1, a);
+      if (a % 2 == 0) ny[a / 2] = yfrag(u + 1, a / 2);
+      FENCE;
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b) fy[b] = ny[b];
   }
+  const int rem = (t1 - t0) - (units - 1) * TK;   // tokens of the last unit: 4 kb + e and 16 + 4 kb + e in a lane
+  if (rem < TK) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const bool on = (e < 4 ? 4 * kb + e : 12 + 4 * kb + e) < rem;
+#pragma unroll
+      for (int a = 0; a < 8; ++a) fx[a][e] = on ? fx[a][e] : (__bf16)0.f;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) fy[b][e] = on ? fy[b][e] : (__bf16)0.f;
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < 8; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[a][b] = mfma16(fx[a], fy[b], acc[a][b]);
   // acc[a][b]: columns i0 + wi + 16 a + 4 kb .. + 4 of row o0 + wo + 16 b + l16
   float* const out = p.part + ((int64_t)sp * p.rows + p.row0[q]) * p.I;
 #pragma unroll
@@ -140,7 +179,7 @@ __global__ __launch_bounds__(256) void wgrad_sum_kernel(const WG p) {
   Elem<bf16_t>::st8(p.dw[q] + (int64_t)(r - p.row0[q]) * p.I + c, s);
 }
 
-// Token splits: a round of the chip is 256 workgroups; a step of 64 tokens costs 1.4 us and a workgroup's start and end 6,
+// Token splits: a round of the chip is 256 workgroups; a unit of 32 tokens costs 0.6 us and a workgroup's start and end 6,
 // a split's round trip in fp32 its bytes (4 written and 4 read per element) at 4.5 TB/s.
 int wgrad_split(int tiles, int T, int64_t elements) {
   const int steps = (T + TK - 1) / TK;
@@ -148,7 +187,7 @@ int wgrad_split(int tiles, int T, int64_t elements) {
   double cost = 1e30;
   for (int s = 1; s <= 32 && s <= steps; ++s) {
     const double rounds = (double)(((int64_t)tiles * s + 255) / 256);
-    const double us = rounds * (((steps + s - 1) / s) * 1.4 + 6.0) + s * (double)elements * 8.0 / 4.5e6;
+    const double us = rounds * (((steps + s - 1) / s) * 0.6 + 6.0) + s * (double)elements * 8.0 / 4.5e6;
     if (us < cost) {
       cost = us;
       best = s;

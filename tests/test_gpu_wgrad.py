@@ -23,6 +23,23 @@ def test_wgrad(T, width, outs):
         assert rel <= 4e-3, f"{tuple(dw.shape)}: relative L2 error {rel:.3e}"
 
 
+# units of 32 tokens, of which four lie in LDS: one token to five units, a token less and more
+@pytest.mark.parametrize("T", [31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 160, 161])
+def test_wgrad_few_units(T):
+    """Tokens past the last one add nothing, whatever the last one holds: an infinite gradient stays infinite, and reaches its row
+    of the weights only."""
+    from nha_amd.ops import nha_wgrad
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    x, dy = (torch.randn(T, n, generator=gen, device="cuda").bfloat16() for n in (264, 272))
+    x[-1] = x[-1].abs() + 1
+    dy[-1, 7] = float("inf")
+    dw, = nha_wgrad(x, [dy])
+    assert (dw[7] == float("inf")).all()
+    rest = [i for i in range(272) if i != 7]
+    ref = (dy.double().t() @ x.double())[rest]
+    assert ((dw[rest].double() - ref).norm() / ref.norm()).item() <= 4e-3
+
+
 def test_wgrad_row_stride():
     from nha_amd.ops import nha_wgrad
     gen = torch.Generator(device="cuda").manual_seed(9)
