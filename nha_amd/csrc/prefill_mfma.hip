@@ -66,8 +66,8 @@ __device__ __forceinline__ void tile_r2l(lbf16* lds, const TileRegs<ROWS, D, NTH
 // decay accumulated since the segment start; per segment, the local end state and total decay.
 // Level 2 carries the true state across segments element-wise, h_seg[s+1] = h_seg[s] * dtot[s] + hend[s],
 // in one of two forms.  The forward turns every chunk-start state into the true one, h_loc + h_seg * dcum,
-// rounded to bf16 in place, so that the output pass reads plain operand tiles (state_final_kernel inside the
-// scan, or state_scan_kernel followed by state_apply_kernel).  The backward (state_scan_kernel) keeps the
+// rounded to bf16 in place, so that the output pass reads plain operand tiles (state_link_kernel, or
+// state_scan_kernel followed by state_apply_kernel).  The backward (state_scan_kernel) keeps the
 // segment-local states and writes the segment-start states h_seg beside them: it needs the sum in fp32.
 // Both states are kept as C[d][m] accumulators (slot m = lane % 16).
 
@@ -294,12 +294,13 @@ __global__ __launch_bounds__(256) void mfma_state_local_kernel(const MP p) {
 // being combined: a thread waits for memory once per group, not once per segment.
 // grid (N*H, 2*MS*D/1024): the first MS*D/4 groups are the k-state ([m][d]), the rest the v-state.
 constexpr int SCAN_AHEAD = 4;
+constexpr int LINK_SEGS = 16;   // average segments of a sequence up to which the forward takes state_link_kernel instead
 
 // What a workgroup of level 2 owns: 16 slots x 64 columns of one state, a slot and four consecutive columns per thread (256
 // consecutive bytes of a row of the scratch's [m][d] states per 16 threads).  The caller's k-states lie [d][m]: they pass through
 // LDS, 16 slots (64 bytes) of a row side by side.  With a thread's own four columns read and written there one by one, level 2 of a call
 // with initial and final states was bound by that (16 packed sequences, 4 heads of 256, 32768 tokens:
-// state_scan_kernel 31 -> 23 us, state_final_kernel 43 -> 38).
+// state_scan_kernel 31 -> 23 us).
 template <int D>
 struct StatePart {
   static constexpr int GROUPS = MS * D / 1024;   // workgroups per state
@@ -404,106 +405,123 @@ __global__ __launch_bounds__(256) void state_scan_kernel(const MP p) {
 // quickly (log-gates of about -1 per token: e^-80 per chunk) leave only the first chunk of a segment to rewrite;
 // with slow gates (the layers' logsigmoid / 8: e^-5 per chunk) every chunk is rewritten.
 //
-// Two forms.  state_final_kernel does it inside the scan (no h_seg round trip through memory; a thread's chain
-// costs about a memory latency per segment): for sequences of a few segments.  state_apply_kernel runs after
-// state_scan_kernel, one thread per (segment, slot, four d) with no chain: for long sequences.
+// Two forms.  state_link_kernel forms the state that enters a segment itself, from the end states of the segments before it: for
+// sequences of up to LINK_SEGS segments.  state_apply_kernel runs after state_scan_kernel, which hands that state on through memory.
 constexpr float CARRY_FLOOR = 0x1p-100f;
 
-// Four consecutive d of one slot per thread, sequential over the segments of its sequence; the small loads of
-// segment sg + 2 (decays, end state) and the local states of segment sg + 1 that need rewriting are requested
-// before segment sg is combined.
-// grid (N*H, 2*MS*D/1024): the first MS*D/4 groups are the k-state ([m][d]), the rest the v-state.
-template <int D>
-__global__ __launch_bounds__(256) void state_final_kernel(const MP p) {
-  __shared__ float trs[64 * 17];
-  lfloat* const tr = (lfloat*)trs;
-  const int H = p.H;
-  const int n = blockIdx.x / H, h = blockIdx.x % H;
-  const StatePart<D> part(blockIdx.y, threadIdx.x);
-  const bool isv = part.isv;
-  const int m = part.m, d = part.d;
-  const int bos = p.cu[n], eos = p.cu[n + 1];
-  const int nchunks = (eos - bos + BT - 1) / BT;
-  const int nseg = (nchunks + (1 << p.seg_sh) - 1) >> p.seg_sh;
-  const int64_t nh = (int64_t)n * H + h;
-  float hcur[4] = {0.f, 0.f, 0.f, 0.f};
-  if (p.h0k) {
-    const float4 x = isv ? *reinterpret_cast<const float4*>(p.h0v + (nh * MS + m) * D + d) : part.load_k(p.h0k + nh * D * MS, tr, threadIdx.x);
-    hcur[0] = x.x; hcur[1] = x.y; hcur[2] = x.z; hcur[3] = x.w;
+// What a thread of either form does: four consecutive d of a slot in every chunk of a segment
+struct Rewrite {
+  uint2 loc[SEG];
+  float dc[SEG];
+  unsigned need;
+  __device__ __forceinline__ void request_decays(const float* dcum, int64_t step, int nloc) {
+#pragma unroll
+    for (int jc = 0; jc < SEG; ++jc) dc[jc] = jc < nloc ? dcum[(int64_t)jc * step] : 0.f;
   }
-  const float* hend = isv ? p.hend_v : p.hend_k;
-  bf16_t* hloc = isv ? p.hvc : p.hkT;
-  const int chunk0 = p.coff[n];
-  const int slot0 = (chunk0 >> p.seg_sh) + n;
-  struct Small {      // what the chain itself needs of a segment
-    float dc[SEG];
-    float dt;
-    float4 he;
-  };
-  struct Loc {        // local chunk-start states of a segment (those that are rewritten)
-    uint2 v[SEG];
-    unsigned need;
-  };
-  auto request_small = [&](Small& r, int sg) {
-    const int64_t sl = (int64_t)(slot0 + sg) * H + h;
+  // hloc: the thread's place in the first chunk, step elements before that of the next
+  __device__ __forceinline__ void request(const bf16_t* hloc, int64_t step, float amax) {
+    need = 0;
 #pragma unroll
     for (int jc = 0; jc < SEG; ++jc) {
-      r.dc[jc] = 0.f;
-      if (jc < (1 << p.seg_sh) && (sg << p.seg_sh) + jc < nchunks) r.dc[jc] = p.dcum[((int64_t)(chunk0 + (sg << p.seg_sh) + jc) * H + h) * MS + m];
-    }
-    r.dt = p.dtot[sl * MS + m];
-    r.he = *reinterpret_cast<const float4*>(hend + (sl * MS + m) * D + d);
-  };
-  // hs: the state that enters segment sg
-  auto request_loc = [&](Loc& r, const Small& sm, int sg, const float (&hs)[4]) {
-    const float amax = fmaxf(fmaxf(fabsf(hs[0]), fabsf(hs[1])), fmaxf(fabsf(hs[2]), fabsf(hs[3])));
-    r.need = 0;
-#pragma unroll
-    for (int jc = 0; jc < SEG; ++jc) {
-      r.v[jc] = make_uint2(0, 0);
-      if (jc < (1 << p.seg_sh) && (sg << p.seg_sh) + jc < nchunks && amax * sm.dc[jc] >= CARRY_FLOOR) {
-        r.need |= 1u << jc;
-        r.v[jc] = *reinterpret_cast<const uint2*>(hloc + (((int64_t)(chunk0 + (sg << p.seg_sh) + jc) * H + h) * MS + m) * D + d);
+      loc[jc] = make_uint2(0, 0);
+      if (amax * dc[jc] >= CARRY_FLOOR) {
+        need |= 1u << jc;
+        loc[jc] = *reinterpret_cast<const uint2*>(hloc + jc * step);
       }
     }
-  };
-  Small s_cur, s_nxt, s_nn;
-  Loc l_cur, l_nxt;
-  request_small(s_cur, 0);
-  if (nseg > 1) request_small(s_nxt, 1);
-  request_loc(l_cur, s_cur, 0, hcur);
-  for (int sg = 0; sg < nseg; ++sg) {
-    float hn[4];
-    hn[0] = hcur[0] * s_cur.dt + s_cur.he.x;
-    hn[1] = hcur[1] * s_cur.dt + s_cur.he.y;
-    hn[2] = hcur[2] * s_cur.dt + s_cur.he.z;
-    hn[3] = hcur[3] * s_cur.dt + s_cur.he.w;
-    if (sg + 2 < nseg) request_small(s_nn, sg + 2);
-    if (sg + 1 < nseg) request_loc(l_nxt, s_nxt, sg + 1, hn);
+  }
+  __device__ __forceinline__ void store(bf16_t* hloc, int64_t step, const float (&hs)[4]) const {
 #pragma unroll
     for (int jc = 0; jc < SEG; ++jc) {
-      if (l_cur.need & (1u << jc)) {
-        const int64_t cg = (int64_t)(chunk0 + (sg << p.seg_sh) + jc) * H + h;
-        const uint32_t w[2] = {l_cur.v[jc].x, l_cur.v[jc].y};
+      if (need & (1u << jc)) {
+        const uint32_t w[2] = {loc[jc].x, loc[jc].y};
         bf16x4 o4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float a0 = __uint_as_float((i & 1) ? (w[i >> 1] & 0xffff0000u) : (w[i >> 1] << 16));
-          o4[i] = (__bf16)(a0 + hcur[i] * s_cur.dc[jc]);
+          o4[i] = (__bf16)(a0 + hs[i] * dc[jc]);
         }
-        *reinterpret_cast<bf16x4*>(hloc + (cg * MS + m) * D + d) = o4;
+        *reinterpret_cast<bf16x4*>(hloc + jc * step) = o4;
       }
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) hcur[i] = hn[i];
-    s_cur = s_nxt;
-    s_nxt = s_nn;
-    l_cur = l_nxt;
   }
-  if (p.hkt) {
-    const float4 x = make_float4(hcur[0], hcur[1], hcur[2], hcur[3]);
+};
+
+// (sequence, first chunk) of a segment slot (seg_slot)
+__device__ __forceinline__ void segment_of(const MP& p, int slot, int& n, int& it0) {
+  int lo = 0, hi = p.N - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if ((p.coff[mid] >> p.seg_sh) + mid <= slot) lo = mid; else hi = mid - 1;
+  }
+  n = lo;
+  it0 = (slot - ((p.coff[n] >> p.seg_sh) + n)) << p.seg_sh;
+}
+
+// One launch instead of scan and rewrite: four consecutive d of one slot per thread, every segment at once.  The state that enters a
+// segment is the sum of the end states before it, each times the decays between, the nearest first; the walk ends where the decay of
+// the whole wave has gone to zero (gates of the layers, logsigmoid / 8: three segments).  Bound: the rewritten states' bytes.
+// Before, up to eight segments: four elements of a state per thread, which walked the segments of their sequence and rewrote their
+// chunks on the way, a memory latency each; beyond, scan and rewrite.  16 packed sequences, 32768 tokens, 4 heads of 256, with states
+// 43 -> 28 us; 2 x 8192 tokens, 8 heads of 128 (16 segments each) 30.5 -> 24.5; 331 tokens, 4 heads of 128 7.3 -> 4.
+// Gates that never decay read every end state before their own: as fast as the scan at 16 segments (2 x 8192 tokens, W = 64: call
+// 246 -> 244 us), slower at 32 (476 -> 482; gates of the layers 478 -> 467) and at 64 (481 -> 505), so longer sequences keep the scan.
+// One-dimensional grid (segment slots, H, StatePart's groups), the groups fastest: there are 8, 16 or 32 of them, so the segments that
+// read the same part of an end state are on one XCD.
+template <int D>
+__global__ __launch_bounds__(256) void state_link_kernel(const MP p) {
+  __shared__ float trs[64 * 17];
+  lfloat* const tr = (lfloat*)trs;
+  constexpr int G = 2 * StatePart<D>::GROUPS;
+  const int H = p.H, slot = blockIdx.x / (G * H), h = blockIdx.x / G % H, tid = threadIdx.x;
+  int n, it0;
+  segment_of(p, slot, n, it0);
+  const int nchunks = p.coff[n + 1] - p.coff[n];
+  if (it0 > 0 && it0 >= nchunks) return;   // (a sequence without tokens has a slot: its final state is the initial one)
+  const StatePart<D> part(blockIdx.x % G, tid);
+  const bool isv = part.isv;
+  const int m = part.m, d = part.d;
+  const int nloc = (nchunks - it0) < (1 << p.seg_sh) ? (nchunks - it0) : 1 << p.seg_sh;
+  const int64_t cg0 = (int64_t)(p.coff[n] + it0) * H + h, nh = (int64_t)n * H + h;
+  bf16_t* const hloc = (isv ? p.hvc : p.hkT) + (cg0 * MS + m) * D + d;
+  const float* const hend = (isv ? p.hend_v : p.hend_k) + (int64_t)h * MS * D + m * D + d;   // + slot H MS D
+  const float* const dtot = p.dtot + h * MS + m;                                              // + slot H MS
+  Rewrite rw;
+  rw.request_decays(p.dcum + cg0 * MS + m, (int64_t)H * MS, nloc);
+  const bool last = it0 + nloc == nchunks;
+  float4 own = make_float4(0.f, 0.f, 0.f, 0.f);
+  float own_dt = 1.f;
+  if (last && p.hkt && nloc > 0) {
+    own = *reinterpret_cast<const float4*>(hend + (int64_t)slot * H * MS * D);
+    own_dt = dtot[(int64_t)slot * H * MS];
+  }
+  float hs[4] = {0.f, 0.f, 0.f, 0.f}, dec = 1.f;
+  const int first = slot - (it0 >> p.seg_sh);
+  for (int j = slot - 1; j >= first && __any(dec != 0.f); j -= 2) {   // the loads of two segments together
+    const int j1 = j > first ? j - 1 : j;
+    const float4 a = *reinterpret_cast<const float4*>(hend + (int64_t)j * H * MS * D), b = *reinterpret_cast<const float4*>(hend + (int64_t)j1 * H * MS * D);
+    const float da = dtot[(int64_t)j * H * MS], db = dtot[(int64_t)j1 * H * MS];
+    if (dec != 0.f) {
+      hs[0] += a.x * dec; hs[1] += a.y * dec; hs[2] += a.z * dec; hs[3] += a.w * dec;
+    }
+    dec *= da;
+    if (j > first) {
+      if (dec != 0.f) {
+        hs[0] += b.x * dec; hs[1] += b.y * dec; hs[2] += b.z * dec; hs[3] += b.w * dec;
+      }
+      dec *= db;
+    }
+  }
+  if (p.h0k && __syncthreads_or(dec != 0.f)) {
+    const float4 x = isv ? *reinterpret_cast<const float4*>(p.h0v + (nh * MS + m) * D + d) : part.load_k(p.h0k + nh * D * MS, tr, tid);
+    hs[0] += x.x * dec; hs[1] += x.y * dec; hs[2] += x.z * dec; hs[3] += x.w * dec;
+  }
+  rw.request(hloc, (int64_t)H * MS * D, fmaxf(fmaxf(fabsf(hs[0]), fabsf(hs[1])), fmaxf(fabsf(hs[2]), fabsf(hs[3]))));
+  rw.store(hloc, (int64_t)H * MS * D, hs);
+  if (last && p.hkt) {
+    const float4 x = make_float4(hs[0] * own_dt + own.x, hs[1] * own_dt + own.y, hs[2] * own_dt + own.z, hs[3] * own_dt + own.w);
     if (isv) *reinterpret_cast<float4*>(p.hvt + (nh * MS + m) * D + d) = x;
-    else part.store_k(p.hkt + nh * D * MS, x, tr, threadIdx.x);
+    else part.store_k(p.hkt + nh * D * MS, x, tr, tid);
   }
 }
 
@@ -513,16 +531,8 @@ template <int D>
 __global__ __launch_bounds__(256) void state_apply_kernel(const MP p) {
   const int H = p.H;
   const int slot = blockIdx.x, h = blockIdx.y;
-  int n = 0;
-  {
-    int lo = 0, hi = p.N - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if ((p.coff[mid] >> p.seg_sh) + mid <= slot) lo = mid; else hi = mid - 1;
-    }
-    n = lo;
-  }
-  const int it0 = (slot - ((p.coff[n] >> p.seg_sh) + n)) << p.seg_sh;
+  int n, it0;
+  segment_of(p, slot, n, it0);
   const int nchunks = p.coff[n + 1] - p.coff[n];
   if (it0 >= nchunks) return;
   const int nloc = (nchunks - it0) < (1 << p.seg_sh) ? (nchunks - it0) : 1 << p.seg_sh;
@@ -531,38 +541,16 @@ __global__ __launch_bounds__(256) void state_apply_kernel(const MP p) {
   const int em = (isv ? e4 - MS * D / 4 : e4) * 4;
   const int m = em / D, d = em % D;
   const int64_t sl = (int64_t)slot * H + h;
-  const float4 hs = *reinterpret_cast<const float4*>((isv ? p.hseg_v : p.hseg_k) + (sl * MS + m) * D + d);
-  const float amax = fmaxf(fmaxf(fabsf(hs.x), fabsf(hs.y)), fmaxf(fabsf(hs.z), fabsf(hs.w)));
+  const float4 x = *reinterpret_cast<const float4*>((isv ? p.hseg_v : p.hseg_k) + (sl * MS + m) * D + d);
+  const float hs[4] = {x.x, x.y, x.z, x.w};
+  const float amax = fmaxf(fmaxf(fabsf(hs[0]), fabsf(hs[1])), fmaxf(fabsf(hs[2]), fabsf(hs[3])));
   if (!(amax >= CARRY_FLOOR)) return;      // nothing is carried into this segment (its first, without initial state)
-  bf16_t* hloc = isv ? p.hvc : p.hkT;
   const int64_t cg0 = (int64_t)(p.coff[n] + it0) * H + h;
-  float dc[SEG];
-#pragma unroll
-  for (int jc = 0; jc < SEG; ++jc) dc[jc] = jc < nloc ? p.dcum[(cg0 + (int64_t)jc * H) * MS + m] : 0.f;
-  uint2 loc[SEG];
-  unsigned need = 0;
-#pragma unroll
-  for (int jc = 0; jc < SEG; ++jc) {
-    loc[jc] = make_uint2(0, 0);
-    if (amax * dc[jc] >= CARRY_FLOOR) {
-      need |= 1u << jc;
-      loc[jc] = *reinterpret_cast<const uint2*>(hloc + ((cg0 + (int64_t)jc * H) * MS + m) * D + d);
-    }
-  }
-  const float hv4[4] = {hs.x, hs.y, hs.z, hs.w};
-#pragma unroll
-  for (int jc = 0; jc < SEG; ++jc) {
-    if (need & (1u << jc)) {
-      const uint32_t w[2] = {loc[jc].x, loc[jc].y};
-      bf16x4 o4;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float a0 = __uint_as_float((i & 1) ? (w[i >> 1] & 0xffff0000u) : (w[i >> 1] << 16));
-        o4[i] = (__bf16)(a0 + hv4[i] * dc[jc]);
-      }
-      *reinterpret_cast<bf16x4*>(hloc + ((cg0 + (int64_t)jc * H) * MS + m) * D + d) = o4;
-    }
-  }
+  bf16_t* const hloc = (isv ? p.hvc : p.hkT) + (cg0 * MS + m) * D + d;
+  Rewrite rw;
+  rw.request_decays(p.dcum + cg0 * MS + m, (int64_t)H * MS, nloc);
+  rw.request(hloc, (int64_t)H * MS * D, amax);
+  rw.store(hloc, (int64_t)H * MS * D, hs);
 }
 
 // ==========================================================================================
@@ -1212,12 +1200,9 @@ int run_state_pass(const MP& p, bool segment_form, hipStream_t st) {
   }
   hipLaunchKernelGGL((mfma_state_local_kernel<D, DW>), dim3((unsigned)l1_grid), dim3(256), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma state pass, level 1)");
-  // the forward's chunk states: inside the scan while a sequence has about eight segments or fewer (a thread's
-  // chain there costs a memory latency per segment: 15 us at 4 segments, 21 us at 16 on one box), after it beyond
-  // (two launches without a chain: 16-18 us whatever the length)
-  const bool in_scan = !segment_form && (int64_t)p.NT <= ((int64_t)8 * p.N << p.seg_sh);
-  if (in_scan) {
-    hipLaunchKernelGGL((state_final_kernel<D>), dim3(p.N * p.H, 2 * MS * D / 1024), dim3(256), 0, st, p);
+  const int64_t link_grid = (int64_t)nslot * p.H * (2 * MS * D / 1024);
+  if (!segment_form && (int64_t)p.NT <= ((int64_t)LINK_SEGS * p.N << p.seg_sh) && link_grid <= 0x7fffffff) {
+    hipLaunchKernelGGL((state_link_kernel<D>), dim3((unsigned)link_grid), dim3(256), 0, st, p);
   } else {
     hipLaunchKernelGGL((state_scan_kernel<D>), dim3(p.N * p.H, 2 * MS * D / 1024), dim3(256), 0, st, p);
     if (!segment_form) hipLaunchKernelGGL((state_apply_kernel<D>), dim3(nslot + 1, p.H, 2 * MS * D / 1024), dim3(256), 0, st, p);

@@ -184,8 +184,8 @@ def test_mfma_matches_simple_kernels_at_size():
 @pytest.mark.parametrize("B,T", [(1, 6144), (2, 3072)])
 @pytest.mark.parametrize("gate_div,gate_mean", [(8.0, 0.0), (1.0, -1.0)])
 def test_mfma_long_sequences_both_forms_of_the_state_carry(B, T, gate_div, gate_mean):
-    """Sequences of 12 and 6 segments: the first takes the scan-then-apply form of the state pass's second level, the
-    second the form inside the scan; with the layers' slow gates (logsigmoid / 8: the carried state reaches every chunk
+    """Sequences of 24 and 12 segments: the first takes the scan-then-apply form of the state pass's second level, the
+    second the form that links the segments itself; with the layers' slow gates (logsigmoid / 8: the carried state reaches every chunk
     of a segment) and with fast ones (everything past a segment's first chunks is left as it is).  Initial states, so
     that the first segment carries something too.  Against the fp32-math kernels."""
     from nha_amd import chunk_nha
