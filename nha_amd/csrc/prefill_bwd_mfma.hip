@@ -96,14 +96,14 @@ __device__ __forceinline__ float logaddexp_f(float a, float b) {
 }
 
 // rows [0, vhi) of a ROWS x D tile whose row r is global row grow0 + r of a [*, heads, D] tensor
-template <int ROWS, int D>
+template <int ROWS, int D, int THREADS = 256>
 struct Tile {
-  static constexpr int NPC = ROWS * D / 8 / 256;
+  static constexpr int NPC = ROWS * D / 8 / THREADS;
   uint4 r[NPC];
   __device__ __forceinline__ void load(const bf16_t* base, int64_t row_stride, int64_t grow0, int vhi, int tid) {
 #pragma unroll
     for (int u = 0; u < NPC; ++u) {
-      const int c = tid + 256 * u;
+      const int c = tid + THREADS * u;
       const int row = c / (D / 8), col = (c % (D / 8)) * 8;
       uint4 x = make_uint4(0, 0, 0, 0);
       if (row < vhi) x = *reinterpret_cast<const uint4*>(base + (grow0 + row) * row_stride + col);
@@ -113,7 +113,7 @@ struct Tile {
   __device__ __forceinline__ void store(lbf16* lds, int tid) const {
 #pragma unroll
     for (int u = 0; u < NPC; ++u) {
-      const int c = tid + 256 * u;
+      const int c = tid + THREADS * u;
       const int row = c / (D / 8), col = (c % (D / 8)) * 8;
       lds_st16(lds + row * (D + 16) + col, r[u]);
     }
@@ -241,16 +241,21 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(const WP p) {
 // dk_swa, dv: grid (H, NT), 4 waves x 16 keys.  MODE 0: both; 1: dk only; 2: dv only (D = 256: both accumulators do not
 // fit the register file, and the workgroups of one launch (SPLIT) take 1 or 2; as two launches a small call ran each on
 // half of the chip: 1700 tokens, 4 heads 50 -> 26 us; 8 x 2048 tokens 217 -> 201 us)
+// G = 2: eight waves, every tile's queries halved between two groups of four, whose sums are added at the end.  A step of
+// one wave per SIMD is a chain of LDS reads, products and exponentials (2.8 us for 64 x 64 scores at D = 128, whose products
+// take 0.4); where a call has no second workgroup for the CU the second group fills the gaps: 1.9 us, 2001 packed tokens, 32 / 8
+// heads, W = 571 114 -> 79 us.  Past that LDS itself bounds the step: each wave reads both tiles for its 16 keys.
 // ------------------------------------------------------------------------------------------
-template <int D, int TQ, int MODE>
+template <int D, int TQ, int MODE, int G>
 __device__ __forceinline__ void bwd_dkv_tile(const WP& p) {
-  constexpr int KS = D / 32, DB = D / 16, LDT = D + 16, NH = TQ / 32, TILE = TQ * LDT;
+  constexpr int KS = D / 32, DB = D / 16, LDT = D + 16, NH = TQ / 32 / G, TILE = TQ * LDT;
   constexpr bool DO_K = MODE != 2, DO_V = MODE != 1;
   extern __shared__ __align__(16) unsigned char smem[];
   lbf16* const tiles = (lbf16*)smem;                 // Q0, Q1, dO0, dO1
   lfloat* const lsb = (lfloat*)(tiles + 4 * TILE);   // [2][TQ] lse * log2(e)
   lfloat* const dlb = lsb + 2 * TQ;                  // [2][TQ] delta
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) & 3;
+  const int hf0 = G == 1 ? 0 : NH * (tid >> 8);   // first block of 32 queries of this group of waves
   const int l16 = lane & 15, kb = lane >> 4;
   const int H = p.H, HQ = p.HQ, NG = p.NG;
   int h, chunk;
@@ -285,7 +290,7 @@ __device__ __forceinline__ void bwd_dkv_tile(const WP& p) {
   if (p.wl >= 0 && j0 + 64 + p.wl < eos) qend = j0 + 64 + p.wl;
   const int nqt = (qend - j0 + TQ - 1) / TQ;
   const int niter = nqt * NG;
-  Tile<TQ, D> rq, ro;
+  Tile<TQ, D, 256 * G> rq, ro;
   float rls = 0.f, rlg = 0.f, rd = 0.f;
   // iteration i = (q-head of the group, query tile), tiles innermost: the workgroup of the next
   // chunk (same XCD, started together) reads the same tile one iteration earlier, so the tile is
@@ -330,7 +335,8 @@ __device__ __forceinline__ void bwd_dkv_tile(const WP& p) {
     const int ybase = TQ * (i % nqt);   // first query of the tile, relative to j0
     const bool edge = (ybase < 63) || (p.wl >= 0 && ybase + TQ - 1 > p.wl) || (j0 + ybase + TQ > eos);
 #pragma unroll
-    for (int hf = 0; hf < NH; ++hf) {
+    for (int hh = 0; hh < NH; ++hh) {
+      const int hf = hf0 + hh;
       f32x4 S[2], dP[2];
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
@@ -388,17 +394,35 @@ __device__ __forceinline__ void bwd_dkv_tile(const WP& p) {
     }
     lds_barrier();
   }
+  if constexpr (G == 2) {
+    // The two groups of waves have each summed one half of every tile's queries: the second hands over dK, the first dV (with
+    // one of the two here, the second hands that over), a lane's sums at its own place in the tiles' memory.
+    NHA_LDS f32x4* const xk = (NHA_LDS f32x4*)smem + (wave * DB) * 64 + lane;
+    NHA_LDS f32x4* const xv = xk + (MODE == 0 ? 4 * DB * 64 : 0);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      if (DO_K && hf0) xk[db * 64] = dK[db];
+      if (DO_V && (MODE == 2 ? hf0 != 0 : hf0 == 0)) xv[db * 64] = dV[db];
+    }
+    lds_barrier();
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      if (DO_K && !hf0) dK[db] += xk[db * 64];
+      if (DO_V && (MODE == 2 ? hf0 == 0 : hf0 != 0)) dV[db] += xv[db * 64];
+    }
+  }
+  const bool out_k = G == 1 || hf0 == 0, out_v = G == 1 || (MODE == 2 ? hf0 == 0 : hf0 != 0);
   if (valid) {
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
       const int64_t off = jk * D + 16 * db + 4 * kb;
       bf16x4 pk;
-      if (DO_K) {
+      if (DO_K && out_k) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) pk[r] = (__bf16)dK[db][r];
         *reinterpret_cast<bf16x4*>(p.dk + off) = pk;
       }
-      if (DO_V) {
+      if (DO_V && out_v) {
         const float4 sv = *reinterpret_cast<const float4*>(p.dvs + off);
         pk[0] = (__bf16)(dV[db][0] + sv.x);
         pk[1] = (__bf16)(dV[db][1] + sv.y);
@@ -410,13 +434,13 @@ __device__ __forceinline__ void bwd_dkv_tile(const WP& p) {
   }
 }
 
-template <int D, int TQ, bool SPLIT>
-__global__ __launch_bounds__(256) void bwd_dkv_kernel(const WP p) {
+template <int D, int TQ, bool SPLIT, int G>
+__global__ __launch_bounds__(256 * G) void bwd_dkv_kernel(const WP p) {
   if constexpr (SPLIT) {
-    if (blockIdx.z == 0) bwd_dkv_tile<D, TQ, 1>(p);
-    else bwd_dkv_tile<D, TQ, 2>(p);
+    if (blockIdx.z == 0) bwd_dkv_tile<D, TQ, 1, G>(p);
+    else bwd_dkv_tile<D, TQ, 2, G>(p);
   } else {
-    bwd_dkv_tile<D, TQ, 0>(p);
+    bwd_dkv_tile<D, TQ, 0, G>(p);
   }
 }
 
@@ -697,19 +721,19 @@ int launch_dq(const WP& p, int NT, hipStream_t st) {
   return NHA_OK;
 }
 
-template <int D, int TQ, bool SPLIT>
+template <int D, int TQ, bool SPLIT, int G>
 int launch_dkv(const WP& p, int NT, hipStream_t st) {
   const size_t lds = (size_t)4 * TQ * (D + 16) * 2 + 4 * TQ * 4;
   static std::atomic<bool> configured{false};   // the attribute call is idempotent: a second thread may repeat it
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void*)bwd_dkv_kernel<D, TQ, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = hipFuncSetAttribute((const void*)bwd_dkv_kernel<D, TQ, SPLIT, G>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) {
       set_error("nha_prefill_bwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
       return NHA_ERR_LAUNCH;
     }
     configured = true;
   }
-  hipLaunchKernelGGL((bwd_dkv_kernel<D, TQ, SPLIT>), dim3(p.H, NT, SPLIT ? 2 : 1), dim3(256), lds, st, p);
+  hipLaunchKernelGGL((bwd_dkv_kernel<D, TQ, SPLIT, G>), dim3(p.H, NT, SPLIT ? 2 : 1), dim3(256 * G), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(window dk, dv)");
   return NHA_OK;
 }
@@ -749,9 +773,14 @@ int bwd_window_mfma_dkv(const NhaPrefillBwdArgs* a, const float* delta, const fl
   if (bwd_ring256_dkv_supported(a)) return bwd_ring256_dkv(a, (const float2*)ld, dvs);
   const WP p = make_wp(a, delta, dvs);
   hipStream_t st = (hipStream_t)a->stream;
-  if (a->K == 64) return launch_dkv<64, 64, false>(p, a->NT, st);
-  if (a->K == 128) return launch_dkv<128, 64, false>(p, a->NT, st);
-  return launch_dkv<256, 32, true>(p, a->NT, st);
+  // Eight waves per workgroup where all of them have a place at once: one workgroup per CU, at head size 64 two.  us, four / eight
+  // waves: head size 64, 16 / 4 heads, W = 174, 63 to 624 workgroups 41 / 27, 49 / 39 (312), 61 / 61 (624), 16 / 16, W = 128, 15.7 /
+  // 14.3 (480), 19 / 22 (752); 128, 8 / 2, W = 169 54 / 39 (240), 32 / 8, W = 571 114 / 79 (256), 4 / 4, W = 512 43 / 48 (512); 256, 8
+  // / 2 48 / 38 (152), 86 / 98 (304).
+  const bool two = (int64_t)a->H * a->NT * (a->K == 256 ? 2 : 1) <= (a->K == 64 ? 512 : 256);
+  if (a->K == 64) return two ? launch_dkv<64, 64, false, 2>(p, a->NT, st) : launch_dkv<64, 64, false, 1>(p, a->NT, st);
+  if (a->K == 128) return two ? launch_dkv<128, 64, false, 2>(p, a->NT, st) : launch_dkv<128, 64, false, 1>(p, a->NT, st);
+  return two ? launch_dkv<256, 64, true, 2>(p, a->NT, st) : launch_dkv<256, 32, true, 1>(p, a->NT, st);
 }
 
 template <int D>

@@ -663,7 +663,7 @@ static bool short_groups(const NhaPrefillBwdArgs* a) { return a->wl >= 0 && a->w
 
 // A workgroup of ring_dkv_kernel walks all queries that see its key group, four heads of them, whatever the size of the
 // call.  Where its groups would fill half of the chip or less, bwd_dkv_kernel's groups of 64 keys are up to four times as
-// many and each walks fewer queries: 1700 tokens, 32 / 8 heads, W = 256 (56 groups) 114 -> 62 us; 4000 tokens, W = 1000
+// many and each walks fewer queries (measured with four waves each): 1700 tokens, 32 / 8 heads, W = 256 (56 groups) 114 -> 62 us; 4000 tokens, W = 1000
 // (128) 308 -> 236; 3000 tokens, 32 / 4 heads, W = 512 (48) 333 -> 188.  Beyond, the groups of 64 pass one round of
 // places (two per CU) and pull every q / do row four times as often: 5000 tokens, 32 / 8 heads, W = 512 (160) 187 against
 // 217 us; 4000 tokens, W = 128 (256) 51 against 57.

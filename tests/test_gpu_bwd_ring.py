@@ -45,6 +45,15 @@ def test_window_gradients_of_many_key_groups(wl, H, NG, D, cu):
     compare(cu, wl, H, NG, D, ("q_swa", "k_swa", "v"))
 
 
+@pytest.mark.parametrize("H,NG,D", [(24, 2, 64), (25, 2, 64), (12, 3, 128), (13, 3, 128), (5, 1, 128), (6, 2, 256), (7, 2, 256)])
+@pytest.mark.parametrize("wl", [-1, 0, 64, 159])
+def test_window_gradients_of_few_key_groups(wl, H, NG, D):
+    """dk and dv of 64 keys by four or by eight waves: the last sizes of the one and the first of the other (21 groups of keys per
+    kv-head), tiles of 64 queries whose second half is empty, and ends inside either half."""
+    print("case", wl, H, NG, D, flush=True)
+    compare(CU, wl, H, NG, D, ("k_swa", "v"))
+
+
 @pytest.mark.parametrize("wl", [40, 400])
 def test_more_sequences_than_lanes(wl):
     """150 ragged sequences of up to 130 tokens, empty ones among them: the forward's workgroups of two chunks search among them, the
