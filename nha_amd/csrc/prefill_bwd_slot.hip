@@ -178,6 +178,16 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
   const bool vs = wave >= 4;
   const int H = p.H, HQ = p.HQ, NG = p.NG;
+  // Several heads, two rounds of workgroups or more: the 32 CUs of an XCD start 0.2 us after one another (the second round follows from
+  // the first).  All in step, their products come at the same moments, and some cards then run every matrix kernel of the following
+  // milliseconds 5 % slower, at the same clock: steps of 2 x 8192 tokens, 32 / 8 heads of 128, W = 2048 one after another 2950 -> 2740
+  // us, W = 512 1686 -> 1565, 5000 tokens 666 -> 640 (0.1 us 641, 2820 and 1615; 0.4 us 2735 and 1563); on a card that does not, the
+  // same times within 0.2 %.  One round: 2001 tokens 273 -> 280 us, not staggered.
+  if (!ONE && !EXACT && gridDim.x * gridDim.y >= 512) {
+    const unsigned L = blockIdx.y * gridDim.x + blockIdx.x;
+    if (L < 256)
+      for (unsigned i = 0; i < L >> 3; ++i) __builtin_amdgcn_s_sleep(8);
+  }
   int h, chunk;
   xcd_tile(D / DW, p.NT, h, chunk);
   const int x0 = (h % (D / DW)) * DW;
