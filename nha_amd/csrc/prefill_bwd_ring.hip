@@ -311,15 +311,30 @@ struct DkvP {
 
 // an item: q tile | do tile | 32 (lse, delta) pairs
 constexpr int KV_Q = 0, KV_O = UB, KV_LD = 2 * UB, KV_ITEM = 2 * UB + 256;
-template <int KEYS> constexpr int KV_BYTES = NR * KV_ITEM + KEYS * D * 2;   // ring, then the V rows of the workgroup's keys
+template <int G> constexpr int KV_NR = G == 2 ? 7 : 4;   // items in LDS
+template <int KEYS, int G> constexpr int KV_BYTES = KV_NR<G> * KV_ITEM + KEYS * D * 2;   // ring, then the V rows of the workgroup's keys
 
-// KEYS: keys per workgroup, 256 or 128 (a wave holds KEYS / 8 of them).  With 256 every q / do fragment read from LDS
-// feeds two matrix products, with 128 one: long windows, which are bound by those reads, take 256 (headline shape:
-// 1.17 ms against 1.5 ms); windows up to 160 keys, where a workgroup's walk is a few items long and the half-size
-// key groups spread more evenly over the CUs, take 128 (window 64: whole backward 1.63 against 1.70 ms).
-template <int KEYS>
+// KEYS: keys per workgroup, 256 or 128, G: the waves in G groups, each with all keys and every G-th item, whose sums are added at the end.
+// A wave with 32 keys feeds two matrix products with every q / do fragment it reads from LDS, one with 16 keys (128, G = 1) only one:
+// long windows are bound by those reads (B=2, T=8192, 32/8 heads, W=2048: 256 keys 1.17 ms, 128 1.5, 128 in two groups 1.26).  Windows up
+// to 160 keys, where a workgroup's walk is a few items long, take 128 keys and one group (W=64 145 us, two groups 169); two groups are
+// for calls whose groups of 256 keys leave CUs without work (key_groups): 4000 tokens, W=1000 263 -> 172 us, 233 with bwd_dkv_kernel.
+// waits until at most `younger` items' requests of this wave are in flight
+template <int LPW, int G>
+__device__ __forceinline__ void wait_items(int younger) {
+  if (G == 2 && younger >= 5) wait_vm<5 * LPW>();
+  else if (G == 2 && younger == 4) wait_vm<4 * LPW>();
+  else if (G == 2 && younger == 3) wait_vm<3 * LPW>();
+  else if (younger >= 2) wait_vm<2 * LPW>();
+  else if (younger == 1) wait_vm<LPW>();
+  else wait_vm<0>();
+}
+
+template <int KEYS, int G>
 __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
-  constexpr int NKB = KEYS / 16 / 8;       // 16-key blocks per wave
+  constexpr int KW = 8 / G;                // waves that hold the keys, each of G groups all of them
+  constexpr int NKB = KEYS / 16 / KW;      // 16-key blocks per wave
+  constexpr int NR = KV_NR<G>;
   constexpr int CPG = KEYS / 64;           // chunks per key group
   constexpr int UPG = KEYS / 32;           // 32-query units that a key group spans
   constexpr int KV_LPW = 2;                // tile loads per wave and item (16 blocks of 1 KB, 8 waves)
@@ -328,6 +343,7 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
   const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, kb = lane >> 4;
+  const int kw = wave % KW, grp = wave / KW;
   const int H = p.H, HQ = p.HQ, NG = p.NG;
   // grid = (kv-head, chunk): the workgroup of every CPG-th chunk of a sequence (every fourth, at 256 keys) takes that
   // chunk and the next CPG - 1; the others leave at once.  Workgroups are handed to the shader engines in turn, in
@@ -427,18 +443,19 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
   };
   // This lane's keys (one per 16-key block of the wave) and their K / V rows (B operands: K[key][32 ks + 8 kb ..]).  The V rows
   // lie in LDS, in the order in which their wave reads them; K and V both in registers would leave none to read ahead with.
-  const int kbase = 16 * NKB * wave;               // first key of the wave, relative to c0
-  const uint32_t vrows = (uint32_t)(NR * KV_ITEM + wave * (NKB * KS * 1024));
+  const int kbase = 16 * NKB * kw;               // first key of the wave, relative to c0
+  const uint32_t vrows = (uint32_t)(NR * KV_ITEM + kw * (NKB * KS * 1024));
 #pragma unroll
-  for (int kk = 0; kk < NKB; ++kk) {
+  for (int k2 = 0; k2 < NKB / G; ++k2) {
+    const int kk = G == 1 ? k2 : grp;
     const int tk = c0 + kbase + 16 * kk + l16;
     const uint32_t row = (uint32_t)((tk < eos ? tk : eos - 1) - bos) * (uint32_t)(H * D);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       g2l16(p.v + ((int64_t)bos * H + h) * D, (row + 32 * ks + 8 * kb) * 2, lds0 + vrows + (kk * KS + ks) * 1024);
   }
-  int issued = 0;
-  for (; issued < NR - 1 && issued < total; ++issued) issue_next(issued);
+  int issued = 0, islot = 0, cslot = 0;   // items requested; slots of the next request and of item k below
+  for (; issued < NR - 1 && issued < total; ++issued) issue_next(islot++);
 
   bf16x8 kfr[NKB][KS];
 #pragma unroll
@@ -483,46 +500,66 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
   auto no_work = [&](int u) { return (32 * u + 31 < kbase) || (p.wl >= 0 && 32 * u > kbase + 16 * NKB - 1 + p.wl); };
   Walk cw = {0, rot0, 0};
   for (int k = 0; k < total;) {
-    // a step is a unit and its complement, of which a wave takes the one it has work in, or up to two units in a row
+    // G = 1: a step is a unit and its complement, of which a wave takes the one it has work in, or up to two units in a row.
+    // G = 2: each group of waves has a unit of its own, alone or with its complement.
     const int prim = cw.u;
     const bool pair = prim < npair;
     advance(cw);
     int need = pair ? 2 : 1, next = -1;   // items of this step: k .. k + need - 1
-    if (!pair && k + 1 < total && cw.u >= npair) {
-      next = cw.u;
-      need = 2;
-      advance(cw);
+    int u = prim, slot = G == 1 ? k : cslot;
+    bool idle = false;
+    if constexpr (G == 1) {
+      if (!pair && k + 1 < total && cw.u >= npair) {
+        next = cw.u;
+        need = 2;
+        advance(cw);
+      }
+    } else {
+      const int n2 = k + need < total ? (cw.u < npair ? 2 : 1) : 0;
+      const bool both = n2 && k + need + n2 <= issued;   // else the second group sits this step out
+      if (grp) {
+        idle = !both;
+        u = cw.u;
+        slot += need;
+      }
+      if (both) {
+        need += n2;
+        advance(cw);
+      }
     }
     // they have landed (this wave's part; wave 0 carries one more load per item), then everybody's; the
     // requests after them stay in flight
     const int younger = issued - (k + need);
-    if (younger >= 2) {
-      if (wave == 0) wait_vm<2 * (KV_LPW + 1)>();
-      else wait_vm<2 * KV_LPW>();
-    } else if (younger == 1) {
-      if (wave == 0) wait_vm<KV_LPW + 1>();
-      else wait_vm<KV_LPW>();
-    } else {
-      wait_vm<0>();
-    }
+    if (wave == 0) wait_items<KV_LPW + 1, G>(younger);
+    else wait_items<KV_LPW, G>(younger);
     lds_barrier();
     // every wave is past the items before k: their slots take the next requests
-    for (; issued < total && issued < k + NR; ++issued) issue_next(issued & (NR - 1));
-    int u = prim, slot = k;
-    if (pair && no_work(prim)) {
-      u = prim + K0;
-      slot = k + 1;
+    for (; issued < total && issued < k + NR; ++issued) {
+      if constexpr (G == 1) {
+        issue_next(issued & (NR - 1));
+      } else {
+        issue_next(islot);
+        islot = islot + 1 < NR ? islot + 1 : 0;
+      }
+    }
+    if (u < npair && no_work(u)) {
+      u += K0;
+      ++slot;
     }
     k += need;
+    if constexpr (G == 2) {
+      slot = slot < NR ? slot : slot - NR;
+      cslot = cslot + need < NR ? cslot + need : cslot + need - NR;
+    }
     do {
-      const uint32_t base = (uint32_t)((slot & (NR - 1)) * KV_ITEM);
+      const uint32_t base = (uint32_t)((G == 1 ? slot & (NR - 1) : slot) * KV_ITEM);
       int lc = threadIdx.x & 63;
       asm volatile("" : "+v"(lc));
       const int l16 = lc & 15, kb = lc >> 4;
       kaddr = (uint32_t)((kb >> 1) * 512 + l16 * 32 + (kb & 1) * 16);
       vaddr = (uint32_t)((4 * kb + (l16 >> 2)) * 32 + 8 * (l16 & 3));
       faddr = vrows + (uint32_t)(lc * 16);
-      if (!no_work(u)) {
+      if (!idle && !no_work(u)) {
         const bool edge = (32 * u < kbase + 16 * NKB - 1) || (p.wl >= 0 && 32 * u + 31 > kbase + p.wl) || (c0 + 32 * u + 32 > eos);
         // One stream of products: S = Q K^T, dP = dO V^T beside the exponentials of S, dV^T[d][key] += dO^T[d][q] P[q][key]
         // beside dS, dK^T[d][key] += Q^T[d][q] dS[q][key]; what a step multiplies was requested from LDS a step (1 KB row
@@ -619,6 +656,25 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
       ++slot;
     } while (u >= 0);
   }
+  // two groups: the second hands over dK, the first dV, a lane's sums at its own place in the memory of ring and V rows
+  if (G == 2) {
+    lds_barrier();
+    NHA_LDS f32x4* const xk = (NHA_LDS f32x4*)lds + kw * (DB * NKB * 64) + lane;
+    NHA_LDS f32x4* const xv = xk + KW * (DB * NKB * 64);
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int kk = 0; kk < NKB; ++kk)
+        if (grp) xk[(db * NKB + kk) * 64] = dK[db][kk];
+        else xv[(db * NKB + kk) * 64] = dV[db][kk];
+    lds_barrier();
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int kk = 0; kk < NKB; ++kk)
+        if (grp) dV[db][kk] += xv[(db * NKB + kk) * 64];
+        else dK[db][kk] += xk[(db * NKB + kk) * 64];
+  }
 #pragma unroll
   for (int kk = 0; kk < NKB; ++kk) {
     const int tk = c0 + kbase + 16 * kk + l16;
@@ -627,12 +683,12 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
     for (int db = 0; db < DB; ++db) {
       const int64_t off = ((int64_t)tk * H + h) * D + 16 * db + 4 * kb;
       bf16x4 pk;
-      {
+      if (G == 1 || !grp) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) pk[r] = (__bf16)(dK[db][kk][r] * p.scale);
         *reinterpret_cast<bf16x4*>(p.dk + off) = pk;
       }
-      {
+      if (G == 1 || grp) {
         const float4 sv = *reinterpret_cast<const float4*>(p.dvs + off);
         pk[0] = (__bf16)(dV[db][kk][0] + sv.x);
         pk[1] = (__bf16)(dV[db][kk][1] + sv.y);
@@ -658,20 +714,28 @@ bool bwd_ring_supported(const NhaPrefillBwdArgs* a) {
   return (int64_t)a->T_tot * a->HQ * 128 * 2 < ((int64_t)1 << 32);
 }
 
-// key groups of 128 instead of 256: windows of less than 160 keys
-static bool short_groups(const NhaPrefillBwdArgs* a) { return a->wl >= 0 && a->wl < 160; }
+static bool short_window(const NhaPrefillBwdArgs* a) { return a->wl >= 0 && a->wl < 160; }
 
-// A workgroup of ring_dkv_kernel walks all queries that see its key group, four heads of them, whatever the size of the
-// call.  Where its groups would fill half of the chip or less, bwd_dkv_kernel's groups of 64 keys are up to four times as
-// many and each walks fewer queries (measured with four waves each): 1700 tokens, 32 / 8 heads, W = 256 (56 groups) 114 -> 62 us; 4000 tokens, W = 1000
-// (128) 308 -> 236; 3000 tokens, 32 / 4 heads, W = 512 (48) 333 -> 188.  Beyond, the groups of 64 pass one round of
-// places (two per CU) and pull every q / do row four times as often: 5000 tokens, 32 / 8 heads, W = 512 (160) 187 against
-// 217 us; 4000 tokens, W = 128 (256) 51 against 57.
+// Keys per workgroup of the dk / dv kernel here, 0 where bwd_dkv_kernel takes the call.  Windows of less than 160 keys: 128.  Others: a
+// workgroup of 128 keys takes 0.6 of the time of one of 256, so the fewer rounds of the 256 CUs decide.  us, 256 / 128 keys, 32 / 8
+// heads: 5000 tokens, W = 512 (160 groups of 256 keys) 161 / 188, 2 x 5000 (320) W = 160 202 / 162, W = 300 241 / 220, W = 1000 467
+// / 454, 3 x 4000 (384) W = 1000 520 / 483, 2 x 8192 (512) W = 512 373 / 422, W = 2048 1016 / 1262.
+// The workgroup walks all queries that see its keys, whatever the size of the call; where even the groups of 128 fill half of the
+// chip or less, bwd_dkv_kernel's of 64 are up to twice as many and each walks fewer queries: 3500 tokens, 32 / 4 heads, W = 300 (110
+// groups of 128) 91 against 128 us, 2001, 32 / 8, W = 200 (128) 45 / 57.  Beyond, they pass one round of places and pull every q / do row
+// twice as often: 2200 tokens, W = 200 (144) 65 / 59, W = 1000 183 / 160, 3000, W = 600 (192) 153 / 115, 4000, W = 1000 (256) 233 /
+// 172, 8 / 2 heads, 4 x 4096, W = 512 132 / 105; short windows, 4000 tokens, W = 128 57 / 51.
 // A scale of (almost) zero goes to bwd_dkv_kernel too: the scores here start from -lse / scale.
+static int key_groups(const NhaPrefillBwdArgs* a) {
+  if (!(fabsf(a->scale) > 1e-30f) || !bwd_ring_supported(a)) return 0;
+  const int64_t g256 = (int64_t)a->H * ((a->NT + 3) / 4), g128 = (int64_t)a->H * ((a->NT + 1) / 2);
+  if (g128 <= 128) return 0;
+  if (short_window(a)) return 128;
+  return (g128 + 255) / 256 * 6 < (g256 + 255) / 256 * 10 ? 128 : 256;
+}
+
 bool bwd_ring_dkv_supported(const NhaPrefillBwdArgs* a) {
-  if (!(fabsf(a->scale) > 1e-30f)) return false;
-  const int64_t groups = (int64_t)a->H * (short_groups(a) ? (a->NT + 1) / 2 : (a->NT + 3) / 4);
-  return bwd_ring_supported(a) && groups > 128;
+  return key_groups(a) != 0;
 }
 
 int bwd_ring_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld) {
@@ -703,19 +767,24 @@ int bwd_ring_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs)
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(once, [&] {
-    attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<256>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES<256>);
+    attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<256, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES<256, 1>);
     if (attr_err == hipSuccess)
-      attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES<128>);
+      attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES<128, 1>);
+    if (attr_err == hipSuccess)
+      attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<128, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES<128, 2>);
   });
   if (attr_err != hipSuccess) {
-    set_error("nha_prefill_bwd: cannot reserve %d bytes of LDS: %s", KV_BYTES<256>, hipGetErrorString(attr_err));
+    set_error("nha_prefill_bwd: cannot reserve %d bytes of LDS: %s", KV_BYTES<256, 1>, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
   // one launch row per chunk, rounded up to whole key groups (4 chunks of 256 keys, 2 of 128)
-  if (short_groups(a))
-    hipLaunchKernelGGL(ring_dkv_kernel<128>, dim3(p.H, 2 * ((p.NT + 1) / 2)), dim3(512), KV_BYTES<128>, (hipStream_t)a->stream, p);
+  const dim3 halves(p.H, 2 * ((p.NT + 1) / 2));
+  if (key_groups(a) == 256)
+    hipLaunchKernelGGL((ring_dkv_kernel<256, 1>), dim3(p.H, 4 * ((p.NT + 3) / 4)), dim3(512), (KV_BYTES<256, 1>), (hipStream_t)a->stream, p);
+  else if (short_window(a))
+    hipLaunchKernelGGL((ring_dkv_kernel<128, 1>), halves, dim3(512), (KV_BYTES<128, 1>), (hipStream_t)a->stream, p);
   else
-    hipLaunchKernelGGL(ring_dkv_kernel<256>, dim3(p.H, 4 * ((p.NT + 3) / 4)), dim3(512), KV_BYTES<256>, (hipStream_t)a->stream, p);
+    hipLaunchKernelGGL((ring_dkv_kernel<128, 2>), halves, dim3(512), (KV_BYTES<128, 2>), (hipStream_t)a->stream, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(window dk, dv, ring)");
   return NHA_OK;
 }

@@ -54,6 +54,15 @@ def test_window_gradients_of_few_key_groups(wl, H, NG, D):
     compare(CU, wl, H, NG, D, ("k_swa", "v"))
 
 
+@pytest.mark.parametrize("H,NG", [(11, 4), (12, 8), (13, 4), (23, 4), (24, 4), (43, 4)])
+@pytest.mark.parametrize("wl", [-1, 160, 192, 500])
+def test_window_gradients_of_128_keys_in_two_groups(wl, H, NG):
+    """Head size 128, 11 groups of 128 keys and 6 of 256 per kv-head: the last size without (11) and the first and last (12, 23; 43) with two
+    groups of waves on 128 keys; units alone and with their complements, an odd number of them, items of fewer queries than 32."""
+    print("case", wl, H, NG, flush=True)
+    compare(CU, wl, H, NG, 128, ("k_swa", "v"))
+
+
 @pytest.mark.parametrize("wl", [40, 400])
 def test_more_sequences_than_lanes(wl):
     """150 ragged sequences of up to 130 tokens, empty ones among them: the forward's workgroups of two chunks search among them, the
