@@ -8,11 +8,13 @@
 // (:233-240), both reads (:242-283) and the branch LSEs (nha_fla/ops/nha/chunk.py:459-470).
 //
 // Who does it: a launch of its own (mfma_repair_kernel) takes 4 us of a call to find nothing to do -- three dependent misses: code,
-// arguments, flags -- a tenth of a call of 300 tokens, and 3 to 4 us of host time; the LDS-direct output passes can do it at their
-// end, in the workgroup that has formed the other rows, but an instance with this code in it takes 1.5 to 2.5 % longer (chunks of
+// arguments, flags -- a tenth of a call of 300 tokens, and 3 to 4 us of host time; an output pass can do it at its end, in the
+// workgroup that has formed the other rows, but an instance with this code in it takes 1.5 to 2.5 % longer (chunks of
 // four heads of 128, W = 2048, 2 x 16384 tokens: 1141 -> 1160 us; W = 64, 2 x 8192: 178 -> 180; 331 tokens 17.9 -> 18.1; head size
 // 256, 32768 tokens, W = 512: 192 -> 197, 16384: 91 -> 92).  So calls whose output pass is short, EXACT_INSIDE_US as estimated from
-// its rounds of workgroups, take that instance and the others the launch.
+// its rounds of workgroups, take that instance and the others the launch.  Whole calls, the launch / inside: 16 heads of 64, 300 tokens
+// 30.4 / 27.2 us, 5003 74.4 / 72.4, 2 x 8192, W = 64 (estimate 87) 176.6 / 172.7; 16 of 128, 2 x 2280, W = 984 (90) 124 / 121;
+// 8 / 4 heads of 64, 500 tokens 29.5 / 26.3.
 #pragma once
 #include "mfma_common.h"
 
@@ -27,11 +29,12 @@ inline double window_units(const MP& p, int rows) {
   return (w + rows) / 32;
 }
 
-// Floats of LDS: the states and gates of a chunk, and what each group of 256 threads keeps of its row.
-template <int D, int GROUPS>
+// Floats of LDS: the states and gates of a chunk, and what each group of 256 threads keeps of its row.  HV: the v-state too, where
+// there is room for it.
+template <int D, int GROUPS, bool HV>
 struct ExactSmem {
   static constexpr int LDH = D + 1;
-  static constexpr int SHARED = MS * LDH + MS * D + BT * MS;
+  static constexpr int SHARED = MS * LDH + (HV ? MS * D : 0) + BT * MS;
   static constexpr int ROW = 2 * D + 2 * MS + 2 * BT + 256 + 4 + BT;
   static constexpr size_t bytes = (size_t)(SHARED + GROUPS * ROW) * 4;
 };
@@ -54,15 +57,15 @@ __device__ __forceinline__ float group_sum(float v, float* red, int t) {
 
 // The rows of the 16-row blocks in `bits` of a chunk (rows c0 .. of the sequence [bos, eos)) for the query heads hq0 .. hq0 + nheads - 1
 // of kv-head h.  GROUPS groups of 256 threads take a head each, or rows of the one head there is; whoever has none left repeats the
-// last one.  Called by the whole workgroup; rsm: ExactSmem<D, GROUPS>::bytes that nobody uses any more.
-template <int D, int GROUPS>
+// last one.  Called by the whole workgroup; rsm: ExactSmem<D, GROUPS, HV>::bytes that nobody uses any more.
+template <int D, int GROUPS, bool HV = true>
 __device__ __forceinline__ void exact_rows(const MP& p, float* rsm, int chunk, int h, int hq0, int nheads, int bits) {
-  typedef ExactSmem<D, GROUPS> S;
+  typedef ExactSmem<D, GROUPS, HV> S;
   constexpr int LDH = S::LDH, NT = 256 * GROUPS;
   const int tid = threadIdx.x, t = tid & 255, group = GROUPS > 1 ? tid >> 8 : 0;
   float* const hk = rsm;                     // [MS][LDH] true chunk-start k-state, transposed
   float* const hv = hk + MS * LDH;           // [MS][D]   true chunk-start v-state
-  float* const gcl = hv + MS * D;            // [BT][MS]  gate cumsum
+  float* const gcl = hv + (HV ? MS * D : 0); // [BT][MS]  gate cumsum
   float* const qg = rsm + S::SHARED + group * S::ROW;   // [D] scaled slot-branch query
   float* const qs = qg + D;                  // [D] scaled window query
   float* const okl = qs + D;                 // [MS] slot logits -> probabilities
@@ -81,7 +84,7 @@ __device__ __forceinline__ void exact_rows(const MP& p, float* rsm, int chunk, i
   for (int e = tid; e < MS * D; e += NT) {
     const int m = e / D, d = e % D;
     hk[m * LDH + d] = bf16_to_f32(p.hkT[(cg * MS + m) * D + d]);
-    hv[m * D + d] = bf16_to_f32(p.hvc[(cg * MS + m) * D + d]);
+    if (HV) hv[m * D + d] = bf16_to_f32(p.hvc[(cg * MS + m) * D + d]);
   }
   for (int e = tid; e < BT * MS; e += NT) gcl[e] = p.gc[cg * BT * MS + e];
 
@@ -161,7 +164,7 @@ __device__ __forceinline__ void exact_rows(const MP& p, float* rsm, int chunk, i
     __syncthreads();
     float acc = 0.f;   // value column t (D <= 256 == threads of a group)
     if (t < D) {
-      for (int m = 0; m < MS; ++m) acc += okl[m] * expf(gct[m]) * hv[m * D + t];
+      for (int m = 0; m < MS; ++m) acc += okl[m] * expf(gct[m]) * (HV ? hv[m * D + t] : bf16_to_f32(p.hvc[(cg * MS + m) * D + t]));
       for (int j = 0; j <= r; ++j) {
         const int sj = src[j];
         if (sj >= 0) acc += Avj[j] * bf16_to_f32(p.v[((int64_t)sj * H + h) * D + t]);

@@ -578,7 +578,8 @@ struct OutSmem {
 
 // SIGN: a scale that is not above zero (in the ordinary kernel the few instructions for it took 2 to 4 % of short windows: 60
 // ragged documents of 300 tokens, 4 heads of 128, W = 64, 50.2 -> 52.5 us).
-template <int D, int G, int NW, int TK, bool OWN, bool SIGN>
+// EXACT: the flagged rows are formed again at the end (prefill_exact.h has when).
+template <int D, int G, int NW, int TK, bool OWN, bool SIGN, bool EXACT>
 __global__ __launch_bounds__(64 * NW, OWN ? NW / 2 : 1) void mfma_out_kernel(const MP p) {
   constexpr int NTHR = 64 * NW;      // threads per workgroup
   constexpr int WPU = NW / G;        // waves per (chunk, head)
@@ -634,6 +635,8 @@ __global__ __launch_bounds__(64 * NW, OWN ? NW / 2 : 1) void mfma_out_kernel(con
     return as_bf16x8(make_uint4((x.x & keep) ^ sign, (x.y & keep) ^ sign, (x.z & keep) ^ sign, (x.w & keep) ^ sign));
   };
   const int64_t cg = (int64_t)chunk * H + h;
+  int exact = 0;   // 16-row blocks of the chunk that decay too fast for the split decay (flags of the state pass)
+  if constexpr (EXACT) exact = p.flags[cg * 4] | p.flags[cg * 4 + 1] | p.flags[cg * 4 + 2] | p.flags[cg * 4 + 3];
 
   // ---- window tile schedule: tile i covers keys [c0 + 64 - TK (i+1), c0 + 64 - TK i) ----------
   int lowest = bos;
@@ -1128,6 +1131,11 @@ __global__ __launch_bounds__(64 * NW, OWN ? NW / 2 : 1) void mfma_out_kernel(con
         p.lse_swa[(int64_t)(c0 + irow) * HQ + hq] = (mrun[qb] * cs + __builtin_amdgcn_logf(lwt)) * LN2;
     }
   }
+  if constexpr (EXACT) {
+    if (exact == 0) return;
+    before_exact();
+    exact_rows<D, NTHR / 256, false>(p, reinterpret_cast<float*>(smem), chunk, h, h * NG + grp * G, G, exact);
+  }
 }
 
 // ==========================================================================================
@@ -1148,7 +1156,7 @@ template <int D>
 int launch_repair(const MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  const size_t lds = ExactSmem<D, 1>::bytes;
+  const size_t lds = ExactSmem<D, 1, true>::bytes;
   std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)mfma_repair_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));
@@ -1159,23 +1167,32 @@ int launch_repair(const MP& p, hipStream_t st) {
   return NHA_OK;
 }
 
-template <int D, int G, int NW, int TK, bool OWN, bool SIGN>
+template <int D, int G, int NW, int TK, bool OWN, bool SIGN, bool EXACT>
 int launch_out_of(const MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  const size_t lds = OutSmem<D, TK, OWN>::bytes;
-  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)mfma_out_kernel<D, G, NW, TK, OWN, SIGN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+  constexpr size_t own = OutSmem<D, TK, OWN>::bytes, rows = EXACT ? ExactSmem<D, NW / 4, false>::bytes : 0;
+  constexpr size_t lds = own > rows ? own : rows;
+  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)mfma_out_kernel<D, G, NW, TK, OWN, SIGN, EXACT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL((mfma_out_kernel<D, G, NW, TK, OWN, SIGN>), dim3(p.H * (p.NG / G), p.NT), dim3(64 * NW), lds, st, p);
+  hipLaunchKernelGGL((mfma_out_kernel<D, G, NW, TK, OWN, SIGN, EXACT>), dim3(p.H * (p.NG / G), p.NT), dim3(64 * NW), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma output pass)");
   return NHA_OK;
 }
 template <int D, int G, int NW, int TK, bool OWN>
-int launch_out(const MP& p, hipStream_t st) {
-  return p.scale > 0.f ? launch_out_of<D, G, NW, TK, OWN, false>(p, st) : launch_out_of<D, G, NW, TK, OWN, true>(p, st);
+int launch_out(const MP& p, bool* exact, hipStream_t st) {
+  if (!(p.scale > 0.f)) return launch_out_of<D, G, NW, TK, OWN, true, false>(p, st);
+  // One or two heads at head sizes 64 and 128 (not the eight waves of two heads that have their own fragments and 128 registers: the
+  // code for the rows spills 50 of them); a workgroup takes 14 us and 0.6 (D = 64) or 0.8 per unit.
+  if constexpr (D <= 128 && (G == 1 || (G == 2 && !OWN))) {
+    constexpr int PER_CU = !OWN ? 1 : D == 64 ? 3 : 2;
+    *exact = (double)p.NT * p.HQ / G / (256 * PER_CU) * (14 + (D == 64 ? 0.6 : 0.8) * window_units(p, BT)) <= EXACT_INSIDE_US;
+    if (*exact) return launch_out_of<D, G, NW, TK, OWN, false, true>(p, st);
+  }
+  return launch_out_of<D, G, NW, TK, OWN, false, false>(p, st);
 }
 
 // state pass: level 1, then level 2 in the forward form (true chunk-start states in place) or, for
@@ -1242,13 +1259,13 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
     } else if (!ring_off && prefill_ring256_supported(p, D)) {
       rc = prefill_ring256_launch(p, &exact, st);
     } else if constexpr (D <= 128) {
-      if (p.NG % 4 == 0) rc = launch_out<D, 4, 8, 64, false>(p, st);
-      else if (p.NG % 2 == 0 && (int64_t)p.HQ / 2 * p.NT > 256) rc = launch_out<D, 2, 8, D == 128 ? 32 : 64, true>(p, st);
-      else if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 64, false>(p, st);
-      else rc = launch_out<D, 1, 4, 32, true>(p, st);
+      if (p.NG % 4 == 0) rc = launch_out<D, 4, 8, 64, false>(p, &exact, st);
+      else if (p.NG % 2 == 0 && (int64_t)p.HQ / 2 * p.NT > 256) rc = launch_out<D, 2, 8, D == 128 ? 32 : 64, true>(p, &exact, st);
+      else if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 64, false>(p, &exact, st);
+      else rc = launch_out<D, 1, 4, 32, true>(p, &exact, st);
     } else {
-      if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 32, false>(p, st);
-      else rc = launch_out<D, 1, 4, 32, true>(p, st);
+      if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 32, false>(p, &exact, st);
+      else rc = launch_out<D, 1, 4, 32, true>(p, &exact, st);
     }
     return rc != NHA_OK || exact ? rc : launch_repair<D>(p, st);
   }

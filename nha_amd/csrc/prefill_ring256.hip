@@ -67,7 +67,7 @@ struct Cfg {
   static constexpr int SS = GC + 16384;        // s bf16 [64][64], pieces XORed with row % 8
   static constexpr int ETAB = SS + 8192;       // decay tables, 6 units of 4 KB
   static constexpr int GC2 = ETAB + 6 * 4096;  // gate cumsums of the second chunk (NCH == 2)
-  static constexpr int USED = GC2 + (NCH - 1) * 16384, EXACT = ExactSmem<D, NCH>::bytes;
+  static constexpr int USED = GC2 + (NCH - 1) * 16384, EXACT = ExactSmem<D, NCH, true>::bytes;
   static constexpr int BYTES = USED > EXACT ? USED : EXACT;
 };
 
