@@ -244,9 +244,11 @@ __device__ __forceinline__ int seb_base(int Q) { return Q == 0 ? 0 : Q == 1 ? 2 
 
 // prefill_mfma.hip: the state pass in segment form
 int prefill_mfma_segment_states(const NhaPrefillArgs* a, mf::MP* out);
-// prefill_bwd_slot.hip: the slot branch of the backward but for the carried state gradient, from a state pass in segment form
+// prefill_bwd_slot.hip: the slot branch of the backward but for the carried state gradient, from a state pass in segment form; in
+// how many parts the query heads of a kv-head are summed, each part's sums of its own after those of the one before
+int bwd_slot_parts(const NhaPrefillBwdArgs* a);
 int bwd_slot_branch(const NhaPrefillBwdArgs* a, const mf::MP& m, float* delta, float* xg, float* dsi, float* ek, float* ev, float* dks,
-                    float* dvs);
+                    float* dvs, int parts);
 // output pass with LDS-direct window loads (prefill_ring.hip); false when the shape is not served
 bool prefill_ring_supported(const mf::MP& p, int D);
 // (*exact: it has formed the flagged rows itself, no exact pass is needed after it)

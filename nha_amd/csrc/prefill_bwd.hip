@@ -55,6 +55,7 @@ struct BP {
   float *dks;             // [T_tot][H][K]     intra-chunk part of dk_gsa, indexed by SOURCE token
   float *ek, *ev;         // [NT][H][K][M], [NT][H][V][M]  N_c, then E_c (see the state-gradient kernels)
   int T_tot, N, NT, HQ, H, K, V, M, wl, shift, nbk, nbv, xNG;   // xNG: heads of a group that xg still keeps apart
+  float *gsum[2], *dsum[2];   // xg, dsi and dks, dvs where the slot branch summed a kv-head's query heads in parts: all of one part, then the next
   float scale;
 };
 
@@ -502,9 +503,31 @@ __global__ __launch_bounds__(256) void bwd_state_direct_kernel(const BP p) {
   }
 }
 
-// grid (N*H, ceil((K+V)*M / 256)): one thread per state element, sequential over the chunks
+// grid (N*H, ceil((K+V)*M / 256)): one thread per state element, sequential over the chunks.  With PARTS > 1 N lies in as many
+// parts, added up as they are read, and the workgroups beyond N*H in x add up those of xg, dsi, dks and dvs (which no one else reads or
+// writes meanwhile, and which would each cost the kernels that read them a memory latency per part).
+template <int PARTS>
 __global__ __launch_bounds__(256) void bwd_state_scan_kernel(const BP p) {
   const int K = p.K, V = p.V, M = p.M, H = p.H;
+  if constexpr (PARTS > 1) {
+    if ((int)blockIdx.x >= p.N * H) {
+      const int64_t ng = (int64_t)p.T_tot * H * M / 4, nd = (int64_t)p.T_tot * H * K / 4;   // (K == V, M == 64)
+      int64_t i = ((int64_t)(blockIdx.x - p.N * H) * gridDim.y + blockIdx.y) * 256 + threadIdx.x;
+      if (i >= 2 * (ng + nd)) return;
+      const bool gates = i < 2 * ng;
+      if (!gates) i -= 2 * ng;
+      const int64_t n = gates ? ng : nd;
+      const int t = i >= n;
+      float4* const at = reinterpret_cast<float4*>(gates ? p.gsum[t] : p.dsum[t]) + (t ? i - n : i);
+      float4 x[PARTS];
+#pragma unroll
+      for (int z = 0; z < PARTS; ++z) x[z] = at[z * n];
+#pragma unroll
+      for (int z = 1; z < PARTS; ++z) { x[0].x += x[z].x; x[0].y += x[z].y; x[0].z += x[z].z; x[0].w += x[z].w; }
+      *at = x[0];
+      return;
+    }
+  }
   const int n = blockIdx.x / H, h = blockIdx.x % H;
   const int e = blockIdx.y * 256 + threadIdx.x;
   if (e >= (K + V) * M) return;
@@ -527,24 +550,36 @@ __global__ __launch_bounds__(256) void bwd_state_scan_kernel(const BP p) {
     if (p.gcx) return p.gcx[(((int64_t)(p.coff[n] + it) * H + h) * BT + R - 1) * M + m];
     return p.gc[((int64_t)(bos + it * BT + R - 1) * H + h) * M + m];
   };
+  const int64_t pstride = (int64_t)p.NT * cstride;
+  auto n_of = [&](int it, float* x) {
+#pragma unroll
+    for (int z = 0; z < PARTS; ++z) x[z] = ebn[z * pstride + it * cstride];
+  };
+  auto sum = [](const float* x) {
+    float a = x[0];
+#pragma unroll
+    for (int z = 1; z < PARTS; ++z) a += x[z];
+    return a;
+  };
   int it = nchunks - 1;
   for (; it >= 3; it -= 4) {
-    float nc[4], gl[4];
+    float nc[4][PARTS], gl[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      nc[u] = ebn[(it - u) * cstride];
+      n_of(it - u, nc[u]);
       gl[u] = gl_of(it - u);
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       ebn[(it - u) * cstride] = E;
-      E = E * expf(gl[u]) + nc[u];
+      E = E * expf(gl[u]) + sum(nc[u]);
     }
   }
   for (; it >= 0; --it) {
-    const float nc = ebn[it * cstride];
+    float nc[PARTS];
+    n_of(it, nc);
     ebn[it * cstride] = E;
-    E = E * expf(gl_of(it)) + nc;
+    E = E * expf(gl_of(it)) + sum(nc);
   }
   float* dh0 = isv ? p.dh0v : p.dh0k;
   if (dh0) {
@@ -987,15 +1022,19 @@ size_t aligned(size_t x) { return (x + 255) & ~(size_t)255; }
 struct BwdPlan {
   size_t fwd, hkct, hvct, hkT, hvT, dus, pp, xg, delta, ld, ck, cv, dsi, dsp, dvs, gtot, dks, ek, ev, total;
   bool use_mfma;   // the slot branch runs on the matrix cores
-  int nbk, nbv;
+  int nbk, nbv, parts;
 };
+// How much of the room that makes a call faster it takes: FULL all of it; WHOLE short segments, the slot branch's sums in one part;
+// LEAST long segments too.
+enum Room { FULL, WHOLE, LEAST };
 // fwd_bytes: the room of the forward's state pass
-BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f, size_t fwd_bytes) {
+BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f, size_t fwd_bytes, Room room) {
   BwdPlan s = {};
   // bf16 shapes the matrix-core state pass covers
   s.use_mfma = prefill_mfma_supported(&f);
   s.nbk = s.use_mfma ? 0 : (a->K + CB - 1) / CB;   // (the matrix-core path keeps these sums on the chip)
   s.nbv = s.use_mfma ? 0 : (a->V + CB - 1) / CB;
+  s.parts = s.use_mfma && room == FULL ? bwd_slot_parts(a) : 1;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
@@ -1016,19 +1055,19 @@ BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f, size_t fwd
     s.ck = take(cc);
     s.cv = take(cc);
   }
-  s.xg = take(s.use_mfma ? thm : tqm);
+  s.xg = take(s.use_mfma ? thm * s.parts : tqm);
   s.delta = take((size_t)a->T_tot * a->HQ * 4);
   // What the LDS-direct dk / dv kernels start their sums from, a pair per (token, query head).  Head size 128: (-lse / scale,
   // -delta), from ring_dq_kernel to ring_dkv_kernel.  Head size 256: (-lse log2(e), -delta), from ring256_dq_kernel or
   // bwd_dq_kernel to ring256_dkv_kernel.
   s.ld = take((size_t)a->T_tot * a->HQ * 8);
-  s.dsi = take(thm);
+  s.dsi = take(thm * s.parts);
   s.dsp = take(thm * (s.nbk + s.nbv));
-  s.dvs = take((size_t)a->T_tot * a->H * a->V * 4);
+  s.dvs = take((size_t)a->T_tot * a->H * a->V * 4 * s.parts);
   s.gtot = take((size_t)a->NT * a->H * a->M * 4);
-  s.dks = take((size_t)a->T_tot * a->H * a->K * 4);
-  s.ek = take(states_k);
-  s.ev = take(states_v);
+  s.dks = take((size_t)a->T_tot * a->H * a->K * 4 * s.parts);
+  s.ek = take(states_k * s.parts);
+  s.ev = take(states_v * s.parts);
   s.total = off;
   return s;
 }
@@ -1045,17 +1084,18 @@ NhaPrefillArgs forward_args(const NhaPrefillBwdArgs* a) {
   return f;
 }
 
-BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, bool least, NhaPrefillArgs* f) {
+BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, Room room, NhaPrefillArgs* f) {
   *f = forward_args(a);
-  f->scratch_bytes = !prefill_mfma_supported(f) ? prefill_simple_scratch_bytes(f) : least ? prefill_mfma_least_scratch_bytes(f) : prefill_mfma_scratch_bytes(f);
-  return plan_bwd(a, *f, f->scratch_bytes);
+  f->scratch_bytes = !prefill_mfma_supported(f) ? prefill_simple_scratch_bytes(f) : room == LEAST ? prefill_mfma_least_scratch_bytes(f) : prefill_mfma_scratch_bytes(f);
+  return plan_bwd(a, *f, f->scratch_bytes, room);
 }
 
 template <typename T>
 int run_bwd(const NhaPrefillBwdArgs* a) {
   NhaPrefillArgs f;
-  BwdPlan sp = plan_bwd(a, false, &f);
-  if (sp.total > a->scratch_bytes) sp = plan_bwd(a, true, &f);   // a workspace sized for another call: long segments
+  BwdPlan sp = plan_bwd(a, FULL, &f);
+  if (sp.total > a->scratch_bytes) sp = plan_bwd(a, WHOLE, &f);   // a workspace sized for another call
+  if (sp.total > a->scratch_bytes) sp = plan_bwd(a, LEAST, &f);
   char* sc = (char*)a->scratch;
   f.hkt = (float*)(sc + sp.hkT);
   f.hvt = (float*)(sc + sp.hvT);
@@ -1074,7 +1114,7 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
     rc = prefill_mfma_segment_states(&f, &states);
     if (rc == NHA_OK)
       rc = bwd_slot_branch(a, states, (float*)(sc + sp.delta), (float*)(sc + sp.xg), (float*)(sc + sp.dsi), (float*)(sc + sp.ek),
-                           (float*)(sc + sp.ev), (float*)(sc + sp.dks), (float*)(sc + sp.dvs));
+                           (float*)(sc + sp.ev), (float*)(sc + sp.dks), (float*)(sc + sp.dvs), sp.parts);
   } else {
     rc = prefill_simple_impl(&f, 1);   // the state pass only
   }
@@ -1146,7 +1186,16 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
     NHA_CHECK_LAUNCH("nha_prefill_bwd(dq_gsa pass)");
     hipLaunchKernelGGL((bwd_state_direct_kernel<T>), dim3(a->NT, a->H * nbmax, 2), dim3(256), lds_s1, st, p);
   }
-  hipLaunchKernelGGL(bwd_state_scan_kernel, dim3(a->N * a->H, ((K + V) * M + 255) / 256), dim3(256), 0, st, p);
+  p.gsum[0] = p.xg; p.gsum[1] = p.dsi; p.dsum[0] = p.dks; p.dsum[1] = p.dvs;
+  const int sblocks = ((K + V) * M + 255) / 256;
+  auto scan = [&](auto kernel) {   // (several parts: two float4 of xg and dsi, of dks and dvs, for each of M and K)
+    const int64_t sums = sp.parts == 1 ? 0 : ((int64_t)a->T_tot * a->H * (M + K) / 2 + 255) / 256;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(a->N * a->H + (sums + sblocks - 1) / sblocks), sblocks), dim3(256), 0, st, p);
+  };
+  if (sp.parts == 8) scan(bwd_state_scan_kernel<8>);
+  else if (sp.parts == 4) scan(bwd_state_scan_kernel<4>);
+  else if (sp.parts == 2) scan(bwd_state_scan_kernel<2>);
+  else scan(bwd_state_scan_kernel<1>);
   if (sp.use_mfma) {
     rc = bwd_slot_inter(a, states.gc, p.ek, p.ev, p.dks, p.dvs, p.xg, p.dsi, p.gtot);
     if (rc != NHA_OK) return rc;
@@ -1168,11 +1217,11 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
 
 size_t prefill_bwd_scratch_bytes(const NhaPrefillBwdArgs* a) {
   NhaPrefillArgs f;
-  return plan_bwd(a, false, &f).total;
+  return plan_bwd(a, FULL, &f).total;
 }
 size_t prefill_bwd_least_scratch_bytes(const NhaPrefillBwdArgs* a) {
   NhaPrefillArgs f;
-  return plan_bwd(a, true, &f).total;
+  return plan_bwd(a, LEAST, &f).total;
 }
 
 bool prefill_bwd_supported(const NhaPrefillBwdArgs* a) { return a->K <= 256 && a->V <= 256 && a->M <= 64 && a->K % 8 == 0 && a->V % 8 == 0; }

@@ -107,7 +107,8 @@ struct SlotP {
   float *xg, *dsi;                             // [T,H,64] (row token)
   float *ek, *ev;                              // [NT][H][D][64]
   float *dks, *dvs;                            // [T,H,D] (source token)
-  int HQ, H, NG, NT, shift, seg_sh;
+  int64_t pm, pe, pd;                          // floats between the sums of two parts of a kv-head's query heads: xg, dsi; ek, ev; dks, dvs
+  int HQ, H, NG, NT, shift, seg_sh;            // NG: query heads of a workgroup (a kv-head's are shared out over gridDim.z)
   float scale;
 };
 
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
   const int tid = threadIdx.x, lane0 = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
   const bool vs = wave >= 4;
-  const int H = p.H, HQ = p.HQ, NG = p.NG;
+  const int H = p.H, HQ = p.HQ, NG = p.NG, part = ONE ? 0 : blockIdx.z;
   // Several heads, two rounds of workgroups or more: the 32 CUs of an XCD start 0.2 us after one another (the second round follows from
   // the first).  All in step, their products come at the same moments, and some cards then run every matrix kernel of the following
   // milliseconds 5 % slower, at the same clock: steps of 2 x 8192 tokens, 32 / 8 heads of 128, W = 2048 one after another 2950 -> 2740
@@ -192,6 +193,7 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
   xcd_tile(D / DW, p.NT, h, chunk);
   const int x0 = (h % (D / DW)) * DW;
   h /= D / DW;
+  const int hq0 = ONE ? h : (h * gridDim.z + part) * NG;   // the workgroup's first query head
   const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
   const int bos = p.cu[n], eos = p.cu[n + 1], c0 = bos + it * BT;
   const int R = (eos - c0) < BT ? (eos - c0) : BT;
@@ -326,8 +328,8 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
     Elem<float>::ld8(gc + j * MS + m8, g);
     Elem<float>::ld8(gc + 31 * MS + m8, ref);
     Head head;
-    load_head(head, h * NG, lane0);
-    if constexpr (ONE) load_o(orow, h, lane0);
+    load_head(head, hq0, lane0);
+    if constexpr (ONE) load_o(orow, hq0, lane0);
     const float dc = p.dcum[cg * MS + col];
 #pragma unroll
     for (int ks = 0; ks < (KEEP ? KS : 2); ++ks) load_operands(ks, ks, lane0);
@@ -368,8 +370,8 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
 #pragma unroll
   for (int rb = 0; rb < 4; ++rb) accS[rb] = (f32x4){0.f, 0.f, 0.f, 0.f};
   xg[0] = xg[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  float* const ep = (vs ? p.ev : p.ek) + (cg * D + x0) * MS;            // N [x][m]
-  float* const op = (vs ? p.dvs : p.dks) + ((int64_t)(bos + tl0) * H + h) * D + x0;   // out, at the rows' source tokens
+  float* const ep = (vs ? p.ev : p.ek) + part * p.pe + (cg * D + x0) * MS;            // N [x][m]
+  float* const op = (vs ? p.dvs : p.dks) + part * p.pd + ((int64_t)(bos + tl0) * H + h) * D + x0;   // out, at the rows' source tokens
 
   // xg and ds_intra (the sum of both sides): rows 32.. from the v side, the others from the k side
   lfloat* const sums = ONE ? (lfloat*)(NHA_LDS void*)(sm + L::Y) : transit;
@@ -394,8 +396,8 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
         const unsigned at = (r * H * MS + col) * 4;
         const float d = vs ? g31 - gi[2 + b][e] : -gi[b][e];
         if (r < R) {
-          st_at(p.xg + ((int64_t)c0 * H + h) * MS, at, xg[b][e]);
-          st_at(p.dsi + ((int64_t)c0 * H + h) * MS, at, EXACT ? z[e] : z[e] * __expf(d));
+          st_at(p.xg + part * p.pm + ((int64_t)c0 * H + h) * MS, at, xg[b][e]);
+          st_at(p.dsi + part * p.pm + ((int64_t)c0 * H + h) * MS, at, EXACT ? z[e] : z[e] * __expf(d));
         }
       }
     }
@@ -406,7 +408,7 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
     if (col < R && tl >= 0) st_at(op + 16 * d, ((tl - tl0) * H * D + 4 * kb) * 4, o);
   };
   for (int a = 0; a < (ONE ? 1 : NG); ++a) {
-    const int hq = h * NG + a;
+    const int hq = hq0 + a;
     // what depends on the lane's number is derived anew for every head: hoisted out of the loop, the addresses and decay
     // factors of a whole head are kept across it -- in memory, there are no registers for them
     int lane = lane0;
@@ -865,21 +867,33 @@ int launch_one(const SlotP& p, hipStream_t st) {
     }
     configured = true;
   }
-  hipLaunchKernelGGL((bwd_slot_kernel<D, DW, EXACT, ONE>), dim3(p.H * (D / DW), p.NT), dim3(512), lds, st, p);
+  hipLaunchKernelGGL((bwd_slot_kernel<D, DW, EXACT, ONE>), dim3(p.H * (D / DW), p.NT, p.HQ / (p.H * p.NG)), dim3(512), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(slot branch)");
   return NHA_OK;
 }
 template <int D>
 int launch(const SlotP& p, hipStream_t st) {
   constexpr int DW = D < 128 ? D : 128;
-  const int rc = p.NG == 1 ? launch_one<D, D, false, true>(p, st) : launch_one<D, DW, false, false>(p, st);
+  const int rc = p.HQ == p.H ? launch_one<D, D, false, true>(p, st) : launch_one<D, DW, false, false>(p, st);
   return rc != NHA_OK ? rc : launch_one<D, DW, true, false>(p, st);
 }
 
 }  // namespace
 
+// A workgroup walks its query heads one after the other, 8 to 9 us each, so where the chunks and kv-heads of a call leave CUs without
+// work the heads are shared out, as many ways as all workgroups still have a place at once; the scan over the chunks adds up the parts'
+// sums.  32 / 4 heads of 128, us: 2 x 533 tokens (72 groups) 80 -> 49, the scan 5.3 -> 9.5; 2000 (128) 87 -> 53; forward and backward of
+// the first at W = 950 308 -> 281.  With two rounds of smaller workgroups a call would pay their first loads (14 us) twice.
+int bwd_slot_parts(const NhaPrefillBwdArgs* a) {
+  const int NG = a->HQ / a->H;
+  const int64_t groups = (int64_t)a->H * a->NT * (a->K == 256 ? 2 : 1);
+  int parts = 1;
+  while (parts < 8 && NG % (2 * parts) == 0 && 2 * parts * groups <= 256) parts *= 2;
+  return parts;
+}
+
 int bwd_slot_branch(const NhaPrefillBwdArgs* a, const mf::MP& m, float* delta, float* xg, float* dsi, float* ek, float* ev, float* dks,
-                    float* dvs) {
+                    float* dvs, int parts) {
   SlotP p;
   p.q = (const bf16_t*)a->q_gsa; p.dout = (const bf16_t*)a->dout; p.o = (const bf16_t*)a->o;
   p.kg = (const bf16_t*)a->k_gsa; p.v = (const bf16_t*)a->v; p.s = (const bf16_t*)a->s;
@@ -887,7 +901,8 @@ int bwd_slot_branch(const NhaPrefillBwdArgs* a, const mf::MP& m, float* delta, f
   p.hk = m.hkT; p.hv = m.hvc; p.hsk = m.hseg_k; p.hsv = m.hseg_v; p.dcum = m.dcum; p.gc = m.gc;
   p.cu = a->cu_seqlens; p.cidx = a->chunk_indices; p.coff = a->chunk_offsets;
   p.dq = (bf16_t*)a->dq_gsa; p.delta = delta; p.xg = xg; p.dsi = dsi; p.ek = ek; p.ev = ev; p.dks = dks; p.dvs = dvs;
-  p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H; p.NT = a->NT; p.shift = a->shift; p.seg_sh = m.seg_sh; p.scale = a->scale;
+  p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H / parts; p.NT = a->NT; p.shift = a->shift; p.seg_sh = m.seg_sh; p.scale = a->scale;
+  p.pm = (int64_t)a->T_tot * a->H * MS; p.pe = (int64_t)a->NT * a->H * a->K * MS; p.pd = (int64_t)a->T_tot * a->H * a->K;
   hipStream_t st = (hipStream_t)a->stream;
   if (a->K == 64) return launch<64>(p, st);
   if (a->K == 128) return launch<128>(p, st);

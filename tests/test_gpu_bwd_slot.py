@@ -55,3 +55,16 @@ def test_slot_branch_one_head_per_kv_head(D, gate_mean):
     d = prefill_inputs(8400 + D, 1, CU[-1], 3, 3, D, D, 64, dtype=BF, qk_scale=D ** -0.5, gate_div=1.0, gate_mean=gate_mean,
                        with_state=True, N=len(CU) - 1)
     run_bwd_case(f"slot one head {gate_mean} D{D}", d, wl=40, shift=33, dtype=BF, cu=CU, with_lse=True)
+
+
+@pytest.mark.parametrize("gate_mean", [0.0, -2.0])
+@pytest.mark.parametrize("NG", [4, 6, 8])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_slot_branch_heads_in_parts(D, NG, gate_mean):
+    """Few chunks and kv-heads: a kv-head's query heads are shared out over 4, 2 and 8 workgroups (six heads: three to each of two),
+    whose sums the scan over the chunks adds up; a shift that leaves tokens without a row, and at -2 chunks of the launch for
+    strongly decaying ones.  The bound of dg is that of the strong gates with final states (test_gpu_prefill_bwd.py): their
+    cotangents enter it at every token with terms that cancel, and all heads summed in one workgroup give the same 0.9 to 1.12e-2."""
+    d = prefill_inputs(8500 + D + NG, 1, CU[-1], 2 * NG, 2, D, D, 64, dtype=BF, qk_scale=D ** -0.5, gate_div=1.0, gate_mean=gate_mean,
+                       with_state=True, N=len(CU) - 1)
+    run_bwd_case(f"slot parts {gate_mean} D{D} NG{NG}", d, wl=40, shift=33, dtype=BF, cu=CU, with_dht=True, dg_bar=2e-2)
