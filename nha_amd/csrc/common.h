@@ -177,13 +177,18 @@ int bwd_window_mfma_dq(const NhaPrefillBwdArgs* a, const float* delta, void* ld)
 bool bwd_ring_supported(const NhaPrefillBwdArgs* a);
 bool bwd_ring_dkv_supported(const NhaPrefillBwdArgs* a);
 int bwd_ring_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld);
-int bwd_ring_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs);
+int bwd_ring_dkv_parts(const NhaPrefillBwdArgs* a);
+int bwd_ring_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs, int parts, float* wk, float* wv);
 // prefill_bwd_ring256.hip: the same for K = V = 256, any number of query heads per kv-head
 bool bwd_ring256_dq_supported(const NhaPrefillBwdArgs* a);
 bool bwd_ring256_dkv_supported(const NhaPrefillBwdArgs* a);
 int bwd_ring256_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld);
-int bwd_ring256_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs);
-int bwd_window_mfma_dkv(const NhaPrefillBwdArgs* a, const float* delta, const float* dvs, const void* ld);
+int bwd_ring256_dkv_parts(const NhaPrefillBwdArgs* a);
+int bwd_ring256_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs, int parts, float* wk, float* wv);
+// parts > 1 (bwd_window_mfma_parts at most, the LDS-direct kernels only): a kv-head's query heads in as many parts, whose fp32 sums go to
+// wk and wv, all of one part and then the next; dk_swa and dv are left to whom it may concern
+int bwd_window_mfma_parts(const NhaPrefillBwdArgs* a);
+int bwd_window_mfma_dkv(const NhaPrefillBwdArgs* a, const float* delta, const float* dvs, const void* ld, int parts, float* wk, float* wv);
 
 }  // namespace nha
 

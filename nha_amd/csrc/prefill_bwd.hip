@@ -55,6 +55,8 @@ struct BP {
   float *dks;             // [T_tot][H][K]     intra-chunk part of dk_gsa, indexed by SOURCE token
   float *ek, *ev;         // [NT][H][K][M], [NT][H][V][M]  N_c, then E_c (see the state-gradient kernels)
   int T_tot, N, NT, HQ, H, K, V, M, wl, shift, nbk, nbv, xNG;   // xNG: heads of a group that xg still keeps apart
+  const float *wk, *wv;       // window parts of dk_swa and dv, [parts][T_tot][H][K], where the window's kernel summed in `wparts` > 1 parts
+  int wparts;
   float *gsum[2], *dsum[2];   // xg, dsi and dks, dvs where the slot branch summed a kv-head's query heads in parts: all of one part, then the next
   float scale;
 };
@@ -852,6 +854,7 @@ __global__ void bwd_gate_scan_kernel(const BP p) {
   }
 }
 
+// z > 0: dk_swa and dv of 1024 elements of the chunk's tokens, from the parts of the window's kernel (K == V; bf16)
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_gate_final_kernel(const BP p) {
   const int M = p.M, H = p.H;
@@ -860,6 +863,30 @@ __global__ __launch_bounds__(256) void bwd_gate_final_kernel(const BP p) {
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int c0 = bos + it * BT;
   const int R = (eos - c0) < BT ? (eos - c0) : BT;
+  if (blockIdx.z) {
+    const int i = (int)(blockIdx.z - 1) * 256 + threadIdx.x, row = i / (p.K / 4);
+    if (row >= R) return;
+    const int64_t off = ((int64_t)(c0 + row) * H + h) * p.K + i % (p.K / 4) * 4, pd = (int64_t)p.T_tot * H * p.K;
+    float4 k[8], v[8], s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int z = 0; z < 8; ++z) {
+      if (z >= p.wparts) break;
+      k[z] = *reinterpret_cast<const float4*>(p.wk + z * pd + off);
+      v[z] = *reinterpret_cast<const float4*>(p.wv + z * pd + off);
+    }
+    // (the last `shift` tokens have no slot part: the zeros of theirs are being written by z = 0)
+    if (row < eos - p.shift - c0) s = *reinterpret_cast<const float4*>(p.dvs + off);
+#pragma unroll
+    for (int z = 1; z < 8; ++z) {
+      if (z >= p.wparts) break;
+      k[0].x += k[z].x; k[0].y += k[z].y; k[0].z += k[z].z; k[0].w += k[z].w;
+      v[0].x += v[z].x; v[0].y += v[z].y; v[0].z += v[z].z; v[0].w += v[z].w;
+    }
+    T* const dk = (T*)p.dk_swa + off, * const dv = (T*)p.dv + off;
+    Elem<T>::st(dk, k[0].x); Elem<T>::st(dk + 1, k[0].y); Elem<T>::st(dk + 2, k[0].z); Elem<T>::st(dk + 3, k[0].w);
+    Elem<T>::st(dv, v[0].x + s.x); Elem<T>::st(dv + 1, v[0].y + s.y); Elem<T>::st(dv + 2, v[0].z + s.z); Elem<T>::st(dv + 3, v[0].w + s.w);
+    return;
+  }
   if (M == BT) {
     __shared__ float4 part[16][16];
     // four consecutive slots of four rows per thread, their 16-byte reads requested together
@@ -1020,11 +1047,11 @@ __global__ __launch_bounds__(256) void bwd_kv_window_kernel(const BP p) {
 size_t aligned(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct BwdPlan {
-  size_t fwd, hkct, hvct, hkT, hvT, dus, pp, xg, delta, ld, ck, cv, dsi, dsp, dvs, gtot, dks, ek, ev, total;
+  size_t fwd, hkct, hvct, hkT, hvT, dus, pp, xg, delta, ld, ck, cv, dsi, dsp, dvs, gtot, dks, ek, ev, wk, wv, total;
   bool use_mfma;   // the slot branch runs on the matrix cores
-  int nbk, nbv, parts;
+  int nbk, nbv, parts, wparts;
 };
-// How much of the room that makes a call faster it takes: FULL all of it; WHOLE short segments, the slot branch's sums in one part;
+// How much of the room that makes a call faster it takes: FULL all of it; WHOLE short segments, the sums of the slot branch and of the window in one part;
 // LEAST long segments too.
 enum Room { FULL, WHOLE, LEAST };
 // fwd_bytes: the room of the forward's state pass
@@ -1035,6 +1062,7 @@ BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f, size_t fwd
   s.nbk = s.use_mfma ? 0 : (a->K + CB - 1) / CB;   // (the matrix-core path keeps these sums on the chip)
   s.nbv = s.use_mfma ? 0 : (a->V + CB - 1) / CB;
   s.parts = s.use_mfma && room == FULL ? bwd_slot_parts(a) : 1;
+  s.wparts = bwd_window_mfma_supported(a) && room == FULL ? bwd_window_mfma_parts(a) : 1;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
@@ -1068,6 +1096,10 @@ BwdPlan plan_bwd(const NhaPrefillBwdArgs* a, const NhaPrefillArgs& f, size_t fwd
   s.dks = take((size_t)a->T_tot * a->H * a->K * 4 * s.parts);
   s.ek = take(states_k * s.parts);
   s.ev = take(states_v * s.parts);
+  if (s.wparts > 1) {
+    s.wk = take((size_t)a->T_tot * a->H * a->K * 4 * s.wparts);
+    s.wv = take((size_t)a->T_tot * a->H * a->V * 4 * s.wparts);
+  }
   s.total = off;
   return s;
 }
@@ -1205,9 +1237,16 @@ int run_bwd(const NhaPrefillBwdArgs* a) {
   }
   NHA_CHECK_LAUNCH("nha_prefill_bwd(state gradients)");
   if (p.scanned) hipLaunchKernelGGL((bwd_gate_scan_kernel<T>), dim3(a->N * a->H), dim3(64), 0, st, p);
-  hipLaunchKernelGGL((bwd_gate_final_kernel<T>), dim3(a->NT, a->H), dim3(256), 0, st, p);
+  // in parts the window's kernel comes first, and the last pass of the gates adds them up
+  p.wparts = wmfma && (bwd_ring_dkv_supported(a) || bwd_ring256_dkv_supported(a)) ? sp.wparts : 1;
+  p.wk = (const float*)(sc + sp.wk); p.wv = (const float*)(sc + sp.wv);
+  if (p.wparts > 1) {
+    rc = bwd_window_mfma_dkv(a, p.delta, p.dvs, sc + sp.ld, p.wparts, (float*)(sc + sp.wk), (float*)(sc + sp.wv));
+    if (rc != NHA_OK) return rc;
+  }
+  hipLaunchKernelGGL((bwd_gate_final_kernel<T>), dim3(a->NT, a->H, p.wparts > 1 ? 1 + K / 16 : 1), dim3(256), 0, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(gate scan)");
-  if (wmfma) return bwd_window_mfma_dkv(a, p.delta, p.dvs, sc + sp.ld);
+  if (wmfma) return p.wparts > 1 ? NHA_OK : bwd_window_mfma_dkv(a, p.delta, p.dvs, sc + sp.ld, 1, nullptr, nullptr);
   hipLaunchKernelGGL((bwd_kv_window_kernel<T>), dim3(a->T_tot, a->H), dim3(256), lds_w, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(key pass)");
   return NHA_OK;

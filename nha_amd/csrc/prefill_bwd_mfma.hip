@@ -768,9 +768,11 @@ int bwd_window_mfma_dq(const NhaPrefillBwdArgs* a, const float* delta, void* ld)
   return launch_dq<256, 32>(p, a->NT, st);
 }
 
-int bwd_window_mfma_dkv(const NhaPrefillBwdArgs* a, const float* delta, const float* dvs, const void* ld) {
-  if (bwd_ring_dkv_supported(a)) return bwd_ring_dkv(a, (const float2*)ld, dvs);
-  if (bwd_ring256_dkv_supported(a)) return bwd_ring256_dkv(a, (const float2*)ld, dvs);
+int bwd_window_mfma_parts(const NhaPrefillBwdArgs* a) { return a->K == 256 ? bwd_ring256_dkv_parts(a) : bwd_ring_dkv_parts(a); }
+
+int bwd_window_mfma_dkv(const NhaPrefillBwdArgs* a, const float* delta, const float* dvs, const void* ld, int parts, float* wk, float* wv) {
+  if (bwd_ring_dkv_supported(a)) return bwd_ring_dkv(a, (const float2*)ld, dvs, parts, wk, wv);
+  if (bwd_ring256_dkv_supported(a)) return bwd_ring256_dkv(a, (const float2*)ld, dvs, parts, wk, wv);
   const WP p = make_wp(a, delta, dvs);
   hipStream_t st = (hipStream_t)a->stream;
   // Eight waves per workgroup where all of them have a place at once: one workgroup per CU, at head size 64 two.  us, four / eight

@@ -304,8 +304,10 @@ struct DkvP {
   const float2* ld;                        // [T,HQ] (-lse / scale, -delta): what the two score accumulators start from
   const float* dvs;                        // [T,H,D] slot-branch part of dv
   bf16_t *dk, *dv;
+  float *wk, *wv;                          // PARTS: in their place fp32 sums, [gridDim.z][T,H,D] (pd floats each)
+  int64_t pd;
   const int32_t *cu, *cidx;
-  int HQ, H, NG, NT, wl;
+  int HQ, H, NG, NT, wl;                   // NG: query heads of a workgroup (PARTS: a kv-head's are shared out over gridDim.z)
   float scale;
 };
 
@@ -330,7 +332,7 @@ __device__ __forceinline__ void wait_items(int younger) {
   else wait_vm<0>();
 }
 
-template <int KEYS, int G>
+template <int KEYS, int G, bool PARTS>
 __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
   constexpr int KW = 8 / G;                // waves that hold the keys, each of G groups all of them
   constexpr int NKB = KEYS / 16 / KW;      // 16-key blocks per wave
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
   const int cperm = CPG * (blockIdx.y % nq) + blockIdx.y / nq;
   if (cperm >= p.NT) return;
   const int chunk = p.NT - 1 - cperm;
-  const int h = blockIdx.x;
+  const int h = blockIdx.x, hq0 = PARTS ? (h * gridDim.z + blockIdx.z) * NG : h * NG;
   const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
   if (it & (CPG - 1)) return;
   const int bos = p.cu[n], eos = p.cu[n + 1];
@@ -369,14 +371,14 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
 
   // block (16-row half wave / 4, 32-column block wave % 4) of both tiles of an item
   const int rh = wave >> 2, cq = wave & 3;
-  // item (g, u): rows [c0 + 32 u, c0 + 32 u + 32) of query head h NG + g; rows past eos are read from row
+  // item (g, u): rows [c0 + 32 u, c0 + 32 u + 32) of query head hq0 + g; rows past eos are read from row
   // eos - 1 (always masked, always finite)
   auto issue_item = [&](int g, int u, int slot) {
     // what follows from the lane number is derived again at every request: kept across the loop it would
     // cost registers the accumulators need
     int ln = threadIdx.x & 63;
     asm volatile("" : "+v"(ln));
-    const int hq = h * NG + g;
+    const int hq = hq0 + g;
     const int q0 = c0 + 32 * u;
     const bf16_t* const qbase = p.q + ((int64_t)bos * HQ + hq) * D;
     const bf16_t* const obase = p.dout + ((int64_t)bos * HQ + hq) * D;
@@ -686,9 +688,14 @@ __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
       if (G == 1 || !grp) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) pk[r] = (__bf16)(dK[db][kk][r] * p.scale);
-        *reinterpret_cast<bf16x4*>(p.dk + off) = pk;
+        if constexpr (PARTS) *reinterpret_cast<f32x4*>(p.wk + blockIdx.z * p.pd + off) = dK[db][kk] * p.scale;
+        else *reinterpret_cast<bf16x4*>(p.dk + off) = pk;
       }
       if (G == 1 || grp) {
+        if constexpr (PARTS) {
+          *reinterpret_cast<f32x4*>(p.wv + blockIdx.z * p.pd + off) = dV[db][kk];
+          continue;
+        }
         const float4 sv = *reinterpret_cast<const float4*>(p.dvs + off);
         pk[0] = (__bf16)(dV[db][kk][0] + sv.x);
         pk[1] = (__bf16)(dV[db][kk][1] + sv.y);
@@ -716,20 +723,34 @@ bool bwd_ring_supported(const NhaPrefillBwdArgs* a) {
 
 static bool short_window(const NhaPrefillBwdArgs* a) { return a->wl >= 0 && a->wl < 160; }
 
+// Parts of a kv-head's query heads: as many as all groups of 128 keys (at most) still have a place at once in (the scale is left out of it, as
+// it is of a workspace's size).
+int bwd_ring_dkv_parts(const NhaPrefillBwdArgs* a) {
+  if (!bwd_ring_supported(a)) return 1;
+  const int NG = a->HQ / a->H;
+  const int64_t g128 = (int64_t)a->H * ((a->NT + a->N) / 2);
+  int parts = 1;
+  while (parts < 8 && NG % (2 * parts) == 0 && 2 * parts * g128 <= 256) parts *= 2;
+  return parts;
+}
+
 // Keys per workgroup of the dk / dv kernel here, 0 where bwd_dkv_kernel takes the call.  Windows of less than 160 keys: 128.  Others: a
 // workgroup of 128 keys takes 0.6 of the time of one of 256, so the fewer rounds of the 256 CUs decide.  us, 256 / 128 keys, 32 / 8
 // heads: 5000 tokens, W = 512 (160 groups of 256 keys) 161 / 188, 2 x 5000 (320) W = 160 202 / 162, W = 300 241 / 220, W = 1000 467
 // / 454, 3 x 4000 (384) W = 1000 520 / 483, 2 x 8192 (512) W = 512 373 / 422, W = 2048 1016 / 1262.
-// The workgroup walks all queries that see its keys, whatever the size of the call; where even the groups of 128 fill half of the
-// chip or less, bwd_dkv_kernel's of 64 are up to twice as many and each walks fewer queries: 3500 tokens, 32 / 4 heads, W = 300 (110
-// groups of 128) 91 against 128 us, 2001, 32 / 8, W = 200 (128) 45 / 57.  Beyond, they pass one round of places and pull every q / do row
-// twice as often: 2200 tokens, W = 200 (144) 65 / 59, W = 1000 183 / 160, 3000, W = 600 (192) 153 / 115, 4000, W = 1000 (256) 233 /
-// 172, 8 / 2 heads, 4 x 4096, W = 512 132 / 105; short windows, 4000 tokens, W = 128 57 / 51.
+// The workgroup walks all queries that see its keys, whatever the size of the call; where even the groups of 128 fill half of the chip
+// or less, the query heads are shared out (bwd_ring_dkv_parts), or, with many short sequences, bwd_dkv_kernel's groups of 64 take the
+// call: us, bwd_dkv_kernel / this in parts and their sum, 32 / 4 heads: 525 packed tokens, W = 134 47 / 17, 2 x 533, W = 950 117 / 50,
+// 2000, W = 300 86 / 46, 3500, W = 300 89 / 75, 4000, W = 500 131 / 102, 2969 packed, W = 70 51 / 41; 32 / 8, 2001, W = 200 44 / 42, 1500, W
+// = 800 95 / 73; 8 / 2, 700, W = 100 29 / 16, 2778, W = 448 58 / 35, 4500, W = 300 48 / 43.
+// Beyond, the groups of 64 pass one round of places and pull every q / do row twice as often: 2200 tokens, W = 200 (144) 65 / 59, W =
+// 1000 183 / 160, 3000, W = 600 (192) 153 / 115, 4000, W = 1000 (256) 233 / 172, 8 / 2 heads, 4 x 4096, W = 512 132 / 105; short
+// windows, 4000 tokens, W = 128 57 / 51.
 // A scale of (almost) zero goes to bwd_dkv_kernel too: the scores here start from -lse / scale.
 static int key_groups(const NhaPrefillBwdArgs* a) {
   if (!(fabsf(a->scale) > 1e-30f) || !bwd_ring_supported(a)) return 0;
   const int64_t g256 = (int64_t)a->H * ((a->NT + 3) / 4), g128 = (int64_t)a->H * ((a->NT + 1) / 2);
-  if (g128 <= 128) return 0;
+  if (g128 <= 128) return bwd_ring_dkv_parts(a) > 1 ? 128 : 0;
   if (short_window(a)) return 128;
   return (g128 + 255) / 256 * 6 < (g256 + 255) / 256 * 10 ? 128 : 256;
 }
@@ -757,34 +778,42 @@ int bwd_ring_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld) {
   return NHA_OK;
 }
 
-int bwd_ring_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs) {
+int bwd_ring_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs, int parts, float* wk, float* wv) {
   DkvP p;
   p.q = (const bf16_t*)a->q_swa; p.k = (const bf16_t*)a->k_swa; p.v = (const bf16_t*)a->v; p.dout = (const bf16_t*)a->dout;
-  p.ld = ld; p.dvs = dvs;
+  p.ld = ld; p.dvs = dvs; p.wk = wk; p.wv = wv; p.pd = (int64_t)a->T_tot * a->H * a->K;
   p.dk = (bf16_t*)a->dk_swa; p.dv = (bf16_t*)a->dv;
   p.cu = a->cu_seqlens; p.cidx = a->chunk_indices;
-  p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H; p.NT = a->NT; p.wl = a->wl; p.scale = a->scale;
+  p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H / parts; p.NT = a->NT; p.wl = a->wl; p.scale = a->scale;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(once, [&] {
-    attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<256, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES<256, 1>);
-    if (attr_err == hipSuccess)
-      attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES<128, 1>);
-    if (attr_err == hipSuccess)
-      attr_err = hipFuncSetAttribute((const void*)ring_dkv_kernel<128, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, KV_BYTES<128, 2>);
+    auto reserve = [&](const void* kernel, int bytes) {
+      if (attr_err == hipSuccess) attr_err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    };
+    reserve((const void*)ring_dkv_kernel<256, 1, false>, KV_BYTES<256, 1>);
+    reserve((const void*)ring_dkv_kernel<128, 1, false>, KV_BYTES<128, 1>);
+    reserve((const void*)ring_dkv_kernel<128, 2, false>, KV_BYTES<128, 2>);
+    reserve((const void*)ring_dkv_kernel<128, 1, true>, KV_BYTES<128, 1>);
+    reserve((const void*)ring_dkv_kernel<128, 2, true>, KV_BYTES<128, 2>);
   });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_bwd: cannot reserve %d bytes of LDS: %s", KV_BYTES<256, 1>, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
   // one launch row per chunk, rounded up to whole key groups (4 chunks of 256 keys, 2 of 128)
-  const dim3 halves(p.H, 2 * ((p.NT + 1) / 2));
+  const dim3 halves(p.H, 2 * ((p.NT + 1) / 2), parts);
+  hipStream_t st = (hipStream_t)a->stream;
   if (key_groups(a) == 256)
-    hipLaunchKernelGGL((ring_dkv_kernel<256, 1>), dim3(p.H, 4 * ((p.NT + 3) / 4)), dim3(512), (KV_BYTES<256, 1>), (hipStream_t)a->stream, p);
+    hipLaunchKernelGGL((ring_dkv_kernel<256, 1, false>), dim3(p.H, 4 * ((p.NT + 3) / 4)), dim3(512), (KV_BYTES<256, 1>), st, p);
+  else if (short_window(a) && parts > 1)
+    hipLaunchKernelGGL((ring_dkv_kernel<128, 1, true>), halves, dim3(512), (KV_BYTES<128, 1>), st, p);
   else if (short_window(a))
-    hipLaunchKernelGGL((ring_dkv_kernel<128, 1>), halves, dim3(512), (KV_BYTES<128, 1>), (hipStream_t)a->stream, p);
+    hipLaunchKernelGGL((ring_dkv_kernel<128, 1, false>), halves, dim3(512), (KV_BYTES<128, 1>), st, p);
+  else if (parts > 1)
+    hipLaunchKernelGGL((ring_dkv_kernel<128, 2, true>), halves, dim3(512), (KV_BYTES<128, 2>), st, p);
   else
-    hipLaunchKernelGGL((ring_dkv_kernel<128, 2>), halves, dim3(512), (KV_BYTES<128, 2>), (hipStream_t)a->stream, p);
+    hipLaunchKernelGGL((ring_dkv_kernel<128, 2, false>), halves, dim3(512), (KV_BYTES<128, 2>), st, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(window dk, dv, ring)");
   return NHA_OK;
 }

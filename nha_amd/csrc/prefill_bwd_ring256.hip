@@ -32,6 +32,8 @@ struct WinP {
   const float *lse_swa, *lse_gsa, *delta;  // [T,HQ]
   float2* ld;                              // [T,HQ] (-lse log2(e), -delta): left by the dq kernel, read by the other
   const float* dvs;                        // [T,H,D] slot-branch part of dv
+  float *wk, *wv;                          // fp32 sums of the dk / dv kernel's parts, [gridDim.z][T,H,D] (pd floats each)
+  int64_t pd;
   bf16_t *dq, *dk, *dv;
   const int32_t *cu, *coff;
   int HQ, H, NG, N, wl;
@@ -254,6 +256,8 @@ constexpr int KV_P = KV_NR * KV_ITEM;             // P in fp32: [item parity][pa
 constexpr int KV_BYTES = KV_P + 2 * 4 * 4096;
 constexpr int UPG = ROWS / 32;                    // 32-query units that a key group spans
 
+// PARTS: a kv-head's query heads are shared out over gridDim.z, and fp32 sums take the place of dk and dv
+template <bool PARTS>
 __global__ __launch_bounds__(512, 1) void ring256_dkv_kernel(const WinP p) {
   extern __shared__ __align__(1024) unsigned char smem_[];
   lbyte* const lds = (lbyte*)smem_;
@@ -264,6 +268,7 @@ __global__ __launch_bounds__(512, 1) void ring256_dkv_kernel(const WinP p) {
   const int H = p.H, HQ = p.HQ, NG = p.NG;
   int h, n, it;
   if (!pair_tile(p.coff, p.N, H, 1, h, n, it)) return;
+  const int hq0 = PARTS ? (h * gridDim.z + blockIdx.z) * NG : h * NG;
   const int bos = p.cu[n], eos = p.cu[n + 1], c0 = bos + it * BT;
   const int rows = (eos - c0) < ROWS ? (eos - c0) : ROWS;
   const int row0 = 32 * pair;   // first key of the wave, relative to c0
@@ -290,7 +295,7 @@ __global__ __launch_bounds__(512, 1) void ring256_dkv_kernel(const WinP p) {
   auto issue_item = [&]() {   // rows past eos are read from row eos - 1: masked, finite
     int ln = threadIdx.x & 63;
     asm volatile("" : "+v"(ln));   // derived anew at every request: kept across the loop it would cost registers
-    const int hq = h * NG + iw.g, q0 = c0 + 32 * iw.u;
+    const int hq = hq0 + iw.g, q0 = c0 + 32 * iw.u;
     const bf16_t* const qbase = p.q + ((int64_t)bos * HQ + hq) * D;
     const bf16_t* const obase = p.dout + ((int64_t)bos * HQ + hq) * D;
     const uint32_t dst = lds0 + islot * KV_ITEM + wave * 1024, pcol = LineTile<D>::load_col(wave, ln);
@@ -449,6 +454,10 @@ __global__ __launch_bounds__(512, 1) void ring256_dkv_kernel(const WinP p) {
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
       const int64_t off = ((int64_t)(c0 + x) * H + h) * D + 16 * db + 4 * (le >> 4);
+      if constexpr (PARTS) {
+        *reinterpret_cast<f32x4*>((second ? p.wk : p.wv) + blockIdx.z * p.pd + off) = second ? acc[db][kk] * p.scale : acc[db][kk];
+        continue;
+      }
       bf16x4 pk;
       if (second) {
 #pragma unroll
@@ -471,19 +480,22 @@ WinP make_p(const NhaPrefillBwdArgs* a, const float* delta, float2* ld, const fl
   p.q = (const bf16_t*)a->q_swa; p.k = (const bf16_t*)a->k_swa; p.v = (const bf16_t*)a->v; p.dout = (const bf16_t*)a->dout;
   p.lse_swa = a->lse_swa; p.lse_gsa = a->lse_gsa; p.delta = delta; p.ld = ld; p.dvs = dvs;
   p.dq = (bf16_t*)a->dq_swa; p.dk = (bf16_t*)a->dk_swa; p.dv = (bf16_t*)a->dv;
+  p.wk = p.wv = nullptr; p.pd = 0;
   p.cu = a->cu_seqlens; p.coff = a->chunk_offsets;
   p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H; p.N = a->N; p.wl = a->wl; p.scale = a->scale;
   return p;
 }
 
 template <class K>
-int launch(K kernel, int lds, int heads, const NhaPrefillBwdArgs* a, const WinP& p, std::once_flag& once, hipError_t& err, const char* what) {
+int launch(K kernel, int lds, int heads, int parts, const NhaPrefillBwdArgs* a, const WinP& p, std::once_flag& once, hipError_t& err, const char* what) {
   std::call_once(once, [&] { err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds); });
   if (err != hipSuccess) {
     set_error("nha_prefill_bwd: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(err));
     return NHA_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL(kernel, pair_grid(heads, a->NT, a->N), dim3(512), lds, (hipStream_t)a->stream, p);
+  dim3 grid = pair_grid(heads, a->NT, a->N);
+  grid.z = parts;
+  hipLaunchKernelGGL(kernel, grid, dim3(512), lds, (hipStream_t)a->stream, p);
   NHA_CHECK_LAUNCH(what);
   return NHA_OK;
 }
@@ -513,6 +525,19 @@ static bool filled(const NhaPrefillBwdArgs* a, int percent) {
 // %) 142 / 145, 60 of 600 (93 %) 160 / 157.
 bool bwd_ring256_dq_supported(const NhaPrefillBwdArgs* a) { return served(a) && (a->wl < 0 || a->wl >= 384) && filled(a, 91); }
 
+// Parts of a kv-head's query heads: as many as all workgroups still have a place at once in, windows of 192 keys or more.  8 / 2
+// heads, bwd_dkv_kernel / ring256_dkv_kernel in parts and their sum, us: 5500 tokens, W = 900 (2 parts) 247 / 142, 2 x 3000, W = 300
+// 107 / 76, 2786, W = 254 52 / 44, 4000, W = 512 91 / 65; 1500 packed, W = 700 (4) 73 / 44; short windows 4000, W = 64 29 / 38, 2500, W
+// = 64 28 / 32, 700, W = 100 36 / 32.
+int bwd_ring256_dkv_parts(const NhaPrefillBwdArgs* a) {
+  if (!served(a) || (a->wl >= 0 && a->wl < 192)) return 1;
+  const int NG = a->HQ / a->H;
+  const int64_t groups = (int64_t)a->H * ((a->NT + a->N) / 2);
+  int parts = 1;
+  while (parts < 8 && NG % (2 * parts) == 0 && 2 * parts * groups <= 256) parts *= 2;
+  return parts;
+}
+
 // One workgroup of 128 keys fills a CU where bwd_dkv_kernel has four of 64 (two per CU), and walks all heads of its group: it pays
 // from half of the chip on, and with one head and short windows not yet.  us, bwd_dkv_kernel / ring256_dkv_kernel: 4 / 4 heads, 2 x
 // 4000 tokens (256 groups) W = 64 47 / 43, W = 256 69 / 52, W = 512 102 / 73, W = 1024 149 / 92; 2 x 6000 (376) 72 / 81, 104 / 101,
@@ -524,7 +549,7 @@ bool bwd_ring256_dq_supported(const NhaPrefillBwdArgs* a) { return served(a) && 
 // 64: 120 of 130 122 / 130, of 256 198 / 157, of 400 297 / 302, of 600 443 / 375; ragged, 300 of 100 194 / 216, 80 of 400 201 /
 // 217, 500 of 600 (93 %) 1807 / 1525.
 bool bwd_ring256_dkv_supported(const NhaPrefillBwdArgs* a) {
-  if (!served(a) || (int64_t)a->H * a->NT <= 256) return false;
+  if (!served(a) || ((int64_t)a->H * a->NT <= 256 && bwd_ring256_dkv_parts(a) == 1)) return false;
   const bool wide = a->wl < 0 || a->wl >= 192;
   if (a->HQ > a->H) return filled(a, wide ? 78 : 91);
   return wide && filled(a, 88);
@@ -533,13 +558,18 @@ bool bwd_ring256_dkv_supported(const NhaPrefillBwdArgs* a) {
 int bwd_ring256_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld) {
   static std::once_flag once;
   static hipError_t err = hipSuccess;
-  return launch(ring256_dq_kernel, DQ_BYTES, a->HQ, a, make_p(a, delta, ld, nullptr), once, err, "nha_prefill_bwd(window dq, ring 256)");
+  return launch(ring256_dq_kernel, DQ_BYTES, a->HQ, 1, a, make_p(a, delta, ld, nullptr), once, err, "nha_prefill_bwd(window dq, ring 256)");
 }
 
-int bwd_ring256_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs) {
-  static std::once_flag once;
-  static hipError_t err = hipSuccess;
-  return launch(ring256_dkv_kernel, KV_BYTES, a->H, a, make_p(a, nullptr, (float2*)ld, dvs), once, err, "nha_prefill_bwd(window dk, dv, ring 256)");
+int bwd_ring256_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs, int parts, float* wk, float* wv) {
+  static std::once_flag once, once_parts;
+  static hipError_t err = hipSuccess, err_parts = hipSuccess;
+  WinP p = make_p(a, nullptr, (float2*)ld, dvs);
+  p.wk = wk; p.wv = wv; p.pd = (int64_t)a->T_tot * a->H * a->K;
+  p.NG /= parts;
+  const char* const what = "nha_prefill_bwd(window dk, dv, ring 256)";
+  if (parts > 1) return launch(ring256_dkv_kernel<true>, KV_BYTES, a->H, parts, a, p, once_parts, err_parts, what);
+  return launch(ring256_dkv_kernel<false>, KV_BYTES, a->H, 1, a, p, once, err, what);
 }
 
 }  // namespace nha

@@ -12,7 +12,7 @@ from tests.util import prefill_inputs
 pytestmark = pytest.mark.gpu
 
 
-def compare(cu, wl, H, NG, D, keys, scale=None):
+def compare(cu, wl, H, NG, D, keys, scale=None, shift=0):
     from nha_amd import chunk_nha
     d = prefill_inputs(9100 + wl + NG, 1, cu[-1], H * NG, H, D, D, 64, dtype=BF, qk_scale=1.0)
     do = torch.randn(1, cu[-1], H * NG, D, generator=torch.Generator().manual_seed(wl + 5)).to(BF)
@@ -20,7 +20,7 @@ def compare(cu, wl, H, NG, D, keys, scale=None):
     for dt in (BF, torch.float32):
         x = [d[k].cuda().to(dt).requires_grad_(True) for k in KEYS]
         o = chunk_nha(*x, cu_seqlens=torch.tensor(cu, dtype=torch.int32).cuda(),
-                      scale=D ** -0.5 if scale is None else scale, window_size_left=wl, gsa_kv_shift=0)[0]
+                      scale=D ** -0.5 if scale is None else scale, window_size_left=wl, gsa_kv_shift=shift)[0]
         o.backward(do.cuda().to(dt))
         outs.append(o.detach())
         grads.append([t.grad for t in x])
@@ -61,6 +61,16 @@ def test_window_gradients_of_128_keys_in_two_groups(wl, H, NG):
     groups of waves on 128 keys; units alone and with their complements, an odd number of them, items of fewer queries than 32."""
     print("case", wl, H, NG, flush=True)
     compare(CU, wl, H, NG, 128, ("k_swa", "v"))
+
+
+@pytest.mark.parametrize("H,NG,D", [(10, 4, 128), (9, 4, 128), (4, 12, 128), (2, 8, 128), (1, 4, 128), (10, 2, 256), (3, 6, 256), (5, 4, 256), (2, 8, 256)])
+@pytest.mark.parametrize("wl", [-1, 40, 159, 160, 300])
+def test_window_gradients_of_query_heads_in_parts(wl, H, NG, D):
+    """Few groups of 128 keys: a kv-head's query heads are shared out over 2, 4 (three heads to each of four at 12) and 8 workgroups whose
+    fp32 sums the last pass of the gates adds up; (10, 4, 128) is the first size without.  A shift that leaves the last tokens of a
+    sequence, and whole sequences, without a slot part of dv."""
+    print("case", wl, H, NG, D, flush=True)
+    compare(CU256 if D == 256 else CU, wl, H, NG, D, ("k_swa", "v", "q_swa"), shift=50)
 
 
 @pytest.mark.parametrize("wl", [40, 400])

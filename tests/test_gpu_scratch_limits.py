@@ -30,7 +30,7 @@ def _smaller_workspace(cls, query, T, HQ, H, D):
     return (own, least) if least < own else (own, None)
 
 
-@pytest.mark.parametrize("T,HQ,H,D", [(1000, 8, 8, 128), (1152, 8, 8, 128), (1216, 16, 4, 64), (1088, 4, 4, 256)])
+@pytest.mark.parametrize("T,HQ,H,D", [(1000, 8, 8, 128), (1152, 8, 8, 128), (1216, 16, 4, 64), (1088, 4, 4, 256), (2048, 8, 2, 128), (2048, 8, 2, 256)])
 def test_forward_and_backward_in_a_longer_calls_workspace(T, HQ, H, D):
     lib = _lib.load()
     dev = torch.device("cuda:0")
