@@ -251,10 +251,9 @@ int bwd_slot_branch(const NhaPrefillBwdArgs* a, const mf::MP& m, float* delta, f
                     float* dvs, int parts);
 // output pass with LDS-direct window loads (prefill_ring.hip); false when the shape is not served
 bool prefill_ring_supported(const mf::MP& p, int D);
-// (*exact: it has formed the flagged rows itself, no exact pass is needed after it)
-int prefill_ring_launch(const mf::MP& p, int D, bool* exact, hipStream_t st);
+int prefill_ring_launch(const mf::MP& p, int D, hipStream_t st);
 // the same for head size 256, one query head per workgroup (prefill_ring256.hip)
 bool prefill_ring256_supported(const mf::MP& p, int D);
-int prefill_ring256_launch(const mf::MP& p, bool* exact, hipStream_t st);
+int prefill_ring256_launch(const mf::MP& p, hipStream_t st);
 
 }  // namespace nha

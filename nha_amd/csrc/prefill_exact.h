@@ -7,26 +7,27 @@
 // again with the unfactored decay (<= 1): slot logits (nha_fla/ops/nha/chunk_fused.py:186-222), window logits, one softmax
 // (:233-240), both reads (:242-283) and the branch LSEs (nha_fla/ops/nha/chunk.py:459-470).
 //
-// Who does it: a launch of its own (mfma_repair_kernel) takes 4 us of a call to find nothing to do -- three dependent misses: code,
-// arguments, flags -- a tenth of a call of 300 tokens, and 3 to 4 us of host time; an output pass can do it at its end, in the
-// workgroup that has formed the other rows, but an instance with this code in it takes 1.5 to 2.5 % longer (chunks of
-// four heads of 128, W = 2048, 2 x 16384 tokens: 1141 -> 1160 us; W = 64, 2 x 8192: 178 -> 180; 331 tokens 17.9 -> 18.1; head size
-// 256, 32768 tokens, W = 512: 192 -> 197, 16384: 91 -> 92).  So calls whose output pass is short, EXACT_INSIDE_US as estimated from
-// its rounds of workgroups, take that instance and the others the launch.  Whole calls, the launch / inside: 16 heads of 64, 300 tokens
-// 30.4 / 27.2 us, 5003 74.4 / 72.4, 2 x 8192, W = 64 (estimate 87) 176.6 / 172.7; 16 of 128, 2 x 2280, W = 984 (90) 124 / 121;
-// 8 / 4 heads of 64, 500 tokens 29.5 / 26.3.
+// Who does it: the output pass at its end, in the workgroup that has formed the other rows.  A launch of its own (mfma_repair_kernel)
+// takes 4 to 5 us of a call to find nothing to do -- three dependent misses: code, arguments, flags -- and 3 to 4 us of host time.
+// The arguments are read again for it (arguments_again): kept from the beginning they cost ring_out_kernel 23 spilled scalar registers
+// and 1.5 %.  Whole calls, the launch / inside, us: four heads of 128, 2 x 8192 tokens, W = 64 232.5 / 228.8, 2 x 16384, W = 2048 1170.5
+// / 1170; head size 256, 32768 packed, W = 512 307 / 304, 4 x 8192, 8 / 2 heads, W = 2000 659 / 654; 16 heads of 128, 4 x 8192, W = 64
+// 532 / 523.  At head size 64 with one or two heads the instance has room for it only at some cost: 16 heads, 2 x 8192, W = 2048 330 /
+// 333, W = 64 176.6 / 172.7, 5003 tokens 74.4 / 72.4, 300 30.4 / 27.2; there short passes, EXACT_INSIDE_US as estimated from the rounds
+// of workgroups, take it and the others the launch.  Every row flagged: four heads of 128, 4096 tokens, W = 512 23.5 / 22.7 ms, 4 heads
+// of 256 7.3 / 7.1.
 #pragma once
 #include "mfma_common.h"
 
 namespace nha {
 namespace mf {
 
-// Output passes up to this long form the exact rows themselves.
+// Output passes of head size 64 up to this long form the exact rows themselves.
 constexpr double EXACT_INSIDE_US = 100;
-// units of 32 keys that a workgroup of `rows` rows walks on average, from the call's totals
-inline double window_units(const MP& p, int rows) {
+// units of 32 keys that a workgroup walks on average, from the call's totals
+inline double window_units(const MP& p) {
   const double len = (double)p.T_tot / p.N, w = p.wl < 0 || p.wl > len / 2 ? len / 2 : p.wl;
-  return (w + rows) / 32;
+  return (w + BT) / 32;
 }
 
 // Floats of LDS: the states and gates of a chunk, and what each group of 256 threads keeps of its row.  HV: the v-state too, where
@@ -181,6 +182,14 @@ __device__ __forceinline__ void exact_rows(const MP& p, float* rsm, int chunk, i
     }
     if (t < D) p.o[((int64_t)tok * HQ + hq) * D + t] = f32_to_bf16(acc);
   }
+}
+
+// The kernel's arguments (its only parameter), read anew: what a rare branch at the end of a kernel takes of them would otherwise be
+// kept from the beginning, in scalar registers that the loop before it does not have to spare.
+__device__ __forceinline__ const MP& arguments_again() {
+  const __attribute__((address_space(4))) void* a = (const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return *(const MP*)a;
 }
 
 // This wave's stores have been written and everybody's LDS reads are done: exact_rows may write over both.

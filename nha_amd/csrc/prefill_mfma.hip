@@ -1134,7 +1134,7 @@ __global__ __launch_bounds__(64 * NW, OWN ? NW / 2 : 1) void mfma_out_kernel(con
   if constexpr (EXACT) {
     if (exact == 0) return;
     before_exact();
-    exact_rows<D, NTHR / 256, false>(p, reinterpret_cast<float*>(smem), chunk, h, h * NG + grp * G, G, exact);
+    exact_rows<D, NTHR / 256, false>(arguments_again(), reinterpret_cast<float*>(smem), chunk, h, h * NG + grp * G, G, exact);
   }
 }
 
@@ -1186,10 +1186,10 @@ template <int D, int G, int NW, int TK, bool OWN>
 int launch_out(const MP& p, bool* exact, hipStream_t st) {
   if (!(p.scale > 0.f)) return launch_out_of<D, G, NW, TK, OWN, true, false>(p, st);
   // One or two heads at head sizes 64 and 128 (not the eight waves of two heads that have their own fragments and 128 registers: the
-  // code for the rows spills 50 of them); a workgroup takes 14 us and 0.6 (D = 64) or 0.8 per unit.
+  // code for the rows spills 50 of them); at D = 64, where the pass is short: a workgroup takes 14 us and 0.6 per unit.
   if constexpr (D <= 128 && (G == 1 || (G == 2 && !OWN))) {
     constexpr int PER_CU = !OWN ? 1 : D == 64 ? 3 : 2;
-    *exact = (double)p.NT * p.HQ / G / (256 * PER_CU) * (14 + (D == 64 ? 0.6 : 0.8) * window_units(p, BT)) <= EXACT_INSIDE_US;
+    *exact = D == 128 || (double)p.NT * p.HQ / G / (256 * PER_CU) * (14 + 0.6 * window_units(p)) <= EXACT_INSIDE_US;
     if (*exact) return launch_out_of<D, G, NW, TK, OWN, false, true>(p, st);
   }
   return launch_out_of<D, G, NW, TK, OWN, false, false>(p, st);
@@ -1254,11 +1254,9 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
 #else
     constexpr bool ring_off = false;
 #endif
-    if (!ring_off && prefill_ring_supported(p, D)) {
-      rc = prefill_ring_launch(p, D, &exact, st);
-    } else if (!ring_off && prefill_ring256_supported(p, D)) {
-      rc = prefill_ring256_launch(p, &exact, st);
-    } else if constexpr (D <= 128) {
+    if (!ring_off && prefill_ring_supported(p, D)) return prefill_ring_launch(p, D, st);
+    if (!ring_off && prefill_ring256_supported(p, D)) return prefill_ring256_launch(p, st);
+    if constexpr (D <= 128) {
       if (p.NG % 4 == 0) rc = launch_out<D, 4, 8, 64, false>(p, &exact, st);
       else if (p.NG % 2 == 0 && (int64_t)p.HQ / 2 * p.NT > 256) rc = launch_out<D, 2, 8, D == 128 ? 32 : 64, true>(p, &exact, st);
       else if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 64, false>(p, &exact, st);

@@ -129,9 +129,8 @@ __device__ __forceinline__ void sink_exact_rows(const MP& p, float* rsm, int chu
 // (position in its sequence) still sees clamp(p.wl - t, 0, p.sinks): the "full attention" layers of the hybrid models
 // (nha_fla/models/qwen3_moe_nha/qwennha.py:323-336, :400-413).  No slot operands are requested, the slot branch and its
 // tables are skipped, and the sinks join the denominator in the epilogue with the weight 2^(-reference) each.
-// EXACT: rows that leave the range of the kernel's arithmetic are formed again at the end (prefill_exact.h has when); without it
-// they are flagged for the exact pass after it.
-template <int D, bool SINK, bool EXACT>
+// Rows that leave the range of the kernel's arithmetic are formed again at the end (prefill_exact.h).
+template <int D, bool SINK>
 __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   using C = RingCfg<D>;
   constexpr int KS = C::KS, DB = C::DB, UB = C::UB, HB = C::HB, NR = C::NR, LPW = C::LPW;
@@ -160,7 +159,7 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   const float cs = p.scale * LOG2E;
   const int64_t cg = (int64_t)chunk * H + h;
   int exact = 0;   // 16-row blocks of the chunk that decay too fast for the split decay (flags of the state pass)
-  if constexpr (!SINK && EXACT) exact = p.flags[cg * 4] | p.flags[cg * 4 + 1] | p.flags[cg * 4 + 2] | p.flags[cg * 4 + 3];
+  if constexpr (!SINK) exact = p.flags[cg * 4] | p.flags[cg * 4 + 1] | p.flags[cg * 4 + 2] | p.flags[cg * 4 + 3];
 
   // window units: unit u covers keys [c0 + 32 - 32 u, c0 + 64 - 32 u); c0 - bos is a multiple of 64, so no
   // unit starts before its sequence; units 0 and 1 are the chunk's own rows and may run past eos
@@ -550,11 +549,7 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
     if (__any(16 * (qb0 + qb) + l16 < rows && (Lw[qb][0] >= 0x1p100f || Lw[qb][0] < 0x1p-100f))) bad |= 1 << (qb0 + qb);
   constexpr int FLAGS = SINK ? 0 : C::FLAGS;
   if constexpr (SINK) lds_barrier();   // the ring is done with
-  if constexpr (EXACT) {
-    if (lane == 0) *reinterpret_cast<NHA_LDS int*>(lds + FLAGS + 4 * wave) = bad;
-  } else if (bad && lane == 0) {
-    atomicOr(p.flags + cg * 4, bad);
-  }
+  if (lane == 0) *reinterpret_cast<NHA_LDS int*>(lds + FLAGS + 4 * wave) = bad;
   float lg[RQB];
   if constexpr (SINK) {
     // the sinks still in view: logit 0, i.e. 2^(0 - reference) each relative to the row's reference; value 0
@@ -575,11 +570,9 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   if (nunits <= NR) wait_vm<4 * LPW>();
   else wait_vm<0>();
   lds_barrier();
-  if constexpr (EXACT) {
 #pragma unroll
-    for (int w = 0; w < 8; ++w) exact |= *reinterpret_cast<const NHA_LDS int*>(lds + C::FLAGS + 4 * w);
-    exact = __builtin_amdgcn_readfirstlane(exact);
-  }
+  for (int w = 0; w < 8; ++w) exact |= *reinterpret_cast<const NHA_LDS int*>(lds + C::FLAGS + 4 * w);
+  exact = __builtin_amdgcn_readfirstlane(exact);
   auto gc_at = [&](int j, int m) -> const lfloat* { return (const lfloat*)(lds + C::GC + j * 256 + (((m >> 2) ^ (j & 15)) * 16) + (m & 3) * 4); };
   auto s_at = [&](int j, int m) -> const lbf16* { return (const lbf16*)(lds + C::SS + j * 128 + (((m >> 3) ^ (j & 7)) * 16) + (m & 7) * 2); };
   // decay tables E_Q[j][m] = s_j[m] exp(min(gr_Q[m] - gc_j[m], DECAY_CLAMP)) for the rows j of the 16-row
@@ -824,7 +817,6 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
     }
   }
   // ---- rows that have to be formed again, for the four heads of the workgroup -----------------------
-  if constexpr (!EXACT) return;
   if constexpr (SINK) {
     lds_barrier();
 #pragma unroll
@@ -833,23 +825,23 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   }
   if (exact == 0) return;
   before_exact();
-  if constexpr (SINK) sink_exact_rows<D>(p, reinterpret_cast<float*>(smem_), chunk, h, h * NG + grp * 4, exact);
-  else if constexpr (EXACT) exact_rows<D, 2>(p, reinterpret_cast<float*>(smem_), chunk, h, h * NG + grp * 4, 4, exact);
+  if constexpr (SINK) sink_exact_rows<D>(arguments_again(), reinterpret_cast<float*>(smem_), chunk, h, h * NG + grp * 4, exact);
+  else exact_rows<D, 2>(arguments_again(), reinterpret_cast<float*>(smem_), chunk, h, h * NG + grp * 4, 4, exact);
 }
 
-template <int D, bool SINK, bool EXACT>
+template <int D, bool SINK>
 int launch_ring(const MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   // the window-only launch has no slot operands: the ring and the eight waves' window queries behind it (128 KB at D = 128, 96 at
   // 64; its registers leave room for one workgroup per CU as well)
   const size_t lds = SINK ? (size_t)(RingCfg<D>::QT + 8 * RingCfg<D>::UB) : (size_t)RingCfg<D>::BYTES;
-  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring_out_kernel<D, SINK, EXACT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring_out_kernel<D, SINK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL((ring_out_kernel<D, SINK, EXACT>), dim3(p.H * (p.NG / 4), p.NT), dim3(512), lds, st, p);
+  hipLaunchKernelGGL((ring_out_kernel<D, SINK>), dim3(p.H * (p.NG / 4), p.NT), dim3(512), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma output pass, ring)");
   return NHA_OK;
 }
@@ -864,11 +856,8 @@ bool prefill_ring_supported(const mf::MP& p, int D) {
   return (int64_t)p.T_tot * p.H * D * 2 < ((int64_t)1 << 32) && (int64_t)p.T_tot * p.H * MS * 2 < ((int64_t)1 << 32);
 }
 
-int prefill_ring_launch(const mf::MP& p, int D, bool* exact, hipStream_t st) {
-  // a workgroup takes 18 us and 0.85 per unit at D = 128
-  *exact = (double)p.NT * p.HQ / 4 / 256 * (18 + 0.85 * window_units(p, BT)) <= EXACT_INSIDE_US;
-  if (*exact) return D == 64 ? launch_ring<64, false, true>(p, st) : launch_ring<128, false, true>(p, st);
-  return D == 64 ? launch_ring<64, false, false>(p, st) : launch_ring<128, false, false>(p, st);
+int prefill_ring_launch(const mf::MP& p, int D, hipStream_t st) {
+  return D == 64 ? launch_ring<64, false>(p, st) : launch_ring<128, false>(p, st);
 }
 
 // Sliding-window attention with zero sinks (nha_sink_window_fwd): the window loop of ring_out_kernel alone.  (What
@@ -889,7 +878,7 @@ int sink_window_impl(const NhaSinkWindowArgs* a) {
     return NHA_ERR_UNSUPPORTED;
   }
   hipStream_t st = (hipStream_t)a->stream;
-  return a->D == 64 ? launch_ring<64, true, true>(p, st) : launch_ring<128, true, true>(p, st);
+  return a->D == 64 ? launch_ring<64, true>(p, st) : launch_ring<128, true>(p, st);
 }
 
 }  // namespace nha

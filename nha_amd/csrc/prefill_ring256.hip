@@ -72,8 +72,7 @@ struct Cfg {
 };
 
 // LDS layout of a 32-row buffer: LineTile.
-// EXACT: as in ring_out_kernel (prefill_ring.hip).
-template <int NCH, bool EXACT>
+template <int NCH>
 __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
   using C = Cfg<NCH>;
   constexpr int XB0 = 64 * NCH - 32;           // first key of unit 0, relative to the workgroup's first row
@@ -112,7 +111,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
     exact[c] = 0;
-    if (EXACT && rows_wg > BT * c) {
+    if (rows_wg > BT * c) {
       const int* const f = p.flags + (cg + (int64_t)c * H) * 4;
       exact[c] = f[0] | f[1] | f[2] | f[3];
     }
@@ -501,11 +500,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     // is ever taken.  fp32 sums and bf16 probabilities hold 2^BIG above it; a score beyond that sends the
     // wave's 16 rows to the exact pass and is clamped.
     if (__any(m0 > BIG)) {
-      if constexpr (EXACT) {
-        if (16 * Q < rows) bad = 1 << Q;   // (a chunk that is not there has no flags)
-      } else if (lane == 0 && 16 * Q < rows) {
-        atomicOr(p.flags + (cg + (int64_t)ch * H) * 4, 1 << Q);
-      }
+      if (16 * Q < rows) bad = 1 << Q;   // (a chunk that is not there has no rows)
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -769,7 +764,6 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     }
   }
   // ---- rows that have to be formed again (prefill_exact.h) ------------------------------------------
-  if constexpr (!EXACT) return;
   lds_barrier();
   if (lane == 0) *reinterpret_cast<NHA_LDS int*>(lds + 4 * wave) = bad;
   lds_barrier();
@@ -780,7 +774,7 @@ __global__ __launch_bounds__(256 * NCH, 1) void ring256_out_kernel(const MP p) {
     const int bits = __builtin_amdgcn_readfirstlane(exact[c]);
     if (bits == 0) continue;
     before_exact();
-    exact_rows<D, NCH>(p, reinterpret_cast<float*>(smem_), chunk + c, h, hq, 1, bits);
+    exact_rows<D, NCH>(arguments_again(), reinterpret_cast<float*>(smem_), chunk + c, h, hq, 1, bits);
   }
 }
 
@@ -795,29 +789,26 @@ bool prefill_ring256_supported(const mf::MP& p, int D) {
 }
 
 namespace {
-template <int NCH, bool EXACT>
+template <int NCH>
 int launch_ring256(const mf::MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring256_out_kernel<NCH, EXACT>, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg<NCH>::BYTES); });
+  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring256_out_kernel<NCH>, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg<NCH>::BYTES); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %d bytes of LDS: %s", Cfg<NCH>::BYTES, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL((ring256_out_kernel<NCH, EXACT>), NCH == 1 ? dim3(p.HQ, p.NT) : pair_grid(p.HQ, p.NT, p.N), dim3(256 * NCH), Cfg<NCH>::BYTES, st, p);
+  hipLaunchKernelGGL((ring256_out_kernel<NCH>), NCH == 1 ? dim3(p.HQ, p.NT) : pair_grid(p.HQ, p.NT, p.N), dim3(256 * NCH), Cfg<NCH>::BYTES, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma output pass, ring, head size 256)");
   return NHA_OK;
 }
 }  // namespace
 
-int prefill_ring256_launch(const mf::MP& p, bool* exact, hipStream_t st) {
+int prefill_ring256_launch(const mf::MP& p, hipStream_t st) {
   // two chunks per workgroup unless most sequences have a single chunk (fewer than three chunks per two sequences):
   // there the second half of a two-chunk workgroup would mostly idle
   const bool one = 2 * (int64_t)p.NT < 3 * (int64_t)p.N;
-  // a workgroup takes 18 us and 0.9 per unit
-  *exact = (double)p.NT / (one ? 1 : 2) * p.HQ / 256 * (18 + 0.9 * window_units(p, one ? BT : 2 * BT)) <= EXACT_INSIDE_US * 3 / 5;
-  if (one) return *exact ? launch_ring256<1, true>(p, st) : launch_ring256<1, false>(p, st);
-  return *exact ? launch_ring256<2, true>(p, st) : launch_ring256<2, false>(p, st);
+  return one ? launch_ring256<1>(p, st) : launch_ring256<2>(p, st);
 }
 
 }  // namespace nha

@@ -1,5 +1,5 @@
-"""Rows that leave the range of the output pass's arithmetic are formed again by the pass itself where it is short and by a launch
-after it where it is long (prefill_exact.h).  The same sequences, some of whose rows decay too fast, in one long call and each alone:
+"""Rows that leave the range of the output pass's arithmetic are formed again by the pass itself, and by a launch after it where a pass
+of one or two heads of 64 is long or two heads of 128 share a kv-head in many workgroups (prefill_exact.h).  The same sequences, some of whose rows decay too fast, in one long call and each alone:
 the two forms share their arithmetic but not their instances, and calls of other sizes may cut their states into other segments, which
 rounds chunk-start states of bf16 (2^-9) differently; outputs 2e-2 absolute + 1e-2 relative per element as in the parity tests, which
 hold the short calls against the oracle."""
@@ -13,8 +13,8 @@ BF = torch.bfloat16
 KEYS = ["q_swa", "k_swa", "q_gsa", "k_gsa", "v", "s", "g"]
 
 
-# estimates of the output pass (us, of which 100 or, at head size 256, 60 are the line): above 118 in one call, below 5 alone (two heads
-# per kv-head: the one call takes the kernel that leaves the rows to the launch)
+# estimates of the output pass (us, of which 100 are the line at head size 64): above 118 in one call, below 5 alone (two heads per
+# kv-head: the one call takes the kernel that leaves the rows to the launch)
 @pytest.mark.parametrize("D,HQ,H,N", [(128, 32, 8, 42), (64, 16, 4, 70), (256, 8, 2, 64), (64, 16, 16, 40), (128, 4, 4, 80), (64, 8, 4, 42),
                                       (128, 8, 4, 42)])
 def test_exact_rows_inside_and_after(D, HQ, H, N):
