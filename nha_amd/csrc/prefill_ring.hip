@@ -1,4 +1,4 @@
-// Output pass of the bf16 matrix-core prefill for groups of four query heads per kv-head (K == V == D
+// Output pass of the bf16 matrix-core prefill for groups of four query heads per kv-head, or of two (K == V == D
 // in {64, 128}, M == 64): same mathematics as mfma_out_kernel (prefill_mfma.hip; chunk algebra of
 // nha_fla/ops/nha/chunk_fused.py:186-283, one softmax over [slots | window] as in
 // nha_fla/ops/nha/chunk.py:459-470), different data movement and order.
@@ -12,7 +12,7 @@
 //  * The window loop is software-pipelined inside each wave: while the matrix core forms the scores
 //    of unit u+1, the VALU exponentiates unit u.  The scale and the softmax reference are folded into
 //    the score product itself (pre-scaled queries, accumulator started at -reference), so a score
-//    needs one v_exp_f32 and half a v_cvt_pk_bf16_f32 and nothing else.
+//    needs one v_exp_f32 and half a v_cvt_pk_bf16_f32 and nothing else (groups of two: a multiplication too, on unrounded queries).
 //  * The softmax reference of a query row is fixed once, from the first unit (the row's own and
 //    nearest keys; 0 for rows that unit does not reach): fp32 sums relative to a fixed reference are
 //    exact while every score stays within 2^+-100 of it, and the loop carries no maxima, no
@@ -130,11 +130,12 @@ __device__ __forceinline__ void sink_exact_rows(const MP& p, float* rsm, int chu
 // (nha_fla/models/qwen3_moe_nha/qwennha.py:323-336, :400-413).  No slot operands are requested, the slot branch and its
 // tables are skipped, and the sinks join the denominator in the epilogue with the weight 2^(-reference) each.
 // Rows that leave the range of the kernel's arithmetic are formed again at the end (prefill_exact.h).
-template <int D, bool SINK>
+// RQB: 16-row query blocks per wave, 2 (a workgroup takes four heads) or 1 (two heads).
+template <int D, bool SINK, int RQB>
 __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   using C = RingCfg<D>;
   constexpr int KS = C::KS, DB = C::DB, UB = C::UB, HB = C::HB, NR = C::NR, LPW = C::LPW;
-  constexpr int RQB = 2;                        // 16-row query blocks per wave
+  constexpr int HEADS = 2 * RQB;                // query heads of the workgroup
   constexpr int NPRE = NR - 1;                  // units requested before the loop
   extern __shared__ __align__(1024) unsigned char smem_[];
   lbyte* const lds = (lbyte*)smem_;
@@ -142,21 +143,26 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, kb = lane >> 4;
   const int H = p.H, HQ = p.HQ, NG = p.NG;
-  // grid = (kv-head x group of four q-heads, chunk), chunks from the last to the first (prefill_mfma.hip)
-  const int ngrp = NG / 4;
+  // grid = (kv-head x group of HEADS q-heads, chunk), chunks from the last to the first (prefill_mfma.hip)
+  const int ngrp = NG / HEADS;
   int vx, vy;
   xcd_tile(ngrp, p.NT, vx, vy);   // with 8 (kv-head, group) pairs this is the launch order itself
   const int chunk = p.NT - 1 - vy;
   const int h = vx / ngrp, grp = vx % ngrp;
-  const int hq = h * NG + grp * 4 + wave / 2;
-  // rows 0..31 or 32..63 of the chunk: the later rows have more intra-chunk work in the slot branch, so the two
-  // waves that share a SIMD (w and w + 4) take one half each
-  const int qb0 = ((wave ^ (wave >> 2)) & 1) * RQB;
+  const int hq = h * NG + grp * HEADS + wave * HEADS / 8;
+  // the wave's first 16-row block of the chunk: the later rows have more intra-chunk work in the slot branch, so the two
+  // waves that share a SIMD (w and w + 4) take one half each, or blocks as far from the chunk's ends
+  const int qb0 = RQB == 2 ? ((wave ^ (wave >> 2)) & 1) * 2 : wave < 4 ? wave : 7 - wave;
   const int n = p.cidx[2 * chunk], it = p.cidx[2 * chunk + 1];
   const int bos = p.cu[n], eos = p.cu[n + 1];
   const int c0 = bos + it * BT;
   const int rows = (eos - c0) < BT ? (eos - c0) : BT;
   const float cs = p.scale * LOG2E;
+  // One block per wave: the window's scores are scaled as they leave the products, by csw > 0; the sign of the scale is the queries',
+  // and where it is 0 they are.  Two: the queries are scaled, and rounded, before them.
+  constexpr bool RAW = RQB == 1;
+  const float csw = cs == 0.f ? LOG2E : fabsf(cs);
+  const uint32_t qkeep = cs == 0.f ? 0u : ~0u, qsign = cs < 0.f ? 0x80008000u : 0u;
   const int64_t cg = (int64_t)chunk * H + h;
   int exact = 0;   // 16-row blocks of the chunk that decay too fast for the split decay (flags of the state pass)
   if constexpr (!SINK) exact = p.flags[cg * 4] | p.flags[cg * 4 + 1] | p.flags[cg * 4 + 2] | p.flags[cg * 4 + 3];
@@ -216,7 +222,7 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   // ---- requests, in the order of their first use: the query fragments and unit 0 (first scores), then the other
   //      first units.  A CU serves the loads of its waves in the order they were issued: the barrier keeps the
   //      other units of the early waves from queueing in front of the last wave's queries and unit 0 ----
-  // the wave's 32 query rows, whole lines into the room of the slot operands (which are requested once they have been read);
+  // the wave's query rows, whole lines into the room of the slot operands (which are requested once they have been read);
   // rows past the end of the sequence read its last row and are zeroed afterwards
   const uint32_t qtile = (uint32_t)(C::QT + wave * UB);
 #pragma unroll
@@ -242,7 +248,7 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   NHA_FENCE();
 
   const uint32_t kaddr = LineTile<D>::row_at(lane), vaddr = LineTile<D>::col_at(lane);
-  // window-query fragments, pre-scaled by scale * log2(e): scores come out of the matrix core in the
+  // window-query fragments, pre-scaled by scale * log2(e) unless RAW: scores come out of the matrix core in the
   // units the exponential wants
   bf16x8 qs[RQB][KS];
 #pragma unroll
@@ -252,6 +258,11 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
     for (int ks = 0; ks < KS; ++ks) {
       u32x4 x = *reinterpret_cast<const NHA_LDS u32x4*>(lds + qtile + kaddr + qb * HB + ks * 1024);
       if (irow >= rows) x = (u32x4){0u, 0u, 0u, 0u};
+      if constexpr (RAW) {
+        x = (x & qkeep) ^ qsign;
+        qs[qb][ks] = __builtin_bit_cast(bf16x8, x);
+        continue;
+      }
       const uint32_t w[4] = {x[0], x[1], x[2], x[3]};
       bf16x8 r;
 #pragma unroll
@@ -388,6 +399,10 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
         Sc[1][qb] = mfma16(a1, qs[qb][ks], Sc[1][qb]);
       }
     }
+    if constexpr (RAW) {
+      Sc[0][0] *= csw;
+      Sc[1][0] *= csw;
+    }
     mask_unit(Sc, 0);   // unit 0 is always an edge unit
     float rmax[RQB];
     bool need = false;
@@ -428,9 +443,17 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
       q[ks] = as_bf16x8(x);
     }
   };
-  // exponentials of the current unit's block for contraction step ks, element j (see phase A)
+  // exponentials of the current unit's blocks, an equal share for each score product (contraction step ks, number j; see phase A)
+  constexpr int SJ = 2 * RQB;   // score products of a contraction step
   auto exp_step = [&](int ks, int j) {
-    if (KS == 4) {
+    if (RQB == 1) {
+#pragma unroll
+      for (int x = 0; x < 4 / KS; ++x) {
+        const int e = (2 * ks + j) * (4 / KS) + x;
+        Sc[e >> 2][0][e & 3] = fexp2(Sc[e >> 2][0][e & 3]);
+        NHA_PIN(Sc[e >> 2][0][e & 3]);
+      }
+    } else if (KS == 4) {
       Sc[ks & 1][ks >> 1][j] = fexp2(Sc[ks & 1][ks >> 1][j]);
       NHA_PIN(Sc[ks & 1][ks >> 1][j]);
     } else {
@@ -459,11 +482,12 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < SJ; ++j) {
         const int kk = j & 1, qb = j >> 1;
-        // DB / (4 KS) = 1/2 V fragment per score product
-        if ((j & 1) == 0) vf[2 * ks + (j >> 1)] = vfrag(v_c, 2 * ks + (j >> 1));
-        Sn[kk][qb] = mfma16(kf[ks][kk], qs[qb][ks], ks == 0 ? nmv[qb] : Sn[kk][qb]);
+        // two V fragments per contraction step
+        if (RQB == 1) vf[2 * ks + j] = vfrag(v_c, 2 * ks + j);
+        else if ((j & 1) == 0) vf[2 * ks + (j >> 1)] = vfrag(v_c, 2 * ks + (j >> 1));
+        Sn[kk][qb] = mfma16(kf[ks][kk], qs[qb][ks], ks == 0 ? (RAW ? (f32x4){0.f, 0.f, 0.f, 0.f} : nmv[qb]) : Sn[kk][qb]);
         // a score block of the current unit per contraction step: with KS = 4 block (ks & 1, ks >> 1),
         // with KS = 2 blocks (0, ks) and (1, ks)
         exp_step(ks, j);
@@ -515,7 +539,9 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int qb = 0; qb < RQB; ++qb) Sc[kk][qb] = Sn[kk][qb];
+      for (int qb = 0; qb < RQB; ++qb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Sc[kk][qb][r] = RAW ? Sn[kk][qb][r] * csw + nm[qb] : Sn[kk][qb][r];
   }
   // ---- the last unit: no further scores; the slot-branch queries of the first query block are
   //      requested into the registers the window queries leave ----
@@ -529,7 +555,7 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) exp_step(ks, j);
+      for (int j = 0; j < SJ; ++j) exp_step(ks, j);
     bf16x8 Pq[RQB];
     pack_p(Pq);
 #pragma unroll
@@ -816,7 +842,7 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
       if (irow < rows) *reinterpret_cast<uint4*>(op + dcol) = make_uint4(a[0], a[1], b[0], b[1]);
     }
   }
-  // ---- rows that have to be formed again, for the four heads of the workgroup -----------------------
+  // ---- rows that have to be formed again, for the heads of the workgroup -----------------------
   if constexpr (SINK) {
     lds_barrier();
 #pragma unroll
@@ -826,38 +852,47 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   if (exact == 0) return;
   before_exact();
   if constexpr (SINK) sink_exact_rows<D>(arguments_again(), reinterpret_cast<float*>(smem_), chunk, h, h * NG + grp * 4, exact);
-  else exact_rows<D, 2>(arguments_again(), reinterpret_cast<float*>(smem_), chunk, h, h * NG + grp * 4, 4, exact);
+  else exact_rows<D, 2>(arguments_again(), reinterpret_cast<float*>(smem_), chunk, h, h * NG + grp * HEADS, HEADS, exact);
 }
 
-template <int D, bool SINK>
+template <int D, bool SINK, int RQB>
 int launch_ring(const MP& p, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   // the window-only launch has no slot operands: the ring and the eight waves' window queries behind it (128 KB at D = 128, 96 at
   // 64; its registers leave room for one workgroup per CU as well)
   const size_t lds = SINK ? (size_t)(RingCfg<D>::QT + 8 * RingCfg<D>::UB) : (size_t)RingCfg<D>::BYTES;
-  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring_out_kernel<D, SINK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring_out_kernel<D, SINK, RQB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_fwd(mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL((ring_out_kernel<D, SINK>), dim3(p.H * (p.NG / 4), p.NT), dim3(512), lds, st, p);
+  hipLaunchKernelGGL((ring_out_kernel<D, SINK, RQB>), dim3(p.H * (p.NG / (2 * RQB)), p.NT), dim3(512), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma output pass, ring)");
   return NHA_OK;
 }
 
 }  // namespace
 
-// Served: four (or a multiple of four) query heads per kv-head at D = 64 or 128.  The per-lane byte
-// offsets of the LDS-direct loads are 32 bits: the tensors of one sequence must stay below 4 GiB, which
+// Served: a multiple of four query heads per kv-head at D = 64, an even number at 128.  us, 8 / 4 heads of 128, mfma_out_kernel (and
+// the launch after it from 2500 tokens) / this: 300 tokens 15.9 / 13.7, 2 x 1500, W = 400 28 / 23, 2 x 2500 49 / 41, 4000 packed, W = 200
+// 38 / 29, 2 x 3500, W = 2000 90 / 76, 4 x 8192, W = 64 147 / 126, W = 1000 290 / 276; at 64 (1500 tokens, W = 500 18.6 / 16.6, 4 x
+// 8192, W = 1500 197 / 207) mfma_out_kernel keeps them: its running maximum is 2 to 4 % nearer to 64 bits where single logits dominate.
+// The per-lane byte offsets of the LDS-direct loads are 32 bits: the tensors of one sequence must stay below 4 GiB, which
 // the caller's 32-bit token count times the row size decides.
 bool prefill_ring_supported(const mf::MP& p, int D) {
-  if (!(D == 64 || D == 128) || p.NG % 4 != 0) return false;
+  if (!(D == 64 && p.NG % 4 == 0) && !(D == 128 && p.NG % 2 == 0)) return false;
   return (int64_t)p.T_tot * p.H * D * 2 < ((int64_t)1 << 32) && (int64_t)p.T_tot * p.H * MS * 2 < ((int64_t)1 << 32);
 }
 
+// One 16-row block per wave, a workgroup two heads: where a kv-head's heads are no multiple of four, and where all of these workgroups
+// have a place at once.  us, two blocks / one: 8 / 2 heads of 128, 95 tokens 16.3 / 13.0; 32 / 4, 331, W = 64 18.2 / 14.5, 525, W = 950
+// 27.3 / 21.0; 32 / 8, 1000, W = 1000 (256 workgroups) 39.3 / 29.4; 16 / 4 heads of 64, 2000, W = 1000 32.2 / 25.2.
+static bool rows_alone(const mf::MP& p) { return p.NG % 4 != 0 || (int64_t)p.HQ / 2 * p.NT <= 256; }
+
 int prefill_ring_launch(const mf::MP& p, int D, hipStream_t st) {
-  return D == 64 ? launch_ring<64, false>(p, st) : launch_ring<128, false>(p, st);
+  if (rows_alone(p)) return D == 64 ? launch_ring<64, false, 1>(p, st) : launch_ring<128, false, 1>(p, st);
+  return D == 64 ? launch_ring<64, false, 2>(p, st) : launch_ring<128, false, 2>(p, st);
 }
 
 // Sliding-window attention with zero sinks (nha_sink_window_fwd): the window loop of ring_out_kernel alone.  (What
@@ -872,13 +907,13 @@ int sink_window_impl(const NhaSinkWindowArgs* a) {
   p.cu = a->cu_seqlens; p.cidx = a->chunk_indices; p.coff = a->chunk_offsets;
   p.T_tot = a->T_tot; p.N = a->N; p.NT = a->NT; p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H;
   p.wl = a->window - 1; p.shift = 0; p.scale = a->scale; p.sinks = a->sinks;
-  if (a->dtype != NHA_DTYPE_BF16 || !prefill_ring_supported(p, a->D) || p.NT > 65535) {
+  if (a->dtype != NHA_DTYPE_BF16 || p.NG % 4 != 0 || !prefill_ring_supported(p, a->D) || p.NT > 65535) {
     set_error("nha_sink_window_fwd: built for bf16, head size 64 or 128, a multiple of four query heads per kv-head, "
               "at most 65535 chunks and tensors below 4 GiB (dtype=%d D=%d HQ/H=%d NT=%d)", a->dtype, a->D, p.NG, p.NT);
     return NHA_ERR_UNSUPPORTED;
   }
   hipStream_t st = (hipStream_t)a->stream;
-  return a->D == 64 ? launch_ring<64, true>(p, st) : launch_ring<128, true>(p, st);
+  return a->D == 64 ? launch_ring<64, true, 2>(p, st) : launch_ring<128, true, 2>(p, st);
 }
 
 }  // namespace nha

@@ -265,3 +265,22 @@ def test_mfma_layer_workloads_match_c_oracle(name):
                      ("hk", got[3][0], ref[3]), ("hv", got[3][1], ref[4])):
         rel = ((a.double().cpu() - b.double()).norm() / b.double().norm()).item()
         assert rel <= 5e-3, f"{nm}: relative L2 error {rel:.3e}"
+
+
+@pytest.mark.parametrize("H,NG,D", [(18, 4, 128), (16, 4, 128), (9, 8, 64), (8, 8, 64), (2, 2, 128), (33, 2, 128), (3, 6, 128)])
+@pytest.mark.parametrize("scale", [1.0, -1.0, 0.0])
+@pytest.mark.parametrize("wl", [-1, 0, 64, 200])
+def test_ring_one_and_two_row_blocks_per_wave(H, NG, D, scale, wl):
+    """Eight chunks: 72 query heads are the first multiple of four whose workgroups take four heads each, 64 the last with two; two and six
+    heads per kv-head always take two.  Sequences that end inside a row block, scales of both signs and zero, against the generic fp32
+    kernels on the same bf16-rounded inputs: probabilities and outputs rounded to bf16, 1e-2 in relative L2."""
+    from nha_amd import chunk_nha
+    from tests.test_gpu_prefill_bwd import check_grad
+    print("case", H, NG, D, scale, wl, flush=True)
+    cu = torch.tensor([0, 1, 40, 104, 361], dtype=torch.int32).cuda()
+    d = prefill_inputs(880 + D + NG, 1, 361, H * NG, H, D, D, 64, dtype=BF, with_state=True, N=4)
+    h0 = tuple(x.cuda() for x in d["h0"])
+    res = [chunk_nha(*(d[k].cuda().to(dt) for k in KEYS), cu_seqlens=cu, scale=scale * D ** -0.5, window_size_left=wl, gsa_kv_shift=16,
+                     initial_state=h0, impl=impl)[:3] for dt, impl in ((BF, "mfma"), (torch.float32, "simple"))]
+    for name, got, ref in zip(("o", "lse_swa", "lse_gsa"), *res):
+        check_grad(name, got, ref.double().cpu(), BF)
