@@ -62,6 +62,9 @@ constexpr int LPW = 2;                // LDS-direct loads per wave and unit (16 
 constexpr int BYTES = NRU * UNIT;
 constexpr int RQB = 2;                // 16-row query blocks per wave
 
+// RAW: the forward of the call formed its scores from queries that were not scaled, and rounded, before the products (ring_out_kernel with
+// one 16-row block per wave), and so do these: with rounded ones dq of calls of strong logits was up to a sixth further from 64 bits.
+template <bool RAW>
 __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
   extern __shared__ __align__(1024) unsigned char smem_[];
   lbyte* const lds = (lbyte*)smem_;
@@ -109,7 +112,7 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
   for (int u = 0; u < NRU - 2; ++u)
     if (u < nunits) issue_unit(u);
 
-  // query-side fragments: q pre-scaled by scale * log2(e) (the rounding the forward's scores saw), do as it is.  The rows come in
+  // query-side fragments: q pre-scaled by scale * log2(e) unless RAW (the rounding the forward's scores saw), do as it is.  The rows come in
   // whole lines, as 1 KB blocks of 16 rows x 32 columns (a fragment as it lies in memory, 16 bytes of 16 rows, takes three
   // times as long to load), and are put into fragment order through the two ring slots that no unit has been requested into.
   uint4 qraw[RQB][KS], draw[RQB][KS];
@@ -146,7 +149,7 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
         const float f = __uint_as_float((e & 1) ? (x[e >> 1] & 0xffff0000u) : (x[e >> 1] << 16));
         r[e] = (__bf16)(f * cs);
       }
-      qf[qb][ks] = r;
+      qf[qb][ks] = RAW ? __builtin_bit_cast(bf16x8, x) : r;
       df[qb][ks] = __builtin_bit_cast(bf16x8, turned(draw[qb][ks], (2 * ks + 1) & 3) & on);
     }
     float ls = 0.f, lg = 0.f;
@@ -195,7 +198,10 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
   auto columns = [&](uint32_t a) { return Frags{{tfrag(a, 0), tfrag(a, 1)}}; };
   auto scores = [&](Unit& t, uint32_t base, const Frags& first, auto beside, auto tail) {   // S = K Q^T - lse
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) t.S[q] = (f32x4){nlse[q & 1], nlse[q & 1], nlse[q & 1], nlse[q & 1]};
+    for (int q = 0; q < NQ; ++q) {
+      const float from = RAW ? 0.f : nlse[q & 1];
+      t.S[q] = (f32x4){from, from, from, from};
+    }
     Frags ka[KS];
     ka[0] = first;
 #pragma unroll
@@ -211,6 +217,11 @@ __global__ __launch_bounds__(512, 1) void ring_dq_kernel(const DqP p) {
     __builtin_amdgcn_sched_barrier(0);
   };
   auto mask = [&](Unit& t, int u) {
+    if constexpr (RAW)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t.S[q][r] = t.S[q][r] * cs + nlse[q & 1];
     if (!is_edge(u)) return;
     const int xbase = 32 - 32 * u;
 #pragma unroll
@@ -768,12 +779,17 @@ int bwd_ring_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld) {
   p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H; p.NT = a->NT; p.wl = a->wl; p.scale = a->scale;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)ring_dq_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, BYTES); });
+  std::call_once(once, [&] {
+    attr_err = hipFuncSetAttribute((const void*)ring_dq_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);
+    if (attr_err == hipSuccess) attr_err = hipFuncSetAttribute((const void*)ring_dq_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);
+  });
   if (attr_err != hipSuccess) {
     set_error("nha_prefill_bwd: cannot reserve %d bytes of LDS: %s", BYTES, hipGetErrorString(attr_err));
     return NHA_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL(ring_dq_kernel, dim3(p.H * (p.NG / 4), p.NT), dim3(512), BYTES, (hipStream_t)a->stream, p);
+  const dim3 grid(p.H * (p.NG / 4), p.NT);
+  if (prefill_ring_raw(a->HQ, a->H, a->NT)) hipLaunchKernelGGL(ring_dq_kernel<true>, grid, dim3(512), BYTES, (hipStream_t)a->stream, p);
+  else hipLaunchKernelGGL(ring_dq_kernel<false>, grid, dim3(512), BYTES, (hipStream_t)a->stream, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(window dq, ring)");
   return NHA_OK;
 }
