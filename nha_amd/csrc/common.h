@@ -186,7 +186,7 @@ int bwd_ring256_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld);
 int bwd_ring256_dkv_parts(const NhaPrefillBwdArgs* a);
 int bwd_ring256_dkv(const NhaPrefillBwdArgs* a, const float2* ld, const float* dvs, int parts, float* wk, float* wv);
 // parts > 1 (bwd_window_mfma_parts at most, the LDS-direct kernels only): a kv-head's query heads in as many parts, whose fp32 sums go to
-// wk and wv, all of one part and then the next; dk_swa and dv are left to whom it may concern
+// wk and wv, all of one part and then the next; dk_swa and dv are left to the last pass of the gates
 int bwd_window_mfma_parts(const NhaPrefillBwdArgs* a);
 int bwd_window_mfma_dkv(const NhaPrefillBwdArgs* a, const float* delta, const float* dvs, const void* ld, int parts, float* wk, float* wv);
 

@@ -1,5 +1,5 @@
-"""Window gradients from the LDS-direct kernels (K = V = 128: four or eight query heads per kv-head, more key groups than 128;
-K = V = 256: any grouping, more than 256 chunks x kv-heads, few empty halves of 128-row workgroups) against the fp32 call (generic
+"""Window gradients from the LDS-direct kernels (K = V = 128: a multiple of four query heads per kv-head; K = V =
+256: any grouping, more than 256 chunks x kv-heads or query heads to share out, few empty halves of 128-row workgroups) against the fp32 call (generic
 kernels) on the same bf16-rounded inputs: ragged packed sequences that end inside a 32-row unit, a chunk and a group of chunks,
 windows below and above those where the kernels and their key groups change, odd and even numbers of units, longer than every
 sequence and unbounded."""
