@@ -252,7 +252,7 @@ int bwd_slot_branch(const NhaPrefillBwdArgs* a, const mf::MP& m, float* delta, f
 // output pass with LDS-direct window loads (prefill_ring.hip); false when the shape is not served
 bool prefill_ring_supported(const mf::MP& p, int D);
 int prefill_ring_launch(const mf::MP& p, int D, hipStream_t st);
-bool prefill_ring_raw(int HQ, int H, int NT);   // whether its queries are not scaled before the products
+bool prefill_ring_raw(int HQ, int NT);   // whether its queries are not scaled before the products
 
 // the same for head size 256, one query head per workgroup (prefill_ring256.hip)
 bool prefill_ring256_supported(const mf::MP& p, int D);

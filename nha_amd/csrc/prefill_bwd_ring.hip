@@ -788,7 +788,7 @@ int bwd_ring_dq(const NhaPrefillBwdArgs* a, const float* delta, float2* ld) {
     return NHA_ERR_LAUNCH;
   }
   const dim3 grid(p.H * (p.NG / 4), p.NT);
-  if (prefill_ring_raw(a->HQ, a->H, a->NT)) hipLaunchKernelGGL(ring_dq_kernel<true>, grid, dim3(512), BYTES, (hipStream_t)a->stream, p);
+  if (prefill_ring_raw(a->HQ, a->NT)) hipLaunchKernelGGL(ring_dq_kernel<true>, grid, dim3(512), BYTES, (hipStream_t)a->stream, p);
   else hipLaunchKernelGGL(ring_dq_kernel<false>, grid, dim3(512), BYTES, (hipStream_t)a->stream, p);
   NHA_CHECK_LAUNCH("nha_prefill_bwd(window dq, ring)");
   return NHA_OK;

@@ -1245,8 +1245,8 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
     // (D = 64) workgroups per CU, which 64-key tiles or decay fragments in LDS do not leave room for:
     // 16 heads, 8192 tokens, W = 2048: D = 64 291 -> 147 us, D = 128 434 -> 269 us (with 64-key tiles 165, 375);
     // 5003 packed tokens, W = 300: 93 -> 46, 119 -> 70.  G = 2: where there is more than a workgroup for
-    // every CU, two fit one as well (8 / 4 heads of 64, 4 x 8000 tokens, W = 1500: 244 -> 198); below, one with the
-    // fragments shared is faster (3000 tokens, 188 workgroups: 17.5 against 19).
+    // every CU, two fit one as well (8 / 4 heads, 4 x 8000 tokens, W = 1500: D = 128 378 -> 330-353 us, with 32-key tiles; D = 64
+    // 244 -> 198); below, one with the fragments shared is faster (3000 tokens, 188 workgroups: 25 against 31, 17.5 against 19)
     int rc;
     bool exact = false;   // the output pass has formed the flagged rows itself
 #ifdef NHA_AB_SWITCHES   // measurement builds only (-DNHA_AB_SWITCHES): run the kernels the LDS-direct ones replaced
@@ -1258,10 +1258,9 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
     if (!ring_off && prefill_ring256_supported(p, D)) return prefill_ring256_launch(p, st);
     if constexpr (D <= 128) {
       if (p.NG % 4 == 0) rc = launch_out<D, 4, 8, 64, false>(p, &exact, st);
-      else if (p.NG % 2 != 0) rc = launch_out<D, 1, 4, 32, true>(p, &exact, st);
-      else if constexpr (D == 128) rc = launch_out<D, 2, 8, 32, true>(p, &exact, st);   // (tensors of 4 GiB)
-      else if ((int64_t)p.HQ / 2 * p.NT > 256) rc = launch_out<D, 2, 8, 64, true>(p, &exact, st);
-      else rc = launch_out<D, 2, 8, 64, false>(p, &exact, st);
+      else if (p.NG % 2 == 0 && (int64_t)p.HQ / 2 * p.NT > 256) rc = launch_out<D, 2, 8, D == 128 ? 32 : 64, true>(p, &exact, st);
+      else if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 64, false>(p, &exact, st);
+      else rc = launch_out<D, 1, 4, 32, true>(p, &exact, st);
     } else {
       if (p.NG % 2 == 0) rc = launch_out<D, 2, 8, 32, false>(p, &exact, st);
       else rc = launch_out<D, 1, 4, 32, true>(p, &exact, st);

@@ -1,4 +1,4 @@
-// Output pass of the bf16 matrix-core prefill for groups of four query heads per kv-head, or of two (K == V == D
+// Output pass of the bf16 matrix-core prefill for groups of four query heads per kv-head (K == V == D
 // in {64, 128}, M == 64): same mathematics as mfma_out_kernel (prefill_mfma.hip; chunk algebra of
 // nha_fla/ops/nha/chunk_fused.py:186-283, one softmax over [slots | window] as in
 // nha_fla/ops/nha/chunk.py:459-470), different data movement and order.
@@ -12,7 +12,7 @@
 //  * The window loop is software-pipelined inside each wave: while the matrix core forms the scores
 //    of unit u+1, the VALU exponentiates unit u.  The scale and the softmax reference are folded into
 //    the score product itself (pre-scaled queries, accumulator started at -reference), so a score
-//    needs one v_exp_f32 and half a v_cvt_pk_bf16_f32 and nothing else (groups of two: a multiplication too, on unrounded queries).
+//    needs one v_exp_f32 and half a v_cvt_pk_bf16_f32 and nothing else (two heads per workgroup: a multiplication too, on unrounded queries).
 //  * The softmax reference of a query row is fixed once, from the first unit (the row's own and
 //    nearest keys; 0 for rows that unit does not reach): fp32 sums relative to a fixed reference are
 //    exact while every score stays within 2^+-100 of it, and the loop carries no maxima, no
@@ -882,24 +882,23 @@ int launch_ring(const MP& p, hipStream_t st) {
 
 }  // namespace
 
-// Served: a multiple of four query heads per kv-head at D = 64, an even number at 128.  us, 8 / 4 heads of 128, mfma_out_kernel (and
-// the launch after it from 2500 tokens) / this: 300 tokens 15.9 / 13.7, 2 x 1500, W = 400 28 / 23, 2 x 2500 49 / 41, 4000 packed, W = 200
-// 38 / 29, 2 x 3500, W = 2000 90 / 76, 4 x 8192, W = 64 147 / 126, W = 1000 290 / 276; at 64 (1500 tokens, W = 500 18.6 / 16.6, 4 x
-// 8192, W = 1500 197 / 207) mfma_out_kernel keeps them: its running maximum is 2 to 4 % nearer to 64 bits where single logits dominate.
+// Served: four (or a multiple of four) query heads per kv-head at D = 64 or 128.  Groups of two and six stay with mfma_out_kernel, whose
+// reference is the maximum of the slots and then follows the window's: where single logits dominate it is nearer to 64 bits (logits of
+// std 4, 8 / 4 heads, 54 calls of 300 to 3000 tokens: o 2 to 3 % at D = 128, 2 to 4 % at 64, the window's log-sum-exp 30 to 50 %), for
+// which the kernel here is 5 to 15 % faster (8 / 4 heads of 128, 4 x 8192 tokens, W = 64 147 / 126 us, W = 1000 290 / 276).
 // The per-lane byte offsets of the LDS-direct loads are 32 bits: the tensors of one sequence must stay below 4 GiB, which
 // the caller's 32-bit token count times the row size decides.
 bool prefill_ring_supported(const mf::MP& p, int D) {
-  if (!(D == 64 && p.NG % 4 == 0) && !(D == 128 && p.NG % 2 == 0)) return false;
+  if (!(D == 64 || D == 128) || p.NG % 4 != 0) return false;
   return (int64_t)p.T_tot * p.H * D * 2 < ((int64_t)1 << 32) && (int64_t)p.T_tot * p.H * MS * 2 < ((int64_t)1 << 32);
 }
 
-// One 16-row block per wave, a workgroup two heads: where a kv-head's heads are no multiple of four, and where all of these workgroups
-// have a place at once.  us, two blocks / one: 8 / 2 heads of 128, 95 tokens 16.3 / 13.0; 32 / 4, 331, W = 64 18.2 / 14.5, 525, W = 950
+// One 16-row block per wave, a workgroup two heads: where all of these workgroups have a place at once.  us, two blocks / one: 8 / 2 heads of 128, 95 tokens 16.3 / 13.0; 32 / 4, 331, W = 64 18.2 / 14.5, 525, W = 950
 // 27.3 / 21.0; 32 / 8, 1000, W = 1000 (256 workgroups) 39.3 / 29.4; 16 / 4 heads of 64, 2000, W = 1000 32.2 / 25.2.
-bool prefill_ring_raw(int HQ, int H, int NT) { return HQ / H % 4 != 0 || (int64_t)HQ / 2 * NT <= 256; }
+bool prefill_ring_raw(int HQ, int NT) { return (int64_t)HQ / 2 * NT <= 256; }
 
 int prefill_ring_launch(const mf::MP& p, int D, hipStream_t st) {
-  if (prefill_ring_raw(p.HQ, p.H, p.NT)) return D == 64 ? launch_ring<64, false, 1>(p, st) : launch_ring<128, false, 1>(p, st);
+  if (prefill_ring_raw(p.HQ, p.NT)) return D == 64 ? launch_ring<64, false, 1>(p, st) : launch_ring<128, false, 1>(p, st);
   return D == 64 ? launch_ring<64, false, 2>(p, st) : launch_ring<128, false, 2>(p, st);
 }
 
@@ -915,7 +914,7 @@ int sink_window_impl(const NhaSinkWindowArgs* a) {
   p.cu = a->cu_seqlens; p.cidx = a->chunk_indices; p.coff = a->chunk_offsets;
   p.T_tot = a->T_tot; p.N = a->N; p.NT = a->NT; p.HQ = a->HQ; p.H = a->H; p.NG = a->HQ / a->H;
   p.wl = a->window - 1; p.shift = 0; p.scale = a->scale; p.sinks = a->sinks;
-  if (a->dtype != NHA_DTYPE_BF16 || p.NG % 4 != 0 || !prefill_ring_supported(p, a->D) || p.NT > 65535) {
+  if (a->dtype != NHA_DTYPE_BF16 || !prefill_ring_supported(p, a->D) || p.NT > 65535) {
     set_error("nha_sink_window_fwd: built for bf16, head size 64 or 128, a multiple of four query heads per kv-head, "
               "at most 65535 chunks and tensors below 4 GiB (dtype=%d D=%d HQ/H=%d NT=%d)", a->dtype, a->D, p.NG, p.NT);
     return NHA_ERR_UNSUPPORTED;
