@@ -317,12 +317,10 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
 #pragma unroll
   for (int qb = 0; qb < RQB; ++qb) {
     Lw[qb] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    // RAW: just above zero, so that the probabilities of small scores lie below 1 and not around it, where bf16 is half as fine (8 / 4
-    // heads, 1500 tokens, scores of 1e-2: relative error of the output 2.61e-3 with 0, 2.25e-3 like this, 2.24e-3 with the row's maximum).
-    // The probability of a score of 0 is a bf16 number, and its logarithm what the log-sum-exp below subtracts.
-    float one = 0x1.eap-1f;   // 245 / 256
-    asm volatile("" : "+v"(one));
-    nm[qb] = RAW ? __builtin_amdgcn_logf(one) : 0.f;
+    // Zero, also where the queries are not scaled beforehand.  245/256 there, below which the probabilities of small scores stay (bf16 is
+    // half as fine above 1), took 4 to 8 % off the output's error for some gates and added 1 to 2 % for gates that forget within a few
+    // tokens (scores of std 0.1, 54 calls of 331 to 1000 tokens: 2.31e-3 -> 2.35e-3); with zero it is nowhere above pre-scaled queries'.
+    nm[qb] = 0.f;
     nmv[qb] = (f32x4){0.f, 0.f, 0.f, 0.f};
   }
   bf16x8 ones;

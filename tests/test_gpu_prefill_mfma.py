@@ -301,3 +301,21 @@ def test_strong_logits_of_two_and_six_heads(HQ, H, lens, wl):
         rel = ((got[1] - ref[1]).norm() / ref[1].norm()).item()
         print("log-sum-exp", HQ, H, lens, rel, flush=True)
         assert rel < bound
+
+
+@pytest.mark.parametrize("HQ,H,D,lens,wl,qk", [(32, 4, 128, [1000], 300, 0.3), (32, 4, 128, [331], 63, 0.3), (16, 4, 64, [331], 63, 0.2)])
+def test_small_logits_and_fast_gates_of_small_calls(HQ, H, D, lens, wl, qk):
+    """Small calls of four heads per kv-head, window logits around zero, gates that forget within a few tokens: where the softmax
+    reference lies decides how finely bf16 holds the probabilities.  Mean relative error of the output against fp32 over four seeds, with a reference
+    of 0 / of log2(245/256): 2.307e-3 / 2.339e-3, 2.300e-3 / 2.335e-3, 2.298e-3 / 2.342e-3; the bound lies between."""
+    from nha_amd import chunk_nha
+    cu = torch.tensor([0, *itertools.accumulate(lens)], dtype=torch.int32).cuda()
+    errors = []
+    for seed in range(4):
+        d = prefill_inputs(7200 + seed, 1, sum(lens), HQ, H, D, D, 64, dtype=BF, gate_div=1.0, gate_mean=-1.0, qk_scale=qk)
+        d["v"] = (d["v"].float() / qk).to(BF)
+        got, ref = (chunk_nha(*(d[k].cuda().to(dt) for k in KEYS), cu_seqlens=cu, window_size_left=wl, impl=impl)[0].double()
+                    for dt, impl in ((BF, "mfma"), (torch.float32, "simple")))
+        errors.append(((got - ref).norm() / ref.norm()).item())
+    print("output", HQ, H, D, lens, errors, flush=True)
+    assert sum(errors) / 4 < 2.32e-3
