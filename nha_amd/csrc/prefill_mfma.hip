@@ -73,6 +73,15 @@ __device__ __forceinline__ void tile_r2l(lbf16* lds, const TileRegs<ROWS, D, NTH
 
 // DW: columns of the state one workgroup carries (D, or D/2: twice the workgroups with half the
 // tile, which this latency-bound kernel turns into bandwidth; the gates are then read once more).
+template <int D> constexpr int LOCAL_DW = D >= 256 ? D / 2 : D;   // measured: 96 -> 88 us at B=8 T=2048 H=4 D=256; no gain at D = 128
+
+// What state_link_kernel may not leave out although the decays after it multiply to zero: initial and end states that are not finite, or not
+// far below fp32's limit, and segments that grow.  A word per (segment slot, kv-head, state and column range of level 1, 16 slots), where
+// the scan, if it follows instead, leaves its segment-start states.
+__device__ __forceinline__ unsigned magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }   // (NaNs count too: this file is built without them)
+constexpr unsigned ODD_STATE = 0x5f800000u;   // 2^64
+__device__ __forceinline__ int* odd_words(const MP& p) { return (int*)p.hseg_k; }
+
 template <int D, int DW>
 __global__ __launch_bounds__(256) void mfma_state_local_kernel(const MP p) {
   constexpr int LDT = DW + 16;
@@ -280,12 +289,32 @@ __global__ __launch_bounds__(256) void mfma_state_local_kernel(const MP p) {
       hx[b] = mfma16(lds_frag_tr(Xt, LDT, 32, 48, 16 * b, lane), sg1, hx[b]);
     }
   }
+  // the initial state's part of the first segment's word: this wave's 16 slots and the workgroup's columns of it
+  unsigned most = 0;
+  if (kseg == 0 && p.h0k) {
+    const int64_t nh = (int64_t)n * H + h;
+    const float* const src = isv ? p.h0v + (nh * MS + 16 * wave) * D + dcol0 : p.h0k + (nh * D + dcol0) * MS + 16 * wave;
+    constexpr int VL = DW / 4;   // lanes to a row of the v-state
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int e = lane + 64 * i;
+      const float4 x = *reinterpret_cast<const float4*>(src + (isv ? e / VL * D + e % VL * 4 : e / 4 * MS + e % 4 * 4));
+      most = max(most, max(max(magnitude(x.x), magnitude(x.y)), max(magnitude(x.z), magnitude(x.w))));
+    }
+  }
   // segment end: local state (fp32, [m][d]) and total decay
   const int64_t sl = (int64_t)seg_slot(p.coff, n, it0, p.seg_sh) * H + h;
 #pragma unroll
   for (int b = 0; b < NB; ++b)
     *reinterpret_cast<float4*>(hend + (sl * MS + m) * D + dcol0 + 16 * b + 4 * kb) = make_float4(hx[b][0], hx[b][1], hx[b][2], hx[b][3]);
-  if (kb == 0 && !isv && lead) p.dtot[sl * MS + m] = fexp(gsum);
+  const float dt = fexp(gsum);
+  if (kb == 0 && !isv && lead) p.dtot[sl * MS + m] = dt;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) most = max(most, magnitude(hx[b][r]));
+  const int odd = __any(most >= ODD_STATE || magnitude(dt) > __float_as_uint(1.f));
+  if (lane == 0) odd_words(p)[(sl * Z + z) * 4 + wave] = odd;
 }
 
 // Level 2, the scan: four consecutive d of one slot per thread, sequential over the segments of its sequence;
@@ -466,6 +495,8 @@ __device__ __forceinline__ void segment_of(const MP& p, int slot, int& n, int& i
 // 43 -> 28 us; 2 x 8192 tokens, 8 heads of 128 (16 segments each) 30.5 -> 24.5; 331 tokens, 4 heads of 128 7.3 -> 4.
 // Gates that never decay read every end state before their own: as fast as the scan at 16 segments (2 x 8192 tokens, W = 64: call
 // 246 -> 244 us), slower at 32 (476 -> 482; gates of the layers 478 -> 467) and at 64 (481 -> 505), so longer sequences keep the scan.
+// An infinity or a NaN of an earlier segment, or of the initial state, reaches every later one whatever lies between, as it does token
+// by token: where there is one (odd_words), the segments are walked in their order as the scan walks them.
 // One-dimensional grid (segment slots, H, StatePart's groups), the groups fastest: there are 8, 16 or 32 of them, so the segments that
 // read the same part of an end state are on one XCD.
 template <int D>
@@ -495,8 +526,12 @@ __global__ __launch_bounds__(256) void state_link_kernel(const MP p) {
     own = *reinterpret_cast<const float4*>(hend + (int64_t)slot * H * MS * D);
     own_dt = dtot[(int64_t)slot * H * MS];
   }
-  float hs[4] = {0.f, 0.f, 0.f, 0.f}, dec = 1.f;
   const int first = slot - (it0 >> p.seg_sh);
+  // (the first segment itself, which has none before it, reads its own word: the walk below is the same either way)
+  constexpr int Z = 2 * (D / LOCAL_DW<D>);
+  const int* const words = odd_words(p) + (((int64_t)first * H + h) * Z + 2 * (d / LOCAL_DW<D>) + (isv ? 1 : 0)) * 4 + (m >> 4);
+  int odd = words[(int64_t)max(min(tid & 63, slot - first - 1), 0) * H * Z * 4];
+  float hs[4] = {0.f, 0.f, 0.f, 0.f}, dec = 1.f;
   for (int j = slot - 1; j >= first && __any(dec != 0.f); j -= 2) {   // the loads of two segments together
     const int j1 = j > first ? j - 1 : j;
     const float4 a = *reinterpret_cast<const float4*>(hend + (int64_t)j * H * MS * D), b = *reinterpret_cast<const float4*>(hend + (int64_t)j1 * H * MS * D);
@@ -512,9 +547,20 @@ __global__ __launch_bounds__(256) void state_link_kernel(const MP p) {
       dec *= db;
     }
   }
-  if (p.h0k && __syncthreads_or(dec != 0.f)) {
-    const float4 x = isv ? *reinterpret_cast<const float4*>(p.h0v + (nh * MS + m) * D + d) : part.load_k(p.h0k + nh * D * MS, tr, tid);
-    hs[0] += x.x * dec; hs[1] += x.y * dec; hs[2] += x.z * dec; hs[3] += x.w * dec;
+  for (int i = 64 + (tid & 63); i < slot - first; i += 64) odd |= words[(int64_t)i * H * Z * 4];
+  odd = __any(odd);
+  float4 h0 = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (p.h0k && __syncthreads_or(odd || dec != 0.f)) {
+    h0 = isv ? *reinterpret_cast<const float4*>(p.h0v + (nh * MS + m) * D + d) : part.load_k(p.h0k + nh * D * MS, tr, tid);
+    hs[0] += h0.x * dec; hs[1] += h0.y * dec; hs[2] += h0.z * dec; hs[3] += h0.w * dec;
+  }
+  if (odd) {
+    hs[0] = h0.x; hs[1] = h0.y; hs[2] = h0.z; hs[3] = h0.w;
+    for (int j = first; j < slot; ++j) {
+      const float4 a = *reinterpret_cast<const float4*>(hend + (int64_t)j * H * MS * D);
+      const float da = dtot[(int64_t)j * H * MS];
+      hs[0] = hs[0] * da + a.x; hs[1] = hs[1] * da + a.y; hs[2] = hs[2] * da + a.z; hs[3] = hs[3] * da + a.w;
+    }
   }
   rw.request(hloc, (int64_t)H * MS * D, fmaxf(fmaxf(fabsf(hs[0]), fabsf(hs[1])), fmaxf(fabsf(hs[2]), fabsf(hs[3]))));
   rw.store(hloc, (int64_t)H * MS * D, hs);
@@ -1201,7 +1247,7 @@ template <int D>
 int run_state_pass(const MP& p, bool segment_form, hipStream_t st) {
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
-  constexpr int DW = D >= 256 ? D / 2 : D;   // measured: 96 -> 88 us at B=8 T=2048 H=4 D=256; no gain at D = 128
+  constexpr int DW = LOCAL_DW<D>;
   const size_t lds = (size_t)BT * (DW + 16) * 2 + (size_t)2 * BT * SLD * 2;
   std::call_once(once, [&] { attr_err = hipFuncSetAttribute((const void*)mfma_state_local_kernel<D, DW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
   if (attr_err != hipSuccess) {
