@@ -158,11 +158,9 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
   const int c0 = bos + it * BT;
   const int rows = (eos - c0) < BT ? (eos - c0) : BT;
   const float cs = p.scale * LOG2E;
-  // One block per wave: the window's scores are scaled as they leave the products, by csw > 0; the sign of the scale is the queries',
-  // and where it is 0 they are.  Two: the queries are scaled, and rounded, before them.
+  // One block per wave: the window's scores are scaled as they leave the products, and masked after that (0 times an infinity or a NaN of
+  // a query or a key is a NaN, as token by token; of a mask it must not be).  Two: the queries are scaled, and rounded, before them.
   constexpr bool RAW = RQB == 1;
-  const float csw = cs == 0.f ? LOG2E : fabsf(cs);
-  const uint32_t qkeep = cs == 0.f ? 0u : ~0u, qsign = cs < 0.f ? 0x80008000u : 0u;
   const int64_t cg = (int64_t)chunk * H + h;
   int exact = 0;   // 16-row blocks of the chunk that decay too fast for the split decay (flags of the state pass)
   if constexpr (!SINK) exact = p.flags[cg * 4] | p.flags[cg * 4 + 1] | p.flags[cg * 4 + 2] | p.flags[cg * 4 + 3];
@@ -259,7 +257,6 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
       u32x4 x = *reinterpret_cast<const NHA_LDS u32x4*>(lds + qtile + kaddr + qb * HB + ks * 1024);
       if (irow >= rows) x = (u32x4){0u, 0u, 0u, 0u};
       if constexpr (RAW) {
-        x = (x & qkeep) ^ qsign;
         qs[qb][ks] = __builtin_bit_cast(bf16x8, x);
         continue;
       }
@@ -405,8 +402,8 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
     if constexpr (RAW) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        Sc[0][0][r] = Sc[0][0][r] * csw + nm[0];
-        Sc[1][0][r] = Sc[1][0][r] * csw + nm[0];
+        Sc[0][0][r] = Sc[0][0][r] * cs + nm[0];
+        Sc[1][0][r] = Sc[1][0][r] * cs + nm[0];
       }
     }
     mask_unit(Sc, 0);   // unit 0 is always an edge unit
@@ -541,13 +538,16 @@ __global__ __launch_bounds__(512, 1) void ring_out_kernel(const MP p) {
         NHA_FENCE();
       }
     }
+    if constexpr (RAW)
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Sn[kk][0][r] = Sn[kk][0][r] * cs + nm[0];
     if (is_edge(u + 1)) mask_unit(Sn, u + 1);
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int qb = 0; qb < RQB; ++qb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) Sc[kk][qb][r] = RAW ? Sn[kk][qb][r] * csw + nm[qb] : Sn[kk][qb][r];
+      for (int qb = 0; qb < RQB; ++qb) Sc[kk][qb] = Sn[kk][qb];
   }
   // ---- the last unit: no further scores; the slot-branch queries of the first query block are
   //      requested into the registers the window queries leave ----

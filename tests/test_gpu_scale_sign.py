@@ -25,3 +25,16 @@ def test_forward_and_gradients(H, NG, D, sign, wl):
         res.append([*(t.detach() for t in out), *torch.autograd.grad(out[0], x, do.cuda().to(dt))])
     for name, got, ref in zip(("o", "lse_swa", "lse_gsa", *("d" + k for k in KEYS)), *res):
         check_grad(name, got, ref.double().cpu(), BF)
+
+
+@pytest.mark.parametrize("HQ,H,D,T", [(8, 2, 128, 95), (16, 4, 64, 300), (72, 18, 128, 500)])   # two heads a workgroup, two, four
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_broken_window_queries_at_a_scale_of_zero(HQ, H, D, T, value):
+    """0 times an infinity or a NaN is a NaN: the query's own output row is not finite, and no other (fp32 kernels)."""
+    from nha_amd import chunk_nha
+    d = prefill_inputs(78, 1, T, HQ, H, D, D, 64, dtype=BF)
+    d["q_swa"][0, 70, 3, 5] = value
+    got, ref = (chunk_nha(*(d[k].cuda().to(dt) for k in KEYS), scale=0.0, window_size_left=63, impl=impl)[0].isfinite()
+                for dt, impl in ((BF, "mfma"), (torch.float32, "simple")))
+    assert not ref[0, 70, 3].any() and ref.sum().item() == ref.numel() - D
+    assert (got != ref).sum().item() == 0
