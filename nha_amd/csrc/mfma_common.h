@@ -242,7 +242,9 @@ __device__ __forceinline__ int seb_base(int Q) { return Q == 0 ? 0 : Q == 1 ? 2 
 
 }  // namespace mf
 
-// prefill_mfma.hip: the state pass in segment form
+// prefill_mfma.hip: the workgroups of level 2 of the forward's state pass in one launch, 0 where it takes two
+int64_t state_link_grid(int NT, int N, int H, int D, int seg_sh);
+// the state pass in segment form
 int prefill_mfma_segment_states(const NhaPrefillArgs* a, mf::MP* out);
 // prefill_bwd_slot.hip: the slot branch of the backward but for the carried state gradient, from a state pass in segment form; in
 // how many parts the query heads of a kv-head are summed, each part's sums of its own after those of the one before

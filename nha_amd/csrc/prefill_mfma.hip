@@ -1263,8 +1263,8 @@ int run_state_pass(const MP& p, bool segment_form, hipStream_t st) {
   }
   hipLaunchKernelGGL((mfma_state_local_kernel<D, DW>), dim3((unsigned)l1_grid), dim3(256), lds, st, p);
   NHA_CHECK_LAUNCH("nha_prefill_fwd(mfma state pass, level 1)");
-  const int64_t link_grid = (int64_t)nslot * p.H * (2 * MS * D / 1024);
-  if (!segment_form && (int64_t)p.NT <= ((int64_t)LINK_SEGS * p.N << p.seg_sh) && link_grid <= 0x7fffffff) {
+  const int64_t link_grid = segment_form ? 0 : state_link_grid(p.NT, p.N, p.H, D, p.seg_sh);
+  if (link_grid) {
     hipLaunchKernelGGL((state_link_kernel<D>), dim3((unsigned)link_grid), dim3(256), 0, st, p);
   } else {
     hipLaunchKernelGGL((state_scan_kernel<D>), dim3(p.N * p.H, 2 * MS * D / 1024), dim3(256), 0, st, p);
@@ -1319,6 +1319,13 @@ int run_mfma(const MP& p, int phases, hipStream_t st) {
 static size_t aligned(size_t x) { return (x + 255) & ~(size_t)255; }
 
 }  // namespace
+
+// A launch holds fewer than 2^32 threads, 2^24 workgroups here; scan and rewrite, whose grids have three dimensions, take larger calls
+// (65535 sequences of one chunk, 16 kv-heads of 128: 33 M).
+int64_t state_link_grid(int NT, int N, int H, int D, int seg_sh) {
+  const int64_t grid = ((int64_t)(NT >> seg_sh) + N) * H * (2 * MS * D / 1024);
+  return (int64_t)NT <= ((int64_t)LINK_SEGS * N << seg_sh) && grid < 1 << 24 ? grid : 0;
+}
 
 bool prefill_mfma_supported(const NhaPrefillArgs* a) {
   return a->dtype == NHA_DTYPE_BF16 && a->K == a->V && (a->K == 64 || a->K == 128 || a->K == 256) && a->M == MS;
