@@ -391,10 +391,11 @@ int nha_hybrid_prologue(const NhaHybridPrologueArgs* a);
  *   o_t = sum_j e^(scale q_t.k_j) v_j / (sum_j e^(scale q_t.k_j) + sinks_in_view(t)).
  * q [T_tot,HQ,D] and k, v [T_tot,H,D] packed as for nha_prefill_fwd (q and k already rotated), with the
  * same three index tables; o [T_tot,HQ,D]; lse [T_tot,HQ] fp32 or NULL: the log of the denominator.
- * One launch of the prefill's window loop (no slot branch, no state pass) + an exact pass for rows whose
- * sums leave the range of the fixed softmax reference.  Served: bf16, D = 64 or 128, HQ / H a
+ * One launch of the prefill's window loop (no slot branch, no state pass), which forms rows whose sums leave
+ * the range of the fixed softmax reference again, exactly.  Served: bf16, D = 64 or 128, HQ / H a
  * multiple of four; other shapes return NHA_ERR_UNSUPPORTED (callers then run nha_prefill_fwd with
- * zero slot writes and nha_zero_sink_rescale).  scratch: nha_sink_window_scratch_bytes(a) bytes. */
+ * zero slot writes and nha_zero_sink_rescale).  scratch is not used and may be NULL: nha_sink_window_scratch_bytes(a)
+ * is 0. */
 typedef struct NhaSinkWindowArgs {
   const void* q;
   const void* k;

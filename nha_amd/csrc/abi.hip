@@ -309,25 +309,18 @@ static int check_sink_window(const NhaSinkWindowArgs* a, bool pointers) {
     NHA_CHECK_ARG(a->q && a->k && a->v && a->o, "nha_sink_window_fwd: q, k, v, o are required");
     NHA_CHECK_ARG(a->cu_seqlens && a->chunk_indices && a->chunk_offsets,
                   "nha_sink_window_fwd: cu_seqlens, chunk_indices and chunk_offsets are required");
-    NHA_CHECK_ARG(a->scratch != nullptr, "nha_sink_window_fwd: scratch is required");
   }
   return NHA_OK;
 }
 
 size_t nha_sink_window_scratch_bytes(const NhaSinkWindowArgs* a) {
-  if (check_sink_window(a, false) != NHA_OK) return 0;
-  return sink_window_scratch_bytes(a);
+  check_sink_window(a, false);
+  return 0;
 }
 
 int nha_sink_window_fwd(const NhaSinkWindowArgs* a) {
   const int rc = check_sink_window(a, true);
-  if (rc != NHA_OK) return rc;
-  const size_t need = sink_window_scratch_bytes(a);
-  if (a->scratch_bytes < need) {
-    set_error("nha_sink_window_fwd: scratch has %zu bytes, %zu needed", a->scratch_bytes, need);
-    return NHA_ERR_SCRATCH;
-  }
-  return sink_window_impl(a);
+  return rc != NHA_OK ? rc : sink_window_impl(a);
 }
 
 int nha_layer_epilogue(const NhaLayerEpilogueArgs* a) {

@@ -900,10 +900,7 @@ int prefill_ring_launch(const mf::MP& p, int D, hipStream_t st) {
   return D == 64 ? launch_ring<64, false, 2>(p, st) : launch_ring<128, false, 2>(p, st);
 }
 
-// Sliding-window attention with zero sinks (nha_sink_window_fwd): the window loop of ring_out_kernel alone.  (What
-// goes to the exact pass stays on the chip: the scratch that callers bring is not used any more.)
-size_t sink_window_scratch_bytes(const NhaSinkWindowArgs* a) { return ((size_t)a->NT * a->H * 4 * sizeof(int) + 255) & ~(size_t)255; }
-
+// Sliding-window attention with zero sinks (nha_sink_window_fwd): the window loop of ring_out_kernel alone.
 int sink_window_impl(const NhaSinkWindowArgs* a) {
   mf::MP p = {};
   p.q_swa = (const bf16_t*)a->q; p.k_swa = (const bf16_t*)a->k; p.v = (const bf16_t*)a->v;

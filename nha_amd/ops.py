@@ -932,11 +932,7 @@ def zero_sink_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, windo
                                chunk_indices=_ptr(idx_d), chunk_offsets=_ptr(off_d), T_tot=B * T, N=cu_host.size - 1, NT=NT,
                                HQ=HQ, H=H, D=D, window=int(window), sinks=int(num_sinks), dtype=_dtype_code(q),
                                scale=float(scale), stream=_stream(dev))
-    lib = _lib.load()
-    nbytes = lib.nha_sink_window_scratch_bytes(C.byref(a))
-    scratch = _workspace(nbytes, dev, a.stream or 0)
-    a.scratch, a.scratch_bytes = _ptr(scratch), nbytes
-    _lib.check(lib.nha_sink_window_fwd(C.byref(a)))
+    _lib.check(_lib.load().nha_sink_window_fwd(C.byref(a)))
     o = o.view(B, T, HQ, D)
     return (o, lse.view(B, T, HQ)) if output_lse else o
 

@@ -131,6 +131,18 @@ def test_argument_validation_without_gpu():
         chunk_tables([1, 5])             # does not start at 0
 
 
+def test_sink_window_needs_no_scratch():
+    """Neither a size to allocate nor, of a valid block, anything but the pointers that it reads and writes."""
+    lib = _lib.load()
+    a = _lib.NhaSinkWindowArgs(T_tot=130, N=1, NT=3, HQ=8, H=2, D=128, window=96, sinks=64, dtype=_lib.NHA_DTYPE_BF16, scale=0.1)
+    assert lib.nha_sink_window_scratch_bytes(C.byref(a)) == 0 and lib.nha_sink_window_scratch_bytes(None) == 0
+    for f in ("q", "k", "v", "o", "cu_seqlens", "chunk_indices", "chunk_offsets"):
+        assert lib.nha_sink_window_fwd(C.byref(a)) == _lib.NHA_ERR_INVALID and b"required" in lib.nha_last_error()
+        setattr(a, f, 4096)
+    a.dtype = _lib.NHA_DTYPE_F32
+    assert lib.nha_sink_window_fwd(C.byref(a)) == _lib.NHA_ERR_UNSUPPORTED
+
+
 def test_varlen_tables_bit_exact_vs_oracle():
     random.seed(0)
     cases = [[128] * 4, [128, 64, 200, 10], [4096, 2048, 1, 1024, 2],
