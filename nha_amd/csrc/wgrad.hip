@@ -9,10 +9,11 @@
 // Bound: the matrix rate that this chip sustains (1.2 PFLOP/s, as a large library product) where the tiles
 // fill it, and the fp32 sums' way through memory where few outputs make many splits.  Eight waves hold 128 x 64 of a tile
 // each; a unit's fragments are in registers when its products begin and are replaced as they are done with.  Through registers and
-// padded rows, two buffers of 64 tokens, no read ahead: 16384 tokens, 1024 columns, outputs of 3 x 1024 + 256 127 us with the sum,
-// now 119 (0.93 PFLOP/s; four library products, which run 64 x 64 tiles without a split, 415); one output of 1024 53, 53 (library
-// 104); 2048 columns, 2048 + 2 x 512 + 256 217, 207 (468); 3072 columns, 3072 + 2 x 768 + 512 460, 440; 4096 tokens, 1024 columns,
-// 1024 + 2 x 256 + 128 44.5, 39.  A fifth unit in LDS: 123 and 40 where four take 119 and 39.
+// padded rows, two buffers of 64 tokens, no read ahead / now, in turn on one card, with the sum: 16384 tokens, 1024 columns, outputs of
+// 3 x 1024 + 256 118 / 112 us (1.0 PFLOP/s; four library products, which run 64 x 64 tiles without a split, 415), one output of 1024 57 / 55
+// (library 104); 2048 columns, 2048 + 2 x 512 + 256 221 / 208 (468); 3072 columns, 3072 + 2 x 768 + 512 462 / 429; 4096 tokens, 1024
+// columns, 1024 + 2 x 256 + 128 44 / 35.5.  Inside a training step of the layer (8 x 2048 tokens), where the operands come from HBM, both
+// launches of each 181 / 175.  A fifth unit in LDS is no faster.
 #include "mfma_common.h"
 
 #include <atomic>
@@ -179,15 +180,17 @@ __global__ __launch_bounds__(256) void wgrad_sum_kernel(const WG p) {
   Elem<bf16_t>::st8(p.dw[q] + (int64_t)(r - p.row0[q]) * p.I + c, s);
 }
 
-// Token splits: a round of the chip is 256 workgroups; a unit of 32 tokens costs 0.6 us and a workgroup's start and end 6,
-// a split's round trip in fp32 its bytes (4 written and 4 read per element) at 4.5 TB/s.
+// Token splits: a round of the chip is 256 workgroups; a unit of 32 tokens costs 0.5 us and a workgroup's start and end 4, a split's round
+// trip in fp32 (which mostly stays in the caches) its bytes, 4 written and 4 read per element, at 10 TB/s.  Fitted to the calls' times with 1
+// to 32 splits.  With 0.6, 6 and 4.5 TB/s, us before / now: 16384 tokens, 1024 columns, one output of 1024 58.0 (12 splits) / 55.1 (16),
+// 12000 47.3 (10) / 43.4 (15), 8192 43.8 (8) / 39.8 (13); 4096, outputs of 1024 + 2 x 256 + 128 38.9 (5) / 35.5 (8).
 int wgrad_split(int tiles, int T, int64_t elements) {
   const int steps = (T + TK - 1) / TK;
   int best = 1;
   double cost = 1e30;
   for (int s = 1; s <= 32 && s <= steps; ++s) {
     const double rounds = (double)(((int64_t)tiles * s + 255) / 256);
-    const double us = rounds * (((steps + s - 1) / s) * 0.6 + 6.0) + s * (double)elements * 8.0 / 4.5e6;
+    const double us = rounds * (((steps + s - 1) / s) * 0.5 + 4.0) + s * (double)elements * 8.0 / 1e7;
     if (us < cost) {
       cost = us;
       best = s;
