@@ -179,12 +179,14 @@ __global__ __launch_bounds__(512) void bwd_slot_kernel(const SlotP p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
   const bool vs = wave >= 4;
   const int H = p.H, HQ = p.HQ, NG = p.NG, part = ONE ? 0 : blockIdx.z;
-  // Several heads, two rounds of workgroups or more: the 32 CUs of an XCD start 0.2 us after one another (the second round follows from
-  // the first).  All in step, their products come at the same moments, and some cards then run every matrix kernel of the following
-  // milliseconds 5 % slower, at the same clock: steps of 2 x 8192 tokens, 32 / 8 heads of 128, W = 2048 one after another 2950 -> 2740
-  // us, W = 512 1686 -> 1565, 5000 tokens 666 -> 640 (0.1 us 641, 2820 and 1615; 0.4 us 2735 and 1563); on a card that does not, the
-  // same times within 0.2 %.  One round: 2001 tokens 273 -> 280 us, not staggered.
-  if (!ONE && !EXACT && gridDim.x * gridDim.y >= 512) {
+  // Several heads of 128 columns, two rounds of workgroups or more: the 32 CUs of an XCD start 0.2 us after one another (the second round
+  // follows from the first).  All in step, their products come at the same moments, and two of the three cards that this was measured on
+  // then run every matrix kernel of the following milliseconds up to 5 % slower, at the same clock: steps of 2 x 8192 tokens, 32 / 8 heads of 128, W =
+  // 2048 one after another 2950 -> 2740 us, W = 512 1686 -> 1565, 5000 tokens 666 -> 640 (0.1 us 641, 2820 and 1615; 0.4 us 2735 and 1563).
+  // On the second 2748 -> 2712, 1595 -> 1516, 630 -> 624; on the third 2658 -> 2657, 1512 -> 1506, 623 -> 622.  4 x 4096 tokens, 8 / 2
+  // heads of 256: 957 on all.  Not at head size 64, where it only costs (2 x 4096 tokens, 16 / 4 heads, W = 300 282.4 -> 284.4), nor in one
+  // round (2001 tokens 273 -> 280 us).
+  if (D >= 128 && !ONE && !EXACT && gridDim.x * gridDim.y >= 512) {
     const unsigned L = blockIdx.y * gridDim.x + blockIdx.x;
     if (L < 256)
       for (unsigned i = 0; i < L >> 3; ++i) __builtin_amdgcn_s_sleep(8);
