@@ -327,11 +327,6 @@ constexpr int KV_Q = 0, KV_O = UB, KV_LD = 2 * UB, KV_ITEM = 2 * UB + 256;
 template <int G> constexpr int KV_NR = G == 2 ? 7 : 4;   // items in LDS
 template <int KEYS, int G> constexpr int KV_BYTES = KV_NR<G> * KV_ITEM + KEYS * D * 2;   // ring, then the V rows of the workgroup's keys
 
-// KEYS: keys per workgroup, 256 or 128, G: the waves in G groups, each with all keys and every G-th item, whose sums are added at the end.
-// A wave with 32 keys feeds two matrix products with every q / do fragment it reads from LDS, one with 16 keys (128, G = 1) only one:
-// long windows are bound by those reads (B=2, T=8192, 32/8 heads, W=2048: 256 keys 1.17 ms, 128 1.5, 128 in two groups 1.26).  Windows up
-// to 160 keys, where a workgroup's walk is a few items long, take 128 keys and one group (W=64 145 us, two groups 169); two groups are
-// for calls whose groups of 256 keys leave CUs without work (key_groups): 4000 tokens, W=1000 263 -> 172 us, 233 with bwd_dkv_kernel.
 // waits until at most `younger` items' requests of this wave are in flight
 template <int LPW, int G>
 __device__ __forceinline__ void wait_items(int younger) {
@@ -343,6 +338,11 @@ __device__ __forceinline__ void wait_items(int younger) {
   else wait_vm<0>();
 }
 
+// KEYS: keys per workgroup, 256 or 128, G: the waves in G groups, each with all keys and every G-th item, whose sums are added at the end.
+// A wave with 32 keys feeds two matrix products with every q / do fragment it reads from LDS, one with 16 keys (128, G = 1) only one:
+// long windows are bound by those reads (B=2, T=8192, 32/8 heads, W=2048: 256 keys 1.17 ms, 128 1.5, 128 in two groups 1.26).  Windows up
+// to 160 keys, where a workgroup's walk is a few items long, take 128 keys and one group (W=64 145 us, two groups 169); two groups are
+// for calls whose groups of 256 keys leave CUs without work (key_groups): 4000 tokens, W=1000 263 -> 172 us, 233 with bwd_dkv_kernel.
 template <int KEYS, int G, bool PARTS>
 __global__ __launch_bounds__(512, 1) void ring_dkv_kernel(const DkvP p) {
   constexpr int KW = 8 / G;                // waves that hold the keys, each of G groups all of them

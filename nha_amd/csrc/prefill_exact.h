@@ -14,7 +14,7 @@
 // / 1170; head size 256, 32768 packed, W = 512 307 / 304, 4 x 8192, 8 / 2 heads, W = 2000 659 / 654; 16 heads of 128, 4 x 8192, W = 64
 // 532 / 523.  At head size 64 with one or two heads the instance has room for it only at some cost: 16 heads, 2 x 8192, W = 2048 330 /
 // 333, W = 64 176.6 / 172.7, 5003 tokens 74.4 / 72.4, 300 30.4 / 27.2; there short passes, EXACT_INSIDE_US as estimated from the rounds
-// of workgroups, take it and the others the launch.  Every row flagged: four heads of 128, 4096 tokens, W = 512 23.5 / 22.7 ms, 4 heads
+// of workgroups, take it and the others the launch; so do two heads of 128 or 64 with more than a workgroup for every CU (no registers).  Every row flagged: four heads of 128, 4096 tokens, W = 512 23.5 / 22.7 ms, 4 heads
 // of 256 7.3 / 7.1.
 #pragma once
 #include "mfma_common.h"

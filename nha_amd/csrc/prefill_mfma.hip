@@ -237,7 +237,7 @@ __global__ __launch_bounds__(256) void mfma_state_local_kernel(const MP p) {
     if (!isv && lead) {
       if (kb == 0) p.dcum[cg * MS + m] = fexp(gsum);
       // 16-row sub-blocks over which some slot decays by more than exp(DECAY_CLAMP): the output
-      // pass cannot factor their intra-block decay; mfma_repair_kernel recomputes their rows
+      // pass cannot factor their intra-block decay, and their rows are formed again exactly (prefill_exact.h)
       int bits = 0;
       if (kb == 3) {
 #pragma unroll
@@ -1357,12 +1357,14 @@ ScratchPlan plan_scratch(const NhaPrefillArgs* a, int seg_sh) {
   return s;
 }
 
-// Chunks per segment: 8, where the chip is full.  Level 1 walks its segment at 2.4 us per chunk whatever else runs, so a
-// call that leaves places on the chip empty takes shorter segments, as long as all its workgroups are resident at once
-// (two per CU at head sizes 128 and 256, three at 64, by registers); level 2 then combines more of them, at about 0.25 us
-// each: hence the weights 11 : 1.  Level 1 / state pass at 1000 tokens, 8 kv-heads of 128: 25.4 / 31.6 us with 8 chunks,
-// 15.9 / 21.3 with 4, 9.0 / 20.3 with 1; 4 heads of 256 25.4 / 31.9, 16.7 / 21.9, 9.7 / 21.3.  More workgroups than places
-// lose: 2 x 2048 tokens, 8 heads of 128 take 35 us with 8 chunks, 30 with 4 and 43 with 1.
+// Chunks per segment: 8, where the chip is full.  Level 1 walks its segment at 2 us per chunk whatever else runs, so a call that leaves
+// places on the chip empty takes shorter segments, as long as all its workgroups are resident at once (two per CU at head sizes 128 and
+// 256, three at 64, by registers); level 2 then combines more of them.  The weights 11 : 1 are those of level 2 as a chain over the segments,
+// about 0.25 us each, as in the backward and in sequences of more than LINK_SEGS segments; in one launch a segment costs 0.3 us with
+// slow gates and 0.2 with fast ones.  Level 1 + level 2 in one launch, slow gates, with 8, 4, 2 and 1 chunks, us: 1000 tokens, 8 kv-heads of
+// 128 24.2 + 5.0, 16.3 + 5.5, 12.9 + 6.5, 11.9 + 9.7; 4 of 256 23.4 + 4.9, 16.2 + 5.0, 13.4 + 6.0, 12.5 + 9.4; so there the rule takes 1 chunk
+// where 2 would be 1 to 2 us faster.  More workgroups than places lose: 2 x 2048 tokens, 8 heads of 128 32.5 us with 8 chunks, 26.0 with
+// 4, 29.1 with 2.
 // A call whose workspace fits the library's own array with 8 chunks keeps fitting it.
 ScratchPlan plan_scratch(const NhaPrefillArgs* a) {
   const ScratchPlan full = plan_scratch(a, 3);

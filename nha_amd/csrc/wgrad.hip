@@ -13,7 +13,7 @@
 // 3 x 1024 + 256 118 / 112 us (1.0 PFLOP/s; four library products, which run 64 x 64 tiles without a split, 415), one output of 1024 57 / 55
 // (library 104); 2048 columns, 2048 + 2 x 512 + 256 221 / 208 (468); 3072 columns, 3072 + 2 x 768 + 512 462 / 429; 4096 tokens, 1024
 // columns, 1024 + 2 x 256 + 128 44 / 35.5.  Inside a training step of the layer (8 x 2048 tokens), where the operands come from HBM, both
-// launches of each 181 / 175.  A fifth unit in LDS is no faster.
+// launches of each 192 / 182.  A fifth unit in LDS is no faster.
 #include "mfma_common.h"
 
 #include <atomic>
